@@ -9,13 +9,12 @@ merge, MoE, grouped GEMM) are exported under ``py*`` names in the same style.
 """
 from __future__ import annotations
 
-import ctypes as C
 import weakref
 from typing import Optional
 
 import torch
 
-from . import _lib
+from . import _host, _lib
 
 __all__ = ["add_tensors", "pygemm", "dense_gemm", "dense_ok", "keep_transposed", "refresh_transposed", "wgrad_gemm", "wgrad_layout", "pygelu", "pybda", "pymha_varlen_fwd", "pymha_varlen_bwd", "pyattn_merge",
            "pyrmsnorm_fwd", "pyrmsnorm_bwd", "pyrope_fwd", "pyrope_bwd", "pyswiglu_fwd", "pyswiglu_bwd",
@@ -45,19 +44,18 @@ def add_tensors(a, b):
     return a + b
 
 
-GEMM_WORKSPACE_BYTES = 32 << 20
-_gemm_ws: dict = {}
+GEMM_WORKSPACE_BYTES = _host.GEMM_WORKSPACE_BYTES
 
 
-def _gemm_workspace(device, stream_ptr: int) -> torch.Tensor:
-    """One workspace per (device, stream): kernels that split a product over workgroups keep partial tiles
-    there, so two streams must not share one."""
-    key = (str(device), stream_ptr)
-    ws = _gemm_ws.get(key)
-    if ws is None:
-        ws = torch.empty(GEMM_WORKSPACE_BYTES, dtype=torch.uint8, device=device)
-        _gemm_ws[key] = ws
-    return ws
+class _GemmWorkspaces:
+    """The (device, stream handle) pairs that have a GEMM workspace.  One per stream: kernels that split a product over
+    workgroups keep partial tiles there, so two streams must not share one."""
+
+    def __iter__(self):
+        return iter(_host.scratch_keys(_host.SCRATCH_GEMM))
+
+
+_gemm_ws = _GemmWorkspaces()
 
 
 def dense_ok(*tensors) -> bool:
@@ -65,35 +63,11 @@ def dense_ok(*tensors) -> bool:
     return all(t.is_cuda and t.dim() == 2 and t.is_contiguous() for t in tensors)
 
 
-def dense_gemm(A, B, D, transa: bool, transb: bool, accumulate: bool, workspace=None, workspace_bytes: int = 0) -> None:
-    """``dh_gemm`` on the current stream, in the reference's operand convention (see ``pygemm``)."""
-    if not dense_ok(A, B, D):
-        raise RuntimeError("dense_gemm: operands must be contiguous 2-D GPU tensors")
-    if A.dtype != B.dtype or D.dtype not in (A.dtype, torch.float32):
-        raise RuntimeError(f"dense_gemm: operand types {A.dtype}, {B.dtype} -> {D.dtype} not supported")
-    m = A.shape[0] if transa else A.shape[1]
-    n = B.shape[1] if transb else B.shape[0]
-    if tuple(D.shape) != (n, m):
-        raise RuntimeError(f"dense_gemm: output is {tuple(D.shape)}, the product is {(n, m)}")
-    stream = torch.cuda.current_stream()
+def dense_gemm(A, B, D, transa: bool, transb: bool, accumulate: bool, workspace=None, workspace_bytes: int = 0,
+               stream=None) -> None:
+    """``dh_gemm`` on ``stream`` (default: the current one), in the reference's operand convention (see ``pygemm``)."""
     _lib.mark_written(D)
-    if workspace is None or not getattr(workspace, "is_cuda", False) or workspace_bytes <= 0:
-        workspace = _gemm_workspace(A.device, stream.cuda_stream)
-        workspace_bytes = workspace.numel()
-    elif workspace.numel() * workspace.element_size() < workspace_bytes:
-        raise RuntimeError("dense_gemm: workspace tensor smaller than workspaceSize")
-    if (transa and A.shape[1] == 0) or (not transa and A.shape[0] == 0):
-        if not accumulate:
-            D.zero_()
-        return
-    if transa and transb:      # refused by dh_gemm as by the reference's cublas_gemm; the library's own entry for it
-        _lib.check(_lib.load().dh_gemm_tt(A.data_ptr(), B.data_ptr(), D.data_ptr(), A.shape[0], A.shape[1], B.shape[0],
-                                          B.shape[1], int(accumulate), _lib.dt(A), _lib.dt(D), workspace.data_ptr(),
-                                          workspace_bytes, stream.cuda_stream))
-        return
-    _lib.check(_lib.load().dh_gemm(A.data_ptr(), B.data_ptr(), D.data_ptr(), A.shape[0], A.shape[1], B.shape[0],
-                                   B.shape[1], int(transa), int(transb), int(accumulate), _lib.dt(A), _lib.dt(D),
-                                   workspace.data_ptr(), workspace_bytes, stream.cuda_stream))
+    _host.dense_gemm(A, B, D, transa, transb, accumulate, workspace, workspace_bytes, stream)
 
 
 def pygemm(inputA, inputB, outputD, input_workspace, workspaceSize, transa, transb, grad_accumulate, math_sm_count,
@@ -165,19 +139,9 @@ def _confined(stream, math_sm_count, launch):
     return res
 
 
-def transpose_2d(src: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """Row-major [rows, cols] -> row-major [cols, rows] (16-bit elements) on the current stream."""
-    _lib.need_cuda(src)
-    if not (src.dim() == 2 and src.stride(1) == 1):
-        raise RuntimeError("transpose_2d: src must be 2-D with unit inner stride")
-    rows, cols = src.shape
-    if out is None:
-        out = torch.empty((cols, rows), dtype=src.dtype, device=src.device)
-    elif not (out.shape == (cols, rows) and out.stride(1) == 1 and out.dtype == src.dtype):
-        raise RuntimeError("transpose_2d: out must be [cols, rows] of src's dtype with unit inner stride")
-    _lib.check(_lib.load().dh_transpose_2d(src.data_ptr(), out.data_ptr(), rows, cols, src.stride(0), out.stride(0),
-                                           _lib.dt(src), torch.cuda.current_stream().cuda_stream))
-    return out
+def transpose_2d(src: torch.Tensor, out: Optional[torch.Tensor] = None, stream=None) -> torch.Tensor:
+    """Row-major [rows, cols] -> row-major [cols, rows] (16-bit elements) on ``stream`` (default: the current one)."""
+    return _host.transpose_2d(src, out, stream)
 
 
 # The weight-gradient product dW[N, K] = dY[T, N]^T X[T, K] reads both operands along their strided dimension, the
@@ -225,7 +189,7 @@ def wgrad_operands(grad: torch.Tensor, data: torch.Tensor):
 
 
 def wgrad_gemm(grad: torch.Tensor, data: torch.Tensor, out: torch.Tensor, accumulate: bool, workspace=None,
-               workspace_bytes: int = 0) -> None:
+               workspace_bytes: int = 0, stream=None) -> None:
     """out [N, K] (+)= grad [T, N]^T @ data [T, K] through the GEMM library, in the layout ``wgrad_layout`` picks."""
     layout = wgrad_layout(grad, data)
     if layout == "NN":
@@ -233,16 +197,16 @@ def wgrad_gemm(grad: torch.Tensor, data: torch.Tensor, out: torch.Tensor, accumu
         version, gt = getattr(grad, "_dh_rows_transposed", None) or (None, None)
         if (gt is None or version != grad._version or gt.shape != (grad.shape[1], grad.shape[0])
                 or gt.dtype != grad.dtype):
-            gt = transpose_2d(grad)
-        dense_gemm(data, gt, out, False, False, accumulate, workspace, workspace_bytes)
+            gt = transpose_2d(grad, None, stream)
+        dense_gemm(data, gt, out, False, False, accumulate, workspace, workspace_bytes, stream)
     elif layout == "TT":
         version, xt = getattr(data, "_dh_rows_transposed", None) or (None, None)
         if (xt is None or version != data._version or xt.shape != (data.shape[1], data.shape[0])
                 or xt.dtype != data.dtype):
-            xt = transpose_2d(data)
-        dense_gemm(xt, grad, out, True, True, accumulate, workspace, workspace_bytes)
+            xt = transpose_2d(data, None, stream)
+        dense_gemm(xt, grad, out, True, True, accumulate, workspace, workspace_bytes, stream)
     else:
-        dense_gemm(data, grad, out, False, True, accumulate, workspace, workspace_bytes)
+        dense_gemm(data, grad, out, False, True, accumulate, workspace, workspace_bytes, stream)
 
 
 # The data-gradient product dX[T, K] = dY[T, N] W[N, K] reads the weight along its strided dimension ("NN").  With
@@ -322,44 +286,47 @@ def refresh_transposed(weights=None) -> int:
     return n
 
 
-def transposed_of(weight: torch.Tensor) -> Optional[torch.Tensor]:
-    """The resident transpose of a registered weight, brought up to date and safe to read on the current stream;
-    None for a weight that was not registered with ``keep_transposed``.  The reader calls ``_note_read`` after
-    it has queued its work."""
+def transposed_of(weight: torch.Tensor, stream=None) -> Optional[torch.Tensor]:
+    """The resident transpose of a registered weight, brought up to date and safe to read on ``stream`` (default: the
+    current one); None for a weight that was not registered with ``keep_transposed``.  The reader calls ``_note_read``
+    after it has queued its work."""
     held = getattr(weight, "_dh_transposed", None)
     if held is None:
         return None
     if held.version != weight._version:
-        return keep_transposed(weight, refresh=True)
-    stream = torch.cuda.current_stream()
-    if held.stream_ptr != stream.cuda_stream:
-        stream.wait_event(held.built)
+        with torch.cuda.stream(stream):
+            return keep_transposed(weight, refresh=True)
+    if held.stream_ptr != _host.stream_ptr(stream):
+        (stream or torch.cuda.current_stream()).wait_event(held.built)
     return held.wt
 
 
-def _note_read(weight: torch.Tensor) -> None:
-    """Marks the point on the current stream up to which the resident transpose of ``weight`` is being read."""
+def _note_read(weight: torch.Tensor, stream=None) -> None:
+    """Marks the point on ``stream`` (default: the current one) up to which the resident transpose of ``weight`` is
+    being read."""
     held = getattr(weight, "_dh_transposed", None)
     if held is None:
         return
-    stream = torch.cuda.current_stream()
-    if stream.cuda_stream == held.stream_ptr:
+    ptr = _host.stream_ptr(stream)
+    if ptr == held.stream_ptr:
         return                                        # same stream as the builder: already ordered
-    ev = held.readers.get(stream.cuda_stream)
+    ev = held.readers.get(ptr)
     if ev is None:
-        ev = held.readers[stream.cuda_stream] = torch.cuda.Event()
-    ev.record(stream)
+        ev = held.readers[ptr] = torch.cuda.Event()
+    ev.record(stream or torch.cuda.current_stream())
 
 
-def dgrad_gemm(grad: torch.Tensor, weight: torch.Tensor, out: torch.Tensor) -> None:
-    """out [T, K] = grad [T, N] @ weight [N, K] through ``dh_gemm``: in the forward's layout against the resident
-    transpose when the weight has one, else as given."""
-    wt = transposed_of(weight)
+def dgrad_gemm(grad: torch.Tensor, weight: torch.Tensor, out: Optional[torch.Tensor] = None, stream=None) -> torch.Tensor:
+    """out [T, K] (made on ``stream`` if not given) = grad [T, N] @ weight [N, K] through ``dh_gemm``: in the forward's
+    layout against the resident transpose when the weight has one, else as given."""
+    if out is not None:
+        _lib.mark_written(out)
+    wt = transposed_of(weight, stream)
     if wt is not None and wt.dtype == grad.dtype:
-        dense_gemm(wt, grad, out, True, False, False)
-        _note_read(weight)
-    else:
-        dense_gemm(weight, grad, out, False, False, False)
+        out = _host.matmul(wt, grad, out, True, stream)
+        _note_read(weight, stream)
+        return out
+    return _host.matmul(weight, grad, out, False, stream)
 
 
 def pygelu(input, output, profiling):
@@ -389,20 +356,6 @@ def pybda(input, bias, residual, output, prob, profiling):
 # ---------------------------------------------------------------------------------------
 # attention
 # ---------------------------------------------------------------------------------------
-def _tok_stride(t: torch.Tensor) -> int:
-    if not (t.dim() == 3 and t.stride(2) == 1 and t.stride(1) == t.shape[2]):
-        raise RuntimeError("attention tensors must be [tokens, heads, d] with contiguous (heads, d)")
-    return t.stride(0)
-
-
-def _attn_fwd_raw(q, k, v, out, lse, cu_q, cu_k, max_q, max_k, scale, causal, stream_ptr):
-    lib = _lib.load()
-    _lib.check(lib.dh_attn_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr(),
-                               cu_q.data_ptr(), cu_k.data_ptr(), cu_q.numel() - 1, int(max_q), int(max_k),
-                               q.shape[1], k.shape[1], q.shape[2], _tok_stride(q), _tok_stride(k), _tok_stride(v),
-                               _tok_stride(out), float(scale), int(bool(causal)), _lib.dt(q), stream_ptr))
-
-
 HEAD_DIMS_16BIT = (64, 96, 128, 192, 256)      # head dims the 16-bit kernels are compiled for
 
 
@@ -418,10 +371,10 @@ def _pad_head_dim(t: torch.Tensor, d_to: int) -> torch.Tensor:
     return out
 
 
-def _kernel_head_dim(t: torch.Tensor) -> int:
-    """The head dim the kernels run ``t`` at: its own for fp32 and for the compiled 16-bit sizes, else the next
-    compiled size (d <= 256 as in the reference, flash_atten.cu:284)."""
-    d = t.shape[-1]
+def _kernel_head_dim(t: torch.Tensor, d: Optional[int] = None) -> int:
+    """The head dim the kernels run ``t`` (of head dim ``d``, default: its last dimension) at: its own for fp32 and for
+    the compiled 16-bit sizes, else the next compiled size (d <= 256 as in the reference, flash_atten.cu:284)."""
+    d = t.shape[-1] if d is None else d
     if t.dtype == torch.float32 or d in HEAD_DIMS_16BIT:
         return d
     for s_ in HEAD_DIMS_16BIT:
@@ -458,28 +411,27 @@ def pymha_varlen_fwd(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seql
         raise RuntimeError("pymha_varlen_fwd: dropout is not implemented (p_dropout must be 0)")
     if return_softmax:
         raise RuntimeError("pymha_varlen_fwd: return_softmax is only supported with dropout in the reference")
-    _lib.need_cuda(q, k, v, cu_seqlens_q, cu_seqlens_k)
-    if cu_seqlens_q.dtype != torch.int32 or cu_seqlens_k.dtype != torch.int32:
-        raise RuntimeError("cu_seqlens must be int32")
-    stream = torch.cuda.current_stream()
-    b = cu_seqlens_q.numel() - 1
     d, dk_ = q.shape[-1], _kernel_head_dim(q)
     if dk_ != d:        # the padded tensors are what the "padded" slots of the return list hold (flash_atten.cu:429-433)
         q, k, v = _pad_head_dim(q, dk_), _pad_head_dim(k, dk_), _pad_head_dim(v, dk_)
-    out_padded = torch.empty(q.shape, dtype=q.dtype, device=q.device)
-    lse = torch.empty((b, q.shape[1], int(max_seqlen_q)), dtype=torch.float32, device=q.device)
-    ms = _timed(profiling, stream, lambda: _confined(stream, math_sm_count, lambda st: _attn_fwd_raw(
-        q, k, v, out_padded, lse, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, softmax_scale, is_causal,
-        st.cuda_stream)))
+    args = (q, k, v, cu_seqlens_q, cu_seqlens_k, int(max_seqlen_q), int(max_seqlen_k), softmax_scale, bool(is_causal))
+    ms = 0.0
+    if not profiling and not math_sm_count:
+        out_padded, lse = _host.attn_fwd(*args, None)
+    else:
+        stream, res = torch.cuda.current_stream(), []
+        ms = _timed(profiling, stream, lambda: _confined(stream, math_sm_count, lambda st: res.extend(
+            _host.attn_fwd(*args, st))))
+        out_padded, lse = res
+        if math_sm_count:          # made on the masked stream, handed to the current one
+            out_padded.record_stream(stream)
+            lse.record_stream(stream)
     out = out_padded if dk_ == d else out_padded[..., :d]
     p = torch.empty(0, dtype=q.dtype, device=q.device)
     res = [out, q, k, v, out_padded, lse, p, _zero_rng_state(q.device)]
     if profiling:
         res.append(torch.tensor([ms], dtype=torch.float32))
     return res
-
-
-_bwd_ws: dict = {}
 
 
 ATTN_BWD_DS_LIMIT_DEFAULT = 1280 << 20
@@ -492,30 +444,12 @@ def set_attn_bwd_ds_limit(nbytes: int = ATTN_BWD_DS_LIMIT_DEFAULT) -> None:
     _lib.load().dh_attn_bwd_set_ds_limit(int(nbytes))
 
 
-def _attn_bwd_workspace(nbytes: int, device, stream_ptr: int) -> torch.Tensor:
-    key = (str(device), stream_ptr)
-    ws = _bwd_ws.get(key)
-    if ws is None or ws.numel() < nbytes:
-        ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
-        _bwd_ws[key] = ws
-    return ws
-
-
-def _attn_bwd_raw(dout, q, k, v, out, lse, dq, dk, dv, delta, cu_q, cu_k, max_q, max_k, scale, causal, stream_ptr,
+def _attn_bwd_raw(dout, q, k, v, out, lse, dq, dk, dv, delta, cu_q, cu_k, max_q, max_k, scale, causal, stream=None,
                   accumulate_dq=False):
-    """``dh_attn_bwd``; with ``accumulate_dq`` the call's dq is added to the contents of ``dq`` inside the kernel."""
-    lib = _lib.load()
-    b = cu_q.numel() - 1
-    nbytes = lib.dh_attn_bwd_workspace_bytes(q.shape[0], k.shape[0], b, int(max_q), q.shape[1], k.shape[1],
-                                             q.shape[2], _lib.dt(q))
-    ws = _attn_bwd_workspace(nbytes, q.device, stream_ptr)
-    _lib.check(lib.dh_attn_bwd_acc(dout.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
-                                   lse.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), _lib.ptr(delta),
-                                   ws.data_ptr(), ws.numel(), cu_q.data_ptr(), cu_k.data_ptr(), b, int(max_q), int(max_k),
-                                   q.shape[0], k.shape[0], q.shape[1], k.shape[1], q.shape[2], _tok_stride(q),
-                                   _tok_stride(k), _tok_stride(v), _tok_stride(out), _tok_stride(dout),
-                                   _tok_stride(dq), _tok_stride(dk), _tok_stride(dv), float(scale), int(bool(causal)),
-                                   int(bool(accumulate_dq)), _lib.dt(q), stream_ptr))
+    """``dh_attn_bwd`` on ``stream``; with ``accumulate_dq`` the call's dq is added to the contents of ``dq`` inside the
+    kernel."""
+    _host.attn_bwd(dout, q, k, v, out, lse, dq, dk, dv, delta, cu_q, cu_k, int(max_q), int(max_k), scale, bool(causal),
+                   accumulate_dq, stream)
 
 
 def pymha_varlen_bwd(dout, q, k, v, out, softmax_lse, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k,
@@ -540,7 +474,7 @@ def pymha_varlen_bwd(dout, q, k, v, out, softmax_lse, cu_seqlens_q, cu_seqlens_k
         softmax_d = torch.zeros((b, q.shape[1], int(max_seqlen_q)), dtype=torch.float32, device=q.device)
         ms = _timed(profiling, ext, lambda: _confined(ext, math_sm_count, lambda st: _attn_bwd_raw(
             dout, q, k, v, out, softmax_lse, dq, dk, dv, softmax_d, cu_seqlens_q, cu_seqlens_k, max_seqlen_q,
-            max_seqlen_k, softmax_scale, is_causal, int(st.cuda_stream))))
+            max_seqlen_k, softmax_scale, is_causal, st)))
         if dk_ != d:
             dq, dk, dv = dq[..., :d].contiguous(), dk[..., :d].contiguous(), dv[..., :d].contiguous()
     res = [dq, dk, dv, softmax_d]
@@ -553,21 +487,7 @@ def pyattn_merge(outs, lses, row_begin, rows, out, lse):
     """Fused merge of ring-attention partial results (dhellam/operators/ring_attn.py:26-40
     applied as in :146-195) on the current stream.  outs[s] [b*rows[s], hq, d], lses[s]
     fp32 [b, hq, rows[s]]; out [b*sq, hq, d]; lse fp32 [b, hq, sq]."""
-    lib = _lib.load()
-    n = len(outs)
-    b, hq, sq = lse.shape
-    d = out.shape[-1]
-    po = (C.c_void_p * n)(*[o.data_ptr() for o in outs])
-    pl = (C.c_void_p * n)(*[l.data_ptr() for l in lses])
-    rb = (C.c_int32 * n)(*[int(x) for x in row_begin])
-    rr = (C.c_int32 * n)(*[int(x) for x in rows])
-    for s in range(n):
-        assert outs[s].is_contiguous() and lses[s].is_contiguous() and lses[s].dtype == torch.float32
-        assert outs[s].shape == (b * rows[s], hq, d) and lses[s].shape == (b, hq, rows[s])
-    assert out.is_contiguous() and lse.is_contiguous()
-    _lib.check(lib.dh_attn_merge(C.cast(po, C.c_void_p), C.cast(pl, C.c_void_p), C.cast(rb, C.c_void_p),
-                                 C.cast(rr, C.c_void_p), n, out.data_ptr(), lse.data_ptr(), b, sq, hq, d,
-                                 _lib.dt(out), torch.cuda.current_stream().cuda_stream))
+    _host.attn_merge(outs, lses, row_begin, rows, out, lse, None)
 
 
 # ---------------------------------------------------------------------------------------

@@ -12,6 +12,7 @@ from __future__ import annotations
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -167,45 +168,63 @@ def check_grouped_gemm_loops(verbose: bool = False) -> int:
     return checked
 
 
-EXT_SRC = CSRC / "torchapi.cpp"
 EXT_PKG = ROOT / "dhellam"
+EXT_SUFFIX = sysconfig.get_config_var("EXT_SUFFIX")
+PY_INCLUDE = sysconfig.get_paths()["include"]
 
 
 def torch_extension_path() -> Path:
-    import sysconfig
-    return EXT_PKG / ("_Clib" + sysconfig.get_config_var("EXT_SUFFIX"))
+    return EXT_PKG / ("_Clib" + EXT_SUFFIX)
 
 
-def build_torch_extension(verbose: bool = False) -> Path:
-    """Compiles ``csrc/torchapi.cpp`` into the pybind11 torch extension ``dhellam._Clib`` (the reference builds a
-    module of that name from its csrc/torchapi.cpp, setup.py:234-244).  Host code only: the host compiler with
-    torch's headers, linked against ``libdhellam_hip.so`` (found at run time relative to the extension)."""
-    import sysconfig
+def host_extension_path() -> Path:
+    return PKG / ("_host" + EXT_SUFFIX)
 
+
+def _build_extension(src: Path, out: Path, rpath: str, verbose: bool) -> Path:
+    """Host code only: the host compiler with torch's headers, linked against ``libdhellam_hip.so`` (found at run
+    time relative to the extension)."""
     import torch
     from torch.utils import cpp_extension as E
     if not LIB_PATH.exists():
         raise RuntimeError(f"{LIB_PATH} must be built first")
     rocm = Path(os.environ.get("ROCM_PATH", "/opt/rocm"))
-    out = torch_extension_path()
+    name = out.name.split(".")[0]
     tmp = out.with_suffix(".so.tmp")
     torch_lib = E.library_paths()[0]
     cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-Wno-unused-function",
-           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-DTORCH_EXTENSION_NAME=_Clib", "-DTORCH_API_INCLUDE_EXTENSION_H",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-DTORCH_EXTENSION_NAME={name}", "-DTORCH_API_INCLUDE_EXTENSION_H",
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
            f"-I{ROOT / 'include'}", *[f"-isystem{p}" for p in E.include_paths()], f"-isystem{rocm / 'include'}",
-           f"-I{sysconfig.get_paths()['include']}", str(EXT_SRC), "-o", str(tmp),
+           f"-I{PY_INCLUDE}", str(src), "-o", str(tmp),
            f"-L{torch_lib}", "-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python", "-lamdhip64",
-           f"-L{LIB_DIR}", "-ldhellam_hip", "-Wl,-rpath,$ORIGIN/../dhellam_amd/lib", f"-Wl,-rpath,{torch_lib}"]
+           f"-L{LIB_DIR}", "-ldhellam_hip", f"-Wl,-rpath,{rpath}", f"-Wl,-rpath,{torch_lib}"]
     if verbose:
         print(" ".join(cmd), flush=True)
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
-        raise RuntimeError(f"building dhellam._Clib failed:\n{res.stderr}")
+        raise RuntimeError(f"building {name} failed:\n{res.stderr}")
     if res.stderr.strip() and verbose:
         print(res.stderr, file=sys.stderr)
     os.replace(tmp, out)
     return out
+
+
+def build_torch_extension(verbose: bool = False) -> Path:
+    """Compiles ``csrc/torchapi.cpp`` into the pybind11 torch extension ``dhellam._Clib`` (the reference builds a
+    module of that name from its csrc/torchapi.cpp, setup.py:234-244)."""
+    return _build_extension(CSRC / "torchapi.cpp", torch_extension_path(), "$ORIGIN/../dhellam_amd/lib", verbose)
+
+
+def build_host_extension(verbose: bool = False) -> Path:
+    """Compiles ``csrc/hostapi.cpp`` into ``dhellam_amd._host``, the host path of the Python operators."""
+    return _build_extension(CSRC / "hostapi.cpp", host_extension_path(), "$ORIGIN/lib", verbose)
+
+
+def build_extensions(verbose: bool = False) -> list[Path]:
+    """Both extensions, side by side."""
+    with ThreadPoolExecutor(max_workers=2) as ex:
+        return [f.result() for f in [ex.submit(build_host_extension, verbose), ex.submit(build_torch_extension, verbose)]]
 
 
 if __name__ == "__main__":
@@ -213,4 +232,5 @@ if __name__ == "__main__":
     print(path)
     print(f"grouped GEMM main loops checked: {check_grouped_gemm_loops(verbose='-v' in sys.argv)}")
     if "--no-ext" not in sys.argv:
-        print(build_torch_extension(verbose="-v" in sys.argv))
+        for path in build_extensions(verbose="-v" in sys.argv):
+            print(path)

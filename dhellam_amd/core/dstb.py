@@ -45,10 +45,10 @@ from typing import List, Optional
 
 import torch
 
-from .. import _lib
+from .. import _host, _lib
 from ..common.global_variables import GLOBAL_VARIABLES
 from .._Clib import (WGRAD_TRANSPOSE_GRAD_MIN_K, WGRAD_TRANSPOSE_MIN_ELEMS, keep_transposed, pymha_varlen_bwd,
-                      pymha_varlen_fwd, _attn_bwd_raw)
+                      pymha_varlen_fwd, _attn_bwd_raw, _kernel_head_dim, _zero_rng_state)
 from ..operators.bda import bda_bwd, bda_fwd
 from ..operators.layernorm import pylayernorm_bwd, pylayernorm_fwd
 from ..operators.layernorm_column import dgrad_bwd, gemm_fwd, wgrad_bwd
@@ -258,13 +258,17 @@ class DCFunc:
     @staticmethod
     def attn(config, data, stream, apply_rope=False):
         qkv, cu_seqlens_q, cu_seqlens_kv = data
+        s = config.seq_length
+        if config.groups_per_rank == 1 and not apply_rope and _kernel_head_dim(qkv, config.head_dim) == config.head_dim:
+            q, k, v = _split_qkv(config, qkv)       # views: nothing here runs but the kernel, on ``stream``
+            out, lse = _host.attn_fwd(q, k, v, cu_seqlens_q, cu_seqlens_kv, s, s, config.softmax_scale, True, stream)
+            return out.view(config.tokens, -1), q, k, v, out, _zero_rng_state(q.device), lse
         with torch.cuda.stream(stream):
             q, k, v = _split_qkv(config, qkv)
             if apply_rope and config.rope_theta is not None:
-                rope_fwd(q, k, None, config.rope_theta, config.seq_length, stream, False, inplace=True)
+                rope_fwd(q, k, None, config.rope_theta, s, stream, False, inplace=True)
             out, q_p, k_p, v_p, out_p, lse, _, rng_state = pymha_varlen_fwd(
-                q, k, v, cu_seqlens_q, cu_seqlens_kv, config.seq_length, config.seq_length, 0.0,
-                config.softmax_scale, True, False, 0, False)
+                q, k, v, cu_seqlens_q, cu_seqlens_kv, s, s, 0.0, config.softmax_scale, True, False, 0, False)
             output = out.view(config.tokens, -1)
         return output, q_p, k_p, v_p, out_p, rng_state, lse
 
@@ -403,7 +407,7 @@ class DCFunc:
             else:
                 dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
             _attn_bwd_raw(dout, q, k, v, out, lse, dq, dk, dv, None, cu_seqlens_q, cu_seqlens_kv, config.seq_length,
-                          config.seq_length, config.softmax_scale, True, stream.cuda_stream)
+                          config.seq_length, config.softmax_scale, True, stream)
             if apply_rope and config.rope_theta is not None:
                 rope_bwd(dq, dk, None, config.rope_theta, config.seq_length, stream, False, inplace=True)
             if hk != 1:

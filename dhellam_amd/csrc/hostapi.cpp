@@ -1,0 +1,632 @@
+// pybind11 torch extension `dhellam_amd._host`: the host path of the Python operators (dhellam_amd/operators,
+// dhellam_amd/_Clib.py) in native code.  One call per operator: it checks the tensors, makes the results and the
+// scratch on the stream the operator runs on, and calls the C ABI (include/dhellam_hip.h).
+//
+// What bounds a small operator is the host: with its checks, allocations, stream switches and ctypes call in Python an
+// operator took 20-25 us to issue (seven bandwidth operators on 64 tokens: 178 us of host time for 28 us of kernels).
+// torch.cuda.current_stream() alone is 7 us, entering and leaving torch.cuda.stream() another 5.  From here the same seven
+// take 56 us to issue (8 us each, most of it the kernel launch), and the pass went from 151 to 41 us.
+//
+// Conventions: `stream` is None (torch's current stream) or a torch.cuda.Stream, under which results and scratch are
+// allocated; a failed argument check raises AssertionError where the Python operator asserted and RuntimeError
+// otherwise; the GIL is released around the library call, as ctypes does.
+#include <torch/extension.h>
+#include <c10/hip/HIPCachingAllocator.h>
+#include <c10/hip/HIPGuard.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/Stream.h>
+
+#include <array>
+#include <map>
+#include <mutex>
+#include <optional>
+#include <tuple>
+#include <vector>
+
+#include "dhellam_hip.h"
+
+namespace {
+
+namespace py = pybind11;
+using at::Tensor;
+using OptTensor = std::optional<Tensor>;
+using OptStream = py::object;      // None, a torch.cuda.Stream, or a raw handle
+
+[[noreturn]] void assertion(const char *msg) {
+  PyErr_SetString(PyExc_AssertionError, msg);
+  throw py::error_already_set();
+}
+#define PY_ASSERT(cond, msg) \
+  do {                       \
+    if (!(cond)) assertion(msg); \
+  } while (0)
+
+int dt(const Tensor &t) {
+  switch (t.scalar_type()) {
+    case at::kFloat: return DH_F32;
+    case at::kBFloat16: return DH_BF16;
+    case at::kHalf: return DH_F16;
+    default: TORCH_CHECK(false, "unsupported dtype ", t.scalar_type());
+  }
+}
+
+void need_gpu(std::initializer_list<const Tensor *> ts) {
+  for (const Tensor *t : ts) TORCH_CHECK(t->is_cuda(), "dhellam operators need tensors on the GPU");
+}
+
+// Runs fn() -> status without the GIL and raises its error.
+template <typename F> void launch(F &&fn) {
+  int rc;
+  {
+    py::gil_scoped_release nogil;
+    rc = fn();
+  }
+  TORCH_CHECK(rc == 0, "dhellam_hip error ", rc, ": ", dh_last_error());
+}
+
+// The stream an operator runs on: torch's current one, or the given one made current while this object lives (as
+// `with torch.cuda.stream(s)` does), so that allocations belong to it.
+class On {
+ public:
+  explicit On(const OptStream &s) {
+    if (THPStream_Check(s.ptr())) {
+      const c10::hip::HIPStream want = of(s);
+      if (want != c10::hip::getCurrentHIPStream()) guard_.emplace(want.unwrap());
+      raw_ = want.stream();
+    } else if (s.is_none()) {
+      raw_ = c10::hip::getCurrentHIPStream().stream();
+    } else {      // a handle: launched there, allocations stay with the current stream
+      raw_ = (hipStream_t)s.cast<uint64_t>();
+    }
+  }
+  // The runtime masquerades as CUDA in Python and is HIP in c10: same stream, other device type.
+  static c10::hip::HIPStream of(const OptStream &s) {
+    auto *t = (THPStream *)s.ptr();
+    return c10::hip::HIPStream(c10::Stream::unpack3(t->stream_id, (c10::DeviceIndex)t->device_index, c10::DeviceType::HIP));
+  }
+  void *get() const { return raw_; }
+
+ private:
+  std::optional<c10::hip::HIPStreamGuard> guard_;
+  hipStream_t raw_;
+};
+
+const void *ptr(const OptTensor &t) { return t.has_value() ? t->data_ptr() : nullptr; }
+void *mptr(const OptTensor &t) { return t.has_value() ? t->data_ptr() : nullptr; }
+
+// Scratch kept per (device, stream) and purpose: kernels on one stream are ordered, so consecutive calls may share it;
+// it grows to the largest call seen.  Never freed at exit: the allocator may be gone by then.
+enum Scratch { kNorm, kGemm, kAttnBwd, kGrouped, kScratchKinds };
+struct Key {
+  int device;
+  void *stream;
+  bool operator<(const Key &o) const { return device != o.device ? device < o.device : stream < o.stream; }
+};
+std::mutex g_scratch_mu;
+std::map<Key, Tensor> &scratch_map(int kind) {
+  static auto *maps = new std::array<std::map<Key, Tensor>, kScratchKinds>();
+  return (*maps)[kind];
+}
+Tensor scratch(Scratch kind, int64_t bytes, const Tensor &like, void *stream) {
+  std::lock_guard<std::mutex> lock(g_scratch_mu);
+  Tensor &t = scratch_map(kind)[Key{like.device().index(), stream}];
+  if (!t.defined() || t.numel() < bytes) t = at::empty({bytes}, like.options().dtype(at::kByte));
+  return t;
+}
+// (device index, stream handle) of the scratch buffers of one kind that exist.
+std::vector<std::pair<int, uint64_t>> scratch_keys(int kind) {
+  std::lock_guard<std::mutex> lock(g_scratch_mu);
+  std::vector<std::pair<int, uint64_t>> r;
+  for (auto &kv : scratch_map(kind)) r.emplace_back(kv.first.device, (uint64_t)kv.first.stream);
+  return r;
+}
+
+uint64_t stream_ptr(const OptStream &s) {
+  if (THPStream_Check(s.ptr())) return (uint64_t)On::of(s).stream();
+  return (uint64_t)c10::hip::getCurrentHIPStream().stream();
+}
+
+// ---- norm ---------------------------------------------------------------------------------------------------------
+// -> (ln_out like inp, mu or None, rsigma, sum or None)
+std::tuple<Tensor, OptTensor, Tensor, OptTensor> norm_fwd(const Tensor &inp, const Tensor &weight, const OptTensor &bias,
+                                                          double eps, bool zero_centered, const OptTensor &residual,
+                                                          OptTensor sum_out, const OptTensor &ln_out,
+                                                          const OptStream &stream) {
+  PY_ASSERT(inp.is_cuda(), "dhellam needs a GPU.");
+  const int64_t cols = weight.numel();
+  PY_ASSERT(inp.dim() > 0 && inp.size(-1) == cols, "LayerNorm not possible");
+  PY_ASSERT(inp.is_contiguous() && weight.is_contiguous(), "norm: input and weight must be contiguous");
+  const int64_t rows = cols ? inp.numel() / cols : 0;
+  const int type = dt(inp);
+  On on(stream);
+  Tensor y;
+  if (ln_out.has_value()) {
+    PY_ASSERT(ln_out->is_contiguous() && ln_out->numel() == inp.numel() && ln_out->scalar_type() == inp.scalar_type(),
+              "norm: ln_out must be contiguous, of the input's size and type");
+    y = ln_out->view(inp.sizes());
+  } else {
+    y = at::empty(inp.sizes(), inp.options());
+  }
+  const auto f32 = inp.options().dtype(at::kFloat);
+  Tensor rsigma = at::empty({rows}, f32);
+  OptTensor mu;
+  if (bias.has_value()) mu = at::empty({rows}, f32);
+  if (!residual.has_value()) {
+    launch([&] {
+      return dh_norm_fwd(inp.data_ptr(), weight.data_ptr(), ptr(bias), y.data_ptr(), (float *)mptr(mu),
+                         rsigma.data_ptr<float>(), rows, cols, (float)eps, zero_centered, type, on.get());
+    });
+    return {y, mu, rsigma, std::nullopt};
+  }
+  PY_ASSERT(residual->is_contiguous() && residual->numel() == inp.numel() && residual->scalar_type() == inp.scalar_type(),
+            "norm: residual must be contiguous, of the input's size and type");
+  if (!sum_out.has_value()) sum_out = at::empty(residual->sizes(), residual->options());
+  PY_ASSERT(sum_out->is_contiguous() && sum_out->numel() == inp.numel() && sum_out->scalar_type() == inp.scalar_type(),
+            "norm: sum_out must be contiguous, of the input's size and type");
+  launch([&] {
+    return dh_add_norm_fwd(inp.data_ptr(), residual->data_ptr(), sum_out->data_ptr(), weight.data_ptr(), ptr(bias),
+                           y.data_ptr(), (float *)mptr(mu), rsigma.data_ptr<float>(), rows, cols, (float)eps,
+                           zero_centered, type, on.get());
+  });
+  return {y, mu, rsigma, sum_out};
+}
+
+// -> (dinp like inp, dgamma, dbeta or None)
+std::tuple<Tensor, Tensor, OptTensor> norm_bwd(const Tensor &dy, const Tensor &inp, const OptTensor &mu,
+                                               const Tensor &rsigma, const Tensor &weight, bool zero_centered,
+                                               const OptTensor &add, const OptTensor &dgamma_out,
+                                               const OptTensor &dbeta_out, const OptTensor &dgrad_out,
+                                               const OptStream &stream) {
+  PY_ASSERT(inp.is_cuda(), "dhellam needs a GPU.");
+  const int64_t cols = weight.numel();
+  PY_ASSERT(inp.dim() > 0 && inp.size(-1) == cols, "LayerNorm not possible");
+  PY_ASSERT(inp.is_contiguous() && dy.is_contiguous() && dy.numel() == inp.numel(),
+            "norm: input and gradient must be contiguous and of one size");
+  const int64_t rows = cols ? inp.numel() / cols : 0;
+  const int type = dt(inp);
+  PY_ASSERT(!add.has_value() || (add->is_contiguous() && add->numel() == inp.numel()),
+            "norm: add_to_dgrad must be contiguous, of the input's size");
+  On on(stream);
+  Tensor dx;
+  if (dgrad_out.has_value()) {
+    PY_ASSERT(dgrad_out->is_contiguous() && dgrad_out->numel() == inp.numel() &&
+                  dgrad_out->scalar_type() == inp.scalar_type(),
+              "norm: dgrad_out must be contiguous, of the input's size and type");
+    dx = dgrad_out->view(inp.sizes());
+  } else {
+    dx = at::empty(inp.sizes(), inp.options());
+  }
+  const bool accumulate = dgamma_out.has_value();
+  PY_ASSERT(!accumulate || dgamma_out->scalar_type() == weight.scalar_type(), "dgamma_out must have the weight's dtype");
+  PY_ASSERT(!dbeta_out.has_value() || dbeta_out->scalar_type() == weight.scalar_type(),
+            "dbeta_out must have the weight's dtype");
+  Tensor dgamma = accumulate ? *dgamma_out : at::empty_like(weight);
+  OptTensor dbeta;
+  if (mu.has_value()) {
+    PY_ASSERT(dbeta_out.has_value() == accumulate, "pass both or neither of dgamma_out/dbeta_out");
+    dbeta = dbeta_out.has_value() ? *dbeta_out : at::empty_like(weight);
+  }
+  Tensor ws = scratch(kNorm, (int64_t)dh_norm_bwd_workspace_bytes(rows, cols), inp, on.get());
+  launch([&] {
+    return dh_norm_bwd(dy.data_ptr(), inp.data_ptr(), (const float *)ptr(mu), rsigma.data_ptr<float>(),
+                       weight.data_ptr(), ptr(add), dx.data_ptr(), dgamma.data_ptr(), mptr(dbeta), ws.data_ptr(),
+                       (size_t)ws.numel(), rows, cols, zero_centered, accumulate, type, on.get());
+  });
+  return {dx, dgamma, dbeta};
+}
+
+// ---- SwiGLU, residual add, RoPE -------------------------------------------------------------------------------------
+bool transposable(int64_t rows, int64_t f, std::initializer_list<const Tensor *> ts) {
+  if (!(rows > 0 && f > 0 && rows % 8 == 0 && f % 8 == 0 && rows < 64 * 65535)) return false;
+  const auto type = (*ts.begin())->scalar_type();
+  if (type != at::kBFloat16 && type != at::kHalf) return false;
+  for (const Tensor *t : ts)
+    if (t->scalar_type() != type || (uintptr_t)t->data_ptr() % 16 != 0) return false;
+  return true;
+}
+
+// -> (out, its transpose or None)
+std::tuple<Tensor, OptTensor> swiglu_fwd(const Tensor &y, bool with_transposed, const OptStream &stream) {
+  PY_ASSERT(y.is_cuda() && y.is_contiguous() && y.dim() > 0 && y.size(-1) % 2 == 0,
+            "swiglu: input must be a contiguous GPU tensor with an even last dimension");
+  const int64_t f = y.size(-1) / 2, rows = f ? y.numel() / (2 * f) : 0;
+  const int type = dt(y);
+  On on(stream);
+  auto sizes = y.sizes().vec();
+  sizes.back() = f;
+  Tensor out = at::empty(sizes, y.options());
+  OptTensor ot;
+  if (with_transposed && transposable(rows, f, {&y, &out})) {
+    ot = at::empty({f, rows}, y.options());
+    launch([&] { return dh_swiglu_fwd_t(y.data_ptr(), out.data_ptr(), ot->data_ptr(), rows, f, type, on.get()); });
+  } else {
+    launch([&] { return dh_swiglu_fwd(y.data_ptr(), out.data_ptr(), rows, f, type, on.get()); });
+  }
+  return {out, ot};
+}
+
+// -> (dy, its transpose or None)
+std::tuple<Tensor, OptTensor> swiglu_bwd(const Tensor &g, const Tensor &y, const OptTensor &o, bool with_transposed,
+                                         const OptStream &stream) {
+  PY_ASSERT(y.is_cuda() && y.is_contiguous() && g.is_contiguous() && y.dim() > 0 && y.size(-1) % 2 == 0,
+            "swiglu: inputs must be contiguous GPU tensors with an even last dimension");
+  const int64_t f = y.size(-1) / 2, rows = f ? y.numel() / (2 * f) : 0;
+  PY_ASSERT(g.numel() == rows * f, "grad shape does not match swiglu input");
+  const int type = dt(y);
+  On on(stream);
+  Tensor out = o.has_value() ? *o : at::empty(y.sizes(), y.options());
+  PY_ASSERT(out.is_contiguous() && out.sizes() == y.sizes(), "swiglu: o must be contiguous, of the input's shape");
+  OptTensor ot;
+  if (with_transposed && transposable(rows, f, {&y, &g, &out})) {
+    ot = at::empty({2 * f, rows}, y.options());
+    launch([&] {
+      return dh_swiglu_bwd_t(g.data_ptr(), y.data_ptr(), out.data_ptr(), ot->data_ptr(), rows, f, type, on.get());
+    });
+  } else {
+    launch([&] { return dh_swiglu_bwd(g.data_ptr(), y.data_ptr(), out.data_ptr(), rows, f, type, on.get()); });
+  }
+  return {out, ot};
+}
+
+Tensor residual_add(const Tensor &x, const Tensor &residual, const OptTensor &out, const OptStream &stream) {
+  PY_ASSERT(x.is_cuda() && x.is_contiguous() && residual.is_contiguous(), "bda: tensors must be contiguous on the GPU");
+  PY_ASSERT(x.numel() == residual.numel() && x.scalar_type() == residual.scalar_type(), "bda: sizes or types differ");
+  const Tensor &dst = out.has_value() ? *out : x;
+  PY_ASSERT(dst.is_contiguous() && dst.numel() == x.numel() && dst.scalar_type() == x.scalar_type(),
+            "bda: out must be contiguous, of the input's size and type");
+  const int type = dt(x);
+  On on(stream);
+  launch([&] { return dh_residual_add(x.data_ptr(), residual.data_ptr(), dst.data_ptr(), x.numel(), type, on.get()); });
+  return dst;
+}
+
+int64_t head_rows_stride(const Tensor &t) {
+  PY_ASSERT(t.dim() == 3 && t.stride(2) == 1 && t.stride(1) == t.size(2), "expected [tokens, heads, d] with contiguous heads");
+  return t.stride(0);
+}
+
+std::tuple<Tensor, OptTensor> rope(const Tensor &q, const OptTensor &k, const Tensor &inv_freq, const OptTensor &positions,
+                                   int64_t seq_len, bool backward, bool inplace, const OptStream &stream) {
+  PY_ASSERT(q.is_cuda(), "rope: tensors must be on the GPU");
+  const int64_t qs = head_rows_stride(q), d = q.size(2);
+  PY_ASSERT(!positions.has_value() || (positions->scalar_type() == at::kInt && positions->numel() == q.size(0)),
+            "rope: positions must be int32, one per token");
+  int64_t ks = 0;
+  if (k.has_value()) {
+    ks = head_rows_stride(*k);
+    PY_ASSERT(k->size(0) == q.size(0) && k->size(2) == d && k->scalar_type() == q.scalar_type(), "rope: q and k differ");
+  }
+  const int type = dt(q);
+  On on(stream);
+  Tensor qo = inplace ? q : at::empty(q.sizes(), q.options());
+  OptTensor ko;
+  if (k.has_value()) ko = inplace ? *k : at::empty(k->sizes(), k->options());
+  launch([&] {
+    return dh_rope(q.data_ptr(), ptr(k), qo.data_ptr(), mptr(ko), inv_freq.data_ptr<float>(),
+                   (const int32_t *)ptr(positions), q.size(0), (int)q.size(1), k.has_value() ? (int)k->size(1) : 0, (int)d,
+                   qs, ks, head_rows_stride(qo), ko.has_value() ? head_rows_stride(*ko) : 0, seq_len, backward, type, on.get());
+  });
+  return {qo, ko};
+}
+
+// ---- dense GEMM, transpose ------------------------------------------------------------------------------------------
+constexpr int64_t kGemmWorkspace = 32 << 20;
+
+bool dense_ok(std::initializer_list<const Tensor *> ts) {
+  for (const Tensor *t : ts)
+    if (!(t->is_cuda() && t->dim() == 2 && t->is_contiguous())) return false;
+  return true;
+}
+
+void gemm_on(const Tensor &A, const Tensor &B, const Tensor &D, bool transa, bool transb, bool accumulate,
+             const OptTensor &workspace, int64_t workspace_bytes, void *st) {
+  TORCH_CHECK(dense_ok({&A, &B, &D}), "dense_gemm: operands must be contiguous 2-D GPU tensors");
+  TORCH_CHECK(A.scalar_type() == B.scalar_type() && (D.scalar_type() == A.scalar_type() || D.scalar_type() == at::kFloat),
+              "dense_gemm: operand types ", A.scalar_type(), ", ", B.scalar_type(), " -> ", D.scalar_type(), " not supported");
+  const int64_t m = transa ? A.size(0) : A.size(1), n = transb ? B.size(1) : B.size(0);
+  TORCH_CHECK(D.size(0) == n && D.size(1) == m, "dense_gemm: output is ", D.sizes(), ", the product is [", n, ", ", m, "]");
+  Tensor ws;
+  if (!workspace.has_value() || !workspace->is_cuda() || workspace_bytes <= 0) {
+    ws = scratch(kGemm, kGemmWorkspace, A, st);
+    workspace_bytes = ws.numel();
+  } else {
+    TORCH_CHECK((int64_t)workspace->nbytes() >= workspace_bytes, "dense_gemm: workspace tensor smaller than workspaceSize");
+    ws = *workspace;
+  }
+  if ((transa ? A.size(1) : A.size(0)) == 0) {
+    if (!accumulate) D.zero_();
+    return;
+  }
+  const int type = dt(A), out_type = dt(D);
+  launch([&] {
+    if (transa && transb)      // refused by dh_gemm as by the reference's cublas_gemm; the library's own entry for it
+      return dh_gemm_tt(A.data_ptr(), B.data_ptr(), D.data_ptr(), A.size(0), A.size(1), B.size(0), B.size(1), accumulate,
+                        type, out_type, ws.data_ptr(), (size_t)workspace_bytes, st);
+    return dh_gemm(A.data_ptr(), B.data_ptr(), D.data_ptr(), A.size(0), A.size(1), B.size(0), B.size(1), transa, transb,
+                   accumulate, type, out_type, ws.data_ptr(), (size_t)workspace_bytes, st);
+  });
+}
+
+void dense_gemm(const Tensor &A, const Tensor &B, const Tensor &D, bool transa, bool transb, bool accumulate,
+                const OptTensor &workspace, int64_t workspace_bytes, const OptStream &stream) {
+  On on(stream);
+  gemm_on(A, B, D, transa, transb, accumulate, workspace, workspace_bytes, on.get());
+}
+
+// input [..., K] @ weight [N, K]^T in `output` (made here if not given); None where dh_gemm does not take the operands.
+OptTensor linear(const Tensor &input, const Tensor &weight, OptTensor output, const OptStream &stream) {
+  if (!input.is_contiguous() || !input.is_cuda() || input.dim() < 1 || !dense_ok({&weight}) ||
+      weight.scalar_type() != input.scalar_type() || input.size(-1) != weight.size(1) ||
+      (output.has_value() && !(output->is_contiguous() && output->scalar_type() == input.scalar_type())))
+    return std::nullopt;
+  const int64_t n = weight.size(0), k = weight.size(1), rows = k ? input.numel() / k : 0;
+  if (k == 0) return std::nullopt;
+  On on(stream);
+  if (!output.has_value()) {
+    auto sizes = input.sizes().vec();
+    sizes.back() = n;
+    output = at::empty(sizes, input.options());
+  }
+  gemm_on(weight, input.view({rows, k}), output->view({-1, n}), true, false, false, std::nullopt, 0, on.get());
+  return output;
+}
+
+// B [T, k] @ A^T (transa, A [m, k]) or B @ A (A [k, m]) in `out`, made here if not given
+Tensor matmul(const Tensor &A, const Tensor &B, const OptTensor &out, bool transa, const OptStream &stream) {
+  TORCH_CHECK(A.dim() == 2 && B.dim() == 2, "dense_gemm: operands must be contiguous 2-D GPU tensors");
+  On on(stream);
+  Tensor d = out.has_value() ? *out : at::empty({B.size(0), transa ? A.size(0) : A.size(1)}, B.options());
+  gemm_on(A, B, d, transa, false, false, std::nullopt, 0, on.get());
+  return d;
+}
+
+Tensor transpose_2d(const Tensor &src, const OptTensor &out, const OptStream &stream) {
+  need_gpu({&src});
+  TORCH_CHECK(src.dim() == 2 && src.stride(1) == 1, "transpose_2d: src must be 2-D with unit inner stride");
+  const int64_t rows = src.size(0), cols = src.size(1);
+  const int type = dt(src);
+  On on(stream);
+  Tensor o;
+  if (out.has_value()) {
+    o = *out;
+    TORCH_CHECK(o.dim() == 2 && o.size(0) == cols && o.size(1) == rows && o.stride(1) == 1 && o.scalar_type() == src.scalar_type(),
+                "transpose_2d: out must be [cols, rows] of src's dtype with unit inner stride");
+  } else {
+    o = at::empty({cols, rows}, src.options());
+  }
+  launch([&] {
+    return dh_transpose_2d(src.data_ptr(), o.data_ptr(), rows, cols, src.stride(0), o.stride(0), type, on.get());
+  });
+  return o;
+}
+
+// ---- attention ------------------------------------------------------------------------------------------------------
+int64_t token_stride(const Tensor &t) {
+  TORCH_CHECK(t.dim() == 3 && t.stride(2) == 1 && t.stride(1) == t.size(2),
+              "attention tensors must be [tokens, heads, d] with contiguous (heads, d)");
+  return t.stride(0);
+}
+
+// -> (out, lse)
+std::tuple<Tensor, Tensor> attn_fwd(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &cu_q,
+                                    const Tensor &cu_k, int max_q, int max_k, double scale, bool causal,
+                                    const OptStream &stream) {
+  need_gpu({&q, &k, &v, &cu_q, &cu_k});
+  TORCH_CHECK(cu_q.scalar_type() == at::kInt && cu_k.scalar_type() == at::kInt, "cu_seqlens must be int32");
+  const int64_t qs = token_stride(q), ks = token_stride(k), vs = token_stride(v);
+  const int b = (int)cu_q.numel() - 1, type = dt(q);
+  On on(stream);
+  Tensor out = at::empty(q.sizes(), q.options());
+  Tensor lse = at::empty({b, q.size(1), max_q}, q.options().dtype(at::kFloat));
+  launch([&] {
+    return dh_attn_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr<float>(), cu_q.data_ptr<int>(),
+                       cu_k.data_ptr<int>(), b, max_q, max_k, (int)q.size(1), (int)k.size(1), (int)q.size(2), qs, ks, vs,
+                       token_stride(out), (float)scale, causal, type, on.get());
+  });
+  return {out, lse};
+}
+
+// dq, dk, dv and (optional) delta are the caller's; with accumulate_dq this call's dq is added to what dq holds.
+void attn_bwd(const Tensor &dout, const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &out, const Tensor &lse,
+              const Tensor &dq, const Tensor &dk, const Tensor &dv, const OptTensor &delta, const Tensor &cu_q,
+              const Tensor &cu_k, int max_q, int max_k, double scale, bool causal, bool accumulate_dq,
+              const OptStream &stream) {
+  need_gpu({&dout, &q, &k, &v, &out, &lse});
+  const int b = (int)cu_q.numel() - 1, hq = (int)q.size(1), hk = (int)k.size(1), d = (int)q.size(2), type = dt(q);
+  On on(stream);
+  const size_t bytes = dh_attn_bwd_workspace_bytes(q.size(0), k.size(0), b, max_q, hq, hk, d, type);
+  Tensor ws = scratch(kAttnBwd, (int64_t)bytes, q, on.get());
+  launch([&] {
+    return dh_attn_bwd_acc(dout.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr<float>(),
+                           dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), (float *)mptr(delta), ws.data_ptr(),
+                           (size_t)ws.numel(), cu_q.data_ptr<int>(), cu_k.data_ptr<int>(), b, max_q, max_k, q.size(0),
+                           k.size(0), hq, hk, d, token_stride(q), token_stride(k), token_stride(v), token_stride(out),
+                           token_stride(dout), token_stride(dq), token_stride(dk), token_stride(dv), (float)scale, causal,
+                           accumulate_dq, type, on.get());
+  });
+}
+
+void attn_merge(const std::vector<Tensor> &outs, const std::vector<Tensor> &lses, const std::vector<int> &row_begin,
+                const std::vector<int> &rows, const Tensor &out, const Tensor &lse, const OptStream &stream) {
+  const size_t n = outs.size();
+  PY_ASSERT(lses.size() == n && row_begin.size() == n && rows.size() == n, "merge: one entry per step in every list");
+  PY_ASSERT(lse.dim() == 3 && out.dim() == 3, "merge: out [b*sq, hq, d], lse [b, hq, sq]");
+  const int64_t b = lse.size(0), hq = lse.size(1), sq = lse.size(2), d = out.size(2);
+  std::vector<const void *> po(n);
+  std::vector<const float *> pl(n);
+  for (size_t s = 0; s < n; ++s) {
+    PY_ASSERT(outs[s].is_contiguous() && lses[s].is_contiguous() && lses[s].scalar_type() == at::kFloat,
+              "merge: partial results must be contiguous, lse in fp32");
+    PY_ASSERT(outs[s].sizes() == at::IntArrayRef({b * rows[s], hq, d}) && lses[s].sizes() == at::IntArrayRef({b, hq, (int64_t)rows[s]}),
+              "merge: a partial result has the wrong shape");
+    po[s] = outs[s].data_ptr();
+    pl[s] = lses[s].data_ptr<float>();
+  }
+  PY_ASSERT(out.is_contiguous() && lse.is_contiguous(), "merge: out and lse must be contiguous");
+  const int type = dt(out);
+  On on(stream);
+  launch([&] {
+    return dh_attn_merge(po.data(), pl.data(), row_begin.data(), rows.data(), (int)n, out.data_ptr(), lse.data_ptr<float>(),
+                         (int)b, (int)sq, (int)hq, (int)d, type, on.get());
+  });
+}
+
+// ---- MoE ------------------------------------------------------------------------------------------------------------
+std::tuple<Tensor, Tensor> moe_route(const Tensor &logits, int k, const OptStream &stream) {
+  PY_ASSERT(logits.is_cuda() && logits.scalar_type() == at::kFloat && logits.is_contiguous() && logits.dim() == 2,
+            "route_topk: logits must be a contiguous fp32 [T, E] GPU tensor");
+  const int64_t t = logits.size(0);
+  On on(stream);
+  Tensor idx = at::empty({t, k}, logits.options().dtype(at::kInt)), gates = at::empty({t, k}, logits.options());
+  launch([&] {
+    return dh_moe_route_topk(logits.data_ptr<float>(), idx.data_ptr<int>(), gates.data_ptr<float>(), t, (int)logits.size(1), k,
+                             on.get());
+  });
+  return {idx, gates};
+}
+
+// -> (tokens_per_expert, expert_offsets, sorted_idx, dest_row)
+std::tuple<Tensor, Tensor, Tensor, Tensor> moe_sort(const Tensor &topk_idx, int experts, const OptStream &stream) {
+  PY_ASSERT(topk_idx.is_cuda() && topk_idx.scalar_type() == at::kInt && topk_idx.is_contiguous() && topk_idx.dim() == 2,
+            "sort_assignments: topk_idx must be a contiguous int32 [T, k] GPU tensor");
+  const int64_t n = topk_idx.numel();
+  On on(stream);
+  const auto opt = topk_idx.options();
+  Tensor tpe = at::empty({experts}, opt), offs = at::empty({experts + 1}, opt), order = at::empty({n}, opt), dest = at::empty({n}, opt);
+  Tensor ws = at::empty({(int64_t)dh_moe_sort_workspace_bytes(n, experts)}, opt.dtype(at::kByte));
+  launch([&] {
+    return dh_moe_sort(topk_idx.data_ptr<int>(), tpe.data_ptr<int>(), offs.data_ptr<int>(), order.data_ptr<int>(),
+                       dest.data_ptr<int>(), ws.data_ptr(), (size_t)ws.numel(), n, experts, on.get());
+  });
+  return {tpe, offs, order, dest};
+}
+
+Tensor moe_gather(const Tensor &x, const Tensor &sorted_idx, const OptTensor &row_scale, const Tensor &offs, int e_lo, int e_hi,
+                  int64_t max_rows, int k, const OptStream &stream) {
+  PY_ASSERT(x.is_cuda() && x.is_contiguous() && x.dim() == 2, "permute: rows must be a contiguous 2-D GPU tensor");
+  const int type = dt(x);
+  On on(stream);
+  Tensor out = at::empty({max_rows, x.size(1)}, x.options());      // the kernel zeroes the unused rows
+  launch([&] {
+    return dh_moe_gather_rows(x.data_ptr(), sorted_idx.data_ptr<int>(), (const float *)ptr(row_scale), out.data_ptr(),
+                              offs.data_ptr<int>(), e_lo, e_hi, max_rows, k, x.size(1), type, on.get());
+  });
+  return out;
+}
+
+Tensor moe_scatter(const Tensor &y, const Tensor &dest_row, const OptTensor &gates, const Tensor &offs, int e_lo, int e_hi,
+                   int64_t tokens, int k, const OptStream &stream) {
+  PY_ASSERT(y.is_cuda() && y.is_contiguous() && y.dim() == 2, "unpermute: rows must be a contiguous 2-D GPU tensor");
+  const int type = dt(y);
+  On on(stream);
+  Tensor out = at::empty({tokens, y.size(1)}, y.options());
+  launch([&] {
+    return dh_moe_scatter_rows(y.data_ptr(), dest_row.data_ptr<int>(), (const float *)ptr(gates), out.data_ptr(),
+                               offs.data_ptr<int>(), e_lo, e_hi, tokens, k, y.size(1), type, on.get());
+  });
+  return out;
+}
+
+Tensor moe_gate_grad(const Tensor &dout, const Tensor &y, const Tensor &dest_row, const Tensor &offs, int e_lo, int e_hi,
+                     int64_t tokens, int k, const OptStream &stream) {
+  const int type = dt(dout);
+  On on(stream);
+  Tensor dg = at::empty({tokens, k}, dout.options().dtype(at::kFloat));
+  launch([&] {
+    return dh_moe_gate_grad(dout.data_ptr(), y.data_ptr(), dest_row.data_ptr<int>(), dg.data_ptr<float>(), offs.data_ptr<int>(),
+                            e_lo, e_hi, tokens, k, dout.size(1), type, on.get());
+  });
+  return dg;
+}
+
+// c [R, N] = per group a [R, K] times b [G, N, K]^T (transposed) or b [G, K, N]
+Tensor grouped_gemm(const Tensor &a, const Tensor &b, const Tensor &offs, std::optional<int64_t> max_rows, const OptTensor &out,
+                    bool transposed, const OptStream &stream) {
+  PY_ASSERT(a.dim() == 2 && b.dim() == 3 && a.is_contiguous() && b.is_contiguous(), "grouped_gemm: contiguous a [R, K], b [G, ., .]");
+  const int64_t g = b.size(0), n = b.size(transposed ? 1 : 2), k = b.size(transposed ? 2 : 1), held = a.size(0);
+  PY_ASSERT(a.size(1) == k && offs.numel() == g + 1, "grouped_gemm: shapes differ");
+  const int type = dt(a);
+  On on(stream);
+  // rows past the last group are zeroed by the library; everything else is written
+  Tensor c = out.has_value() ? *out : at::empty({held, n}, a.options());
+  const int64_t rows = max_rows.value_or(held);
+  if (!out.has_value() && rows < held) c.narrow(0, rows, held - rows).zero_();
+  // split-k workspace: products with fewer 256x256 tiles than compute units do not use one
+  void *ws = nullptr;
+  size_t ws_bytes = 0;
+  if (((rows + 255) / 256) * ((n + 255) / 256) >= 256) {
+    Tensor t = scratch(kGrouped, (int64_t)dh_grouped_gemm_workspace_bytes(), a, on.get());
+    ws = t.data_ptr();
+    ws_bytes = (size_t)t.numel();
+  }
+  launch([&] {
+    return (transposed ? dh_grouped_gemm_nt : dh_grouped_gemm_nn)(a.data_ptr(), b.data_ptr(), c.data_ptr(), offs.data_ptr<int>(),
+                                                                  (int)g, rows, n, k, type, ws, ws_bytes, on.get());
+  });
+  return c;
+}
+
+// c [G, M, N] (+)= per group a [R, M]^T b [R, N]
+Tensor grouped_gemm_tn(const Tensor &a, const Tensor &b, const Tensor &offs, const OptTensor &out, bool accumulate,
+                       const OptStream &stream) {
+  PY_ASSERT(a.dim() == 2 && b.dim() == 2 && a.is_contiguous() && b.is_contiguous() && a.size(0) == b.size(0),
+            "grouped_gemm_tn: contiguous a [R, M], b [R, N]");
+  PY_ASSERT(out.has_value() || !accumulate, "grouped_gemm_tn: nothing to accumulate into");
+  const int64_t g = offs.numel() - 1, m = a.size(1), n = b.size(1);
+  const int type = dt(a);
+  On on(stream);
+  Tensor c = out.has_value() ? *out : at::empty({g, m, n}, a.options());
+  launch([&] {
+    return dh_grouped_gemm_tn(a.data_ptr(), b.data_ptr(), c.data_ptr(), offs.data_ptr<int>(), (int)g, a.size(0), m, n, accumulate,
+                              type, on.get());
+  });
+  return c;
+}
+
+// ---- head -----------------------------------------------------------------------------------------------------------
+Tensor embedding_fwd(const Tensor &vocab, const Tensor &ids, int64_t vocab_start) {
+  need_gpu({&vocab, &ids});
+  PY_ASSERT(vocab.dim() == 2 && vocab.is_contiguous() && ids.scalar_type() == at::kLong, "embedding: contiguous table, int64 ids");
+  const Tensor i = ids.contiguous();
+  auto sizes = i.sizes().vec();
+  sizes.push_back(vocab.size(1));
+  const int type = dt(vocab);
+  On on(py::none{});
+  Tensor out = at::empty(sizes, vocab.options());
+  launch([&] {
+    return dh_embedding_fwd(vocab.data_ptr(), i.data_ptr<int64_t>(), i.numel(), vocab.size(1), vocab.size(0), vocab_start, type,
+                            out.data_ptr(), on.get());
+  });
+  return out;
+}
+
+}  // namespace
+
+PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  m.doc() = "host path of the dhellam_amd operators over libdhellam_hip.so";
+  m.attr("SCRATCH_GEMM") = (int)kGemm;
+  m.attr("GEMM_WORKSPACE_BYTES") = kGemmWorkspace;
+  m.def("scratch_keys", &scratch_keys);
+  m.def("stream_ptr", &stream_ptr);
+  m.def("norm_fwd", &norm_fwd);
+  m.def("norm_bwd", &norm_bwd);
+  m.def("swiglu_fwd", &swiglu_fwd);
+  m.def("swiglu_bwd", &swiglu_bwd);
+  m.def("residual_add", &residual_add);
+  m.def("rope", &rope);
+  m.def("dense_gemm", &dense_gemm);
+  m.def("linear", &linear);
+  m.def("matmul", &matmul);
+  m.def("transpose_2d", &transpose_2d);
+  m.def("attn_fwd", &attn_fwd);
+  m.def("attn_bwd", &attn_bwd);
+  m.def("attn_merge", &attn_merge);
+  m.def("moe_route", &moe_route);
+  m.def("moe_sort", &moe_sort);
+  m.def("moe_gather", &moe_gather);
+  m.def("moe_scatter", &moe_scatter);
+  m.def("moe_gate_grad", &moe_gate_grad);
+  m.def("grouped_gemm", &grouped_gemm);
+  m.def("grouped_gemm_tn", &grouped_gemm_tn);
+  m.def("embedding_fwd", &embedding_fwd);
+}

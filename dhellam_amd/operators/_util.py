@@ -13,6 +13,17 @@ import contextlib
 import torch
 
 
+def issue(fn, stream, profiling, *args):
+    """``(fn(*args, stream), elapsed)`` for a function of ``dhellam_amd._host``, which takes the stream (None: the
+    current one) as its last argument: without ``profiling`` nothing but that one native call is made."""
+    if not profiling:
+        return fn(*args, stream), 0
+    el: list = []
+    with on_stream(stream, True, el) as st:
+        res = fn(*args, st)
+    return res, el[0]
+
+
 @contextlib.contextmanager
 def on_stream(stream, profiling: bool, elapsed: list):
     """Run the body on ``stream``; with ``profiling`` bracket it with events and

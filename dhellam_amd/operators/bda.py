@@ -8,8 +8,8 @@ from __future__ import annotations
 
 import torch
 
-from .. import _lib
-from ._util import on_stream
+from .. import _host
+from ._util import issue, on_stream
 
 
 def bda_fwd(input, residual, stream=None, profiling=False, p: float = 0.0, return_mask: bool = False, out=None):
@@ -18,22 +18,19 @@ def bda_fwd(input, residual, stream=None, profiling=False, p: float = 0.0, retur
     tensor)."""
     if p != 0.0:
         raise NotImplementedError("bda_fwd: only p = 0 (no dropout) is implemented")
-    assert input.is_cuda and input.is_contiguous() and residual.is_contiguous()
-    assert input.numel() == residual.numel() and input.dtype == residual.dtype
-    lib = _lib.load()
-    el: list = []
-    with on_stream(stream, profiling, el) as st:
-        dst = input if out is None else out
-        assert dst.is_contiguous() and dst.numel() == input.numel() and dst.dtype == input.dtype
-        _lib.check(lib.dh_residual_add(input.data_ptr(), residual.data_ptr(), dst.data_ptr(), input.numel(),
-                                       _lib.dt(input), st.cuda_stream))
-        mask = torch.ones_like(input, dtype=torch.int8) if return_mask else None
-    return dst, mask, el[0]
+    dst, ms = issue(_host.residual_add, stream, profiling, input, residual, out)
+    mask = None
+    if return_mask:
+        with on_stream(stream, False, []):
+            mask = torch.ones_like(input, dtype=torch.int8)
+    return dst, mask, ms
 
 
 def bda_bwd(dgrad, mask, output=None, stream=None, profiling=False):
     """Returns (dgrad_residual, dgrad_input, ms).  With p = 0 both branches receive
     ``dgrad`` itself; no kernel runs (``mask`` must be None or all ones)."""
+    if output is None and not profiling:
+        return dgrad, dgrad, 0
     el: list = []
     with on_stream(stream, profiling, el):
         if output is not None:

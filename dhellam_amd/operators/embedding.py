@@ -12,7 +12,7 @@ from typing import Sequence
 
 import torch
 
-from .. import _lib
+from .. import _host, _lib
 from ..common.parallel_state import get_tensor_model_parallel_rank, get_tensor_model_parallel_world_size
 
 
@@ -29,14 +29,7 @@ def _vocab_start(vocab) -> int:
 
 def word_embedding_fwd(inputs):
     vocab, token_ids = inputs["vocab"], inputs["token_ids"]
-    _lib.need_cuda(vocab, token_ids)
-    assert vocab.dim() == 2 and vocab.is_contiguous() and token_ids.dtype == torch.int64
-    ids = token_ids.contiguous()
-    out = torch.empty(*ids.shape, vocab.shape[1], dtype=vocab.dtype, device=vocab.device)
-    _lib.check(_lib.load().dh_embedding_fwd(vocab.data_ptr(), ids.data_ptr(), ids.numel(), vocab.shape[1],
-                                            vocab.shape[0], _vocab_start(vocab), _lib.dt(vocab), out.data_ptr(),
-                                            torch.cuda.current_stream().cuda_stream))
-    return {"word_embeddings": out}
+    return {"word_embeddings": _host.embedding_fwd(vocab, token_ids, _vocab_start(vocab))}
 
 
 def word_embedding_bwd(context, dout):
@@ -53,7 +46,7 @@ def word_embedding_bwd(context, dout):
     assert grad.is_contiguous() and grad.shape == vocab.shape
     _lib.check(_lib.load().dh_embedding_bwd(dout.data_ptr(), ids.data_ptr(), ids.numel(), vocab.shape[1],
                                             vocab.shape[0], _vocab_start(vocab), _lib.dt(dout), grad.data_ptr(),
-                                            _lib.dt(grad), torch.cuda.current_stream().cuda_stream))
+                                            _lib.dt(grad), _host.stream_ptr(None)))
     return None
 
 

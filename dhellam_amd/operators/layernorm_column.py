@@ -18,10 +18,11 @@ from typing import Optional
 
 import torch
 
-from .._Clib import _note_read, dense_gemm, dense_ok, dgrad_gemm, transposed_of
+from .. import _host, _lib
+from .._Clib import _note_read, dense_ok, dgrad_gemm, transposed_of
 from .._Clib import pygemm as gemm
 from .._Clib import wgrad_gemm
-from ._util import on_stream
+from ._util import issue, on_stream
 
 
 def gemm_fwd(args, input: torch.Tensor, weight: torch.Tensor, output: Optional[torch.Tensor] = None,
@@ -29,19 +30,18 @@ def gemm_fwd(args, input: torch.Tensor, weight: torch.Tensor, output: Optional[t
              stream=None):
     transa = layout[0] == "T"
     transb = layout[1] == "T"
+    if is_matmul and transa and not transb:
+        if output is not None:
+            _lib.mark_written(output)
+        res, ms = issue(_host.linear, stream, profiling, input, weight, output)
+        if res is not None:
+            return res, ms
     el: list = []
     with on_stream(stream, profiling, el):
         if is_matmul:
-            x2 = input.reshape(-1, input.shape[-1]) if input.is_contiguous() else input
-            if (transa and not transb and dense_ok(weight, x2) and weight.dtype == input.dtype
-                    and (output is None or (output.is_contiguous() and output.dtype == input.dtype))):
-                if output is None:
-                    output = torch.empty(*input.shape[:-1], weight.shape[0], dtype=input.dtype, device=input.device)
-                dense_gemm(weight, x2, output.view(-1, weight.shape[0]), True, False, False)
-            else:
-                w = weight.t() if transa else weight
-                x = input.t() if transb else input
-                output = torch.matmul(x, w) if output is None else torch.matmul(x, w, out=output)
+            w = weight.t() if transa else weight
+            x = input.t() if transb else input
+            output = torch.matmul(x, w) if output is None else torch.matmul(x, w, out=output)
         else:
             if output is None:
                 output = torch.empty(input.shape[1] if transb else input.shape[0],
@@ -63,6 +63,10 @@ def dgrad_bwd(args, input_grad: torch.Tensor, weight: torch.Tensor, dgrad_output
               stream=None):
     transa = layout[0] == "T"
     transb = layout[1] == "T"
+    if (is_matmul and not profiling and not transa and not transb and dense_ok(weight, input_grad)
+            and weight.dtype == input_grad.dtype
+            and (dgrad_output is None or (dense_ok(dgrad_output) and dgrad_output.dtype == weight.dtype))):
+        return dgrad_gemm(input_grad, weight, dgrad_output, stream), 0
     el: list = []
     with on_stream(stream, profiling, el):
         if dgrad_output is None:
@@ -94,6 +98,11 @@ def wgrad_bwd(args, input_grad: torch.Tensor, input_data: torch.Tensor, wgrad_ou
     (layernorm_column.py:289-292) a given ``wgrad_output`` is ACCUMULATED into."""
     transa = layout[0] == "T"
     transb = layout[1] == "T"
+    if (is_matmul and not profiling and wgrad_output is not None and transb and not transa
+            and dense_ok(input_grad, input_data, wgrad_output) and input_grad.dtype == input_data.dtype
+            and wgrad_output.dtype in (input_grad.dtype, torch.float32)):
+        wgrad_gemm(input_grad, input_data, wgrad_output, True, stream=stream)
+        return wgrad_output, 0
     el: list = []
     with on_stream(stream, profiling, el):
         if is_matmul:

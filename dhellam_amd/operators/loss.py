@@ -23,7 +23,7 @@ from __future__ import annotations
 
 import torch
 
-from .. import _lib
+from .. import _host, _lib
 from ..common.parallel_state import get_tensor_model_parallel_rank, get_tensor_model_parallel_world_size
 from .embedding import vocab_range_from_per_partition_vocab_size
 
@@ -49,7 +49,7 @@ def cross_entropy_fwd(inputs, label_smoothing=0.0, keep_softmax=True):
         x.data_ptr(), tgt.data_ptr(), rows, cols, x.stride(0), start, float(label_smoothing), _lib.dt(x),
         stats[0].data_ptr(), stats[1].data_ptr(), stats[2].data_ptr(), stats[3].data_ptr(),
         softmax.data_ptr() if keep_softmax else None, cols, mask.data_ptr(), masked_target.data_ptr(),
-        torch.cuda.current_stream().cuda_stream))
+        _host.stream_ptr(None)))
     return {
         "loss": stats[0, :rows].view(target.shape),
         "label_smoothing": label_smoothing,
@@ -74,7 +74,7 @@ def cross_entropy_bwd(context, dout, grad_out=None):
     tgt = target.contiguous()
     rows = tgt.numel()
     assert d.numel() == rows
-    lib, st = _lib.load(), torch.cuda.current_stream().cuda_stream
+    lib, st = _lib.load(), _host.stream_ptr(None)
     if out["softmax"] is not None:
         sm = out["softmax"]
         s2 = sm.view(-1, cols)
@@ -104,7 +104,7 @@ def mask_scale_loss_fwd(inputs):
     scale = float(inputs["loss_scale"]) / float(inputs["num_microbatch"])
     out = torch.empty(2, dtype=torch.float32, device=x.device)
     _lib.check(_lib.load().dh_masked_mean_fwd(x.data_ptr(), m.data_ptr(), x.numel(), scale, out.data_ptr(),
-                                              torch.cuda.current_stream().cuda_stream))
+                                              _host.stream_ptr(None)))
     return {"loss": out[0], "mask_sum": out[1:2], "mask_f32": m}
 
 
@@ -115,5 +115,5 @@ def mask_scale_loss_bwd(context, dout=None):
     scale = float(inputs["loss_scale"]) / float(inputs["num_microbatch"])
     g = torch.empty(m.numel(), dtype=torch.float32, device=m.device)
     _lib.check(_lib.load().dh_masked_mean_bwd(m.data_ptr(), out["mask_sum"].data_ptr(), m.numel(), scale, g.data_ptr(),
-                                              torch.cuda.current_stream().cuda_stream))
+                                              _host.stream_ptr(None)))
     return g.view(losses.shape).to(losses.dtype)

@@ -160,7 +160,6 @@ def fa_cp_block_bwd(dout, out, q, dq, kv, dkv_, softmax_lse, rng_states, cu_seql
     hq, d = q.shape[-2], q.shape[-1]
     step = cp_size - 1 - i
     kv_in = p2p_comm_buffers[step]
-    sp = stream.cuda_stream
 
     with torch.cuda.stream(stream):
         if dkv_ is None:
@@ -221,11 +220,11 @@ def fa_cp_block_bwd(dout, out, q, dq, kv, dkv_, softmax_lse, rng_states, cu_seql
             dq[:, 0].zero_()
         if dq_rows.is_contiguous() or dq_rows.shape[0] == 1:
             tgt = dq_rows.reshape(-1, hq, d) if dq_rows.is_contiguous() else dq_rows[0]
-            _Clib._attn_bwd_raw(do_, q_, k_, v_, o_, lse_, tgt, dk_, dv_, None, cq, ck, mq, mk, scale, cz, sp,
+            _Clib._attn_bwd_raw(do_, q_, k_, v_, o_, lse_, tgt, dk_, dv_, None, cq, ck, mq, mk, scale, cz, stream,
                                 accumulate_dq=not first_store)
         else:
             dq_step = torch.empty(q_.shape, dtype=q.dtype, device=q.device)
-            _Clib._attn_bwd_raw(do_, q_, k_, v_, o_, lse_, dq_step, dk_, dv_, None, cq, ck, mq, mk, scale, cz, sp)
+            _Clib._attn_bwd_raw(do_, q_, k_, v_, o_, lse_, dq_step, dk_, dv_, None, cq, ck, mq, mk, scale, cz, stream)
             dq_step = dq_step.view(dq_rows.shape)
             if first_store:
                 dq_rows.copy_(dq_step)
