@@ -356,3 +356,13 @@ def test_attention_head_dim_above_256_is_refused():
     cu = _cu([8]).cuda()
     with pytest.raises(RuntimeError, match="256"):
         _Clib.pymha_varlen_fwd(q, q, q, cu, cu, 8, 8, 0.0, 1.0, True, False, 0, False)
+
+
+@pytest.mark.parametrize("lens_q,lens_k,hq,hk,d,causal", [
+    ([32, 1, 129], [32, 1, 129], 2, 1, 64, True),        # tile edges, one row, more tiles than wavefronts
+    ([33], [160], 4, 2, 64, False), ([161, 31], [31, 64], 2, 2, 60, False),
+    ([97], [97], 4, 1, 128, True), ([40], [300], 2, 2, 124, False), ([5], [5], 1, 1, 4, True),
+])
+def test_attention_f32_matrix_core_kernels(lens_q, lens_k, hq, hk, d, causal):
+    """fp32 kernels for head dims up to 128: tile edges of both sequences, full and partial column tiles, GQA."""
+    _run_fwd_bwd(torch.float32, lens_q, lens_k, hq, hk, d, causal)
