@@ -2,10 +2,10 @@
 // floating-point atomics).
 //
 // Three kernels:
-//   delta   : delta_i = sum_d dO[i,d] * O[i,d]                      (streaming; head dim 64 only: the
-//             head dim 128 dQ kernel forms delta in its prologue and runs first)
+//   delta   : delta_i = sum_d dO[i,d] * O[i,d]                      (streaming; the dQ kernels of head
+//             dims 64 and 128 form delta in their prologue and run first)
 //   dK/dV   : a workgroup owns 64 key/value rows (K, V fragments stay in
-//             registers for head dim 64, in LDS for head dim 128), walks the
+//             registers, for head dim 128 in LDS), walks the
 //             query heads of its GQA group and the query tiles that attend to
 //             it; S = Q K^T and dP = dO V^T are computed
 //             with the key index on lanes so that P and dS feed dV^T += dO^T P
@@ -113,7 +113,7 @@ __global__ void __launch_bounds__(64 * NW) attn_bwd_dkv_kernel(const AttnBwdPara
   float *sLse = reinterpret_cast<float *>(sdO + 2 * BM * QS);  // [2][BM]  (lse * log2e, +inf for rows >= sq)
   float *sDel = sLse + 2 * BM;                                 // [2][BM]
 
-  const int b = blockIdx.z;
+  const int b = seq_by_length(p.cu_q, gridDim.z, blockIdx.z);
   const int hkv = blockIdx.y / p.hsplit, hs = blockIdx.y % p.hsplit;
   const int q0 = p.cu_q[b], sq = p.cu_q[b + 1] - q0;
   const int k0 = p.cu_k[b], sk = p.cu_k[b + 1] - k0;
@@ -338,7 +338,7 @@ __global__ void __launch_bounds__(64 * NW) attn_bwd_dq_kernel(const AttnBwdParam
   T *sK = reinterpret_cast<T *>(smem_raw);  // [2][BN*KS]
   T *sV = sK + 2 * BN * KS;                 // [2][BN*VS]
 
-  const int b = blockIdx.z, h = blockIdx.y;
+  const int b = seq_by_length(p.cu_q, gridDim.z, blockIdx.z), h = blockIdx.y;
   const int mt = gridDim.x - 1 - blockIdx.x;
   const int q0 = p.cu_q[b], sq = p.cu_q[b + 1] - q0;
   const int k0 = p.cu_k[b], sk = p.cu_k[b + 1] - k0;
@@ -503,7 +503,7 @@ __global__ void __launch_bounds__(512) attn_bwd_dq_d128_kernel(const AttnBwdPara
   __shared__ __attribute__((aligned(1024))) T sAll[4 * SLOT];   // K slots 0..1, V slots 0..1
   __shared__ float sDel[RG * 32];                               // delta of the workgroup's rows
 
-  const int b = blockIdx.y;
+  const int b = seq_by_length(p.cu_q, gridDim.y, blockIdx.y);
   // the query heads of one kv head read the same K / V rows: keep a kv head on one XCD's L2
   const int ratio = p.hq / p.hk, P = gridDim.x / p.hq;
   int hkv, item;
@@ -801,7 +801,7 @@ __global__ void __launch_bounds__(512) attn_bwd_dq2_d128_kernel(const AttnBwdPar
   constexpr int NST = 3;                               // stages: the copies of a step go out two steps ahead of it
   __shared__ __attribute__((aligned(1024))) char sAll[NST * SLOTB + NST * DSLOTB];   // 144 KB
 
-  const int b = blockIdx.y;
+  const int b = seq_by_length(p.cu_q, gridDim.y, blockIdx.y);
   // a head's dS blocks were written from one XCD (the dK/dV kernel keeps a head group there): read them from the
   // same one; the K rows of the kv head are small next to them
   const int ratio = p.hq / p.hk, P = gridDim.x / p.hq;
@@ -1050,7 +1050,7 @@ __global__ void __launch_bounds__(512) attn_bwd_dkv_d128_kernel(const AttnBwdPar
   constexpr int KVTB = KVT * (int)sizeof(T);
   __shared__ __attribute__((aligned(1024))) T sAll[2 * STAGE + 2 * KVT];
 
-  const int b = blockIdx.y;
+  const int b = seq_by_length(p.cu_q, gridDim.y, blockIdx.y);
   const int G = p.hk * p.hsplit;
   int hg, px;
   xcd_group_item(blockIdx.x, G, gridDim.x / G, hg, px);
@@ -1403,6 +1403,12 @@ static int launch_dkv_d128(const AttnBwdParams &p, int batch, int max_sk, hipStr
   return DH_OK;
 }
 
+}  // namespace dh
+
+#include "attn_bwd_d64.h"
+
+namespace dh {
+
 // ---- host -------------------------------------------------------------------------------------
 // Query heads of a kv head are split over workgroups (each with fp32 partial dK / dV that a second kernel adds up)
 // only as far as it takes to give every compute unit one workgroup: beyond that the partials cost more than the
@@ -1480,6 +1486,41 @@ static bool dq_big_grid(int batch, int max_sq, int hq, int causal) {
   return (causal ? (t + 1) / 2 : t) * hq * batch >= 256;
 }
 
+// The kernels behind delta of one call.
+template <typename T, int D>
+static int bwd_passes(const AttnBwdParams &p, int batch, int max_sq, int max_sk, hipStream_t st) {
+  const bool small_q = cdiv(max_sq, 128) * p.hq * batch < 2 * 256;
+  int rc = DH_OK;
+  // recomputing dQ kernels that form delta run first
+  if constexpr (D == 64) {
+    if (max_sq > 0) rc = small_q ? launch_dq_d64<T, 2, 4>(p, batch, st) : launch_dq_d64<T, 4, 2>(p, batch, st);
+  }
+  if constexpr (D == 128) {
+    if (max_sq > 0 && !p.ds)
+      rc = dq_big_grid(batch, max_sq, p.hq, p.causal) ? launch_dq_d128<T, 4, 2, 32>(p, batch, st) : launch_dq_d128<T, 2, 4, 32>(p, batch, st);
+  }
+  if (rc == DH_OK && max_sk > 0) {
+    if constexpr (D == 64) rc = launch_dkv_d64<T, 2, 4>(p, batch, max_sk, st);
+    else if constexpr (D == 128) rc = launch_dkv_d128<T>(p, batch, max_sk, st);
+    else rc = launch_dkv<T, D, DKV_NW>(p, batch, max_sk, st);
+  }
+  if (rc == DH_OK && p.hsplit > 1 && p.total_k > 0) {
+    int64_t blocks = cdiv(p.total_k * p.hk * (D / 4), 256);
+    if (blocks > 256 * 16) blocks = 256 * 16;
+    hipLaunchKernelGGL((attn_bwd_gqa_sum_kernel<T>), dim3((unsigned)blocks), dim3(256), 0, st, p.dk_part, p.dv_part, (T *)p.dk,
+                       (T *)p.dv, p.total_k, p.hk, D, p.hsplit, p.dk_stride, p.dv_stride);
+  }
+  if (rc == DH_OK && max_sq > 0) {
+    if constexpr (D == 128) {
+      if (p.ds) rc = launch_dq2_d128<T>(p, batch, st);
+    } else if constexpr (D != 64) {
+      if (small_q || !dq_takes_4_waves(D)) rc = launch_dq<T, D, 2>(p, batch, st);
+      else rc = launch_dq<T, D, dq_takes_4_waves(D) ? 4 : 2>(p, batch, st);
+    }
+  }
+  return rc;
+}
+
 // Bytes of the dS blocks for these sizes (key count as an upper bound of the longest sequence); 0 for calls that
 // never keep dS, whatever space there is (other head dims, fp32, a chip-filling recomputing kernel).
 static size_t ds_bytes_wanted(int batch, int max_sq, int64_t max_sk, int hq, int d, int dtype, int causal) {
@@ -1501,7 +1542,7 @@ static size_t ds_bytes(int batch, int max_sq, int64_t max_sk, int hq, int d, int
 static size_t bwd_base_bytes(int64_t total_k, int batch, int max_seqlen_q, int hq, int hk, int d, int dtype) {
   const size_t sq = (size_t)(max_seqlen_q > 0 ? max_seqlen_q : 0);
   size_t n = align256((size_t)batch * hq * sq * sizeof(float));            // delta
-  if (dtype != DH_F32 && d == 128) n += 2 * align256((size_t)batch * hq * ((sq + 31) / 32 * 32) * sizeof(float));
+  if (dtype != DH_F32 && (d == 128 || d == 64)) n += 2 * align256((size_t)batch * hq * ((sq + 31) / 32 * 32) * sizeof(float));
   if (dtype != DH_F32 && hk > 0 && hq / hk > 1)
     n += 2 * align256((size_t)(hq / hk) * (size_t)total_k * hk * d * sizeof(float));
   return n + 256;                                                          // the base pointer is rounded up to 256
@@ -1553,7 +1594,7 @@ static int attn_bwd_entry(const void *dout, const void *q, const void *k, const 
   float *ld2 = nullptr;
   const int ld2_pitch = (max_seqlen_q + 31) / 32 * 32;
   const size_t plane2 = align256((size_t)batch * hq * (size_t)ld2_pitch * sizeof(float));
-  if (dtype != DH_F32 && d == 128) {
+  if (dtype != DH_F32 && (d == 128 || d == 64)) {
     ld2 = (float *)ws;
     ws += 2 * plane2;
     DH_CHECK(plane2 < (1ull << 31), "batch * heads * max_seqlen_q too large");
@@ -1572,7 +1613,7 @@ static int attn_bwd_entry(const void *dout, const void *q, const void *k, const 
   if (dsb > 0 && base_bytes + align256(dsb) > workspace_bytes) dsb = 0;
   const bool keep_ds = dsb > 0 && max_seqlen_k > 0;
   uint8_t *ds_ws = (uint8_t *)(((uintptr_t)workspace + 255) & ~(uintptr_t)255) + (base_bytes - 256);
-  const bool delta_in_dq = dtype != DH_F32 && d == 128 && !keep_ds;
+  const bool delta_in_dq = dtype != DH_F32 && (d == 64 || (d == 128 && !keep_ds));
   if (max_seqlen_q > 0 && !delta_in_dq) {
     DH_DISPATCH_DTYPE(dtype, {
       launch_delta<T>(dout, out, delta, lse, ld2, (int64_t)(plane2 / sizeof(float)), ld2_pitch, cu_seqlens_q, batch, max_seqlen_q, hq, d,
@@ -1617,36 +1658,20 @@ static int attn_bwd_entry(const void *dout, const void *q, const void *k, const 
     p.dk_part = (float *)ws;
     p.dv_part = (float *)(ws + part);
   }
-  const bool small_q = cdiv(max_seqlen_q, 128) * hq * batch < 2 * 256;
-  const bool big_q = dq_big_grid(batch, max_seqlen_q, hq, causal);
   DH_CHECK(k_stride < (1ll << 31) && v_stride < (1ll << 31) && q_stride < (1ll << 31) && do_stride < (1ll << 31),
            "token stride too large");
   int rc = DH_OK;
-#define DH_BWD(TT, DD)                                                                         \
-  do {                                                                                         \
-    if (DD == 128 && max_seqlen_q > 0 && !keep_ds)                                             \
-      rc = big_q ? launch_dq_d128<TT, 4, 2, 32>(p, batch, st) : launch_dq_d128<TT, 2, 4, 32>(p, batch, st); \
-    if (rc == DH_OK && max_seqlen_k > 0)                                                       \
-      rc = DD == 128 ? launch_dkv_d128<TT>(p, batch, max_seqlen_k, st) : launch_dkv<TT, DD, DKV_NW>(p, batch, max_seqlen_k, st); \
-    if (rc == DH_OK && p.hsplit > 1 && total_k > 0) {                                          \
-      int64_t blocks = cdiv(total_k * hk * (DD / 4), 256);                                     \
-      if (blocks > 256 * 16) blocks = 256 * 16;                                                \
-      hipLaunchKernelGGL((attn_bwd_gqa_sum_kernel<TT>), dim3((unsigned)blocks), dim3(256), 0, st, p.dk_part, \
-                         p.dv_part, (TT *)dk, (TT *)dv, total_k, hk, DD, p.hsplit, dk_stride, dv_stride);    \
-    }                                                                                          \
-    if (rc == DH_OK && max_seqlen_q > 0 && DD != 128)                                          \
-      rc = (small_q || !dq_takes_4_waves(DD)) ? launch_dq<TT, DD, 2>(p, batch, st)             \
-                                              : launch_dq<TT, DD, dq_takes_4_waves(DD) ? 4 : 2>(p, batch, st); \
-    if (rc == DH_OK && max_seqlen_q > 0 && DD == 128 && keep_ds) rc = launch_dq2_d128<TT>(p, batch, st); \
-  } while (0)
 #define DH_BWD_D(TT)                                                                            \
   do {                                                                                          \
-    if (d == 128) DH_BWD(TT, 128); else if (d == 64) DH_BWD(TT, 64); else if (d == 96) DH_BWD(TT, 96); \
-    else if (d == 192) DH_BWD(TT, 192); else DH_BWD(TT, 256);                                   \
+    const auto run = d == 64    ? bwd_passes<TT, 64>                                            \
+                     : d == 96  ? bwd_passes<TT, 96>                                            \
+                     : d == 128 ? bwd_passes<TT, 128>                                           \
+                     : d == 192 ? bwd_passes<TT, 192>                                           \
+                                : bwd_passes<TT, 256>;                                          \
+    rc = run(p, batch, max_seqlen_q, max_seqlen_k, st);                                         \
   } while (0)
   if (dtype == DH_BF16) DH_BWD_D(bf16_t); else DH_BWD_D(f16_t);
 #undef DH_BWD_D
-#undef DH_BWD
   if (rc != DH_OK) return rc;
   DH_LAUNCH_CHECK();
   return DH_OK;

@@ -1,0 +1,409 @@
+// Head dim 64 backward (16 bits), two passes as at the other head dims: dQ (which forms delta = rowsum(dO O) and runs
+// first) and dK/dV.  Tile layout and copies: attn_d64.h; workgroup shape and what bounds it: as the forward kernel of this
+// head dim (attn_fwd_d64.h).
+// dK/dV keeps K and V fragments and both accumulators in registers (202): two wavefronts a SIMD.
+// Measured against the register-staged kernels: 2 x 512 rows, 16 heads, delta + dQ 28.6 -> 11.5 us, dK/dV 31.3 -> 13.9 us;
+// larger shapes in attn_fwd_d64.h.
+#include "attn_d64.h"
+
+namespace dh {
+
+// dQ: RG row groups of 32 query rows x SPLIT splits of the keys, 32-key tiles of K and V.
+template <typename T, int RG, int SPLIT>
+__global__ void __launch_bounds__(512, RG == 4 ? 4 : 2) attn_bwd_dq_d64_kernel(const AttnBwdParams p) {
+  using M = Mma<T>;
+  using Frag = typename M::Frag;
+  static_assert(RG * SPLIT == 8, "8 wavefronts per workgroup");
+  constexpr int D = 64, BM = 32 * RG, BN = 32;
+  constexpr int TILEB = BN * D * (int)sizeof(T);
+  constexpr int STAGEB = SPLIT * 2 * TILEB;
+  constexpr int CB = SPLIT * 2 * (BN / 8) / 8;            // copy blocks per wavefront and iteration: 4 or 2
+  constexpr int EXB = (SPLIT - 1) * RG * 8192;
+  constexpr int LDSB = 2 * STAGEB > EXB ? 2 * STAGEB : EXB;
+  __shared__ __attribute__((aligned(1024))) char sAll[LDSB];
+  __shared__ float sDel[32 * RG];
+
+  const int b = seq_by_length(p.cu_q, gridDim.y, blockIdx.y);
+  const int ratio = p.hq / p.hk, P = gridDim.x / p.hq;
+  int hkv, item;
+  xcd_group_item(blockIdx.x, p.hk, ratio * P, hkv, item);
+  const int h = hkv * ratio + item % ratio, px = item / ratio;
+  const int q0 = p.cu_q[b], sq = p.cu_q[b + 1] - q0;
+  const int k0 = p.cu_k[b], sk = p.cu_k[b + 1] - k0;
+  const int nqt = (sq + BM - 1) / BM;
+  if (px >= nqt) return;
+  const int m0 = (nqt - 1 - px) * BM;          // late causal tiles carry the most work and come first
+  const int causal = p.causal;
+  const float scale_log2 = p.scale_log2;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 31, hh = lane >> 5;
+  const int rg = w % RG, sp = w / RG;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)sAll;
+
+  // copies of this wavefront: rows cp_r0 .. + 8 CB - 1 of the K or V tile of split cp_sp
+  constexpr int PARTS = BN / (8 * CB);
+  const int cp_r0 = 8 * CB * (w % PARTS), cp_v = (w / PARTS) & 1, cp_sp = w / (2 * PARTS);
+  const int64_t cp_stride = cp_v ? p.v_stride : p.k_stride;
+  const T *cp_g = reinterpret_cast<const T *>(cp_v ? p.v : p.k) + (int64_t)k0 * cp_stride + (int64_t)hkv * D;
+  const Copy64 cl = copy64_lane(lane, (uint32_t)(cp_stride * (int64_t)sizeof(T)));
+  const uint32_t cp_dst = lds0 + (uint32_t)(cp_v * SPLIT * TILEB + cp_sp * TILEB + cp_r0 * D * (int)sizeof(T));
+
+  int nk_end = sk;
+  if (causal && m0 + BM < nk_end) nk_end = m0 + BM;
+  const int ntiles = (nk_end + BN - 1) / BN;
+  const int niter = (ntiles + SPLIT - 1) / SPLIT;
+  auto issue = [&](int it) {
+    const int tile = it * SPLIT + cp_sp;
+    if (tile < ntiles) copy64<T, CB>(cp_g, cp_stride, tile * BN + cp_r0, sk, cp_dst + (uint32_t)((it & 1) * STAGEB), cl);
+  };
+  if (niter > 0) issue(0);
+
+  const int wrow0 = m0 + rg * 32, row_q = wrow0 + c;
+  const bool row_ok = row_q < sq;
+  const int row_ld = row_ok ? row_q : sq - 1;
+  Frag Qf[D / 16], dOf[D / 16];
+  {
+    const T *qp = reinterpret_cast<const T *>(p.q) + (int64_t)(q0 + row_ld) * p.q_stride + (int64_t)h * D + 8 * hh;
+    const T *dp = reinterpret_cast<const T *>(p.dout) + (int64_t)(q0 + row_ld) * p.do_stride + (int64_t)h * D + 8 * hh;
+#pragma unroll
+    for (int ks = 0; ks < D / 16; ++ks) {
+      Qf[ks] = frag_ld<T>(qp + ks * 16);
+      dOf[ks] = frag_ld<T>(dp + ks * 16);
+    }
+  }
+  const int64_t stat = ((int64_t)b * p.hq + h) * p.max_sq + row_q;
+  const float lse_c = row_ok ? p.lse[stat] * 1.4426950408889634f : INFINITY;        // rows past the end: P = 0
+  float del_c = 0.f;
+  if (sp == 0) {       // delta of the workgroup's rows, for the other splits and for the dK/dV pass
+    const T *op = reinterpret_cast<const T *>(p.out) + (int64_t)(q0 + row_ld) * p.o_stride + (int64_t)h * D + 8 * hh;
+#pragma unroll
+    for (int ks = 0; ks < D / 16; ++ks) {
+      const Frag of = frag_ld<T>(op + ks * 16);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) del_c += to_f(dOf[ks][j]) * to_f(of[j]);
+    }
+    del_c = row_ok ? pair32_sum(del_c) : 0.f;
+    if (hh == 0) {
+      sDel[rg * 32 + c] = del_c;
+      if (row_ok) p.delta[stat] = del_c;
+      if (row_q < p.ld2_pitch) {          // both, side by side, in whole 32-row tiles (padding rows: zeros)
+        const int64_t a2 = ((int64_t)b * p.hq + h) * p.ld2_pitch + row_q;
+        p.ld2[a2] = row_ok ? lse_c : 0.f;
+        p.ld2[p.ld2_plane + a2] = del_c;
+      }
+    }
+  }
+  const uint32_t k_lane = lds0 + (uint32_t)(sp * TILEB) + row64_lane(lane);
+  const uint32_t ta_lane = lds0 + (uint32_t)(sp * TILEB) + tr64_lane(lane);
+
+  floatx16 dQt[D / 32];
+#pragma unroll
+  for (int t = 0; t < D / 32; ++t)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) dQt[t][v] = 0.f;
+  dma_wait_all();
+  __syncthreads();
+  del_c = sDel[rg * 32 + c];
+
+#pragma unroll 1
+  for (int it = 0; it < niter; ++it) {
+    if (it + 1 < niter) issue(it + 1);
+    const int tile = it * SPLIT + sp, n0 = tile * BN;
+    if (tile < ntiles && !(causal && n0 > wrow0 + 31)) {
+      const uint32_t st = (uint32_t)((it & 1) * STAGEB);
+      const uint32_t kb = k_lane + st, ta = ta_lane + st, tb = tr64_next(ta);
+      floatx16 S, dP;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        S[v] = 0.f;
+        dP[v] = 0.f;
+      }
+#pragma unroll
+      for (int ks = 0; ks < D / 16; ++ks) {
+        S = M::mma(row64<T>(kb ^ (uint32_t)(ks << 5)), Qf[ks], S);
+        dP = M::mma(row64<T>((kb ^ (uint32_t)(ks << 5)) + (uint32_t)(SPLIT * TILEB)), dOf[ks], dP);
+      }
+      if ((causal && n0 + BN - 1 > wrow0) || n0 + BN > sk) {
+        const int lim = causal && row_q + 1 < sk ? row_q + 1 : sk;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) S[v] = n0 + acc_row(v, hh) < lim ? S[v] : -INFINITY;        // P = dS = 0
+      }
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        float ds[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) ds[j] = fast_exp2(S[8 * s + j] * scale_log2 - lse_c) * (dP[8 * s + j] - del_c);
+        const Frag dSb = frag_pack<T>(ds);
+#pragma unroll
+        for (int t = 0; t < D / 32; ++t)
+          dQt[t] = M::mma(tr64<T>((ta ^ (uint32_t)(t << 6)) + 2048u * s, (tb ^ (uint32_t)(t << 6)) + 2048u * s), dSb, dQt[t]);
+      }
+    }
+    dma_wait_all();
+    __syncthreads();
+  }
+
+  // add the splits' partial dQ through LDS, in split order: slot x = (split - 1) * RG + row group, 8 KB each
+  float *xo = reinterpret_cast<float *>(sAll);
+  if (sp > 0) {
+#pragma unroll
+    for (int t = 0; t < D / 32; ++t)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) xo[((sp - 1) * RG + rg) * 2048 + (t * 16 + v) * 64 + lane] = dQt[t][v];
+  }
+  __syncthreads();
+  if (sp > 0 || !row_ok) return;
+#pragma unroll
+  for (int s2 = 1; s2 < SPLIT; ++s2)
+#pragma unroll
+    for (int t = 0; t < D / 32; ++t)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) dQt[t][v] += xo[((s2 - 1) * RG + rg) * 2048 + (t * 16 + v) * 64 + lane];
+  T *dqp = reinterpret_cast<T *>(p.dq) + (int64_t)(q0 + row_q) * p.dq_stride + (int64_t)h * D;
+#pragma unroll
+  for (int t = 0; t < D / 32; ++t)
+#pragma unroll
+    for (int vb = 0; vb < 4; ++vb) {
+      Quad<T> *at = reinterpret_cast<Quad<T> *>(dqp + 32 * t + 8 * vb + 4 * hh), a;
+      if (p.dq_accumulate) a = *at;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        a.v[e] = static_cast<T>((p.dq_accumulate ? static_cast<float>(a.v[e]) : 0.f) + dQt[t][4 * vb + e] * p.scale);
+      *at = a;
+    }
+}
+
+// dK, dV: KG row groups of 32 key rows x QSPLIT splits of the query tiles (32 rows of Q and dO each); K and V row
+// fragments stay in registers, lse / delta come straight from the planes that the dQ kernel wrote.
+template <typename T, int KG, int QSPLIT>
+__global__ void __launch_bounds__(64 * KG * QSPLIT, 2) attn_bwd_dkv_d64_kernel(const AttnBwdParams p) {
+  using M = Mma<T>;
+  using Frag = typename M::Frag;
+  constexpr int D = 64, BN = 32 * KG, BM = 32, NW = KG * QSPLIT;
+  constexpr int TILEB = BM * D * (int)sizeof(T);          // bytes of one Q (or dO) tile
+  constexpr int STAGEB = QSPLIT * 2 * TILEB;              // per split: Q tile, dO tile
+  constexpr int CB = QSPLIT * 2 * 4 / NW;                 // copy blocks per wavefront and iteration
+  static_assert(CB == 4 && QSPLIT * 2 == NW, "one whole tile per wavefront");
+  __shared__ __attribute__((aligned(1024))) char sAll[2 * STAGEB];
+
+  const int b = seq_by_length(p.cu_k, gridDim.y, blockIdx.y);
+  const int G = p.hk * p.hsplit;
+  int hg, px;
+  xcd_group_item(blockIdx.x, G, gridDim.x / G, hg, px);
+  const int hkv = hg / p.hsplit, hs = hg % p.hsplit;
+  const int q0 = p.cu_q[b], sq = p.cu_q[b + 1] - q0;
+  const int k0 = p.cu_k[b], sk = p.cu_k[b + 1] - k0;
+  const int j0 = px * BN;          // early causal tiles carry the most work and come first
+  if (j0 >= sk) return;
+  const int causal = p.causal;
+  const float scale_log2 = p.scale_log2;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 31, hh = lane >> 5;
+  const int kg = w % KG, qs = w / KG;
+  const int ratio = p.hq / p.hk, hper = ratio / p.hsplit;
+  const int h_first = hkv * ratio + hs * hper;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)sAll;
+  const int jw0 = j0 + 32 * kg, jrow = jw0 + c;
+
+  // copies of this wavefront: the Q (even) or dO (odd) tile of split w / 2
+  const int cp_do = w & 1, cp_sp = w >> 1;
+  const int64_t cp_stride = cp_do ? p.do_stride : p.q_stride;
+  const T *cp_g = reinterpret_cast<const T *>(cp_do ? p.dout : p.q) + (int64_t)q0 * cp_stride;
+  const Copy64 cl = copy64_lane(lane, (uint32_t)(cp_stride * (int64_t)sizeof(T)));
+  const uint32_t cp_dst = lds0 + (uint32_t)((cp_sp * 2 + cp_do) * TILEB);
+
+  const int i_begin = causal ? j0 : 0;
+  const int ntq = i_begin < sq ? (sq - i_begin + BM - 1) / BM : 0;
+  const int it_per_head = (ntq + QSPLIT - 1) / QSPLIT;
+  const int niter = it_per_head * hper;
+  auto issue = [&](int stage, int g, int ti) {
+    const int tq = ti * QSPLIT + cp_sp;
+    if (tq < ntq)
+      copy64<T, CB>(cp_g + (int64_t)(h_first + g) * D, cp_stride, i_begin + tq * BM, sq, cp_dst + (uint32_t)(stage * STAGEB), cl);
+  };
+  if (niter > 0) issue(0, 0, 0);
+
+  Frag Kf[D / 16], Vf[D / 16];
+  {
+    const int jl = jrow < sk ? jrow : sk - 1;
+    const T *kp = reinterpret_cast<const T *>(p.k) + (int64_t)(k0 + jl) * p.k_stride + (int64_t)hkv * D + 8 * hh;
+    const T *vp = reinterpret_cast<const T *>(p.v) + (int64_t)(k0 + jl) * p.v_stride + (int64_t)hkv * D + 8 * hh;
+#pragma unroll
+    for (int ks = 0; ks < D / 16; ++ks) {
+      Kf[ks] = frag_ld<T>(kp + ks * 16);
+      Vf[ks] = frag_ld<T>(vp + ks * 16);
+    }
+  }
+  floatx16 dKt[D / 32], dVt[D / 32];
+#pragma unroll
+  for (int t = 0; t < D / 32; ++t)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      dKt[t][v] = 0.f;
+      dVt[t][v] = 0.f;
+    }
+  const uint32_t q_lane = lds0 + (uint32_t)(qs * 2 * TILEB) + row64_lane(lane);
+  const uint32_t ta_lane = lds0 + (uint32_t)(qs * 2 * TILEB) + tr64_lane(lane);
+  // lse (exp2 units) and delta of the rows 8 vb + 4 hh + e of this wavefront's query tile (no branch: past the last tile it
+  // loads the last one's)
+  floatx4 l4[4], d4[4];
+  auto load_ld = [&](int g, int ti) {
+    const int tq = ti * QSPLIT + qs < ntq ? ti * QSPLIT + qs : ntq - 1;
+    const float *src = p.ld2 + ((int64_t)b * p.hq + (h_first + g)) * p.ld2_pitch + (i_begin + tq * BM) + 4 * hh;
+#pragma unroll
+    for (int vb = 0; vb < 4; ++vb) {
+      l4[vb] = *reinterpret_cast<const floatx4 *>(src + 8 * vb);
+      d4[vb] = *reinterpret_cast<const floatx4 *>(src + p.ld2_plane + 8 * vb);
+    }
+  };
+#pragma unroll
+  for (int vb = 0; vb < 4; ++vb) {
+    l4[vb] = (floatx4)(0.f);
+    d4[vb] = (floatx4)(0.f);
+  }
+  if (niter > 0) load_ld(0, 0);
+  dma_wait_all();
+  __syncthreads();
+
+  int g = 0, ti = 0;                                // head and step of iteration it
+#pragma unroll 1
+  for (int it = 0; it < niter; ++it) {
+    int gn = g, tn = ti + 1;                        // ... and of iteration it + 1
+    if (tn == it_per_head) { tn = 0; ++gn; }
+    const bool have_next = it + 1 < niter;
+    if (have_next) issue((it + 1) & 1, gn, tn);
+    const int tq = ti * QSPLIT + qs, i0 = i_begin + tq * BM;
+    if (tq < ntq && !(causal && i0 + BM - 1 < jw0)) {
+      const uint32_t st = (uint32_t)((it & 1) * STAGEB);
+      const uint32_t qb = q_lane + st, ta = ta_lane + st, tb = tr64_next(ta);
+      floatx16 S, dP;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        S[v] = 0.f;
+        dP[v] = 0.f;
+      }
+#pragma unroll
+      for (int ks = 0; ks < D / 16; ++ks) {
+        S = M::mma(row64<T>(qb ^ (uint32_t)(ks << 5)), Kf[ks], S);
+        dP = M::mma(row64<T>((qb ^ (uint32_t)(ks << 5)) + (uint32_t)TILEB), Vf[ks], dP);
+      }
+      if ((causal && i0 < jw0 + 31) || i0 + BM > sq) {
+        const int lo = causal ? jrow : 0;           // first query row that attends to this lane's key
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          const int i = i0 + acc_row(v, hh);
+          S[v] = i >= lo && i < sq ? S[v] : -INFINITY;        // P = dS = 0
+        }
+      }
+      Frag Pb[2], dSb[2];
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        float pv[8], dsv[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const int v = 8 * s + j;
+          pv[j] = fast_exp2(S[v] * scale_log2 - l4[v >> 2][v & 3]);
+          dsv[j] = pv[j] * (dP[v] - d4[v >> 2][v & 3]);
+        }
+        Pb[s] = frag_pack<T>(pv);
+        dSb[s] = frag_pack<T>(dsv);
+      }
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int t = 0; t < D / 32; ++t) {
+          const uint32_t a = (ta ^ (uint32_t)(t << 6)) + 2048u * s, bb = (tb ^ (uint32_t)(t << 6)) + 2048u * s;
+          dVt[t] = M::mma(tr64<T>(a + (uint32_t)TILEB, bb + (uint32_t)TILEB), Pb[s], dVt[t]);
+          dKt[t] = M::mma(tr64<T>(a, bb), dSb[s], dKt[t]);
+        }
+    }
+    if (have_next) {
+      g = gn;
+      ti = tn;
+    }
+    load_ld(g, ti);
+    dma_wait_all();
+    __syncthreads();
+  }
+
+  // add the splits' partial sums through LDS in a fixed order, halving: (0 += 2, 1 += 3), then 0 += 1; 16 KB per
+  // (split, key group): dK, then dV
+  static_assert(2 * STAGEB >= (QSPLIT / 2) * KG * 16384, "exchange area");
+  float *xo = reinterpret_cast<float *>(sAll);
+#pragma unroll
+  for (int from = QSPLIT / 2; from >= 1; from >>= 1) {
+    if (qs >= from && qs < 2 * from) {
+      float *dst = xo + ((qs - from) * KG + kg) * 4096 + lane;
+#pragma unroll
+      for (int t = 0; t < D / 32; ++t)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          dst[(t * 16 + v) * 64] = dKt[t][v];
+          dst[2048 + (t * 16 + v) * 64] = dVt[t][v];
+        }
+    }
+    __syncthreads();
+    if (qs < from) {
+      const float *src = xo + (qs * KG + kg) * 4096 + lane;
+#pragma unroll
+      for (int t = 0; t < D / 32; ++t)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          dKt[t][v] += src[(t * 16 + v) * 64];
+          dVt[t][v] += src[2048 + (t * 16 + v) * 64];
+        }
+    }
+    __syncthreads();
+  }
+  if (qs > 0 || jrow >= sk) return;
+  if (p.hsplit == 1) {
+    T *dkp = reinterpret_cast<T *>(p.dk) + (int64_t)(k0 + jrow) * p.dk_stride + (int64_t)hkv * D;
+    T *dvp = reinterpret_cast<T *>(p.dv) + (int64_t)(k0 + jrow) * p.dv_stride + (int64_t)hkv * D;
+#pragma unroll
+    for (int t = 0; t < D / 32; ++t)
+#pragma unroll
+      for (int vb = 0; vb < 4; ++vb) {
+        Quad<T> a, bq;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          a.v[e] = static_cast<T>(dKt[t][4 * vb + e] * p.scale);
+          bq.v[e] = static_cast<T>(dVt[t][4 * vb + e]);
+        }
+        *reinterpret_cast<Quad<T> *>(dkp + 32 * t + 8 * vb + 4 * hh) = a;
+        *reinterpret_cast<Quad<T> *>(dvp + 32 * t + 8 * vb + 4 * hh) = bq;
+      }
+  } else {
+    const int64_t off = (((int64_t)hs * p.total_k + (k0 + jrow)) * p.hk + hkv) * D;
+#pragma unroll
+    for (int t = 0; t < D / 32; ++t)
+#pragma unroll
+      for (int vb = 0; vb < 4; ++vb) {
+        floatx4 a, bq;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          a[e] = dKt[t][4 * vb + e] * p.scale;
+          bq[e] = dVt[t][4 * vb + e];
+        }
+        *reinterpret_cast<floatx4 *>(p.dk_part + off + 32 * t + 8 * vb + 4 * hh) = a;
+        *reinterpret_cast<floatx4 *>(p.dv_part + off + 32 * t + 8 * vb + 4 * hh) = bq;
+      }
+  }
+}
+
+template <typename T, int RG, int SPLIT>
+static int launch_dq_d64(const AttnBwdParams &p, int batch, hipStream_t st) {
+  dim3 grid((unsigned)(cdiv(p.max_sq, 32 * RG) * p.hq), (unsigned)batch);
+  hipLaunchKernelGGL((attn_bwd_dq_d64_kernel<T, RG, SPLIT>), grid, dim3(512), 0, st, p);
+  return DH_OK;
+}
+
+template <typename T, int KG, int QSPLIT>
+static int launch_dkv_d64(const AttnBwdParams &p, int batch, int max_sk, hipStream_t st) {
+  dim3 grid((unsigned)(cdiv(max_sk, 32 * KG) * p.hk * p.hsplit), (unsigned)batch);
+  hipLaunchKernelGGL((attn_bwd_dkv_d64_kernel<T, KG, QSPLIT>), grid, dim3(64 * KG * QSPLIT), 0, st, p);
+  return DH_OK;
+}
+
+}  // namespace dh

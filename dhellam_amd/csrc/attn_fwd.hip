@@ -48,7 +48,7 @@ __global__ void __launch_bounds__(64 * NW) attn_fwd_kernel(const AttnFwdParams p
   T *sK = reinterpret_cast<T *>(smem_raw);  // [2][BN*KS]
   T *sV = sK + 2 * BN * KS;                 // [2][BN*VS]
 
-  const int b = blockIdx.z, h = blockIdx.y;
+  const int b = seq_by_length(p.cu_q, gridDim.z, blockIdx.z), h = blockIdx.y;
   const int mt = gridDim.x - 1 - blockIdx.x;  // heavy (late) causal tiles first
   const int q0 = p.cu_q[b], sq = p.cu_q[b + 1] - q0;
   const int k0 = p.cu_k[b], sk = p.cu_k[b + 1] - k0;
@@ -242,7 +242,7 @@ __global__ void __launch_bounds__(512) attn_fwd_d128_kernel(const AttnFwdParams 
   constexpr int NV = 3;                           // V slots: read one iteration late, copied one ahead
   __shared__ __attribute__((aligned(1024))) T sAll[(2 + NV) * SLOT];   // K slots 0..1, then the V slots
 
-  const int b = blockIdx.y;
+  const int b = seq_by_length(p.cu_q, gridDim.y, blockIdx.y);
   // the query heads of one kv head read the same K / V rows: keep a kv head on one XCD's L2
   const int ratio = p.hq / p.hk, P = gridDim.x / p.hq;
   int hkv, item;
@@ -591,6 +591,12 @@ static int launch_attn_fwd_d128(const AttnFwdParams &p, int batch, hipStream_t s
   return DH_OK;
 }
 
+}  // namespace dh
+
+#include "attn_fwd_d64.h"
+
+namespace dh {
+
 // fewest workgroups of 128 query rows for which the 128-row kernel is taken
 #ifndef DH_FWD_128ROW_MIN_WG
 #define DH_FWD_128ROW_MIN_WG 256
@@ -653,6 +659,11 @@ extern "C" int dh_attn_fwd(const void *q, const void *k, const void *v, void *ou
     const bool big = wg128 >= DH_FWD_128ROW_MIN_WG;
     if (dtype == DH_BF16) rc = big ? launch_attn_fwd_d128<bf16_t, 4, 2, 64, DH_FWD_LAG>(p, batch, st) : launch_attn_fwd_d128<bf16_t, 2, 4, 32, DH_FWD_LAG>(p, batch, st);
     else rc = big ? launch_attn_fwd_d128<f16_t, 4, 2, 64, DH_FWD_LAG>(p, batch, st) : launch_attn_fwd_d128<f16_t, 2, 4, 32, DH_FWD_LAG>(p, batch, st);
+  } else if (d == 64) {
+    // 128-row query tiles when they give every compute unit its two workgroups, else 64-row tiles with four key splits.
+    const bool big = cdiv(max_seqlen_q, 128) * hq * batch >= 2 * 256;
+    if (dtype == DH_BF16) rc = big ? launch_attn_fwd_d64<bf16_t, 4, 2, 64>(p, batch, st) : launch_attn_fwd_d64<bf16_t, 2, 4, 32>(p, batch, st);
+    else rc = big ? launch_attn_fwd_d64<f16_t, 4, 2, 64>(p, batch, st) : launch_attn_fwd_d64<f16_t, 2, 4, 32>(p, batch, st);
   } else {
     // Few query tiles (small batch*heads) -> smaller workgroups so the grid still covers the chip.
     const int64_t blocks128 = cdiv(max_seqlen_q, 128) * hq * batch;
@@ -664,8 +675,7 @@ extern "C" int dh_attn_fwd(const void *q, const void *k, const void *v, void *ou
   } while (0)
     // the register-staged kernel, compiled per head dim (the other head dims of the reference's d <= 256 reach
     // these through zero padding in the binding, as flash_atten.cu:303-312 pads to a multiple of 8)
-    if (d == 64) DH_FWD_GENERIC(64);
-    else if (d == 96) DH_FWD_GENERIC(96);
+    if (d == 96) DH_FWD_GENERIC(96);
     else if (d == 192) DH_FWD_GENERIC(192);
     else DH_FWD_GENERIC(256);
 #undef DH_FWD_GENERIC

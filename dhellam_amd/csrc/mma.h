@@ -243,6 +243,22 @@ __device__ __forceinline__ float pair32_sum(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// The sequence of a batch with the given place in the order of falling length (ties: lower index first), for batches of up
+// to 64 sequences; longer ones keep their order.  Workgroups start in the order of their ids, so with the longest
+// sequences first the chip drains on short work (seven packed documents of 1 to 3324 tokens, the longest last, 32 / 8
+// heads: forward and backward 955 -> 915 us).  One load and about 10 cycles per sequence, none for a single one.
+__device__ __forceinline__ int seq_by_length(const int32_t *cu, int n, int place) {
+  if (n <= 1 || n > 64) return place;
+  const int lane = threadIdx.x & 63;
+  const int len = lane < n ? cu[lane + 1] - cu[lane] : -1;
+  int before = 0;
+  for (int j = 0; j < n; ++j) {
+    const int o = __builtin_amdgcn_readlane(len, j);
+    before += (o > len || (o == len && j < lane)) ? 1 : 0;
+  }
+  return (int)__builtin_ctzll(__ballot(lane < n && before == place));
+}
+
 // Row index inside a 32-row accumulator block held by register v of lane half h.
 __device__ __forceinline__ int acc_row(int v, int h) { return 8 * (v >> 2) + 4 * h + (v & 3); }
 

@@ -366,3 +366,15 @@ def test_attention_head_dim_above_256_is_refused():
 def test_attention_f32_matrix_core_kernels(lens_q, lens_k, hq, hk, d, causal):
     """fp32 kernels for head dims up to 128: tile edges of both sequences, full and partial column tiles, GQA."""
     _run_fwd_bwd(torch.float32, lens_q, lens_k, hq, hk, d, causal)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("lens_q,lens_k,hq,hk,causal", [
+    ([1, 33, 300], [1, 33, 300], 4, 2, True),            # tile edges, more sequences than one, longest last
+    ([129], [129], 2, 1, True), ([70, 31], [257, 64], 2, 2, False), ([5], [3], 1, 1, False),
+    ([1100], [1100], 64, 64, True),                      # the chip-filling form (128-row query tiles)
+    ([520, 40], [200, 700], 64, 8, False),
+])
+def test_attention_head_dim_64(dtype, lens_q, lens_k, hq, hk, causal):
+    """Head dim 64 kernels: both workgroup shapes, tile edges of both sequences, ragged batches, GQA groups."""
+    _run_fwd_bwd(dtype, lens_q, lens_k, hq, hk, 64, causal)
