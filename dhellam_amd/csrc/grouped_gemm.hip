@@ -497,11 +497,17 @@ __global__ void __launch_bounds__(256) grouped_gemm_w4_kernel(const GGParams p) 
   // the scalar offset with the length, so a row past the end reads as zero whichever 32-row block it is in.
   // (k-strided operands: cut at the last k row, i.e. the group's last row for TN; their tiles are whole in the
   // other direction, which the host checks)
-  const gg_i32x4 rsa = AKS ? gg_rsrc(ag, (int64_t)(row_end - row_begin) * lda_b - (int64_t)m0 * (int)sizeof(T))
+  const gg_i32x4 rsa_ = AKS ? gg_rsrc(ag, (int64_t)(row_end - row_begin) * lda_b - (int64_t)m0 * (int)sizeof(T))
                            : gg_rsrc(ag, (int64_t)(a_rext < 256 ? a_rext : 256) * lda_b);
-  const gg_i32x4 rsb = AKS ? gg_rsrc(bg, (int64_t)(row_end - row_begin) * ldb_b - (int64_t)n0 * (int)sizeof(T))
+  const gg_i32x4 rsb_ = AKS ? gg_rsrc(bg, (int64_t)(row_end - row_begin) * ldb_b - (int64_t)n0 * (int)sizeof(T))
                      : BKS ? gg_rsrc(bg, (int64_t)p.k_dim * ldb_b - (int64_t)n0 * (int)sizeof(T))
                            : gg_rsrc(bg, (int64_t)(b_rext < 256 ? b_rext : 256) * ldb_b);
+  // The descriptors come out of v_readfirstlane, and a memory instruction may read such a scalar register five wait
+  // states later at the earliest.  The compiler keeps that distance for its own instructions, not for the loads issued
+  // from assembly below: without this the first of them went out with the previous contents of the length, now and then
+  // (a group of fewer than 64 rows then took rows of its neighbour into its weight gradient).
+  gg_i32x4 rsa = rsa_, rsb = rsb_;
+  asm volatile("s_nop 4" : "+s"(rsa), "+s"(rsb));
   const int cnt = s1 - s0;                              // slices of this segment
   floatx16 acc[4][4];
 #pragma unroll
