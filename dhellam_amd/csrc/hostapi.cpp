@@ -527,16 +527,23 @@ Tensor moe_scatter(const Tensor &y, const Tensor &dest_row, const OptTensor &gat
   return out;
 }
 
-Tensor moe_gate_grad(const Tensor &dout, const Tensor &y, const Tensor &dest_row, const Tensor &offs, int e_lo, int e_hi,
-                     int64_t tokens, int k, const OptStream &stream) {
+// -> (dy [max_rows, H], dgates [T, k])
+std::tuple<Tensor, Tensor> moe_unpermute_bwd(const Tensor &dout, const Tensor &y, const Tensor &sorted_idx, const Tensor &dest_row,
+                                             const Tensor &gates, const Tensor &offs, int e_lo, int e_hi, int64_t max_rows,
+                                             int64_t tokens, int k, const OptStream &stream) {
+  PY_ASSERT(dout.is_cuda() && dout.is_contiguous() && dout.dim() == 2, "unpermute: rows must be a contiguous 2-D GPU tensor");
+  PY_ASSERT(y.is_contiguous() && y.dim() == 2 && y.size(1) == dout.size(1) && y.scalar_type() == dout.scalar_type(),
+            "unpermute: expert outputs must be rows like dout's");
   const int type = dt(dout);
   On on(stream);
+  Tensor dy = at::empty({max_rows, dout.size(1)}, dout.options());
   Tensor dg = at::empty({tokens, k}, dout.options().dtype(at::kFloat));
   launch([&] {
-    return dh_moe_gate_grad(dout.data_ptr(), y.data_ptr(), dest_row.data_ptr<int>(), dg.data_ptr<float>(), offs.data_ptr<int>(),
-                            e_lo, e_hi, tokens, k, dout.size(1), type, on.get());
+    return dh_moe_unpermute_bwd(dout.data_ptr(), y.data_ptr(), sorted_idx.data_ptr<int>(), dest_row.data_ptr<int>(),
+                                gates.data_ptr<float>(), dy.data_ptr(), dg.data_ptr<float>(), offs.data_ptr<int>(), e_lo, e_hi,
+                                max_rows, tokens, k, dout.size(1), type, on.get());
   });
-  return dg;
+  return {dy, dg};
 }
 
 // c [R, N] = per group a [R, K] times b [G, N, K]^T (transposed) or b [G, K, N]
@@ -551,17 +558,11 @@ Tensor grouped_gemm(const Tensor &a, const Tensor &b, const Tensor &offs, std::o
   Tensor c = out.has_value() ? *out : at::empty({held, n}, a.options());
   const int64_t rows = max_rows.value_or(held);
   if (!out.has_value() && rows < held) c.narrow(0, rows, held - rows).zero_();
-  // split-k workspace: products with fewer 256x256 tiles than compute units do not use one
-  void *ws = nullptr;
-  size_t ws_bytes = 0;
-  if (((rows + 255) / 256) * ((n + 255) / 256) >= 256) {
-    Tensor t = scratch(kGrouped, (int64_t)dh_grouped_gemm_workspace_bytes(), a, on.get());
-    ws = t.data_ptr();
-    ws_bytes = (size_t)t.numel();
-  }
+  Tensor ws = scratch(kGrouped, (int64_t)dh_grouped_gemm_workspace_bytes(), a, on.get());      // split-k pieces
   launch([&] {
     return (transposed ? dh_grouped_gemm_nt : dh_grouped_gemm_nn)(a.data_ptr(), b.data_ptr(), c.data_ptr(), offs.data_ptr<int>(),
-                                                                  (int)g, rows, n, k, type, ws, ws_bytes, on.get());
+                                                                  (int)g, rows, n, k, type, ws.data_ptr(),
+                                                                  (size_t)ws.numel(), on.get());
   });
   return c;
 }
@@ -576,11 +577,33 @@ Tensor grouped_gemm_tn(const Tensor &a, const Tensor &b, const Tensor &offs, con
   const int type = dt(a);
   On on(stream);
   Tensor c = out.has_value() ? *out : at::empty({g, m, n}, a.options());
+  Tensor ws = scratch(kGrouped, (int64_t)dh_grouped_gemm_workspace_bytes(), a, on.get());
   launch([&] {
-    return dh_grouped_gemm_tn(a.data_ptr(), b.data_ptr(), c.data_ptr(), offs.data_ptr<int>(), (int)g, a.size(0), m, n, accumulate,
-                              type, on.get());
+    return dh_grouped_gemm_tn_ws(a.data_ptr(), b.data_ptr(), c.data_ptr(), offs.data_ptr<int>(), (int)g, a.size(0), m, n,
+                                 accumulate, type, ws.data_ptr(), (size_t)ws.numel(), on.get());
   });
   return c;
+}
+
+// The SwiGLU expert FFN on permuted rows -> (y [R, H], h [R, 2F], a [R, F]).
+std::tuple<Tensor, Tensor, Tensor> expert_ffn_fwd(const Tensor &xp, const Tensor &w1, const Tensor &w2, const Tensor &offs,
+                                                  const OptStream &stream) {
+  Tensor h = grouped_gemm(xp, w1, offs, std::nullopt, std::nullopt, true, stream);
+  Tensor a = std::get<0>(swiglu_fwd(h, false, stream));
+  return {grouped_gemm(a, w2, offs, std::nullopt, std::nullopt, true, stream), h, a};
+}
+
+// Its backward -> (dxp, dw1, dw2).  w1t / w2t: the weights' resident transposes, if kept: the data gradients then run in
+// the forward's layout.  dw1 / dw2 are accumulated into when given.
+std::tuple<Tensor, Tensor, Tensor> expert_ffn_bwd(const Tensor &dy, const Tensor &xp, const Tensor &w1, const Tensor &w2,
+                                                  const OptTensor &w1t, const OptTensor &w2t, const Tensor &offs, const Tensor &h,
+                                                  const Tensor &a, const OptTensor &dw1, const OptTensor &dw2,
+                                                  const OptStream &stream) {
+  Tensor da = grouped_gemm(dy, w2t.has_value() ? *w2t : w2, offs, std::nullopt, std::nullopt, w2t.has_value(), stream);
+  Tensor g2 = grouped_gemm_tn(dy, a, offs, dw2, dw2.has_value(), stream);
+  Tensor dh = std::get<0>(swiglu_bwd(da, h, std::nullopt, false, stream));
+  Tensor dxp = grouped_gemm(dh, w1t.has_value() ? *w1t : w1, offs, std::nullopt, std::nullopt, w1t.has_value(), stream);
+  return {dxp, grouped_gemm_tn(dh, xp, offs, dw1, dw1.has_value(), stream), g2};
 }
 
 // ---- head -----------------------------------------------------------------------------------------------------------
@@ -625,7 +648,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("moe_sort", &moe_sort);
   m.def("moe_gather", &moe_gather);
   m.def("moe_scatter", &moe_scatter);
-  m.def("moe_gate_grad", &moe_gate_grad);
+  m.def("moe_unpermute_bwd", &moe_unpermute_bwd);
+  m.def("expert_ffn_fwd", &expert_ffn_fwd);
+  m.def("expert_ffn_bwd", &expert_ffn_bwd);
   m.def("grouped_gemm", &grouped_gemm);
   m.def("grouped_gemm_tn", &grouped_gemm_tn);
   m.def("embedding_fwd", &embedding_fwd);

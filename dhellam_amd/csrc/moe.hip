@@ -117,15 +117,11 @@ moe_scan_kernel(int32_t *__restrict__ hist, int32_t *__restrict__ tokens_per_exp
   }
 }
 
-__global__ void __launch_bounds__(256)
-moe_rank_scatter_kernel(const int32_t *__restrict__ expert_of, const int32_t *__restrict__ start,
-                        int32_t *__restrict__ sorted_idx, int32_t *__restrict__ dest_row, int64_t n, int E) {
-  __shared__ int running[MOE_MAX_E];
-  __shared__ int wcnt[4][MOE_MAX_E];
+// The SORT_ITEMS items from `base` on get their places: running[e] is where the next item of expert e goes.
+__device__ __forceinline__ void moe_rank_items(const int32_t *__restrict__ expert_of, int32_t *__restrict__ sorted_idx,
+                                               int32_t *__restrict__ dest_row, int *running, int (*wcnt)[MOE_MAX_E],
+                                               int64_t base, int64_t n, int E) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  if ((int)threadIdx.x < E) running[threadIdx.x] = start[(int64_t)blockIdx.x * E + threadIdx.x];
-  __syncthreads();
-  const int64_t base = (int64_t)blockIdx.x * SORT_ITEMS;
   const uint64_t lt_mask = lane == 0 ? 0ull : (~0ull >> (64 - lane));
   for (int r = 0; r < SORT_ITEMS / 256; ++r) {
     const int64_t i = base + r * 256 + threadIdx.x;
@@ -150,6 +146,88 @@ moe_rank_scatter_kernel(const int32_t *__restrict__ expert_of, const int32_t *__
     if ((int)threadIdx.x < E) running[threadIdx.x] += wcnt[0][threadIdx.x] + wcnt[1][threadIdx.x] + wcnt[2][threadIdx.x] + wcnt[3][threadIdx.x];
     __syncthreads();
   }
+}
+
+__global__ void __launch_bounds__(256)
+moe_rank_scatter_kernel(const int32_t *__restrict__ expert_of, const int32_t *__restrict__ start,
+                        int32_t *__restrict__ sorted_idx, int32_t *__restrict__ dest_row, int64_t n, int E) {
+  __shared__ int running[MOE_MAX_E];
+  __shared__ int wcnt[4][MOE_MAX_E];
+  if ((int)threadIdx.x < E) running[threadIdx.x] = start[(int64_t)blockIdx.x * E + threadIdx.x];
+  __syncthreads();
+  moe_rank_items(expert_of, sorted_idx, dest_row, running, wcnt, (int64_t)blockIdx.x * SORT_ITEMS, n, E);
+}
+
+// The whole sort in one launch for lists of up to MOE_ONE_LAUNCH assignments: every workgroup counts the experts of ALL of
+// them (each thread in counters of its own: LDS adds that never meet), once up to its own items and once to the end, so no
+// pass over the list has to wait for another.  2000 assignments of 8 experts: three launches 14.6 us -> 5.5 us; up to 65536
+// a workgroup's 256 KB come out of L2 in less time than the launches that it saves.
+constexpr int64_t MOE_ONE_LAUNCH = 65536;
+__global__ void __launch_bounds__(256)
+moe_sort_one_kernel(const int32_t *__restrict__ expert_of, int32_t *__restrict__ tokens_per_expert,
+                    int32_t *__restrict__ expert_offsets, int32_t *__restrict__ sorted_idx, int32_t *__restrict__ dest_row,
+                    int n, int E) {
+  extern __shared__ int cnt[];                                    // [E][256]
+  __shared__ int running[MOE_MAX_E], total[MOE_MAX_E], wcnt[4][MOE_MAX_E];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int base = (int)blockIdx.x * SORT_ITEMS;
+  for (int e = 0; e < E; ++e) cnt[e * 256 + tid] = 0;
+  auto count = [&](int from, int to) {                            // both multiples of 4, or `to` the end of the list
+    constexpr int U = 4;                                          // loads in flight
+    for (int i0 = from; i0 < to; i0 += 256 * 4 * U) {
+      int4 v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int i = i0 + (u * 256 + tid) * 4;
+        v[u] = make_int4(-1, -1, -1, -1);
+        if (i + 3 < to) {
+          v[u] = *reinterpret_cast<const int4 *>(expert_of + i);
+        } else {
+          if (i < to) v[u].x = expert_of[i];
+          if (i + 1 < to) v[u].y = expert_of[i + 1];
+          if (i + 2 < to) v[u].z = expert_of[i + 2];
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {                               // ids outside [0, E) are left out of the sort
+        if ((unsigned)v[u].x < (unsigned)E) atomicAdd(&cnt[v[u].x * 256 + tid], 1);
+        if ((unsigned)v[u].y < (unsigned)E) atomicAdd(&cnt[v[u].y * 256 + tid], 1);
+        if ((unsigned)v[u].z < (unsigned)E) atomicAdd(&cnt[v[u].z * 256 + tid], 1);
+        if ((unsigned)v[u].w < (unsigned)E) atomicAdd(&cnt[v[u].w * 256 + tid], 1);
+      }
+    }
+  };
+  auto sums = [&](int *out) {
+    __syncthreads();
+    for (int e = w; e < E; e += 4) {
+      int s = cnt[e * 256 + lane] + cnt[e * 256 + 64 + lane] + cnt[e * 256 + 128 + lane] + cnt[e * 256 + 192 + lane];
+#pragma unroll
+      for (int d = 32; d > 0; d >>= 1) s += __shfl_xor(s, d, 64);
+      if (lane == 0) out[e] = s;
+    }
+    __syncthreads();
+  };
+  if (blockIdx.x > 0) count(0, base);
+  sums(running);
+  count(base, n);
+  sums(total);
+  if (w == 0) {
+    const int t = lane < E ? total[lane] : 0;
+    int incl = t;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int o = __shfl_up(incl, d, 64);
+      if (lane >= d) incl += o;
+    }
+    if (lane < E) running[lane] += incl - t;
+    if (blockIdx.x == 0 && lane < E) {
+      tokens_per_expert[lane] = t;
+      expert_offsets[lane] = incl - t;
+      if (lane == E - 1) expert_offsets[E] = incl;
+    }
+  }
+  __syncthreads();
+  moe_rank_items(expert_of, sorted_idx, dest_row, running, wcnt, base, n, E);
 }
 
 // A workgroup moves RPB rows per trip and issues every load of the trip before its first store: a row is only
@@ -328,6 +406,77 @@ moe_gate_grad_kernel(const T *__restrict__ dout, const T *__restrict__ y, const 
   }
 }
 
+// The backward of unpermute in one pass over the local rows: dy[r] = gate * dout[token] and dgates[a] = <dout[token], y[r]>
+// of the assignment a that row r holds (the sums as in moe_gate_grad_kernel), zeros for the assignments of other ranks.
+// One launch and one reading of dout less than the two kernels.
+template <typename T>
+__global__ void __launch_bounds__(256)
+moe_unpermute_bwd_kernel(const T *__restrict__ dout, const T *__restrict__ y, const int32_t *__restrict__ sorted_idx,
+                         const int32_t *__restrict__ dest_row, const float *__restrict__ gates, T *__restrict__ dy,
+                         float *__restrict__ dgates, const int32_t *__restrict__ offs, int e_lo, int e_hi, int64_t max_rows,
+                         int64_t assigns, int K, int64_t hidden, int vec_ok) {
+  __shared__ float red[4];
+  constexpr int N = Vec<T>::N;
+  constexpr int U = 2;
+  const int first = offs[e_lo];
+  int64_t n_rows = (int64_t)offs[e_hi] - first;
+  if (n_rows > max_rows) n_rows = max_rows;
+  if (n_rows < 0) n_rows = 0;
+  for (int64_t a = (int64_t)blockIdx.x * 256 + threadIdx.x; a < assigns; a += (int64_t)gridDim.x * 256) {
+    const int64_t rr = (int64_t)dest_row[a] - first;
+    if (rr < 0 || rr >= n_rows) dgates[a] = 0.f;
+  }
+  for (int64_t r = blockIdx.x; r < max_rows; r += gridDim.x) {
+    T *dst = dy + r * hidden;
+    if (r >= n_rows) {
+      if (vec_ok) {
+        Vec<T> z;
+#pragma unroll
+        for (int j = 0; j < N; ++j) z.v[j] = from_f<T>(0.f);
+        for (int64_t c = threadIdx.x; c < hidden / N; c += 256) stg(dst + c * N, z);
+      } else {
+        for (int64_t c = threadIdx.x; c < hidden; c += 256) dst[c] = from_f<T>(0.f);
+      }
+      continue;
+    }
+    const int a = sorted_idx[first + r];
+    const T *src = dout + (int64_t)(a / K) * hidden, *q = y + r * hidden;
+    const float sc = gates[a];
+    float s = 0.f;
+    if (vec_ok) {
+      const int64_t nv = hidden / N;
+      for (int64_t c0 = threadIdx.x; c0 < nv; c0 += U * 256) {
+        Vec<T> v[U], o[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          if (c0 + u * 256 < nv) {
+            v[u] = ldg(src + (c0 + u * 256) * N);
+            o[u] = ldg(q + (c0 + u * 256) * N);
+          }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          if (c0 + u * 256 < nv) {
+#pragma unroll
+            for (int j = 0; j < N; ++j) {
+              const float f = to_f(v[u].v[j]);
+              s += f * to_f(o[u].v[j]);
+              v[u].v[j] = from_f<T>(f * sc);
+            }
+            stg(dst + (c0 + u * 256) * N, v[u]);
+          }
+      }
+    } else {
+      for (int64_t c = threadIdx.x; c < hidden; c += 256) {
+        const float f = to_f(src[c]);
+        s += f * to_f(q[c]);
+        dst[c] = from_f<T>(f * sc);
+      }
+    }
+    s = block256_sum(s, red);
+    if (threadIdx.x == 0) dgates[a] = s;
+  }
+}
+
 }  // namespace dh
 
 extern "C" int dh_moe_route_topk(const float *logits, int32_t *topk_idx, float *gates, int64_t tokens, int experts,
@@ -356,6 +505,13 @@ static int moe_sort_launch(const int32_t *topk_idx, int32_t *tokens_per_expert, 
                            hipStream_t st) {
   using namespace dh;
   const int nb = (int)cdiv(n_assign, SORT_ITEMS);
+  if (nb > 0 && n_assign <= MOE_ONE_LAUNCH && aligned16(topk_idx)) {
+    DH_CHECK(topk_idx && sorted_idx && dest_row, "null pointer");
+    hipLaunchKernelGGL(moe_sort_one_kernel, dim3(nb), dim3(256), (size_t)experts * 256 * sizeof(int), st, topk_idx,
+                       tokens_per_expert, expert_offsets, sorted_idx, dest_row, (int)n_assign, experts);
+    DH_LAUNCH_CHECK();
+    return DH_OK;
+  }
   if (nb > 0) {
     DH_CHECK(topk_idx && sorted_idx && dest_row, "null pointer");
     hipLaunchKernelGGL(moe_hist_kernel, dim3(nb), dim3(256), 0, st, topk_idx, hist, n_assign, experts);
@@ -494,6 +650,28 @@ extern "C" int dh_moe_gate_grad(const void *dout, const void *y, const int32_t *
     hipLaunchKernelGGL((moe_gate_grad_kernel<T>), dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream,
                        (const T *)dout, (const T *)y, dest_row, dgates, expert_offsets, e_lo, e_hi, tokens, k, hidden,
                        vec_ok);
+  });
+  DH_LAUNCH_CHECK();
+  return DH_OK;
+}
+
+extern "C" int dh_moe_unpermute_bwd(const void *dout, const void *y, const int32_t *sorted_idx, const int32_t *dest_row,
+                                    const float *gates, void *dy, float *dgates, const int32_t *expert_offsets, int e_lo,
+                                    int e_hi, int64_t max_rows, int64_t tokens, int k, int64_t hidden, int dtype,
+                                    void *stream) {
+  using namespace dh;
+  DH_CHECK(max_rows >= 0 && tokens >= 0 && hidden >= 0 && k >= 1, "bad shape");
+  DH_CHECK(moe_range_check(e_lo, e_hi), "bad expert range [%d, %d)", e_lo, e_hi);
+  if (tokens == 0 && (max_rows == 0 || hidden == 0)) return DH_OK;
+  DH_CHECK(sorted_idx && dest_row && gates && dgates && expert_offsets, "null pointer");
+  DH_CHECK(max_rows == 0 || hidden == 0 || (dout && y && dy), "null pointer");
+  const int64_t need = max_rows > cdiv(tokens * k, 256) ? max_rows : cdiv(tokens * k, 256);
+  const int64_t blocks = need < 65536 ? need : 65536;
+  DH_DISPATCH_DTYPE(dtype, {
+    const int vec_ok = hidden % Vec<T>::N == 0 && aligned16(dout) && aligned16(y) && aligned16(dy);
+    hipLaunchKernelGGL((moe_unpermute_bwd_kernel<T>), dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream,
+                       (const T *)dout, (const T *)y, sorted_idx, dest_row, gates, (T *)dy, dgates, expert_offsets, e_lo,
+                       e_hi, max_rows, tokens * k, k, hidden, vec_ok);
   });
   DH_LAUNCH_CHECK();
   return DH_OK;

@@ -16,7 +16,6 @@ import torch
 from .. import _host
 from .._Clib import _note_read, transposed_of
 from ._util import issue
-from .swiglu import swiglu, swiglu_back
 
 
 @dataclass
@@ -76,10 +75,8 @@ def unpermute_fwd(y, plan, gates, e_lo, e_hi, stream=None, profiling=False):
 def unpermute_bwd(dout, y, plan, gates, e_lo, e_hi, max_rows, stream=None, profiling=False):
     """Returns (dy [max_rows, H], dgates fp32 [T, k], ms): dy[r] = gate * dout[token(r)],
     dgates[t, j] = <dout[t], y[row(t, j)]> (0 for assignments owned by other ranks)."""
-    def both(st):
-        dy = _host.moe_gather(dout, plan.sorted_idx, gates, plan.expert_offsets, e_lo, e_hi, max_rows, plan.k, st)
-        return dy, _host.moe_gate_grad(dout, y, plan.dest_row, plan.expert_offsets, e_lo, e_hi, plan.tokens, plan.k, st)
-    (dy, dgates), ms = issue(both, stream, profiling)
+    (dy, dgates), ms = issue(_host.moe_unpermute_bwd, stream, profiling, dout, y, plan.sorted_idx, plan.dest_row, gates,
+                             plan.expert_offsets, e_lo, e_hi, max_rows, plan.tokens, plan.k)
     return dy, dgates, ms
 
 
@@ -105,12 +102,8 @@ def expert_ffn_fwd(xp, w1, w2, offs, stream=None, profiling=False):
     """SwiGLU FFN of the local experts on permuted rows.  xp [R, H]; w1 [G, 2F, H] (gate |
     up); w2 [G, H, F]; offs int32 [G + 1] (a slice of MoEPlan.expert_offsets).
     Returns (y [R, H], (h, a) saved for backward, ms)."""
-    def ffn(st):
-        h = grouped_gemm_nt(xp, w1, offs, stream=st)
-        a, _ = swiglu(h, st)
-        return grouped_gemm_nt(a, w2, offs, stream=st), (h, a)
-    (y, saved), ms = issue(ffn, stream, profiling)
-    return y, saved, ms
+    (y, h, a), ms = issue(_host.expert_ffn_fwd, stream, profiling, xp, w1, w2, offs)
+    return y, (h, a), ms
 
 
 def expert_ffn_bwd(dy, xp, w1, w2, offs, saved, dw1=None, dw2=None, stream=None, profiling=False):
@@ -123,13 +116,10 @@ def expert_ffn_bwd(dy, xp, w1, w2, offs, saved, dw1=None, dw2=None, stream=None,
         # data gradients: against the resident transposes of the expert weights where the caller keeps them
         # (``_Clib.keep_transposed``): the same products in the forward's layout, which the grouped kernel runs faster
         w2t, w1t = transposed_of(w2, st), transposed_of(w1, st)
-        da = grouped_gemm_nt(dy, w2t, offs, stream=st) if w2t is not None else grouped_gemm_nn(dy, w2, offs, stream=st)   # [R, F] = dy @ w2[g]
-        g2 = grouped_gemm_tn(dy, a, offs, out=dw2, accumulate=dw2 is not None, stream=st)   # [G, H, F]
-        dh, _ = swiglu_back(da, h, None, st)
-        dxp = grouped_gemm_nt(dh, w1t, offs, stream=st) if w1t is not None else grouped_gemm_nn(dh, w1, offs, stream=st)   # [R, H] = dh @ w1[g]
-        g1 = grouped_gemm_tn(dh, xp, offs, out=dw1, accumulate=dw1 is not None, stream=st)  # [G, 2F, H]
-        _note_read(w2, st)
-        _note_read(w1, st)
-        return dxp, g1, g2
+        res = _host.expert_ffn_bwd(dy, xp, w1, w2, w1t, w2t, offs, h, a, dw1, dw2, st)
+        if w1t is not None or w2t is not None:
+            _note_read(w2, st)
+            _note_read(w1, st)
+        return res
     (dxp, g1, g2), ms = issue(ffn, stream, profiling)
     return dxp, g1, g2, ms

@@ -306,6 +306,14 @@ int dh_moe_gate_grad(const void *dout, const void *y, const int32_t *dest_row,
                      int e_hi, int64_t tokens, int k, int64_t hidden, int dtype,
                      void *stream);
 
+/* Backward of unpermute in one launch: dy [max_rows, hidden] as dh_moe_gather_rows(dout, gates) and dgates [tokens * k] as
+ * dh_moe_gate_grad. */
+int dh_moe_unpermute_bwd(const void *dout, const void *y, const int32_t *sorted_idx,
+                         const int32_t *dest_row, const float *gates, void *dy,
+                         float *dgates, const int32_t *expert_offsets, int e_lo,
+                         int e_hi, int64_t max_rows, int64_t tokens, int k,
+                         int64_t hidden, int dtype, void *stream);
+
 /* ------------------------------------------------------------------------
  * Grouped GEMM on MFMA (bf16/fp16 in, fp32 accumulate).  No counterpart in
  * the reference.  Group g owns rows [offs[g]-offs[0], offs[g+1]-offs[0]) of
@@ -317,8 +325,8 @@ int dh_moe_gate_grad(const void *dout, const void *y, const int32_t *dest_row,
  * max_rows is the number of rows the stacked operands hold: it bounds the launch grid, group ranges read
  * from offs are cut off there (no row past it is read or written), and NT / NN zero the rows of c from the
  * last group's end up to max_rows, so c may be uninitialised on entry.
- * workspace (NT, NN; may be NULL): device memory of at least dh_grouped_gemm_workspace_bytes() bytes.  With it,
- * a product that fills the chip may have its last round of tiles split along k: the tiles run in rounds of one
+ * workspace (may be NULL): device memory of at least dh_grouped_gemm_workspace_bytes() bytes.  With it, a product
+ * of few tiles is split along k (fp32 pieces through the workspace, added in k order by a second kernel), and a product that fills the chip may have its last round of tiles split along k: the tiles run in rounds of one
  * per compute unit, and when the last round holds at most half as many tiles as there are compute units a second
  * kernel computes them in as many k pieces as fit, whose fp32 sums go through the workspace and are added in k order
  * by a third kernel (deterministic).  288 tiles on 256 compute units then cost 1 1/8 tile times instead of 2; when
@@ -339,6 +347,11 @@ int dh_grouped_gemm_tn(const void *a, const void *b, void *c,
                        const int32_t *offs, int groups, int64_t max_rows,
                        int64_t m, int64_t n, int accumulate, int dtype,
                        void *stream);
+/* The same with a workspace: a product with few tiles is then split along the rows. */
+int dh_grouped_gemm_tn_ws(const void *a, const void *b, void *c,
+                          const int32_t *offs, int groups, int64_t max_rows,
+                          int64_t m, int64_t n, int accumulate, int dtype,
+                          void *workspace, size_t workspace_bytes, void *stream);
 
 /* Plain device-to-device copy kernel: a known-size streaming kernel used to
  * calibrate the profiler's HBM byte counters, and the local stand-in for the

@@ -436,3 +436,49 @@ def test_grouped_gemm_tn_chip_filling(dtype, M, N):
     moe.grouped_gemm_tn(a, b, offs, out=acc, accumulate=True)
     assert_close(acc, ref + acc0.double(), dtype, "TN accumulate")
     assert torch.equal(acc[1].cpu(), acc0[1]), "accumulating an empty group must leave the output as it was"
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,N,K", [
+    ([5, 0, 24, 1], 136, 72),             # 32-row tiles, n and k end inside a tile
+    ([5, 9, 0, 33], 264, 2056),           # the same, split along k
+    ([64, 65, 130, 1], 264, 4168),        # 64-row tiles, split along k
+    ([700, 0, 1365, 35], 1536, 1288),     # 128x128 tiles
+    ([700, 1, 699], 1544, 1608),          # 128x256 tiles
+    ([4200, 0, 37], 4104, 1536),          # 256x256 tiles that reach past n (the weight gradient: past m and n)
+])
+def test_grouped_gemm_tile_sizes(dtype, rows, N, K):
+    """Every tile size the products choose from, at sizes that end inside a tile: NT, NN and TN against fp32 products, rows
+    past the last group zeroed, nothing written behind the output, the same bits on every run."""
+    from dhellam_amd.operators import moe
+    G, R, pad = len(rows), sum(rows), 7
+    st = np.concatenate(([0], np.cumsum(rows)))
+    offs = torch.tensor(3 + st, dtype=torch.int32).cuda()
+    a = randn((R + pad, K), dtype, 41, std=0.5).cuda()
+    d = randn((R + pad, N), dtype, 42, std=0.5).cuda()
+    b = randn((G, N, K), dtype, 43, std=0.5).cuda()
+    ref = torch.cat([a[st[g]:st[g + 1]].float() @ b[g].float().T for g in range(G)])
+    wref = torch.stack([d[st[g]:st[g + 1]].float().T @ a[st[g]:st[g + 1]].float() for g in range(G)])
+    for name, fn, w in (("NT", moe.grouped_gemm_nt, b), ("NN", moe.grouped_gemm_nn, b.transpose(1, 2).contiguous())):
+        out = torch.full((R + pad + 64, N), 3.0, dtype=dtype, device="cuda")
+        c = fn(a, w, offs, out=out)
+        assert bool((out[R + pad:] == 3.0).all()), f"{name}: wrote past the output"
+        assert_close(c[:R], ref, dtype, name)
+        assert bool((c[R:R + pad] == 0).all()), f"{name}: rows past the last group"
+        assert torch.equal(c[:R], fn(a, w, offs)[:R]), f"{name}: runs differ"
+    w = moe.grouped_gemm_tn(d, a, offs)
+    assert_close(w, wref, dtype, "TN")
+    assert torch.equal(w, moe.grouped_gemm_tn(d, a, offs)), "TN: runs differ"
+    acc = torch.ones((G, N, K), dtype=dtype, device="cuda")
+    moe.grouped_gemm_tn(d, a, offs, out=acc, accumulate=True)
+    assert_close(acc, wref + 1, dtype, "TN accumulate")
+
+
+@pytest.mark.parametrize("T,E,k", [(8192, 64, 8), (8193, 64, 8), (257, 1, 1), (1027, 5, 3)])
+def test_sort_at_the_one_launch_limit(T, E, k):
+    """65536 assignments (the longest list sorted in one launch), eight more, one expert, a length that is no multiple of 4."""
+    from dhellam_amd.operators.moe import sort_assignments
+    io, _ = OM.route_topk(_logits(T, E, 6, True).numpy(), k)
+    plan, _ = sort_assignments(torch.from_numpy(io).cuda(), E)
+    for got, want in zip((plan.tokens_per_expert, plan.expert_offsets, plan.sorted_idx, plan.dest_row), OM.sort_assignments(io, E)):
+        assert np.array_equal(got.cpu().numpy(), want)
