@@ -97,204 +97,6 @@ attn_delta_kernel(const T *__restrict__ dout, const T *__restrict__ out, float *
   }
 }
 
-// ---- dK, dV ---------------------------------------------------------------------------------
-template <typename T, int D, int NW>
-__global__ void __launch_bounds__(64 * NW) attn_bwd_dkv_kernel(const AttnBwdParams p) {
-  using M = Mma<T>;
-  using Frag = typename M::Frag;
-  constexpr int BN = 32 * NW, BM = 32, NT = 64 * NW;
-  constexpr int QS = D + 16;  // row stride of the Q / dO tiles (row reads and transpose reads)
-  constexpr int VPR = D / 8;
-  constexpr int LPT = BM * VPR / NT;
-  static_assert(BM * VPR % NT == 0, "tile must divide over the block");
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-  T *sQ = reinterpret_cast<T *>(smem_raw);        // [2][BM*QS]
-  T *sdO = sQ + 2 * BM * QS;                      // [2][BM*QS]
-  float *sLse = reinterpret_cast<float *>(sdO + 2 * BM * QS);  // [2][BM]  (lse * log2e, +inf for rows >= sq)
-  float *sDel = sLse + 2 * BM;                                 // [2][BM]
-
-  const int b = seq_by_length(p.cu_q, gridDim.z, blockIdx.z);
-  const int hkv = blockIdx.y / p.hsplit, hs = blockIdx.y % p.hsplit;
-  const int q0 = p.cu_q[b], sq = p.cu_q[b + 1] - q0;
-  const int k0 = p.cu_k[b], sk = p.cu_k[b + 1] - k0;
-  const int j0 = blockIdx.x * BN;  // causal: low tiles carry the most work and come first
-  if (j0 >= sk) return;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int c = lane & 31, hh = lane >> 5;
-  const int jw0 = j0 + 32 * w;
-  const int jrow = jw0 + c;
-  const int ratio = p.hq / p.hk;
-  const int hper = ratio / p.hsplit;
-
-  Frag Kf[D / 16], Vf[D / 16];
-  {
-    const int jl = jrow < sk ? jrow : sk - 1;
-    const T *kp = reinterpret_cast<const T *>(p.k) + (int64_t)(k0 + jl) * p.k_stride + (int64_t)hkv * D;
-    const T *vp = reinterpret_cast<const T *>(p.v) + (int64_t)(k0 + jl) * p.v_stride + (int64_t)hkv * D;
-#pragma unroll
-    for (int ks = 0; ks < D / 16; ++ks) {
-      Kf[ks] = frag_ld<T>(kp + ks * 16 + 8 * hh);
-      Vf[ks] = frag_ld<T>(vp + ks * 16 + 8 * hh);
-    }
-  }
-  floatx16 dKt[D / 32], dVt[D / 32];
-#pragma unroll
-  for (int t = 0; t < D / 32; ++t)
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      dKt[t][v] = 0.f;
-      dVt[t][v] = 0.f;
-    }
-
-  const int i_begin = p.causal ? (j0 / BM) * BM : 0;
-  const int ntq = i_begin < sq ? (sq - i_begin + BM - 1) / BM : 0;
-  const int nsteps = ntq * hper;
-
-  uint4 rq[LPT], rdo[LPT];
-  float rl = 0.f, rd = 0.f;
-  auto gload = [&](int step) {
-    const int g = step / ntq, ti = step % ntq;
-    const int h = hkv * ratio + hs * hper + g;
-    const int i0 = i_begin + ti * BM;
-    const T *qg = reinterpret_cast<const T *>(p.q) + (int64_t)q0 * p.q_stride + (int64_t)h * D;
-    const T *dg = reinterpret_cast<const T *>(p.dout) + (int64_t)q0 * p.do_stride + (int64_t)h * D;
-#pragma unroll
-    for (int i = 0; i < LPT; ++i) {
-      const int idx = tid + i * NT;
-      const int r = idx / VPR, cv = idx % VPR;
-      const int ir = i0 + r;
-      if (ir < sq) {
-        rq[i] = *reinterpret_cast<const uint4 *>(qg + (int64_t)ir * p.q_stride + cv * 8);
-        rdo[i] = *reinterpret_cast<const uint4 *>(dg + (int64_t)ir * p.do_stride + cv * 8);
-      } else {
-        rq[i] = make_uint4(0, 0, 0, 0);
-        rdo[i] = make_uint4(0, 0, 0, 0);
-      }
-    }
-    if (tid < BM) {
-      const int ir = i0 + tid;
-      if (ir < sq) {
-        rl = p.lse[((int64_t)b * p.hq + h) * p.max_sq + ir] * 1.4426950408889634f;
-        rd = p.delta[((int64_t)b * p.hq + h) * p.max_sq + ir];
-      } else {
-        rl = INFINITY;
-        rd = 0.f;
-      }
-    }
-  };
-  auto sstore = [&](int st) {
-#pragma unroll
-    for (int i = 0; i < LPT; ++i) {
-      const int idx = tid + i * NT;
-      const int r = idx / VPR, cv = idx % VPR;
-      *reinterpret_cast<uint4 *>(sQ + st * BM * QS + r * QS + cv * 8) = rq[i];
-      *reinterpret_cast<uint4 *>(sdO + st * BM * QS + r * QS + cv * 8) = rdo[i];
-    }
-    if (tid < BM) {
-      sLse[st * BM + tid] = rl;
-      sDel[st * BM + tid] = rd;
-    }
-  };
-
-  if (nsteps > 0) {
-    gload(0);
-    sstore(0);
-  }
-  __syncthreads();
-
-  for (int step = 0; step < nsteps; ++step) {
-    const int st = step & 1;
-    if (step + 1 < nsteps) gload(step + 1);
-    const int i0 = i_begin + (step % ntq) * BM;
-    // causal: the whole 32-row query block lies above this wavefront's keys -> nothing to add
-    const bool skip = p.causal && i0 + BM - 1 < jw0;
-    if (!skip) {
-      const T *tQ = sQ + st * BM * QS;
-      const T *tdO = sdO + st * BM * QS;
-      floatx16 S, dP;
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        S[v] = 0.f;
-        dP[v] = 0.f;
-      }
-#pragma unroll
-      for (int ks = 0; ks < D / 16; ++ks) {
-        const Frag aq = frag_ld<T>(tQ + c * QS + ks * 16 + 8 * hh);
-        S = M::mma(aq, Kf[ks], S);
-        const Frag ad = frag_ld<T>(tdO + c * QS + ks * 16 + 8 * hh);
-        dP = M::mma(ad, Vf[ks], dP);
-      }
-      const bool need_mask = p.causal && i0 < jw0 + 31;
-      float pv[16], dsv[16];
-#pragma unroll
-      for (int vb = 0; vb < 4; ++vb) {
-        const float4 l4 = *reinterpret_cast<const float4 *>(sLse + st * BM + 8 * vb + 4 * hh);
-        const float4 d4 = *reinterpret_cast<const float4 *>(sDel + st * BM + 8 * vb + 4 * hh);
-        const float ls[4] = {l4.x, l4.y, l4.z, l4.w};
-        const float dl[4] = {d4.x, d4.y, d4.z, d4.w};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int v = 4 * vb + e;
-          float pe = fast_exp2(S[v] * p.scale_log2 - ls[e]);
-          if (need_mask && jrow > i0 + acc_row(v, hh)) pe = 0.f;
-          pv[v] = pe;
-          dsv[v] = pe * (dP[v] - dl[e]);
-        }
-      }
-      Frag Pb[2], dSb[2];
-      Pb[0] = frag_pack<T>(pv);
-      Pb[1] = frag_pack<T>(pv + 8);
-      dSb[0] = frag_pack<T>(dsv);
-      dSb[1] = frag_pack<T>(dsv + 8);
-#pragma unroll
-      for (int s = 0; s < 2; ++s) {
-#pragma unroll
-        for (int t = 0; t < D / 32; ++t) {
-          const int n0 = 32 * t + 16 * ((lane >> 4) & 1);
-          const Frag ad = frag_ld_tr<T>(tdO, QS, 16 * s + 4 * hh, 16 * s + 8 + 4 * hh, n0, lane);
-          dVt[t] = M::mma(ad, Pb[s], dVt[t]);
-          const Frag aq = frag_ld_tr<T>(tQ, QS, 16 * s + 4 * hh, 16 * s + 8 + 4 * hh, n0, lane);
-          dKt[t] = M::mma(aq, dSb[s], dKt[t]);
-        }
-      }
-    }
-    if (step + 1 < nsteps) sstore(st ^ 1);
-    __syncthreads();
-  }
-
-  if (jrow < sk) {
-    if (p.hsplit == 1) {
-      T *dkp = reinterpret_cast<T *>(p.dk) + (int64_t)(k0 + jrow) * p.dk_stride + (int64_t)hkv * D;
-      T *dvp = reinterpret_cast<T *>(p.dv) + (int64_t)(k0 + jrow) * p.dv_stride + (int64_t)hkv * D;
-#pragma unroll
-      for (int t = 0; t < D / 32; ++t)
-#pragma unroll
-        for (int vb = 0; vb < 4; ++vb) {
-          struct alignas(8) { T v[4]; } a, bq;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            a.v[e] = static_cast<T>(dKt[t][4 * vb + e] * p.scale);
-            bq.v[e] = static_cast<T>(dVt[t][4 * vb + e]);
-          }
-          *reinterpret_cast<decltype(a) *>(dkp + 32 * t + 8 * vb + 4 * hh) = a;
-          *reinterpret_cast<decltype(bq) *>(dvp + 32 * t + 8 * vb + 4 * hh) = bq;
-        }
-    } else {
-      const int64_t off = (((int64_t)hs * p.total_k + (k0 + jrow)) * p.hk + hkv) * D;
-#pragma unroll
-      for (int t = 0; t < D / 32; ++t)
-#pragma unroll
-        for (int vb = 0; vb < 4; ++vb) {
-          *reinterpret_cast<float4 *>(p.dk_part + off + 32 * t + 8 * vb + 4 * hh) =
-              make_float4(dKt[t][4 * vb] * p.scale, dKt[t][4 * vb + 1] * p.scale, dKt[t][4 * vb + 2] * p.scale,
-                          dKt[t][4 * vb + 3] * p.scale);
-          *reinterpret_cast<float4 *>(p.dv_part + off + 32 * t + 8 * vb + 4 * hh) =
-              make_float4(dVt[t][4 * vb], dVt[t][4 * vb + 1], dVt[t][4 * vb + 2], dVt[t][4 * vb + 3]);
-        }
-    }
-  }
-}
-
 // Sum of the head-split partials, in split order: part fp32 [hsplit][total_k][hk][d] -> dst (T, strided rows).
 template <typename T>
 __global__ void __launch_bounds__(256)
@@ -323,161 +125,8 @@ attn_bwd_gqa_sum_kernel(const float *__restrict__ dk_part, const float *__restri
   }
 }
 
-// ---- dQ ---------------------------------------------------------------------------------------
-template <typename T, int D, int NW>
-__global__ void __launch_bounds__(64 * NW) attn_bwd_dq_kernel(const AttnBwdParams p) {
-  using M = Mma<T>;
-  using Frag = typename M::Frag;
-  constexpr int BM = 32 * NW, BN = 32, NT = 64 * NW;
-  constexpr int KS = D + 16;  // K tile: row reads and transpose reads
-  constexpr int VS = D + 8;   // V tile: row reads only
-  constexpr int VPR = D / 8;
-  constexpr int LPT = BN * VPR / NT;
-  static_assert(BN * VPR % NT == 0, "tile must divide over the block");
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-  T *sK = reinterpret_cast<T *>(smem_raw);  // [2][BN*KS]
-  T *sV = sK + 2 * BN * KS;                 // [2][BN*VS]
-
-  const int b = seq_by_length(p.cu_q, gridDim.z, blockIdx.z), h = blockIdx.y;
-  const int mt = gridDim.x - 1 - blockIdx.x;
-  const int q0 = p.cu_q[b], sq = p.cu_q[b + 1] - q0;
-  const int k0 = p.cu_k[b], sk = p.cu_k[b + 1] - k0;
-  const int m0 = mt * BM;
-  if (m0 >= sq) return;
-  const int hkv = h / (p.hq / p.hk);
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int c = lane & 31, hh = lane >> 5;
-  const int wrow0 = m0 + w * 32;
-  const int row_q = wrow0 + c;
-  const bool row_ok = row_q < sq;
-  const int row_ld = row_ok ? row_q : sq - 1;
-
-  Frag Qf[D / 16], dOf[D / 16];
-  {
-    const T *qp = reinterpret_cast<const T *>(p.q) + (int64_t)(q0 + row_ld) * p.q_stride + (int64_t)h * D;
-    const T *dp = reinterpret_cast<const T *>(p.dout) + (int64_t)(q0 + row_ld) * p.do_stride + (int64_t)h * D;
-#pragma unroll
-    for (int ks = 0; ks < D / 16; ++ks) {
-      Qf[ks] = frag_ld<T>(qp + ks * 16 + 8 * hh);
-      dOf[ks] = frag_ld<T>(dp + ks * 16 + 8 * hh);
-    }
-  }
-  const float lse_c = row_ok ? p.lse[((int64_t)b * p.hq + h) * p.max_sq + row_q] * 1.4426950408889634f : INFINITY;
-  const float del_c = row_ok ? p.delta[((int64_t)b * p.hq + h) * p.max_sq + row_q] : 0.f;
-
-  const T *kg = reinterpret_cast<const T *>(p.k) + (int64_t)k0 * p.k_stride + (int64_t)hkv * D;
-  const T *vg = reinterpret_cast<const T *>(p.v) + (int64_t)k0 * p.v_stride + (int64_t)hkv * D;
-  int nk_end = sk;
-  if (p.causal && m0 + BM < nk_end) nk_end = m0 + BM;
-  const int ntiles = (nk_end + BN - 1) / BN;
-
-  floatx16 dQt[D / 32];
-#pragma unroll
-  for (int t = 0; t < D / 32; ++t)
-#pragma unroll
-    for (int v = 0; v < 16; ++v) dQt[t][v] = 0.f;
-
-  uint4 rk[LPT], rv[LPT];
-  auto gload = [&](int n0) {
-#pragma unroll
-    for (int i = 0; i < LPT; ++i) {
-      const int idx = tid + i * NT;
-      const int r = idx / VPR, cv = idx % VPR;
-      const int kr = n0 + r;
-      if (kr < sk) {
-        rk[i] = *reinterpret_cast<const uint4 *>(kg + (int64_t)kr * p.k_stride + cv * 8);
-        rv[i] = *reinterpret_cast<const uint4 *>(vg + (int64_t)kr * p.v_stride + cv * 8);
-      } else {
-        rk[i] = make_uint4(0, 0, 0, 0);
-        rv[i] = make_uint4(0, 0, 0, 0);
-      }
-    }
-  };
-  auto sstore = [&](int st) {
-#pragma unroll
-    for (int i = 0; i < LPT; ++i) {
-      const int idx = tid + i * NT;
-      const int r = idx / VPR, cv = idx % VPR;
-      *reinterpret_cast<uint4 *>(sK + st * BN * KS + r * KS + cv * 8) = rk[i];
-      *reinterpret_cast<uint4 *>(sV + st * BN * VS + r * VS + cv * 8) = rv[i];
-    }
-  };
-  if (ntiles > 0) {
-    gload(0);
-    sstore(0);
-  }
-  __syncthreads();
-
-  for (int it = 0; it < ntiles; ++it) {
-    const int n0 = it * BN;
-    const int st = it & 1;
-    if (it + 1 < ntiles) gload(n0 + BN);
-    const bool skip = p.causal && n0 > wrow0 + 31;
-    if (!skip) {
-      const T *tK = sK + st * BN * KS;
-      const T *tV = sV + st * BN * VS;
-      floatx16 S, dP;
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        S[v] = 0.f;
-        dP[v] = 0.f;
-      }
-#pragma unroll
-      for (int ks = 0; ks < D / 16; ++ks) {
-        const Frag ak = frag_ld<T>(tK + c * KS + ks * 16 + 8 * hh);
-        S = M::mma(ak, Qf[ks], S);
-        const Frag av = frag_ld<T>(tV + c * VS + ks * 16 + 8 * hh);
-        dP = M::mma(av, dOf[ks], dP);
-      }
-      const bool need_mask = (p.causal && n0 + BN - 1 > wrow0) || (n0 + BN > sk);
-      float dsv[16];
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        float pe = fast_exp2(S[v] * p.scale_log2 - lse_c);
-        if (need_mask) {
-          const int kv = n0 + acc_row(v, hh);
-          if (kv >= sk || (p.causal && kv > row_q)) pe = 0.f;
-        }
-        dsv[v] = pe * (dP[v] - del_c);
-      }
-      Frag dSb[2];
-      dSb[0] = frag_pack<T>(dsv);
-      dSb[1] = frag_pack<T>(dsv + 8);
-#pragma unroll
-      for (int s = 0; s < 2; ++s) {
-#pragma unroll
-        for (int t = 0; t < D / 32; ++t) {
-          const Frag ak = frag_ld_tr<T>(tK, KS, 16 * s + 4 * hh, 16 * s + 8 + 4 * hh, 32 * t + 16 * ((lane >> 4) & 1), lane);
-          dQt[t] = M::mma(ak, dSb[s], dQt[t]);
-        }
-      }
-    }
-    if (it + 1 < ntiles) sstore(st ^ 1);
-    __syncthreads();
-  }
-
-  if (row_ok) {
-    T *dqp = reinterpret_cast<T *>(p.dq) + (int64_t)(q0 + row_q) * p.dq_stride + (int64_t)h * D;
-#pragma unroll
-    for (int t = 0; t < D / 32; ++t)
-#pragma unroll
-      for (int vb = 0; vb < 4; ++vb) {
-        struct alignas(8) { T v[4]; } a;
-        if (p.dq_accumulate) {
-          a = *reinterpret_cast<const decltype(a) *>(dqp + 32 * t + 8 * vb + 4 * hh);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) a.v[e] = static_cast<T>(static_cast<float>(a.v[e]) + dQt[t][4 * vb + e] * p.scale);
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) a.v[e] = static_cast<T>(dQt[t][4 * vb + e] * p.scale);
-        }
-        *reinterpret_cast<decltype(a) *>(dqp + 32 * t + 8 * vb + 4 * hh) = a;
-      }
-  }
-}
-
 // ---------------------------------------------------------------------------------------------
-// Head dim 128, second-generation kernels: direct global->LDS copies into swizzled tiles
+// Head dim 128: direct global->LDS copies into swizzled tiles
 // (no staging registers, no bank conflicts), two pipeline stages held in separate LDS
 // objects, causal work made uniform by pairing tile i with tile n-1-i.
 // ---------------------------------------------------------------------------------------------
@@ -1405,7 +1054,7 @@ static int launch_dkv_d128(const AttnBwdParams &p, int batch, int max_sk, hipStr
 
 }  // namespace dh
 
-#include "attn_bwd_d64.h"
+#include "attn_bwd_tile.h"
 
 namespace dh {
 
@@ -1424,26 +1073,6 @@ static int pick_hsplit(int max_sk, int batch, int hq, int hk, int bn) {
 }
 
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
-
-template <typename T, int D, int NW>
-static int launch_dkv(const AttnBwdParams &p, int batch, int max_sk, hipStream_t st) {
-  constexpr int BN = 32 * NW, BM = 32;
-  constexpr size_t smem = 2 * 2 * BM * (D + 16) * sizeof(T) + 4 * BM * sizeof(float);
-  DH_MAX_DYNAMIC_LDS_PER_DEVICE((&attn_bwd_dkv_kernel<T, D, NW>), smem);
-  dim3 grid((unsigned)cdiv(max_sk, BN), (unsigned)(p.hk * p.hsplit), (unsigned)batch);
-  hipLaunchKernelGGL((attn_bwd_dkv_kernel<T, D, NW>), grid, dim3(64 * NW), smem, st, p);
-  return DH_OK;
-}
-
-template <typename T, int D, int NW>
-static int launch_dq(const AttnBwdParams &p, int batch, hipStream_t st) {
-  constexpr int BM = 32 * NW, BN = 32;
-  constexpr size_t smem = 2 * BN * ((D + 16) + (D + 8)) * sizeof(T);
-  DH_MAX_DYNAMIC_LDS_PER_DEVICE((&attn_bwd_dq_kernel<T, D, NW>), smem);
-  dim3 grid((unsigned)cdiv(p.max_sq, BM), (unsigned)p.hq, (unsigned)batch);
-  hipLaunchKernelGGL((attn_bwd_dq_kernel<T, D, NW>), grid, dim3(64 * NW), smem, st, p);
-  return DH_OK;
-}
 
 template <typename T>
 static int launch_delta(const void *dout, const void *out, float *delta, const float *lse, float *ld2, int64_t ld2_plane,
@@ -1468,9 +1097,7 @@ int attn_bwd_f32(const void *dout, const void *q, const void *k, const void *v, 
                  int64_t do_stride, int64_t dq_stride, int64_t dk_stride, int64_t dv_stride, float scale, int causal,
                  int dq_accumulate, hipStream_t st);
 
-constexpr int DKV_NW = 2;  // wavefronts per dK/dV workgroup (64 key rows)
-// the dQ kernel's 32-key tile must divide evenly over the workgroup's threads (head dim 96 does not over 256)
-constexpr bool dq_takes_4_waves(int d) { return (32 * (d / 8)) % 256 == 0; }
+constexpr int DKV_ROWS = 64;  // key rows of a dK/dV workgroup
 
 // Keeping dS for the dQ product costs 2 bytes per (head, query, key) of workspace, written once and read once.
 // It pays where the recomputing dQ kernel runs its small-grid form (fewer than 256 workgroups of 128 query rows:
@@ -1491,18 +1118,21 @@ template <typename T, int D>
 static int bwd_passes(const AttnBwdParams &p, int batch, int max_sq, int max_sk, hipStream_t st) {
   const bool small_q = cdiv(max_sq, 128) * p.hq * batch < 2 * 256;
   int rc = DH_OK;
-  // recomputing dQ kernels that form delta run first
-  if constexpr (D == 64) {
-    if (max_sq > 0) rc = small_q ? launch_dq_d64<T, 2, 4>(p, batch, st) : launch_dq_d64<T, 4, 2>(p, batch, st);
-  }
-  if constexpr (D == 128) {
-    if (max_sq > 0 && !p.ds)
-      rc = dq_big_grid(batch, max_sq, p.hq, p.causal) ? launch_dq_d128<T, 4, 2, 32>(p, batch, st) : launch_dq_d128<T, 2, 4, 32>(p, batch, st);
+  // recomputing dQ kernels form delta and run first
+  if (max_sq > 0) {
+    if constexpr (D == 128) {
+      if (!p.ds)
+        rc = dq_big_grid(batch, max_sq, p.hq, p.causal) ? launch_dq_d128<T, 4, 2, 32>(p, batch, st) : launch_dq_d128<T, 2, 4, 32>(p, batch, st);
+    } else if constexpr (D < 128) {
+      rc = small_q ? launch_dq_tile<T, D, 2, 4, 2>(p, batch, st) : launch_dq_tile<T, D, 4, 2, D == 64 ? 4 : 2>(p, batch, st);
+    } else {
+      rc = launch_dq_tile<T, D, 2, 2, 1>(p, batch, st);
+    }
   }
   if (rc == DH_OK && max_sk > 0) {
-    if constexpr (D == 64) rc = launch_dkv_d64<T, 2, 4>(p, batch, max_sk, st);
-    else if constexpr (D == 128) rc = launch_dkv_d128<T>(p, batch, max_sk, st);
-    else rc = launch_dkv<T, D, DKV_NW>(p, batch, max_sk, st);
+    if constexpr (D == 128) rc = launch_dkv_d128<T>(p, batch, max_sk, st);
+    else if constexpr (D < 128) rc = launch_dkv_tile<T, D, 2, 4, 2>(p, batch, max_sk, st);
+    else rc = launch_dkv_tile<T, D, 2, 2, 1>(p, batch, max_sk, st);
   }
   if (rc == DH_OK && p.hsplit > 1 && p.total_k > 0) {
     int64_t blocks = cdiv(p.total_k * p.hk * (D / 4), 256);
@@ -1510,13 +1140,8 @@ static int bwd_passes(const AttnBwdParams &p, int batch, int max_sq, int max_sk,
     hipLaunchKernelGGL((attn_bwd_gqa_sum_kernel<T>), dim3((unsigned)blocks), dim3(256), 0, st, p.dk_part, p.dv_part, (T *)p.dk,
                        (T *)p.dv, p.total_k, p.hk, D, p.hsplit, p.dk_stride, p.dv_stride);
   }
-  if (rc == DH_OK && max_sq > 0) {
-    if constexpr (D == 128) {
-      if (p.ds) rc = launch_dq2_d128<T>(p, batch, st);
-    } else if constexpr (D != 64) {
-      if (small_q || !dq_takes_4_waves(D)) rc = launch_dq<T, D, 2>(p, batch, st);
-      else rc = launch_dq<T, D, dq_takes_4_waves(D) ? 4 : 2>(p, batch, st);
-    }
+  if constexpr (D == 128) {
+    if (rc == DH_OK && max_sq > 0 && p.ds) rc = launch_dq2_d128<T>(p, batch, st);
   }
   return rc;
 }
@@ -1542,7 +1167,7 @@ static size_t ds_bytes(int batch, int max_sq, int64_t max_sk, int hq, int d, int
 static size_t bwd_base_bytes(int64_t total_k, int batch, int max_seqlen_q, int hq, int hk, int d, int dtype) {
   const size_t sq = (size_t)(max_seqlen_q > 0 ? max_seqlen_q : 0);
   size_t n = align256((size_t)batch * hq * sq * sizeof(float));            // delta
-  if (dtype != DH_F32 && (d == 128 || d == 64)) n += 2 * align256((size_t)batch * hq * ((sq + 31) / 32 * 32) * sizeof(float));
+  if (dtype != DH_F32) n += 2 * align256((size_t)batch * hq * ((sq + 31) / 32 * 32) * sizeof(float));
   if (dtype != DH_F32 && hk > 0 && hq / hk > 1)
     n += 2 * align256((size_t)(hq / hk) * (size_t)total_k * hk * d * sizeof(float));
   return n + 256;                                                          // the base pointer is rounded up to 256
@@ -1594,7 +1219,7 @@ static int attn_bwd_entry(const void *dout, const void *q, const void *k, const 
   float *ld2 = nullptr;
   const int ld2_pitch = (max_seqlen_q + 31) / 32 * 32;
   const size_t plane2 = align256((size_t)batch * hq * (size_t)ld2_pitch * sizeof(float));
-  if (dtype != DH_F32 && (d == 128 || d == 64)) {
+  if (dtype != DH_F32) {
     ld2 = (float *)ws;
     ws += 2 * plane2;
     DH_CHECK(plane2 < (1ull << 31), "batch * heads * max_seqlen_q too large");
@@ -1606,14 +1231,14 @@ static int attn_bwd_entry(const void *dout, const void *q, const void *k, const 
            "dout/out rows must be 16-byte aligned");
   // head dim 128 in 16 bits, two ways: with room for dS in the workspace the dK/dV kernel keeps it and dQ is one
   // product over it (delta from the delta kernel, which runs first); otherwise the dQ kernel recomputes S and dP,
-  // forms delta itself and runs first.  Everything else uses the delta kernel.
+  // forms delta itself and runs first.  fp32 uses the delta kernel.
   // dS is kept only if the blocks fit behind everything else in the workspace THIS call was given (and under the
   // process-wide limit); they take the tail of the workspace
   size_t dsb = ds_bytes(batch, max_seqlen_q, total_k, hq, d, dtype, causal);
   if (dsb > 0 && base_bytes + align256(dsb) > workspace_bytes) dsb = 0;
   const bool keep_ds = dsb > 0 && max_seqlen_k > 0;
   uint8_t *ds_ws = (uint8_t *)(((uintptr_t)workspace + 255) & ~(uintptr_t)255) + (base_bytes - 256);
-  const bool delta_in_dq = dtype != DH_F32 && (d == 64 || (d == 128 && !keep_ds));
+  const bool delta_in_dq = dtype != DH_F32 && !keep_ds;
   if (max_seqlen_q > 0 && !delta_in_dq) {
     DH_DISPATCH_DTYPE(dtype, {
       launch_delta<T>(dout, out, delta, lse, ld2, (int64_t)(plane2 / sizeof(float)), ld2_pitch, cu_seqlens_q, batch, max_seqlen_q, hq, d,
@@ -1650,7 +1275,7 @@ static int attn_bwd_entry(const void *dout, const void *q, const void *k, const 
   p.ds = keep_ds ? (void *)ds_ws : nullptr;
   p.ds_nqt = 2 * (int)cdiv(max_seqlen_q, 64);
   p.ds_nkb = 2 * (int)cdiv(max_seqlen_k < total_k ? max_seqlen_k : total_k, 64) + 1;
-  p.hsplit = pick_hsplit(d == 128 && causal ? (max_seqlen_k + 1) / 2 : max_seqlen_k, batch, hq, hk, 32 * DKV_NW);
+  p.hsplit = pick_hsplit(d == 128 && causal ? (max_seqlen_k + 1) / 2 : max_seqlen_k, batch, hq, hk, DKV_ROWS);
   p.dk_part = nullptr;
   p.dv_part = nullptr;
   if (p.hsplit > 1) {

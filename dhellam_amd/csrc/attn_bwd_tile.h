@@ -4,21 +4,21 @@
 // dK/dV keeps K and V fragments and both accumulators in registers (202): two wavefronts a SIMD.
 // Measured against the register-staged kernels: 2 x 512 rows, 16 heads, delta + dQ 28.6 -> 11.5 us, dK/dV 31.3 -> 13.9 us;
 // larger shapes in attn_fwd_d64.h.
-#include "attn_d64.h"
+#include "attn_tile.h"
 
 namespace dh {
 
 // dQ: RG row groups of 32 query rows x SPLIT splits of the keys, 32-key tiles of K and V.
-template <typename T, int RG, int SPLIT>
-__global__ void __launch_bounds__(512, RG == 4 ? 4 : 2) attn_bwd_dq_d64_kernel(const AttnBwdParams p) {
+template <typename T, int D, int RG, int SPLIT, int WPS>
+__global__ void __launch_bounds__(64 * RG * SPLIT, WPS) attn_bwd_dq_tile_kernel(const AttnBwdParams p) {
   using M = Mma<T>;
   using Frag = typename M::Frag;
-  static_assert(RG * SPLIT == 8, "8 wavefronts per workgroup");
-  constexpr int D = 64, BM = 32 * RG, BN = 32;
+  constexpr int BM = 32 * RG, BN = 32, NW = RG * SPLIT, SLOTF = 32 * D;
   constexpr int TILEB = BN * D * (int)sizeof(T);
   constexpr int STAGEB = SPLIT * 2 * TILEB;
-  constexpr int CB = SPLIT * 2 * (BN / 8) / 8;            // copy blocks per wavefront and iteration: 4 or 2
-  constexpr int EXB = (SPLIT - 1) * RG * 8192;
+  constexpr int RPW = SPLIT * 2 * BN / NW;                // rows that a wavefront copies per iteration
+  constexpr int EXB = (SPLIT - 1) * RG * SLOTF * 4;
+  static_assert(RPW % 16 == 0 && RPW <= BN, "whole copy patterns of one tile per wavefront");
   constexpr int LDSB = 2 * STAGEB > EXB ? 2 * STAGEB : EXB;
   __shared__ __attribute__((aligned(1024))) char sAll[LDSB];
   __shared__ float sDel[32 * RG];
@@ -41,12 +41,12 @@ __global__ void __launch_bounds__(512, RG == 4 ? 4 : 2) attn_bwd_dq_d64_kernel(c
   const int rg = w % RG, sp = w / RG;
   const uint32_t lds0 = (uint32_t)(uintptr_t)sAll;
 
-  // copies of this wavefront: rows cp_r0 .. + 8 CB - 1 of the K or V tile of split cp_sp
-  constexpr int PARTS = BN / (8 * CB);
-  const int cp_r0 = 8 * CB * (w % PARTS), cp_v = (w / PARTS) & 1, cp_sp = w / (2 * PARTS);
+  // copies of this wavefront: rows cp_r0 .. + RPW - 1 of the K or V tile of split cp_sp
+  constexpr int PARTS = BN / RPW;
+  const int cp_r0 = RPW * (w % PARTS), cp_v = (w / PARTS) & 1, cp_sp = w / (2 * PARTS);
   const int64_t cp_stride = cp_v ? p.v_stride : p.k_stride;
   const T *cp_g = reinterpret_cast<const T *>(cp_v ? p.v : p.k) + (int64_t)k0 * cp_stride + (int64_t)hkv * D;
-  const Copy64 cl = copy64_lane(lane, (uint32_t)(cp_stride * (int64_t)sizeof(T)));
+  const TileCopy<D> cl = tile_copy<D>(lane, (uint32_t)(cp_stride * (int64_t)sizeof(T)));
   const uint32_t cp_dst = lds0 + (uint32_t)(cp_v * SPLIT * TILEB + cp_sp * TILEB + cp_r0 * D * (int)sizeof(T));
 
   int nk_end = sk;
@@ -55,7 +55,7 @@ __global__ void __launch_bounds__(512, RG == 4 ? 4 : 2) attn_bwd_dq_d64_kernel(c
   const int niter = (ntiles + SPLIT - 1) / SPLIT;
   auto issue = [&](int it) {
     const int tile = it * SPLIT + cp_sp;
-    if (tile < ntiles) copy64<T, CB>(cp_g, cp_stride, tile * BN + cp_r0, sk, cp_dst + (uint32_t)((it & 1) * STAGEB), cl);
+    if (tile < ntiles) copy_tile<T, D, RPW>(cp_g, cp_stride, tile * BN + cp_r0, sk, cp_dst + (uint32_t)((it & 1) * STAGEB), cl, lane);
   };
   if (niter > 0) issue(0);
 
@@ -94,8 +94,8 @@ __global__ void __launch_bounds__(512, RG == 4 ? 4 : 2) attn_bwd_dq_d64_kernel(c
       }
     }
   }
-  const uint32_t k_lane = lds0 + (uint32_t)(sp * TILEB) + row64_lane(lane);
-  const uint32_t ta_lane = lds0 + (uint32_t)(sp * TILEB) + tr64_lane(lane);
+  const RowLane rl = row_lane<D>(lane);
+  const TrLane tl = tr_lane<D>(lane);
 
   floatx16 dQt[D / 32];
 #pragma unroll
@@ -111,8 +111,7 @@ __global__ void __launch_bounds__(512, RG == 4 ? 4 : 2) attn_bwd_dq_d64_kernel(c
     if (it + 1 < niter) issue(it + 1);
     const int tile = it * SPLIT + sp, n0 = tile * BN;
     if (tile < ntiles && !(causal && n0 > wrow0 + 31)) {
-      const uint32_t st = (uint32_t)((it & 1) * STAGEB);
-      const uint32_t kb = k_lane + st, ta = ta_lane + st, tb = tr64_next(ta);
+      const uint32_t kt = lds0 + (uint32_t)((it & 1) * STAGEB + sp * TILEB);
       floatx16 S, dP;
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
@@ -121,8 +120,8 @@ __global__ void __launch_bounds__(512, RG == 4 ? 4 : 2) attn_bwd_dq_d64_kernel(c
       }
 #pragma unroll
       for (int ks = 0; ks < D / 16; ++ks) {
-        S = M::mma(row64<T>(kb ^ (uint32_t)(ks << 5)), Qf[ks], S);
-        dP = M::mma(row64<T>((kb ^ (uint32_t)(ks << 5)) + (uint32_t)(SPLIT * TILEB)), dOf[ks], dP);
+        S = M::mma(row_frag<T, D>(kt, rl, ks), Qf[ks], S);
+        dP = M::mma(row_frag<T, D>(kt + (uint32_t)(SPLIT * TILEB), rl, ks), dOf[ks], dP);
       }
       if ((causal && n0 + BN - 1 > wrow0) || n0 + BN > sk) {
         const int lim = causal && row_q + 1 < sk ? row_q + 1 : sk;
@@ -137,20 +136,20 @@ __global__ void __launch_bounds__(512, RG == 4 ? 4 : 2) attn_bwd_dq_d64_kernel(c
         const Frag dSb = frag_pack<T>(ds);
 #pragma unroll
         for (int t = 0; t < D / 32; ++t)
-          dQt[t] = M::mma(tr64<T>((ta ^ (uint32_t)(t << 6)) + 2048u * s, (tb ^ (uint32_t)(t << 6)) + 2048u * s), dSb, dQt[t]);
+          dQt[t] = M::mma(tr_frag<T, D>(kt, tl, t, s), dSb, dQt[t]);
       }
     }
     dma_wait_all();
     __syncthreads();
   }
 
-  // add the splits' partial dQ through LDS, in split order: slot x = (split - 1) * RG + row group, 8 KB each
+  // add the splits' partial dQ through LDS, in split order: slot x = (split - 1) * RG + row group
   float *xo = reinterpret_cast<float *>(sAll);
   if (sp > 0) {
 #pragma unroll
     for (int t = 0; t < D / 32; ++t)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) xo[((sp - 1) * RG + rg) * 2048 + (t * 16 + v) * 64 + lane] = dQt[t][v];
+      for (int v = 0; v < 16; ++v) xo[((sp - 1) * RG + rg) * SLOTF + (t * 16 + v) * 64 + lane] = dQt[t][v];
   }
   __syncthreads();
   if (sp > 0 || !row_ok) return;
@@ -159,7 +158,7 @@ __global__ void __launch_bounds__(512, RG == 4 ? 4 : 2) attn_bwd_dq_d64_kernel(c
 #pragma unroll
     for (int t = 0; t < D / 32; ++t)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) dQt[t][v] += xo[((s2 - 1) * RG + rg) * 2048 + (t * 16 + v) * 64 + lane];
+      for (int v = 0; v < 16; ++v) dQt[t][v] += xo[((s2 - 1) * RG + rg) * SLOTF + (t * 16 + v) * 64 + lane];
   T *dqp = reinterpret_cast<T *>(p.dq) + (int64_t)(q0 + row_q) * p.dq_stride + (int64_t)h * D;
 #pragma unroll
   for (int t = 0; t < D / 32; ++t)
@@ -176,15 +175,14 @@ __global__ void __launch_bounds__(512, RG == 4 ? 4 : 2) attn_bwd_dq_d64_kernel(c
 
 // dK, dV: KG row groups of 32 key rows x QSPLIT splits of the query tiles (32 rows of Q and dO each); K and V row
 // fragments stay in registers, lse / delta come straight from the planes that the dQ kernel wrote.
-template <typename T, int KG, int QSPLIT>
-__global__ void __launch_bounds__(64 * KG * QSPLIT, 2) attn_bwd_dkv_d64_kernel(const AttnBwdParams p) {
+template <typename T, int D, int KG, int QSPLIT, int WPS>
+__global__ void __launch_bounds__(64 * KG * QSPLIT, WPS) attn_bwd_dkv_tile_kernel(const AttnBwdParams p) {
   using M = Mma<T>;
   using Frag = typename M::Frag;
-  constexpr int D = 64, BN = 32 * KG, BM = 32, NW = KG * QSPLIT;
+  constexpr int BN = 32 * KG, BM = 32, NW = KG * QSPLIT, SLOTF = 32 * D;
   constexpr int TILEB = BM * D * (int)sizeof(T);          // bytes of one Q (or dO) tile
   constexpr int STAGEB = QSPLIT * 2 * TILEB;              // per split: Q tile, dO tile
-  constexpr int CB = QSPLIT * 2 * 4 / NW;                 // copy blocks per wavefront and iteration
-  static_assert(CB == 4 && QSPLIT * 2 == NW, "one whole tile per wavefront");
+  static_assert(QSPLIT * 2 == NW, "one whole tile per wavefront");
   __shared__ __attribute__((aligned(1024))) char sAll[2 * STAGEB];
 
   const int b = seq_by_length(p.cu_k, gridDim.y, blockIdx.y);
@@ -211,7 +209,7 @@ __global__ void __launch_bounds__(64 * KG * QSPLIT, 2) attn_bwd_dkv_d64_kernel(c
   const int cp_do = w & 1, cp_sp = w >> 1;
   const int64_t cp_stride = cp_do ? p.do_stride : p.q_stride;
   const T *cp_g = reinterpret_cast<const T *>(cp_do ? p.dout : p.q) + (int64_t)q0 * cp_stride;
-  const Copy64 cl = copy64_lane(lane, (uint32_t)(cp_stride * (int64_t)sizeof(T)));
+  const TileCopy<D> cl = tile_copy<D>(lane, (uint32_t)(cp_stride * (int64_t)sizeof(T)));
   const uint32_t cp_dst = lds0 + (uint32_t)((cp_sp * 2 + cp_do) * TILEB);
 
   const int i_begin = causal ? j0 : 0;
@@ -221,7 +219,7 @@ __global__ void __launch_bounds__(64 * KG * QSPLIT, 2) attn_bwd_dkv_d64_kernel(c
   auto issue = [&](int stage, int g, int ti) {
     const int tq = ti * QSPLIT + cp_sp;
     if (tq < ntq)
-      copy64<T, CB>(cp_g + (int64_t)(h_first + g) * D, cp_stride, i_begin + tq * BM, sq, cp_dst + (uint32_t)(stage * STAGEB), cl);
+      copy_tile<T, D, BM>(cp_g + (int64_t)(h_first + g) * D, cp_stride, i_begin + tq * BM, sq, cp_dst + (uint32_t)(stage * STAGEB), cl, lane);
   };
   if (niter > 0) issue(0, 0, 0);
 
@@ -244,8 +242,8 @@ __global__ void __launch_bounds__(64 * KG * QSPLIT, 2) attn_bwd_dkv_d64_kernel(c
       dKt[t][v] = 0.f;
       dVt[t][v] = 0.f;
     }
-  const uint32_t q_lane = lds0 + (uint32_t)(qs * 2 * TILEB) + row64_lane(lane);
-  const uint32_t ta_lane = lds0 + (uint32_t)(qs * 2 * TILEB) + tr64_lane(lane);
+  const RowLane rl = row_lane<D>(lane);
+  const TrLane tl = tr_lane<D>(lane);
   // lse (exp2 units) and delta of the rows 8 vb + 4 hh + e of this wavefront's query tile (no branch: past the last tile it
   // loads the last one's)
   floatx4 l4[4], d4[4];
@@ -276,8 +274,7 @@ __global__ void __launch_bounds__(64 * KG * QSPLIT, 2) attn_bwd_dkv_d64_kernel(c
     if (have_next) issue((it + 1) & 1, gn, tn);
     const int tq = ti * QSPLIT + qs, i0 = i_begin + tq * BM;
     if (tq < ntq && !(causal && i0 + BM - 1 < jw0)) {
-      const uint32_t st = (uint32_t)((it & 1) * STAGEB);
-      const uint32_t qb = q_lane + st, ta = ta_lane + st, tb = tr64_next(ta);
+      const uint32_t qt = lds0 + (uint32_t)((it & 1) * STAGEB + qs * 2 * TILEB), dt = qt + (uint32_t)TILEB;
       floatx16 S, dP;
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
@@ -286,8 +283,8 @@ __global__ void __launch_bounds__(64 * KG * QSPLIT, 2) attn_bwd_dkv_d64_kernel(c
       }
 #pragma unroll
       for (int ks = 0; ks < D / 16; ++ks) {
-        S = M::mma(row64<T>(qb ^ (uint32_t)(ks << 5)), Kf[ks], S);
-        dP = M::mma(row64<T>((qb ^ (uint32_t)(ks << 5)) + (uint32_t)TILEB), Vf[ks], dP);
+        S = M::mma(row_frag<T, D>(qt, rl, ks), Kf[ks], S);
+        dP = M::mma(row_frag<T, D>(dt, rl, ks), Vf[ks], dP);
       }
       if ((causal && i0 < jw0 + 31) || i0 + BM > sq) {
         const int lo = causal ? jrow : 0;           // first query row that attends to this lane's key
@@ -314,9 +311,8 @@ __global__ void __launch_bounds__(64 * KG * QSPLIT, 2) attn_bwd_dkv_d64_kernel(c
       for (int s = 0; s < 2; ++s)
 #pragma unroll
         for (int t = 0; t < D / 32; ++t) {
-          const uint32_t a = (ta ^ (uint32_t)(t << 6)) + 2048u * s, bb = (tb ^ (uint32_t)(t << 6)) + 2048u * s;
-          dVt[t] = M::mma(tr64<T>(a + (uint32_t)TILEB, bb + (uint32_t)TILEB), Pb[s], dVt[t]);
-          dKt[t] = M::mma(tr64<T>(a, bb), dSb[s], dKt[t]);
+          dVt[t] = M::mma(tr_frag<T, D>(dt, tl, t, s), Pb[s], dVt[t]);
+          dKt[t] = M::mma(tr_frag<T, D>(qt, tl, t, s), dSb[s], dKt[t]);
         }
     }
     if (have_next) {
@@ -328,31 +324,31 @@ __global__ void __launch_bounds__(64 * KG * QSPLIT, 2) attn_bwd_dkv_d64_kernel(c
     __syncthreads();
   }
 
-  // add the splits' partial sums through LDS in a fixed order, halving: (0 += 2, 1 += 3), then 0 += 1; 16 KB per
-  // (split, key group): dK, then dV
-  static_assert(2 * STAGEB >= (QSPLIT / 2) * KG * 16384, "exchange area");
+  // add the splits' partial sums through LDS in a fixed order, halving: (0 += 2, 1 += 3), then 0 += 1; per (split, key
+  // group): dK, then dV
+  static_assert(2 * STAGEB >= (QSPLIT / 2) * KG * 2 * SLOTF * 4, "exchange area");
   float *xo = reinterpret_cast<float *>(sAll);
 #pragma unroll
   for (int from = QSPLIT / 2; from >= 1; from >>= 1) {
     if (qs >= from && qs < 2 * from) {
-      float *dst = xo + ((qs - from) * KG + kg) * 4096 + lane;
+      float *dst = xo + ((qs - from) * KG + kg) * (2 * SLOTF) + lane;
 #pragma unroll
       for (int t = 0; t < D / 32; ++t)
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
           dst[(t * 16 + v) * 64] = dKt[t][v];
-          dst[2048 + (t * 16 + v) * 64] = dVt[t][v];
+          dst[SLOTF + (t * 16 + v) * 64] = dVt[t][v];
         }
     }
     __syncthreads();
     if (qs < from) {
-      const float *src = xo + (qs * KG + kg) * 4096 + lane;
+      const float *src = xo + (qs * KG + kg) * (2 * SLOTF) + lane;
 #pragma unroll
       for (int t = 0; t < D / 32; ++t)
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
           dKt[t][v] += src[(t * 16 + v) * 64];
-          dVt[t][v] += src[2048 + (t * 16 + v) * 64];
+          dVt[t][v] += src[SLOTF + (t * 16 + v) * 64];
         }
     }
     __syncthreads();
@@ -392,17 +388,17 @@ __global__ void __launch_bounds__(64 * KG * QSPLIT, 2) attn_bwd_dkv_d64_kernel(c
   }
 }
 
-template <typename T, int RG, int SPLIT>
-static int launch_dq_d64(const AttnBwdParams &p, int batch, hipStream_t st) {
+template <typename T, int D, int RG, int SPLIT, int WPS>
+static int launch_dq_tile(const AttnBwdParams &p, int batch, hipStream_t st) {
   dim3 grid((unsigned)(cdiv(p.max_sq, 32 * RG) * p.hq), (unsigned)batch);
-  hipLaunchKernelGGL((attn_bwd_dq_d64_kernel<T, RG, SPLIT>), grid, dim3(512), 0, st, p);
+  hipLaunchKernelGGL((attn_bwd_dq_tile_kernel<T, D, RG, SPLIT, WPS>), grid, dim3(64 * RG * SPLIT), 0, st, p);
   return DH_OK;
 }
 
-template <typename T, int KG, int QSPLIT>
-static int launch_dkv_d64(const AttnBwdParams &p, int batch, int max_sk, hipStream_t st) {
+template <typename T, int D, int KG, int QSPLIT, int WPS>
+static int launch_dkv_tile(const AttnBwdParams &p, int batch, int max_sk, hipStream_t st) {
   dim3 grid((unsigned)(cdiv(max_sk, 32 * KG) * p.hk * p.hsplit), (unsigned)batch);
-  hipLaunchKernelGGL((attn_bwd_dkv_d64_kernel<T, KG, QSPLIT>), grid, dim3(64 * KG * QSPLIT), 0, st, p);
+  hipLaunchKernelGGL((attn_bwd_dkv_tile_kernel<T, D, KG, QSPLIT, WPS>), grid, dim3(64 * KG * QSPLIT), 0, st, p);
   return DH_OK;
 }
 

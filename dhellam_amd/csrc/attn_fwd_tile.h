@@ -10,21 +10,23 @@
 // Measured against the register-staged kernel that this head dim ran before (one wavefront per row group, padded tiles):
 // 2 x 512 rows, 16 heads 15.5 -> 9.4 us; forward and backward together, causal: 16 heads x 4096 548 -> 287 us, 32 query /
 // 8 kv heads x 4096 1505 -> 410 us.
-#include "attn_d64.h"
+#include "attn_tile.h"
 
 namespace dh {
 
-template <typename T, int RG, int SPLIT, int BN>
-__global__ void __launch_bounds__(512, 4) attn_fwd_d64_kernel(const AttnFwdParams p) {
+template <typename T, int D, int RG, int SPLIT, int BN, int WPS>
+__global__ void __launch_bounds__(64 * RG * SPLIT, WPS) attn_fwd_tile_kernel(const AttnFwdParams p) {
   using M = Mma<T>;
   using Frag = typename M::Frag;
-  static_assert(RG * SPLIT == 8, "8 wavefronts per workgroup");
-  constexpr int D = 64, BM = 32 * RG, NB = BN / 32, NS = BN / 16;
+  using A = AttnTile<D>;
+  constexpr int BM = 32 * RG, NB = BN / 32, NS = BN / 16, NW = RG * SPLIT;
   constexpr int TILEB = BN * D * (int)sizeof(T);          // bytes of one K (or V) tile
   constexpr int STAGEB = SPLIT * 2 * TILEB;               // K tiles of all splits, then V tiles
-  constexpr int CB = SPLIT * 2 * (BN / 8) / 8;            // copy blocks per wavefront and iteration
-  static_assert(CB == 4, "32 rows of one tile per wavefront");
-  __shared__ __attribute__((aligned(1024))) char sAll[2 * STAGEB];
+  constexpr int RPW = SPLIT * 2 * BN / NW;                // rows that a wavefront copies per iteration
+  constexpr int SLOTF = 32 * D;                           // floats of a wavefront's O
+  constexpr int EXB = (SPLIT - 1) * RG * (SLOTF + 128) * 4;
+  static_assert(RPW % 16 == 0 && RPW <= BN, "whole copy patterns of one tile per wavefront");
+  __shared__ __attribute__((aligned(1024))) char sAll[2 * STAGEB > EXB ? 2 * STAGEB : EXB];
 
   const int b = seq_by_length(p.cu_q, gridDim.y, blockIdx.y);
   // the query heads of one kv head read the same K / V rows: keep a kv head on one XCD's L2, late causal tiles first
@@ -45,12 +47,12 @@ __global__ void __launch_bounds__(512, 4) attn_fwd_d64_kernel(const AttnFwdParam
   const int rg = w % RG, sp = w / RG;
   const uint32_t lds0 = (uint32_t)(uintptr_t)sAll;
 
-  // copies of this wavefront: rows cp_r0 .. + 31 of the K or V tile of split cp_sp
-  constexpr int HALVES = BN / 32;
-  const int cp_r0 = 32 * (w % HALVES), cp_v = (w / HALVES) & 1, cp_sp = w / (2 * HALVES);
+  // copies of this wavefront: rows cp_r0 .. + RPW - 1 of the K or V tile of split cp_sp
+  constexpr int PARTS = BN / RPW;
+  const int cp_r0 = RPW * (w % PARTS), cp_v = (w / PARTS) & 1, cp_sp = w / (2 * PARTS);
   const int64_t cp_stride = cp_v ? p.v_stride : p.k_stride;
   const T *cp_g = reinterpret_cast<const T *>(cp_v ? p.v : p.k) + (int64_t)k0 * cp_stride + (int64_t)hkv * D;
-  const Copy64 cl = copy64_lane(lane, (uint32_t)(cp_stride * (int64_t)sizeof(T)));
+  const TileCopy<D> cl = tile_copy<D>(lane, (uint32_t)(cp_stride * (int64_t)sizeof(T)));
   const uint32_t cp_dst = lds0 + (uint32_t)(cp_v * SPLIT * TILEB + cp_sp * TILEB + cp_r0 * D * (int)sizeof(T));
 
   const int wrow0 = m0 + rg * 32, row_q = wrow0 + c;
@@ -59,8 +61,8 @@ __global__ void __launch_bounds__(512, 4) attn_fwd_d64_kernel(const AttnFwdParam
   Frag Qf[D / 16];
 #pragma unroll
   for (int ks = 0; ks < D / 16; ++ks) Qf[ks] = frag_ld<T>(qp + ks * 16 + 8 * hh);
-  const uint32_t k_lane = lds0 + (uint32_t)(sp * TILEB) + row64_lane(lane);
-  const uint32_t va_lane = lds0 + (uint32_t)(SPLIT * TILEB + sp * TILEB) + tr64_lane(lane);
+  const RowLane rl = row_lane<D>(lane);
+  const TrLane tl = tr_lane<D>(lane);
 
   int nk_end = sk;
   if (causal && m0 + BM < nk_end) nk_end = m0 + BM;
@@ -76,7 +78,7 @@ __global__ void __launch_bounds__(512, 4) attn_fwd_d64_kernel(const AttnFwdParam
 
   auto issue = [&](int it) {
     const int tile = it * SPLIT + cp_sp;
-    if (tile < ntiles) copy64<T, CB>(cp_g, cp_stride, tile * BN + cp_r0, sk, cp_dst + (uint32_t)((it & 1) * STAGEB), cl);
+    if (tile < ntiles) copy_tile<T, D, RPW>(cp_g, cp_stride, tile * BN + cp_r0, sk, cp_dst + (uint32_t)((it & 1) * STAGEB), cl, lane);
   };
   if (niter > 0) issue(0);
   dma_wait_all();
@@ -87,8 +89,7 @@ __global__ void __launch_bounds__(512, 4) attn_fwd_d64_kernel(const AttnFwdParam
     if (it + 1 < niter) issue(it + 1);
     const int tile = it * SPLIT + sp, n0 = tile * BN;
     if (tile < ntiles && !(causal && n0 > wrow0 + 31)) {
-      const uint32_t st = (uint32_t)((it & 1) * STAGEB);
-      const uint32_t kb = k_lane + st, va = va_lane + st, vb = tr64_next(va);
+      const uint32_t kt = lds0 + (uint32_t)((it & 1) * STAGEB + sp * TILEB), vt = kt + (uint32_t)(SPLIT * TILEB);
       floatx16 S[NB];
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb)
@@ -97,7 +98,7 @@ __global__ void __launch_bounds__(512, 4) attn_fwd_d64_kernel(const AttnFwdParam
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-        for (int ks = 0; ks < D / 16; ++ks) S[nb] = M::mma(row64<T>((kb ^ (uint32_t)(ks << 5)) + 4096u * nb), Qf[ks], S[nb]);
+        for (int ks = 0; ks < D / 16; ++ks) S[nb] = M::mma(row_frag<T, D>(kt + (uint32_t)(nb * 32 * A::PITCH), rl, ks), Qf[ks], S[nb]);
       if ((causal && n0 + BN - 1 > wrow0) || n0 + BN > sk) {
         const int lim = causal && row_q + 1 < sk ? row_q + 1 : sk;        // keys this lane's row attends to
 #pragma unroll
@@ -140,21 +141,20 @@ __global__ void __launch_bounds__(512, 4) attn_fwd_d64_kernel(const AttnFwdParam
       for (int s = 0; s < NS; ++s)
 #pragma unroll
         for (int t = 0; t < D / 32; ++t)
-          O[t] = M::mma(tr64<T>((va ^ (uint32_t)(t << 6)) + 2048u * s, (vb ^ (uint32_t)(t << 6)) + 2048u * s), Pb[s], O[t]);
+          O[t] = M::mma(tr_frag<T, D>(vt, tl, t, s), Pb[s], O[t]);
     }
     dma_wait_all();
     __syncthreads();   // the next stage has landed, and everyone is done with the current one
   }
 
-  // merge the splits: slot x = (split - 1) * RG + row group holds O (8 KB), the m and l planes follow the slots
-  float *xo = reinterpret_cast<float *>(sAll), *xml = xo + 6 * 2048;
-  static_assert((SPLIT - 1) * RG <= 6 && 2 * STAGEB >= 6 * (8192 + 512), "exchange area");
+  // merge the splits: slot x = (split - 1) * RG + row group holds O, the m and l planes follow the slots
+  float *xo = reinterpret_cast<float *>(sAll), *xml = xo + (SPLIT - 1) * RG * SLOTF;
   if (sp > 0) {
     const int x = (sp - 1) * RG + rg;
 #pragma unroll
     for (int t = 0; t < D / 32; ++t)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) xo[x * 2048 + (t * 16 + v) * 64 + lane] = O[t][v];
+      for (int v = 0; v < 16; ++v) xo[x * SLOTF + (t * 16 + v) * 64 + lane] = O[t][v];
     xml[x * 128 + lane] = m_run;
     xml[x * 128 + 64 + lane] = l_run;
   }
@@ -170,7 +170,7 @@ __global__ void __launch_bounds__(512, 4) attn_fwd_d64_kernel(const AttnFwdParam
 #pragma unroll
     for (int t = 0; t < D / 32; ++t)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) O[t][v] = O[t][v] * a_me + xo[x * 2048 + (t * 16 + v) * 64 + lane] * a_o;
+      for (int v = 0; v < 16; ++v) O[t][v] = O[t][v] * a_me + xo[x * SLOTF + (t * 16 + v) * 64 + lane] * a_o;
     m_run = m_new;
   }
   const float l_tot = pair32_sum(l_run);
@@ -190,10 +190,10 @@ __global__ void __launch_bounds__(512, 4) attn_fwd_d64_kernel(const AttnFwdParam
   }
 }
 
-template <typename T, int RG, int SPLIT, int BN>
-static int launch_attn_fwd_d64(const AttnFwdParams &p, int batch, hipStream_t st) {
+template <typename T, int D, int RG, int SPLIT, int BN, int WPS>
+static int launch_attn_fwd_tile(const AttnFwdParams &p, int batch, hipStream_t st) {
   dim3 grid((unsigned)(cdiv(p.max_sq, 32 * RG) * p.hq), (unsigned)batch);
-  hipLaunchKernelGGL((attn_fwd_d64_kernel<T, RG, SPLIT, BN>), grid, dim3(512), 0, st, p);
+  hipLaunchKernelGGL((attn_fwd_tile_kernel<T, D, RG, SPLIT, BN, WPS>), grid, dim3(64 * RG * SPLIT), 0, st, p);
   return DH_OK;
 }
 
