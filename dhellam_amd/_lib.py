@@ -22,6 +22,7 @@ _vp, _i64, _i32, _f32, _sz = C.c_void_p, C.c_int64, C.c_int, C.c_float, C.c_size
 SIGNATURES = {
     "dh_version": (_i32, []),
     "dh_last_error": (C.c_char_p, []),
+    "dh_zero_many": (_i32, [_vp, _vp, _i32, _vp]),
     "dh_copy_bytes": (_i32, [_vp, _vp, _i64, _vp]),
     "dh_delay": (_i32, [_i64, _vp]),
     "dh_host_delay": (_i32, [_i64, _vp]),
@@ -63,6 +64,8 @@ SIGNATURES = {
     "dh_attn_bwd_set_ds_limit": (None, [_sz]),
     "dh_attn_bwd_set_ds_when_full": (None, [_i32]),
     "dh_attn_bwd_acc": (_i32, [_vp] * 11 + [_sz] + [_vp] * 2 + [_i32] * 3 + [_i64] * 2 + [_i32] * 3 + [_i64] * 8 + [_f32, _i32, _i32, _i32, _vp]),
+    "dh_attn_fwd_halves": (_i32, [_vp] * 7 + [_i32] * 8 + [_i64] * 4 + [_f32, _i32, _i32, _vp]),
+    "dh_attn_bwd_halves": (_i32, [_vp] * 11 + [_sz] + [_vp] * 2 + [_i32] * 6 + [_i64] * 2 + [_i32] * 3 + [_i64] * 8 + [_f32, _i32, _i32, _i32, _vp]),
     "dh_attn_merge": (_i32, [_vp, _vp, _vp, _vp, _i32, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _vp]),
     "dh_moe_route_topk": (_i32, [_vp, _vp, _vp, _i64, _i32, _i32, _vp]),
     "dh_moe_sort_workspace_bytes": (_sz, [_i64, _i32]),

@@ -48,12 +48,12 @@ import torch
 from .. import _host, _lib
 from ..common.global_variables import GLOBAL_VARIABLES
 from .._Clib import (WGRAD_TRANSPOSE_GRAD_MIN_K, WGRAD_TRANSPOSE_MIN_ELEMS, keep_transposed, pymha_varlen_bwd,
-                      pymha_varlen_fwd, _attn_bwd_raw, _kernel_head_dim, _zero_rng_state)
+                      pymha_varlen_fwd, wgrad_rows_ok, _attn_bwd_raw, _kernel_head_dim, _zero_rng_state)
 from ..operators.bda import bda_bwd, bda_fwd
 from ..operators.layernorm import pylayernorm_bwd, pylayernorm_fwd
 from ..operators.layernorm_column import dgrad_bwd, gemm_fwd, wgrad_bwd
 from ..operators.ring_attn import RingGroup, fa_cp_block_bwd, fa_cp_block_fwd
-from ..operators.rope import rope_bwd, rope_fwd
+from ..operators.rope import rope_bwd, rope_fwd, rope_inv_freq
 from ..operators.swiglu import swiglu, swiglu_back
 
 
@@ -259,9 +259,11 @@ class DCFunc:
     def attn(config, data, stream, apply_rope=False):
         qkv, cu_seqlens_q, cu_seqlens_kv = data
         s = config.seq_length
-        if config.groups_per_rank == 1 and not apply_rope and _kernel_head_dim(qkv, config.head_dim) == config.head_dim:
-            q, k, v = _split_qkv(config, qkv)       # views: nothing here runs but the kernel, on ``stream``
-            out, lse = _host.attn_fwd(q, k, v, cu_seqlens_q, cu_seqlens_kv, s, s, config.softmax_scale, True, stream)
+        if _kernel_head_dim(qkv, config.head_dim) == config.head_dim:
+            inv = rope_inv_freq(config.rope_theta, config.head_dim, qkv.device) if apply_rope and config.rope_theta is not None else None
+            out, q, k, v, lse = _host.attn_fwd_packed(qkv, cu_seqlens_q, cu_seqlens_kv, config.heads_per_rank,
+                                                      config.groups_per_rank, config.head_dim, s, config.softmax_scale, inv,
+                                                      stream)
             return out.view(config.tokens, -1), q, k, v, out, _zero_rng_state(q.device), lse
         with torch.cuda.stream(stream):
             q, k, v = _split_qkv(config, qkv)
@@ -344,7 +346,8 @@ class DCFunc:
         # the weight-gradient product of the row projection behind the activation takes this result transposed when
         # the projection has fewer inputs than outputs (``_Clib.wgrad_layout``): the kernel then writes it alongside
         f = input.shape[-1] // 2
-        want_t = f < config.hidden_size and config.tokens * f >= WGRAD_TRANSPOSE_MIN_ELEMS
+        want_t = (f < config.hidden_size and config.tokens * f >= WGRAD_TRANSPOSE_MIN_ELEMS
+                  and wgrad_rows_ok(config.tokens, config.hidden_size))
         output, _ = swiglu(input, stream, False, with_transposed=want_t)
         return output
 
@@ -390,7 +393,7 @@ class DCFunc:
         # wide enough for that layout to pay (``_Clib.wgrad_layout``): the kernel then writes it alongside
         rows, n2 = swiglu_input.shape
         want_t = (config.hidden_size >= WGRAD_TRANSPOSE_GRAD_MIN_K and rows * n2 >= WGRAD_TRANSPOSE_MIN_ELEMS
-                  and config.hidden_size >= n2)     # (fewer inputs than outputs: the input is the operand transposed)
+                  and config.hidden_size >= n2 and wgrad_rows_ok(rows, n2))     # (fewer inputs than outputs: the input is the operand transposed)
         dgrad, _ = swiglu_back(grad_output, swiglu_input, None, stream, profiling=False, with_transposed=want_t)
         return dgrad
 
@@ -399,6 +402,10 @@ class DCFunc:
         grad_output, q, k, v, out, lse, cu_seqlens_q, cu_seqlens_kv, rng_state = data
         hq, hk, d = config.heads_per_rank, config.groups_per_rank, config.head_dim
         T = grad_output.shape[0]
+        if q.shape[-1] == d:
+            inv = rope_inv_freq(config.rope_theta, d, q.device) if apply_rope and config.rope_theta is not None else None
+            return _host.attn_bwd_packed(grad_output, q, k, v, out, lse, cu_seqlens_q, cu_seqlens_kv, config.seq_length,
+                                         config.softmax_scale, inv, stream)
         with torch.cuda.stream(stream):
             dout = grad_output.view(T, hq, d)
             dqkv = torch.empty((T, config.qkv_per_rank), dtype=q.dtype, device=q.device)
@@ -999,7 +1006,7 @@ def init_DCBlocks(config=None, stream1=None, stream2=None, context_parallel_size
     movable = set()
 
     def build(section):
-        blocks = []
+        blocks = _Blocks()
         raw = data.get(section) or DEFAULT_PLAN[section]
         for blk in (_insert_rope(raw) if cp <= 1 else _ring_names_for(raw, cp)):
             if len(blk) != 3:
@@ -1023,44 +1030,72 @@ def init_DCBlocks(config=None, stream1=None, stream2=None, context_parallel_size
     return Plan(build("DCBlocks"), build("fwd_only"), build("bwd_only"), movable, ops)
 
 
-def _run_column(col, dcoperation, config, weight, act, first_input, stream_of, result, movable):
+class _Step:
+    """One op of a column with everything that does not change from call to call looked up."""
+    __slots__ = ("op", "num", "name", "strand", "is_comm", "next", "handler", "free", "fused")
+
+    def __init__(self, op, after):
+        self.op, self.num, self.name, self.is_comm = op, op.get_op_num(), op.name, op.is_comm
+        self.strand = getattr(op, "strand", 1)
+        self.next = op.get_next_op()
+        num = self.num.value if isinstance(self.num, FuncChoice) else int(self.num)
+        self.handler, self.free = _HANDLERS.get(num), _FREE_AFTER.get(num, ())
+        # handler that runs this op and the one after it in the column together
+        self.fused = _FUSED.get((op.name, after.name)) if after is not None and after in self.next else None
+
+
+class _Blocks(list):
+    """The DCBlocks of one plan section and, once they have run, their columns in running order."""
+    steps = None
+
+
+def _block_steps(blk: DCBlock):
+    """[(forward side?, [_Step ...]) ...] of a block in running order: the communication ops one by one, then the two
+    compute columns; the strand whose communication was just posted goes second (dstb.py:1174-1264)."""
+    cols, fwd_comm_first = [], False
+    for op in blk.stream3_op or ():
+        fwd_comm_first |= op.is_comm == 1
+        cols.append((op.is_comm == 1, [op]))
+    for strand in ((2, 1) if fwd_comm_first else (1, 2)):
+        col = blk.stream1_op if strand == 1 else blk.stream2_op
+        if col is not None:
+            cols.append((strand == 1, col))
+    return [(fwd, [_Step(op, col[i + 1] if i + 1 < len(col) else None) for i, op in enumerate(col)]) for fwd, col in cols]
+
+
+def _run_column(steps, dcoperation, config, weight, act, first_input, stream1, stream2, result, movable, fuse):
+    direct = dcoperation is DCoperation
     skip = False
-    for idx, now_op in enumerate(col):
+    for i, s in enumerate(steps):
         if skip:                    # ran together with the op before it
             skip = False
             continue
-        src = now_op.get_output()
-        inp = first_input if src is None else src
-        st = stream_of(now_op)
-        nxt_in_col = col[idx + 1] if idx + 1 < len(col) else None
-        if (nxt_in_col is not None and (now_op.name, nxt_in_col.name) in _FUSED and getattr(config, "fuse_adjacent", True)
-                and hasattr(dcoperation, "perform_fused") and nxt_in_col in now_op.get_next_op()):
-            output = dcoperation.perform_fused(DCFunc, (now_op.name, nxt_in_col.name), config, weight, act, output=inp,
-                                               stream=st, movable=movable)
-            now_op.set_output(None)
-            now_op = nxt_in_col         # successors and result bookkeeping are those of the second op
-            skip = True
-            handle = None
-            now_op.set_output(None)
-            nxt = now_op.get_next_op()
-            if output is not None and len(nxt) == 0:
-                result[0] = output
-            for nop in nxt:
-                nop.set_output(output)
-                nop.set_handle(handle)
-            continue
-        output = dcoperation.perform_operation(DCFunc, now_op.get_op_num(), config, weight, act, output=inp, stream=st,
-                                               name=now_op.name, movable=movable)
+        op = s.op
+        inp = first_input if op.output is None else op.output
+        op.output = None
+        st = stream1 if s.strand == 1 else stream2
         handle = None
-        if now_op.is_comm:
+        if fuse and s.fused is not None:
+            nxt = steps[i + 1]
+            output = dcoperation.perform_fused(DCFunc, (s.name, nxt.name), config, weight, act, output=inp, stream=st,
+                                               movable=movable)
+            s, skip = nxt, True     # successors and result bookkeeping are those of the second op
+            s.op.output = None
+        elif direct and s.handler is not None:
+            output = s.handler(_Ctx(DCFunc, s.num, config, weight, act, inp, st, s.name, movable))
+            for key in s.free:
+                act.pop(key, None)
+        else:
+            output = dcoperation.perform_operation(DCFunc, s.num, config, weight, act, output=inp, stream=st, name=s.name,
+                                                   movable=movable)
+        if s.is_comm:
             output, handle = output
-        now_op.set_output(None)
-        nxt = now_op.get_next_op()
-        if output is not None and len(nxt) == 0:
+        if s.next:
+            for nop in s.next:
+                nop.output = output
+                nop.handle = handle
+        elif output is not None:
             result[0] = output
-        for nop in nxt:
-            nop.set_output(output)
-            nop.set_handle(handle)
 
 
 def exec(config, dcoperation, fwd_weight, bwd_weight, input, grad_output, dcblocks: List[DCBlock], stream1, stream2,
@@ -1080,13 +1115,15 @@ def exec(config, dcoperation, fwd_weight, bwd_weight, input, grad_output, dcbloc
         if ev is not None:
             stream2.wait_event(ev)
     ran_fwd = False
-
-    def stream_of(op):
-        return stream1 if getattr(op, "strand", 1) == 1 else stream2
-
+    fuse = getattr(config, "fuse_adjacent", True) and hasattr(dcoperation, "perform_fused")
+    steps = dcblocks.steps if isinstance(dcblocks, _Blocks) else None
+    if steps is None:
+        steps = [_block_steps(blk) for blk in dcblocks]
+        if isinstance(dcblocks, _Blocks):
+            dcblocks.steps = steps
     lockstep = (getattr(config, "lockstep_blocks", False) and stream1 is not None and stream2 is not None
                 and stream1 != stream2)
-    for now_block in dcblocks:
+    for columns in steps:
         if lockstep:
             # both strands enter a block together (device-side events, no host wait): keeps the block's pairing,
             # which matters when the stand-in collectives have a duration to hide; without it the forward strand
@@ -1096,27 +1133,14 @@ def exec(config, dcoperation, fwd_weight, bwd_weight, input, grad_output, dcbloc
             e2.record(stream2)
             stream1.wait_event(e2)
             stream2.wait_event(e1)
-        fwd_comm_first = False
-        if now_block.stream3_op is not None:
-            for now_op in now_block.stream3_op:
-                if now_op.is_comm == 1:
-                    fwd_comm_first = True
-                    _run_column([now_op], dcoperation, config, fwd_weight, new_activation_dict, input, stream_of,
-                                fwd_res, movable)
-                    ran_fwd = True
-                else:
-                    _run_column([now_op], dcoperation, config, bwd_weight, activation_dict, grad_output, stream_of,
-                                bwd_res, movable)
-        # The strand whose communication was just posted goes second (dstb.py:1174-1264).
-        order = (2, 1) if fwd_comm_first else (1, 2)
-        for strand in order:
-            if strand == 1 and now_block.stream1_op is not None:
-                _run_column(now_block.stream1_op, dcoperation, config, fwd_weight, new_activation_dict, input, stream_of,
-                            fwd_res, movable)
+        for fwd, col in columns:
+            if fwd:
+                _run_column(col, dcoperation, config, fwd_weight, new_activation_dict, input, stream1, stream2, fwd_res,
+                            movable, fuse)
                 ran_fwd = True
-            if strand == 2 and now_block.stream2_op is not None:
-                _run_column(now_block.stream2_op, dcoperation, config, bwd_weight, activation_dict, grad_output,
-                            stream_of, bwd_res, movable)
+            else:
+                _run_column(col, dcoperation, config, bwd_weight, activation_dict, grad_output, stream1, stream2, bwd_res,
+                            movable, fuse)
     # deferred wgrads that no placeholder op picked up run at the end (dstb.py:1268-1279)
     if activation_dict is not None and activation_dict.get("_parked"):
         for key in list(activation_dict["_parked"]):

@@ -9,10 +9,12 @@ This module reproduces that order for one layer on one GPU without Megatron.
 """
 from __future__ import annotations
 
+import dataclasses
 from typing import Dict, List, Optional
 
 import torch
 
+from .. import _host
 from .._Clib import keep_transposed, refresh_transposed
 from .dstb import DCoperation, LayerConfig, Plan, exec as exec_blocks, init_DCBlocks
 
@@ -109,6 +111,12 @@ def _shared_proxy():
     return _PROXY[0]
 
 
+# Rows of all micro-batches of a step from which keeping W^T pays.  Rebuilding the four transposes of a 70B shard's layer
+# costs 71 us; what they save per micro-batch: 94 us at 4096 rows, 57 at 2048, 39 at 1000, of which less is left against
+# the kernel that ``dgrad_gemm`` uses for few rows (22 us at 1000).
+TRANSPOSES_MIN_ROWS = 3072
+
+
 class LayerRunner:
     """Runs micro-batches through one layer, serially or double-stranded."""
 
@@ -118,17 +126,18 @@ class LayerRunner:
         if cfg.comm_standin_engine == "proxy" and cfg.comm_standin_us > 0:
             # the stand-in collectives go to the resident communication proxy (one per process: its flags are
             # signal memory that stays allocated); slot 0 = forward strand, slot 1 = backward strand
-            import dataclasses
             self.proxy = cfg.comm_proxy or _shared_proxy()
             cfg = dataclasses.replace(cfg, comm_proxy=self.proxy)
         self.cfg = cfg
+        # for steps too short for the resident transposes to pay: the data gradients take the weights as they are
+        self.cfg_short = dataclasses.replace(cfg, resident_weight_transposes=False)
         self.weights = weights
         self.stream1 = stream1 or torch.cuda.Stream()
         self.stream2 = stream2 or torch.cuda.Stream()
         self.plan: Plan = init_DCBlocks(plan, self.stream1, self.stream2, cfg.context_parallel_size)
 
-    def _exec(self, blocks, x, dy, act_prev, act_new, s1, s2):
-        return exec_blocks(self.cfg, DCoperation, self.weights if act_new is not None else None,
+    def _exec(self, cfg, blocks, x, dy, act_prev, act_new, s1, s2):
+        return exec_blocks(cfg, DCoperation, self.weights if act_new is not None else None,
                            self.weights if act_prev is not None else None, x, dy, blocks, s1, s2, act_prev, act_new,
                            movable=self.plan.movable)
 
@@ -139,19 +148,28 @@ class LayerRunner:
         if self.cfg.resident_weight_transposes:
             refresh_transposed(self.weights.values())
 
+    def _step_config(self, mbs, refresh):
+        """The configuration a step runs with, its W^T rebuilt if it uses them (a caller that does not refresh keeps
+        them current itself)."""
+        if not refresh:
+            return self.cfg
+        if not self.cfg.resident_weight_transposes or self.cfg.tokens * len(mbs) < TRANSPOSES_MIN_ROWS:
+            return self.cfg_short
+        self.refresh_weight_transposes()
+        return self.cfg
+
     def run_serial(self, mbs: List[dict], refresh_transposes: bool = True):
         """F0 B0 F1 B1 ... on ONE stream with the fwd_only / bwd_only plans.  ``refresh_transposes=False`` is for a
         caller that runs several such calls between two weight updates."""
-        if refresh_transposes:
-            self.refresh_weight_transposes()
+        cfg = self._step_config(mbs, refresh_transposes)
         s = self.stream1
         s.wait_stream(torch.cuda.current_stream())
         self._proxy_begin()
         outs, dxs = [], []
         for mb in mbs:
             act = fresh_activation_dict(mb)
-            out, _ = self._exec(self.plan.fwd_only, mb["x"], None, None, act, s, s)
-            _, dx = self._exec(self.plan.bwd_only, None, mb["dy"], act, None, s, s)
+            out, _ = self._exec(cfg, self.plan.fwd_only, mb["x"], None, None, act, s, s)
+            _, dx = self._exec(cfg, self.plan.bwd_only, None, mb["dy"], act, None, s, s)
             outs.append(out)
             dxs.append(dx)
         self._proxy_end(s, s)
@@ -161,8 +179,7 @@ class LayerRunner:
     def run_double_strand(self, mbs: List[dict], refresh_transposes: bool = True):
         """F0 . (F1 || B0) . (F2 || B1) ... B_last: forward strand on stream1, backward strand
         on stream2, paired steps following the plan's DCBlocks."""
-        if refresh_transposes:
-            self.refresh_weight_transposes()
+        cfg = self._step_config(mbs, refresh_transposes)
         s1, s2 = self.stream1, self.stream2
         cur = torch.cuda.current_stream()
         s1.wait_stream(cur)
@@ -171,12 +188,12 @@ class LayerRunner:
         n = len(mbs)
         outs, dxs = [None] * n, [None] * n
         act = fresh_activation_dict(mbs[0])
-        outs[0], _ = self._exec(self.plan.fwd_only, mbs[0]["x"], None, None, act, s1, s2)
+        outs[0], _ = self._exec(cfg, self.plan.fwd_only, mbs[0]["x"], None, None, act, s1, s2)
         for i in range(1, n):
             act_new = fresh_activation_dict(mbs[i])
-            outs[i], dxs[i - 1] = self._exec(self.plan.dcblocks, mbs[i]["x"], mbs[i - 1]["dy"], act, act_new, s1, s2)
+            outs[i], dxs[i - 1] = self._exec(cfg, self.plan.dcblocks, mbs[i]["x"], mbs[i - 1]["dy"], act, act_new, s1, s2)
             act = act_new
-        _, dxs[n - 1] = self._exec(self.plan.bwd_only, None, mbs[n - 1]["dy"], act, None, s1, s2)
+        _, dxs[n - 1] = self._exec(cfg, self.plan.bwd_only, None, mbs[n - 1]["dy"], act, None, s1, s2)
         self._proxy_end(s1, s2)
         cur.wait_stream(s1)
         cur.wait_stream(s2)
@@ -194,9 +211,7 @@ class LayerRunner:
             torch.cuda.current_stream().wait_stream(self.proxy.stream)
 
     def zero_grads(self):
-        for t in self.weights.values():
-            if hasattr(t, "main_grad"):
-                t.main_grad.zero_()
+        _host.zero_all([t.main_grad for t in self.weights.values() if hasattr(t, "main_grad")], None)
 
     def grads(self) -> Dict[str, torch.Tensor]:
         return {k: t.main_grad for k, t in self.weights.items() if hasattr(t, "main_grad")}

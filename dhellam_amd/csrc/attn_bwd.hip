@@ -2,8 +2,8 @@
 // floating-point atomics).
 //
 // Three kernels:
-//   delta   : delta_i = sum_d dO[i,d] * O[i,d]                      (streaming; the dQ kernels of head
-//             dims 64 and 128 form delta in their prologue and run first)
+//   delta   : delta_i = sum_d dO[i,d] * O[i,d]                      (streaming; for fp32 and where dS is kept: the
+//             recomputing dQ kernels form delta in their prologue and run first)
 //   dK/dV   : a workgroup owns 64 key/value rows (K, V fragments stay in
 //             registers, for head dim 128 in LDS), walks the
 //             query heads of its GQA group and the query tiles that attend to
@@ -28,11 +28,11 @@ namespace dh {
 
 struct AttnBwdParams {
   const void *dout, *q, *k, *v;
-  const void *out;           // forward output (d = 128: the dQ kernel forms delta from it)
+  const void *out;           // forward output (the dQ kernels form delta from it)
   int64_t o_stride;
   const float *lse;
-  float *delta;              // fp32 [batch][hq][max_sq]: rowsum(dO * O); written by the delta kernel, or (d = 128) by the dQ kernel
-  float *ld2;                // fp32 [2][plane]: lse * log2(e), then delta, each [batch][hq][ld2_pitch] (d = 128 kernels)
+  float *delta;              // fp32 [batch][hq][max_sq]: rowsum(dO * O); written by the delta kernel or by the dQ kernel
+  float *ld2;                // fp32 [2][plane]: lse * log2(e), then delta, each [batch][hq][ld2_pitch]
   int64_t ld2_plane;         // elements between the two planes
   int ld2_pitch;             // max_sq rounded up to 32: every 32-row query tile of a head is one aligned 128-byte run
   void *dq, *dk, *dv;
@@ -43,6 +43,8 @@ struct AttnBwdParams {
   int64_t q_stride, k_stride, v_stride, do_stride, dq_stride, dk_stride, dv_stride;
   float scale, scale_log2;
   int causal;
+  int q_shift, k_shift;      // sequence bounds are cu >> shift (the halves of a context-parallel chunk)
+  int lse_pitch;             // rows of a head in lse
   int dq_accumulate;         // dq += this call's gradient (read, add in fp32, round once) instead of dq =
   // dS = P * (dP - delta) kept for the dQ product (head dim 128, 16 bits, when the workspace allows): 2 KB blocks of
   // 32 keys x 32 query rows, block (b, h, query tile, key block); inside a block the 16-byte piece (s, hh, key)
@@ -57,11 +59,11 @@ template <typename T>
 __global__ void __launch_bounds__(256)
 attn_delta_kernel(const T *__restrict__ dout, const T *__restrict__ out, float *__restrict__ delta,
                   const float *__restrict__ lse, float *__restrict__ ld2, int64_t ld2_plane, int ld2_pitch,
-                  const int32_t *__restrict__ cu_q, int max_sq, int hq, int d, int lanes_per, int64_t do_stride,
-                  int64_t o_stride) {
+                  const int32_t *__restrict__ cu_q, int q_shift, int lse_pitch, int max_sq, int hq, int d, int lanes_per,
+                  int64_t do_stride, int64_t o_stride) {
   constexpr int N = Vec<T>::N;
   const int b = blockIdx.y;
-  const int q0 = cu_q[b], sq = cu_q[b + 1] - q0;
+  const int q0 = cu_q[b] >> q_shift, sq = (cu_q[b + 1] >> q_shift) - q0;
   const int per_block = 256 / lanes_per;
   const int sub = threadIdx.x / lanes_per, ln = threadIdx.x % lanes_per;
   const int nvec = d / N;
@@ -88,9 +90,9 @@ attn_delta_kernel(const T *__restrict__ dout, const T *__restrict__ out, float *
     if (ln == 0) {
       const int64_t at = ((int64_t)b * hq + h) * max_sq + i;
       delta[at] = s;
-      if (ld2) {             // the copy the d = 128 kernels stream: lse in exp2 units next to delta
+      if (ld2) {             // the copy the dK/dV kernels stream: lse in exp2 units next to delta
         const int64_t a2 = ((int64_t)b * hq + h) * ld2_pitch + i;
-        ld2[a2] = lse[at] * 1.4426950408889634f;
+        ld2[a2] = lse[((int64_t)b * hq + h) * lse_pitch + i] * 1.4426950408889634f;
         ld2[ld2_plane + a2] = s;
       }
     }
@@ -158,8 +160,8 @@ __global__ void __launch_bounds__(512) attn_bwd_dq_d128_kernel(const AttnBwdPara
   int hkv, item;
   xcd_group_item(blockIdx.x, p.hk, ratio * P, hkv, item);
   const int h = hkv * ratio + item / P, px = item % P;
-  const int q0 = p.cu_q[b], sq = p.cu_q[b + 1] - q0;
-  const int k0 = p.cu_k[b], sk = p.cu_k[b + 1] - k0;
+  const int q0 = p.cu_q[b] >> p.q_shift, sq = (p.cu_q[b + 1] >> p.q_shift) - q0;
+  const int k0 = p.cu_k[b] >> p.k_shift, sk = (p.cu_k[b + 1] >> p.k_shift) - k0;
   const int nqt = (sq + BM - 1) / BM;
   const int causal = p.causal;
   const int k_stride = (int)p.k_stride, v_stride = (int)p.v_stride;
@@ -226,7 +228,7 @@ __global__ void __launch_bounds__(512) attn_bwd_dq_d128_kernel(const AttnBwdPara
         dOf[ks] = frag_ld<T>(dp + ks * 16 + 8 * hh);
       }
     }
-    const float lse_c = row_ok ? p.lse[((int64_t)b * p.hq + h) * p.max_sq + row_q] * 1.4426950408889634f : INFINITY;
+    const float lse_c = row_ok ? p.lse[((int64_t)b * p.hq + h) * p.lse_pitch + row_q] * 1.4426950408889634f : INFINITY;
     // delta = rowsum(dO * O) of this lane's row, formed by the first key split of each row group: the lane holds
     // one half of the row's dO (its k-step chunks), reads the same chunks of O, and the two halves meet through
     // the partner lane.  The other splits get it through LDS after the barrier that publishes the first tiles.
@@ -457,8 +459,8 @@ __global__ void __launch_bounds__(512) attn_bwd_dq2_d128_kernel(const AttnBwdPar
   int h, px;
   xcd_group_item(blockIdx.x, p.hq, P, h, px);
   const int hkv = h / ratio;
-  const int q0 = p.cu_q[b], sq = p.cu_q[b + 1] - q0;
-  const int k0 = p.cu_k[b], sk = p.cu_k[b + 1] - k0;
+  const int q0 = p.cu_q[b] >> p.q_shift, sq = (p.cu_q[b + 1] >> p.q_shift) - q0;
+  const int k0 = p.cu_k[b] >> p.k_shift, sk = (p.cu_k[b + 1] >> p.k_shift) - k0;
   const int nqt = (sq + BM - 1) / BM;
   const int causal = p.causal;
   const int k_stride = (int)p.k_stride;
@@ -704,8 +706,8 @@ __global__ void __launch_bounds__(512) attn_bwd_dkv_d128_kernel(const AttnBwdPar
   int hg, px;
   xcd_group_item(blockIdx.x, G, gridDim.x / G, hg, px);
   const int hkv = hg / p.hsplit, hs = hg % p.hsplit;
-  const int q0 = p.cu_q[b], sq = p.cu_q[b + 1] - q0;
-  const int k0 = p.cu_k[b], sk = p.cu_k[b + 1] - k0;
+  const int q0 = p.cu_q[b] >> p.q_shift, sq = (p.cu_q[b + 1] >> p.q_shift) - q0;
+  const int k0 = p.cu_k[b] >> p.k_shift, sk = (p.cu_k[b + 1] >> p.k_shift) - k0;
   const int nkt = (sk + BN - 1) / BN;
   const int causal = p.causal;
   const int q_stride = (int)p.q_stride, do_stride = (int)p.do_stride;
@@ -1076,7 +1078,8 @@ static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 template <typename T>
 static int launch_delta(const void *dout, const void *out, float *delta, const float *lse, float *ld2, int64_t ld2_plane,
-                        int ld2_pitch, const int32_t *cu_q, int batch, int max_sq, int hq, int d, int64_t do_stride, int64_t o_stride,
+                        int ld2_pitch, const int32_t *cu_q, int q_shift, int lse_pitch, int batch, int max_sq, int hq, int d,
+                        int64_t do_stride, int64_t o_stride,
                         hipStream_t st) {
   const int nvec = d / Vec<T>::N;
   int lanes_per = 1;
@@ -1086,8 +1089,8 @@ static int launch_delta(const void *dout, const void *out, float *delta, const f
   if (blocks > 256 * 16) blocks = 256 * 16;
   if (blocks < 1) blocks = 1;
   hipLaunchKernelGGL((attn_delta_kernel<T>), dim3((unsigned)blocks, (unsigned)batch), dim3(256), 0, st,
-                     (const T *)dout, (const T *)out, delta, lse, ld2, ld2_plane, ld2_pitch, cu_q, max_sq, hq, d, lanes_per, do_stride,
-                     o_stride);
+                     (const T *)dout, (const T *)out, delta, lse, ld2, ld2_plane, ld2_pitch, cu_q, q_shift, lse_pitch, max_sq, hq, d, lanes_per,
+                     do_stride, o_stride);
   return DH_OK;
 }
 
@@ -1113,6 +1116,11 @@ static bool dq_big_grid(int batch, int max_sq, int hq, int causal) {
   return (causal ? (t + 1) / 2 : t) * hq * batch >= 256;
 }
 
+// Head dim 128 with short sequences: the kernels of the other head dims start and end sooner than the hand-ordered ones
+// (backward of 32 / 8 heads x 100 36 -> 27 us, 8 heads x 300 41 -> 34 us; at 600 rows 46 / 42, at 1000 level), and dS is
+// not kept.
+static bool bwd_short(int max_sq, int max_sk) { return max_sq < 512 && max_sk < 512; }
+
 // The kernels behind delta of one call.
 template <typename T, int D>
 static int bwd_passes(const AttnBwdParams &p, int batch, int max_sq, int max_sk, hipStream_t st) {
@@ -1121,7 +1129,11 @@ static int bwd_passes(const AttnBwdParams &p, int batch, int max_sq, int max_sk,
   // recomputing dQ kernels form delta and run first
   if (max_sq > 0) {
     if constexpr (D == 128) {
-      if (!p.ds)
+      // (packed batches: most workgroups of the longest sequence's grid have nothing to do, and the smaller workgroups
+      // balance the rest: documents of 4 to 1298 tokens, 16 heads 47 -> 38 us)
+      if (bwd_short(max_sq, max_sk) || (!p.ds && p.causal && batch > 2))
+        rc = small_q ? launch_dq_tile<T, D, 2, 4, 2>(p, batch, st) : launch_dq_tile<T, D, 4, 2, 2>(p, batch, st);
+      else if (!p.ds)
         rc = dq_big_grid(batch, max_sq, p.hq, p.causal) ? launch_dq_d128<T, 4, 2, 32>(p, batch, st) : launch_dq_d128<T, 2, 4, 32>(p, batch, st);
     } else if constexpr (D < 128) {
       rc = small_q ? launch_dq_tile<T, D, 2, 4, 2>(p, batch, st) : launch_dq_tile<T, D, 4, 2, D == 64 ? 4 : 2>(p, batch, st);
@@ -1130,7 +1142,7 @@ static int bwd_passes(const AttnBwdParams &p, int batch, int max_sq, int max_sk,
     }
   }
   if (rc == DH_OK && max_sk > 0) {
-    if constexpr (D == 128) rc = launch_dkv_d128<T>(p, batch, max_sk, st);
+    if constexpr (D == 128) rc = bwd_short(max_sq, max_sk) ? launch_dkv_tile<T, D, 2, 2, 1>(p, batch, max_sk, st) : launch_dkv_d128<T>(p, batch, max_sk, st);
     else if constexpr (D < 128) rc = launch_dkv_tile<T, D, 2, 4, 2>(p, batch, max_sk, st);
     else rc = launch_dkv_tile<T, D, 2, 2, 1>(p, batch, max_sk, st);
   }
@@ -1200,7 +1212,8 @@ static int attn_bwd_entry(const void *dout, const void *q, const void *k, const 
                           int max_seqlen_q, int max_seqlen_k, int64_t total_q, int64_t total_k, int hq, int hk, int d,
                           int64_t q_stride, int64_t k_stride, int64_t v_stride, int64_t o_stride,
                           int64_t do_stride, int64_t dq_stride, int64_t dk_stride, int64_t dv_stride,
-                          float softmax_scale, int causal, int dq_accumulate, int dtype, void *stream) {
+                          float softmax_scale, int causal, int dq_accumulate, int q_shift, int k_shift, int lse_pitch, int dtype,
+                          void *stream) {
   using namespace dh;
   DH_CHECK(batch >= 0 && max_seqlen_q >= 0 && max_seqlen_k >= 0 && total_q >= 0 && total_k >= 0, "negative size");
   DH_CHECK(hq > 0 && hk > 0 && hq % hk == 0, "hq=%d must be a positive multiple of hk=%d", hq, hk);
@@ -1236,13 +1249,13 @@ static int attn_bwd_entry(const void *dout, const void *q, const void *k, const 
   // process-wide limit); they take the tail of the workspace
   size_t dsb = ds_bytes(batch, max_seqlen_q, total_k, hq, d, dtype, causal);
   if (dsb > 0 && base_bytes + align256(dsb) > workspace_bytes) dsb = 0;
-  const bool keep_ds = dsb > 0 && max_seqlen_k > 0;
+  const bool keep_ds = dsb > 0 && max_seqlen_k > 0 && !bwd_short(max_seqlen_q, max_seqlen_k);
   uint8_t *ds_ws = (uint8_t *)(((uintptr_t)workspace + 255) & ~(uintptr_t)255) + (base_bytes - 256);
   const bool delta_in_dq = dtype != DH_F32 && !keep_ds;
   if (max_seqlen_q > 0 && !delta_in_dq) {
     DH_DISPATCH_DTYPE(dtype, {
-      launch_delta<T>(dout, out, delta, lse, ld2, (int64_t)(plane2 / sizeof(float)), ld2_pitch, cu_seqlens_q, batch, max_seqlen_q, hq, d,
-                      do_stride, o_stride, st);
+      launch_delta<T>(dout, out, delta, lse, ld2, (int64_t)(plane2 / sizeof(float)), ld2_pitch, cu_seqlens_q, q_shift, lse_pitch,
+                      batch, max_seqlen_q, hq, d, do_stride, o_stride, st);
     });
   }
   if (dtype == DH_F32) {
@@ -1271,6 +1284,7 @@ static int attn_bwd_entry(const void *dout, const void *q, const void *k, const 
   p.scale = softmax_scale;
   p.scale_log2 = softmax_scale * 1.4426950408889634f;
   p.causal = causal;
+  p.q_shift = q_shift; p.k_shift = k_shift; p.lse_pitch = lse_pitch;
   p.dq_accumulate = dq_accumulate ? 1 : 0;
   p.ds = keep_ds ? (void *)ds_ws : nullptr;
   p.ds_nqt = 2 * (int)cdiv(max_seqlen_q, 64);
@@ -1311,7 +1325,7 @@ extern "C" int dh_attn_bwd(const void *dout, const void *q, const void *k, const
                            float softmax_scale, int causal, int dtype, void *stream) {
   return attn_bwd_entry(dout, q, k, v, out, lse, dq, dk, dv, delta_out, workspace, workspace_bytes, cu_seqlens_q, cu_seqlens_k, batch,
                         max_seqlen_q, max_seqlen_k, total_q, total_k, hq, hk, d, q_stride, k_stride, v_stride, o_stride,
-                        do_stride, dq_stride, dk_stride, dv_stride, softmax_scale, causal, 0, dtype, stream);
+                        do_stride, dq_stride, dk_stride, dv_stride, softmax_scale, causal, 0, 0, 0, max_seqlen_q, dtype, stream);
 }
 
 extern "C" int dh_attn_bwd_acc(const void *dout, const void *q, const void *k, const void *v, const void *out,
@@ -1323,5 +1337,22 @@ extern "C" int dh_attn_bwd_acc(const void *dout, const void *q, const void *k, c
                                float softmax_scale, int causal, int accumulate_dq, int dtype, void *stream) {
   return attn_bwd_entry(dout, q, k, v, out, lse, dq, dk, dv, delta_out, workspace, workspace_bytes, cu_seqlens_q, cu_seqlens_k, batch,
                         max_seqlen_q, max_seqlen_k, total_q, total_k, hq, hk, d, q_stride, k_stride, v_stride, o_stride,
-                        do_stride, dq_stride, dk_stride, dv_stride, softmax_scale, causal, accumulate_dq, dtype, stream);
+                        do_stride, dq_stride, dk_stride, dv_stride, softmax_scale, causal, accumulate_dq, 0, 0, max_seqlen_q, dtype, stream);
+}
+
+extern "C" int dh_attn_bwd_halves(const void *dout, const void *q, const void *k, const void *v, const void *out,
+                                  const float *lse, void *dq, void *dk, void *dv, float *delta_out, void *workspace,
+                                  size_t workspace_bytes, const int32_t *cu_seqlens_q, const int32_t *cu_seqlens_k,
+                                  int q_shift, int k_shift, int lse_pitch, int batch, int max_seqlen_q,
+                                  int max_seqlen_k, int64_t total_q, int64_t total_k, int hq, int hk, int d,
+                                  int64_t q_stride, int64_t k_stride, int64_t v_stride, int64_t o_stride,
+                                  int64_t do_stride, int64_t dq_stride, int64_t dk_stride, int64_t dv_stride,
+                                  float softmax_scale, int causal, int accumulate_dq, int dtype, void *stream) {
+  DH_CHECK((q_shift == 0 || q_shift == 1) && (k_shift == 0 || k_shift == 1), "sequences are taken whole or halved");
+  DH_CHECK(dtype != DH_F32 || (q_shift + k_shift == 0 && lse_pitch == max_seqlen_q), "fp32 attention takes whole sequences");
+  DH_CHECK(lse_pitch >= max_seqlen_q, "lse rows are shorter than max_seqlen_q");
+  return attn_bwd_entry(dout, q, k, v, out, lse, dq, dk, dv, delta_out, workspace, workspace_bytes, cu_seqlens_q, cu_seqlens_k, batch,
+                        max_seqlen_q, max_seqlen_k, total_q, total_k, hq, hk, d, q_stride, k_stride, v_stride, o_stride,
+                        do_stride, dq_stride, dk_stride, dv_stride, softmax_scale, causal, accumulate_dq, q_shift, k_shift,
+                        lse_pitch, dtype, stream);
 }

@@ -1,9 +1,9 @@
-// Head dim 64 backward (16 bits), two passes as at the other head dims: dQ (which forms delta = rowsum(dO O) and runs
-// first) and dK/dV.  Tile layout and copies: attn_d64.h; workgroup shape and what bounds it: as the forward kernel of this
-// head dim (attn_fwd_d64.h).
-// dK/dV keeps K and V fragments and both accumulators in registers (202): two wavefronts a SIMD.
-// Measured against the register-staged kernels: 2 x 512 rows, 16 heads, delta + dQ 28.6 -> 11.5 us, dK/dV 31.3 -> 13.9 us;
-// larger shapes in attn_fwd_d64.h.
+// Attention backward on the tile layout of attn_tile.h (16 bits), two passes: dQ (which forms delta = rowsum(dO O) and runs
+// first) and dK/dV.  Workgroup shape and what bounds it: as the forward kernel (attn_fwd_tile.h).
+// dK/dV keeps K and V fragments and both accumulators in registers (210 at head dim 64, 255 at 96): two wavefronts a SIMD, one
+// at the larger head dims (348 at 128, all 512 at 256, where a few spill).
+// Measured against the register-staged kernels, backward, causal: 16 heads x 2 x 512, head dim 64 58 -> 24 us; 32 query / 8
+// kv heads x 4096, head dim 64 1313 -> 324, 96 1562 -> 438, 256 10871 -> 1841 us; 16 heads x 2048, head dim 192 642 -> 201 us.
 #include "attn_tile.h"
 
 namespace dh {
@@ -28,8 +28,8 @@ __global__ void __launch_bounds__(64 * RG * SPLIT, WPS) attn_bwd_dq_tile_kernel(
   int hkv, item;
   xcd_group_item(blockIdx.x, p.hk, ratio * P, hkv, item);
   const int h = hkv * ratio + item % ratio, px = item / ratio;
-  const int q0 = p.cu_q[b], sq = p.cu_q[b + 1] - q0;
-  const int k0 = p.cu_k[b], sk = p.cu_k[b + 1] - k0;
+  const int q0 = p.cu_q[b] >> p.q_shift, sq = (p.cu_q[b + 1] >> p.q_shift) - q0;
+  const int k0 = p.cu_k[b] >> p.k_shift, sk = (p.cu_k[b + 1] >> p.k_shift) - k0;
   const int nqt = (sq + BM - 1) / BM;
   if (px >= nqt) return;
   const int m0 = (nqt - 1 - px) * BM;          // late causal tiles carry the most work and come first
@@ -73,7 +73,7 @@ __global__ void __launch_bounds__(64 * RG * SPLIT, WPS) attn_bwd_dq_tile_kernel(
     }
   }
   const int64_t stat = ((int64_t)b * p.hq + h) * p.max_sq + row_q;
-  const float lse_c = row_ok ? p.lse[stat] * 1.4426950408889634f : INFINITY;        // rows past the end: P = 0
+  const float lse_c = row_ok ? p.lse[((int64_t)b * p.hq + h) * p.lse_pitch + row_q] * 1.4426950408889634f : INFINITY;        // rows past the end: P = 0
   float del_c = 0.f;
   if (sp == 0) {       // delta of the workgroup's rows, for the other splits and for the dK/dV pass
     const T *op = reinterpret_cast<const T *>(p.out) + (int64_t)(q0 + row_ld) * p.o_stride + (int64_t)h * D + 8 * hh;
@@ -190,8 +190,8 @@ __global__ void __launch_bounds__(64 * KG * QSPLIT, WPS) attn_bwd_dkv_tile_kerne
   int hg, px;
   xcd_group_item(blockIdx.x, G, gridDim.x / G, hg, px);
   const int hkv = hg / p.hsplit, hs = hg % p.hsplit;
-  const int q0 = p.cu_q[b], sq = p.cu_q[b + 1] - q0;
-  const int k0 = p.cu_k[b], sk = p.cu_k[b + 1] - k0;
+  const int q0 = p.cu_q[b] >> p.q_shift, sq = (p.cu_q[b + 1] >> p.q_shift) - q0;
+  const int k0 = p.cu_k[b] >> p.k_shift, sk = (p.cu_k[b + 1] >> p.k_shift) - k0;
   const int j0 = px * BN;          // early causal tiles carry the most work and come first
   if (j0 >= sk) return;
   const int causal = p.causal;

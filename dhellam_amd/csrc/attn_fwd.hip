@@ -27,6 +27,7 @@ struct AttnFwdParams {
   int64_t q_stride, k_stride, v_stride, o_stride;
   float scale, scale_log2;
   int causal;
+  int q_shift, k_shift;      // sequence bounds are cu >> shift (the halves of a context-parallel chunk)
 };
 
 // ---------------------------------------------------------------------------------------------
@@ -72,8 +73,8 @@ __global__ void __launch_bounds__(512) attn_fwd_d128_kernel(const AttnFwdParams 
   int hkv, item;
   xcd_group_item(blockIdx.x, p.hk, ratio * P, hkv, item);
   const int h = hkv * ratio + item / P, px = item % P;
-  const int q0 = p.cu_q[b], sq = p.cu_q[b + 1] - q0;
-  const int k0 = p.cu_k[b], sk = p.cu_k[b + 1] - k0;
+  const int q0 = p.cu_q[b] >> p.q_shift, sq = (p.cu_q[b + 1] >> p.q_shift) - q0;
+  const int k0 = p.cu_k[b] >> p.k_shift, sk = (p.cu_k[b + 1] >> p.k_shift) - k0;
   const int nqt = (sq + BM - 1) / BM;
   const int causal = p.causal;
   const int k_stride = (int)p.k_stride, v_stride = (int)p.v_stride;
@@ -426,13 +427,33 @@ namespace dh {
 #define DH_FWD_128ROW_MIN_WG 256
 #endif
 
-// Head dims 64, 96, 192 and 256: 128-row query tiles when they give every compute unit its workgroups (two at 64 and 96,
+// Workgroups of the head-dim-128 kernel with query tiles of `rows`.
+static int64_t attn_fwd_wgs(int max_sq, int rows, int hq, int batch, int causal) {
+  const int64_t t = cdiv(max_sq, rows);
+  return (causal ? (t + 1) / 2 : t) * hq * batch;
+}
+
+// Head dim 128: the hand-ordered kernel is the faster one where its workgroups, one per compute unit and causal ones all
+// of one length, come out in full rounds: 16 heads x 2048 causal (256 workgroups) 35 against 38 us, 32 heads x 4096 152
+// against 163 us.  Elsewhere its fixed costs and an almost empty last round lose to the smaller workgroups of the kernel
+// that the other head dims run: 8 heads x 300 17.2 against 9.9 us, 16 heads x 600 20 / 13, 12 heads x 3000 79 / 57 us,
+// packed documents of 4 to 1298 tokens (most workgroups of the longest one's grid have nothing to do) 35 / 28 us.
+static bool attn_fwd_fills(int max_sq, int hq, int batch, int causal) {
+  if (!causal) return attn_fwd_wgs(max_sq, 64, hq, batch, 0) >= 96;
+  if (batch > 2) return false;
+  int64_t wgs = attn_fwd_wgs(max_sq, 128, hq, batch, 1);
+  if (wgs < DH_FWD_128ROW_MIN_WG) wgs = attn_fwd_wgs(max_sq, 64, hq, batch, 1);
+  return wgs >= 240 && 20 * wgs >= 17 * 256 * cdiv(wgs, 256);
+}
+
+// All other cases: 128-row query tiles when they give every compute unit its workgroups (two at 64 and 96,
 // one of the larger head dims), else 64-row tiles; more key splits where registers and LDS allow.
 template <typename T>
 static int launch_attn_fwd_other(const AttnFwdParams &p, int d, int batch, hipStream_t st) {
   const int64_t wg128 = cdiv(p.max_sq, 128) * p.hq * batch;
   if (d == 64) return wg128 >= 2 * 256 ? launch_attn_fwd_tile<T, 64, 4, 2, 64, 4>(p, batch, st) : launch_attn_fwd_tile<T, 64, 2, 4, 32, 4>(p, batch, st);
   if (d == 96) return wg128 >= 2 * 256 ? launch_attn_fwd_tile<T, 96, 4, 2, 32, 4>(p, batch, st) : launch_attn_fwd_tile<T, 96, 2, 4, 32, 2>(p, batch, st);
+  if (d == 128) return wg128 >= 256 ? launch_attn_fwd_tile<T, 128, 4, 2, 64, 2>(p, batch, st) : launch_attn_fwd_tile<T, 128, 2, 4, 32, 2>(p, batch, st);
   if (d == 192) return wg128 >= 256 ? launch_attn_fwd_tile<T, 192, 4, 2, 32, 2>(p, batch, st) : launch_attn_fwd_tile<T, 192, 2, 2, 32, 1>(p, batch, st);
   return wg128 >= 256 ? launch_attn_fwd_tile<T, 256, 4, 2, 32, 2>(p, batch, st) : launch_attn_fwd_tile<T, 256, 2, 2, 32, 1>(p, batch, st);
 }
@@ -443,12 +464,14 @@ int attn_fwd_f32(const void *q, const void *k, const void *v, void *out, float *
 
 }  // namespace dh
 
-extern "C" int dh_attn_fwd(const void *q, const void *k, const void *v, void *out, float *lse,
-                           const int32_t *cu_seqlens_q, const int32_t *cu_seqlens_k, int batch, int max_seqlen_q,
-                           int max_seqlen_k, int hq, int hk, int d, int64_t q_stride, int64_t k_stride,
-                           int64_t v_stride, int64_t o_stride, float softmax_scale, int causal, int dtype,
-                           void *stream) {
+extern "C" int dh_attn_fwd_halves(const void *q, const void *k, const void *v, void *out, float *lse,
+                                  const int32_t *cu_seqlens_q, const int32_t *cu_seqlens_k, int q_shift, int k_shift,
+                                  int batch, int max_seqlen_q, int max_seqlen_k, int hq, int hk, int d,
+                                  int64_t q_stride, int64_t k_stride, int64_t v_stride, int64_t o_stride,
+                                  float softmax_scale, int causal, int dtype, void *stream) {
   using namespace dh;
+  DH_CHECK((q_shift == 0 || q_shift == 1) && (k_shift == 0 || k_shift == 1), "sequences are taken whole or halved");
+  DH_CHECK(dtype != DH_F32 || q_shift + k_shift == 0, "fp32 attention takes whole sequences");
   DH_CHECK(batch >= 0 && max_seqlen_q >= 0 && max_seqlen_k >= 0, "negative size");
   DH_CHECK(hq > 0 && hk > 0 && hq % hk == 0, "hq=%d must be a positive multiple of hk=%d", hq, hk);
   if (batch == 0 || max_seqlen_q == 0) return DH_OK;
@@ -477,11 +500,10 @@ extern "C" int dh_attn_fwd(const void *q, const void *k, const void *v, void *ou
   p.scale = softmax_scale;
   p.scale_log2 = softmax_scale * 1.4426950408889634f;
   p.causal = causal;
+  p.q_shift = q_shift; p.k_shift = k_shift;
   int rc;
-  if (d == 128) {
-    // 128-row query tiles when that still gives every CU a workgroup, else 64-row tiles.
-    const int64_t wg128 = (causal ? (cdiv(max_seqlen_q, 128) + 1) / 2 : cdiv(max_seqlen_q, 128)) * hq * batch;
-    const bool big = wg128 >= DH_FWD_128ROW_MIN_WG;
+  if (d == 128 && attn_fwd_fills(max_seqlen_q, hq, batch, causal)) {
+    const bool big = attn_fwd_wgs(max_seqlen_q, 128, hq, batch, causal) >= DH_FWD_128ROW_MIN_WG;
     if (dtype == DH_BF16) rc = big ? launch_attn_fwd_d128<bf16_t, 4, 2, 64, DH_FWD_LAG>(p, batch, st) : launch_attn_fwd_d128<bf16_t, 2, 4, 32, DH_FWD_LAG>(p, batch, st);
     else rc = big ? launch_attn_fwd_d128<f16_t, 4, 2, 64, DH_FWD_LAG>(p, batch, st) : launch_attn_fwd_d128<f16_t, 2, 4, 32, DH_FWD_LAG>(p, batch, st);
   } else {
@@ -490,4 +512,13 @@ extern "C" int dh_attn_fwd(const void *q, const void *k, const void *v, void *ou
   if (rc != DH_OK) return rc;
   DH_LAUNCH_CHECK();
   return DH_OK;
+}
+
+extern "C" int dh_attn_fwd(const void *q, const void *k, const void *v, void *out, float *lse,
+                           const int32_t *cu_seqlens_q, const int32_t *cu_seqlens_k, int batch, int max_seqlen_q,
+                           int max_seqlen_k, int hq, int hk, int d, int64_t q_stride, int64_t k_stride,
+                           int64_t v_stride, int64_t o_stride, float softmax_scale, int causal, int dtype,
+                           void *stream) {
+  return dh_attn_fwd_halves(q, k, v, out, lse, cu_seqlens_q, cu_seqlens_k, 0, 0, batch, max_seqlen_q, max_seqlen_k, hq, hk, d,
+                            q_stride, k_stride, v_stride, o_stride, softmax_scale, causal, dtype, stream);
 }

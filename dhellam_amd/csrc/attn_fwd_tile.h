@@ -1,15 +1,16 @@
-// Head dim 64 forward (16 bits).  A workgroup is 8 wavefronts = RG row groups (32 query rows each) x SPLIT key splits; an
-// iteration has SPLIT tiles of BN keys (K and V) in LDS, split s works on tile it * SPLIT + s, and the tiles of the next
-// iteration are copied global -> LDS meanwhile (two stages).  S^T = K Q^T puts a query row on each lane, P^T goes straight
-// back in as the operand of O^T += V^T P^T; the splits' (O, m, l) are merged through LDS in split order.
+// Attention forward on the tile layout of attn_tile.h (16 bits).  A workgroup is RG row groups (32 query rows each) x SPLIT
+// key splits; an iteration has SPLIT tiles of BN keys (K and V) in LDS, split s works on tile it * SPLIT + s, and the tiles of
+// the next iteration are copied global -> LDS meanwhile (two stages).  S^T = K Q^T puts a query row on each lane, P^T goes
+// straight back in as the operand of O^T += V^T P^T; the splits' (O, m, l) are merged through LDS in split order.
 //
-// What bounds it: at head dim 64 a 32 x 32 score block is 8 matrix instructions (256 cycles) and about 100 vector
-// instructions of softmax (400 cycles), so the vector unit and, for short sequences, the chain of one wavefront.  The kernel
-// therefore fits 128 registers: two workgroups, 16 wavefronts, on a compute unit, whose matrix, softmax and LDS phases fill
-// each other's waits without hand-written ordering.
-// Measured against the register-staged kernel that this head dim ran before (one wavefront per row group, padded tiles):
-// 2 x 512 rows, 16 heads 15.5 -> 9.4 us; forward and backward together, causal: 16 heads x 4096 548 -> 287 us, 32 query /
-// 8 kv heads x 4096 1505 -> 410 us.
+// What bounds it: a 32 x 32 score block is D / 8 matrix instructions (D / 8 x 32 cycles) and about 100 vector instructions of
+// softmax (400 cycles and more), so at head dim 64 the vector unit, at all of them the issue rate of the few wavefronts that
+// fit, and for short sequences the chain of one wavefront.  Head dims 64 and 96 therefore fit 128 registers: two
+// workgroups, 16 wavefronts, on a compute unit, whose matrix, softmax and LDS phases fill each other's waits without
+// hand-written ordering (WPS: wavefronts per SIMD).
+// Measured against the register-staged kernels that these head dims ran before, forward, causal: 16 heads x 2 x 512,
+// head dim 64 15.5 -> 9.4 us; 32 query / 8 kv heads x 4096, head dim 64 192 -> 94, 96 272 -> 132, 256 910 -> 329 us; 16
+// heads x 2048, head dim 192 324 -> 56 us.
 #include "attn_tile.h"
 
 namespace dh {
@@ -34,8 +35,8 @@ __global__ void __launch_bounds__(64 * RG * SPLIT, WPS) attn_fwd_tile_kernel(con
   int hkv, item;
   xcd_group_item(blockIdx.x, p.hk, ratio * P, hkv, item);
   const int h = hkv * ratio + item % ratio, px = item / ratio;
-  const int q0 = p.cu_q[b], sq = p.cu_q[b + 1] - q0;
-  const int k0 = p.cu_k[b], sk = p.cu_k[b + 1] - k0;
+  const int q0 = p.cu_q[b] >> p.q_shift, sq = (p.cu_q[b + 1] >> p.q_shift) - q0;
+  const int k0 = p.cu_k[b] >> p.k_shift, sk = (p.cu_k[b + 1] >> p.k_shift) - k0;
   const int nqt = (sq + BM - 1) / BM;
   if (px >= nqt) return;
   const int m0 = (nqt - 1 - px) * BM;

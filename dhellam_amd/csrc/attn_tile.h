@@ -1,10 +1,11 @@
-// Tile layout of the attention kernels that leave scheduling to the compiler (16 bits; head dims 64, 96, 192, 256).
+// Tile layout of the attention kernels that leave scheduling to the compiler (16 bits; all head dims, 128
+// where its hand-ordered kernels are not the faster ones).
 //
 // A tile of 32 n rows of D elements lies in LDS without padding; the 16-byte chunk index of a row is XORed with swz(row).
 // Both ways of reading are then free of bank conflicts:
 //   * row fragments (ds_read_b128, 16 lanes = one chunk of 16 consecutive rows): where the row pitch 2 D puts 16 / n of the
 //     rows on different multiples of 16 n bytes of the 256 that the banks span (n = 4 at D = 96, 8 at 64 and 192, 16 at
-//     256), the XOR of the low log2(n) chunk bits tells the others apart: 16 different chunks;
+//     128 and 256), the XOR of the low log2(n) chunk bits tells the others apart: 16 different chunks;
 //   * transpose reads (32 lanes = 4 consecutive rows x 4 neighbouring chunks): the pitch or bits 2 and 3 of the XOR put
 //     the rows into the four 64-byte quarters of the banks, the chunks fill a quarter.
 // Tiles are filled by global -> LDS copies of 1 KB per wavefront instruction with the swizzle on the global side; the

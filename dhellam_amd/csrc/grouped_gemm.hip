@@ -57,6 +57,9 @@ __device__ __forceinline__ void gg_tile_of(int t, int tiles_m, int tiles_n, int 
   tn = in_band / gm;
 }
 
+// Entry i of the offsets table; without a table there is one group of all max_rows rows.
+__device__ __forceinline__ int gg_off(const GGParams &p, int i) { return p.offs ? p.offs[i] : i * p.max_rows; }
+
 // A group's row range as the kernels use it: relative to the first group and never past the rows the caller's
 // buffers hold, whatever the offsets say (they live on the device, so the host cannot check them).
 __device__ __forceinline__ int gg_clamp_row(int r, int max_rows) { return r < 0 ? 0 : (r > max_rows ? max_rows : r); }
@@ -70,8 +73,8 @@ __device__ __forceinline__ GGGroupTable gg_group_table(const GGParams &p, int ba
   const int lane = threadIdx.x & 63;
   int rb = 0, re = 0;
   if (lane < p.groups) {
-    rb = gg_clamp_row(p.offs[lane] - base, p.max_rows);
-    re = gg_clamp_row(p.offs[lane + 1] - base, p.max_rows);
+    rb = gg_clamp_row(gg_off(p, lane) - base, p.max_rows);
+    re = gg_clamp_row(gg_off(p, lane + 1) - base, p.max_rows);
   }
   int incl = (re - rb + BM - 1) / BM;
 #pragma unroll
@@ -221,13 +224,13 @@ __global__ void __launch_bounds__(256) grouped_gemm_w4_kernel(const GGParams p) 
   const int nsl = (int)(p.k_dim / 64);
   const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
   const uint32_t lda_b = (uint32_t)p.lda * (uint32_t)sizeof(T), ldb_b = (uint32_t)p.ldb * (uint32_t)sizeof(T);
-  const int base = p.offs[0];
+  const int base = gg_off(p, 0);
 
   // Rows of c past the last group, up to max_rows (usually none): zeroed here, a row per workgroup at a time, instead
   // of by a kernel of its own in front of this one (5 us per product).
   if constexpr (!AKS) {
     if (p.zero_tail) {
-      const int first = gg_clamp_row(p.offs[p.groups] - base, p.max_rows);
+      const int first = gg_clamp_row(gg_off(p, p.groups) - base, p.max_rows);
       const int nv = (int)(p.n_dim / 8);
       for (int r = first + (int)blockIdx.x; r < p.max_rows; r += (int)gridDim.x) {
         T *row = reinterpret_cast<T *>(p.c) + (int64_t)r * p.ldc;
@@ -464,7 +467,7 @@ __global__ void __launch_bounds__(256) grouped_gemm_w4_kernel(const GGParams p) 
     int pid = blockIdx.x;
     pid = gg_xcd_chunk(pid, ntiles);
     const int g = blockIdx.y;
-    const int rb = gg_clamp_row(p.offs[g] - base, p.max_rows), re = gg_clamp_row(p.offs[g + 1] - base, p.max_rows);
+    const int rb = gg_clamp_row(gg_off(p, g) - base, p.max_rows), re = gg_clamp_row(gg_off(p, g + 1) - base, p.max_rows);
     int tm, tn;
     gg_tile_of(pid, p.tiles_m, p.tiles_n, tm, tn);
     segment(g, rb, re, tm, tn, 0, (re - rb + 63) / 64, nullptr);
@@ -516,10 +519,10 @@ template <typename T>
 __global__ void __launch_bounds__(256) gg_split_reduce_kernel(const GGParams p, int sk_grid) {
   constexpr int BM = 256;
   const int nsl = (int)(p.k_dim / 64);
-  const int base = p.offs[0];
+  const int base = gg_off(p, 0);
   int tiles_m = 0;
   for (int gi = 0; gi < p.groups; ++gi)
-    tiles_m += (gg_clamp_row(p.offs[gi + 1] - base, p.max_rows) - gg_clamp_row(p.offs[gi] - base, p.max_rows) + BM - 1) / BM;
+    tiles_m += (gg_clamp_row(gg_off(p, gi + 1) - base, p.max_rows) - gg_clamp_row(gg_off(p, gi) - base, p.max_rows) + BM - 1) / BM;
   const int tiles = tiles_m * p.tiles_n, full = tiles / sk_grid, rem = tiles - full * sk_grid;
   const int ts = blockIdx.x / 16;                       // tile of the last round
   if (ts >= rem || nsl == 0) return;
@@ -541,7 +544,7 @@ __global__ void __launch_bounds__(256) gg_split_reduce_kernel(const GGParams p, 
   gg_tile_of(t, tiles_m, p.tiles_n, tm, tn);
   int rb = 0, re = 0;
   for (int gi = 0; gi < p.groups; ++gi) {
-    rb = gg_clamp_row(p.offs[gi] - base, p.max_rows); re = gg_clamp_row(p.offs[gi + 1] - base, p.max_rows);
+    rb = gg_clamp_row(gg_off(p, gi) - base, p.max_rows); re = gg_clamp_row(gg_off(p, gi + 1) - base, p.max_rows);
     const int nt = (re - rb + BM - 1) / BM;
     if (tm < nt) break;
     tm -= nt;
@@ -617,7 +620,7 @@ struct GGUnit { int g, rb, re, tm, tn, s0, s1, piece; bool on; };   // slices s0
 template <int FORM, int BM, int BN>
 __device__ __forceinline__ GGUnit gg_t_unit(const GGParams &p, int id) {
   GGUnit u{};
-  const int base = p.offs[0];
+  const int base = gg_off(p, 0);
   int t, tiles_m, ntiles, nsl = 0, pieces;
   GGGroupTable gt{};
   if constexpr (FORM == 2) {
@@ -639,8 +642,8 @@ __device__ __forceinline__ GGUnit gg_t_unit(const GGParams &p, int id) {
     u.g = __builtin_amdgcn_readfirstlane(t / (tiles_m * p.tiles_n));
     t -= u.g * tiles_m * p.tiles_n;
     gg_tile_of(t, tiles_m, p.tiles_n, u.tm, u.tn);
-    u.rb = gg_clamp_row(p.offs[u.g] - base, p.max_rows);
-    u.re = gg_clamp_row(p.offs[u.g + 1] - base, p.max_rows);
+    u.rb = gg_clamp_row(gg_off(p, u.g) - base, p.max_rows);
+    u.re = gg_clamp_row(gg_off(p, u.g + 1) - base, p.max_rows);
     nsl = u.re > u.rb ? (u.re - u.rb + 63) / 64 : 0;
   } else {
     int tm_all;
@@ -671,7 +674,7 @@ __global__ void __launch_bounds__(2 * BN, 2) grouped_gemm_t_kernel(const GGParam
 
   // rows of c past the last group, up to max_rows, are zeroed here
   if constexpr (!AKS) {
-    const int first = gg_clamp_row(p.offs[p.groups] - p.offs[0], p.max_rows);
+    const int first = gg_clamp_row(gg_off(p, p.groups) - gg_off(p, 0), p.max_rows);
     const int nv = (int)(p.n_dim / 8);
     for (int r = first + (int)blockIdx.x; r < p.max_rows; r += (int)gridDim.x) {
       T *row = reinterpret_cast<T *>(p.c) + (int64_t)r * p.ldc;
@@ -888,7 +891,7 @@ template <typename T, int FORM, int BM, int BN>
 __global__ void __launch_bounds__(256) gg_t_reduce_kernel(const GGParams p) {
   using C = GGT<FORM, BM, BN>;
   constexpr int BLOCKS = BM * BN / 1024;                          // 32x32 blocks of a tile
-  const int lane = threadIdx.x & 63, base = p.offs[0];
+  const int lane = threadIdx.x & 63, base = gg_off(p, 0);
   const int id = (int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int t = id / BLOCKS, blk = id % BLOCKS;
   int ntiles, tm, tn, rb, re, g, pieces;
@@ -1065,7 +1068,7 @@ static bool gg_w4_pays(int64_t rows, int64_t n, int64_t k) {
 static int gg_common_checks(const void *a, const void *b, void *c, const int32_t *offs, int groups, int dtype) {
   DH_CHECK(groups >= 1 && groups <= GG_MAX_GROUPS, "groups=%d must be in [1, %d]", groups, GG_MAX_GROUPS);
   DH_CHECK(dtype == DH_BF16 || dtype == DH_F16, "grouped GEMM supports bf16/fp16 (dtype %d)", dtype);
-  DH_CHECK(a && b && c && offs, "null pointer");
+  DH_CHECK(a && b && c && (offs || groups == 1), "null pointer");
   DH_CHECK(aligned16(a) && aligned16(b) && aligned16(c), "operands must be 16-byte aligned");
   return DH_OK;
 }

@@ -380,6 +380,29 @@ Tensor matmul(const Tensor &A, const Tensor &B, const OptTensor &out, bool trans
   return d;
 }
 
+// Data gradient grad [T, N] @ weight [N, K] as given.  Long reductions of few rows go to the grouped kernel with one group,
+// which splits them over the chip: us, library / here, T = 256 and 1000: N, K = 8192, 1024 28 / 22 and 44 / 31; 8192, 3584
+// 45 / 29 and 74 / 70; 7168, 8192 71 / 43 and 107 / 113 (hence few rows only for wide results).
+Tensor dgrad(const Tensor &grad, const Tensor &weight, const OptTensor &out, const OptStream &stream) {
+  const int64_t t = grad.size(0), n = weight.size(0), k = weight.size(1);
+  const auto ok = [](const Tensor &x) { return x.is_contiguous() && (uintptr_t)x.data_ptr() % 16 == 0; };
+  if (grad.dim() == 2 && weight.dim() == 2 && grad.size(1) == n && n >= 5120 && t > 0 && (t <= 256 || (k <= 4096 && t <= 1024)) &&
+      n % 64 == 0 && k % 8 == 0 && weight.is_cuda() && grad.is_cuda() &&
+      (grad.scalar_type() == at::kBFloat16 || grad.scalar_type() == at::kHalf) && weight.scalar_type() == grad.scalar_type() &&
+      ok(grad) && ok(weight) && (!out.has_value() || (ok(*out) && out->scalar_type() == grad.scalar_type() && out->numel() == t * k))) {
+    On on(stream);
+    Tensor d = out.has_value() ? *out : at::empty({t, k}, grad.options());
+    Tensor ws = scratch(kGrouped, (int64_t)dh_grouped_gemm_workspace_bytes(), grad, on.get());
+    const int type = dt(grad);
+    launch([&] {
+      return dh_grouped_gemm_nn(grad.data_ptr(), weight.data_ptr(), d.data_ptr(), nullptr, 1, t, k, n, type, ws.data_ptr(),
+                                (size_t)ws.numel(), on.get());
+    });
+    return d;
+  }
+  return matmul(weight, grad, out, false, stream);
+}
+
 Tensor transpose_2d(const Tensor &src, const OptTensor &out, const OptStream &stream) {
   need_gpu({&src});
   TORCH_CHECK(src.dim() == 2 && src.stride(1) == 1, "transpose_2d: src must be 2-D with unit inner stride");
@@ -446,6 +469,142 @@ void attn_bwd(const Tensor &dout, const Tensor &q, const Tensor &k, const Tensor
   });
 }
 
+// ---- attention on the packed projection, as a layer calls it: split, RoPE (inv_freq given), attention in one call ------------
+// Packed rows are [q heads of the group | k | v] per kv group; one group: q, k, v are views, several: contiguous copies.
+// -> (out [T, hq, d], q, k, v, lse)
+std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor> attn_fwd_packed(const Tensor &qkv, const Tensor &cu_q, const Tensor &cu_k, int64_t hq,
+                                                                   int64_t hk, int64_t d, int seq, double scale,
+                                                                   const OptTensor &inv_freq, const OptStream &stream) {
+  TORCH_CHECK(qkv.dim() == 2 && qkv.is_contiguous() && qkv.size(1) == (hq + 2 * hk) * d && hq % hk == 0, "packed qkv: [T, (hq + 2 hk) d]");
+  On on(stream);
+  const int64_t t = qkv.size(0), r = hq / hk;
+  Tensor q, k, v;
+  if (hk == 1) {
+    q = qkv.as_strided({t, hq, d}, {qkv.size(1), d, 1});
+    k = qkv.as_strided({t, 1, d}, {qkv.size(1), d, 1}, qkv.storage_offset() + hq * d);
+    v = qkv.as_strided({t, 1, d}, {qkv.size(1), d, 1}, qkv.storage_offset() + (hq + 1) * d);
+  } else {
+    const Tensor g = qkv.view({t, hk, (r + 2) * d});
+    q = g.narrow(2, 0, r * d).contiguous().view({t, hq, d});
+    k = g.narrow(2, r * d, d).contiguous();
+    v = g.narrow(2, (r + 1) * d, d).contiguous();
+  }
+  if (inv_freq.has_value()) rope(q, k, *inv_freq, std::nullopt, seq, false, true, stream);
+  auto [out, lse] = attn_fwd(q, k, v, cu_q, cu_k, seq, seq, scale, true, stream);
+  return {out, q, k, v, lse};
+}
+
+// -> the packed gradient [T, (hq + 2 hk) d]
+Tensor attn_bwd_packed(const Tensor &dout, const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &out, const Tensor &lse,
+                       const Tensor &cu_q, const Tensor &cu_k, int seq, double scale, const OptTensor &inv_freq,
+                       const OptStream &stream) {
+  const int64_t t = q.size(0), hq = q.size(1), hk = k.size(1), d = q.size(2), r = hq / hk, width = (hq + 2 * hk) * d;
+  On on(stream);
+  Tensor packed = at::empty({t, width}, q.options()), dq, dk, dv;
+  if (hk == 1) {
+    dq = packed.as_strided({t, hq, d}, {width, d, 1});
+    dk = packed.as_strided({t, 1, d}, {width, d, 1}, hq * d);
+    dv = packed.as_strided({t, 1, d}, {width, d, 1}, (hq + 1) * d);
+  } else {
+    dq = at::empty(q.sizes(), q.options());
+    dk = at::empty(k.sizes(), k.options());
+    dv = at::empty(v.sizes(), v.options());
+  }
+  attn_bwd(dout.view({t, hq, d}), q, k, v, out, lse, dq, dk, dv, std::nullopt, cu_q, cu_k, seq, seq, scale, true, false, stream);
+  if (inv_freq.has_value()) rope(dq, dk, *inv_freq, std::nullopt, seq, true, true, stream);
+  if (hk != 1) {
+    Tensor to = packed.view({t, hk, (r + 2) * d});
+    at::cat_out(to, {dq.view({t, hk, r * d}), dk, dv}, 2);
+  }
+  return packed;
+}
+
+// ---- context-parallel ring steps, causal, batch 1: one call each, on halves addressed in place ---------------------------
+// q [1, 2, c, hq, d], kv [2, 1, 2, c, hk, d]; step 0 is the diagonal, steps up to the rank take the first half of the visiting
+// keys, later ones the second half of the queries.  A step in Python is a dozen views, a halved cu_seqlens (a kernel each) and
+// for the backward a copy of half of lse: 40 us of host time forward and 55 us backward, 12 and 17 us from here.
+struct RingStep {
+  bool fits = false, half_q = false, half_k = false;
+  int64_t c = 0, hq = 0, hk = 0, d = 0;
+  RingStep(const Tensor &q, const Tensor &kv, int step, int rank) {
+    if (!(q.is_cuda() && kv.is_cuda() && q.dim() == 5 && kv.dim() == 6 && q.is_contiguous() && kv.is_contiguous() &&
+          q.scalar_type() == kv.scalar_type() && (q.scalar_type() == at::kBFloat16 || q.scalar_type() == at::kHalf)))
+      return;
+    c = q.size(2);
+    hq = q.size(3);
+    d = q.size(4);
+    hk = kv.size(4);
+    fits = q.size(0) == 1 && q.size(1) == 2 && kv.size(0) == 2 && kv.size(1) == 1 && kv.size(2) == 2 && kv.size(3) == c &&
+           kv.size(5) == d && c > 0 && (d == 64 || d == 96 || d == 128 || d == 192 || d == 256) &&
+           (uintptr_t)q.data_ptr() % 16 == 0 && (uintptr_t)kv.data_ptr() % 16 == 0;
+    half_k = step > 0 && step <= rank;
+    half_q = step > rank;
+    if (step == 0) half_q = false;
+  }
+  int64_t rows_q() const { return half_q ? c : 2 * c; }
+  int64_t rows_k() const { return half_k ? c : 2 * c; }
+};
+char *at_row(const Tensor &t, int64_t row, int64_t heads, int64_t d) { return (char *)t.data_ptr() + row * heads * d * t.element_size(); }
+
+// -> (out [rows, hq, d], lse [1, hq, rows]), or None where the operands are not of that form
+py::object ring_fwd(const Tensor &q, const Tensor &kv, const Tensor &cu_q, const Tensor &cu_k, int64_t max_q, int64_t max_k,
+                    int step, int rank, double scale, const OptStream &stream) {
+  const RingStep r(q, kv, step, rank);
+  if (!r.fits || max_q != 2 * r.c || max_k != 2 * r.c || cu_q.scalar_type() != at::kInt || cu_k.scalar_type() != at::kInt ||
+      cu_q.numel() != 2 || cu_k.numel() != 2)
+    return py::none();
+  const int type = dt(q);
+  const int64_t nq = r.rows_q(), nk = r.rows_k(), qs = r.hq * r.d, ks = r.hk * r.d;
+  On on(stream);
+  Tensor out = at::empty({nq, r.hq, r.d}, q.options()), lse = at::empty({1, r.hq, nq}, q.options().dtype(at::kFloat));
+  launch([&] {
+    return dh_attn_fwd_halves(at_row(q, r.half_q ? r.c : 0, r.hq, r.d), kv.data_ptr(), at_row(kv, 2 * r.c, r.hk, r.d), out.data_ptr(),
+                              lse.data_ptr<float>(), cu_q.data_ptr<int>(), cu_k.data_ptr<int>(), r.half_q, r.half_k, 1, (int)nq,
+                              (int)nk, (int)r.hq, (int)r.hk, (int)r.d, qs, ks, ks, qs, (float)scale, step == 0, type, on.get());
+  });
+  return py::make_tuple(out, lse);
+}
+
+// -> (dq like q, dkv like kv), or None; a step's dq is stored by the backward's first call and added by the later ones
+py::object ring_bwd(const Tensor &dout, const Tensor &out, const Tensor &q, const OptTensor &dq_in, const Tensor &kv, const Tensor &lse,
+                    const Tensor &cu_q, const Tensor &cu_k, int64_t max_q, int64_t max_k, int step, int rank, bool first, double scale,
+                    const OptStream &stream) {
+  const RingStep r(q, kv, step, rank);
+  if (!r.fits || max_q != 2 * r.c || max_k != 2 * r.c || cu_q.scalar_type() != at::kInt || cu_k.scalar_type() != at::kInt ||
+      cu_q.numel() != 2 || cu_k.numel() != 2 || !dout.is_contiguous() || !out.is_contiguous() || dout.numel() != q.numel() ||
+      out.numel() != q.numel() || dout.scalar_type() != q.scalar_type() || out.scalar_type() != q.scalar_type() ||
+      !lse.is_contiguous() || lse.scalar_type() != at::kFloat || lse.numel() != 2 * r.c * r.hq ||
+      (dq_in.has_value() && !(dq_in->is_contiguous() && dq_in->numel() == q.numel() && dq_in->scalar_type() == q.scalar_type())))
+    return py::none();
+  const int type = dt(q);
+  const int64_t nq = r.rows_q(), nk = r.rows_k(), q_at = r.half_q ? r.c : 0, qs = r.hq * r.d, ks = r.hk * r.d;
+  On on(stream);
+  Tensor dq = dq_in.has_value() ? *dq_in : at::empty(q.sizes(), q.options());
+  Tensor dkv = at::empty(kv.sizes(), kv.options());
+  if (r.half_k) dkv.select(2, 1).zero_();
+  if (first && r.half_q) dq.select(1, 0).zero_();      // the first contribution to these rows is an addition
+  const size_t bytes = dh_attn_bwd_workspace_bytes(nq, nk, 1, (int)nq, (int)r.hq, (int)r.hk, (int)r.d, type);
+  Tensor ws = scratch(kAttnBwd, (int64_t)bytes, q, on.get());
+  launch([&] {
+    return dh_attn_bwd_halves(at_row(dout, q_at, r.hq, r.d), at_row(q, q_at, r.hq, r.d), kv.data_ptr(), at_row(kv, 2 * r.c, r.hk, r.d),
+                              at_row(out, q_at, r.hq, r.d), lse.data_ptr<float>() + q_at, at_row(dq, q_at, r.hq, r.d), dkv.data_ptr(),
+                              at_row(dkv, 2 * r.c, r.hk, r.d), nullptr, ws.data_ptr(), (size_t)ws.numel(), cu_q.data_ptr<int>(),
+                              cu_k.data_ptr<int>(), r.half_q, r.half_k, (int)(2 * r.c), 1, (int)nq, (int)nk, nq, nk, (int)r.hq, (int)r.hk,
+                              (int)r.d, qs, ks, ks, qs, qs, qs, ks, ks, (float)scale, step == 0, !first, type, on.get());
+  });
+  return py::make_tuple(dq, dkv);
+}
+
+// Running log-sum-exp of a ring: a copy of the first step's, or `next` folded into it in place (half: its second half of rows).
+Tensor ring_lse(const OptTensor &running, const Tensor &next, bool half, const OptStream &stream) {
+  On on(stream);
+  if (!running.has_value()) return next.clone();
+  Tensor dst = *running;
+  if (half) dst = dst.narrow(-1, dst.size(-1) / 2, dst.size(-1) / 2);
+  at::logaddexp_out(dst, dst, next);
+  return *running;
+}
+
 void attn_merge(const std::vector<Tensor> &outs, const std::vector<Tensor> &lses, const std::vector<int> &row_begin,
                 const std::vector<int> &rows, const Tensor &out, const Tensor &lse, const OptStream &stream) {
   const size_t n = outs.size();
@@ -469,6 +628,18 @@ void attn_merge(const std::vector<Tensor> &outs, const std::vector<Tensor> &lses
     return dh_attn_merge(po.data(), pl.data(), row_begin.data(), rows.data(), (int)n, out.data_ptr(), lse.data_ptr<float>(),
                          (int)b, (int)sq, (int)hq, (int)d, type, on.get());
   });
+}
+
+// attn_merge into new tensors: (out [b * sq, hq, d], lse [b, hq, sq])
+std::tuple<Tensor, Tensor> attn_merge_new(const std::vector<Tensor> &outs, const std::vector<Tensor> &lses,
+                                          const std::vector<int> &row_begin, const std::vector<int> &rows, int64_t b, int64_t sq,
+                                          const OptStream &stream) {
+  PY_ASSERT(!outs.empty() && outs.size() == lses.size() && outs[0].dim() == 3, "merge: one entry per step in every list");
+  On on(stream);
+  Tensor out = at::empty({b * sq, outs[0].size(1), outs[0].size(2)}, outs[0].options());
+  Tensor lse = at::empty({b, outs[0].size(1), sq}, lses[0].options());
+  attn_merge(outs, lses, row_begin, rows, out, lse, stream);
+  return {out, lse};
 }
 
 // ---- MoE ------------------------------------------------------------------------------------------------------------
@@ -623,6 +794,107 @@ Tensor embedding_fwd(const Tensor &vocab, const Tensor &ids, int64_t vocab_start
   return out;
 }
 
+void embedding_bwd(const Tensor &dout_in, const Tensor &ids_in, const Tensor &grad, int64_t vocab_start) {
+  need_gpu({&grad, &dout_in, &ids_in});
+  const Tensor dout = dout_in.contiguous(), ids = ids_in.contiguous();
+  PY_ASSERT(grad.dim() == 2 && grad.is_contiguous() && ids.scalar_type() == at::kLong && dout.numel() == ids.numel() * grad.size(1),
+            "embedding: contiguous gradient, int64 ids, one row of dout per id");
+  const int type = dt(dout), gtype = dt(grad);
+  On on(py::none{});
+  launch([&] {
+    return dh_embedding_bwd(dout.data_ptr(), ids.data_ptr<int64_t>(), ids.numel(), grad.size(1), grad.size(0), vocab_start, type,
+                            grad.data_ptr(), gtype, on.get());
+  });
+}
+
+Tensor rows_of(const Tensor &t, int64_t cols) {      // [..., cols] as rows of unit inner stride
+  Tensor x = t.reshape({-1, cols});
+  return x.stride(1) == 1 ? x : x.contiguous();
+}
+
+// -> (statistics [4, rows]: loss, row max, exp sum, target logit; softmax or None, target mask [rows], local target [rows])
+std::tuple<Tensor, OptTensor, Tensor, Tensor> cross_entropy_fwd(const Tensor &logits, const Tensor &target, int64_t vocab_start,
+                                                                double label_smoothing, bool keep_softmax) {
+  need_gpu({&logits, &target});
+  PY_ASSERT(logits.stride(-1) == 1 && target.scalar_type() == at::kLong && target.sizes() == logits.sizes().slice(0, logits.dim() - 1),
+            "cross_entropy: logits of unit inner stride, one int64 target per row");
+  const int64_t cols = logits.size(-1);
+  const Tensor x = rows_of(logits, cols), tgt = target.contiguous();
+  const int64_t rows = x.size(0);
+  const int type = dt(x);
+  On on(py::none{});
+  Tensor stats = at::empty({4, rows > 0 ? rows : 1}, logits.options().dtype(at::kFloat));
+  OptTensor softmax;
+  if (keep_softmax) softmax = at::empty({rows, cols}, logits.options());
+  Tensor mask = at::empty({rows}, logits.options().dtype(at::kBool)), local = at::empty({rows}, target.options());
+  float *st = stats.data_ptr<float>();
+  const int64_t pitch = stats.size(1);
+  launch([&] {
+    return dh_cross_entropy_fwd(x.data_ptr(), tgt.data_ptr<int64_t>(), rows, cols, x.stride(0), vocab_start, (float)label_smoothing, type,
+                                st, st + pitch, st + 2 * pitch, st + 3 * pitch, mptr(softmax), cols, (uint8_t *)mask.data_ptr(),
+                                local.data_ptr<int64_t>(), on.get());
+  });
+  return {stats, softmax, mask, local};
+}
+
+// grad (made here if not given) from the logits and their row statistics
+Tensor cross_entropy_bwd(const Tensor &logits, const Tensor &row_max, const Tensor &sum_exp, const Tensor &target, const Tensor &dout,
+                         int64_t vocab_start, double label_smoothing, const OptTensor &grad_out) {
+  need_gpu({&logits, &row_max, &sum_exp, &target, &dout});
+  const int64_t cols = logits.size(-1);
+  const Tensor x = rows_of(logits, cols), tgt = target.contiguous(), d = dout.to(at::kFloat).contiguous();
+  PY_ASSERT(d.numel() == tgt.numel() && x.size(0) == tgt.numel() && row_max.is_contiguous() && sum_exp.is_contiguous(),
+            "cross_entropy: one gradient and one pair of statistics per row");
+  const int type = dt(x);
+  On on(py::none{});
+  const Tensor g = grad_out.has_value() ? grad_out->view({-1, cols}) : at::empty({x.size(0), cols}, logits.options());
+  PY_ASSERT(g.scalar_type() == x.scalar_type() && g.stride(1) == 1, "cross_entropy: gradient of the logits' type, unit inner stride");
+  launch([&] {
+    return dh_cross_entropy_bwd(x.data_ptr(), x.stride(0), 1, row_max.data_ptr<float>(), sum_exp.data_ptr<float>(),
+                                tgt.data_ptr<int64_t>(), d.data_ptr<float>(), x.size(0), cols, vocab_start, (float)label_smoothing, type,
+                                g.data_ptr(), g.stride(0), on.get());
+  });
+  return g.view(logits.sizes());
+}
+
+// -> (out fp32 [2]: loss, mask sum; mask in fp32)
+std::tuple<Tensor, Tensor> masked_mean_fwd(const Tensor &losses, const Tensor &mask, double scale) {
+  need_gpu({&losses, &mask});
+  const Tensor x = losses.to(at::kFloat).contiguous(), m = mask.reshape({-1}).to(at::kFloat).contiguous();
+  PY_ASSERT(x.numel() == m.numel() && x.numel() > 0, "masked mean: one mask value per loss");
+  On on(py::none{});
+  Tensor out = at::empty({2}, x.options());
+  launch([&] {
+    return dh_masked_mean_fwd(x.data_ptr<float>(), m.data_ptr<float>(), x.numel(), (float)scale, out.data_ptr<float>(), on.get());
+  });
+  return {out, m};
+}
+
+Tensor masked_mean_bwd(const Tensor &mask, const Tensor &mask_sum, double scale) {
+  On on(py::none{});
+  Tensor g = at::empty({mask.numel()}, mask.options());
+  launch([&] {
+    return dh_masked_mean_bwd(mask.data_ptr<float>(), mask_sum.data_ptr<float>(), mask.numel(), (float)scale, g.data_ptr<float>(), on.get());
+  });
+  return g;
+}
+
+// Zeros in every tensor of the list (contiguous ones, neighbours in the list or not): one launch.
+void zero_all(const std::vector<Tensor> &ts, const OptStream &stream) {
+  On on(stream);
+  std::vector<void *> ptrs;
+  std::vector<int64_t> bytes;
+  for (const Tensor &t : ts) {
+    if (t.is_cuda() && t.is_contiguous() && t.nbytes() % 4 == 0 && (uintptr_t)t.data_ptr() % 16 == 0) {
+      ptrs.push_back(t.data_ptr());
+      bytes.push_back((int64_t)t.nbytes());
+    } else {
+      t.zero_();
+    }
+  }
+  if (!ptrs.empty()) launch([&] { return dh_zero_many(ptrs.data(), bytes.data(), (int)ptrs.size(), on.get()); });
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -640,10 +912,17 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("dense_gemm", &dense_gemm);
   m.def("linear", &linear);
   m.def("matmul", &matmul);
+  m.def("dgrad", &dgrad);
   m.def("transpose_2d", &transpose_2d);
   m.def("attn_fwd", &attn_fwd);
   m.def("attn_bwd", &attn_bwd);
+  m.def("attn_fwd_packed", &attn_fwd_packed);
+  m.def("attn_bwd_packed", &attn_bwd_packed);
+  m.def("ring_fwd", &ring_fwd);
+  m.def("ring_bwd", &ring_bwd);
+  m.def("ring_lse", &ring_lse);
   m.def("attn_merge", &attn_merge);
+  m.def("attn_merge_new", &attn_merge_new);
   m.def("moe_route", &moe_route);
   m.def("moe_sort", &moe_sort);
   m.def("moe_gather", &moe_gather);
@@ -654,4 +933,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("grouped_gemm", &grouped_gemm);
   m.def("grouped_gemm_tn", &grouped_gemm_tn);
   m.def("embedding_fwd", &embedding_fwd);
+  m.def("embedding_bwd", &embedding_bwd);
+  m.def("cross_entropy_fwd", &cross_entropy_fwd);
+  m.def("cross_entropy_bwd", &cross_entropy_bwd);
+  m.def("masked_mean_fwd", &masked_mean_fwd);
+  m.def("masked_mean_bwd", &masked_mean_bwd);
+  m.def("zero_all", &zero_all);
 }

@@ -12,7 +12,7 @@ from typing import Sequence
 
 import torch
 
-from .. import _host, _lib
+from .. import _host
 from ..common.parallel_state import get_tensor_model_parallel_rank, get_tensor_model_parallel_world_size
 
 
@@ -34,19 +34,15 @@ def word_embedding_fwd(inputs):
 
 def word_embedding_bwd(context, dout):
     inputs = context[0]
-    vocab, ids = inputs["vocab"], inputs["token_ids"].contiguous()
-    _lib.need_cuda(vocab, dout)
-    dout = dout.contiguous()
-    assert dout.dtype == vocab.dtype and dout.numel() == ids.numel() * vocab.shape[1]
+    vocab = inputs["vocab"]
+    assert dout.dtype == vocab.dtype
     grad = getattr(vocab, "main_grad", None)
     if grad is None:
         if vocab.grad is None:
             vocab.grad = torch.zeros_like(vocab)
         grad = vocab.grad
-    assert grad.is_contiguous() and grad.shape == vocab.shape
-    _lib.check(_lib.load().dh_embedding_bwd(dout.data_ptr(), ids.data_ptr(), ids.numel(), vocab.shape[1],
-                                            vocab.shape[0], _vocab_start(vocab), _lib.dt(dout), grad.data_ptr(),
-                                            _lib.dt(grad), _host.stream_ptr(None)))
+    assert grad.shape == vocab.shape
+    _host.embedding_bwd(dout, inputs["token_ids"], grad, _vocab_start(vocab))
     return None
 
 

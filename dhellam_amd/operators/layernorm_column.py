@@ -66,7 +66,7 @@ def dgrad_bwd(args, input_grad: torch.Tensor, weight: torch.Tensor, dgrad_output
     if (is_matmul and not profiling and not transa and not transb and dense_ok(weight, input_grad)
             and weight.dtype == input_grad.dtype
             and (dgrad_output is None or (dense_ok(dgrad_output) and dgrad_output.dtype == weight.dtype))):
-        return dgrad_gemm(input_grad, weight, dgrad_output, stream), 0
+        return dgrad_gemm(input_grad, weight, dgrad_output, stream, getattr(args, "resident_weight_transposes", True)), 0
     el: list = []
     with on_stream(stream, profiling, el):
         if dgrad_output is None:

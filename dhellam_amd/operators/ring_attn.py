@@ -30,7 +30,7 @@ from dataclasses import dataclass
 
 import torch
 
-from .. import _Clib
+from .. import _Clib, _host
 
 
 @dataclass(frozen=True)
@@ -60,6 +60,13 @@ def _scale(q, softmax_scale):
     return float(softmax_scale) if softmax_scale is not None else 1.0 / math.sqrt(q.shape[-1])
 
 
+def _merge(q, b, out_per_step, lse_per_step, rank, causal, sq, stream):
+    """(out [b sq, hq, d], lse [b, hq, sq]) from the steps' partial results, on ``stream``."""
+    halves = [causal and s > rank for s in range(len(out_per_step))]
+    return _host.attn_merge_new(out_per_step, lse_per_step, [sq // 2 if h else 0 for h in halves],
+                                [sq // 2 if h else sq for h in halves], b, sq, stream)
+
+
 def fa_cp_block_fwd(q, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, p2p_comm_buffers, out_per_step,
                     softmax_lse_per_step, rng_states, softmax_lse, softmax_lse_, i, causal, cp_group,
                     cp_global_ranks, stream, softmax_scale=None):
@@ -78,9 +85,24 @@ def fa_cp_block_fwd(q, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, p
         out_per_step = [None] * cp_size
         softmax_lse_per_step = [None] * cp_size
         rng_states = [None] * cp_size
+    hq, d = q.shape[-2], q.shape[-1]
+    if causal:       # batch 1 in 16 bits: the step is one native call
+        res = _host.ring_fwd(q, kv_inputs, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, i, rank, scale, stream)
+        if res is not None:
+            out_per_step[i], softmax_lse_per_step[i] = res
+            rng_states[i] = _Clib._zero_rng_state(q.device)
+            if i == cp_size - 1:
+                out, softmax_lse = _merge(q, 1, out_per_step, softmax_lse_per_step, rank, causal, max_seqlen_q, stream)
+                return out, q, p2p_comm_buffers[-1], softmax_lse, rng_states
+            if i > 0:        # running log-sum-exp over the steps before this one, as below
+                prev = softmax_lse_per_step[i - 1]
+                softmax_lse = _host.ring_lse(None if i == 1 else softmax_lse, prev, i - 1 > rank, stream)
+                if i == 1:
+                    softmax_lse_ = softmax_lse.view(*softmax_lse.shape[:-1], 2, -1)
+            return [q, p2p_comm_buffers, out_per_step, softmax_lse_per_step, rng_states, softmax_lse, softmax_lse_,
+                    i + 1], []
     if stream is None:
         stream = torch.cuda.current_stream()
-    hq, d = q.shape[-2], q.shape[-1]
 
     with torch.cuda.stream(stream):
         if causal:
@@ -121,15 +143,7 @@ def fa_cp_block_fwd(q, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, p
                 torch.logaddexp(softmax_lse, prev, out=softmax_lse)
 
         if i == cp_size - 1:
-            sq = max_seqlen_q
-            row_begin, rows = [], []
-            for s in range(cp_size):
-                half = causal and s > rank
-                row_begin.append(sq // 2 if half else 0)
-                rows.append(sq // 2 if half else sq)
-            out = torch.empty((b * sq, hq, d), dtype=q.dtype, device=q.device)
-            softmax_lse = torch.empty((b, hq, sq), dtype=torch.float32, device=q.device)
-            _Clib.pyattn_merge(out_per_step, softmax_lse_per_step, row_begin, rows, out, softmax_lse)
+            out, softmax_lse = _merge(q, b, out_per_step, softmax_lse_per_step, rank, causal, max_seqlen_q, stream)
             kv = p2p_comm_buffers[-1]
             return out, q, kv, softmax_lse, rng_states
     return [q, p2p_comm_buffers, out_per_step, softmax_lse_per_step, rng_states, softmax_lse, softmax_lse_,
@@ -155,11 +169,18 @@ def fa_cp_block_bwd(dout, out, q, dq, kv, dkv_, softmax_lse, rng_states, cu_seql
             dq = dq.view(q.shape[0], -1, *q.shape[-2:])
         return dq, dkv_
     scale = _scale(q, softmax_scale)
-    if stream is None:
-        stream = torch.cuda.current_stream()
     hq, d = q.shape[-2], q.shape[-1]
     step = cp_size - 1 - i
     kv_in = p2p_comm_buffers[step]
+    if causal:       # batch 1 in 16 bits: the step is one native call
+        res = _host.ring_bwd(dout, out, q, dq, kv_in, softmax_lse, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k,
+                             step, rank, i == 0, scale, stream)
+        if res is not None:
+            dkv_ = [None] * cp_size if dkv_ is None else dkv_
+            dq, dkv_[step] = res
+            return [dout if dout.shape == q.shape else dout.view(q.shape), dq, dkv_, p2p_comm_buffers, i + 1], []
+    if stream is None:
+        stream = torch.cuda.current_stream()
 
     with torch.cuda.stream(stream):
         if dkv_ is None:

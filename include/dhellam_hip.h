@@ -227,6 +227,29 @@ int dh_attn_bwd_acc(const void *dout, const void *q, const void *k,
                     int64_t dk_stride, int64_t dv_stride, float softmax_scale,
                     int causal, int accumulate_dq, int dtype, void *stream);
 
+/* The two steps of context parallelism that take half of every sequence: with q_shift (k_shift) = 1 sequence b's query
+ * (key) rows are cu[b] / 2 .. cu[b + 1] / 2 of what q (k, v) points to, and lse may be the table of the whole sequences
+ * (lse_pitch rows per head, the pointer at the half's first row).  16-bit types. */
+int dh_attn_fwd_halves(const void *q, const void *k, const void *v, void *out,
+                       float *lse, const int32_t *cu_seqlens_q,
+                       const int32_t *cu_seqlens_k, int q_shift, int k_shift,
+                       int batch, int max_seqlen_q, int max_seqlen_k, int hq,
+                       int hk, int d, int64_t q_stride, int64_t k_stride,
+                       int64_t v_stride, int64_t o_stride, float softmax_scale,
+                       int causal, int dtype, void *stream);
+int dh_attn_bwd_halves(const void *dout, const void *q, const void *k,
+                       const void *v, const void *out, const float *lse,
+                       void *dq, void *dk, void *dv, float *delta_out,
+                       void *workspace, size_t workspace_bytes,
+                       const int32_t *cu_seqlens_q, const int32_t *cu_seqlens_k,
+                       int q_shift, int k_shift, int lse_pitch, int batch,
+                       int max_seqlen_q, int max_seqlen_k, int64_t total_q,
+                       int64_t total_k, int hq, int hk, int d, int64_t q_stride,
+                       int64_t k_stride, int64_t v_stride, int64_t o_stride,
+                       int64_t do_stride, int64_t dq_stride, int64_t dk_stride,
+                       int64_t dv_stride, float softmax_scale, int causal,
+                       int accumulate_dq, int dtype, void *stream);
+
 /* ------------------------------------------------------------------------
  * Ring-attention merge of per-step partial results.
  * dhellam/operators/ring_attn.py:26-40 (lse and out correction) applied as in
@@ -322,6 +345,7 @@ int dh_moe_unpermute_bwd(const void *dout, const void *y, const int32_t *sorted_
  *   NT: c[rows_g, n] = a[rows_g, k] * b[g][n, k]^T          (forward)
  *   NN: c[rows_g, n] = a[rows_g, k] * b[g][k, n]            (dgrad)
  *   TN: c[g][m, n] (+)= a[rows_g, m]^T * b[rows_g, n]       (wgrad)
+ * offs may be NULL with one group: it then owns all max_rows rows (a plain product).
  * max_rows is the number of rows the stacked operands hold: it bounds the launch grid, group ranges read
  * from offs are cut off there (no row past it is read or written), and NT / NN zero the rows of c from the
  * last group's end up to max_rows, so c may be uninitialised on entry.
@@ -352,6 +376,9 @@ int dh_grouped_gemm_tn_ws(const void *a, const void *b, void *c,
                           const int32_t *offs, int groups, int64_t max_rows,
                           int64_t m, int64_t n, int accumulate, int dtype,
                           void *workspace, size_t workspace_bytes, void *stream);
+
+/* Zeros in n device buffers (16-byte aligned, sizes multiples of 4), one launch for up to 32 of them. */
+int dh_zero_many(void *const *ptrs, const int64_t *nbytes, int n, void *stream);
 
 /* Plain device-to-device copy kernel: a known-size streaming kernel used to
  * calibrate the profiler's HBM byte counters, and the local stand-in for the
