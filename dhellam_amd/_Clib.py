@@ -225,7 +225,8 @@ def wgrad_gemm(grad: torch.Tensor, data: torch.Tensor, out: torch.Tensor, accumu
 # transposes (9 / 7 / 38 / 20 us) cost less than one micro-batch saves, so a weight may be registered to be kept in
 # both layouts.  The copy lives on the tensor object.  Who keeps it current: the containers that run a step
 # (``LayerRunner.run_*``, ``DSLLMStep.step``, ``run_microbatches``) rebuild the copies of their weights at the START
-# of every step with ``refresh_transposed`` -- unconditionally, because the writers that matter do not announce
+# of every step with ``refresh_transposed`` (a step too short to read them marks them stale instead, with
+# ``forget_transposed``: the next reader rebuilds) -- unconditionally, because the writers that matter do not announce
 # themselves: ``p.data.copy_()`` / ``p.data.add_()`` (Megatron's fp16 and distributed optimizers), collectives and raw
 # kernels writing into a parameter buffer all leave the tensor's version counter where it was.  In between, a moved
 # version counter (any in-place torch op on the tensor itself) also triggers a rebuild at the next use.  A caller
@@ -241,8 +242,8 @@ def _register_kept(weight: torch.Tensor) -> None:
 
 
 class _Held:
-    """What a registered weight carries: the transpose, the version it was built from, the event and stream of
-    the build, and one event per stream that has read the copy since (a rebuild waits for them)."""
+    """What a registered weight carries: the transpose, the version it was built from (None: stale), the event and
+    stream of the build, and one event per stream that has read the copy since (a rebuild waits for them)."""
     __slots__ = ("version", "wt", "built", "stream_ptr", "readers")
 
     def __init__(self, version, wt, built, stream_ptr):
@@ -292,6 +293,15 @@ def refresh_transposed(weights=None) -> int:
             keep_transposed(w, refresh=True)
             n += 1
     return n
+
+
+def forget_transposed(weights) -> None:
+    """Marks the resident transposes of ``weights`` stale: the next reader rebuilds the copy it reads.  Stands for
+    ``refresh_transposed`` where the caller's own step does not read them."""
+    for w in weights:
+        held = getattr(w, "_dh_transposed", None)
+        if held is not None:
+            held.version = None
 
 
 def transposed_of(weight: torch.Tensor, stream=None) -> Optional[torch.Tensor]:

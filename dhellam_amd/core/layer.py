@@ -15,7 +15,7 @@ from typing import Dict, List, Optional
 import torch
 
 from .. import _host
-from .._Clib import keep_transposed, refresh_transposed
+from .._Clib import forget_transposed, keep_transposed, refresh_transposed
 from .dstb import DCoperation, LayerConfig, Plan, exec as exec_blocks, init_DCBlocks
 
 
@@ -143,20 +143,24 @@ class LayerRunner:
 
     def refresh_weight_transposes(self):
         """Rebuilds W^T of every projection weight on the current stream.  ``run_serial`` / ``run_double_strand``
-        call it at the start of every step: a step is what lies between two optimizer steps, and an optimizer that
-        writes through ``p.data`` (or a raw kernel, or a collective) leaves no trace a lazy check could see."""
+        call it at the start of every step that reads W^T: a step is what lies between two optimizer steps, and an
+        optimizer that writes through ``p.data`` (or a raw kernel, or a collective) leaves no trace a lazy check could
+        see."""
         if self.cfg.resident_weight_transposes:
             refresh_transposed(self.weights.values())
 
     def _step_config(self, mbs, refresh):
-        """The configuration a step runs with, its W^T rebuilt if it uses them (a caller that does not refresh keeps
-        them current itself)."""
-        if not refresh:
+        """The configuration a step runs with, its W^T rebuilt if it uses them and ``refresh`` asks for it.  A step that
+        does not use them leaves their rebuild to whoever reads them next: they are stale from here on."""
+        if not self.cfg.resident_weight_transposes:
             return self.cfg
-        if not self.cfg.resident_weight_transposes or self.cfg.tokens * len(mbs) < TRANSPOSES_MIN_ROWS:
-            return self.cfg_short
-        self.refresh_weight_transposes()
-        return self.cfg
+        short = self.cfg.tokens * len(mbs) < TRANSPOSES_MIN_ROWS
+        if refresh:
+            if short:
+                forget_transposed(self.weights.values())
+            else:
+                self.refresh_weight_transposes()
+        return self.cfg_short if short else self.cfg
 
     def run_serial(self, mbs: List[dict], refresh_transposes: bool = True):
         """F0 B0 F1 B1 ... on ONE stream with the fwd_only / bwd_only plans.  ``refresh_transposes=False`` is for a

@@ -332,22 +332,28 @@ def test_fused_adjacent_ops_give_the_bits_of_the_separate_ops():
         assert torch.equal(a, b)
 
 
+def _small_sharded_layer(seq_length):
+    from dhellam_amd.core.dstb import LayerConfig
+    return LayerConfig(hidden_size=1024, num_attention_heads=16, num_query_groups=2, ffn_hidden_size=2048,
+                       seq_length=seq_length, micro_batch_size=1, tensor_model_parallel_size=2, tp_rank=0,
+                       rope_theta=500000.0, params_dtype=torch.bfloat16)
+
+
 def test_weights_updated_around_the_version_counter_are_seen_by_the_next_step():
     """The projection weights are kept resident as W and W^T, and the data-gradient GEMMs read W^T.  An optimizer
     that writes through ``p.data`` (Megatron's do) does not move the tensor's version counter, so only an
     unconditional rebuild at the step boundary keeps W^T current: the step after such an update must give the
     gradients of the NEW weights: those of a layer that holds no resident transposes (the two take different GEMM
-    kernels for the data gradients, so they agree to rounding; against stale weights they would not agree at all)."""
+    kernels for the data gradients, so they agree to rounding; against stale weights they would not agree at all).
+    The sequences are long enough for a step to read W^T."""
     import dataclasses
-    from dhellam_amd.core.dstb import LayerConfig
     from dhellam_amd.core.layer import LayerRunner, make_microbatch, make_weights
-    cfg = LayerConfig(hidden_size=1024, num_attention_heads=16, num_query_groups=2, ffn_hidden_size=2048,
-                      seq_length=256, micro_batch_size=1, tensor_model_parallel_size=2, tp_rank=0,
-                      rope_theta=500000.0, params_dtype=torch.bfloat16)
+    cfg = _small_sharded_layer(2048)
     assert cfg.resident_weight_transposes
     w = make_weights(cfg, 0)
     mbs = [make_microbatch(cfg, i) for i in range(2)]
     runner = LayerRunner(cfg, w)
+    assert runner._step_config(mbs, True).resident_weight_transposes
     runner.run_double_strand(mbs)                                    # a first step with the initial weights
     new = make_weights(dataclasses.replace(cfg, resident_weight_transposes=False), 7)
     proj = ("column_attn_weight", "linear_attn_weight", "column_mlp_weight", "linear_mlp_weight")
@@ -372,3 +378,34 @@ def test_weights_updated_around_the_version_counter_are_seen_by_the_next_step():
     _, dxs_fresh = runner.run_double_strand(mbs)
     torch.cuda.synchronize()
     assert rel_err(dxs_stale[0], dxs_fresh[0]) > 0.1
+
+
+def test_a_short_step_leaves_no_stale_transposes_behind():
+    """Steps of few rows do not read W^T and do not rebuild it.  What follows such a step without an update in between
+    must still see the weights it saw: another short step, or a long one of a second runner on the same weights, both
+    with ``refresh_transposes=False`` (several calls between two updates)."""
+    import dataclasses
+    from dhellam_amd.core.layer import LayerRunner, make_microbatch, make_weights
+    short, long = _small_sharded_layer(256), _small_sharded_layer(4096)
+    w = make_weights(short, 0)
+    runner = LayerRunner(short, w)
+    runner.run_serial([make_microbatch(short, 0)])
+    new = make_weights(dataclasses.replace(short, resident_weight_transposes=False), 7)
+    for k in ("column_attn_weight", "linear_attn_weight", "column_mlp_weight", "linear_mlp_weight"):
+        w[k].data.copy_(new[k])
+    runner.run_serial([make_microbatch(short, 0)])
+    _, dxs = runner.run_serial([make_microbatch(short, 1)], refresh_transposes=False)
+    _, dxs_r = LayerRunner(dataclasses.replace(short, resident_weight_transposes=False), new).run_serial(
+        [make_microbatch(short, 1)])
+    torch.cuda.synchronize()
+    assert torch.equal(dxs[0], dxs_r[0])
+    cu = torch.tensor([0, 4096], dtype=torch.int32, device="cuda")
+    for d in (w, new):
+        d["cu_seqlens_q"] = d["cu_seqlens_kv"] = cu
+    runner = LayerRunner(long, w)
+    assert runner._step_config([None], False).resident_weight_transposes      # this one reads W^T
+    _, dxs = runner.run_serial([make_microbatch(long, 2)], refresh_transposes=False)
+    _, dxs_r = LayerRunner(dataclasses.replace(long, resident_weight_transposes=False), new).run_serial(
+        [make_microbatch(long, 2)])
+    torch.cuda.synchronize()
+    assert_close(dxs[0], dxs_r[0].cpu(), long.params_dtype, "dx (a stale W^T would be off by ~1)")
