@@ -1063,8 +1063,13 @@ def _block_steps(blk: DCBlock):
     return [(fwd, [_Step(op, col[i + 1] if i + 1 < len(col) else None) for i, op in enumerate(col)]) for fwd, col in cols]
 
 
+_PLAIN_PERFORM = DCoperation.perform_operation
+
+
 def _run_column(steps, dcoperation, config, weight, act, first_input, stream1, stream2, result, movable, fuse):
-    direct = dcoperation is DCoperation
+    # the handlers are called directly where ``perform_operation`` is this module's own; one that a caller has replaced, in
+    # a class of their own or in this one, is called
+    direct = getattr(dcoperation, "perform_operation", None) is _PLAIN_PERFORM
     skip = False
     for i, s in enumerate(steps):
         if skip:                    # ran together with the op before it

@@ -60,6 +60,35 @@ def test_plan_file_schema(tmp_path):
         dstb.init_DCBlocks({"DCBlocks": [[["ln_attn"], "None"]]})
 
 
+def _run_placeholders(plan, dcoperation):
+    """Runs a plan of weight-gradient placeholders (they need no GPU); the order in which parked work ran."""
+    ran = []
+    act = {"_parked": {n: (lambda cfg, args, st, n=n: ran.append(n), (None, (), None)) for n in plan.movable}}
+    dstb.exec(None, dcoperation, None, {}, None, None, plan.dcblocks, None, None, act, None, movable=plan.movable)
+    return ran
+
+
+def test_a_replaced_perform_operation_is_called(monkeypatch):
+    """The scheduler goes through ``perform_operation``: a wrapper put on the class, or one of a class of the caller's."""
+    plan = dstb.init_DCBlocks({"DCBlocks": [["None", ["gemm_wgrad_mlp_c_n", "gemm_wgrad_attn_l_n"], "None"]]})
+    plain, seen = dstb.DCoperation.perform_operation, []
+
+    def wrapper(dcfunc, operation, *args, **kwargs):
+        seen.append(kwargs["name"])
+        return plain(dcfunc, operation, *args, **kwargs)
+
+    class Own(dstb.DCoperation):
+        perform_operation = staticmethod(wrapper)
+
+    _run_placeholders(plan, dstb.DCoperation)
+    assert seen == []
+    _run_placeholders(plan, Own)
+    assert seen == ["gemm_wgrad_mlp_c_n", "gemm_wgrad_attn_l_n"]
+    monkeypatch.setattr(dstb.DCoperation, "perform_operation", staticmethod(wrapper))
+    _run_placeholders(plan, dstb.DCoperation)
+    assert seen == 2 * ["gemm_wgrad_mlp_c_n", "gemm_wgrad_attn_l_n"]
+
+
 def test_layer_config_derived_sizes():
     from dhellam_amd.core.layer import llama70b_tp8_shard, small_fp32_layer
     c = llama70b_tp8_shard()
