@@ -735,6 +735,7 @@ def _h_bda_attn_ln_mlp(c):
 
 # (name, name of the op that follows it in the same column) -> handler that runs both
 _FUSED = {("bda_attn", "ln_mlp"): _h_bda_attn_ln_mlp}
+_FUSED_FIRST = {first for first, _ in _FUSED}
 
 
 # op id -> handler (the reference: one ``if operation == N`` after another, dstb.py:431-657)
@@ -776,6 +777,7 @@ class DCoperation:
 
 class DCOP:
     """A node of the op graph (dstb.py:662-690)."""
+    strand = 1                      # 1 forward, 2 backward
 
     def __init__(self, pre_op, stream, num, is_first_mb, is_comm=0, name=None):
         self.pre = pre_op
@@ -1006,7 +1008,7 @@ def init_DCBlocks(config=None, stream1=None, stream2=None, context_parallel_size
     movable = set()
 
     def build(section):
-        blocks = _Blocks()
+        blocks = []
         raw = data.get(section) or DEFAULT_PLAN[section]
         for blk in (_insert_rope(raw) if cp <= 1 else _ring_names_for(raw, cp)):
             if len(blk) != 3:
@@ -1030,73 +1032,41 @@ def init_DCBlocks(config=None, stream1=None, stream2=None, context_parallel_size
     return Plan(build("DCBlocks"), build("fwd_only"), build("bwd_only"), movable, ops)
 
 
-class _Step:
-    """One op of a column with everything that does not change from call to call looked up."""
-    __slots__ = ("op", "num", "name", "strand", "is_comm", "next", "handler", "free", "fused")
-
-    def __init__(self, op, after):
-        self.op, self.num, self.name, self.is_comm = op, op.get_op_num(), op.name, op.is_comm
-        self.strand = getattr(op, "strand", 1)
-        self.next = op.get_next_op()
-        num = self.num.value if isinstance(self.num, FuncChoice) else int(self.num)
-        self.handler, self.free = _HANDLERS.get(num), _FREE_AFTER.get(num, ())
-        # handler that runs this op and the one after it in the column together
-        self.fused = _FUSED.get((op.name, after.name)) if after is not None and after in self.next else None
-
-
-class _Blocks(list):
-    """The DCBlocks of one plan section and, once they have run, their columns in running order."""
-    steps = None
-
-
-def _block_steps(blk: DCBlock):
-    """[(forward side?, [_Step ...]) ...] of a block in running order: the communication ops one by one, then the two
-    compute columns; the strand whose communication was just posted goes second (dstb.py:1174-1264)."""
-    cols, fwd_comm_first = [], False
-    for op in blk.stream3_op or ():
-        fwd_comm_first |= op.is_comm == 1
-        cols.append((op.is_comm == 1, [op]))
-    for strand in ((2, 1) if fwd_comm_first else (1, 2)):
-        col = blk.stream1_op if strand == 1 else blk.stream2_op
-        if col is not None:
-            cols.append((strand == 1, col))
-    return [(fwd, [_Step(op, col[i + 1] if i + 1 < len(col) else None) for i, op in enumerate(col)]) for fwd, col in cols]
-
-
 _PLAIN_PERFORM = DCoperation.perform_operation
 
 
-def _run_column(steps, dcoperation, config, weight, act, first_input, stream1, stream2, result, movable, fuse):
-    # the handlers are called directly where ``perform_operation`` is this module's own; one that a caller has replaced, in
-    # a class of their own or in this one, is called
-    direct = getattr(dcoperation, "perform_operation", None) is _PLAIN_PERFORM
+def _run_column(col, dcoperation, direct, config, weight, act, first_input, stream1, stream2, result, movable, fuse):
+    """Runs the ops of one column.  ``direct``: their handlers are called as ``perform_operation`` does it."""
     skip = False
-    for i, s in enumerate(steps):
+    for i, op in enumerate(col):
         if skip:                    # ran together with the op before it
             skip = False
             continue
-        op = s.op
         inp = first_input if op.output is None else op.output
         op.output = None
-        st = stream1 if s.strand == 1 else stream2
+        st = stream1 if op.strand == 1 else stream2
         handle = None
-        if fuse and s.fused is not None:
-            nxt = steps[i + 1]
-            output = dcoperation.perform_fused(DCFunc, (s.name, nxt.name), config, weight, act, output=inp, stream=st,
+        num, name = op.op_num, op.name
+        handler = _HANDLERS.get(num) if direct else None
+        if fuse and name in _FUSED_FIRST and i + 1 < len(col) and (name, col[i + 1].name) in _FUSED and col[i + 1] in op.next_op:
+            nxt = col[i + 1]
+            output = dcoperation.perform_fused(DCFunc, (name, nxt.name), config, weight, act, output=inp, stream=st,
                                                movable=movable)
-            s, skip = nxt, True     # successors and result bookkeeping are those of the second op
-            s.op.output = None
-        elif direct and s.handler is not None:
-            output = s.handler(_Ctx(DCFunc, s.num, config, weight, act, inp, st, s.name, movable))
-            for key in s.free:
-                act.pop(key, None)
+            op, skip = nxt, True    # successors and result bookkeeping are those of the second op
+            op.output = None
+        elif handler is not None:
+            output = handler(_Ctx(DCFunc, num, config, weight, act, inp, st, name, movable))
+            if num in _FREE_AFTER:
+                for key in _FREE_AFTER[num]:
+                    act.pop(key, None)
         else:
-            output = dcoperation.perform_operation(DCFunc, s.num, config, weight, act, output=inp, stream=st, name=s.name,
+            output = dcoperation.perform_operation(DCFunc, num, config, weight, act, output=inp, stream=st, name=name,
                                                    movable=movable)
-        if s.is_comm:
+        if op.is_comm:
             output, handle = output
-        if s.next:
-            for nop in s.next:
+        successors = op.next_op
+        if successors:
+            for nop in successors:
                 nop.output = output
                 nop.handle = handle
         elif output is not None:
@@ -1121,14 +1091,15 @@ def exec(config, dcoperation, fwd_weight, bwd_weight, input, grad_output, dcbloc
             stream2.wait_event(ev)
     ran_fwd = False
     fuse = getattr(config, "fuse_adjacent", True) and hasattr(dcoperation, "perform_fused")
-    steps = dcblocks.steps if isinstance(dcblocks, _Blocks) else None
-    if steps is None:
-        steps = [_block_steps(blk) for blk in dcblocks]
-        if isinstance(dcblocks, _Blocks):
-            dcblocks.steps = steps
+    # the handlers are called directly where ``perform_operation`` is this module's own (1.1 us less an op); one that a caller
+    # has replaced, in a class of their own or in this one, is called
+    direct = getattr(dcoperation, "perform_operation", None) is _PLAIN_PERFORM
+    fwd_args = (dcoperation, direct, config, fwd_weight, new_activation_dict, input, stream1, stream2, fwd_res, movable, fuse)
+    bwd_args = (dcoperation, direct, config, bwd_weight, activation_dict, grad_output, stream1, stream2, bwd_res, movable,
+                fuse)
     lockstep = (getattr(config, "lockstep_blocks", False) and stream1 is not None and stream2 is not None
                 and stream1 != stream2)
-    for columns in steps:
+    for blk in dcblocks:
         if lockstep:
             # both strands enter a block together (device-side events, no host wait): keeps the block's pairing,
             # which matters when the stand-in collectives have a duration to hide; without it the forward strand
@@ -1138,14 +1109,23 @@ def exec(config, dcoperation, fwd_weight, bwd_weight, input, grad_output, dcbloc
             e2.record(stream2)
             stream1.wait_event(e2)
             stream2.wait_event(e1)
-        for fwd, col in columns:
-            if fwd:
-                _run_column(col, dcoperation, config, fwd_weight, new_activation_dict, input, stream1, stream2, fwd_res,
-                            movable, fuse)
-                ran_fwd = True
+        # the communication ops one by one, then the two compute columns; the strand whose communication was just posted
+        # goes second (dstb.py:1174-1264)
+        fwd_comm_first = False
+        for op in blk.stream3_op or ():
+            if op.is_comm == 1:
+                fwd_comm_first = ran_fwd = True
+                _run_column((op,), *fwd_args)
             else:
-                _run_column(col, dcoperation, config, bwd_weight, activation_dict, grad_output, stream1, stream2, bwd_res,
-                            movable, fuse)
+                _run_column((op,), *bwd_args)
+        if blk.stream1_op is not None:
+            ran_fwd = True
+            if not fwd_comm_first:
+                _run_column(blk.stream1_op, *fwd_args)
+        if blk.stream2_op is not None:
+            _run_column(blk.stream2_op, *bwd_args)
+        if fwd_comm_first and blk.stream1_op is not None:
+            _run_column(blk.stream1_op, *fwd_args)
     # deferred wgrads that no placeholder op picked up run at the end (dstb.py:1268-1279)
     if activation_dict is not None and activation_dict.get("_parked"):
         for key in list(activation_dict["_parked"]):

@@ -89,6 +89,19 @@ def test_a_replaced_perform_operation_is_called(monkeypatch):
     assert seen == 2 * ["gemm_wgrad_mlp_c_n", "gemm_wgrad_attn_l_n"]
 
 
+def test_a_plan_edited_after_a_run_runs_as_edited():
+    plan = dstb.init_DCBlocks({"DCBlocks": [["None", ["gemm_wgrad_mlp_c_n", "gemm_wgrad_attn_l_n"], "None"],
+                                            ["None", ["gemm_wgrad_mlp_l_n"], "None"]]})
+    c, l, a = "gemm_wgrad_mlp_c_n", "gemm_wgrad_mlp_l_n", "gemm_wgrad_attn_l_n"
+    assert _run_placeholders(plan, dstb.DCoperation) == [c, a, l]
+    plan.dcblocks[0].stream2_op.reverse()                   # inside a column
+    assert _run_placeholders(plan, dstb.DCoperation) == [a, c, l]
+    plan.dcblocks.reverse()                                 # the blocks themselves
+    assert _run_placeholders(plan, dstb.DCoperation) == [l, a, c]
+    plan.dcblocks[1].stream2_op = [plan.ops[c]]             # another column; what nothing runs any more comes last
+    assert _run_placeholders(plan, dstb.DCoperation) == [l, c, a]
+
+
 def test_layer_config_derived_sizes():
     from dhellam_amd.core.layer import llama70b_tp8_shard, small_fp32_layer
     c = llama70b_tp8_shard()
