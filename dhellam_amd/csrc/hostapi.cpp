@@ -454,7 +454,9 @@ void attn_bwd(const Tensor &dout, const Tensor &q, const Tensor &k, const Tensor
               const Tensor &dq, const Tensor &dk, const Tensor &dv, const OptTensor &delta, const Tensor &cu_q,
               const Tensor &cu_k, int max_q, int max_k, double scale, bool causal, bool accumulate_dq,
               const OptStream &stream) {
-  need_gpu({&dout, &q, &k, &v, &out, &lse});
+  need_gpu({&dout, &q, &k, &v, &out, &lse, &dq, &dk, &dv, &cu_q, &cu_k});
+  TORCH_CHECK(!delta.has_value() || delta->is_cuda(), "dhellam operators need tensors on the GPU");
+  TORCH_CHECK(cu_q.scalar_type() == at::kInt && cu_k.scalar_type() == at::kInt, "cu_seqlens must be int32");
   const int b = (int)cu_q.numel() - 1, hq = (int)q.size(1), hk = (int)k.size(1), d = (int)q.size(2), type = dt(q);
   On on(stream);
   const size_t bytes = dh_attn_bwd_workspace_bytes(q.size(0), k.size(0), b, max_q, hq, hk, d, type);
@@ -526,7 +528,9 @@ Tensor attn_bwd_packed(const Tensor &dout, const Tensor &q, const Tensor &k, con
 struct RingStep {
   bool fits = false, half_q = false, half_k = false;
   int64_t c = 0, hq = 0, hk = 0, d = 0;
-  RingStep(const Tensor &q, const Tensor &kv, int step, int rank) {
+  RingStep(const Tensor &q, const Tensor &kv, const Tensor &cu_q, const Tensor &cu_k, int step, int rank) {
+    for (const Tensor *cu : {&cu_q, &cu_k})
+      if (!(cu->is_cuda() && cu->scalar_type() == at::kInt && cu->numel() == 2 && cu->is_contiguous())) return;
     if (!(q.is_cuda() && kv.is_cuda() && q.dim() == 5 && kv.dim() == 6 && q.is_contiguous() && kv.is_contiguous() &&
           q.scalar_type() == kv.scalar_type() && (q.scalar_type() == at::kBFloat16 || q.scalar_type() == at::kHalf)))
       return;
@@ -549,10 +553,8 @@ char *at_row(const Tensor &t, int64_t row, int64_t heads, int64_t d) { return (c
 // -> (out [rows, hq, d], lse [1, hq, rows]), or None where the operands are not of that form
 py::object ring_fwd(const Tensor &q, const Tensor &kv, const Tensor &cu_q, const Tensor &cu_k, int64_t max_q, int64_t max_k,
                     int step, int rank, double scale, const OptStream &stream) {
-  const RingStep r(q, kv, step, rank);
-  if (!r.fits || max_q != 2 * r.c || max_k != 2 * r.c || cu_q.scalar_type() != at::kInt || cu_k.scalar_type() != at::kInt ||
-      cu_q.numel() != 2 || cu_k.numel() != 2)
-    return py::none();
+  const RingStep r(q, kv, cu_q, cu_k, step, rank);
+  if (!r.fits || max_q != 2 * r.c || max_k != 2 * r.c) return py::none();
   const int type = dt(q);
   const int64_t nq = r.rows_q(), nk = r.rows_k(), qs = r.hq * r.d, ks = r.hk * r.d;
   On on(stream);
@@ -569,12 +571,12 @@ py::object ring_fwd(const Tensor &q, const Tensor &kv, const Tensor &cu_q, const
 py::object ring_bwd(const Tensor &dout, const Tensor &out, const Tensor &q, const OptTensor &dq_in, const Tensor &kv, const Tensor &lse,
                     const Tensor &cu_q, const Tensor &cu_k, int64_t max_q, int64_t max_k, int step, int rank, bool first, double scale,
                     const OptStream &stream) {
-  const RingStep r(q, kv, step, rank);
-  if (!r.fits || max_q != 2 * r.c || max_k != 2 * r.c || cu_q.scalar_type() != at::kInt || cu_k.scalar_type() != at::kInt ||
-      cu_q.numel() != 2 || cu_k.numel() != 2 || !dout.is_contiguous() || !out.is_contiguous() || dout.numel() != q.numel() ||
-      out.numel() != q.numel() || dout.scalar_type() != q.scalar_type() || out.scalar_type() != q.scalar_type() ||
-      !lse.is_contiguous() || lse.scalar_type() != at::kFloat || lse.numel() != 2 * r.c * r.hq ||
-      (dq_in.has_value() && !(dq_in->is_contiguous() && dq_in->numel() == q.numel() && dq_in->scalar_type() == q.scalar_type())))
+  const RingStep r(q, kv, cu_q, cu_k, step, rank);
+  const auto like_q = [&](const Tensor &t) {
+    return t.is_cuda() && t.is_contiguous() && t.numel() == q.numel() && t.scalar_type() == q.scalar_type();
+  };
+  if (!r.fits || max_q != 2 * r.c || max_k != 2 * r.c || !like_q(dout) || !like_q(out) || !lse.is_cuda() || !lse.is_contiguous() ||
+      lse.scalar_type() != at::kFloat || lse.numel() != 2 * r.c * r.hq || (dq_in.has_value() && !like_q(*dq_in)))
     return py::none();
   const int type = dt(q);
   const int64_t nq = r.rows_q(), nk = r.rows_k(), q_at = r.half_q ? r.c : 0, qs = r.hq * r.d, ks = r.hk * r.d;

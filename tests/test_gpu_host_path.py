@@ -45,3 +45,35 @@ def test_argument_checks_keep_their_exceptions():
         rope_fwd(x.view(4, 1, 6), x.view(4, 1, 6), torch.zeros(3, dtype=torch.int32, device="cuda"))
     with pytest.raises(RuntimeError, match="dtype"):
         swiglu(x.double())
+
+
+@pytest.mark.parametrize("half", [False, True])
+def test_attention_operands_off_the_gpu_are_refused(half):
+    """Whole and half ring steps and the plain backward: an operand in host memory is an error, never an address that a
+    kernel reads."""
+    from dhellam_amd import _Clib
+    from dhellam_amd.operators.ring_attn import RingGroup, fa_cp_block_bwd, fa_cp_block_fwd
+    c, hq, hk, d = 32, 2, 1, 64
+    g = torch.Generator(device="cuda").manual_seed(3)
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda").to(torch.bfloat16)
+    q, kv, cu = rand(1, 2, c, hq, d), [rand(2, 1, 2, c, hk, d) for _ in range(2)], torch.tensor([0, 2 * c], dtype=torch.int32, device="cuda")
+    group, step, n = RingGroup(0, 2), int(half), 2 * c
+    carry = fa_cp_block_fwd(q, cu, cu, n, n, kv, None, None, None, None, None, 0, True, group, [0, 1], None)[0]
+    out, _, _, lse, rng = fa_cp_block_fwd(q, cu, cu, n, n, kv, *carry[2:7], 1, True, group, [0, 1], None)
+    for at in range(4):
+        a = [q, cu, cu, kv]
+        a[at] = [t.cpu() for t in kv] if at == 3 else a[at].cpu()
+        with pytest.raises((RuntimeError, AssertionError)):
+            fa_cp_block_fwd(a[0], a[1], a[2], n, n, a[3], *([None] * 5 if step == 0 else carry[2:7]), step, True, group, [0, 1], None)
+    for at in range(8):
+        a = [rand(1, 2, c, hq, d), out, q, rand(1, 2, c, hq, d), lse, cu, cu, kv]
+        a[at] = [t.cpu() for t in kv] if at == 7 else a[at].cpu()
+        with pytest.raises((RuntimeError, AssertionError)):
+            fa_cp_block_bwd(a[0], a[1], a[2], a[3], None, None, a[4], rng, a[5], a[6], n, n, a[7], 1 - step, True, group, [0, 1], None)
+    x, s = [q.view(n, hq, d), kv[0][0].reshape(n, hk, d)], torch.empty(1, hq, n, device="cuda")
+    args = [x[0], x[0], x[1], x[1], x[0], s, x[0].clone(), x[1].clone(), x[1].clone(), s.clone(), cu, cu]
+    for at in range(len(args)):
+        a = list(args)
+        a[at] = a[at].cpu()
+        with pytest.raises(RuntimeError):
+            _Clib._attn_bwd_raw(*a, n, n, 0.1, True)
