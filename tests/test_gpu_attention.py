@@ -378,3 +378,22 @@ def test_attention_f32_matrix_core_kernels(lens_q, lens_k, hq, hk, d, causal):
 def test_attention_head_dim_64(dtype, lens_q, lens_k, hq, hk, causal):
     """Head dim 64 kernels: both workgroup shapes, tile edges of both sequences, ragged batches, GQA groups."""
     _run_fwd_bwd(dtype, lens_q, lens_k, hq, hk, 64, causal)
+
+
+@pytest.mark.parametrize("d", [64, 96])
+def test_attention_backward_many_short_sequences_and_a_long_bound(d):
+    """64 short sequences x 64 heads whose bound max_seqlen says 131072: the planes of the row statistics pass 2 GiB (they
+    are laid out by the bound), the work does not.  Same gradients as with the bound at the longest length."""
+    from dhellam_amd import _Clib
+    dtype, lens, hq = torch.bfloat16, [1 + i % 7 for i in range(64)], 64
+    cu = _cu(lens).cuda()
+    t, scale = sum(lens), 1.0 / math.sqrt(d)
+    q, k, v, do = (randn((t, hq, d), dtype, 40 + i).cuda() for i in range(4))
+    got = []
+    for m in (131072, max(lens)):
+        res = _Clib.pymha_varlen_fwd(q, k, v, cu, cu, m, m, 0.0, scale, True, False, 0, False)
+        got.append([res[0]] + _Clib.pymha_varlen_bwd(do, q, k, v, res[0], res[5], cu, cu, m, m, 0.0, scale, True, None, True, 0,
+                                                     False, torch.cuda.current_stream().cuda_stream)[:3])
+    # the bound picks the kernels' tile shapes, so sums may run in another order
+    for a, b, what in zip(*got, ("out", "dq", "dk", "dv")):
+        assert_close(a, b.double().cpu(), dtype, what)
