@@ -591,7 +591,7 @@ __device__ __forceinline__ void gg_copy_lds(uint32_t lane_off, const gg_i32x4 &r
                : "memory", "m0");
 }
 
-constexpr int64_t GG_MAX_LD = 1 << 22;       // row lengths (elements): 128 rows stay inside 31-bit byte offsets
+constexpr int64_t GG_MAX_LD = (1 << 22) - 8;       // row lengths (elements) of the tiled kernels: 256 rows stay inside 31-bit byte offsets
 
 // k pieces per tile: what fills the chip's places, each at least 8 slices long (a piece costs about as much traffic for
 // its fp32 tile, written and read, as four slices of operands).
@@ -943,6 +943,63 @@ __global__ void __launch_bounds__(256) gg_t_reduce_kernel(const GGParams p) {
     }
 }
 
+// Rows longer than GG_MAX_LD elements, whose tiles do not fit the 31-bit byte offsets of the kernels above: a wavefront per
+// row and 8 columns of c, its lanes share the reduction, 64-bit addresses.  Bound by the rate of its loads; such operands
+// are only ever a few rows.
+template <typename T, int FORM>
+__global__ void __launch_bounds__(256) grouped_gemm_long_rows_kernel(const GGParams p) {
+  using V = Vec<T>;
+  const int lane = threadIdx.x & 63, base = gg_off(p, 0);
+  const T *a = reinterpret_cast<const T *>(p.a), *b = reinterpret_cast<const T *>(p.b);
+  T *c = reinterpret_cast<T *>(p.c);
+  const int64_t cols = p.n_dim / 8, rows = FORM == 2 ? p.m_dim * p.groups : p.max_rows;
+  for (int64_t it = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); it < rows * cols; it += (int64_t)gridDim.x * 4) {
+    const int64_t row = it / cols, n = 8 * (it - row * cols);
+    int64_t k0 = 0, k1 = 0;                                       // the reduction: columns of a, or rows (TN)
+    const T *ar = a, *bg = b;
+    int64_t astep = 1;
+    T *dst;
+    if constexpr (FORM == 2) {
+      const int g = (int)(row / p.m_dim);
+      const int64_t m = row - (int64_t)g * p.m_dim;
+      k0 = gg_clamp_row(gg_off(p, g) - base, p.max_rows);
+      k1 = gg_clamp_row(gg_off(p, g + 1) - base, p.max_rows);
+      ar = a + m;
+      astep = p.lda;
+      dst = c + (int64_t)g * p.c_group_stride + m * p.ldc + n;
+    } else {
+      ar = a + row * p.lda;
+      dst = c + row * p.ldc + n;
+      for (int g = 0; g < p.groups; ++g)                          // rows past the last group: zeros
+        if (row >= gg_clamp_row(gg_off(p, g) - base, p.max_rows) && row < gg_clamp_row(gg_off(p, g + 1) - base, p.max_rows)) {
+          bg = b + (int64_t)g * p.b_group_stride;
+          k1 = p.k_dim;
+        }
+    }
+    float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    for (int64_t k = k0 + lane; k < k1; k += 64) {
+      const float x = to_f(ar[k * astep]);
+      if constexpr (FORM == 0) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc[j] += x * to_f(bg[(n + j) * p.ldb + k]);
+      } else {
+        const V v = ldg(bg + k * p.ldb + n);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc[j] += x * to_f(v.v[j]);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      for (int o = 32; o > 0; o >>= 1) acc[j] += __shfl_xor(acc[j], o, 64);
+    if (lane == 0) {
+      V o;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) o.v[j] = static_cast<T>(FORM == 2 && p.accumulate ? acc[j] + to_f(dst[j]) : acc[j]);
+      stg(dst, o);
+    }
+  }
+}
+
 // Workspace of the split last round: one fp32 tile per workgroup of the grid.
 constexpr int GG_SK_MAX_GRID = 256;
 constexpr size_t GG_SK_WS_BYTES = (size_t)GG_SK_MAX_GRID * 256 * 256 * sizeof(float);
@@ -1035,6 +1092,13 @@ static int launch_gg_t(GGParams p, int64_t m_extent, void *workspace, size_t wor
 
 template <typename T, int FORM>
 static int dispatch_gg_t(const GGParams &p, int64_t m_extent, void *workspace, size_t workspace_bytes, hipStream_t st) {
+  // (the columns of an NT product are no row length of an operand: only their tiles are counted in 32 bits)
+  if (p.n_dim > (FORM == 0 ? (int64_t)1 << 30 : GG_MAX_LD) || (FORM == 2 ? p.m_dim : p.k_dim) > GG_MAX_LD) {
+    const int64_t items = (FORM == 2 ? p.m_dim * p.groups : (int64_t)p.max_rows) * (p.n_dim / 8);
+    const int64_t blocks = cdiv(items, 4) < 256 * 16 ? cdiv(items, 4) : 256 * 16;
+    hipLaunchKernelGGL((grouped_gemm_long_rows_kernel<T, FORM>), dim3((unsigned)blocks), dim3(256), 0, st, p);
+    return DH_OK;
+  }
   if constexpr (FORM == 2) {
     return launch_gg_t<T, FORM, 128, 128>(p, m_extent, workspace, workspace_bytes, st);
   } else {
@@ -1086,7 +1150,6 @@ extern "C" int dh_grouped_gemm_nt(const void *a, const void *b, void *c, const i
   int rc = gg_common_checks(a, b, c, offs, groups, dtype);
   if (rc) return rc;
   DH_CHECK(n % 8 == 0 && k % 8 == 0, "n=%lld and k=%lld must be multiples of 8", (long long)n, (long long)k);
-  DH_CHECK(n <= GG_MAX_LD && k <= GG_MAX_LD, "n=%lld and k=%lld must be at most %lld", (long long)n, (long long)k, (long long)GG_MAX_LD);
   GGParams p{};
   p.a = a; p.b = b; p.c = c; p.offs = offs; p.groups = groups;
   p.n_dim = n; p.k_dim = k; p.lda = k; p.ldb = k; p.ldc = n;
@@ -1113,7 +1176,6 @@ extern "C" int dh_grouped_gemm_nn(const void *a, const void *b, void *c, const i
   int rc = gg_common_checks(a, b, c, offs, groups, dtype);
   if (rc) return rc;
   DH_CHECK(n % 8 == 0 && k % 8 == 0, "n=%lld and k=%lld must be multiples of 8", (long long)n, (long long)k);
-  DH_CHECK(n <= GG_MAX_LD && k <= GG_MAX_LD, "n=%lld and k=%lld must be at most %lld", (long long)n, (long long)k, (long long)GG_MAX_LD);
   GGParams p{};
   p.a = a; p.b = b; p.c = c; p.offs = offs; p.groups = groups;
   p.n_dim = n; p.k_dim = k; p.lda = k; p.ldb = n; p.ldc = n;
@@ -1140,7 +1202,6 @@ extern "C" int dh_grouped_gemm_tn_ws(const void *a, const void *b, void *c, cons
   int rc = gg_common_checks(a, b, c, offs, groups, dtype);
   if (rc) return rc;
   DH_CHECK(n % 8 == 0 && m % 8 == 0, "m=%lld and n=%lld must be multiples of 8", (long long)m, (long long)n);
-  DH_CHECK(m <= GG_MAX_LD && n <= GG_MAX_LD, "m=%lld and n=%lld must be at most %lld", (long long)m, (long long)n, (long long)GG_MAX_LD);
   GGParams p{};
   p.a = a; p.b = b; p.c = c; p.offs = offs; p.groups = groups;
   p.m_dim = m; p.n_dim = n; p.lda = m; p.ldb = n; p.ldc = n;

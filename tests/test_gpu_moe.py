@@ -482,3 +482,34 @@ def test_sort_at_the_one_launch_limit(T, E, k):
     plan, _ = sort_assignments(torch.from_numpy(io).cuda(), E)
     for got, want in zip((plan.tokens_per_expert, plan.expert_offsets, plan.sorted_idx, plan.dest_row), OM.sort_assignments(io, E)):
         assert np.array_equal(got.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("form,n,k", [("nt", 16, (1 << 22) - 8), ("nt", 16, 1 << 22), ("nt", (1 << 22) + 8, 16),
+                                      ("nn", (1 << 22) + 8, 16), ("nn", 16, (1 << 22) + 8)])
+def test_grouped_gemm_rows_longer_than_the_tiled_kernels_take(form, n, k):
+    """Row lengths either side of the tiled kernels' limit (below 2^22 elements), few rows, an empty group, rows past the last."""
+    from dhellam_amd.operators import moe
+    rows, R = [3, 0, 2], 7
+    offs = torch.tensor([0, 3, 3, 5], dtype=torch.int32, device="cuda")
+    g = torch.Generator(device="cuda").manual_seed(8)
+    a = (torch.randn(R, k, generator=g, device="cuda") * 0.5).to(torch.bfloat16)
+    b = (torch.randn((3, n, k) if form == "nt" else (3, k, n), generator=g, device="cuda") * 0.5).to(torch.bfloat16)
+    c = (moe.grouped_gemm_nt if form == "nt" else moe.grouped_gemm_nn)(a, b, offs)
+    assert torch.count_nonzero(c[5:]) == 0
+    for lo, hi, e in ((0, 3, 0), (3, 5, 2)):
+        ref = a[lo:hi].double() @ (b[e].double().t() if form == "nt" else b[e].double())
+        assert_close(c[lo:hi], ref, torch.bfloat16, f"{form}, group {e}", local=False)
+
+
+@pytest.mark.parametrize("accumulate", [False, True])
+@pytest.mark.parametrize("m,n", [(16, (1 << 22) + 8), ((1 << 22) + 8, 16)])
+def test_grouped_gemm_tn_rows_longer_than_the_tiled_kernels_take(m, n, accumulate):
+    from dhellam_amd.operators import moe
+    offs = torch.tensor([0, 3, 3, 70], dtype=torch.int32, device="cuda")
+    g = torch.Generator(device="cuda").manual_seed(9)
+    a, b = ((torch.randn(70, w, generator=g, device="cuda") * 0.5).to(torch.bfloat16) for w in (m, n))
+    base = torch.full((3, m, n), 2.0, dtype=torch.bfloat16, device="cuda")
+    c = moe.grouped_gemm_tn(a, b, offs, base.clone() if accumulate else None, accumulate)
+    for e, (lo, hi) in enumerate(((0, 3), (3, 3), (3, 70))):
+        ref = a[lo:hi].double().t() @ b[lo:hi].double() + (2.0 if accumulate else 0.0)
+        assert_close(c[e], ref, torch.bfloat16, f"tn, group {e}", local=False)
