@@ -21,6 +21,7 @@
 // needs no fp32 dQ accumulator in memory and no atomics.
 #include <atomic>
 
+#include "attn_route.h"
 #include "mma.h"
 
 
@@ -1112,8 +1113,7 @@ static std::atomic<int> g_ds_when_full{0};   // 1: keep dS also where the recomp
 
 // Whether the recomputing dQ kernel would fill the chip (its 128-row form).
 static bool dq_big_grid(int batch, int max_sq, int hq, int causal) {
-  const int64_t t = cdiv(max_sq, 128);
-  return (causal ? (t + 1) / 2 : t) * hq * batch >= 256;
+  return attn_wgs(max_sq, 128, hq, batch, causal) >= ATTN_128ROW_MIN_WG;
 }
 
 // Head dim 128 with short sequences: the kernels of the other head dims start and end sooner than the hand-ordered ones
@@ -1121,28 +1121,39 @@ static bool dq_big_grid(int batch, int max_sq, int hq, int causal) {
 // not kept.
 static bool bwd_short(int max_sq, int max_sk) { return max_sq < 512 && max_sk < 512; }
 
+// What one 16-bit call runs.
+struct AttnBwdRoute {
+  bool keep_ds;      // dK/dV keeps dS and dQ is one product over it; else dQ recomputes, first, and forms delta
+  bool hand_dkv, hand_dq;      // head dim 128's hand-ordered kernels
+  bool big_dq;       // 128-row query tiles in dQ
+};
+static AttnBwdRoute attn_bwd_route(int batch, int max_sq, int max_sk, int64_t total_q, int hq, int d, int causal, bool room_for_ds) {
+  const bool short_rows = d == 128 && bwd_short(max_sq, max_sk), big = dq_big_grid(batch, max_sq, hq, causal);
+  AttnBwdRoute r;
+  r.keep_ds = room_for_ds && max_sk > 0 && !short_rows;
+  r.hand_dkv = d == 128 && !short_rows;
+  r.hand_dq = r.hand_dkv && (!causal || !big || attn_causal_fills(max_sq, hq, batch, total_q));
+  r.big_dq = r.hand_dq ? big : d <= 128 && attn_wgs(max_sq, 128, hq, batch, 0) >= 2 * 256;
+  return r;
+}
+
 // The kernels behind delta of one call.
 template <typename T, int D>
-static int bwd_passes(const AttnBwdParams &p, int batch, int max_sq, int max_sk, hipStream_t st) {
-  const bool small_q = cdiv(max_sq, 128) * p.hq * batch < 2 * 256;
+static int bwd_passes(const AttnBwdParams &p, const AttnBwdRoute &r, int batch, int max_sq, int max_sk, hipStream_t st) {
   int rc = DH_OK;
   // recomputing dQ kernels form delta and run first
-  if (max_sq > 0) {
+  if (max_sq > 0 && !r.keep_ds) {
     if constexpr (D == 128) {
-      // (packed batches: most workgroups of the longest sequence's grid have nothing to do, and the smaller workgroups
-      // balance the rest: documents of 4 to 1298 tokens, 16 heads 47 -> 38 us)
-      if (bwd_short(max_sq, max_sk) || (!p.ds && p.causal && batch > 2))
-        rc = small_q ? launch_dq_tile<T, D, 2, 4, 2>(p, batch, st) : launch_dq_tile<T, D, 4, 2, 2>(p, batch, st);
-      else if (!p.ds)
-        rc = dq_big_grid(batch, max_sq, p.hq, p.causal) ? launch_dq_d128<T, 4, 2, 32>(p, batch, st) : launch_dq_d128<T, 2, 4, 32>(p, batch, st);
+      if (r.hand_dq) rc = r.big_dq ? launch_dq_d128<T, 4, 2, 32>(p, batch, st) : launch_dq_d128<T, 2, 4, 32>(p, batch, st);
+      else rc = r.big_dq ? launch_dq_tile<T, D, 4, 2, 2>(p, batch, st) : launch_dq_tile<T, D, 2, 4, 2>(p, batch, st);
     } else if constexpr (D < 128) {
-      rc = small_q ? launch_dq_tile<T, D, 2, 4, 2>(p, batch, st) : launch_dq_tile<T, D, 4, 2, D == 64 ? 4 : 2>(p, batch, st);
+      rc = r.big_dq ? launch_dq_tile<T, D, 4, 2, D == 64 ? 4 : 2>(p, batch, st) : launch_dq_tile<T, D, 2, 4, 2>(p, batch, st);
     } else {
       rc = launch_dq_tile<T, D, 2, 2, 1>(p, batch, st);
     }
   }
   if (rc == DH_OK && max_sk > 0) {
-    if constexpr (D == 128) rc = bwd_short(max_sq, max_sk) ? launch_dkv_tile<T, D, 2, 2, 1>(p, batch, max_sk, st) : launch_dkv_d128<T>(p, batch, max_sk, st);
+    if constexpr (D == 128) rc = r.hand_dkv ? launch_dkv_d128<T>(p, batch, max_sk, st) : launch_dkv_tile<T, D, 2, 2, 1>(p, batch, max_sk, st);
     else if constexpr (D < 128) rc = launch_dkv_tile<T, D, 2, 4, 2>(p, batch, max_sk, st);
     else rc = launch_dkv_tile<T, D, 2, 2, 1>(p, batch, max_sk, st);
   }
@@ -1153,7 +1164,7 @@ static int bwd_passes(const AttnBwdParams &p, int batch, int max_sq, int max_sk,
                        (T *)p.dv, p.total_k, p.hk, D, p.hsplit, p.dk_stride, p.dv_stride);
   }
   if constexpr (D == 128) {
-    if (rc == DH_OK && max_sq > 0 && p.ds) rc = launch_dq2_d128<T>(p, batch, st);
+    if (rc == DH_OK && max_sq > 0 && r.keep_ds) rc = launch_dq2_d128<T>(p, batch, st);
   }
   return rc;
 }
@@ -1206,6 +1217,16 @@ extern "C" size_t dh_attn_bwd_workspace_bytes(int64_t total_q, int64_t total_k, 
          align256(ds_bytes(batch, max_seqlen_q, total_k, hq, d, dtype, 1));
 }
 
+extern "C" int dh_attn_bwd_path(int batch, int max_seqlen_q, int max_seqlen_k, int64_t total_q, int64_t total_k, int hq, int hk, int d,
+                                int causal, size_t workspace_bytes) {
+  using namespace dh;
+  const size_t base = bwd_base_bytes(total_k, batch, max_seqlen_q, hq, hk, d, DH_BF16);
+  const size_t dsb = ds_bytes(batch, max_seqlen_q, total_k, hq, d, DH_BF16, causal);
+  const AttnBwdRoute r = attn_bwd_route(batch, max_seqlen_q, max_seqlen_k, total_q, hq, d, causal,
+                                        dsb > 0 && base + align256(dsb) <= workspace_bytes);
+  return (r.hand_dkv ? 1 : 0) | (r.keep_ds ? 2 : (r.hand_dq ? 4 : 0) | (r.big_dq ? 8 : 0));
+}
+
 static int attn_bwd_entry(const void *dout, const void *q, const void *k, const void *v, const void *out,
                           const float *lse, void *dq, void *dk, void *dv, float *delta_out, void *workspace,
                           size_t workspace_bytes, const int32_t *cu_seqlens_q, const int32_t *cu_seqlens_k, int batch,
@@ -1249,9 +1270,9 @@ static int attn_bwd_entry(const void *dout, const void *q, const void *k, const 
   // process-wide limit); they take the tail of the workspace
   size_t dsb = ds_bytes(batch, max_seqlen_q, total_k, hq, d, dtype, causal);
   if (dsb > 0 && base_bytes + align256(dsb) > workspace_bytes) dsb = 0;
-  const bool keep_ds = dsb > 0 && max_seqlen_k > 0 && !bwd_short(max_seqlen_q, max_seqlen_k);
+  const AttnBwdRoute route = attn_bwd_route(batch, max_seqlen_q, max_seqlen_k, total_q, hq, d, causal, dsb > 0);
   uint8_t *ds_ws = (uint8_t *)(((uintptr_t)workspace + 255) & ~(uintptr_t)255) + (base_bytes - 256);
-  const bool delta_in_dq = dtype != DH_F32 && !keep_ds;
+  const bool delta_in_dq = dtype != DH_F32 && !route.keep_ds;
   if (max_seqlen_q > 0 && !delta_in_dq) {
     DH_DISPATCH_DTYPE(dtype, {
       launch_delta<T>(dout, out, delta, lse, ld2, (int64_t)(plane2 / sizeof(float)), ld2_pitch, cu_seqlens_q, q_shift, lse_pitch,
@@ -1286,7 +1307,7 @@ static int attn_bwd_entry(const void *dout, const void *q, const void *k, const 
   p.causal = causal;
   p.q_shift = q_shift; p.k_shift = k_shift; p.lse_pitch = lse_pitch;
   p.dq_accumulate = dq_accumulate ? 1 : 0;
-  p.ds = keep_ds ? (void *)ds_ws : nullptr;
+  p.ds = route.keep_ds ? (void *)ds_ws : nullptr;
   p.ds_nqt = 2 * (int)cdiv(max_seqlen_q, 64);
   p.ds_nkb = 2 * (int)cdiv(max_seqlen_k < total_k ? max_seqlen_k : total_k, 64) + 1;
   p.hsplit = pick_hsplit(d == 128 && causal ? (max_seqlen_k + 1) / 2 : max_seqlen_k, batch, hq, hk, DKV_ROWS);
@@ -1307,7 +1328,7 @@ static int attn_bwd_entry(const void *dout, const void *q, const void *k, const 
                      : d == 128 ? bwd_passes<TT, 128>                                           \
                      : d == 192 ? bwd_passes<TT, 192>                                           \
                                 : bwd_passes<TT, 256>;                                          \
-    rc = run(p, batch, max_seqlen_q, max_seqlen_k, st);                                         \
+    rc = run(p, route, batch, max_seqlen_q, max_seqlen_k, st);                                         \
   } while (0)
   if (dtype == DH_BF16) DH_BWD_D(bf16_t); else DH_BWD_D(f16_t);
 #undef DH_BWD_D

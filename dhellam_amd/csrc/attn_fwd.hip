@@ -5,6 +5,7 @@
 // of ONE query row: the online-softmax row reductions are in-lane plus a single exchange with lane^32.  P^T never leaves
 // registers: its accumulator layout is fed back as the B operand of O^T += V^T P^T, with the matching V^T fragments
 // produced by LDS transpose reads from the row-major V tile.  fp32 scores are scaled inside the exp2 argument (one FMA).
+#include "attn_route.h"
 #include "mma.h"
 #ifndef DH_FWD_RESCALE_LOG2
 #define DH_FWD_RESCALE_LOG2 8
@@ -422,40 +423,27 @@ static int launch_attn_fwd_d128(const AttnFwdParams &p, int batch, hipStream_t s
 
 namespace dh {
 
-// fewest workgroups of 128 query rows for which the 128-row kernel is taken
-#ifndef DH_FWD_128ROW_MIN_WG
-#define DH_FWD_128ROW_MIN_WG 256
-#endif
-
-// Workgroups of the head-dim-128 kernel with query tiles of `rows`.
-static int64_t attn_fwd_wgs(int max_sq, int rows, int hq, int batch, int causal) {
-  const int64_t t = cdiv(max_sq, rows);
-  return (causal ? (t + 1) / 2 : t) * hq * batch;
-}
-
-// Head dim 128: the hand-ordered kernel is the faster one where its workgroups, one per compute unit and causal ones all
-// of one length, come out in full rounds: 16 heads x 2048 causal (256 workgroups) 35 against 38 us, 32 heads x 4096 152
-// against 163 us.  Elsewhere its fixed costs and an almost empty last round lose to the smaller workgroups of the kernel
-// that the other head dims run: 8 heads x 300 17.2 against 9.9 us, 16 heads x 600 20 / 13, 12 heads x 3000 79 / 57 us,
-// packed documents of 4 to 1298 tokens (most workgroups of the longest one's grid have nothing to do) 35 / 28 us.
-static bool attn_fwd_fills(int max_sq, int hq, int batch, int causal) {
-  if (!causal) return attn_fwd_wgs(max_sq, 64, hq, batch, 0) >= 96;
-  if (batch > 2) return false;
-  int64_t wgs = attn_fwd_wgs(max_sq, 128, hq, batch, 1);
-  if (wgs < DH_FWD_128ROW_MIN_WG) wgs = attn_fwd_wgs(max_sq, 64, hq, batch, 1);
-  return wgs >= 240 && 20 * wgs >= 17 * 256 * cdiv(wgs, 256);
+struct AttnFwdRoute {
+  bool hand;      // head dim 128's hand-ordered kernel
+  bool big;       // 128-row query tiles
+};
+static AttnFwdRoute attn_fwd_route(int max_sq, int hq, int d, int batch, int64_t total_q, int causal) {
+  // not causal: from 96 workgroups of 64 rows on (4 heads x 4277 87 against 93 us, 4 x 6547 129 / 144, 32 x 7813 1028 / 1158;
+  // at 1000 rows and below level)
+  if (d == 128 && (causal ? attn_causal_fills(max_sq, hq, batch, total_q) : attn_wgs(max_sq, 64, hq, batch, 0) >= 96))
+    return {true, attn_wgs(max_sq, 128, hq, batch, causal) >= ATTN_128ROW_MIN_WG};
+  return {false, attn_wgs(max_sq, 128, hq, batch, 0) >= (d < 128 ? 2 * 256 : 256)};
 }
 
 // All other cases: 128-row query tiles when they give every compute unit its workgroups (two at 64 and 96,
 // one of the larger head dims), else 64-row tiles; more key splits where registers and LDS allow.
 template <typename T>
-static int launch_attn_fwd_other(const AttnFwdParams &p, int d, int batch, hipStream_t st) {
-  const int64_t wg128 = cdiv(p.max_sq, 128) * p.hq * batch;
-  if (d == 64) return wg128 >= 2 * 256 ? launch_attn_fwd_tile<T, 64, 4, 2, 64, 4>(p, batch, st) : launch_attn_fwd_tile<T, 64, 2, 4, 32, 4>(p, batch, st);
-  if (d == 96) return wg128 >= 2 * 256 ? launch_attn_fwd_tile<T, 96, 4, 2, 32, 4>(p, batch, st) : launch_attn_fwd_tile<T, 96, 2, 4, 32, 2>(p, batch, st);
-  if (d == 128) return wg128 >= 256 ? launch_attn_fwd_tile<T, 128, 4, 2, 64, 2>(p, batch, st) : launch_attn_fwd_tile<T, 128, 2, 4, 32, 2>(p, batch, st);
-  if (d == 192) return wg128 >= 256 ? launch_attn_fwd_tile<T, 192, 4, 2, 32, 2>(p, batch, st) : launch_attn_fwd_tile<T, 192, 2, 2, 32, 1>(p, batch, st);
-  return wg128 >= 256 ? launch_attn_fwd_tile<T, 256, 4, 2, 32, 2>(p, batch, st) : launch_attn_fwd_tile<T, 256, 2, 2, 32, 1>(p, batch, st);
+static int launch_attn_fwd_other(const AttnFwdParams &p, int d, bool big, int batch, hipStream_t st) {
+  if (d == 64) return big ? launch_attn_fwd_tile<T, 64, 4, 2, 64, 4>(p, batch, st) : launch_attn_fwd_tile<T, 64, 2, 4, 32, 4>(p, batch, st);
+  if (d == 96) return big ? launch_attn_fwd_tile<T, 96, 4, 2, 32, 4>(p, batch, st) : launch_attn_fwd_tile<T, 96, 2, 4, 32, 2>(p, batch, st);
+  if (d == 128) return big ? launch_attn_fwd_tile<T, 128, 4, 2, 64, 2>(p, batch, st) : launch_attn_fwd_tile<T, 128, 2, 4, 32, 2>(p, batch, st);
+  if (d == 192) return big ? launch_attn_fwd_tile<T, 192, 4, 2, 32, 2>(p, batch, st) : launch_attn_fwd_tile<T, 192, 2, 2, 32, 1>(p, batch, st);
+  return big ? launch_attn_fwd_tile<T, 256, 4, 2, 32, 2>(p, batch, st) : launch_attn_fwd_tile<T, 256, 2, 2, 32, 1>(p, batch, st);
 }
 
 int attn_fwd_f32(const void *q, const void *k, const void *v, void *out, float *lse, const int32_t *cu_q,
@@ -464,10 +452,15 @@ int attn_fwd_f32(const void *q, const void *k, const void *v, void *out, float *
 
 }  // namespace dh
 
-extern "C" int dh_attn_fwd_halves(const void *q, const void *k, const void *v, void *out, float *lse,
-                                  const int32_t *cu_seqlens_q, const int32_t *cu_seqlens_k, int q_shift, int k_shift,
-                                  int batch, int max_seqlen_q, int max_seqlen_k, int hq, int hk, int d,
-                                  int64_t q_stride, int64_t k_stride, int64_t v_stride, int64_t o_stride,
+extern "C" int dh_attn_fwd_path(int batch, int max_seqlen_q, int64_t total_q, int hq, int d, int causal) {
+  const dh::AttnFwdRoute r = dh::attn_fwd_route(max_seqlen_q, hq, d, batch, total_q, causal);
+  return (r.hand ? 1 : 0) | (r.big ? 2 : 0);
+}
+
+extern "C" int dh_attn_fwd_total(const void *q, const void *k, const void *v, void *out, float *lse,
+                                 const int32_t *cu_seqlens_q, const int32_t *cu_seqlens_k, int q_shift, int k_shift,
+                                 int batch, int max_seqlen_q, int max_seqlen_k, int64_t total_q, int hq, int hk, int d,
+                                 int64_t q_stride, int64_t k_stride, int64_t v_stride, int64_t o_stride,
                                   float softmax_scale, int causal, int dtype, void *stream) {
   using namespace dh;
   DH_CHECK((q_shift == 0 || q_shift == 1) && (k_shift == 0 || k_shift == 1), "sequences are taken whole or halved");
@@ -501,17 +494,27 @@ extern "C" int dh_attn_fwd_halves(const void *q, const void *k, const void *v, v
   p.scale_log2 = softmax_scale * 1.4426950408889634f;
   p.causal = causal;
   p.q_shift = q_shift; p.k_shift = k_shift;
+  const AttnFwdRoute r = attn_fwd_route(max_seqlen_q, hq, d, batch, total_q, causal);
   int rc;
-  if (d == 128 && attn_fwd_fills(max_seqlen_q, hq, batch, causal)) {
-    const bool big = attn_fwd_wgs(max_seqlen_q, 128, hq, batch, causal) >= DH_FWD_128ROW_MIN_WG;
-    if (dtype == DH_BF16) rc = big ? launch_attn_fwd_d128<bf16_t, 4, 2, 64, DH_FWD_LAG>(p, batch, st) : launch_attn_fwd_d128<bf16_t, 2, 4, 32, DH_FWD_LAG>(p, batch, st);
-    else rc = big ? launch_attn_fwd_d128<f16_t, 4, 2, 64, DH_FWD_LAG>(p, batch, st) : launch_attn_fwd_d128<f16_t, 2, 4, 32, DH_FWD_LAG>(p, batch, st);
+  if (r.hand) {
+    if (dtype == DH_BF16) rc = r.big ? launch_attn_fwd_d128<bf16_t, 4, 2, 64, DH_FWD_LAG>(p, batch, st) : launch_attn_fwd_d128<bf16_t, 2, 4, 32, DH_FWD_LAG>(p, batch, st);
+    else rc = r.big ? launch_attn_fwd_d128<f16_t, 4, 2, 64, DH_FWD_LAG>(p, batch, st) : launch_attn_fwd_d128<f16_t, 2, 4, 32, DH_FWD_LAG>(p, batch, st);
   } else {
-    rc = dtype == DH_BF16 ? launch_attn_fwd_other<bf16_t>(p, d, batch, st) : launch_attn_fwd_other<f16_t>(p, d, batch, st);
+    rc = dtype == DH_BF16 ? launch_attn_fwd_other<bf16_t>(p, d, r.big, batch, st) : launch_attn_fwd_other<f16_t>(p, d, r.big, batch, st);
   }
   if (rc != DH_OK) return rc;
   DH_LAUNCH_CHECK();
   return DH_OK;
+}
+
+extern "C" int dh_attn_fwd_halves(const void *q, const void *k, const void *v, void *out, float *lse,
+                                  const int32_t *cu_seqlens_q, const int32_t *cu_seqlens_k, int q_shift, int k_shift,
+                                  int batch, int max_seqlen_q, int max_seqlen_k, int hq, int hk, int d,
+                                  int64_t q_stride, int64_t k_stride, int64_t v_stride, int64_t o_stride,
+                                  float softmax_scale, int causal, int dtype, void *stream) {
+  return dh_attn_fwd_total(q, k, v, out, lse, cu_seqlens_q, cu_seqlens_k, q_shift, k_shift, batch, max_seqlen_q, max_seqlen_k,
+                           (int64_t)batch * max_seqlen_q, hq, hk, d, q_stride, k_stride, v_stride, o_stride, softmax_scale, causal,
+                           dtype, stream);
 }
 
 extern "C" int dh_attn_fwd(const void *q, const void *k, const void *v, void *out, float *lse,

@@ -442,9 +442,9 @@ std::tuple<Tensor, Tensor> attn_fwd(const Tensor &q, const Tensor &k, const Tens
   Tensor out = at::empty(q.sizes(), q.options());
   Tensor lse = at::empty({b, q.size(1), max_q}, q.options().dtype(at::kFloat));
   launch([&] {
-    return dh_attn_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr<float>(), cu_q.data_ptr<int>(),
-                       cu_k.data_ptr<int>(), b, max_q, max_k, (int)q.size(1), (int)k.size(1), (int)q.size(2), qs, ks, vs,
-                       token_stride(out), (float)scale, causal, type, on.get());
+    return dh_attn_fwd_total(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr<float>(), cu_q.data_ptr<int>(),
+                             cu_k.data_ptr<int>(), 0, 0, b, max_q, max_k, q.size(0), (int)q.size(1), (int)k.size(1),
+                             (int)q.size(2), qs, ks, vs, token_stride(out), (float)scale, causal, type, on.get());
   });
   return {out, lse};
 }

@@ -151,10 +151,11 @@ std::vector<at::Tensor> pymha_varlen_fwd(const at::Tensor &q_in, const at::Tenso
   hipStream_t stream = c10::hip::getCurrentHIPStream().stream();
   const float ms = timed(profiling, stream, [&] {
     confined(stream, q.device().index(), math_sm_count, [&](hipStream_t st) {
-      check(dh_attn_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out_padded.data_ptr(), lse.data_ptr<float>(),
-                        cu_seqlens_q.data_ptr<int>(), cu_seqlens_k.data_ptr<int>(), b, max_seqlen_q, max_seqlen_k,
-                        (int)q.size(1), (int)k.size(1), (int)q.size(2), token_stride(q), token_stride(k),
-                        token_stride(v), token_stride(out_padded), softmax_scale, is_causal ? 1 : 0, dt(q), st));
+      check(dh_attn_fwd_total(q.data_ptr(), k.data_ptr(), v.data_ptr(), out_padded.data_ptr(), lse.data_ptr<float>(),
+                              cu_seqlens_q.data_ptr<int>(), cu_seqlens_k.data_ptr<int>(), 0, 0, b, max_seqlen_q,
+                              max_seqlen_k, q.size(0), (int)q.size(1), (int)k.size(1), (int)q.size(2), token_stride(q),
+                              token_stride(k), token_stride(v), token_stride(out_padded), softmax_scale,
+                              is_causal ? 1 : 0, dt(q), st));
     });
   });
   const at::Tensor out = d_run == d_og ? out_padded : out_padded.narrow(-1, 0, d_og);

@@ -67,6 +67,18 @@ def _run_fwd_bwd(dtype, lens_q, lens_k, hq, hk, d, causal, oracle_dtype=torch.fl
     return out, lse, dq, dk, dv
 
 
+def _fwd_path(lens_q, hq, d, causal):
+    from dhellam_amd import _lib
+    return _lib.load().dh_attn_fwd_path(len(lens_q), max(lens_q), sum(lens_q), hq, d, causal)
+
+
+def _bwd_path(lens_q, lens_k, hq, hk, d, causal):
+    from dhellam_amd import _lib
+    lib, sizes = _lib.load(), (sum(lens_q), sum(lens_k))
+    ws = lib.dh_attn_bwd_workspace_bytes(*sizes, len(lens_q), max(lens_q), hq, hk, d, _lib.DH_BF16)
+    return lib.dh_attn_bwd_path(len(lens_q), max(lens_q), max(lens_k), *sizes, hq, hk, d, causal, ws)
+
+
 @pytest.fixture(params=[True, False], ids=["keep_ds", "recompute"])
 def ds_path(request):
     """Head dim 128 has two backward paths: dQ from the dS that the dK/dV pass keeps, or from recomputed S and dP."""
@@ -397,3 +409,17 @@ def test_attention_backward_many_short_sequences_and_a_long_bound(d):
     # the bound picks the kernels' tile shapes, so sums may run in another order
     for a, b, what in zip(*got, ("out", "dq", "dk", "dv")):
         assert_close(a, b.double().cpu(), dtype, what)
+
+
+# which kernels: forward 1 hand-ordered, 2 128-row tiles; backward 1 hand-ordered dK/dV, 2 dQ from kept dS or 4 hand-ordered dQ
+# (8: with 128-row tiles); (with, without room for dS)
+@pytest.mark.parametrize("lens_q,lens_k,hq,hk,causal,fwd,bwd", [
+    ([512, 491], [512, 491], 64, 64, True, 3, (13, 13)),                # full rounds, rows that end inside a tile, MHA
+    ([640, 300, 77, 513, 1, 200], [640, 300, 77, 513, 1, 200], 64, 8, True, 3, (13, 13)),     # several lengths, one row
+    ([1537], [1537], 19, 19, True, 1, (3, 5)),                           # 64-row tiles
+])
+def test_attention_hand_ordered_kernels(lens_q, lens_k, hq, hk, causal, fwd, bwd, ds_path):
+    """Head dim 128 on the kernels it has of its own."""
+    assert _fwd_path(lens_q, hq, 128, causal) == fwd
+    assert _bwd_path(lens_q, lens_k, hq, hk, 128, causal) == bwd[not ds_path]
+    _run_fwd_bwd(torch.bfloat16, lens_q, lens_k, hq, hk, 128, causal, oracle_dtype=torch.float32)
