@@ -1116,10 +1116,16 @@ static bool dq_big_grid(int batch, int max_sq, int hq, int causal) {
   return attn_wgs(max_sq, 128, hq, batch, causal) >= ATTN_128ROW_MIN_WG;
 }
 
-// Head dim 128 with short sequences: the kernels of the other head dims start and end sooner than the hand-ordered ones
-// (backward of 32 / 8 heads x 100 36 -> 27 us, 8 heads x 300 41 -> 34 us; at 600 rows 46 / 42, at 1000 level), and dS is
-// not kept.
-static bool bwd_short(int max_sq, int max_sk) { return max_sq < 512 && max_sk < 512; }
+// Head dim 128 with short sequences and little to do altogether: the kernels of the other head dims start and end sooner
+// than the hand-ordered ones, and dS is not kept.  Backward, us, hand-ordered / other: causal, query rows times heads up to
+// 16384: 32 heads x 100 36 / 27, 8 x 300 41 / 34, 32 x 500 52 / 47, 8 x 8 x 256 47 / 41; above: 64 heads x 300 50 / 57, 16 x 4 x
+// 300 43 / 51, 32 x 32 x 300 329 / 381, 20 to 470 tokens x 32 heads 72 / 83.  Not causal only the shortest: 12 heads x 19
+// 20.6 / 19.1, 4 x 34 20.9 / 20.1, but 8 x 169 + 18 27 / 30, 16 x 22 to 326 44 / 56.  (512 rows and more: within 5 % at few heads,
+// 60 / 81 at 32 x 2 x 512.)
+static bool bwd_short(int max_sq, int max_sk, int causal, int64_t total_q, int hq) {
+  if (max_sq >= 512 || max_sk >= 512) return false;
+  return causal ? total_q * hq <= 16384 : max_sq <= 48 && max_sk <= 48;
+}
 
 // What one 16-bit call runs.
 struct AttnBwdRoute {
@@ -1128,7 +1134,7 @@ struct AttnBwdRoute {
   bool big_dq;       // 128-row query tiles in dQ
 };
 static AttnBwdRoute attn_bwd_route(int batch, int max_sq, int max_sk, int64_t total_q, int hq, int d, int causal, bool room_for_ds) {
-  const bool short_rows = d == 128 && bwd_short(max_sq, max_sk), big = dq_big_grid(batch, max_sq, hq, causal);
+  const bool short_rows = d == 128 && bwd_short(max_sq, max_sk, causal, total_q, hq), big = dq_big_grid(batch, max_sq, hq, causal);
   AttnBwdRoute r;
   r.keep_ds = room_for_ds && max_sk > 0 && !short_rows;
   r.hand_dkv = d == 128 && !short_rows;

@@ -108,7 +108,7 @@ def test_attention_16bit(dtype, lens_q, lens_k, hq, hk, d, causal, ds_path):
 
 
 @pytest.mark.parametrize("lens_q,lens_k,hq,hk,causal", [
-    ([1024], [1024], 8, 1, True), ([100, 257, 64, 1], [100, 257, 64, 1], 4, 2, True), ([300, 40], [200, 97], 4, 2, False),
+    ([1024], [1024], 8, 1, True), ([300, 457, 64, 1], [300, 457, 64, 1], 24, 12, True), ([300, 40], [200, 97], 4, 2, False),
     ([2048], [1000], 8, 2, False),
 ])
 def test_attention_backward_paths_agree(lens_q, lens_k, hq, hk, causal):
@@ -128,6 +128,7 @@ def test_attention_backward_paths_agree(lens_q, lens_k, hq, hk, causal):
     try:
         for limit in (_Clib.ATTN_BWD_DS_LIMIT_DEFAULT, 0):
             _Clib.set_attn_bwd_ds_limit(limit)
+            assert _bwd_path(lens_q, lens_k, hq, hk, d, causal) == (3 if limit else 5)      # else it is one path twice
             dq, dk, dv = torch.full_like(q, float("nan")), torch.full_like(k, float("nan")), torch.full_like(v, float("nan"))
             _Clib._attn_bwd_raw(do, q, k, v, out, lse, dq, dk, dv, None, cq, ck, mq, mk, scale, causal, sp)
             got.append((dq, dk, dv))
@@ -417,9 +418,15 @@ def test_attention_backward_many_short_sequences_and_a_long_bound(d):
     ([512, 491], [512, 491], 64, 64, True, 3, (13, 13)),                # full rounds, rows that end inside a tile, MHA
     ([640, 300, 77, 513, 1, 200], [640, 300, 77, 513, 1, 200], 64, 8, True, 3, (13, 13)),     # several lengths, one row
     ([1537], [1537], 19, 19, True, 1, (3, 5)),                           # 64-row tiles
+    ([300, 129], [200, 333], 16, 4, False, 1, (3, 5)),
+    ([257, 100], [130, 31], 64, 16, False, 3, (13, 13)),
+    ([100, 257, 64, 1], [100, 257, 64, 1], 48, 16, True, 2, (9, 9)),     # short rows, but many: dK/dV only
+    ([0, 300, 65, 33], [0, 300, 65, 33], 48, 6, True, 2, (9, 9)),        # an empty sequence
+    ([384, 129], [384, 129], 48, 48, True, 2, (3, 5)),                   # dK/dV of a head in one workgroup
+    ([300, 200, 65], [300, 200, 65], 32, 4, True, 2, (3, 5)),
 ])
 def test_attention_hand_ordered_kernels(lens_q, lens_k, hq, hk, causal, fwd, bwd, ds_path):
-    """Head dim 128 on the kernels it has of its own."""
+    """Head dim 128 on the kernels it has of its own, with ragged ends, empty sequences and split / unsplit GQA groups."""
     assert _fwd_path(lens_q, hq, 128, causal) == fwd
     assert _bwd_path(lens_q, lens_k, hq, hk, 128, causal) == bwd[not ds_path]
     _run_fwd_bwd(torch.bfloat16, lens_q, lens_k, hq, hk, 128, causal, oracle_dtype=torch.float32)
