@@ -430,3 +430,16 @@ def test_attention_hand_ordered_kernels(lens_q, lens_k, hq, hk, causal, fwd, bwd
     assert _fwd_path(lens_q, hq, 128, causal) == fwd
     assert _bwd_path(lens_q, lens_k, hq, hk, 128, causal) == bwd[not ds_path]
     _run_fwd_bwd(torch.bfloat16, lens_q, lens_k, hq, hk, 128, causal, oracle_dtype=torch.float32)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d,lens,hq,hk,causal,fwd,bwd", [
+    (96, [257, 40, 1, 130], 64, 64, True, 2, 8), (96, [300, 33, 0, 96], 64, 16, False, 2, 8),
+    (128, [257, 40, 1, 130], 64, 32, True, 2, 9),                # dQ and forward; dK/dV is the hand-ordered one here
+    (192, [257, 33], 64, 64, True, 2, 0), (192, [130, 129], 80, 8, False, 2, 0),
+    (256, [257, 33], 64, 32, True, 2, 0), (256, [130, 129], 80, 8, False, 2, 0),
+])
+def test_attention_chip_filling_tiles_of_other_head_dims(dtype, d, lens, hq, hk, causal, fwd, bwd):
+    """The 128-row query tiles of the compiler-scheduled kernels, at the ends of tiles."""
+    assert _fwd_path(lens, hq, d, causal) == fwd and _bwd_path(lens, lens, hq, hk, d, causal) == bwd
+    _run_fwd_bwd(dtype, lens, lens, hq, hk, d, causal, oracle_dtype=torch.float32)
