@@ -222,8 +222,8 @@ def wgrad_gemm(grad: torch.Tensor, data: torch.Tensor, out: torch.Tensor, accumu
 # k), for which the GEMM library has its fastest kernels here: at T = 4096, bf16 (us, NN -> TN; N, K = 1280, 8192 /
 # 8192, 1024 / 7168, 8192 / 8192, 3584)  90 -> 72 / 94 -> 73 / 366 -> 308 / 205 -> 174, results identical bit for
 # bit.  A weight changes once per optimizer step and is read by every micro-batch's backward in between, and the
-# transposes (9 / 7 / 38 / 20 us) cost less than one micro-batch saves, so a weight may be registered to be kept in
-# both layouts.  The copy lives on the tensor object.  Who keeps it current: the containers that run a step
+# transposes cost 120 us of a step (9 / 7 / 38 / 20 us each and their events) against 63 us that a micro-batch of 4096
+# rows saves in a whole step, so a weight may be registered to be kept in both layouts.  The copy lives on the tensor object.  Who keeps it current: the containers that run a step
 # (``LayerRunner.run_*``, ``DSLLMStep.step``, ``run_microbatches``) rebuild the copies of their weights at the START
 # of every step with ``refresh_transposed`` (a step too short to read them marks them stale instead, with
 # ``forget_transposed``: the next reader rebuilds) -- unconditionally, because the writers that matter do not announce

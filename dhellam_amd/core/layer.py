@@ -111,10 +111,12 @@ def _shared_proxy():
     return _PROXY[0]
 
 
-# Rows of all micro-batches of a step from which keeping W^T pays.  Rebuilding the four transposes of a 70B shard's layer
-# costs 71 us; what they save per micro-batch: 94 us at 4096 rows, 57 at 2048, 39 at 1000, of which less is left against
-# the kernel that ``dgrad_gemm`` uses for few rows (22 us at 1000).
-TRANSPOSES_MIN_ROWS = 3072
+# Rows of a micro-batch from which its data gradients read W^T.  Rebuilding the four transposes of a 70B shard's layer adds
+# 120 us to a step; what they save per micro-batch: 63 us at 4096 rows, 36-44 from 3328 to 3840, 34 at 3072, 20 at 2048 and
+# nothing at 1000, so that from about here on two micro-batches pay for a rebuild (a step of one / two / four at 3072 rows
+# +87 / +54 / -14 us, at 3584 +52 / +9 / -55, at 4096 +59 / +16 / -129).  The line is drawn by the rows of ONE micro-batch:
+# its gradients then do not depend, in their last bits, on how many others share the step.
+TRANSPOSES_MIN_ROWS = 3584
 
 
 class LayerRunner:
@@ -129,7 +131,7 @@ class LayerRunner:
             self.proxy = cfg.comm_proxy or _shared_proxy()
             cfg = dataclasses.replace(cfg, comm_proxy=self.proxy)
         self.cfg = cfg
-        # for steps too short for the resident transposes to pay: the data gradients take the weights as they are
+        # for micro-batches too short for the resident transposes to pay: the data gradients take the weights as they are
         self.cfg_short = dataclasses.replace(cfg, resident_weight_transposes=False)
         self.weights = weights
         self.stream1 = stream1 or torch.cuda.Stream()
@@ -149,12 +151,12 @@ class LayerRunner:
         if self.cfg.resident_weight_transposes:
             refresh_transposed(self.weights.values())
 
-    def _step_config(self, mbs, refresh):
+    def _step_config(self, refresh):
         """The configuration a step runs with, its W^T rebuilt if it uses them and ``refresh`` asks for it.  A step that
         does not use them leaves their rebuild to whoever reads them next: they are stale from here on."""
         if not self.cfg.resident_weight_transposes:
             return self.cfg
-        short = self.cfg.tokens * len(mbs) < TRANSPOSES_MIN_ROWS
+        short = self.cfg.tokens < TRANSPOSES_MIN_ROWS
         if refresh:
             if short:
                 forget_transposed(self.weights.values())
@@ -165,7 +167,7 @@ class LayerRunner:
     def run_serial(self, mbs: List[dict], refresh_transposes: bool = True):
         """F0 B0 F1 B1 ... on ONE stream with the fwd_only / bwd_only plans.  ``refresh_transposes=False`` is for a
         caller that runs several such calls between two weight updates."""
-        cfg = self._step_config(mbs, refresh_transposes)
+        cfg = self._step_config(refresh_transposes)
         s = self.stream1
         s.wait_stream(torch.cuda.current_stream())
         self._proxy_begin()
@@ -183,7 +185,7 @@ class LayerRunner:
     def run_double_strand(self, mbs: List[dict], refresh_transposes: bool = True):
         """F0 . (F1 || B0) . (F2 || B1) ... B_last: forward strand on stream1, backward strand
         on stream2, paired steps following the plan's DCBlocks."""
-        cfg = self._step_config(mbs, refresh_transposes)
+        cfg = self._step_config(refresh_transposes)
         s1, s2 = self.stream1, self.stream2
         cur = torch.cuda.current_stream()
         s1.wait_stream(cur)

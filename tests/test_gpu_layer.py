@@ -348,12 +348,12 @@ def test_weights_updated_around_the_version_counter_are_seen_by_the_next_step():
     The sequences are long enough for a step to read W^T."""
     import dataclasses
     from dhellam_amd.core.layer import LayerRunner, make_microbatch, make_weights
-    cfg = _small_sharded_layer(2048)
+    cfg = _small_sharded_layer(4096)
     assert cfg.resident_weight_transposes
     w = make_weights(cfg, 0)
     mbs = [make_microbatch(cfg, i) for i in range(2)]
     runner = LayerRunner(cfg, w)
-    assert runner._step_config(mbs, True).resident_weight_transposes
+    assert runner._step_config(True).resident_weight_transposes
     runner.run_double_strand(mbs)                                    # a first step with the initial weights
     new = make_weights(dataclasses.replace(cfg, resident_weight_transposes=False), 7)
     proj = ("column_attn_weight", "linear_attn_weight", "column_mlp_weight", "linear_mlp_weight")
@@ -403,9 +403,23 @@ def test_a_short_step_leaves_no_stale_transposes_behind():
     for d in (w, new):
         d["cu_seqlens_q"] = d["cu_seqlens_kv"] = cu
     runner = LayerRunner(long, w)
-    assert runner._step_config([None], False).resident_weight_transposes      # this one reads W^T
+    assert runner._step_config(False).resident_weight_transposes      # this one reads W^T
     _, dxs = runner.run_serial([make_microbatch(long, 2)], refresh_transposes=False)
     _, dxs_r = LayerRunner(dataclasses.replace(long, resident_weight_transposes=False), new).run_serial(
         [make_microbatch(long, 2)])
     torch.cuda.synchronize()
     assert_close(dxs[0], dxs_r[0].cpu(), long.params_dtype, "dx (a stale W^T would be off by ~1)")
+
+
+def test_gradients_do_not_depend_on_the_micro_batches_of_a_step():
+    """dX of a micro-batch, bit for bit, whether it is a step of its own or one of four."""
+    from dhellam_amd.core.layer import LayerRunner, llama70b_tp8_shard, make_microbatch, make_weights
+    cfg = llama70b_tp8_shard(seq_length=1000)
+    w = make_weights(cfg, 0, gen_device="cuda")
+    runner = LayerRunner(cfg, w)
+    mbs = lambda: [make_microbatch(cfg, i, gen_device="cuda") for i in range(4)]
+    _, alone = runner.run_serial(mbs()[:1])
+    _, among = runner.run_double_strand(mbs())
+    _, later = runner.run_serial(mbs()[:1], refresh_transposes=False)
+    torch.cuda.synchronize()
+    assert torch.equal(alone[0], among[0]) and torch.equal(alone[0], later[0])
