@@ -381,12 +381,18 @@ Tensor matmul(const Tensor &A, const Tensor &B, const OptTensor &out, bool trans
 }
 
 // Data gradient grad [T, N] @ weight [N, K] as given.  Long reductions of few rows go to the grouped kernel with one group,
-// which splits them over the chip: us, library / here, T = 256 and 1000: N, K = 8192, 1024 28 / 22 and 44 / 31; 8192, 3584
-// 45 / 29 and 74 / 70; 7168, 8192 71 / 43 and 107 / 113 (hence few rows only for wide results).
+// which splits them over the chip.  us, library / here, at T = 32, 128, 256, 512, 1000, of a sweep over N = 2048 to 12288,
+// K = 512 to 8192:
+//   N = 8192, K = 1024   14 / 15, 29 / 19, 29 / 23, 36 / 24, 46 / 32
+//   N = 8192, K = 3584   24 / 21, 57 / 24, 46 / 31, 58 / 44, 75 / 75
+//   N = 8192, K = 4096   27 / 22, 57 / 25, 46 / 32, 58 / 47, 76 / 79: with K above 3584 not past 512 rows (6144, 4096 at 1000: 58 / 64)
+//   N = 7168, K = 8192   31 / 28, 50 / 32, 74 / 46, 66 / 71, 107 / 115: wide results only up to 256 rows
+//   N = 5120, K = 2048   12 / 13, 21 / 19, 24 / 21, 28 / 26, 40 / 37;  N = 4096, K = 2048 11 / 12, 18 / 17, 21 / 21, 23 / 25, 33 / 34:
+//   the line in N.  (K = 512 loses 2 us at 128 rows.)
 Tensor dgrad(const Tensor &grad, const Tensor &weight, const OptTensor &out, const OptStream &stream) {
   const int64_t t = grad.size(0), n = weight.size(0), k = weight.size(1);
   const auto ok = [](const Tensor &x) { return x.is_contiguous() && (uintptr_t)x.data_ptr() % 16 == 0; };
-  if (grad.dim() == 2 && weight.dim() == 2 && grad.size(1) == n && n >= 5120 && t > 0 && (t <= 256 || (k <= 4096 && t <= 1024)) &&
+  if (grad.dim() == 2 && weight.dim() == 2 && grad.size(1) == n && n >= 5120 && t > 0 && (t <= 256 || (k <= 4096 && t <= 512) || (k <= 3584 && t <= 1024)) &&
       n % 64 == 0 && k % 8 == 0 && weight.is_cuda() && grad.is_cuda() &&
       (grad.scalar_type() == at::kBFloat16 || grad.scalar_type() == at::kHalf) && weight.scalar_type() == grad.scalar_type() &&
       ok(grad) && ok(weight) && (!out.has_value() || (ok(*out) && out->scalar_type() == grad.scalar_type() && out->numel() == t * k))) {
