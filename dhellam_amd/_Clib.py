@@ -158,15 +158,17 @@ def transpose_2d(src: torch.Tensor, out: Optional[torch.Tensor] = None, stream=N
 # stream its own workspace does not change that), while the two schedules are required to agree bit for bit: not
 # used.
 # The library's transposed layouts need a row count of whole 64-deep slices, or enough rows for a ragged last one not to
-# matter: at T = 1000 fc1 takes 157 us as given and 160 + 7 us with dY^T, fc2 79 against 83 + 5, at T = 1024 147 / 125 + 6
-# and 74 / 64 + 4 us.  (A narrow weight keeps its gain: qkv at T = 1000 46 against 33 + 4 us.)
+# matter: at T = 1000 fc1 takes 160 us as given and 165 + 8 us with dY^T, fc2 83 against 85 + 5, at T = 1024 147 / 130 + 6
+# and 75 / 69 + 5 us; at T = 2000 the two are level (262 / 242 + 11, 131 / 124 + 7).  Narrow weights gain earlier: N = 1280
+# (K = 8192) at T = 840 34 / 31 + 5, at 1000 47 / 35 + 5, at 1816 57 / 47 + 5; but N = 1536 36 / 35 + 4 and 40 / 39 + 4,
+# N = 2048 43 / 44 + 5, 47 / 49 + 5 and 71 / 67 + 5.
 WGRAD_TRANSPOSE_GRAD_MIN_K = 3072
 WGRAD_TRANSPOSE_MIN_ELEMS = 1 << 20
 
 
 def wgrad_rows_ok(t: int, n: int) -> bool:
     """Whether ``t`` rows suit the transposed layouts of the weight gradient of a weight with ``n`` outputs."""
-    return t % 64 == 0 or t >= 2048 or (n <= 2048 and t >= 768)
+    return t % 64 == 0 or t >= 2048 or (n <= 1280 and t >= 768)
 
 
 def _can_transpose(t: torch.Tensor) -> bool:
@@ -223,8 +225,8 @@ def wgrad_gemm(grad: torch.Tensor, data: torch.Tensor, out: torch.Tensor, accumu
 # 8192, 1024 / 7168, 8192 / 8192, 3584)  90 -> 72 / 94 -> 73 / 366 -> 308 / 205 -> 174, results identical bit for
 # bit.  A weight changes once per optimizer step and is read by every micro-batch's backward in between, and the
 # transposes cost 120 us of a step (9 / 7 / 38 / 20 us each and their events) against 63 us that a micro-batch of 4096
-# rows saves in a whole step, so a weight may be registered to be kept in both layouts.  The copy lives on the tensor object.  Who keeps it current: the containers that run a step
-# (``LayerRunner.run_*``, ``DSLLMStep.step``, ``run_microbatches``) rebuild the copies of their weights at the START
+# rows saves in a whole step, so a weight may be registered to be kept in both layouts.  The copy lives on the tensor
+# object.  Who keeps it current: the containers that run a step (``LayerRunner.run_*``, ``DSLLMStep.step``, ``run_microbatches``) rebuild the copies of their weights at the START
 # of every step with ``refresh_transposed`` (a step too short to read them marks them stale instead, with
 # ``forget_transposed``: the next reader rebuilds) -- unconditionally, because the writers that matter do not announce
 # themselves: ``p.data.copy_()`` / ``p.data.add_()`` (Megatron's fp16 and distributed optimizers), collectives and raw
