@@ -1103,15 +1103,19 @@ static int dispatch_gg_t(const GGParams &p, int64_t m_extent, void *workspace, s
     return launch_gg_t<T, FORM, 128, 128>(p, m_extent, workspace, workspace_bytes, st);
   } else {
     // Rows per tile.  Small ones where a group's rows fit one tile (weights are then read once, by more workgroups the
-    // narrower the tile), and where tiles of 128 rows are so few that 64-row ones fill the 512 places better: fewer than
-    // half of them (then they are split along k) or about all of them.  us for 32 / 64 / 128 rows, n = 2048 of 1408, 8 groups:
-    // 24 rows a group 12.3 / 14.2 / 23.6, 48 rows 12.6 / 14.3 / 23.9, 128 rows 21.6 / 19.3 / 24.7; 64 groups, n = 1024 of
-    // 704: 16 rows 15.8 / 16.0 / 16.2, 48 rows 20.3 / 17.0 / 17.2, 100 rows 31.7 / 23.4 / 20.0.
+    // narrower the tile), and where tiles of 128 rows are so few that 64-row ones fill the 512 places better: fewer than half
+    // of them (then they are split along k), or about all of them, or, for reductions that the larger tiles cannot split
+    // either, anything in between.  us for 32 / 64 / 128 rows, n = 2048 of 1408, 8 groups: 24 rows a group 12.3 / 14.2 / 23.6,
+    // 48 rows 12.6 / 14.3 / 23.9, 128 rows 21.6 / 19.3 / 24.7; 64 groups, n = 1024 of 704: 16 rows 15.8 / 16.0 / 16.2, 48 rows
+    // 20.3 / 17.0 / 17.2, 100 rows 31.7 / 23.4 / 20.0.  64-row tiles / the better of 128x128 and 128x256, by their number and k:
+    // 256, 1408 15.8 / 24.5; 288, 2048 24.4 / 27.7; 384, 2816 33.3 / 38.9; 448, 1408 17.8 / 25.5; but 256, 2816 (2000 rows) 4 us
+    // more; 256, 7168 71.6 / 47.5; 512, 5632 91.1 / 74.9; 528, 2048 43.6 / 31.8.  Over 360 products of 16 to 65536 rows the tile
+    // picked here is 3.5 % from the best of the five kernels on average.
     const int64_t avg = m_extent / p.groups;
     const int64_t tiles64 = p.groups * (avg / 64 + 1) * cdiv(p.n_dim, 128);
     const bool few = p.groups * cdiv(avg, 128) * cdiv(p.n_dim, 128) < 400;
     if (avg <= 24 || (few && avg <= 56)) return launch_gg_t<T, FORM, 32, 128>(p, m_extent, workspace, workspace_bytes, st);
-    if (avg <= 56 || (few && (tiles64 <= 224 || (tiles64 > 340 && tiles64 <= 512 && p.k_dim <= 3072))))
+    if (avg <= 56 || (few && (tiles64 <= 224 || (tiles64 <= 512 && p.k_dim <= (tiles64 > 340 ? 3072 : 2048)))))
       return launch_gg_t<T, FORM, 64, 128>(p, m_extent, workspace, workspace_bytes, st);
     // long reductions: 128x256 tiles move a quarter less through L2 per product (3062 rows of 8 groups, n = 4096 of 5632:
     // 202 -> 178 us); short ones cannot hide the first loads and last stores of their single workgroup per compute unit
