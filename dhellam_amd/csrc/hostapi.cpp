@@ -395,7 +395,8 @@ Tensor dgrad(const Tensor &grad, const Tensor &weight, const OptTensor &out, con
   if (grad.dim() == 2 && weight.dim() == 2 && grad.size(1) == n && n >= 5120 && t > 0 && (t <= 256 || (k <= 4096 && t <= 512) || (k <= 3584 && t <= 1024)) &&
       n % 64 == 0 && k % 8 == 0 && weight.is_cuda() && grad.is_cuda() &&
       (grad.scalar_type() == at::kBFloat16 || grad.scalar_type() == at::kHalf) && weight.scalar_type() == grad.scalar_type() &&
-      ok(grad) && ok(weight) && (!out.has_value() || (ok(*out) && out->scalar_type() == grad.scalar_type() && out->numel() == t * k))) {
+      ok(grad) && ok(weight) &&
+      (!out.has_value() || (out->is_cuda() && ok(*out) && out->scalar_type() == grad.scalar_type() && out->sizes() == at::IntArrayRef({t, k})))) {
     On on(stream);
     Tensor d = out.has_value() ? *out : at::empty({t, k}, grad.options());
     Tensor ws = scratch(kGrouped, (int64_t)dh_grouped_gemm_workspace_bytes(), grad, on.get());

@@ -77,3 +77,15 @@ def test_attention_operands_off_the_gpu_are_refused(half):
         a[at] = a[at].cpu()
         with pytest.raises(RuntimeError):
             _Clib._attn_bwd_raw(*a, n, n, 0.1, True)
+
+
+def test_data_gradient_results_of_another_shape_or_place_are_refused():
+    """Few rows of a long reduction (the grouped kernel) refuse what the library product refuses."""
+    from dhellam_amd._Clib import dgrad_gemm
+    for n in (512, 8192):
+        g, w = torch.ones(8, n, device="cuda", dtype=torch.bfloat16), torch.ones(n, 16, device="cuda", dtype=torch.bfloat16)
+        assert torch.equal(dgrad_gemm(g, w, torch.empty(8, 16, device="cuda", dtype=torch.bfloat16)), torch.full((8, 16), float(n), device="cuda", dtype=torch.bfloat16))
+        for bad in (torch.empty(16, 8, device="cuda", dtype=torch.bfloat16), torch.empty(8, 16, dtype=torch.bfloat16),
+                    torch.empty(128, device="cuda", dtype=torch.bfloat16)):
+            with pytest.raises(RuntimeError):
+                dgrad_gemm(g, w, bad)
