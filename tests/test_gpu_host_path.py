@@ -89,3 +89,32 @@ def test_data_gradient_results_of_another_shape_or_place_are_refused():
                     torch.empty(128, device="cuda", dtype=torch.bfloat16)):
             with pytest.raises(RuntimeError):
                 dgrad_gemm(g, w, bad)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("t,n,k", [(1, 5120, 8), (256, 8192, 5120), (257, 7168, 4096), (512, 5120, 4096), (513, 5120, 4096), (1024, 8192, 3584),
+                                   (1025, 5120, 512), (33, 5184, 136)])
+def test_data_gradient_of_few_rows(t, n, k, dtype):
+    """Both sides of the lines between the grouped kernel with one group (no table of offsets) and the library."""
+    from dhellam_amd._Clib import dgrad_gemm
+    from tests.util import assert_close
+    g = torch.Generator(device="cuda").manual_seed(4)
+    dy, w = (torch.randn(*s, generator=g, device="cuda").to(dtype) for s in ((t, n), (n, k)))
+    assert_close(dgrad_gemm(dy, w), dy.double() @ w.double(), dtype, "dX")
+
+
+@pytest.mark.parametrize("side", [False, True])
+def test_zero_all(side):
+    """More tensors than one launch takes, of all sizes and types, some of them not in the kernel's form; neighbours stay."""
+    from dhellam_amd import _host
+    sizes = [0, 4, 8, 20, 1000, 4096, 65540] + [12] * 60 + [1 << 20, 3]
+    ts = [torch.full((n,), 7.0, device="cuda", dtype=[torch.float32, torch.bfloat16, torch.float16][i % 3]) for i, n in enumerate(sizes)]
+    guard = torch.full((64, 64), 7.0, device="cuda")
+    ts += [guard[:, :32], guard[40, 33:]]                    # a strided view, an address that is not a multiple of 16
+    st = torch.cuda.Stream() if side else None
+    if side:
+        st.wait_stream(torch.cuda.current_stream())
+    _host.zero_all(ts, st)
+    torch.cuda.synchronize()
+    assert all(torch.count_nonzero(t) == 0 for t in ts)
+    assert (guard[:40, 32:] == 7).all() and (guard[41:, 32:] == 7).all() and guard[40, 32] == 7
