@@ -88,6 +88,14 @@ def test_permute_unpermute(dtype, T, H, E, k, e_lo, e_hi):
     assert_close(dy[:R], dyo, dtype, "unpermute_bwd dy")
     dgo = OM.gate_grad(dout, y[:R], dest, offs, e_lo, e_hi, T, k)
     assert_close(dg, dgo, torch.float32, "dgates")
+    # the gate gradients alone, for callers of the C ABI that form dy themselves: the same bits
+    from dhellam_amd import _lib
+    alone = torch.full_like(dg, float("nan"))
+    dg_, yg = dout.cuda(), y.cuda()
+    _lib.check(_lib.load().dh_moe_gate_grad(dg_.data_ptr(), yg.data_ptr(), plan.dest_row.data_ptr(), alone.data_ptr(),
+                                            plan.expert_offsets.data_ptr(), e_lo, e_hi, T, k, H, _lib.dt(dg_),
+                                            torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(alone, dg)
 
 
 def test_permute_roundtrip_identity():
