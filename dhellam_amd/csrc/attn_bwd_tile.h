@@ -1,7 +1,8 @@
 // Attention backward on the tile layout of attn_tile.h (16 bits), two passes: dQ (which forms delta = rowsum(dO O) and runs
 // first) and dK/dV.  Workgroup shape and what bounds it: as the forward kernel (attn_fwd_tile.h).
 // dK/dV keeps K and V fragments and both accumulators in registers (210 at head dim 64, 255 at 96): two wavefronts a SIMD, one
-// at the larger head dims (348 at 128, all 512 at 256, where a few spill).
+// at the larger head dims (348 at 128; at 256 all 512 and 76 more that are spilled, 212 bytes a lane, of which 9 loads a tile
+// read back 24).  dQ at head dim 128 in its 64-row form spills 8 of 256, outside the loop.
 // Measured against the register-staged kernels, backward, causal: 16 heads x 2 x 512, head dim 64 58 -> 24 us; 32 query / 8
 // kv heads x 4096, head dim 64 1313 -> 324, 96 1562 -> 438, 256 10871 -> 1841 us; 16 heads x 2048, head dim 192 642 -> 201 us.
 #include "attn_tile.h"

@@ -7,7 +7,8 @@
 // softmax (400 cycles and more), so at head dim 64 the vector unit, at all of them the issue rate of the few wavefronts that
 // fit, and for short sequences the chain of one wavefront.  Head dims 64 and 96 therefore fit 128 registers: two
 // workgroups, 16 wavefronts, on a compute unit, whose matrix, softmax and LDS phases fill each other's waits without
-// hand-written ordering (WPS: wavefronts per SIMD).
+// hand-written ordering (WPS: wavefronts per SIMD).  The 128-row form at head dim 256 does not fit its 256 registers: 12 are
+// spilled (52 bytes a lane), read back by 5 loads in the loop.
 // Measured against the register-staged kernels that these head dims ran before, forward, causal: 16 heads x 2 x 512,
 // head dim 64 15.5 -> 9.4 us; 32 query / 8 kv heads x 4096, head dim 64 192 -> 94, 96 272 -> 132, 256 910 -> 329 us; 16
 // heads x 2048, head dim 192 324 -> 56 us.

@@ -169,7 +169,7 @@ __device__ __forceinline__ float pair32_sum(float x) {
 // The sequence of a batch with the given place in the order of falling length (ties: lower index first), for batches of up
 // to 64 sequences; longer ones keep their order.  Workgroups start in the order of their ids, so with the longest
 // sequences first the chip drains on short work (seven packed documents of 1 to 3324 tokens, the longest last, 32 / 8
-// heads: forward and backward 955 -> 915 us).  One load and about 10 cycles per sequence, none for a single one.
+// heads: forward and backward 949 -> 917 us).  One load and about 10 cycles per sequence, none for a single one.
 __device__ __forceinline__ int seq_by_length(const int32_t *cu, int n, int place) {
   if (n <= 1 || n > 64) return place;
   const int lane = threadIdx.x & 63;
