@@ -188,7 +188,7 @@ int dh_attn_bwd_path(int batch, int max_seqlen_q, int max_seqlen_k,
 
 /* Bytes of scratch dh_attn_bwd works in.  dh_attn_bwd_min_workspace_bytes: what
  * every call of these sizes needs (delta = rowsum(dO*O), the lse / delta planes
- * of the head-dim-128 kernels, fp32 dK/dV partials when a GQA group is split
+ * of the 16-bit kernels, fp32 dK/dV partials when a GQA group is split
  * over workgroups); a smaller workspace is refused.  dh_attn_bwd_workspace_bytes:
  * that plus room for the dS blocks of calls that would keep them (below); with
  * it the backward picks its faster form. */
@@ -200,7 +200,8 @@ size_t dh_attn_bwd_workspace_bytes(int64_t total_q, int64_t total_k, int batch,
                                    int dtype);
 
 /* Head dim 128 in 16 bits, calls too small to fill the chip with 128-row
- * query tiles (fewer than 256 of them, halved for causal): the backward keeps
+ * query tiles (fewer than 256 of them, halved for causal), except a few short
+ * rows (dh_attn_bwd_path tells): the backward keeps
  * dS = P * (dP - delta) from its dK/dV pass and forms dQ from it in one
  * product when 2 bytes per (head, query, key) (a) stay under this process-wide
  * limit (default 1280 MiB; 0: never keep) and (b) fit into the workspace the

@@ -3,6 +3,8 @@ import ctypes
 import os
 import re
 
+import pytest
+
 from dhellam_amd import _lib
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -55,6 +57,23 @@ def test_version_and_error_string_without_gpu():
     assert rc == -1 and "multiple" in lib.dh_last_error().decode()
     rc = lib.dh_moe_route_topk(None, None, None, 10, 100, 2, None)
     assert rc == -1 and "experts" in lib.dh_last_error().decode()
+
+
+@pytest.mark.parametrize("batch,max_q,total_q,hq,causal,hand", [
+    (4, 2048, 8192, 8, 1, True), (4, 2048, 8192 - 1300, 8, 1, False),        # one round of workgroups; 84 % of one
+    (7, 3324, 8192, 32, 1, True), (5, 1423, 2118, 32, 1, False),             # several lengths: four rounds of work; one of short rows
+    (1, 4352, 4352, 32, 1, False), (32, 300, 9600, 16, 1, False),            # two rounds and an eighth; short rows
+    (1, 4096, 4096, 8, 1, True), (4, 1024, 4096, 8, 1, False),               # 64-row tiles: long and short rows
+    (1, 384, 384, 16, 0, True), (1, 384, 384, 15, 0, False),                 # not causal: 96 and 90 workgroups
+    (0, 0, 0, 8, 1, False), (3, 0, 0, 8, 1, False), (2, 4096, 0, 64, 1, False), (1, 4096, 1 << 40, 8, 1, True),
+])
+def test_attention_route(batch, max_q, total_q, hq, causal, hand):
+    """Both sides of the lines between the two families of head-dim-128 kernels, and sizes at which nothing is left to divide."""
+    _ensure_lib()
+    lib = _lib.load()
+    assert bool(lib.dh_attn_fwd_path(batch, max_q, total_q, hq, 128, causal) & 1) == hand
+    assert lib.dh_attn_fwd_path(batch, max_q, total_q, hq, 96, causal) & 1 == 0
+    assert lib.dh_attn_bwd_path(batch, max_q, max_q, total_q, total_q, hq, hq, 96, causal, 1 << 40) & 7 == 0
 
 
 def test_product_does_not_import_the_oracle():
