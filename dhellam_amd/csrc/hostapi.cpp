@@ -54,11 +54,15 @@ void need_gpu(std::initializer_list<const Tensor *> ts) {
   for (const Tensor *t : ts) TORCH_CHECK(t->is_cuda(), "dhellam operators need tensors on the GPU");
 }
 
-// Runs fn() -> status without the GIL and raises its error.
-template <typename F> void launch(F &&fn) {
+// Runs fn() -> status without the GIL and raises its error.  `own`: the lock of a shared scratch buffer, held meanwhile:
+// the kernels of one call that hand each other data through it must not have those of another thread's call on the same
+// stream between them.  It is taken and given back without the GIL, so that no thread waits for one holding the other.
+template <typename F> void launch(F &&fn, std::mutex *own = nullptr) {
   int rc;
   {
     py::gil_scoped_release nogil;
+    std::unique_lock<std::mutex> lock;
+    if (own) lock = std::unique_lock<std::mutex>(*own);
     rc = fn();
   }
   TORCH_CHECK(rc == 0, "dhellam_hip error ", rc, ": ", dh_last_error());
@@ -94,8 +98,9 @@ class On {
 const void *ptr(const OptTensor &t) { return t.has_value() ? t->data_ptr() : nullptr; }
 void *mptr(const OptTensor &t) { return t.has_value() ? t->data_ptr() : nullptr; }
 
-// Scratch kept per (device, stream) and purpose: kernels on one stream are ordered, so consecutive calls may share it;
-// it grows to the largest call seen.  Never freed at exit: the allocator may be gone by then.
+// Scratch kept per (device, stream) and purpose: kernels on one stream are ordered, so consecutive calls may share it
+// (calls of several threads one after the other: `own`); it grows to the largest call seen, the replaced buffer staying with
+// the calls that hold it.  Never freed at exit: the allocator may be gone by then.
 enum Scratch { kNorm, kGemm, kAttnBwd, kGrouped, kScratchKinds };
 struct Key {
   int device;
@@ -103,15 +108,25 @@ struct Key {
   bool operator<(const Key &o) const { return device != o.device ? device < o.device : stream < o.stream; }
 };
 std::mutex g_scratch_mu;
-std::map<Key, Tensor> &scratch_map(int kind) {
-  static auto *maps = new std::array<std::map<Key, Tensor>, kScratchKinds>();
+struct Buffer {
+  Tensor t;
+  std::mutex own;
+};
+std::map<Key, Buffer> &scratch_map(int kind) {
+  static auto *maps = new std::array<std::map<Key, Buffer>, kScratchKinds>();
   return (*maps)[kind];
 }
-Tensor scratch(Scratch kind, int64_t bytes, const Tensor &like, void *stream) {
+struct Held {
+  Tensor t;
+  std::mutex *own;
+  void *data_ptr() const { return t.data_ptr(); }
+  int64_t numel() const { return t.numel(); }
+};
+Held scratch(Scratch kind, int64_t bytes, const Tensor &like, void *stream) {
   std::lock_guard<std::mutex> lock(g_scratch_mu);
-  Tensor &t = scratch_map(kind)[Key{like.device().index(), stream}];
-  if (!t.defined() || t.numel() < bytes) t = at::empty({bytes}, like.options().dtype(at::kByte));
-  return t;
+  Buffer &b = scratch_map(kind)[Key{like.device().index(), stream}];
+  if (!b.t.defined() || b.t.numel() < bytes) b.t = at::empty({bytes}, like.options().dtype(at::kByte));
+  return {b.t, &b.own};
 }
 // (device index, stream handle) of the scratch buffers of one kind that exist.
 std::vector<std::pair<int, uint64_t>> scratch_keys(int kind) {
@@ -206,12 +221,12 @@ std::tuple<Tensor, Tensor, OptTensor> norm_bwd(const Tensor &dy, const Tensor &i
     PY_ASSERT(dbeta_out.has_value() == accumulate, "pass both or neither of dgamma_out/dbeta_out");
     dbeta = dbeta_out.has_value() ? *dbeta_out : at::empty_like(weight);
   }
-  Tensor ws = scratch(kNorm, (int64_t)dh_norm_bwd_workspace_bytes(rows, cols), inp, on.get());
+  const Held ws = scratch(kNorm, (int64_t)dh_norm_bwd_workspace_bytes(rows, cols), inp, on.get());
   launch([&] {
     return dh_norm_bwd(dy.data_ptr(), inp.data_ptr(), (const float *)ptr(mu), rsigma.data_ptr<float>(),
                        weight.data_ptr(), ptr(add), dx.data_ptr(), dgamma.data_ptr(), mptr(dbeta), ws.data_ptr(),
                        (size_t)ws.numel(), rows, cols, zero_centered, accumulate, type, on.get());
-  });
+  }, ws.own);
   return {dx, dgamma, dbeta};
 }
 
@@ -325,13 +340,13 @@ void gemm_on(const Tensor &A, const Tensor &B, const Tensor &D, bool transa, boo
               "dense_gemm: operand types ", A.scalar_type(), ", ", B.scalar_type(), " -> ", D.scalar_type(), " not supported");
   const int64_t m = transa ? A.size(0) : A.size(1), n = transb ? B.size(1) : B.size(0);
   TORCH_CHECK(D.size(0) == n && D.size(1) == m, "dense_gemm: output is ", D.sizes(), ", the product is [", n, ", ", m, "]");
-  Tensor ws;
+  Held ws{{}, nullptr};
   if (!workspace.has_value() || !workspace->is_cuda() || workspace_bytes <= 0) {
     ws = scratch(kGemm, kGemmWorkspace, A, st);
     workspace_bytes = ws.numel();
   } else {
     TORCH_CHECK((int64_t)workspace->nbytes() >= workspace_bytes, "dense_gemm: workspace tensor smaller than workspaceSize");
-    ws = *workspace;
+    ws.t = *workspace;
   }
   if ((transa ? A.size(1) : A.size(0)) == 0) {
     if (!accumulate) D.zero_();
@@ -344,7 +359,7 @@ void gemm_on(const Tensor &A, const Tensor &B, const Tensor &D, bool transa, boo
                         type, out_type, ws.data_ptr(), (size_t)workspace_bytes, st);
     return dh_gemm(A.data_ptr(), B.data_ptr(), D.data_ptr(), A.size(0), A.size(1), B.size(0), B.size(1), transa, transb,
                    accumulate, type, out_type, ws.data_ptr(), (size_t)workspace_bytes, st);
-  });
+  }, ws.own);
 }
 
 void dense_gemm(const Tensor &A, const Tensor &B, const Tensor &D, bool transa, bool transb, bool accumulate,
@@ -399,12 +414,12 @@ Tensor dgrad(const Tensor &grad, const Tensor &weight, const OptTensor &out, con
       (!out.has_value() || (out->is_cuda() && ok(*out) && out->scalar_type() == grad.scalar_type() && out->sizes() == at::IntArrayRef({t, k})))) {
     On on(stream);
     Tensor d = out.has_value() ? *out : at::empty({t, k}, grad.options());
-    Tensor ws = scratch(kGrouped, (int64_t)dh_grouped_gemm_workspace_bytes(), grad, on.get());
+    const Held ws = scratch(kGrouped, (int64_t)dh_grouped_gemm_workspace_bytes(), grad, on.get());
     const int type = dt(grad);
     launch([&] {
       return dh_grouped_gemm_nn(grad.data_ptr(), weight.data_ptr(), d.data_ptr(), nullptr, 1, t, k, n, type, ws.data_ptr(),
                                 (size_t)ws.numel(), on.get());
-    });
+    }, ws.own);
     return d;
   }
   return matmul(weight, grad, out, false, stream);
@@ -467,7 +482,7 @@ void attn_bwd(const Tensor &dout, const Tensor &q, const Tensor &k, const Tensor
   const int b = (int)cu_q.numel() - 1, hq = (int)q.size(1), hk = (int)k.size(1), d = (int)q.size(2), type = dt(q);
   On on(stream);
   const size_t bytes = dh_attn_bwd_workspace_bytes(q.size(0), k.size(0), b, max_q, hq, hk, d, type);
-  Tensor ws = scratch(kAttnBwd, (int64_t)bytes, q, on.get());
+  const Held ws = scratch(kAttnBwd, (int64_t)bytes, q, on.get());
   launch([&] {
     return dh_attn_bwd_acc(dout.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr<float>(),
                            dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), (float *)mptr(delta), ws.data_ptr(),
@@ -475,7 +490,7 @@ void attn_bwd(const Tensor &dout, const Tensor &q, const Tensor &k, const Tensor
                            k.size(0), hq, hk, d, token_stride(q), token_stride(k), token_stride(v), token_stride(out),
                            token_stride(dout), token_stride(dq), token_stride(dk), token_stride(dv), (float)scale, causal,
                            accumulate_dq, type, on.get());
-  });
+  }, ws.own);
 }
 
 // ---- attention on the packed projection, as a layer calls it: split, RoPE (inv_freq given), attention in one call ------------
@@ -593,14 +608,14 @@ py::object ring_bwd(const Tensor &dout, const Tensor &out, const Tensor &q, cons
   if (r.half_k) dkv.select(2, 1).zero_();
   if (first && r.half_q) dq.select(1, 0).zero_();      // the first contribution to these rows is an addition
   const size_t bytes = dh_attn_bwd_workspace_bytes(nq, nk, 1, (int)nq, (int)r.hq, (int)r.hk, (int)r.d, type);
-  Tensor ws = scratch(kAttnBwd, (int64_t)bytes, q, on.get());
+  const Held ws = scratch(kAttnBwd, (int64_t)bytes, q, on.get());
   launch([&] {
     return dh_attn_bwd_halves(at_row(dout, q_at, r.hq, r.d), at_row(q, q_at, r.hq, r.d), kv.data_ptr(), at_row(kv, 2 * r.c, r.hk, r.d),
                               at_row(out, q_at, r.hq, r.d), lse.data_ptr<float>() + q_at, at_row(dq, q_at, r.hq, r.d), dkv.data_ptr(),
                               at_row(dkv, 2 * r.c, r.hk, r.d), nullptr, ws.data_ptr(), (size_t)ws.numel(), cu_q.data_ptr<int>(),
                               cu_k.data_ptr<int>(), r.half_q, r.half_k, (int)(2 * r.c), 1, (int)nq, (int)nk, nq, nk, (int)r.hq, (int)r.hk,
                               (int)r.d, qs, ks, ks, qs, qs, qs, ks, ks, (float)scale, step == 0, !first, type, on.get());
-  });
+  }, ws.own);
   return py::make_tuple(dq, dkv);
 }
 
@@ -738,12 +753,12 @@ Tensor grouped_gemm(const Tensor &a, const Tensor &b, const Tensor &offs, std::o
   Tensor c = out.has_value() ? *out : at::empty({held, n}, a.options());
   const int64_t rows = max_rows.value_or(held);
   if (!out.has_value() && rows < held) c.narrow(0, rows, held - rows).zero_();
-  Tensor ws = scratch(kGrouped, (int64_t)dh_grouped_gemm_workspace_bytes(), a, on.get());      // split-k pieces
+  const Held ws = scratch(kGrouped, (int64_t)dh_grouped_gemm_workspace_bytes(), a, on.get());      // split-k pieces
   launch([&] {
     return (transposed ? dh_grouped_gemm_nt : dh_grouped_gemm_nn)(a.data_ptr(), b.data_ptr(), c.data_ptr(), offs.data_ptr<int>(),
                                                                   (int)g, rows, n, k, type, ws.data_ptr(),
                                                                   (size_t)ws.numel(), on.get());
-  });
+  }, ws.own);
   return c;
 }
 
@@ -757,11 +772,11 @@ Tensor grouped_gemm_tn(const Tensor &a, const Tensor &b, const Tensor &offs, con
   const int type = dt(a);
   On on(stream);
   Tensor c = out.has_value() ? *out : at::empty({g, m, n}, a.options());
-  Tensor ws = scratch(kGrouped, (int64_t)dh_grouped_gemm_workspace_bytes(), a, on.get());
+  const Held ws = scratch(kGrouped, (int64_t)dh_grouped_gemm_workspace_bytes(), a, on.get());
   launch([&] {
     return dh_grouped_gemm_tn_ws(a.data_ptr(), b.data_ptr(), c.data_ptr(), offs.data_ptr<int>(), (int)g, a.size(0), m, n,
                                  accumulate, type, ws.data_ptr(), (size_t)ws.numel(), on.get());
-  });
+  }, ws.own);
   return c;
 }
 

@@ -118,3 +118,37 @@ def test_zero_all(side):
     torch.cuda.synchronize()
     assert all(torch.count_nonzero(t) == 0 for t in ts)
     assert (guard[:40, 32:] == 7).all() and (guard[41:, 32:] == 7).all() and guard[40, 32] == 7
+
+
+def test_threads_on_one_stream_keep_their_scratch_apart():
+    """Two threads issue operators of several kernels that hand each other data through the stream's scratch (split-k pieces,
+    partial weight gradients): every result is that of one thread alone."""
+    import threading
+    from dhellam_amd.operators import moe
+    from dhellam_amd.operators.layernorm import pylayernorm_bwd
+    g = torch.Generator(device="cuda").manual_seed(6)
+    jobs = []
+    for i in range(2):
+        a, b = torch.randn(40 + 8 * i, 4096, generator=g, device="cuda").bfloat16(), torch.randn(1, 256, 4096, generator=g, device="cuda").bfloat16()
+        offs = torch.tensor([0, a.shape[0]], dtype=torch.int32, device="cuda")
+        x, dy, w, rs = (torch.randn(*s, generator=g, device="cuda") for s in ((300, 2048), (300, 2048), (2048,), (300,)))
+        jobs.append(lambda a=a, b=b, offs=offs, x=x, dy=dy, w=w, rs=rs: (moe.grouped_gemm_nt(a, b, offs),
+                                                                        pylayernorm_bwd(dy, x, None, rs, w, 0, False, None)[1]))
+    want = [job() for job in jobs]
+    torch.cuda.synchronize()
+    stream, got = torch.cuda.current_stream(), [[], []]
+
+    def work(i):
+        with torch.cuda.stream(stream):
+            for _ in range(150):
+                got[i].append(jobs[i]())
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    for i in range(2):
+        assert len(got[i]) == 150
+        for c, dw in got[i]:
+            assert torch.equal(c, want[i][0]) and torch.equal(dw, want[i][1])
