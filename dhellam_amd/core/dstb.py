@@ -527,8 +527,15 @@ class _Ctx:
     __slots__ = ("dcfunc", "op", "config", "weight", "act", "x", "stream", "name", "movable")
 
     def __init__(self, dcfunc, op, config, weight, act, x, stream, name, movable):
-        self.dcfunc, self.op, self.config, self.weight, self.act = dcfunc, op, config, weight, act
-        self.x, self.stream, self.name, self.movable = x, stream, name, movable
+        self.dcfunc = dcfunc
+        self.op = op
+        self.config = config
+        self.weight = weight
+        self.act = act
+        self.x = x
+        self.stream = stream
+        self.name = name
+        self.movable = movable
 
     def g(self, key):
         """A saved activation, registered with the stream that is about to read it."""
@@ -1035,44 +1042,6 @@ def init_DCBlocks(config=None, stream1=None, stream2=None, context_parallel_size
 _PLAIN_PERFORM = DCoperation.perform_operation
 
 
-def _run_column(col, dcoperation, direct, config, weight, act, first_input, stream1, stream2, result, movable, fuse):
-    """Runs the ops of one column.  ``direct``: their handlers are called as ``perform_operation`` does it."""
-    skip = False
-    for i, op in enumerate(col):
-        if skip:                    # ran together with the op before it
-            skip = False
-            continue
-        inp = first_input if op.output is None else op.output
-        op.output = None
-        st = stream1 if op.strand == 1 else stream2
-        handle = None
-        num, name = op.op_num, op.name
-        handler = _HANDLERS.get(num) if direct else None
-        if fuse and name in _FUSED_FIRST and i + 1 < len(col) and (name, col[i + 1].name) in _FUSED and col[i + 1] in op.next_op:
-            nxt = col[i + 1]
-            output = dcoperation.perform_fused(DCFunc, (name, nxt.name), config, weight, act, output=inp, stream=st,
-                                               movable=movable)
-            op, skip = nxt, True    # successors and result bookkeeping are those of the second op
-            op.output = None
-        elif handler is not None:
-            output = handler(_Ctx(DCFunc, num, config, weight, act, inp, st, name, movable))
-            if num in _FREE_AFTER:
-                for key in _FREE_AFTER[num]:
-                    act.pop(key, None)
-        else:
-            output = dcoperation.perform_operation(DCFunc, num, config, weight, act, output=inp, stream=st, name=name,
-                                                   movable=movable)
-        if op.is_comm:
-            output, handle = output
-        successors = op.next_op
-        if successors:
-            for nop in successors:
-                nop.output = output
-                nop.handle = handle
-        elif output is not None:
-            result[0] = output
-
-
 def exec(config, dcoperation, fwd_weight, bwd_weight, input, grad_output, dcblocks: List[DCBlock], stream1, stream2,
          activation_dict, new_activation_dict, movable=()):
     """Walk the blocks of a plan (dstb.py:1133-1281): forward ops of the NEW micro-batch on
@@ -1094,9 +1063,46 @@ def exec(config, dcoperation, fwd_weight, bwd_weight, input, grad_output, dcbloc
     # the handlers are called directly where ``perform_operation`` is this module's own (1.1 us less an op); one that a caller
     # has replaced, in a class of their own or in this one, is called
     direct = getattr(dcoperation, "perform_operation", None) is _PLAIN_PERFORM
-    fwd_args = (dcoperation, direct, config, fwd_weight, new_activation_dict, input, stream1, stream2, fwd_res, movable, fuse)
-    bwd_args = (dcoperation, direct, config, bwd_weight, activation_dict, grad_output, stream1, stream2, bwd_res, movable,
-                fuse)
+
+    handlers, free_after = _HANDLERS, _FREE_AFTER
+
+    def run(col, weight, act, first_input, result):
+        skip = False
+        for i, op in enumerate(col):
+            if skip:                    # ran together with the op before it
+                skip = False
+                continue
+            inp, op.output = op.output, None
+            if inp is None:
+                inp = first_input
+            st = stream1 if op.strand == 1 else stream2
+            handle = None
+            num, name = op.op_num, op.name
+            if fuse and name in _FUSED_FIRST and i + 1 < len(col) and (name, col[i + 1].name) in _FUSED and col[i + 1] in op.next_op:
+                nxt = col[i + 1]
+                output = dcoperation.perform_fused(DCFunc, (name, nxt.name), config, weight, act, output=inp, stream=st,
+                                                   movable=movable)
+                op, skip = nxt, True    # successors and result bookkeeping are those of the second op
+                op.output = None
+            elif direct and num in handlers:
+                output = handlers[num](_Ctx(DCFunc, num, config, weight, act, inp, st, name, movable))
+                if num in free_after:
+                    for key in free_after[num]:
+                        act.pop(key, None)
+            else:
+                output = dcoperation.perform_operation(DCFunc, num, config, weight, act, output=inp, stream=st, name=name,
+                                                       movable=movable)
+            if op.is_comm:
+                output, handle = output
+            if op.next_op:
+                for nop in op.next_op:
+                    nop.output = output
+                    nop.handle = handle
+            elif output is not None:
+                result[0] = output
+
+    fwd_args = (fwd_weight, new_activation_dict, input, fwd_res)
+    bwd_args = (bwd_weight, activation_dict, grad_output, bwd_res)
     lockstep = (getattr(config, "lockstep_blocks", False) and stream1 is not None and stream2 is not None
                 and stream1 != stream2)
     for blk in dcblocks:
@@ -1115,17 +1121,17 @@ def exec(config, dcoperation, fwd_weight, bwd_weight, input, grad_output, dcbloc
         for op in blk.stream3_op or ():
             if op.is_comm == 1:
                 fwd_comm_first = ran_fwd = True
-                _run_column((op,), *fwd_args)
+                run((op,), *fwd_args)
             else:
-                _run_column((op,), *bwd_args)
+                run((op,), *bwd_args)
         if blk.stream1_op is not None:
             ran_fwd = True
             if not fwd_comm_first:
-                _run_column(blk.stream1_op, *fwd_args)
+                run(blk.stream1_op, *fwd_args)
         if blk.stream2_op is not None:
-            _run_column(blk.stream2_op, *bwd_args)
+            run(blk.stream2_op, *bwd_args)
         if fwd_comm_first and blk.stream1_op is not None:
-            _run_column(blk.stream1_op, *fwd_args)
+            run(blk.stream1_op, *fwd_args)
     # deferred wgrads that no placeholder op picked up run at the end (dstb.py:1268-1279)
     if activation_dict is not None and activation_dict.get("_parked"):
         for key in list(activation_dict["_parked"]):
