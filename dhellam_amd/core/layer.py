@@ -151,18 +151,20 @@ class LayerRunner:
         if self.cfg.resident_weight_transposes:
             refresh_transposed(self.weights.values())
 
+    @property
+    def step_cfg(self) -> LayerConfig:
+        """The configuration that steps run with: without W^T for micro-batches of few rows."""
+        return self.cfg_short if self.cfg.tokens < TRANSPOSES_MIN_ROWS else self.cfg
+
     def _step_config(self, refresh):
-        """The configuration a step runs with, its W^T rebuilt if it uses them and ``refresh`` asks for it.  A step that
-        does not use them leaves their rebuild to whoever reads them next: they are stale from here on."""
-        if not self.cfg.resident_weight_transposes:
-            return self.cfg
-        short = self.cfg.tokens < TRANSPOSES_MIN_ROWS
-        if refresh:
-            if short:
-                forget_transposed(self.weights.values())
-            else:
-                self.refresh_weight_transposes()
-        return self.cfg_short if short else self.cfg
+        """``step_cfg``, its W^T rebuilt if steps use them and ``refresh`` asks for it.  A step that does not use them leaves
+        their rebuild to whoever reads them next: they are stale from here on."""
+        cfg = self.step_cfg
+        if refresh and cfg.resident_weight_transposes:
+            self.refresh_weight_transposes()
+        elif refresh and self.cfg.resident_weight_transposes:
+            forget_transposed(self.weights.values())
+        return cfg
 
     def run_serial(self, mbs: List[dict], refresh_transposes: bool = True):
         """F0 B0 F1 B1 ... on ONE stream with the fwd_only / bwd_only plans.  ``refresh_transposes=False`` is for a

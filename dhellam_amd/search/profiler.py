@@ -43,13 +43,13 @@ class _Recorder:
 
 
 def record_layer(runner: LayerRunner, mb: dict) -> Dict[str, tuple]:
-    """Run one forward and one backward on one stream and record every op."""
+    """Run one forward and one backward, as steps run them, on one stream and record every op."""
     rec = _Recorder()
     s = runner.stream1
     s.wait_stream(torch.cuda.current_stream())
     act = fresh_activation_dict(mb)
-    dstb.exec(runner.cfg, rec, runner.weights, None, mb["x"], None, runner.plan.fwd_only, s, s, None, act)
-    dstb.exec(runner.cfg, rec, None, runner.weights, None, mb["dy"], runner.plan.bwd_only, s, s, act, None)
+    dstb.exec(runner.step_cfg, rec, runner.weights, None, mb["x"], None, runner.plan.fwd_only, s, s, None, act)
+    dstb.exec(runner.step_cfg, rec, None, runner.weights, None, mb["dy"], runner.plan.bwd_only, s, s, act, None)
     torch.cuda.current_stream().wait_stream(s)
     torch.cuda.synchronize()
     return rec.records
@@ -140,7 +140,7 @@ def profile_pairs(runner: LayerRunner, mb: dict, out_path: Optional[str] = None,
             for b in bwd_c:
                 if not f and not b:
                     continue
-                sp, seq, par = time_pair(records, runner.cfg, f, b, s1, s2, repeat, mode)
+                sp, seq, par = time_pair(records, runner.step_cfg, f, b, s1, s2, repeat, mode)
                 prof[(tuple(f), tuple(b))] = par
                 if fp:
                     fp.write(format_record(f, b, sp, seq, par))
