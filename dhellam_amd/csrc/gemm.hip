@@ -74,18 +74,24 @@ int make_plan(hipblasLtHandle_t h, const Key &key, int transa, int transb, int d
   DH_BLAS(hipblasLtMatmulPreferenceCreate(&pref));
   const uint64_t ws = key.ws;
   hipblasStatus_t s = hipblasLtMatmulPreferenceSetAttribute(pref, HIPBLASLT_MATMUL_PREF_MAX_WORKSPACE_BYTES, &ws, sizeof(ws));
-  hipblasLtMatmulHeuristicResult_t res[1];
-  int found = 0;
+  // The first choice may want more workspace than it was told there is (44 MiB of 32 for the data gradient [2680, 1280] x
+  // [1280, 8192]): the next one that fits is taken then.
+  hipblasLtMatmulHeuristicResult_t res[8];
+  int found = 0, pick = 0;
   if (s == HIPBLAS_STATUS_SUCCESS)
     s = hipblasLtMatmulAlgoGetHeuristic(h, pl.op, pl.a, pl.b, pl.d, pl.d, pref, 1, res, &found);
+  if (s == HIPBLAS_STATUS_SUCCESS && found >= 1 && res[0].workspaceSize > key.ws) {
+    s = hipblasLtMatmulAlgoGetHeuristic(h, pl.op, pl.a, pl.b, pl.d, pl.d, pref, 8, res, &found);
+    while (pick + 1 < found && res[pick].workspaceSize > key.ws) ++pick;
+  }
   hipblasLtMatmulPreferenceDestroy(pref);
   if (s != HIPBLAS_STATUS_SUCCESS || found < 1) {
     ::dh::set_error(__FILE__, __LINE__, __func__, "hipBLASLt has no kernel for m=%lld n=%lld k=%lld (status %d)",
                     (long long)m, (long long)n, (long long)k, (int)s);
     return DH_ERR_UNSUPPORTED;
   }
-  pl.algo = res[0].algo;
-  pl.ws_needed = res[0].workspaceSize;
+  pl.algo = res[pick].algo;
+  pl.ws_needed = res[pick].workspaceSize;
   return DH_OK;
 }
 
