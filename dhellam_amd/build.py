@@ -84,14 +84,14 @@ def build(verbose: bool = False, jobs: int | None = None) -> Path:
 
 
 def check_grouped_gemm_loops(verbose: bool = False) -> int:
-    """The chip-filling grouped GEMM kernel (``grouped_gemm_w4_kernel``) issues its loads from assembly, so the compiler
-    does not know that their results arrive later: the kernel is only correct if, between a load and the LDS write
-    that consumes it, NO instruction names the loaded registers (a register copy or a spill there would move data
-    that has not arrived).  The source arranges that; this check holds the generated code to it.  It compiles
+    """The chip-filling grouped GEMM kernel (``grouped_gemm_w8_kernel``) copies its operands to LDS from assembly, which
+    the compiler does not count: that no copy overtakes a fragment read and no read a copy rests on the order of reads,
+    waits, copies and barriers that the source lays down.  This check holds the generated code to it.  It compiles
     ``grouped_gemm.hip`` to device assembly and, in the main loop of every instantiation of the kernel (the innermost
-    loop with 32 loads), follows each ``buffer_load_dwordx4`` destination to its ``ds_write_b128`` across the loop's
-    back edge; it also refuses scratch accesses and register copies inside that loop.  Returns the number of loops
-    checked; raises on a violation."""
+    loop with 128 MFMAs: two k slices), cuts the code at its barriers: clusters of 16 MFMAs have to alternate with
+    clusters of none, copies may stand in the latter only, each of these has to begin by waiting for the wavefront's
+    earlier LDS reads, and where copies are published the wait for them is the one the source counts.  It also refuses
+    scratch accesses and accumulator copies inside the loop.  Returns the number of loops checked; raises on a violation."""
     import re
     import tempfile
     with tempfile.TemporaryDirectory() as td:
@@ -102,69 +102,63 @@ def check_grouped_gemm_loops(verbose: bool = False) -> int:
             raise RuntimeError("hipcc -S failed for grouped_gemm.hip:\n" + res.stderr)
         lines = out.read_text().split("\n")
 
-    def regs(tok: str) -> set:
-        m = re.match(r"v\[(\d+):(\d+)\]$", tok)
-        if m:
-            return set(range(int(m.group(1)), int(m.group(2)) + 1))
-        m = re.match(r"v(\d+)$", tok)
-        return {int(m.group(1))} if m else set()
-
     checked = 0
-    starts = [i for i, l in enumerate(lines) if re.match(r"^_ZN2dh22grouped_gemm_w4_kernel\w+:", l)]
-    for a in starts:
+    for a in [i for i, l in enumerate(lines) if re.match(r"^_ZN2dh22grouped_gemm_w8_kernel\w+:", l)]:
         b = next(i for i in range(a, len(lines)) if lines[i].startswith(".Lfunc_end"))   # (a kernel may hold several s_endpgm)
         fn = lines[a:b]
+        name = fn[0].split(":")[0]
         labels = {m.group(1): i for i, l in enumerate(fn) if (m := re.match(r"^(\.LBB\d+_\d+):", l))}
         loops = []
         for i, l in enumerate(fn):
-            m = re.match(r"\s+s_cbranch_\w+ (\.LBB\d+_\d+)", l)
+            m = re.match(r"\s+s_c?branch\w* (\.LBB\d+_\d+)", l)
             if m and m.group(1) in labels and labels[m.group(1)] < i:
-                body = fn[labels[m.group(1)]:i]
-                if sum("buffer_load_dwordx4" in x for x in body) == 32:
+                body = [x.split(";")[0].strip() for x in fn[labels[m.group(1)] + 1:i]]
+                body = [x for x in body if x and not x.endswith(":")]
+                if sum("v_mfma" in x for x in body) == 128:
                     loops.append(body)
         if not loops:
-            raise RuntimeError(f"{fn[0].split(':')[0]}: no main loop with 32 loads found (the kernel's structure changed: "
-                               "update check_grouped_gemm_loops)")
+            raise RuntimeError(f"{name}: no main loop with 128 MFMAs found (the kernel's structure changed: update "
+                               "check_grouped_gemm_loops)")
         body = min(loops, key=len)
-        name = fn[0].split(":")[0]
         for l in body:
-            if "scratch_" in l or re.match(r"\s+v_mov_b\d+", l) or "v_accvgpr" in l:
-                raise RuntimeError(f"{name}: '{l.strip()}' inside the main loop")
-        if sum("v_mfma" in x for x in body) != 128:
-            raise RuntimeError(f"{name}: {sum('v_mfma' in x for x in body)} MFMAs in the main loop, expected 128")
-        # the same rule from the first load of the function up to the loop (the prologue's loads, whose results the
-        # loop's first slices write to LDS) and from the loop's end to the wait for every load that follows it
-        lo = next(i for i, l in enumerate(fn) if l is body[0])
-        first = next(i for i, l in enumerate(fn) if "buffer_load_dwordx4" in l)
-        hi = lo + len(body)
-        end = next((i for i in range(hi, len(fn)) if "s_waitcnt vmcnt(0)" in fn[i]), None)
-        if first >= lo or end is None:
-            raise RuntimeError(f"{name}: prologue loads or the wait behind the loop not found")
-        pending: dict = {}
-        for n, l in enumerate(fn[first:lo] + body + body + fn[hi:end]):   # the loop twice: values live across the back edge
-            t = l.replace(",", " ").split()
-            if not t or t[0].startswith((";", ".")):
+            if "scratch_" in l or "v_accvgpr" in l:
+                raise RuntimeError(f"{name}: '{l}' inside the main loop")
+        clusters, cluster = [], []
+        for l in body:
+            if l.startswith("s_barrier"):
+                clusters.append(cluster)
+                cluster = []
+            else:
+                cluster.append(l)
+        clusters[0] = cluster + clusters[0]                  # what follows the last barrier runs into the loop's head
+        if len(clusters) != 16:
+            raise RuntimeError(f"{name}: {len(clusters)} barriers in the main loop, expected 16")
+        copies = 0
+        for n, cl in enumerate(clusters):
+            mfma = sum("v_mfma" in x for x in cl)
+            dma = [i for i, x in enumerate(cl) if x.startswith("buffer_load")]
+            if mfma != (16 if n % 2 else 0):
+                raise RuntimeError(f"{name}: cluster {n} holds {mfma} MFMAs")
+            copies += len(dma)
+            if n % 2:
+                if dma:
+                    raise RuntimeError(f"{name}: a copy among the MFMAs of cluster {n}")
                 continue
-            if t[0] == "buffer_load_dwordx4":
-                for r in regs(t[1]):
-                    if r in pending:
-                        raise RuntimeError(f"{name}: v{r} is loaded again before the LDS write of its previous load")
-                    pending[r] = n
-                continue
-            if t[0] == "s_waitcnt" and "vmcnt(0)" in l:     # everything has arrived
-                pending.clear()
-                continue
-            touched = set().union(*[regs(x) for x in t[1:]]) & set(pending)
-            if touched:
-                if t[0] != "ds_write_b128":
-                    raise RuntimeError(f"{name}: '{l.strip()}' names a register whose load may still be in flight")
-                for r in touched:
-                    pending.pop(r)
+            waits = [i for i, x in enumerate(cl) if x == "s_waitcnt lgkmcnt(0)"]
+            reads = [i for i, x in enumerate(cl) if x.startswith("ds_read")]
+            if not waits or (reads and reads[0] < waits[0]) or (dma and dma[0] < waits[0]):
+                raise RuntimeError(f"{name}: cluster {n} does not begin with the wait for the earlier reads")
+            if any(not x.endswith("lds") for x in (cl[i] for i in dma)):
+                raise RuntimeError(f"{name}: a load to registers in cluster {n}")
+            if dma and "s_waitcnt vmcnt(8)" not in cl[dma[-1]:]:
+                raise RuntimeError(f"{name}: cluster {n} publishes copies without the counted wait")
+        if copies != 16:
+            raise RuntimeError(f"{name}: {copies} copies in the main loop, expected 16")
         checked += 1
         if verbose:
             print(f"checked {name}: {len(body)} lines", flush=True)
     if checked == 0:
-        raise RuntimeError("no grouped_gemm_w4_kernel instantiation found in the assembly")
+        raise RuntimeError("no grouped_gemm_w8_kernel instantiation found in the assembly")
     return checked
 
 

@@ -6,8 +6,8 @@
 //   NT  c[r, n]  = sum_k a[r, k] * w[g][n, k]      forward  (both k-contiguous)
 //   NN  c[r, n]  = sum_k a[r, k] * w[g][k, n]      dgrad    (w strided in k)
 //   TN  c[g][m,n] = sum_r a[r, m] * b[r, n]        wgrad    (both strided in k = r)
-// Two kernels.  grouped_gemm_w4_kernel (products that fill the chip): 256x256 tiles, four wavefronts of 128x128 with
-// hand-placed copies, optionally one workgroup per compute unit that takes whole tiles in rounds and a k piece of a tile
+// Two kernels.  grouped_gemm_w8_kernel (products that fill the chip): 256x256 tiles, eight wavefronts in two alternating
+// groups, optionally one workgroup per compute unit that takes whole tiles in rounds and a k piece of a tile
 // of the last round.  grouped_gemm_t_kernel (everything else): smaller tiles, copied straight to LDS, split along k where
 // there are few of them.  k-contiguous operands are read from LDS as 16-byte row fragments; k-strided operands stay
 // row-major in LDS and are read with transpose loads, so no operand is ever transposed in memory.
@@ -35,8 +35,8 @@ struct GGParams {
   int accumulate;
   int max_rows;          // rows the stacked operands hold: group ranges read from offs are cut off there
   float *ws;             // split last round: fp32 partial tiles, one per workgroup
-  int zero_tail;         // NT/NN on grouped_gemm_w4_kernel: the kernel itself zeroes the rows of c past the last group
-  int sk_grid;           // grouped_gemm_w4_kernel: > 0: a split kernel of that many workgroups follows and takes the last round of tiles if it splits it;
+  int zero_tail;         // NT/NN on grouped_gemm_w8_kernel: the kernel itself zeroes the rows of c past the last group
+  int sk_grid;           // grouped_gemm_w8_kernel: > 0: a split kernel of that many workgroups follows and takes the last round of tiles if it splits it;
                          // grouped_gemm_t_kernel, NT/NN: > 0: places for workgroups, over which the tiles may be split along k
   int pieces;            // grouped_gemm_t_kernel, TN: k pieces per tile
 };
@@ -94,26 +94,36 @@ __device__ __forceinline__ void gg_locate(const GGGroupTable &gt, int tm_all, in
   tm = tm_all - (__builtin_amdgcn_readlane(gt.incl, g) - (re - rb + BM - 1) / BM);
 }
 
-// ---- 256x256 tiles with ONE wavefront per SIMD: four wavefronts of 128x128 outputs ------------------------------
-// The 256 accumulator registers of a wavefront live in AGPRs, and the loop is written slot by slot: after every
-// MFMA exactly one LDS or memory instruction (fragment read, staging-register write to LDS, buffer load), so that
-// the matrix pipe never waits for a burst of them and the LDS queue never fills.  A 64-deep k slice is loaded
-// into registers THREE slices ahead (two staging sets of 16 x 16 bytes per lane), written to the LDS stage that
-// is not being read during the first half of a slice, published by the slice's one barrier and read as fragments
-// one k step (16) ahead of the MFMAs that use them.  Against eight wavefronts of 128x64 (two per SIMD): a third
-// fewer fragment reads per MFMA, and the MFMAs of one wavefront run back to back instead of two wavefronts
-// alternating on the pipe.
-// Tiles in LDS: k-contiguous operands as [256 rows][64 k] with unpadded 128-byte rows, the 16-byte chunk index
-// XORed with (row / 2) % 8 (conflict-free 16-byte row-fragment reads); a k-strided operand (B of the NN product,
-// [k][n] row-major) as [64 k][256 n] with 512-byte rows, chunk ^= 4 (k % 4) + (k / 4) % 4 inside each 256-byte
-// half row, read as fragments by LDS transpose reads.
+// ---- 256x256 tiles, eight wavefronts in two alternating groups ---------------------------------------------------
+// Eight wavefronts of 128x64 outputs (two per SIMD) on v_mfma_f32_16x16x32: under a sustained load this board is bound by
+// power, and that instruction delivers 2.03 PFLOP/s where 32x32x16 stops at 1.79 (loops of nothing else on normal data).
+// The operands of a 64-deep k slice are copied straight to LDS (two stages of four 16 KB regions: the A rows and the B
+// columns of the tile in two halves each), and every wavefront works through a slice in four quarters of its outputs, a
+// quarter being [reads of fragments, copies | 16 MFMAs, more reads among them], each half of it ended by a barrier.  The
+// wavefronts 4..7 start one barrier late, so that on every SIMD one wavefront has its 16 MFMAs while the other reads LDS and
+// issues copies.  Slice s, F = the half of B that is multiplied first (s % 2), G = the other:
+//   cluster 0  read G                             1  A0 x F, read A1
+//           2  read A1     copy A0 of s + 2       3  A0 x G, read A1
+//           4  read A0'    copy F of s + 2        5  A1 x G, read A0'      (A0', F': of slice s + 1)
+//           6  read F'     copy G, A1 of s + 2    7  A1 x F, read A0'
+// Fragments are read at least one cluster of MFMAs ahead of their use.  Why no copy overtakes a read: a read cluster begins
+// with the wait for the wavefront's earlier reads, so what was read up to cluster c is in registers, for the leading group by
+// cluster c + 2 and for the other one barrier later; the copies into a region go out behind the next barrier after that.
+// Why no read overtakes a copy: two clusters before a region is read every wavefront waits for its own copies of it (copies
+// complete in order, so `vmcnt` counts those issued behind them); both groups are past that wait when the leading one
+// reads.  8 copies stay in flight across every barrier.
 //
-// The loads are buffer loads issued from assembly: the compiler does not count them, every use of a staging
-// register is ordered by a hand-written s_waitcnt vmcnt (loads return in order), and between its load and its
-// LDS write a staging register is touched by nothing else (every build checks the generated assembly for this:
-// check_grouped_gemm_loops in dhellam_amd/build.py).  The buffer descriptors do the edge handling: their
-// length is cut at the group's (or n's) last row, so that rows past the end read as zero and no access leaves
-// the operands, whatever the offsets table says.
+// LDS regions: a k-contiguous operand as [128 rows][64 k] (128-byte rows, 16-byte chunk XOR (row / 2) % 8: row-fragment reads
+// hit 16 different chunks), a k-strided one as [64 k][128 columns] (256-byte rows, chunk XOR 4 (k % 4) + (k / 4) % 4), read as
+// fragments by LDS transpose reads.  The XOR is applied to the global chunk that a lane fetches.  Buffer descriptors do the edge
+// handling: their length is cut at the group's (or n's) last row, so that rows past the end read as zero and no access leaves
+// the operands, whatever the offsets table says; slices past the last one are copied with a length of zero, or the old
+// tile is copied in their place (below).
+// us, against the kernel before it (four wavefronts on 32x32x16, operands staged through registers); two groups of 2048 rows:
+// NT n = 28672 of 4096 764 -> 705, n = 4096 of 14336 375 -> 331; NN 778 -> 704 and 380 -> 336; TN 862 -> 778 and 425 -> 389,
+// accumulating 1091 -> 806 and 531 -> 413.  One group of 8192 x 8192 x 8192: NT 802 -> 721 (1.52 PFLOP/s; the library 709), TN
+// 849 -> 783 (1.40; the library 928).  What bounds it: power (matrix pipes 82 % busy at 1.76 GHz, TN 71 % at 1.92), and per tile
+// about 8 us of first copies and last stores.
 typedef int gg_i32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ gg_i32x4 gg_rsrc(const void *ptr, int64_t bytes) {
@@ -127,74 +137,63 @@ __device__ __forceinline__ gg_i32x4 gg_rsrc(const void *ptr, int64_t bytes) {
   return r;
 }
 
-// Stores a 256x256 tile held in the accumulator layout of grouped_gemm_w4_kernel (wavefront w = 2 wm + wn owns the
-// 128x128 block (wm, wn); acc[i][j] is its 32x32 block (i, j), transposed: lane column c is output row c).
-template <typename T, bool MAY_ACCUMULATE>
-__device__ __forceinline__ void gg_w4_store(const floatx16 (&acc)[4][4], unsigned char *smem, const GGParams &p, T *cbase, int m0,
-                                            int n0, int a_rext, int b_rext) {
+// One 1 KB copy global -> LDS: lane offset + scalar offset from the descriptor's base, wave-uniform LDS byte address.
+template <typename T>
+__device__ __forceinline__ void gg_copy_lds(uint32_t lane_off, const gg_i32x4 &rsrc, uint32_t off, uint32_t lds_dst) {
+  asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
+               :
+               : "v"(lane_off), "s"(rsrc), "s"(off), "s"(lds_dst)
+               : "memory", "m0");
+}
+
+// The outputs of a wavefront (wm = w / 4, wn = w % 4): quarter (qm, qn) holds rows 128 qm + 64 wm + 16 mi + .. and columns
+// 128 qn + 32 wn + 16 nj + .. of the tile; its 16x16 blocks lie transposed in the accumulators (lane % 16: output row, four
+// consecutive columns 4 (lane / 16) + .. a lane).
+typedef floatx4 GGAcc8[2][2][4][2];          // [qm][qn][mi][nj]
+
+// Stores a tile through LDS ([256][512 bytes], the 16-byte chunk index XORed with row % 16: 8-byte accesses of 16 rows fall on
+// different banks), so that 32 lanes write a row of 512 bytes.  ADD: LDS holds the old tile, to which each lane adds what it
+// holds, with one rounding.
+template <typename T, bool ADD>
+__device__ __forceinline__ void gg_w8_store(const GGAcc8 &acc, unsigned char *smem, const GGParams &p, T *cbase, int m0, int n0,
+                                            int a_rext, int b_rext) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int c = lane & 31, hh = lane >> 5;
-  const int wm = w >> 1, wn = w & 1;
-  // Epilogue: each wavefront passes its 128x128 block through a private LDS region, 64 rows at a time, and stores
-  // whole 256-byte row segments (16 lanes a row, 4 rows per instruction).  Rows of 264 bytes: the 8-byte writes of
-  // 32 lanes (32 rows, one column) fall on different banks.
-  constexpr int EP = 264;
-  static_assert(4 * 64 * EP <= 128 * 1024, "epilogue staging fits in the stage buffers");
-  unsigned char *ep = smem + w * (64 * EP);
-  T *cg = cbase + (int64_t)m0 * p.ldc + n0 + wn * 128;
+  const int wm = w >> 2, wn = w & 3;
   struct alignas(8) Q4 { T v[4]; };
-  if (MAY_ACCUMULATE && p.accumulate) {
-    // c += product with one rounding: straight from the accumulators (a lane owns output row c of each 32x32 block
-    // and 4 consecutive columns per register quad)
+  const int r16 = lane & 15, g4 = lane >> 4;
+  unsigned char *mine = smem + (64 * wm + r16) * 512 + (g4 & 1) * 8;
+  const int ch = (4 * wn + (g4 >> 1)) ^ r16;                      // chunk of columns 32 wn + 4 g4; + 16 columns: two chunks on
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int m = wm * 128 + 32 * i + c;
+  for (int qm = 0; qm < 2; ++qm)
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+    for (int qn = 0; qn < 2; ++qn)
 #pragma unroll
-        for (int vb = 0; vb < 4; ++vb) {
-          const int n = 32 * j + 8 * vb + 4 * hh;
-          if (m < a_rext && wn * 128 + n < b_rext) {
-            Q4 *dst = reinterpret_cast<Q4 *>(cg + (int64_t)m * p.ldc + n);
-            const Q4 old = *dst;
-            Q4 o;
+      for (int mi = 0; mi < 4; ++mi)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) o.v[e] = static_cast<T>(acc[i][j][4 * vb + e] + static_cast<float>(old.v[e]));
-            *dst = o;
-          }
-        }
-    }
-    return;
-  }
-  const int er = lane >> 4, ec = lane & 15;
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-#pragma unroll
-    for (int i2 = 0; i2 < 2; ++i2)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const floatx16 av = acc[2 * h + i2][j];
-#pragma unroll
-        for (int vb = 0; vb < 4; ++vb) {
+        for (int nj = 0; nj < 2; ++nj) {
+          Q4 *dst = reinterpret_cast<Q4 *>(mine + (128 * qm + 16 * mi) * 512 + ((ch ^ (2 * nj)) + 16 * qn) * 16);
+          const floatx4 av = acc[qm][qn][mi][nj];
           Q4 o;
+          if constexpr (ADD) {
+            const Q4 old = *dst;
 #pragma unroll
-          for (int e = 0; e < 4; ++e) o.v[e] = static_cast<T>(av[4 * vb + e]);
-          *reinterpret_cast<Q4 *>(ep + (32 * i2 + c) * EP + (32 * j + 8 * vb + 4 * hh) * (int)sizeof(T)) = o;
+            for (int e = 0; e < 4; ++e) o.v[e] = static_cast<T>(av[e] + static_cast<float>(old.v[e]));
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o.v[e] = static_cast<T>(av[e]);
+          }
+          *dst = o;
         }
-      }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_wave_barrier();
-    const int mh = wm * 128 + 64 * h;                   // first row of this half in the tile
-#pragma unroll
-    for (int it = 0; it < 16; ++it) {
-      const int r = 4 * it + er;
-      const dh_u32x4 o = *reinterpret_cast<const dh_u32x4 *>(ep + r * EP + ec * 16);
-      if (mh + r < a_rext && wn * 128 + 8 * ec < b_rext)
-        *reinterpret_cast<dh_u32x4 *>(cg + (int64_t)(mh + r) * p.ldc + 8 * ec) = o;
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_wave_barrier();
+  __syncthreads();
+  const int er = tid >> 5, ec = tid & 31;                         // row of 16 and chunk
+  const unsigned char *src = smem + er * 512 + ((ec ^ er) << 4);
+  T *row0 = cbase + (int64_t)(m0 + er) * p.ldc + n0 + 8 * ec;
+  if (8 * ec < b_rext) {
+#pragma unroll 8
+    for (int it = 0; it < 16; ++it)
+      if (16 * it + er < a_rext)
+        *reinterpret_cast<dh_u32x4 *>(row0 + (int64_t)(16 * it) * p.ldc) = *reinterpret_cast<const dh_u32x4 *>(src + it * (16 * 512));
   }
 }
 
@@ -208,20 +207,20 @@ __device__ __forceinline__ int gg_sk_pieces(int grid, int rem, int nsl) {
 // FORM 0: NT (both operands k-contiguous); 1: NN (b k-strided); 2: TN (both k-strided, k = the group's rows, one output
 // per group).
 template <typename T, int FORM, bool SK>
-__global__ void __launch_bounds__(256) grouped_gemm_w4_kernel(const GGParams p) {
+__global__ void __launch_bounds__(512) grouped_gemm_w8_kernel(const GGParams p) {
   constexpr bool BKS = FORM >= 1, AKS = FORM == 2;
   static_assert(!(AKS && SK), "the wgrad form has many tiles and a short k: it is never split");
   using M = Mma<T>;
   using Frag = typename M::Frag;
-  constexpr int BM = 256, ROWB = 128, BROWB = 512, TILEB = 256 * ROWB, STAGEB = 2 * TILEB;
-  constexpr int NRD = AKS ? 16 : (BKS ? 12 : 8);        // LDS read instructions per k step
+  constexpr int BM = 256;
+  constexpr uint32_t REG = 16384, STAGEB = 4 * REG, OFF_B = 2 * REG;     // regions A0 A1 B0 B1
   __shared__ __attribute__((aligned(1024))) unsigned char smem[2 * STAGEB];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int c = lane & 31, hh = lane >> 5;
-  const int wm = w >> 1, wn = w & 1;
-  const int nsl = (int)(p.k_dim / 64);
+  const int wm = w >> 2, wn = w & 3;
+  const int c = lane & 15, g4 = lane >> 4;
+  const int nsl = (int)((p.k_dim + 63) / 64);
   const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
   const uint32_t lda_b = (uint32_t)p.lda * (uint32_t)sizeof(T), ldb_b = (uint32_t)p.ldb * (uint32_t)sizeof(T);
   const int base = gg_off(p, 0);
@@ -234,231 +233,232 @@ __global__ void __launch_bounds__(256) grouped_gemm_w4_kernel(const GGParams p) 
       const int nv = (int)(p.n_dim / 8);
       for (int r = first + (int)blockIdx.x; r < p.max_rows; r += (int)gridDim.x) {
         T *row = reinterpret_cast<T *>(p.c) + (int64_t)r * p.ldc;
-        for (int v = tid; v < nv; v += 256) *reinterpret_cast<dh_u32x4 *>(row + 8 * v) = dh_u32x4{0u, 0u, 0u, 0u};
+        for (int v = tid; v < nv; v += 512) *reinterpret_cast<dh_u32x4 *>(row + 8 * v) = dh_u32x4{0u, 0u, 0u, 0u};
       }
     }
   }
 
-  // ---- copies ----------------------------------------------------------------------------------------------
-  // k-contiguous tile [256 rows][64 k]: a lane copies chunk lc of rows lr + 32 i.
-  // k-strided tile [64 k][256 n]: a lane copies chunk cx of k rows kr + 8 i.
-  const int lc = tid & 7, lr = tid >> 3, cx = tid & 31, kr = tid >> 5;
-  const uint32_t goff_a = AKS ? (uint32_t)kr * lda_b + (uint32_t)(cx * 16) : (uint32_t)lr * lda_b + (uint32_t)(lc * 16);
-  const uint32_t goff_b = BKS ? (uint32_t)kr * ldb_b + (uint32_t)(cx * 16) : (uint32_t)lr * ldb_b + (uint32_t)(lc * 16);
-  const uint32_t kstep_a = AKS ? 64 * lda_b : 64 * (uint32_t)sizeof(T);       // bytes from one k slice to the next
-  const uint32_t kstep_b = BKS ? 64 * ldb_b : 64 * (uint32_t)sizeof(T);
-  const uint32_t rstep_a = AKS ? 8 * lda_b : 32 * lda_b, rstep_b = BKS ? 8 * ldb_b : 32 * ldb_b;   // bytes from one copy of a lane to its next
-  const uint32_t wr_kc = (uint32_t)(lr * ROWB + ((lc ^ ((lr >> 1) & 7)) << 4));                     // + i * 4096
-  // k-strided tile: chunk XOR 4 (k % 4) + (k / 4) % 4 with k = kr + 8 i: the i part is bit 1 of the chunk for odd i
-  const uint32_t wr_ks = (uint32_t)(kr * BROWB + (cx >> 4) * 256 + (((cx & 15) ^ (4 * (kr & 3) + (kr >> 2))) << 4));
-  const uint32_t wr_a = AKS ? wr_ks : wr_kc, wr_b = (uint32_t)TILEB + (BKS ? wr_ks : wr_kc);
+  // ---- copies: a region is 16 blocks of 1 KB, a wavefront takes blocks 2 w and 2 w + 1.  k-contiguous: a block is 8 rows (a lane:
+  // row lane / 8, chunk lane % 8); k-strided: 4 k rows (row lane / 16, chunk lane % 16)
+  uint32_t va[2], vb[2];                                                 // lane offsets of the two blocks
+  {
+    const int r8 = lane >> 3, ch = (lane & 7) ^ (r8 >> 1), r4 = lane >> 4, cs = (lane & 15) ^ (4 * r4);
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+      const int b = 2 * w + x;
+      const uint32_t kc = (uint32_t)((ch ^ (4 * x)) << 4), ks = (uint32_t)((cs ^ (b & 3)) << 4);
+      va[x] = AKS ? (uint32_t)(4 * b + r4) * lda_b + ks : (uint32_t)(8 * b + r8) * lda_b + kc;
+      vb[x] = BKS ? (uint32_t)(4 * b + r4) * ldb_b + ks : (uint32_t)(8 * b + r8) * ldb_b + kc;
+    }
+  }
+  const uint32_t kstep_a = AKS ? 64 * lda_b : 128, kstep_b = BKS ? 64 * ldb_b : 128;        // bytes from one k slice to the next
+  const uint32_t half_a = AKS ? 256 : 128 * lda_b, half_b = BKS ? 256 : 128 * ldb_b;        // bytes to the second half of the tile
+  const uint32_t cp_lds = lds0 + (uint32_t)(w * 2048);
 
-  // ---- fragment reads --------------------------------------------------------------------------------------
-  const uint32_t sw = (uint32_t)((hh ^ ((c >> 1) & 7)) << 4);
-  const uint32_t fa_lane = (uint32_t)((wm * 128 + c) * ROWB) + sw;                  // k step: XOR 32 ks; block i: + 4096 i
-  const uint32_t fb_lane = (uint32_t)(TILEB + (wn * 128 + c) * ROWB) + sw;
-  const int r16 = lane & 15;
-  const int t_lc = 2 * ((lane >> 4) & 1) + ((r16 & 3) >> 1);
-  const int tx = 4 * (r16 >> 2) + 2 * hh;
-  const uint32_t t_row = (uint32_t)((8 * hh + (r16 >> 2)) * BROWB + ((r16 & 3) & 1) * 8);
-  const uint32_t t_lo = t_row + (uint32_t)((t_lc ^ tx) << 4);                       // k rows 8 hh + 0..3 of a step
-  const uint32_t t_hi = t_row + 4 * BROWB + (uint32_t)((t_lc ^ (tx + 1)) << 4);     // k rows 8 hh + 4..7
-  const uint32_t tb_a = (uint32_t)(TILEB + wn * 256) + t_lo, tb_b = (uint32_t)(TILEB + wn * 256) + t_hi;   // B tile, this wavefront's 128 columns
-  const uint32_t ta_a = (uint32_t)(wm * 256) + t_lo, ta_b = (uint32_t)(wm * 256) + t_hi;                   // A tile (TN)
+  // ---- fragments: lane row (column) c of a 16-row block, k = 8 g4 + 0..7 of a step of 32
+  const uint32_t sw = (uint32_t)((g4 ^ ((c >> 1) & 7)) << 4);
+  const uint32_t fa_lane = (uint32_t)((wm * 64 + c) * 128) + sw, fb_lane = (uint32_t)((wn * 32 + c) * 128) + sw;   // step: XOR 64; block: + 2048
+  const int tx = 4 * (c >> 2) + ((2 * g4) & 3);
+  const uint32_t t_row = (uint32_t)((8 * g4 + (c >> 2)) * 256 + (c & 1) * 8);
+  const uint32_t t_lo = t_row + (uint32_t)((((c & 3) >> 1) ^ tx) << 4);                    // k rows 8 g4 + 0..3 of a step
+  const uint32_t t_hi = t_row + 1024 + (uint32_t)((((c & 3) >> 1) ^ (tx + 1)) << 4);       // k rows 8 g4 + 4..7
   typedef __attribute__((address_space(3))) const Frag *lds_frag;
   typedef short4v __attribute__((address_space(3))) *lds_tr;
-  typedef __attribute__((address_space(3))) gg_i32x4 *lds_w;
+  auto tr_frag = [&](uint32_t region, int blk, int ks) {                 // 16 columns `blk` of a k-strided region
+    const short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr)(region + (t_lo ^ (uint32_t)(blk << 5)) + (uint32_t)(ks * 8192)));
+    const short4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr)(region + (t_hi ^ (uint32_t)(blk << 5)) + (uint32_t)(ks * 8192)));
+    return frag_join<T>(lo, hi);
+  };
+  auto frag_a = [&](uint32_t region, int mi, int ks) -> Frag {
+    if constexpr (AKS) return tr_frag(region, wm * 4 + mi, ks);
+    else return *(lds_frag)(region + (fa_lane ^ (uint32_t)(ks << 6)) + (uint32_t)(mi * 2048));
+  };
+  auto frag_b = [&](uint32_t region, int nj, int ks) -> Frag {
+    if constexpr (BKS) return tr_frag(region, wn * 2 + nj, ks);
+    else return *(lds_frag)(region + (fb_lane ^ (uint32_t)(ks << 6)) + (uint32_t)(nj * 2048));
+  };
 
   // One segment: slices [s0, s1) of the tile (g, tm, tn).  part == nullptr: the segment is the whole k range and the
   // result goes to c; else the fp32 partial sums go to part (accumulator layout: 1 KB per wavefront instruction;
   // gg_split_reduce_kernel sums the pieces of a tile in k order).
   auto segment = [&](int g, int row_begin, int row_end, int tm, int tn, int s0, int s1, float *part) {
-  // NT / NN: output rows m0.. of the stacked rows; TN: output rows m0.. of group g's own [m_dim, n_dim] result
-  const int n0 = tn * 256, m0 = AKS ? tm * BM : row_begin + tm * BM;
-  const int a_rext = AKS ? (int)(p.m_dim - m0) : row_end - m0, b_rext = (int)(p.n_dim - n0);
-  const T *ag = reinterpret_cast<const T *>(p.a) + (AKS ? (int64_t)row_begin * p.lda + m0 : (int64_t)m0 * p.lda);
-  const T *bg = AKS ? reinterpret_cast<const T *>(p.b) + (int64_t)row_begin * p.ldb + n0
-                    : reinterpret_cast<const T *>(p.b) + (int64_t)g * p.b_group_stride + (BKS ? (int64_t)n0 : (int64_t)n0 * p.ldb);
-  // One descriptor per operand, cut at the last row of the group (of n): the hardware compares the lane offset plus
-  // the scalar offset with the length, so a row past the end reads as zero whichever 32-row block it is in.
-  // (k-strided operands: cut at the last k row, i.e. the group's last row for TN; in the other direction a tile that
-  // reaches past n or m reads what follows in the operand, into outputs that are not stored)
-  const gg_i32x4 rsa_ = AKS ? gg_rsrc(ag, (int64_t)(row_end - row_begin) * lda_b - (int64_t)m0 * (int)sizeof(T))
-                           : gg_rsrc(ag, (int64_t)(a_rext < 256 ? a_rext : 256) * lda_b);
-  const gg_i32x4 rsb_ = AKS ? gg_rsrc(bg, (int64_t)(row_end - row_begin) * ldb_b - (int64_t)n0 * (int)sizeof(T))
-                     : BKS ? gg_rsrc(bg, (int64_t)p.k_dim * ldb_b - (int64_t)n0 * (int)sizeof(T))
-                           : gg_rsrc(bg, (int64_t)(b_rext < 256 ? b_rext : 256) * ldb_b);
-  // The descriptors come out of v_readfirstlane, and a memory instruction may read such a scalar register five wait
-  // states later at the earliest.  The compiler keeps that distance for its own instructions, not for the loads issued
-  // from assembly below: without this the first of them went out with the previous contents of the length, now and then
-  // (a group of fewer than 64 rows then took rows of its neighbour into its weight gradient).
-  gg_i32x4 rsa = rsa_, rsb = rsb_;
-  asm volatile("s_nop 4" : "+s"(rsa), "+s"(rsb));
-  const int cnt = s1 - s0;                              // slices of this segment
-  floatx16 acc[4][4];
+    // NT / NN: output rows m0.. of the stacked rows; TN: output rows m0.. of group g's own [m_dim, n_dim] result
+    const int n0 = tn * 256, m0 = AKS ? tm * BM : row_begin + tm * BM;
+    const int a_rext = AKS ? (int)(p.m_dim - m0) : row_end - m0, b_rext = (int)(p.n_dim - n0);
+    const T *ag = reinterpret_cast<const T *>(p.a) + (AKS ? (int64_t)row_begin * p.lda + m0 : (int64_t)m0 * p.lda);
+    const T *bg = AKS ? reinterpret_cast<const T *>(p.b) + (int64_t)row_begin * p.ldb + n0
+                      : reinterpret_cast<const T *>(p.b) + (int64_t)g * p.b_group_stride + (BKS ? (int64_t)n0 : (int64_t)n0 * p.ldb);
+    // One descriptor per operand, cut at the last row of the group (of n): the hardware compares the lane offset plus
+    // the scalar offset with the length, so a row past the end reads as zero whichever block it is in.
+    // (k-strided operands: cut at the last k row, i.e. the group's last row for TN; in the other direction a tile that
+    // reaches past n or m reads what follows in the operand, into outputs that are not stored)
+    const gg_i32x4 rsa_ = AKS ? gg_rsrc(ag, (int64_t)(row_end - row_begin) * lda_b - (int64_t)m0 * (int)sizeof(T))
+                             : gg_rsrc(ag, (int64_t)(a_rext < 256 ? a_rext : 256) * lda_b);
+    const gg_i32x4 rsb_ = AKS ? gg_rsrc(bg, (int64_t)(row_end - row_begin) * ldb_b - (int64_t)n0 * (int)sizeof(T))
+                       : BKS ? gg_rsrc(bg, (int64_t)p.k_dim * ldb_b - (int64_t)n0 * (int)sizeof(T))
+                             : gg_rsrc(bg, (int64_t)(b_rext < 256 ? b_rext : 256) * ldb_b);
+    // The descriptors come out of v_readfirstlane, and a memory instruction may read such a scalar register five wait
+    // states later at the earliest.  The compiler keeps that distance for its own instructions, not for the copies issued
+    // from assembly: without this the first of them went out with the previous contents of the length, now and then
+    // (a group of fewer than 64 rows then took rows of its neighbour into its weight gradient).
+    gg_i32x4 rsa = rsa_, rsb = rsb_;
+    asm volatile("s_nop 4" : "+s"(rsa), "+s"(rsb));
+    const int cnt = s1 - s0;                                             // slices of this segment
+    // TN: what is added to (nothing to read if nothing is)
+    const uint32_t ldc_b = (uint32_t)p.ldc * (uint32_t)sizeof(T);
+    T *const cbase = reinterpret_cast<T *>(p.c) + (AKS ? (int64_t)g * p.c_group_stride : 0);
+    gg_i32x4 rsc = AKS ? gg_rsrc(cbase + (int64_t)m0 * p.ldc + n0,
+                                 p.accumulate ? (int64_t)(a_rext < 256 ? a_rext : 256) * ldc_b - (int64_t)n0 * (int)sizeof(T) : 0)
+                       : gg_i32x4{0, 0, 0, 0};
+    if constexpr (AKS) asm volatile("s_nop 4" : "+s"(rsc));
+    // What the copies of a slice read.  For the slices past the last one it is switched to nothing, or, for TN, to the old tile: rows
+    // of 512 bytes one behind the other over both stages, which are full of it when the last MFMAs end (a read of its own
+    // behind them took 5 us a tile).
+    uint32_t ca[2] = {va[0], va[1]}, cb[2] = {vb[0], vb[1]};
+    bool past = false;
+    auto past_the_last = [&] {
+      past = true;
+      if constexpr (AKS) {
+        rsa = rsb = rsc;
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+        for (int x = 0; x < 2; ++x)
+          ca[x] = cb[x] = (uint32_t)(2 * (2 * w + x) + (lane >> 5)) * ldc_b + (uint32_t)(((lane & 31) ^ (((4 * w + 2 * x) & 15) | (lane >> 5))) << 4);
+      } else {
+        rsa[2] = rsb[2] = 0;
+      }
+    };
+    // a last slice of k_dim % 64: a k-contiguous operand's chunks past it read as zero (a k-strided one is cut by its descriptor)
+    const int tail = AKS ? 0 : (int)(p.k_dim % 64);
+    auto the_last = [&] {
+      const int ch = (lane & 7) ^ (lane >> 4);                           // global chunk of the lane's copies: XOR 4 for the second
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+      for (int x = 0; x < 2; ++x)
+        if ((ch ^ (4 * x)) * 8 >= tail) {
+          ca[x] = 0x80000000u;                                           // past any descriptor's end
+          if constexpr (!BKS) cb[x] = 0x80000000u;
+        }
+    };
+    // before the copies of slice s (of this segment)
+    auto turn_to = [&](int s) {
+      if (s >= cnt) past_the_last();
+      else if (!AKS && tail != 0 && s0 + s == nsl - 1) the_last();
+    };
+    // half `h` of an operand's slice s (of this segment) into stage `stage`
+    auto copy_a = [&](int h, int s, uint32_t stage) {
+      const uint32_t at = stage + (uint32_t)h * REG;
+      const uint32_t off = AKS && past ? at / 512 * ldc_b : (uint32_t)(s0 + s) * kstep_a + (uint32_t)h * half_a;
 #pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
-
-  gg_i32x4 stg[2][16];
-  Frag fa[2][4];                                        // A fragments, k-contiguous form
-  short4v fat[2][4][2];                                 // k-strided form
-  Frag fbr[2][4];                                       // B fragments, k-contiguous form
-  short4v fbt[2][4][2];                                 // k-strided form: the two transpose reads of a fragment
-
-  auto gload = [&](int set, int idx, uint32_t ka, uint32_t kb) {   // idx 0..7: A, 8..15: B; ka, kb: byte offsets of the slice
-    if (idx < 8) asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen" : "=&v"(stg[set][idx]) : "v"(goff_a), "s"(rsa), "s"(ka + idx * rstep_a) : "memory");
-    else asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen" : "=&v"(stg[set][idx]) : "v"(goff_b), "s"(rsb), "s"(kb + (idx - 8) * rstep_b) : "memory");
-  };
-  // kc_w / kc_a / kc_b: the stage's lane addresses for the k-contiguous operands' writes and fragment reads, formed once
-  // per slice and kept in registers (left to the compiler they are re-added in front of every LDS instruction)
-  auto swrite = [&](int set, int idx, uint32_t stage, uint32_t kc_w) {  // stage: LDS byte address of the stage
-    if (idx < 8 && !AKS) *(lds_w)(kc_w + idx * 4096) = stg[set][idx];
-    else if (idx < 8) *(lds_w)(((stage + wr_a) ^ (uint32_t)((idx & 1) << 5)) + idx * 4096) = stg[set][idx];
-    else if (!BKS) *(lds_w)(kc_w + TILEB + (idx - 8) * 4096) = stg[set][idx];
-    else *(lds_w)(((stage + wr_b) ^ (uint32_t)(((idx - 8) & 1) << 5)) + (idx - 8) * 4096) = stg[set][idx];
-  };
-  // read r of a k step, in the order in which the MFMAs first need the data: B0 A0 B1 B2 B3 A1 A2 A3 (a k-strided
-  // B fragment is two transpose reads).  abase/bbase: lane addresses of the stage with the k step applied.
-  // a stage's lane addresses for k-contiguous fragment reads, and its base for the k-strided ones
-  struct Bases { uint32_t kc_a, kc_b, stage; };
-  auto bases_of = [&](uint32_t stage) { return Bases{stage + fa_lane, stage + fb_lane, stage}; };
-  auto fread = [&](int set, int r, int ks, const Bases &ba) {
-    if constexpr (!BKS) {
-      constexpr int isb[8] = {1, 0, 1, 1, 1, 0, 0, 0}, blk[8] = {0, 0, 1, 2, 3, 1, 2, 3};
-      if (!isb[r]) fa[set][blk[r]] = *(lds_frag)((ba.kc_a ^ (uint32_t)(ks << 5)) + blk[r] * 4096);
-      else fbr[set][blk[r]] = *(lds_frag)((ba.kc_b ^ (uint32_t)(ks << 5)) + blk[r] * 4096);
-    } else if constexpr (AKS) {
-      // B0 A0 B1 B2 B3 A1 A2 A3, two transpose reads each
-      constexpr int isb[8] = {1, 0, 1, 1, 1, 0, 0, 0}, blk[8] = {0, 0, 1, 2, 3, 1, 2, 3};
-      const int f = r >> 1, half = r & 1;
-      const uint32_t lane_addr = isb[f] ? (half ? tb_b : tb_a) : (half ? ta_b : ta_a);
-      const short4v x = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr)(((ba.stage + lane_addr) ^ (uint32_t)(blk[f] << 6)) + (uint32_t)(ks * 16 * BROWB)));
-      if (isb[f]) fbt[set][blk[f]][half] = x;
-      else fat[set][blk[f]][half] = x;
-    } else {
-      constexpr int kind[12] = {1, 2, 0, 1, 2, 1, 2, 1, 2, 0, 0, 0}, blk[12] = {0, 0, 0, 1, 1, 2, 2, 3, 3, 1, 2, 3};
-      if (kind[r] == 0) fa[set][blk[r]] = *(lds_frag)((ba.kc_a ^ (uint32_t)(ks << 5)) + blk[r] * 4096);
-      else if (kind[r] == 1)
-        fbt[set][blk[r]][0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr)(((ba.stage + tb_a) ^ (uint32_t)(blk[r] << 6)) + (uint32_t)(ks * 16 * BROWB)));
-      else
-        fbt[set][blk[r]][1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr)(((ba.stage + tb_b) ^ (uint32_t)(blk[r] << 6)) + (uint32_t)(ks * 16 * BROWB)));
-    }
-  };
-
-  // prologue: slice 0 into stage 0 (through set 0), slice 1 into set 1, slice 2 into set 0.  Loads of slices that
-  // do not exist repeat the last slice (their data is written to a stage nobody reads).
-  const int last = cnt > 0 ? cnt - 1 : 0;
-  auto kof = [&](int s) { return (uint32_t)(s0 + (s < last ? s : last)); };
+      for (int x = 0; x < 2; ++x) gg_copy_lds<T>(ca[x], rsa, off, cp_lds + at + (uint32_t)(x * 1024));
+    };
+    auto copy_b = [&](int h, int s, uint32_t stage) {
+      const uint32_t at = stage + OFF_B + (uint32_t)h * REG;
+      const uint32_t off = AKS && past ? at / 512 * ldc_b : (uint32_t)(s0 + s) * kstep_b + (uint32_t)h * half_b;
 #pragma unroll
-  for (int x = 0; x < 16; ++x) gload(0, x, kof(0) * kstep_a, kof(0) * kstep_b);
+      for (int x = 0; x < 2; ++x) gg_copy_lds<T>(cb[x], rsb, off, cp_lds + at + (uint32_t)(x * 1024));
+    };
+    GGAcc8 acc;
 #pragma unroll
-  for (int x = 0; x < 16; ++x) gload(1, x, kof(1) * kstep_a, kof(1) * kstep_b);
-  asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+    for (int i = 0; i < 32; ++i) acc[i >> 4][(i >> 3) & 1][(i >> 1) & 3][i & 1] = floatx4{0.f, 0.f, 0.f, 0.f};
+    Frag fa[2][4][2], fb[2][2][2];                                       // [half][block][step]
+    // 16 MFMAs; behind every second one a fragment read of what `rd(x)` says
+    auto mma_quarter = [&](int qm, int qn, auto rd) {
+      __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-  for (int x = 0; x < 16; ++x) swrite(0, x, lds0, lds0 + wr_kc);
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  // issue order of a staging set inside the loop: 0..7, 15, 8..14
-#pragma unroll
-  for (int x = 0; x < 8; ++x) gload(0, x, kof(2) * kstep_a, kof(2) * kstep_b);
-  gload(0, 15, kof(2) * kstep_a, kof(2) * kstep_b);
-#pragma unroll
-  for (int x = 8; x < 15; ++x) gload(0, x, kof(2) * kstep_a, kof(2) * kstep_b);
-  asm volatile("s_barrier" ::: "memory");
-  {
-    const Bases b0 = bases_of(lds0);
-#pragma unroll
-    for (int x = 0; x < NRD; ++x) fread(0, x, 0, b0);
-  }
-
-  // Slice s reads stage s % 2, writes slice s + 1 (staging set (s + 1) % 2, loaded two slices ago) into the other
-  // stage during its first half and then loads slice s + 3 into the same set.
-  int st = 0;
-  auto slice = [&](auto xc, auto lastc, int s) {
-    constexpr int X = decltype(xc)::value;              // s % 2
-    constexpr bool LAST = decltype(lastc)::value;       // the last slice of an odd count: nothing to prepare
-    uint32_t cur = lds0 + (uint32_t)(st * STAGEB), nxt = lds0 + (uint32_t)((st ^ 1) * STAGEB);
-    const uint32_t ka = kof(s + 3) * kstep_a, kb = kof(s + 3) * kstep_b;
-    asm volatile("" : "+s"(cur), "+s"(nxt));
-    Bases bc = bases_of(cur), bn = bases_of(nxt);
-    uint32_t wn_ = nxt + wr_kc;
-    if constexpr (!AKS) asm volatile("" : "+v"(bc.kc_a), "+v"(bn.kc_a), "+v"(wn_));
-    if constexpr (!BKS) asm volatile("" : "+v"(bc.kc_b), "+v"(bn.kc_b));
-    // (the k-strided operands' addresses are left to the compiler: pinned, they cost more additions than they save)
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int mi = 0; mi < 64; ++mi) {
-      const int ks = mi >> 4, i = (mi >> 2) & 3, j = mi & 3, q = mi & 15;
-      if constexpr (AKS) acc[i][j] = M::mma(frag_join<T>(fbt[ks & 1][j][0], fbt[ks & 1][j][1]), frag_join<T>(fat[ks & 1][i][0], fat[ks & 1][i][1]), acc[i][j]);
-      else if constexpr (BKS) acc[i][j] = M::mma(frag_join<T>(fbt[ks & 1][j][0], fbt[ks & 1][j][1]), fa[ks & 1][i], acc[i][j]);
-      else acc[i][j] = M::mma(fbr[ks & 1][j], fa[ks & 1][i], acc[i][j]);
-      // fragment reads of the next k step, spread over the quarter (the last quarter: behind the barrier, from the next stage)
-      if (ks < 3) {
-        if (NRD == 8) { if (q % 2 == 0) fread((ks + 1) & 1, q / 2, ks + 1, bc); }
-        else if (NRD == 12) { if (q % 4 != 3) fread((ks + 1) & 1, q - q / 4, ks + 1, bc); }
-        else fread((ks + 1) & 1, q, ks + 1, bc);
-      } else if (!LAST) {
-        if (mi == 50) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        if (NRD == 8) {
-          if (mi >= 50 && mi % 2 == 0) fread(0, (mi - 50) / 2, 0, bn);
-          if (mi == 63) fread(0, 7, 0, bn);
-        } else if (NRD == 12) {
-          if (mi >= 50 && mi < 62) fread(0, mi - 50, 0, bn);
-        } else {
-          if (mi >= 50) fread(0, mi - 50, 0, bn);
-          if (mi == 50) fread(0, 14, 0, bn);
-          if (mi == 51) fread(0, 15, 0, bn);
+      for (int x = 0; x < 16; ++x) {
+        const int ks = x >> 3, mi = (x >> 1) & 3, nj = x & 1;
+        acc[qm][qn][mi][nj] = M::mma16(fb[qn][nj][ks], fa[qm][mi][ks], acc[qm][qn][mi][nj]);   // C^T: lane column = output row
+        if (x & 1) {
+          __builtin_amdgcn_sched_barrier(0);
+          rd(x >> 1);
+          __builtin_amdgcn_sched_barrier(0);
         }
       }
-      if (!LAST && mi < 32 && mi % 2 == 1) {            // LDS writes of slice s + 1: the older of the two sets in flight
-        const int k = mi / 2;
-        if (k == 0) asm volatile("s_waitcnt vmcnt(24)" ::: "memory");
-        if (k == 8) asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
-        swrite(X ^ 1, k, nxt, wn_);
-      }
-      if (!LAST && mi >= 33 && mi <= 61 && mi % 2 == 1) gload(X ^ 1, (mi - 33) / 2, ka, kb);
-      if (!LAST && mi == 48) gload(X ^ 1, 15, ka, kb);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    st ^= 1;
-  };
-  using I0 = std::integral_constant<int, 0>;
-  using I1 = std::integral_constant<int, 1>;
-  int s = 0;
+      __builtin_amdgcn_s_setprio(0);
+    };
+    auto read_a = [&](int h, uint32_t region, int x0, int x1) {          // fragments x0..x1 of the half's eight
+#pragma unroll
+      for (int x = x0; x < x1; ++x) fa[h][x & 3][x >> 2] = frag_a(region, x & 3, x >> 2);
+    };
+    auto read_b = [&](int h, uint32_t region) {
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (int nj = 0; nj < 2; ++nj) fb[h][nj][ks] = frag_b(region, nj, ks);
+    };
+#define GG_W8_BARRIER()                       \
+    do {                                      \
+      __builtin_amdgcn_sched_barrier(0);      \
+      asm volatile("s_barrier" ::: "memory"); \
+      __builtin_amdgcn_sched_barrier(0);      \
+    } while (0)
+#define GG_W8_READS_DONE() asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory")
+#define GG_W8_WAIT_BARRIER(n)                                           \
+    do {                                                                \
+      __builtin_amdgcn_sched_barrier(0);                                \
+      asm volatile("s_waitcnt vmcnt(" #n ")\n\ts_barrier" ::: "memory"); \
+      __builtin_amdgcn_sched_barrier(0);                                \
+    } while (0)
+
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                    // (the zeroed rows' stores are not part of the counts below)
+    turn_to(0);
+    copy_a(0, 0, 0); copy_b(0, 0, 0); copy_b(1, 0, 0); copy_a(1, 0, 0);
+    turn_to(1);
+    copy_a(0, 1, STAGEB); copy_b(1, 1, STAGEB); copy_b(0, 1, STAGEB); copy_a(1, 1, STAGEB);
+    GG_W8_WAIT_BARRIER(8);
+    if (w >= 4) GG_W8_BARRIER();
+    read_a(0, lds0, 0, 8);
+    read_b(0, lds0 + OFF_B);
+    uint32_t cur = 0;
+    auto slice = [&](auto fc, int s) {
+      constexpr int F = decltype(fc)::value, G = F ^ 1;                  // the half of B that is multiplied first (s % 2), and the other
+      const uint32_t nxt = cur ^ STAGEB, sa = lds0 + cur, sb = sa + OFF_B, na = lds0 + nxt, nb = na + OFF_B;
+      turn_to(s + 2);
+      GG_W8_READS_DONE();
+      read_b(G, sb + G * REG);
+      GG_W8_BARRIER();
+      mma_quarter(0, F, [&](int x) { if (x < 3) read_a(1, sa + REG, x, x + 1); });
+      GG_W8_BARRIER();
+      GG_W8_READS_DONE();
+      read_a(1, sa + REG, 3, 6);
+      copy_a(0, s + 2, cur);
+      GG_W8_WAIT_BARRIER(8);
+      mma_quarter(0, G, [&](int x) { if (x < 2) read_a(1, sa + REG, 6 + x, 7 + x); });
+      GG_W8_BARRIER();
+      GG_W8_READS_DONE();
+      read_a(0, na, 0, 3);
+      copy_b(F, s + 2, cur);
+      GG_W8_WAIT_BARRIER(8);
+      mma_quarter(1, G, [&](int x) { if (x < 3) read_a(0, na, 3 + x, 4 + x); });
+      GG_W8_BARRIER();
+      GG_W8_READS_DONE();
+      read_b(G, nb + G * REG);
+      copy_b(G, s + 2, cur);
+      copy_a(1, s + 2, cur);
+      GG_W8_WAIT_BARRIER(8);
+      mma_quarter(1, F, [&](int x) { if (x < 2) read_a(0, na, 6 + x, 7 + x); });
+      GG_W8_BARRIER();
+      cur = nxt;
+    };
+    int s = 0;
 #pragma unroll 1
-  for (; s + 1 < cnt; s += 2) {
-    slice(I0{}, std::false_type{}, s);
-    slice(I1{}, std::false_type{}, s + 1);
-  }
-  // The loads of the last slices (unused data) still target the staging registers: wait for them, and keep the
-  // registers reserved until then (for the compiler a load whose result nobody reads frees its register at once).
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-#pragma unroll
-  for (int x = 0; x < 16; ++x) asm volatile("" ::"v"(stg[0][x]), "v"(stg[1][x]));
-  if (s < cnt) slice(I0{}, std::true_type{}, s);
-  __syncthreads();                                      // everyone is done with the stages: they stage the output below
+    for (; s + 1 < cnt; s += 2) {
+      slice(std::integral_constant<int, 0>{}, s);
+      slice(std::integral_constant<int, 1>{}, s + 1);
+    }
+    if (s < cnt) slice(std::integral_constant<int, 0>{}, s);
+    if (w < 4) GG_W8_BARRIER();
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                    // the last copies (zeros) have landed before the stages are used again
+    __syncthreads();
 
-  if constexpr (SK) {
-    // 16 bytes per lane and instruction: piece ((w * 16 + i * 4 + j) * 4 + vb) of the tile, 1 KB each
-    float *dst = part + ((size_t)w * 64 * 4 + 0) * 64 + (size_t)lane * 4;
+    if constexpr (SK) {
+      // 16 bytes per lane and instruction: piece w * 32 + block of the tile, 1 KB each
+      float *dst = part + (size_t)w * 32 * 256 + (size_t)lane * 4;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int vb = 0; vb < 4; ++vb) {
-          const floatx16 av = acc[i][j];
-          const floatx4 o = {av[4 * vb], av[4 * vb + 1], av[4 * vb + 2], av[4 * vb + 3]};
-          *reinterpret_cast<floatx4 *>(dst + (size_t)(((i * 4 + j) * 4 + vb) * 256)) = o;
-        }
-    __syncthreads();                                    // the next segment's copies reuse the stages
-    return;
-  }
-  gg_w4_store<T, AKS>(acc, smem, p, AKS ? reinterpret_cast<T *>(p.c) + (int64_t)g * p.c_group_stride : reinterpret_cast<T *>(p.c), m0, n0, a_rext, b_rext);
-    __syncthreads();                                    // the next segment's copies reuse the staging area
+      for (int i = 0; i < 32; ++i) *reinterpret_cast<floatx4 *>(dst + (size_t)i * 256) = acc[i >> 4][(i >> 3) & 1][(i >> 1) & 3][i & 1];
+      return;
+    }
+    if (AKS && p.accumulate) gg_w8_store<T, true>(acc, smem, p, cbase, m0, n0, a_rext, b_rext);
+    else gg_w8_store<T, false>(acc, smem, p, cbase, m0, n0, a_rext, b_rext);
   };
 
   if constexpr (AKS) {
@@ -491,7 +491,7 @@ __global__ void __launch_bounds__(256) grouped_gemm_w4_kernel(const GGParams p) 
     segment(g, rb, re, tm, tn, 0, nsl, nullptr);
   } else {
     // The last round of tiles, split along k.  The tiles (in the order of gg_tile_of) run in rounds of gridDim.x = the
-    // number of compute units; grouped_gemm_w4_kernel<.., false> in front of this kernel takes the full rounds, one
+    // number of compute units; grouped_gemm_w8_kernel<.., false> in front of this kernel takes the full rounds, one
     // workgroup per tile.  When the last round holds at most half as many tiles as there are workgroups, it is left to
     // this kernel: as many k pieces per tile as fit (workgroup w: tile w % rem, piece w / rem, so that neighbours work
     // on neighbouring tiles), summed afterwards in k order.  288 tiles on 256 compute units then take 1 1/8 tile
@@ -511,14 +511,17 @@ __global__ void __launch_bounds__(256) grouped_gemm_w4_kernel(const GGParams p) 
     segment(g, rb, re, tm, tn, pc * nsl / pieces, (pc + 1) * nsl / pieces, p.ws + (size_t)wg * (256 * 256));
   }
 }
+#undef GG_W8_BARRIER
+#undef GG_W8_WAIT_BARRIER
+#undef GG_W8_READS_DONE
 
 // Sums the k pieces of the tiles of a split last round, in k order (deterministic), and stores the tiles.
-// 16 workgroups per tile of that round: a wavefront takes one 32x32 block (w, i, j) of the accumulator layout,
-// reads its 4 KB of every piece (1 KB per instruction) and writes 4 columns per lane and register quad.
+// 16 workgroups per tile of that round: a wavefront takes four neighbouring 16x16 blocks (two by two) of the accumulator layout,
+// reads their 4 KB of every piece (1 KB per instruction) and writes 4 columns per lane and block.
 template <typename T>
 __global__ void __launch_bounds__(256) gg_split_reduce_kernel(const GGParams p, int sk_grid) {
   constexpr int BM = 256;
-  const int nsl = (int)(p.k_dim / 64);
+  const int nsl = (int)((p.k_dim + 63) / 64);
   const int base = gg_off(p, 0);
   int tiles_m = 0;
   for (int gi = 0; gi < p.groups; ++gi)
@@ -530,15 +533,15 @@ __global__ void __launch_bounds__(256) gg_split_reduce_kernel(const GGParams p, 
   if (pieces == 1) return;
   const int t = full * sk_grid + ts;
   const int tid = threadIdx.x, lane = tid & 63;
-  const int blk = (blockIdx.x % 16) * 4 + (tid >> 6);   // (w * 4 + i) * 4 + j
-  const int w = blk >> 4, i = (blk >> 2) & 3, j = blk & 3;
+  const int unit = (blockIdx.x % 16) * 4 + (tid >> 6);  // blocks 4 unit .. 4 unit + 3 of the tile's 256
+  const int w = unit >> 3, q = unit & 7;                // wavefront of the tile; (qm, qn, mi / 2)
   floatx4 acc[4];
 #pragma unroll
-  for (int vb = 0; vb < 4; ++vb) acc[vb] = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int x = 0; x < 4; ++x) acc[x] = floatx4{0.f, 0.f, 0.f, 0.f};
   for (int pc = 0; pc < pieces; ++pc) {
-    const float *src = p.ws + (size_t)(pc * rem + ts) * (256 * 256) + (size_t)blk * (4 * 256) + (size_t)lane * 4;
+    const float *src = p.ws + (size_t)(pc * rem + ts) * (256 * 256) + (size_t)unit * (4 * 256) + (size_t)lane * 4;
 #pragma unroll
-    for (int vb = 0; vb < 4; ++vb) acc[vb] += *reinterpret_cast<const floatx4 *>(src + vb * 256);
+    for (int x = 0; x < 4; ++x) acc[x] += *reinterpret_cast<const floatx4 *>(src + x * 256);
   }
   int tm, tn;
   gg_tile_of(t, tiles_m, p.tiles_n, tm, tn);
@@ -549,19 +552,16 @@ __global__ void __launch_bounds__(256) gg_split_reduce_kernel(const GGParams p, 
     if (tm < nt) break;
     tm -= nt;
   }
-  const int c = lane & 31, hh = lane >> 5;
-  const int m = (w >> 1) * 128 + 32 * i + c, n = (w & 1) * 128 + 32 * j + 4 * hh;    // + 8 vb
-  const int m0 = rb + tm * BM, n0 = tn * 256;
-  if (m0 + m >= re) return;
-  T *dst = reinterpret_cast<T *>(p.c) + (int64_t)(m0 + m) * p.ldc + n0 + n;
+  const int m = rb + tm * BM + 128 * (q >> 2) + 64 * (w >> 2) + 32 * (q & 1) + (lane & 15);         // + 16 (x / 2)
+  const int n = tn * 256 + 128 * ((q >> 1) & 1) + 32 * (w & 3) + 4 * (lane >> 4);                   // + 16 (x % 2)
   struct alignas(8) Q4 { T v[4]; };
 #pragma unroll
-  for (int vb = 0; vb < 4; ++vb)
-    if (n0 + n + 8 * vb < p.n_dim) {
+  for (int x = 0; x < 4; ++x)
+    if (m + 16 * (x >> 1) < re && n + 16 * (x & 1) < p.n_dim) {
       Q4 o;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) o.v[e] = static_cast<T>(acc[vb][e]);
-      *reinterpret_cast<Q4 *>(dst + 8 * vb) = o;
+      for (int e = 0; e < 4; ++e) o.v[e] = static_cast<T>(acc[x][e]);
+      *reinterpret_cast<Q4 *>(reinterpret_cast<T *>(p.c) + (int64_t)(m + 16 * (x >> 1)) * p.ldc + n + 16 * (x & 1)) = o;
     }
 }
 
@@ -579,18 +579,10 @@ __global__ void __launch_bounds__(256) gg_split_reduce_kernel(const GGParams p, 
 // (1.13 PFLOP/s, 27 bytes per cycle and compute unit out of L2); the start and end of a round of tiles cost 5 us.
 //
 // LDS: a k-contiguous operand as [rows][64 k] (128-byte rows, 16-byte chunk XOR (row / 2) % 8), a k-strided one as
-// [64 k][128 columns] (256-byte rows, chunk XOR 4 (k % 4) + (k / 4) % 4), as in grouped_gemm_w4_kernel; a wavefront
+// [64 k][128 columns] (256-byte rows, chunk XOR 4 (k % 4) + (k / 4) % 4), as in grouped_gemm_w8_kernel; a wavefront
 // copies 1 KB per instruction, so the XOR is applied to the global chunk that a lane fetches.  Buffer descriptors cut
 // the operands at the group's last row (k-strided: last k row), past which a copy writes zeros; columns past n read
 // what follows in the same operand and end in outputs that are not stored.
-template <typename T>
-__device__ __forceinline__ void gg_copy_lds(uint32_t lane_off, const gg_i32x4 &rsrc, uint32_t off, uint32_t lds_dst) {
-  asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
-               :
-               : "v"(lane_off), "s"(rsrc), "s"(off), "s"(lds_dst)
-               : "memory", "m0");
-}
-
 constexpr int64_t GG_MAX_LD = (1 << 22) - 8;       // row lengths (elements) of the tiled kernels: 256 rows stay inside 31-bit byte offsets
 
 // k pieces per tile: what fills the chip's places, each at least 8 slices long (a piece costs about as much traffic for
@@ -1018,15 +1010,15 @@ static int gg_compute_units(int &cus) {
 }
 
 template <typename T>
-static int launch_gg_w4_tn(GGParams p, hipStream_t st) {
+static int launch_gg_w8_tn(GGParams p, hipStream_t st) {
   p.tiles_m = (int)cdiv(p.m_dim, 256);
   p.tiles_n = (int)cdiv(p.n_dim, 256);
-  hipLaunchKernelGGL((grouped_gemm_w4_kernel<T, 2, false>), dim3((unsigned)(p.tiles_m * p.tiles_n), (unsigned)p.groups), dim3(256), 0, st, p);
+  hipLaunchKernelGGL((grouped_gemm_w8_kernel<T, 2, false>), dim3((unsigned)(p.tiles_m * p.tiles_n), (unsigned)p.groups), dim3(512), 0, st, p);
   return DH_OK;
 }
 
 template <typename T, bool BKS>
-static int launch_gg_w4(GGParams p, int64_t m_extent, void *workspace, size_t workspace_bytes, hipStream_t st) {
+static int launch_gg_w8(GGParams p, int64_t m_extent, void *workspace, size_t workspace_bytes, hipStream_t st) {
   p.tiles_n = (int)cdiv(p.n_dim, 256);
   p.tiles_m = (int)(cdiv(m_extent, 256) + p.groups);
   if (p.tiles_m <= 0 || p.tiles_n <= 0) return DH_OK;
@@ -1043,11 +1035,11 @@ static int launch_gg_w4(GGParams p, int64_t m_extent, void *workspace, size_t wo
   // known): the first kernel then leaves that round to the split kernel.  When nothing is split the two extra
   // launches cost a few microseconds; a split saves up to half a tile time (45 us and more).
   p.sk_grid = grid;
-  hipLaunchKernelGGL((grouped_gemm_w4_kernel<T, BKS ? 1 : 0, false>), dim3((unsigned)(p.tiles_m * p.tiles_n)), dim3(256), 0, st, p);
+  hipLaunchKernelGGL((grouped_gemm_w8_kernel<T, BKS ? 1 : 0, false>), dim3((unsigned)(p.tiles_m * p.tiles_n)), dim3(512), 0, st, p);
   if (grid > 0) {
     p.ws = reinterpret_cast<float *>(workspace);
     p.zero_tail = 0;                                    // done by the kernel above
-    hipLaunchKernelGGL((grouped_gemm_w4_kernel<T, BKS ? 1 : 0, true>), dim3((unsigned)grid), dim3(256), 0, st, p);
+    hipLaunchKernelGGL((grouped_gemm_w8_kernel<T, BKS ? 1 : 0, true>), dim3((unsigned)grid), dim3(512), 0, st, p);
     hipLaunchKernelGGL((gg_split_reduce_kernel<T>), dim3((unsigned)(16 * grid / 2)), dim3(256), 0, st, p, grid);   // at most grid / 2 tiles are split
   }
   return DH_OK;
@@ -1125,12 +1117,46 @@ static int dispatch_gg_t(const GGParams &p, int64_t m_extent, void *workspace, s
   }
 }
 
-// NT / NN: whether 256x256 tiles, one workgroup per compute unit, are the faster ones: enough of them, and a reduction long
-// enough to pay for their start and end (6036 rows of 4 groups, n = 7168 of 4096: 326 us against 380 us in 128x256 tiles;
-// 16384 rows of 8 groups, n = 4096 of 704: 53 against 37 us in 128x128 tiles).
-static bool gg_w4_pays(int64_t rows, int64_t n, int64_t k) {
-  const int64_t tiles = cdiv(rows, 256) * cdiv(n, 256);
-  return tiles >= 256 && (k >= 1536 || (k >= 640 && tiles >= 1500));
+// NT / NN: whether 256x256 tiles, one workgroup per compute unit, are the faster ones.  Both kernels run in rounds of equal
+// tiles, so the two times follow from the number of rounds (the last one of the 256x256 tiles is split along k where it is at
+// most half full) and of k slices; the constants (us) are a least-squares fit to 330 products of 1 to 64 groups, 192 to 4096 rows
+// a group, n and k from 512 to 8192, which the formulas meet to 13 and 11 %.  What is picked is 0.4 % from the better kernel on
+// average (by a count of tiles and a shortest k, as before: 1.8 %).  256x256 / smaller, us: 8 groups of 512 rows, n = 2816 of 2048
+// 50 / 63 (176 tiles); 8 x 1024, n = 5632 of 1024 96 / 113 (704 tiles), n = 3072 of 1024 73 / 62 (384: the second round half
+// empty), n = 1408 of 1024 33 / 35 (192).  Groups of fewer rows leave most of a tile empty.
+static bool gg_w8_pays(int64_t rows, int groups, int64_t n, int64_t k) {
+  const int64_t avg = rows / groups;
+  if (avg < 192) return false;
+  const double ns = (double)cdiv(k, 64);
+  const int64_t tiles = groups * cdiv(avg, 256) * cdiv(n, 256), rem = tiles % 256;
+  const double round = 14.3 + 1.357 * ns;
+  double big = 4.6 + (double)(tiles / 256) * round;
+  if (rem > 128) big += round;
+  else if (rem > 0) big += 26.3 + 1.357 * (ns > 1 ? ns / (double)(256 / rem < ns ? 256 / rem : ns) : 1.0);
+  double small;
+  if (k >= 1536) {
+    const int64_t t = groups * cdiv(avg, 128) * cdiv(n, 256);
+    small = 2 * t <= 256 ? 15.4 + 0.932 * ns * (double)t / 256 : (double)cdiv(t, 256) * (9.4 + 0.932 * ns);
+  } else {
+    const int64_t t = groups * cdiv(avg, 128) * cdiv(n, 128);
+    const double part = (double)t / 512 > 8 / ns ? (double)t / 512 : 8 / ns;
+    small = 2 * t <= 512 ? 6 + 1.205 * ns * part : (double)cdiv(t, 512) * 1.205 * ns;
+  }
+  return big < small;
+}
+
+// The same for TN, its constants from 60 products of 250 to 2048 rows a group (what is picked is 0.9 % from the better kernel on
+// average; below six slices, where uneven groups add some, 10 % is asked for); us, 256x256 / 128x128 tiles: 8 groups of 250 rows, 7168 x 4096 184 / 208, 5632 x 1024 44 / 41; of 1024 rows 443 / 575 and
+// 94 / 113, 3072 x 1024 59 / 62, of 512 rows 39 / 36.  Accumulating, which the smaller tiles do with 8-byte accesses, from two
+// thirds of a tile for every compute unit on: one group of 256 rows, 8192 x 3584 32 / 54, 1280 x 8192 15 / 24, but 8192 x 1024
+// (128 tiles) 15 / 16, of 4096 rows 84 / 74.
+static bool gg_w8_tn_pays(int64_t rows, int groups, int64_t m, int64_t n, int accumulate) {
+  const int64_t avg = rows / groups;
+  if (avg < 192) return false;
+  const double ns = (double)cdiv(avg, 64);
+  const int64_t tiles = groups * cdiv(m, 256) * cdiv(n, 256), small = groups * cdiv(m, 128) * cdiv(n, 128);
+  if (accumulate && tiles >= 160) return true;
+  return (double)cdiv(tiles, 256) * (8.5 + 1.38 * ns) * (avg < 384 ? 1.1 : 1.0) < 0.8 + (double)small / 512 * (3.5 + 1.11 * ns);
 }
 
 static int gg_common_checks(const void *a, const void *b, void *c, const int32_t *offs, int groups, int dtype) {
@@ -1158,10 +1184,10 @@ extern "C" int dh_grouped_gemm_nt(const void *a, const void *b, void *c, const i
   p.a = a; p.b = b; p.c = c; p.offs = offs; p.groups = groups;
   p.n_dim = n; p.k_dim = k; p.lda = k; p.ldb = k; p.ldc = n;
   p.b_group_stride = n * k; p.accumulate = 0; p.max_rows = (int)max_rows;
-  const bool big = gg_w4_pays(max_rows, n, k);
-  if (big && k % 64 == 0 && k <= (1ll << 21)) {
-    rc = dtype == DH_BF16 ? launch_gg_w4<bf16_t, false>(p, max_rows, workspace, workspace_bytes, (hipStream_t)stream)
-                          : launch_gg_w4<f16_t, false>(p, max_rows, workspace, workspace_bytes, (hipStream_t)stream);
+  const bool big = gg_w8_pays(max_rows, groups, n, k);
+  if (big && k <= (1ll << 21)) {
+    rc = dtype == DH_BF16 ? launch_gg_w8<bf16_t, false>(p, max_rows, workspace, workspace_bytes, (hipStream_t)stream)
+                          : launch_gg_w8<f16_t, false>(p, max_rows, workspace, workspace_bytes, (hipStream_t)stream);
   } else {
     rc = dtype == DH_BF16 ? dispatch_gg_t<bf16_t, 0>(p, max_rows, workspace, workspace_bytes, (hipStream_t)stream)
                           : dispatch_gg_t<f16_t, 0>(p, max_rows, workspace, workspace_bytes, (hipStream_t)stream);
@@ -1184,10 +1210,10 @@ extern "C" int dh_grouped_gemm_nn(const void *a, const void *b, void *c, const i
   p.a = a; p.b = b; p.c = c; p.offs = offs; p.groups = groups;
   p.n_dim = n; p.k_dim = k; p.lda = k; p.ldb = n; p.ldc = n;
   p.b_group_stride = n * k; p.accumulate = 0; p.max_rows = (int)max_rows;
-  const bool big = gg_w4_pays(max_rows, n, k);
-  if (big && k % 64 == 0 && k <= (1ll << 21) && k * n * (int64_t)dtype_size(dtype) < (1ll << 31)) {
-    rc = dtype == DH_BF16 ? launch_gg_w4<bf16_t, true>(p, max_rows, workspace, workspace_bytes, (hipStream_t)stream)
-                          : launch_gg_w4<f16_t, true>(p, max_rows, workspace, workspace_bytes, (hipStream_t)stream);
+  const bool big = gg_w8_pays(max_rows, groups, n, k);
+  if (big && k <= (1ll << 21) && k * n * (int64_t)dtype_size(dtype) < (1ll << 31)) {
+    rc = dtype == DH_BF16 ? launch_gg_w8<bf16_t, true>(p, max_rows, workspace, workspace_bytes, (hipStream_t)stream)
+                          : launch_gg_w8<f16_t, true>(p, max_rows, workspace, workspace_bytes, (hipStream_t)stream);
   } else {
     rc = dtype == DH_BF16 ? dispatch_gg_t<bf16_t, 1>(p, max_rows, workspace, workspace_bytes, (hipStream_t)stream)
                           : dispatch_gg_t<f16_t, 1>(p, max_rows, workspace, workspace_bytes, (hipStream_t)stream);
@@ -1210,12 +1236,9 @@ extern "C" int dh_grouped_gemm_tn_ws(const void *a, const void *b, void *c, cons
   p.a = a; p.b = b; p.c = c; p.offs = offs; p.groups = groups;
   p.m_dim = m; p.n_dim = n; p.lda = m; p.ldb = n; p.ldc = n;
   p.c_group_stride = m * n; p.accumulate = accumulate; p.max_rows = (int)max_rows;
-  // 256x256 tiles where the groups have many rows and there is much to do altogether (6000 rows of 8 groups, 7168 x 2048:
-  // 200 against 228 us in 128x128 tiles; 20000 rows of 16 groups, 2816 x 512: 77 against 70 us); their offsets have to fit
-  // the 32-bit buffer addressing
-  if (max_rows / groups >= 384 && cdiv(m, 256) * cdiv(n, 256) * max_rows >= 600000 &&
-      max_rows * (m > n ? m : n) * (int64_t)dtype_size(dtype) < (1ll << 31))
-    rc = dtype == DH_BF16 ? launch_gg_w4_tn<bf16_t>(p, (hipStream_t)stream) : launch_gg_w4_tn<f16_t>(p, (hipStream_t)stream);
+  // (the offsets of the 256x256 tiles have to fit the 32-bit buffer addressing)
+  if (gg_w8_tn_pays(max_rows, groups, m, n, accumulate) && max_rows * (m > n ? m : n) * (int64_t)dtype_size(dtype) < (1ll << 31))
+    rc = dtype == DH_BF16 ? launch_gg_w8_tn<bf16_t>(p, (hipStream_t)stream) : launch_gg_w8_tn<f16_t>(p, (hipStream_t)stream);
   else
     rc = dtype == DH_BF16 ? dispatch_gg_t<bf16_t, 2>(p, m, workspace, workspace_bytes, (hipStream_t)stream)
                           : dispatch_gg_t<f16_t, 2>(p, m, workspace, workspace_bytes, (hipStream_t)stream);

@@ -5,6 +5,8 @@
 //   A operand: 8 values A[row = c][k = 8h + j], j = 0..7
 //   B operand: 8 values B[k = 8h + j][col = c]
 //   D: 16 floats, D[row = 8*(v/4) + 4h + v%4][col = c], v = 0..15
+// The other shape, v_mfma_f32_16x16x32 (r = l % 16, g = l / 16): A operand A[row = r][k = 8g + j], B operand
+// B[k = 8g + j][col = r], D: 4 floats, D[row = 4g + v][col = r].
 // Because A and B index k the same way, any consistent relabelling of k between
 // the two operands leaves the product unchanged; the attention kernels use that
 // to feed an accumulator (whose rows are 8*(v/4)+4h+v%4) straight back in as an
@@ -35,11 +37,17 @@ template <> struct Mma<bf16_t> {
   static __device__ __forceinline__ floatx16 mma(Frag a, Frag b, floatx16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
   }
+  static __device__ __forceinline__ floatx4 mma16(Frag a, Frag b, floatx4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+  }
 };
 template <> struct Mma<f16_t> {
   using Frag = half8;
   static __device__ __forceinline__ floatx16 mma(Frag a, Frag b, floatx16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ floatx4 mma16(Frag a, Frag b, floatx4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
   }
 };
 

@@ -521,3 +521,48 @@ def test_grouped_gemm_tn_rows_longer_than_the_tiled_kernels_take(m, n, accumulat
     for e, (lo, hi) in enumerate(((0, 3), (3, 3), (3, 70))):
         ref = a[lo:hi].double().t() @ b[lo:hi].double() + (2.0 if accumulate else 0.0)
         assert_close(c[e], ref, torch.bfloat16, f"tn, group {e}", local=False)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n,k", [(3848, 1544),      # whole rounds; the last k slice holds 8 columns
+                                 (4104, 1600),      # 272 tiles: the last 16 in pieces of one and two slices
+                                 (4096, 1656)])     # one round exactly, 26 slices, the last one of 56 columns
+def test_grouped_gemm_256_tiles(dtype, n, k):
+    """NT and NN on the 256x256-tile kernel: rows, columns and slices that end inside a tile, an empty group.  Values past the end
+    of a row of ``a`` are the next row's: infinities there must not reach a result through a last slice."""
+    from dhellam_amd.operators import moe
+    rows = [2051, 0, 2045]
+    st = np.concatenate(([0], np.cumsum(rows)))
+    offs = torch.tensor(st, dtype=torch.int32).cuda()
+    a = randn((st[-1], k), dtype, 51, std=0.5).cuda()
+    b = randn((3, n, k), dtype, 52, std=0.5).cuda()
+    a[100, 0] = float("inf")
+    ref = torch.cat([a[st[g]:st[g + 1]].float() @ b[g].float().T for g in range(3)])
+    keep = torch.arange(st[-1], device="cuda") != 100
+    for name, fn, w in (("NT", moe.grouped_gemm_nt, b), ("NN", moe.grouped_gemm_nn, b.transpose(1, 2).contiguous())):
+        c = fn(a, w, offs)
+        assert_close(c[keep], ref[keep], dtype, name)
+        assert torch.equal(torch.isfinite(c[100]), torch.isfinite(ref[100])), f"{name}: the row that holds an infinity"
+        assert torch.equal(c[keep], fn(a, w, offs)[keep]), f"{name}: runs differ"
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_grouped_gemm_tn_256_tiles(dtype):
+    """Weight gradients on the 256x256-tile kernel: groups of none, one, two, three and five slices, the last one cut at the
+    group's rows, tiles that reach past m and n, rows behind the last group (not read), accumulation."""
+    from dhellam_amd.operators import moe
+    rows, m, n = [300, 0, 65, 1, 130], 2056, 2072
+    st = 3 + np.concatenate(([0], np.cumsum(rows)))
+    offs = torch.tensor(st, dtype=torch.int32).cuda()
+    a, b = randn((1500, m), dtype, 61, std=0.5).cuda(), randn((1500, n), dtype, 62, std=0.5).cuda()
+    a[st[-1] - 3:] = float("nan")
+    ref = torch.stack([a[lo - 3:hi - 3].float().T @ b[lo - 3:hi - 3].float() for lo, hi in zip(st[:-1], st[1:])])
+    w = moe.grouped_gemm_tn(a, b, offs)
+    assert_close(w, ref, dtype, "TN")
+    assert bool((w[1] == 0).all()), "empty group"
+    assert torch.equal(w, moe.grouped_gemm_tn(a, b, offs))
+    base = randn((5, m, n), dtype, 63).cuda()
+    acc = base.clone()
+    moe.grouped_gemm_tn(a, b, offs, out=acc, accumulate=True)
+    assert_close(acc, ref + base.float(), dtype, "TN accumulate")
+    assert torch.equal(acc[1], base[1]), "accumulating an empty group must leave the output as it was"
