@@ -145,7 +145,8 @@ def transpose_2d(src: torch.Tensor, out: Optional[torch.Tensor] = None, stream=N
 
 
 # The weight-gradient product dW[N, K] = dY[T, N]^T X[T, K] reads both operands along their strided dimension, the
-# GEMM library's slowest layout here.  Measured at T = 4096, bf16, accumulating (us; N, K = 7168, 8192 / 8192, 3584 /
+# GEMM library's slowest layout here.  Most of these products are the grouped kernel's (``wgrad`` of the host path says which
+# and why); what follows is about the rest, and about fp32 ``main_grad``.  Measured at T = 4096, bf16, accumulating (us; N, K = 7168, 8192 / 8192, 3584 /
 # 1280, 8192 / 8192, 1024):   as given 464 / 233 / 105 / 85;   dY^T row-major 380 / 190 / 87 / 72;   X^T row-major
 # (the layout ``dh_gemm`` refuses, ``dh_gemm_tt``) 383 / 188 / 95 / 70;   both row-major (the forward's layout)
 # 335 / 165 / 76 / 61.  One transposed operand is worth 15-20 % whichever it is, so the SMALLER one is transposed
@@ -200,7 +201,11 @@ def wgrad_operands(grad: torch.Tensor, data: torch.Tensor):
 
 def wgrad_gemm(grad: torch.Tensor, data: torch.Tensor, out: torch.Tensor, accumulate: bool, workspace=None,
                workspace_bytes: int = 0, stream=None) -> None:
-    """out [N, K] (+)= grad [T, N]^T @ data [T, K] through the GEMM library, in the layout ``wgrad_layout`` picks."""
+    """out [N, K] (+)= grad [T, N]^T @ data [T, K]: by the grouped kernel where that is the faster one, else through the
+    GEMM library in the layout ``wgrad_layout`` picks."""
+    if _host.wgrad(grad, data, out, accumulate, stream):
+        _lib.mark_written(out)
+        return
     layout = wgrad_layout(grad, data)
     if layout == "NN":
         # the kernel that produced ``grad`` may have left its transpose on it, stamped with the tensor's version

@@ -347,7 +347,8 @@ class DCFunc:
         # the projection has fewer inputs than outputs (``_Clib.wgrad_layout``): the kernel then writes it alongside
         f = input.shape[-1] // 2
         want_t = (f < config.hidden_size and config.tokens * f >= WGRAD_TRANSPOSE_MIN_ELEMS
-                  and wgrad_rows_ok(config.tokens, config.hidden_size))
+                  and wgrad_rows_ok(config.tokens, config.hidden_size)
+                  and not _host.wgrad_grouped(config.tokens, config.hidden_size, f))
         output, _ = swiglu(input, stream, False, with_transposed=want_t)
         return output
 
@@ -393,7 +394,8 @@ class DCFunc:
         # wide enough for that layout to pay (``_Clib.wgrad_layout``): the kernel then writes it alongside
         rows, n2 = swiglu_input.shape
         want_t = (config.hidden_size >= WGRAD_TRANSPOSE_GRAD_MIN_K and rows * n2 >= WGRAD_TRANSPOSE_MIN_ELEMS
-                  and config.hidden_size >= n2 and wgrad_rows_ok(rows, n2))     # (fewer inputs than outputs: the input is the operand transposed)
+                  and config.hidden_size >= n2 and wgrad_rows_ok(rows, n2)      # (fewer inputs than outputs: the input is the operand transposed)
+                  and not _host.wgrad_grouped(rows, n2, config.hidden_size))
         dgrad, _ = swiglu_back(grad_output, swiglu_input, None, stream, profiling=False, with_transposed=want_t)
         return dgrad
 

@@ -18,6 +18,7 @@
 
 #include <array>
 #include <map>
+#include <algorithm>
 #include <mutex>
 #include <optional>
 #include <tuple>
@@ -395,29 +396,68 @@ Tensor matmul(const Tensor &A, const Tensor &B, const OptTensor &out, bool trans
   return d;
 }
 
-// Data gradient grad [T, N] @ weight [N, K] as given.  Long reductions of few rows go to the grouped kernel with one group,
-// which splits them over the chip.  us, library / here, at T = 32, 128, 256, 512, 1000, of a sweep over N = 2048 to 12288,
-// K = 512 to 8192:
-//   N = 8192, K = 1024   14 / 15, 29 / 19, 29 / 23, 36 / 24, 46 / 32
-//   N = 8192, K = 3584   24 / 21, 57 / 24, 46 / 31, 58 / 44, 75 / 75
-//   N = 8192, K = 4096   27 / 22, 57 / 25, 46 / 32, 58 / 47, 76 / 79: with K above 3584 not past 512 rows (6144, 4096 at 1000: 58 / 64)
-//   N = 7168, K = 8192   31 / 28, 50 / 32, 74 / 46, 66 / 71, 107 / 115: wide results only up to 256 rows
-//   N = 5120, K = 2048   12 / 13, 21 / 19, 24 / 21, 28 / 26, 40 / 37;  N = 4096, K = 2048 11 / 12, 18 / 17, 21 / 21, 23 / 25, 33 / 34:
-//   the line in N.  (K = 512 loses 2 us at 128 rows.)
+// 16-bit matrices that the grouped kernel takes with one group: rows of whole 16-byte pieces, aligned.
+bool grouped_ok(const Tensor &x, at::ScalarType type) {
+  return x.is_cuda() && x.dim() == 2 && x.is_contiguous() && x.scalar_type() == type && (type == at::kBFloat16 || type == at::kHalf) &&
+         x.size(1) % 8 == 0 && (uintptr_t)x.data_ptr() % 16 == 0;
+}
+
+// Data gradient grad [T, N] @ weight [N, K] as given: whether the grouped kernel with one group is the faster one.  It splits
+// long reductions of few rows over the chip and needs no whole slices; the library's kernels for this layout are at their
+// best where N is short.  us, library / here, of a sweep over N = 1000 to 32000, K = 512 to 8192, T = 64 to 4096:
+//   N that is no multiple of 64: 1000 x 1024 at T = 1904 15 / 11, 4000 x 1024 at 1000 27 / 23, 16032 x 4096 at 512 113 / 71
+//   N >= 16000: 32000 x 1024 at 200, 1000, 4096 101 / 33, 175 / 69, 323 / 215; x 4096 209 / 76, 313 / 211, 770 / 738
+//   5120 <= N < 16000, by K T: 8192 x 1024 at 64, 1000, 1904 36 / 16, 44 / 31, 58 / 43, at 3000 65 / 64; x 2048 at 1000 58 / 45,
+//     at 1904 71 / 73, at 3000 94 / 112; x 3584 at 768 84 / 57, at 1000 70 / 70; 7168 x 8192 at 200 50 / 41, at 512 64 / 68;
+//     and again where 256x256 tiles fill the chip: 7168 x 8192 at 1904, 4096 173 / 164, 346 / 330, 8192 x 3584 at 4096 184 / 180
+//   below: the library (3072 x 1024 at 1000 18 / 21, 1280 x 8192 at 1904 38 / 41)
+bool dgrad_grouped(int64_t t, int64_t n, int64_t k) {
+  if (t <= 0 || n < 1000) return false;
+  if (n % 64 != 0 || n >= 16000) return true;
+  return n >= 5120 && (t * k <= 2800000 || t * k >= 14000000);
+}
+
+// Weight gradient dY [T, N]^T X [T, K]: the same question.  The library reads both operands along their strided dimension
+// here, its slowest layout (one of them materialised transposed first gains 10 % and costs most of that); the grouped kernel's
+// LDS transpose reads cost it nothing, and it adds to what is there without a read of its own.  us accumulating, library (the
+// better of its two layouts) / here, N, K at T = 200, 1000, 1904, 4096: 7168, 8192 76 / 62, 154 / 125, 244 / 197, 411 / 378;
+// 8192, 3584 40 / 32, 79 / 61, 124 / 97, 205 / 190; 32000, 2048 at 512, 1064, 4096 93 / 85, 164 / 135, 442 / 432; 1280, 8192 (160
+// tiles) 18 / 15, 40 / 30, 54 / 45, but 80 / 84: few tiles of many whole slices stay with the library, as does 8192, 1024 (128 tiles)
+// 14 / 16, 31 / 29, 44 / 44, 69 / 83.  Small weights of few rows: 3072, 1024 at 64, 256, 368 10.4 / 7.6, 10.5 / 9.4, 12.4 / 10.5, at 512
+// 12.2 / 12.4.
+bool wgrad_grouped(int64_t t, int64_t n, int64_t k) {
+  const int64_t tiles = (n + 255) / 256 * ((k + 255) / 256);
+  if (t >= 192 && tiles >= 160) return !(tiles < 224 && t % 64 == 0 && t >= 2048) && 2 * t * std::max(n, k) < (int64_t)1 << 31;
+  return t > 0 && t <= 384 && n * k <= 3200000;
+}
+
+// out [N, K] (+)= grad [T, N]^T @ data [T, K] by the grouped kernel; false, and nothing done, where it is not the faster one or does
+// not take the operands.
+bool wgrad(const Tensor &grad, const Tensor &data, const Tensor &out, bool accumulate, const OptStream &stream) {
+  const auto type = grad.scalar_type();
+  if (!grouped_ok(grad, type) || !grouped_ok(data, type) || !grouped_ok(out, type)) return false;
+  const int64_t t = grad.size(0), n = grad.size(1), k = data.size(1);
+  if (data.size(0) != t || out.size(0) != n || out.size(1) != k || !wgrad_grouped(t, n, k)) return false;
+  On on(stream);
+  const Held ws = scratch(kGrouped, (int64_t)dh_grouped_gemm_workspace_bytes(), grad, on.get());
+  launch([&] {
+    return dh_grouped_gemm_tn_ws(grad.data_ptr(), data.data_ptr(), out.data_ptr(), nullptr, 1, t, n, k, accumulate, dt(grad),
+                                 ws.data_ptr(), (size_t)ws.numel(), on.get());
+  }, ws.own);
+  return true;
+}
+
 Tensor dgrad(const Tensor &grad, const Tensor &weight, const OptTensor &out, const OptStream &stream) {
-  const int64_t t = grad.size(0), n = weight.size(0), k = weight.size(1);
-  const auto ok = [](const Tensor &x) { return x.is_contiguous() && (uintptr_t)x.data_ptr() % 16 == 0; };
-  if (grad.dim() == 2 && weight.dim() == 2 && grad.size(1) == n && n >= 5120 && t > 0 && (t <= 256 || (k <= 4096 && t <= 512) || (k <= 3584 && t <= 1024)) &&
-      n % 64 == 0 && k % 8 == 0 && weight.is_cuda() && grad.is_cuda() &&
-      (grad.scalar_type() == at::kBFloat16 || grad.scalar_type() == at::kHalf) && weight.scalar_type() == grad.scalar_type() &&
-      ok(grad) && ok(weight) &&
-      (!out.has_value() || (out->is_cuda() && ok(*out) && out->scalar_type() == grad.scalar_type() && out->sizes() == at::IntArrayRef({t, k})))) {
+  const auto type = grad.scalar_type();
+  if (grouped_ok(grad, type) && grouped_ok(weight, type) && grad.size(1) == weight.size(0) &&
+      dgrad_grouped(grad.size(0), weight.size(0), weight.size(1)) &&
+      (!out.has_value() || (grouped_ok(*out, type) && out->sizes() == at::IntArrayRef({grad.size(0), weight.size(1)})))) {
+    const int64_t t = grad.size(0), n = weight.size(0), k = weight.size(1);
     On on(stream);
     Tensor d = out.has_value() ? *out : at::empty({t, k}, grad.options());
     const Held ws = scratch(kGrouped, (int64_t)dh_grouped_gemm_workspace_bytes(), grad, on.get());
-    const int type = dt(grad);
     launch([&] {
-      return dh_grouped_gemm_nn(grad.data_ptr(), weight.data_ptr(), d.data_ptr(), nullptr, 1, t, k, n, type, ws.data_ptr(),
+      return dh_grouped_gemm_nn(grad.data_ptr(), weight.data_ptr(), d.data_ptr(), nullptr, 1, t, k, n, dt(grad), ws.data_ptr(),
                                 (size_t)ws.numel(), on.get());
     }, ws.own);
     return d;
@@ -956,6 +996,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("expert_ffn_bwd", &expert_ffn_bwd);
   m.def("grouped_gemm", &grouped_gemm);
   m.def("grouped_gemm_tn", &grouped_gemm_tn);
+  m.def("wgrad", &wgrad);
+  m.def("wgrad_grouped", &wgrad_grouped);
   m.def("embedding_fwd", &embedding_fwd);
   m.def("embedding_bwd", &embedding_bwd);
   m.def("cross_entropy_fwd", &cross_entropy_fwd);
