@@ -47,6 +47,7 @@ struct AttnBwdParams {
   int q_shift, k_shift;      // sequence bounds are cu >> shift (the halves of a context-parallel chunk)
   int lse_pitch;             // rows of a head in lse
   int dq_accumulate;         // dq += this call's gradient (read, add in fp32, round once) instead of dq =
+  int delta_tail;            // delta is an output: its rows past a sequence's end, up to max_sq, are zeros
   // dS = P * (dP - delta) kept for the dQ product (head dim 128, 16 bits, when the workspace allows): 2 KB blocks of
   // 32 keys x 32 query rows, block (b, h, query tile, key block); inside a block the 16-byte piece (s, hh, key)
   // holds the query rows 16 s + 8 u + 4 hh + x of that key (u = 0, 1; x = 0..3): what a lane of the dK/dV kernel
@@ -55,29 +56,39 @@ struct AttnBwdParams {
   int ds_nqt, ds_nkb;        // query tiles and key blocks (of 32) per (batch, head)
 };
 
+// Zeros in the rows of delta past the end of the sequence, in tile `tile` of BM rows of the grid laid out for max_sq.  A
+// filled-in tensor before the kernels cost a launch of 2 us.
+template <int BM>
+__device__ __forceinline__ void delta_tail_zero(const AttnBwdParams &p, int b, int h, int sq, int tile) {
+  const int row = tile * BM + (int)threadIdx.x;
+  if (p.delta_tail && (int)threadIdx.x < BM && row >= sq && row < p.max_sq) p.delta[((int64_t)b * p.hq + h) * p.max_sq + row] = 0.f;
+}
+
 // ---- delta = rowsum(dO * O) ---------------------------------------------------------------
 template <typename T>
 __global__ void __launch_bounds__(256)
 attn_delta_kernel(const T *__restrict__ dout, const T *__restrict__ out, float *__restrict__ delta,
                   const float *__restrict__ lse, float *__restrict__ ld2, int64_t ld2_plane, int ld2_pitch,
                   const int32_t *__restrict__ cu_q, int q_shift, int lse_pitch, int max_sq, int hq, int d, int lanes_per,
-                  int64_t do_stride, int64_t o_stride) {
+                  int64_t do_stride, int64_t o_stride, int tail) {
   constexpr int N = Vec<T>::N;
   const int b = blockIdx.y;
   const int q0 = cu_q[b] >> q_shift, sq = (cu_q[b + 1] >> q_shift) - q0;
   const int per_block = 256 / lanes_per;
   const int sub = threadIdx.x / lanes_per, ln = threadIdx.x % lanes_per;
   const int nvec = d / N;
-  const int rows = ld2 ? ((sq + 31) / 32) * 32 : sq;   // the side-by-side planes are written in whole 32-row tiles
+  const int rows_ld2 = ld2 ? ((sq + 31) / 32) * 32 : sq;   // the side-by-side planes are written in whole 32-row tiles
+  const int rows = tail && max_sq > rows_ld2 ? max_sq : rows_ld2;
   for (int64_t item = (int64_t)blockIdx.x * per_block + sub; item < (int64_t)rows * hq;
        item += (int64_t)gridDim.x * per_block) {
     const int i = (int)(item / hq), h = (int)(item % hq);
     if (i >= sq) {           // padding rows of the last tile: zeros, so that masked scores stay finite
-      if (ln == 0) {
+      if (ln == 0 && i < rows_ld2) {
         const int64_t a2 = ((int64_t)b * hq + h) * ld2_pitch + i;
         ld2[a2] = 0.f;
         ld2[ld2_plane + a2] = 0.f;
       }
+      if (tail && ln == 0 && i < max_sq) delta[((int64_t)b * hq + h) * max_sq + i] = 0.f;
       continue;
     }
     float s = 0.f;
@@ -168,7 +179,10 @@ __global__ void __launch_bounds__(512) attn_bwd_dq_d128_kernel(const AttnBwdPara
   const int k_stride = (int)p.k_stride, v_stride = (int)p.v_stride;
   const float scale_log2 = p.scale_log2;
   int qt[2], nq;
+  const int tiles = (p.max_sq + BM - 1) / BM;
+  delta_tail_zero<BM>(p, b, h, sq, px);
   if (causal) {
+    if (tiles - 1 - px != px) delta_tail_zero<BM>(p, b, h, sq, tiles - 1 - px);
     const int pair = px;
     if (2 * pair >= nqt) return;
     qt[0] = nqt - 1 - pair; qt[1] = pair;
@@ -1081,7 +1095,7 @@ template <typename T>
 static int launch_delta(const void *dout, const void *out, float *delta, const float *lse, float *ld2, int64_t ld2_plane,
                         int ld2_pitch, const int32_t *cu_q, int q_shift, int lse_pitch, int batch, int max_sq, int hq, int d,
                         int64_t do_stride, int64_t o_stride,
-                        hipStream_t st) {
+                        int tail, hipStream_t st) {
   const int nvec = d / Vec<T>::N;
   int lanes_per = 1;
   while (lanes_per < nvec && lanes_per < 64) lanes_per <<= 1;
@@ -1091,7 +1105,7 @@ static int launch_delta(const void *dout, const void *out, float *delta, const f
   if (blocks < 1) blocks = 1;
   hipLaunchKernelGGL((attn_delta_kernel<T>), dim3((unsigned)blocks, (unsigned)batch), dim3(256), 0, st,
                      (const T *)dout, (const T *)out, delta, lse, ld2, ld2_plane, ld2_pitch, cu_q, q_shift, lse_pitch, max_sq, hq, d, lanes_per,
-                     do_stride, o_stride);
+                     do_stride, o_stride, tail);
   return DH_OK;
 }
 
@@ -1127,19 +1141,70 @@ static bool bwd_short(int max_sq, int max_sk, int causal, int64_t total_q, int h
   return causal ? total_q * hq <= 16384 : max_sq <= 48 && max_sk <= 48;
 }
 
+// Key splits of a GQA group over workgroups.  The hand-ordered causal dK/dV kernel takes two key tiles a workgroup.
+static int bwd_hsplit(int max_sk, int batch, int hq, int hk, bool paired) {
+  return pick_hsplit(paired ? (max_sk + 1) / 2 : max_sk, batch, hq, hk, DKV_ROWS);
+}
+
+// Whether dK/dV and dQ go into one launch of the tile kernels, behind the delta kernel (2.5 us).  Either pass alone leaves
+// compute units idle: all of those that it has no workgroup for, the last round's, and with causal rows those that got short
+// tiles (one workgroup a compute unit in all forms: registers).  Together the long workgroups (dK/dV: 1.3 times a dQ one and
+// once per query head of its group) start first and the others fill in.  `a` and `b`: workgroups of dQ and dK/dV with work.
+// Backward, us, two launches / one, head dims 64 | 192 (96 and 256 behave as they do):
+//   all in one round: 12 heads x 28 12.1 / 9.6 | 19.6 / 13.7, 16 x 300 18.7 / 14.1 | 41.7 / 26.9, causal or not;
+//   causal, a round and a half: 8 x 1500 40.0 / 27.0 | 125 / 72, 32 x 300 19.1 / 17.0 | 43 / 35; two full rounds of short rows
+//     16 x 16 x 60 16.8 / 18.6 | 29.5 / 32.3, of long ones 8 x 2048 49 / 38 | 162 / 106, 16 x 1024 31.4 / 30.3 | 93 / 85; dK/dV in one
+//     round, dQ in several: 32 query / 8 kv heads x 1500 105 / 79 | 342 / 243, but 16 x 1500 (dK/dV in two) 46.1 / 47.8 | 130 / 132;
+//   otherwise by the model: 16 x 1500 not causal (1.28 predicted) 77 / 66 | 255 / 201, 32 / 8 x 600 + 300 (1.38) 54 / 42 | 167 / 116, 32
+//     x 300 (1.15, not taken) 19.8 / 18.5 | 44 / 42, 16 x 1024 (1.0) 32.3 / 34.9 | 95 / 98.
+// Head dim 128 has the hand-ordered kernels to compare with, whose workgroups start and end later but run 1.5 times as fast:
+//   one round: 12 x 28 16.5 / 11.0, 16 x 300 29 / 20 causal, 26 / 21 not, 8 x 1024 51 / 39, not causal 41.7 / 41.9;
+//   causal, up to a round and a half: 8 x 1500 66 / 53; two: 32 x 512 45.5 / 42.2, 16 x 1024 55 / 61, 16 x 16 x 60 23.2 / 22.8.
+// A group split eight ways from 512 rows on (8 query / 1 kv head x 1024: 57.8 / 46.1) and rectangular calls that are not
+// causal stay with the hand-ordered kernels: callers size the workspace there to choose between their two forms of dQ.
+static bool bwd_both_pays(int batch, int max_sq, int max_sk, int64_t total_q, int64_t total_k, int hq, int hk, int d, int causal) {
+  if (max_sq <= 0 || max_sk <= 0) return false;
+  auto tiles = [&](int longest, int64_t total) {
+    const int64_t grid = cdiv(longest, 64) * batch, real = total / 64 + batch;
+    return grid < real ? grid : real;
+  };
+  const int hs = bwd_hsplit(max_sk, batch, hq, hk, false);
+  const int64_t a = tiles(max_sq, total_q) * hq, b = tiles(max_sk, total_k) * hk * hs;
+  if (d == 128) {
+    if (!causal) return a + b <= 256 && max_sq < 1024 && max_sq == max_sk;
+    if (max_sq >= 512 && hs >= 8) return false;
+    return a + b <= 384 || (a + b <= 512 && max_sq >= 256 && max_sq < 1024);
+  }
+  if (a + b <= (causal ? 384 : 256)) return true;
+  if (causal && max_sq >= 1024) return b <= 256;
+  // rounds of 256, in units of a dQ workgroup's time: one pass after the other, and both with the dK/dV workgroups first
+  const double rho = 1.3 * (hq / hk / hs), apart = (double)cdiv(a, 256) + (double)cdiv(b, 256) * rho;
+  const int64_t full = b / 256, more = b % 256;
+  auto room = [&](double t) {        // dQ workgroups that end by t
+    const double x = t - (double)full * rho, y = x - rho;
+    return (x > 0 ? (int64_t)x * (256 - more) : 0) + (y > 0 ? (int64_t)y * more : 0);
+  };
+  const double t = apart / 1.2;
+  return t >= (double)cdiv(b, 256) * rho && room(t) >= a;
+}
+
 // What one 16-bit call runs.
 struct AttnBwdRoute {
   bool keep_ds;      // dK/dV keeps dS and dQ is one product over it; else dQ recomputes, first, and forms delta
   bool hand_dkv, hand_dq;      // head dim 128's hand-ordered kernels
   bool big_dq;       // 128-row query tiles in dQ
+  bool both;         // dK/dV and dQ in one launch of the tile kernels, behind the delta kernel
 };
-static AttnBwdRoute attn_bwd_route(int batch, int max_sq, int max_sk, int64_t total_q, int hq, int d, int causal, bool room_for_ds) {
-  const bool short_rows = d == 128 && bwd_short(max_sq, max_sk, causal, total_q, hq), big = dq_big_grid(batch, max_sq, hq, causal);
+static AttnBwdRoute attn_bwd_route(int batch, int max_sq, int max_sk, int64_t total_q, int64_t total_k, int hq, int hk, int d,
+                                   int causal, bool room_for_ds) {
+  const bool both = bwd_both_pays(batch, max_sq, max_sk, total_q, total_k, hq, hk, d, causal);
+  const bool short_rows = d == 128 && (both || bwd_short(max_sq, max_sk, causal, total_q, hq)), big = dq_big_grid(batch, max_sq, hq, causal);
   AttnBwdRoute r;
   r.keep_ds = room_for_ds && max_sk > 0 && !short_rows;
   r.hand_dkv = d == 128 && !short_rows;
   r.hand_dq = r.hand_dkv && (!causal || !big || attn_causal_fills(max_sq, hq, batch, total_q));
   r.big_dq = r.hand_dq ? big : d <= 128 && attn_wgs(max_sq, 128, hq, batch, 0) >= 2 * 256;
+  r.both = both && !r.big_dq;
   return r;
 }
 
@@ -1148,7 +1213,10 @@ template <typename T, int D>
 static int bwd_passes(const AttnBwdParams &p, const AttnBwdRoute &r, int batch, int max_sq, int max_sk, hipStream_t st) {
   int rc = DH_OK;
   // recomputing dQ kernels form delta and run first
-  if (max_sq > 0 && !r.keep_ds) {
+  if (r.both) {
+    if constexpr (D < 128) rc = launch_both_tile<T, D, 2, 4, 2, 4, 2>(p, batch, max_sk, st);
+    else rc = launch_both_tile<T, D, 2, 2, 2, 2, 1>(p, batch, max_sk, st);
+  } else if (max_sq > 0 && !r.keep_ds) {
     if constexpr (D == 128) {
       if (r.hand_dq) rc = r.big_dq ? launch_dq_d128<T, 4, 2, 32>(p, batch, st) : launch_dq_d128<T, 2, 4, 32>(p, batch, st);
       else rc = r.big_dq ? launch_dq_tile<T, D, 4, 2, 2>(p, batch, st) : launch_dq_tile<T, D, 2, 4, 2>(p, batch, st);
@@ -1158,7 +1226,7 @@ static int bwd_passes(const AttnBwdParams &p, const AttnBwdRoute &r, int batch, 
       rc = launch_dq_tile<T, D, 2, 2, 1>(p, batch, st);
     }
   }
-  if (rc == DH_OK && max_sk > 0) {
+  if (rc == DH_OK && max_sk > 0 && !r.both) {
     if constexpr (D == 128) rc = r.hand_dkv ? launch_dkv_d128<T>(p, batch, max_sk, st) : launch_dkv_tile<T, D, 2, 2, 1>(p, batch, max_sk, st);
     else if constexpr (D < 128) rc = launch_dkv_tile<T, D, 2, 4, 2>(p, batch, max_sk, st);
     else rc = launch_dkv_tile<T, D, 2, 2, 1>(p, batch, max_sk, st);
@@ -1223,12 +1291,17 @@ extern "C" size_t dh_attn_bwd_workspace_bytes(int64_t total_q, int64_t total_k, 
          align256(ds_bytes(batch, max_seqlen_q, total_k, hq, d, dtype, 1));
 }
 
+extern "C" int dh_attn_bwd_one_launch(int batch, int max_seqlen_q, int max_seqlen_k, int64_t total_q, int64_t total_k, int hq, int hk,
+                                      int d, int causal) {
+  return dh::attn_bwd_route(batch, max_seqlen_q, max_seqlen_k, total_q, total_k, hq, hk, d, causal, false).both ? 1 : 0;
+}
+
 extern "C" int dh_attn_bwd_path(int batch, int max_seqlen_q, int max_seqlen_k, int64_t total_q, int64_t total_k, int hq, int hk, int d,
                                 int causal, size_t workspace_bytes) {
   using namespace dh;
   const size_t base = bwd_base_bytes(total_k, batch, max_seqlen_q, hq, hk, d, DH_BF16);
   const size_t dsb = ds_bytes(batch, max_seqlen_q, total_k, hq, d, DH_BF16, causal);
-  const AttnBwdRoute r = attn_bwd_route(batch, max_seqlen_q, max_seqlen_k, total_q, hq, d, causal,
+  const AttnBwdRoute r = attn_bwd_route(batch, max_seqlen_q, max_seqlen_k, total_q, total_k, hq, hk, d, causal,
                                         dsb > 0 && base + align256(dsb) <= workspace_bytes);
   return (r.hand_dkv ? 1 : 0) | (r.keep_ds ? 2 : (r.hand_dq ? 4 : 0) | (r.big_dq ? 8 : 0));
 }
@@ -1276,13 +1349,13 @@ static int attn_bwd_entry(const void *dout, const void *q, const void *k, const 
   // process-wide limit); they take the tail of the workspace
   size_t dsb = ds_bytes(batch, max_seqlen_q, total_k, hq, d, dtype, causal);
   if (dsb > 0 && base_bytes + align256(dsb) > workspace_bytes) dsb = 0;
-  const AttnBwdRoute route = attn_bwd_route(batch, max_seqlen_q, max_seqlen_k, total_q, hq, d, causal, dsb > 0);
+  const AttnBwdRoute route = attn_bwd_route(batch, max_seqlen_q, max_seqlen_k, total_q, total_k, hq, hk, d, causal, dsb > 0);
   uint8_t *ds_ws = (uint8_t *)(((uintptr_t)workspace + 255) & ~(uintptr_t)255) + (base_bytes - 256);
-  const bool delta_in_dq = dtype != DH_F32 && !route.keep_ds;
+  const bool delta_in_dq = dtype != DH_F32 && !route.keep_ds && !route.both;
   if (max_seqlen_q > 0 && !delta_in_dq) {
     DH_DISPATCH_DTYPE(dtype, {
       launch_delta<T>(dout, out, delta, lse, ld2, (int64_t)(plane2 / sizeof(float)), ld2_pitch, cu_seqlens_q, q_shift, lse_pitch,
-                      batch, max_seqlen_q, hq, d, do_stride, o_stride, st);
+                      batch, max_seqlen_q, hq, d, do_stride, o_stride, delta_out ? 1 : 0, st);
     });
   }
   if (dtype == DH_F32) {
@@ -1313,10 +1386,11 @@ static int attn_bwd_entry(const void *dout, const void *q, const void *k, const 
   p.causal = causal;
   p.q_shift = q_shift; p.k_shift = k_shift; p.lse_pitch = lse_pitch;
   p.dq_accumulate = dq_accumulate ? 1 : 0;
+  p.delta_tail = delta_out ? 1 : 0;
   p.ds = route.keep_ds ? (void *)ds_ws : nullptr;
   p.ds_nqt = 2 * (int)cdiv(max_seqlen_q, 64);
   p.ds_nkb = 2 * (int)cdiv(max_seqlen_k < total_k ? max_seqlen_k : total_k, 64) + 1;
-  p.hsplit = pick_hsplit(d == 128 && causal ? (max_seqlen_k + 1) / 2 : max_seqlen_k, batch, hq, hk, DKV_ROWS);
+  p.hsplit = bwd_hsplit(max_seqlen_k, batch, hq, hk, d == 128 && causal && !route.both);
   p.dk_part = nullptr;
   p.dv_part = nullptr;
   if (p.hsplit > 1) {

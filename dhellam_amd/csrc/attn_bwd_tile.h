@@ -10,28 +10,30 @@
 namespace dh {
 
 // dQ: RG row groups of 32 query rows x SPLIT splits of the keys, 32-key tiles of K and V.
-template <typename T, int D, int RG, int SPLIT, int WPS>
-__global__ void __launch_bounds__(64 * RG * SPLIT, WPS) attn_bwd_dq_tile_kernel(const AttnBwdParams p) {
+template <typename T, int D, int RG, int SPLIT> constexpr int dq_tile_lds() {
+  const int stage = SPLIT * 2 * 32 * D * (int)sizeof(T), ex = (SPLIT - 1) * RG * 32 * D * 4;
+  return 2 * stage > ex ? 2 * stage : ex;
+}
+// Workgroup bx of gx of sequence by of gy; DELTA: it forms delta, else delta is there already.
+template <typename T, int D, int RG, int SPLIT, bool DELTA>
+__device__ __forceinline__ void dq_tile_body(const AttnBwdParams &p, int bx, int gx, int by, int gy, char *sAll, float *sDel) {
   using M = Mma<T>;
   using Frag = typename M::Frag;
   constexpr int BM = 32 * RG, BN = 32, NW = RG * SPLIT, SLOTF = 32 * D;
   constexpr int TILEB = BN * D * (int)sizeof(T);
   constexpr int STAGEB = SPLIT * 2 * TILEB;
   constexpr int RPW = SPLIT * 2 * BN / NW;                // rows that a wavefront copies per iteration
-  constexpr int EXB = (SPLIT - 1) * RG * SLOTF * 4;
   static_assert(RPW % 16 == 0 && RPW <= BN, "whole copy patterns of one tile per wavefront");
-  constexpr int LDSB = 2 * STAGEB > EXB ? 2 * STAGEB : EXB;
-  __shared__ __attribute__((aligned(1024))) char sAll[LDSB];
-  __shared__ float sDel[32 * RG];
 
-  const int b = seq_by_length(p.cu_q, gridDim.y, blockIdx.y);
-  const int ratio = p.hq / p.hk, P = gridDim.x / p.hq;
+  const int b = seq_by_length(p.cu_q, gy, by);
+  const int ratio = p.hq / p.hk, P = gx / p.hq;
   int hkv, item;
-  xcd_group_item(blockIdx.x, p.hk, ratio * P, hkv, item);
+  xcd_group_item(bx, p.hk, ratio * P, hkv, item);
   const int h = hkv * ratio + item % ratio, px = item / ratio;
   const int q0 = p.cu_q[b] >> p.q_shift, sq = (p.cu_q[b + 1] >> p.q_shift) - q0;
   const int k0 = p.cu_k[b] >> p.k_shift, sk = (p.cu_k[b + 1] >> p.k_shift) - k0;
   const int nqt = (sq + BM - 1) / BM;
+  if constexpr (DELTA) delta_tail_zero<BM>(p, b, h, sq, px);
   if (px >= nqt) return;
   const int m0 = (nqt - 1 - px) * BM;          // late causal tiles carry the most work and come first
   const int causal = p.causal;
@@ -76,7 +78,9 @@ __global__ void __launch_bounds__(64 * RG * SPLIT, WPS) attn_bwd_dq_tile_kernel(
   const int64_t stat = ((int64_t)b * p.hq + h) * p.max_sq + row_q;
   const float lse_c = row_ok ? p.lse[((int64_t)b * p.hq + h) * p.lse_pitch + row_q] * 1.4426950408889634f : INFINITY;        // rows past the end: P = 0
   float del_c = 0.f;
-  if (sp == 0) {       // delta of the workgroup's rows, for the other splits and for the dK/dV pass
+  if (!DELTA) {
+    if (row_ok) del_c = p.delta[stat];
+  } else if (sp == 0) {       // delta of the workgroup's rows, for the other splits and for the dK/dV pass
     const T *op = reinterpret_cast<const T *>(p.out) + (int64_t)(q0 + row_ld) * p.o_stride + (int64_t)h * D + 8 * hh;
 #pragma unroll
     for (int ks = 0; ks < D / 16; ++ks) {
@@ -105,7 +109,7 @@ __global__ void __launch_bounds__(64 * RG * SPLIT, WPS) attn_bwd_dq_tile_kernel(
     for (int v = 0; v < 16; ++v) dQt[t][v] = 0.f;
   dma_wait_all();
   __syncthreads();
-  del_c = sDel[rg * 32 + c];
+  if constexpr (DELTA) del_c = sDel[rg * 32 + c];
 
 #pragma unroll 1
   for (int it = 0; it < niter; ++it) {
@@ -174,22 +178,29 @@ __global__ void __launch_bounds__(64 * RG * SPLIT, WPS) attn_bwd_dq_tile_kernel(
     }
 }
 
+template <typename T, int D, int RG, int SPLIT, int WPS>
+__global__ void __launch_bounds__(64 * RG * SPLIT, WPS) attn_bwd_dq_tile_kernel(const AttnBwdParams p) {
+  __shared__ __attribute__((aligned(1024))) char sAll[dq_tile_lds<T, D, RG, SPLIT>()];
+  __shared__ float sDel[32 * RG];
+  dq_tile_body<T, D, RG, SPLIT, true>(p, blockIdx.x, gridDim.x, blockIdx.y, gridDim.y, sAll, sDel);
+}
+
 // dK, dV: KG row groups of 32 key rows x QSPLIT splits of the query tiles (32 rows of Q and dO each); K and V row
-// fragments stay in registers, lse / delta come straight from the planes that the dQ kernel wrote.
-template <typename T, int D, int KG, int QSPLIT, int WPS>
-__global__ void __launch_bounds__(64 * KG * QSPLIT, WPS) attn_bwd_dkv_tile_kernel(const AttnBwdParams p) {
+// fragments stay in registers, lse / delta come straight from the planes that the kernel before it wrote.
+template <typename T, int D, int QSPLIT> constexpr int dkv_tile_lds() { return 2 * QSPLIT * 2 * 32 * D * (int)sizeof(T); }
+template <typename T, int D, int KG, int QSPLIT>
+__device__ __forceinline__ void dkv_tile_body(const AttnBwdParams &p, int bx, int gx, int by, int gy, char *sAll) {
   using M = Mma<T>;
   using Frag = typename M::Frag;
   constexpr int BN = 32 * KG, BM = 32, NW = KG * QSPLIT, SLOTF = 32 * D;
   constexpr int TILEB = BM * D * (int)sizeof(T);          // bytes of one Q (or dO) tile
   constexpr int STAGEB = QSPLIT * 2 * TILEB;              // per split: Q tile, dO tile
   static_assert(QSPLIT * 2 == NW, "one whole tile per wavefront");
-  __shared__ __attribute__((aligned(1024))) char sAll[2 * STAGEB];
 
-  const int b = seq_by_length(p.cu_k, gridDim.y, blockIdx.y);
+  const int b = seq_by_length(p.cu_k, gy, by);
   const int G = p.hk * p.hsplit;
   int hg, px;
-  xcd_group_item(blockIdx.x, G, gridDim.x / G, hg, px);
+  xcd_group_item(bx, G, gx / G, hg, px);
   const int hkv = hg / p.hsplit, hs = hg % p.hsplit;
   const int q0 = p.cu_q[b] >> p.q_shift, sq = (p.cu_q[b + 1] >> p.q_shift) - q0;
   const int k0 = p.cu_k[b] >> p.k_shift, sk = (p.cu_k[b + 1] >> p.k_shift) - k0;
@@ -389,6 +400,24 @@ __global__ void __launch_bounds__(64 * KG * QSPLIT, WPS) attn_bwd_dkv_tile_kerne
   }
 }
 
+template <typename T, int D, int KG, int QSPLIT, int WPS>
+__global__ void __launch_bounds__(64 * KG * QSPLIT, WPS) attn_bwd_dkv_tile_kernel(const AttnBwdParams p) {
+  __shared__ __attribute__((aligned(1024))) char sAll[dkv_tile_lds<T, D, QSPLIT>()];
+  dkv_tile_body<T, D, KG, QSPLIT>(p, blockIdx.x, gridDim.x, blockIdx.y, gridDim.y, sAll);
+}
+
+// Both passes in one launch, behind the delta kernel: ndkv workgroups a sequence do dK/dV and, after those of all sequences,
+// ndq a sequence dQ.
+template <typename T, int D, int RG, int SPLIT, int KG, int QSPLIT, int WPS>
+__global__ void __launch_bounds__(64 * RG * SPLIT, WPS) attn_bwd_both_tile_kernel(const AttnBwdParams p, int ndkv, int ndq, int batch) {
+  static_assert(RG * SPLIT == KG * QSPLIT, "one workgroup shape");
+  constexpr int A = dq_tile_lds<T, D, RG, SPLIT>(), B = dkv_tile_lds<T, D, QSPLIT>();
+  __shared__ __attribute__((aligned(1024))) char sAll[A > B ? A : B];
+  const int i = blockIdx.x, j = i - ndkv * batch;
+  if (j < 0) dkv_tile_body<T, D, KG, QSPLIT>(p, i % ndkv, ndkv, i / ndkv, batch, sAll);
+  else dq_tile_body<T, D, RG, SPLIT, false>(p, j % ndq, ndq, j / ndq, batch, sAll, nullptr);
+}
+
 template <typename T, int D, int RG, int SPLIT, int WPS>
 static int launch_dq_tile(const AttnBwdParams &p, int batch, hipStream_t st) {
   dim3 grid((unsigned)(cdiv(p.max_sq, 32 * RG) * p.hq), (unsigned)batch);
@@ -400,6 +429,14 @@ template <typename T, int D, int KG, int QSPLIT, int WPS>
 static int launch_dkv_tile(const AttnBwdParams &p, int batch, int max_sk, hipStream_t st) {
   dim3 grid((unsigned)(cdiv(max_sk, 32 * KG) * p.hk * p.hsplit), (unsigned)batch);
   hipLaunchKernelGGL((attn_bwd_dkv_tile_kernel<T, D, KG, QSPLIT, WPS>), grid, dim3(64 * KG * QSPLIT), 0, st, p);
+  return DH_OK;
+}
+
+template <typename T, int D, int RG, int SPLIT, int KG, int QSPLIT, int WPS>
+static int launch_both_tile(const AttnBwdParams &p, int batch, int max_sk, hipStream_t st) {
+  const int64_t ndkv = cdiv(max_sk, 32 * KG) * p.hk * p.hsplit, ndq = cdiv(p.max_sq, 32 * RG) * p.hq;
+  hipLaunchKernelGGL((attn_bwd_both_tile_kernel<T, D, RG, SPLIT, KG, QSPLIT, WPS>), dim3((unsigned)((ndkv + ndq) * batch)),
+                     dim3(64 * RG * SPLIT), 0, st, p, (int)ndkv, (int)ndq, batch);
   return DH_OK;
 }
 

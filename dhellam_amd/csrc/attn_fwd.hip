@@ -29,7 +29,14 @@ struct AttnFwdParams {
   float scale, scale_log2;
   int causal;
   int q_shift, k_shift;      // sequence bounds are cu >> shift (the halves of a context-parallel chunk)
+  int64_t *rng_state;        // two zeros to write, or null
 };
+
+// The (empty) dropout state of the call, by its first workgroup: a fill of two words beforehand cost a launch of 1.5 us.
+__device__ __forceinline__ void rng_state_zero(const AttnFwdParams &p) {
+  if (p.rng_state && (blockIdx.x | blockIdx.y) == 0 && threadIdx.x < 2) p.rng_state[threadIdx.x] = 0;
+}
+__global__ void rng_state_kernel(int64_t *rng_state) { rng_state[threadIdx.x] = 0; }
 
 // ---------------------------------------------------------------------------------------------
 // Head dim 128.
@@ -67,6 +74,7 @@ __global__ void __launch_bounds__(512) attn_fwd_d128_kernel(const AttnFwdParams 
   static_assert(SPLIT * 2 * BPT == 64, "eight copy blocks per wavefront and iteration");
   constexpr int NV = 3;                           // V slots: read one iteration late, copied one ahead
   __shared__ __attribute__((aligned(1024))) T sAll[(2 + NV) * SLOT];   // K slots 0..1, then the V slots
+  rng_state_zero(p);
 
   const int b = seq_by_length(p.cu_q, gridDim.y, blockIdx.y);
   // the query heads of one kv head read the same K / V rows: keep a kv head on one XCD's L2
@@ -457,11 +465,11 @@ extern "C" int dh_attn_fwd_path(int batch, int max_seqlen_q, int64_t total_q, in
   return (r.hand ? 1 : 0) | (r.big ? 2 : 0);
 }
 
-extern "C" int dh_attn_fwd_total(const void *q, const void *k, const void *v, void *out, float *lse,
+extern "C" int dh_attn_fwd_state(const void *q, const void *k, const void *v, void *out, float *lse, int64_t *rng_state,
                                  const int32_t *cu_seqlens_q, const int32_t *cu_seqlens_k, int q_shift, int k_shift,
                                  int batch, int max_seqlen_q, int max_seqlen_k, int64_t total_q, int hq, int hk, int d,
                                  int64_t q_stride, int64_t k_stride, int64_t v_stride, int64_t o_stride,
-                                  float softmax_scale, int causal, int dtype, void *stream) {
+                                 float softmax_scale, int causal, int dtype, void *stream) {
   using namespace dh;
   DH_CHECK((q_shift == 0 || q_shift == 1) && (k_shift == 0 || k_shift == 1), "sequences are taken whole or halved");
   DH_CHECK(dtype != DH_F32 || q_shift + k_shift == 0, "fp32 attention takes whole sequences");
@@ -475,6 +483,7 @@ extern "C" int dh_attn_fwd_total(const void *q, const void *k, const void *v, vo
   hipStream_t st = (hipStream_t)stream;
   if (dtype == DH_F32) {
     DH_CHECK(d > 0 && d <= 256 && d % 4 == 0, "fp32 attention needs d %% 4 == 0 and d <= 256 (got %d)", d);
+    if (rng_state) hipLaunchKernelGGL(rng_state_kernel, dim3(1), dim3(2), 0, st, rng_state);
     return attn_fwd_f32(q, k, v, out, lse, cu_seqlens_q, cu_seqlens_k, batch, max_seqlen_q, max_seqlen_k, hq, hk, d,
                         q_stride, k_stride, v_stride, o_stride, softmax_scale, causal, st);
   }
@@ -494,6 +503,7 @@ extern "C" int dh_attn_fwd_total(const void *q, const void *k, const void *v, vo
   p.scale_log2 = softmax_scale * 1.4426950408889634f;
   p.causal = causal;
   p.q_shift = q_shift; p.k_shift = k_shift;
+  p.rng_state = rng_state;
   const AttnFwdRoute r = attn_fwd_route(max_seqlen_q, hq, d, batch, total_q, causal);
   int rc;
   if (r.hand) {
@@ -505,6 +515,15 @@ extern "C" int dh_attn_fwd_total(const void *q, const void *k, const void *v, vo
   if (rc != DH_OK) return rc;
   DH_LAUNCH_CHECK();
   return DH_OK;
+}
+
+extern "C" int dh_attn_fwd_total(const void *q, const void *k, const void *v, void *out, float *lse,
+                                 const int32_t *cu_seqlens_q, const int32_t *cu_seqlens_k, int q_shift, int k_shift,
+                                 int batch, int max_seqlen_q, int max_seqlen_k, int64_t total_q, int hq, int hk, int d,
+                                 int64_t q_stride, int64_t k_stride, int64_t v_stride, int64_t o_stride,
+                                 float softmax_scale, int causal, int dtype, void *stream) {
+  return dh_attn_fwd_state(q, k, v, out, lse, nullptr, cu_seqlens_q, cu_seqlens_k, q_shift, k_shift, batch, max_seqlen_q, max_seqlen_k,
+                           total_q, hq, hk, d, q_stride, k_stride, v_stride, o_stride, softmax_scale, causal, dtype, stream);
 }
 
 extern "C" int dh_attn_fwd_halves(const void *q, const void *k, const void *v, void *out, float *lse,

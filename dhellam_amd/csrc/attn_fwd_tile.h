@@ -30,6 +30,7 @@ __global__ void __launch_bounds__(64 * RG * SPLIT, WPS) attn_fwd_tile_kernel(con
   static_assert(RPW % 16 == 0 && RPW <= BN, "whole copy patterns of one tile per wavefront");
   __shared__ __attribute__((aligned(1024))) char sAll[2 * STAGEB > EXB ? 2 * STAGEB : EXB];
 
+  rng_state_zero(p);
   const int b = seq_by_length(p.cu_q, gridDim.y, blockIdx.y);
   // the query heads of one kv head read the same K / V rows: keep a kv head on one XCD's L2, late causal tiles first
   const int ratio = p.hq / p.hk, P = gridDim.x / p.hq;

@@ -148,11 +148,13 @@ std::vector<at::Tensor> pymha_varlen_fwd(const at::Tensor &q_in, const at::Tenso
   const at::Tensor q = pad_head_dim(q_in, d_run), k = pad_head_dim(k_in, d_run), v = pad_head_dim(v_in, d_run);
   auto out_padded = at::empty(q.sizes(), q.options());
   auto lse = at::empty({b, q.size(1), max_seqlen_q}, q.options().dtype(at::kFloat));
+  const bool empty = b == 0 || max_seqlen_q == 0;      // nothing runs that would write the state
+  auto rng_state = empty ? at::zeros({2}, q.options().dtype(at::kLong)) : at::empty({2}, q.options().dtype(at::kLong));
   hipStream_t stream = c10::hip::getCurrentHIPStream().stream();
   const float ms = timed(profiling, stream, [&] {
     confined(stream, q.device().index(), math_sm_count, [&](hipStream_t st) {
-      check(dh_attn_fwd_total(q.data_ptr(), k.data_ptr(), v.data_ptr(), out_padded.data_ptr(), lse.data_ptr<float>(),
-                              cu_seqlens_q.data_ptr<int>(), cu_seqlens_k.data_ptr<int>(), 0, 0, b, max_seqlen_q,
+      check(dh_attn_fwd_state(q.data_ptr(), k.data_ptr(), v.data_ptr(), out_padded.data_ptr(), lse.data_ptr<float>(),
+                              rng_state.data_ptr<int64_t>(), cu_seqlens_q.data_ptr<int>(), cu_seqlens_k.data_ptr<int>(), 0, 0, b, max_seqlen_q,
                               max_seqlen_k, q.size(0), (int)q.size(1), (int)k.size(1), (int)q.size(2), token_stride(q),
                               token_stride(k), token_stride(v), token_stride(out_padded), softmax_scale,
                               is_causal ? 1 : 0, dt(q), st));
@@ -160,7 +162,7 @@ std::vector<at::Tensor> pymha_varlen_fwd(const at::Tensor &q_in, const at::Tenso
   });
   const at::Tensor out = d_run == d_og ? out_padded : out_padded.narrow(-1, 0, d_og);
   std::vector<at::Tensor> res = {out, q, k, v, out_padded, lse, at::empty({0}, q.options()),
-                                 at::zeros({2}, q.options().dtype(at::kLong))};
+                                 rng_state};
   if (profiling) res.push_back(ms_tensor(ms));
   return res;
 }
@@ -185,7 +187,7 @@ std::vector<at::Tensor> pymha_varlen_bwd(const at::Tensor &dout_in, const at::Te
                    v = pad_head_dim(v_in, d_run), out = pad_head_dim(out_in, d_run);
   const int b = (int)cu_seqlens_q.numel() - 1, hq = (int)q.size(1), hk = (int)k.size(1), d = (int)q.size(2);
   auto dq = at::empty(q.sizes(), q.options()), dk = at::empty(k.sizes(), k.options()), dv = at::empty(v.sizes(), v.options());
-  auto softmax_d = at::zeros({b, hq, max_seqlen_q}, q.options().dtype(at::kFloat));
+  auto softmax_d = at::empty({b, hq, max_seqlen_q}, q.options().dtype(at::kFloat));      // the kernels write all of it
   // scratch: the library says how much, and is told how much it got
   const size_t ws_bytes = dh_attn_bwd_workspace_bytes(q.size(0), k.size(0), b, max_seqlen_q, hq, hk, d, dt(q));
   auto ws = at::empty({(int64_t)ws_bytes}, q.options().dtype(at::kByte));

@@ -175,16 +175,33 @@ int dh_attn_fwd_total(const void *q, const void *k, const void *v, void *out,
                       int64_t k_stride, int64_t v_stride, int64_t o_stride,
                       float softmax_scale, int causal, int dtype, void *stream);
 
+/* ... and with the dropout state of the return list: rng_state (two int64, or
+ * null) is set to zero by the same kernels.  An empty call (no sequences or
+ * max_seqlen_q == 0) launches nothing and leaves it alone. */
+int dh_attn_fwd_state(const void *q, const void *k, const void *v, void *out,
+                      float *lse, int64_t *rng_state,
+                      const int32_t *cu_seqlens_q, const int32_t *cu_seqlens_k,
+                      int q_shift, int k_shift, int batch, int max_seqlen_q,
+                      int max_seqlen_k, int64_t total_q, int hq, int hk, int d,
+                      int64_t q_stride, int64_t k_stride, int64_t v_stride,
+                      int64_t o_stride, float softmax_scale, int causal,
+                      int dtype, void *stream);
+
 /* Which kernels a 16-bit call of these sizes runs (what the entries themselves
  * go by).  Forward: bit 0 = head dim 128's hand-ordered kernel, bit 1 = query
  * tiles of 128 rows (else 64).  Backward: bit 0 = head dim 128's hand-ordered
  * dK/dV kernel, bit 1 = dQ from kept dS, else bit 2 = the hand-ordered
- * recomputing dQ kernel and bit 3 = its query tiles have 128 rows. */
+ * recomputing dQ kernel and bit 3 = its query tiles have 128 rows (all
+ * clear: the other kernels, which for small calls run in one launch, as
+ * dh_attn_bwd_one_launch tells). */
 int dh_attn_fwd_path(int batch, int max_seqlen_q, int64_t total_q, int hq,
                      int d, int causal);
 int dh_attn_bwd_path(int batch, int max_seqlen_q, int max_seqlen_k,
                      int64_t total_q, int64_t total_k, int hq, int hk, int d,
                      int causal, size_t workspace_bytes);
+int dh_attn_bwd_one_launch(int batch, int max_seqlen_q, int max_seqlen_k,
+                           int64_t total_q, int64_t total_k, int hq, int hk,
+                           int d, int causal);
 
 /* Bytes of scratch dh_attn_bwd works in.  dh_attn_bwd_min_workspace_bytes: what
  * every call of these sizes needs (delta = rowsum(dO*O), the lse / delta planes

@@ -443,3 +443,64 @@ def test_attention_chip_filling_tiles_of_other_head_dims(dtype, d, lens, hq, hk,
     """The 128-row query tiles of the compiler-scheduled kernels, at the ends of tiles."""
     assert _fwd_path(lens, hq, d, causal) == fwd and _bwd_path(lens, lens, hq, hk, d, causal) == bwd
     _run_fwd_bwd(dtype, lens, lens, hq, hk, d, causal, oracle_dtype=torch.float32)
+
+
+@pytest.mark.parametrize("d,lens_q,lens_k,hq,hk,causal,one", [
+    (64, [28], [28], 3, 3, True, 1), (64, [65, 1, 0, 128], [65, 1, 0, 128], 4, 2, True, 1), (64, [40, 97], [200, 33], 8, 2, False, 1),
+    (64, [512] * 2, [512] * 2, 16, 16, False, 0), (64, [1025], [1025], 32, 8, True, 1),          # both sides of the line
+    (96, [33, 63], [33, 63], 4, 4, True, 1), (96, [200, 1], [64, 130], 4, 1, False, 1),
+    (128, [31], [31], 2, 2, True, 1), (128, [100, 257, 64], [100, 257, 64], 4, 2, True, 1), (128, [70, 129], [70, 129], 8, 2, False, 1),
+    (192, [97, 2], [97, 2], 4, 2, True, 1), (192, [65], [31], 2, 2, False, 1),
+    (256, [129, 60], [129, 60], 2, 1, True, 1), (256, [32], [64], 4, 4, False, 1), (64, [50, 0], [20, 70], 2, 2, False, 1),
+])
+def test_attention_backward_in_one_launch(d, lens_q, lens_k, hq, hk, causal, one):
+    """dK/dV and dQ by one grid behind the delta kernel: ragged ends, empty sequences, split and whole GQA groups,
+    against the oracle; twice the same bits; delta zero past every sequence's end through the compiled module."""
+    import importlib
+    from dhellam_amd import _lib, _Clib
+    t = sum(lens_q), sum(lens_k)
+    assert _lib.load().dh_attn_bwd_one_launch(len(lens_q), max(lens_q), max(lens_k), *t, hq, hk, d, causal) == one
+    _run_fwd_bwd(torch.bfloat16, lens_q, lens_k, hq, hk, d, causal, oracle_dtype=torch.float32)
+    ext = importlib.import_module("dhellam._Clib")
+    cq, ck = _cu(lens_q).cuda(), _cu(lens_k).cuda()
+    q, k, v, do = (randn((n, h, d), torch.float16, 50 + i).cuda() for i, (n, h) in enumerate(zip((*t, t[1], t[0]), (hq, hk, hk, hq))))
+    got = []
+    for mod in (ext, ext, _Clib):
+        junk = [torch.full((n,), float("nan"), device="cuda") for n in (2, 4, len(lens_q) * hq * max(lens_q))]
+        del junk                                    # what the results are made in holds no zeros by chance
+        res = mod.pymha_varlen_fwd(q, k, v, cq, ck, max(lens_q), max(lens_k), 0.0, d ** -0.5, causal, False, 0, False)
+        assert res[7].tolist() == [0, 0]
+        bwd = mod.pymha_varlen_bwd(do, q, k, v, res[0], res[5], cq, ck, max(lens_q), max(lens_k), 0.0, d ** -0.5, causal, res[7], True,
+                                   0, False, torch.cuda.current_stream().cuda_stream)
+        for i, n in enumerate(lens_q):
+            assert (bwd[3][i, :, n:] == 0).all()
+        got.append((res[0], *bwd))
+    for other in got[1:]:
+        for a, b in zip(got[0], other):
+            assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("d,lens,hq,hk,causal,dtype", [
+    (128, [1537, 3], 19, 19, True, torch.bfloat16),              # dS kept: the delta kernel
+    (128, [512, 491], 64, 64, True, torch.bfloat16),             # the hand-ordered dQ, paired tiles
+    (128, [513, 70], 64, 64, False, torch.bfloat16),
+    (64, [1100, 300], 64, 64, True, torch.bfloat16),             # the other dQ kernels
+    (192, [300, 33, 257], 64, 64, True, torch.bfloat16), (64, [70, 33], 3, 3, True, torch.float32),
+])
+def test_attention_delta_is_zero_past_a_sequence(d, lens, hq, hk, causal, dtype):
+    """Every kernel that writes delta as an output writes the rows past a sequence's end too."""
+    from dhellam_amd import _Clib
+    t, m, cu, scale = sum(lens), max(lens), _cu(lens).cuda(), d ** -0.5
+    q, k, v, do = (randn((t, h, d), dtype, 60 + i).cuda() for i, h in enumerate((hq, hk, hk, hq)))
+    out, lse = _Clib.pymha_varlen_fwd(q, k, v, cu, cu, m, m, 0.0, scale, causal, False, 0, False)[:6:5]
+    want = (do.float() * out.float()).sum(-1)
+    dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
+    delta = torch.full((len(lens), hq, m), float("nan"), device="cuda")
+    _Clib._attn_bwd_raw(do, q, k, v, out, lse, dq, dk, dv, delta, cu, cu, m, m, scale, causal)
+    # rowsum of d products in fp32: |error| <= d 2^-24 sum |dO O|
+    bound = d * 2.0 ** -23 * (do.float() * out.float()).abs().sum(-1) + 1e-30
+    at = 0
+    for i, n in enumerate(lens):
+        assert (delta[i, :, n:] == 0).all()
+        assert ((delta[i, :, :n].t() - want[at:at + n]).abs() <= bound[at:at + n]).all()
+        at += n
