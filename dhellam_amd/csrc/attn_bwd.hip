@@ -1146,21 +1146,22 @@ static int bwd_hsplit(int max_sk, int batch, int hq, int hk, bool paired) {
   return pick_hsplit(paired ? (max_sk + 1) / 2 : max_sk, batch, hq, hk, DKV_ROWS);
 }
 
-// Whether dK/dV and dQ go into one launch of the tile kernels, behind the delta kernel (2.5 us).  Either pass alone leaves
+// Whether dK/dV and dQ go into one launch of the tile kernels, behind the delta kernel (2 us).  Either pass alone leaves
 // compute units idle: all of those that it has no workgroup for, the last round's, and with causal rows those that got short
 // tiles (one workgroup a compute unit in all forms: registers).  Together the long workgroups (dK/dV: 1.3 times a dQ one and
 // once per query head of its group) start first and the others fill in.  `a` and `b`: workgroups of dQ and dK/dV with work.
 // Backward, us, two launches / one, head dims 64 | 192 (96 and 256 behave as they do):
-//   all in one round: 12 heads x 28 12.1 / 9.6 | 19.6 / 13.7, 16 x 300 18.7 / 14.1 | 41.7 / 26.9, causal or not;
-//   causal, a round and a half: 8 x 1500 40.0 / 27.0 | 125 / 72, 32 x 300 19.1 / 17.0 | 43 / 35; two full rounds of short rows
-//     16 x 16 x 60 16.8 / 18.6 | 29.5 / 32.3, of long ones 8 x 2048 49 / 38 | 162 / 106, 16 x 1024 31.4 / 30.3 | 93 / 85; dK/dV in one
-//     round, dQ in several: 32 query / 8 kv heads x 1500 105 / 79 | 342 / 243, but 16 x 1500 (dK/dV in two) 46.1 / 47.8 | 130 / 132;
-//   otherwise by the model: 16 x 1500 not causal (1.28 predicted) 77 / 66 | 255 / 201, 32 / 8 x 600 + 300 (1.38) 54 / 42 | 167 / 116, 32
-//     x 300 (1.15, not taken) 19.8 / 18.5 | 44 / 42, 16 x 1024 (1.0) 32.3 / 34.9 | 95 / 98.
+//   all in one round: 16 heads x 300 17.4 / 13.3 | 40 / 26, causal or not;
+//   causal, a round and a half: 8 x 1500 36.9 / 24.9 | 118 / 66, 32 x 300 17.9 / 17.0 | 42 / 35; two full rounds of short rows
+//     16 x 16 x 60 15.9 / 17.8 | 29 / 32, of long ones 8 x 2048 45 / 34 | 152 / 102, 16 x 1024 29.0 / 28.2 | 88 / 83; dK/dV in one
+//     round, dQ in several: 32 query / 8 kv heads x 1500 93 / 67 | 315 / 218, but 16 x 1500 (dK/dV in two) 42.7 / 44.4 | 123 / 127;
+//   otherwise by the model: 16 x 1500 not causal (1.28 predicted) 71 / 58 | 234 / 183, 32 / 8 x 600 + 300 (1.38) 49 / 37 | 152 / 100, 32
+//     x 300 (1.15, not taken) 18.8 / 18.5 | 42 / 42, 16 x 1024 (1.0) 29.3 / 30.9 | 89 / 93.
 // Head dim 128 has the hand-ordered kernels to compare with, whose workgroups start and end later but run 1.5 times as fast:
-//   one round: 12 x 28 16.5 / 11.0, 16 x 300 29 / 20 causal, 26 / 21 not, 8 x 1024 51 / 39, not causal 41.7 / 41.9;
-//   causal, up to a round and a half: 8 x 1500 66 / 53; two: 32 x 512 45.5 / 42.2, 16 x 1024 55 / 61, 16 x 16 x 60 23.2 / 22.8.
-// A group split eight ways from 512 rows on (8 query / 1 kv head x 1024: 57.8 / 46.1) and rectangular calls that are not
+//   one round: 16 x 300 28 / 20 causal, 26 / 20 not, 8 x 1024 51 / 35 causal, 41 / 35 not;
+//   causal, up to a round and a half: 8 x 1500 66 / 47; two: 32 x 512 44 / 40, 16 x 1024 55 / 57, 16 x 16 x 60 22.8 / 22.5; not
+//   causal: 8 x 1500 62 / 84, 32 x 512 36 / 41.
+// A group split eight ways from 512 rows on (8 query / 1 kv head x 1024: 58 / 46) and rectangular calls that are not
 // causal stay with the hand-ordered kernels: callers size the workspace there to choose between their two forms of dQ.
 static bool bwd_both_pays(int batch, int max_sq, int max_sk, int64_t total_q, int64_t total_k, int hq, int hk, int d, int causal) {
   if (max_sq <= 0 || max_sk <= 0) return false;
@@ -1171,7 +1172,7 @@ static bool bwd_both_pays(int batch, int max_sq, int max_sk, int64_t total_q, in
   const int hs = bwd_hsplit(max_sk, batch, hq, hk, false);
   const int64_t a = tiles(max_sq, total_q) * hq, b = tiles(max_sk, total_k) * hk * hs;
   if (d == 128) {
-    if (!causal) return a + b <= 256 && max_sq < 1024 && max_sq == max_sk;
+    if (!causal) return a + b <= 256 && max_sq == max_sk;
     if (max_sq >= 512 && hs >= 8) return false;
     return a + b <= 384 || (a + b <= 512 && max_sq >= 256 && max_sq < 1024);
   }
@@ -1351,7 +1352,7 @@ static int attn_bwd_entry(const void *dout, const void *q, const void *k, const 
   if (dsb > 0 && base_bytes + align256(dsb) > workspace_bytes) dsb = 0;
   const AttnBwdRoute route = attn_bwd_route(batch, max_seqlen_q, max_seqlen_k, total_q, total_k, hq, hk, d, causal, dsb > 0);
   uint8_t *ds_ws = (uint8_t *)(((uintptr_t)workspace + 255) & ~(uintptr_t)255) + (base_bytes - 256);
-  const bool delta_in_dq = dtype != DH_F32 && !route.keep_ds && !route.both;
+  const bool delta_in_dq = dtype != DH_F32 && !route.keep_ds;
   if (max_seqlen_q > 0 && !delta_in_dq) {
     DH_DISPATCH_DTYPE(dtype, {
       launch_delta<T>(dout, out, delta, lse, ld2, (int64_t)(plane2 / sizeof(float)), ld2_pitch, cu_seqlens_q, q_shift, lse_pitch,

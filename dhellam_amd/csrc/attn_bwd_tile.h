@@ -1,18 +1,20 @@
 // Attention backward on the tile layout of attn_tile.h (16 bits), two passes: dQ (which forms delta = rowsum(dO O) and runs
-// first) and dK/dV.  Workgroup shape and what bounds it: as the forward kernel (attn_fwd_tile.h).
-// dK/dV keeps K and V fragments and both accumulators in registers (210 at head dim 64, 255 at 96): two wavefronts a SIMD, one
-// at the larger head dims (348 at 128; at 256 all 512 and 76 more that are spilled, 212 bytes a lane, of which 9 loads a tile
-// read back 24).  dQ at head dim 128 in its 64-row form spills 8 of 256, outside the loop.
-// Measured against the register-staged kernels, backward, causal: 16 heads x 2 x 512, head dim 64 58 -> 24 us; 32 query / 8
-// kv heads x 4096, head dim 64 1313 -> 324, 96 1562 -> 438, 256 10871 -> 1841 us; 16 heads x 2048, head dim 192 642 -> 201 us.
+// first) and dK/dV, or both in one grid behind a delta kernel.  Workgroup shape and what bounds it: as the forward kernel
+// (attn_fwd_tile.h).
+// dK/dV keeps K and V fragments and both accumulators in registers (196 at head dim 64, 244 at 96): two wavefronts a SIMD, one
+// at the larger head dims (332 at 128; at 256 all 512 and 75 more that are spilled, 216 bytes a lane).  dQ at head dim 128
+// in its 64-row form spills 8 of 256, outside the loop.
+// Measured, backward, causal, register-staged kernels / these with a memory latency exposed in every iteration / now: 16 heads x
+// 2 x 512, head dim 64 58 / 24 / 22 us; 32 query / 8 kv heads x 4096, head dim 64 1313 / 326 / 290, 96 1562 / 440 / 420, 256 10871 / 1842
+// / 1736 us; 16 heads x 1024, head dim 192 - / 95 / 82 us.
 #include "attn_tile.h"
 
 namespace dh {
 
 // dQ: RG row groups of 32 query rows x SPLIT splits of the keys, 32-key tiles of K and V.
-template <typename T, int D, int RG, int SPLIT> constexpr int dq_tile_lds() {
-  const int stage = SPLIT * 2 * 32 * D * (int)sizeof(T), ex = (SPLIT - 1) * RG * 32 * D * 4;
-  return 2 * stage > ex ? 2 * stage : ex;
+template <int D, int RG, int SPLIT> constexpr int dq_tile_lds() {
+  const int all = 2 * SPLIT * 2 * 32 * D * 2, ex = (SPLIT - 1) * RG * 32 * D * 4;
+  return all > ex ? all : ex;
 }
 // Workgroup bx of gx of sequence by of gy; DELTA: it forms delta, else delta is there already.
 template <typename T, int D, int RG, int SPLIT, bool DELTA>
@@ -22,6 +24,7 @@ __device__ __forceinline__ void dq_tile_body(const AttnBwdParams &p, int bx, int
   constexpr int BM = 32 * RG, BN = 32, NW = RG * SPLIT, SLOTF = 32 * D;
   constexpr int TILEB = BN * D * (int)sizeof(T);
   constexpr int STAGEB = SPLIT * 2 * TILEB;
+  static_assert(sizeof(T) == 2, "dq_tile_lds");
   constexpr int RPW = SPLIT * 2 * BN / NW;                // rows that a wavefront copies per iteration
   static_assert(RPW % 16 == 0 && RPW <= BN, "whole copy patterns of one tile per wavefront");
 
@@ -107,12 +110,19 @@ __device__ __forceinline__ void dq_tile_body(const AttnBwdParams &p, int bx, int
   for (int t = 0; t < D / 32; ++t)
 #pragma unroll
     for (int v = 0; v < 16; ++v) dQt[t][v] = 0.f;
-  dma_wait_all();
-  __syncthreads();
-  if constexpr (DELTA) del_c = sDel[rg * 32 + c];
+  if constexpr (DELTA) {
+    __syncthreads();
+    del_c = sDel[rg * 32 + c];
+  }
 
+  loaded_here(Qf);
+  loaded_here(dOf);
+  float stats[2] = {lse_c, del_c};
+  loaded_here(stats);
 #pragma unroll 1
   for (int it = 0; it < niter; ++it) {
+    dma_wait_all();
+    __syncthreads();                             // this stage has landed, and everyone is done with the other one
     if (it + 1 < niter) issue(it + 1);
     const int tile = it * SPLIT + sp, n0 = tile * BN;
     if (tile < ntiles && !(causal && n0 > wrow0 + 31)) {
@@ -137,16 +147,15 @@ __device__ __forceinline__ void dq_tile_body(const AttnBwdParams &p, int bx, int
       for (int s = 0; s < 2; ++s) {
         float ds[8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) ds[j] = fast_exp2(S[8 * s + j] * scale_log2 - lse_c) * (dP[8 * s + j] - del_c);
+        for (int j = 0; j < 8; ++j) ds[j] = fast_exp2(S[8 * s + j] * scale_log2 - stats[0]) * (dP[8 * s + j] - stats[1]);
         const Frag dSb = frag_pack<T>(ds);
 #pragma unroll
         for (int t = 0; t < D / 32; ++t)
           dQt[t] = M::mma(tr_frag<T, D>(kt, tl, t, s), dSb, dQt[t]);
       }
     }
-    dma_wait_all();
-    __syncthreads();
   }
+  __syncthreads();
 
   // add the splits' partial dQ through LDS, in split order: slot x = (split - 1) * RG + row group
   float *xo = reinterpret_cast<float *>(sAll);
@@ -180,21 +189,26 @@ __device__ __forceinline__ void dq_tile_body(const AttnBwdParams &p, int bx, int
 
 template <typename T, int D, int RG, int SPLIT, int WPS>
 __global__ void __launch_bounds__(64 * RG * SPLIT, WPS) attn_bwd_dq_tile_kernel(const AttnBwdParams p) {
-  __shared__ __attribute__((aligned(1024))) char sAll[dq_tile_lds<T, D, RG, SPLIT>()];
+  __shared__ __attribute__((aligned(1024))) char sAll[dq_tile_lds<D, RG, SPLIT>()];
   __shared__ float sDel[32 * RG];
   dq_tile_body<T, D, RG, SPLIT, true>(p, blockIdx.x, gridDim.x, blockIdx.y, gridDim.y, sAll, sDel);
 }
 
 // dK, dV: KG row groups of 32 key rows x QSPLIT splits of the query tiles (32 rows of Q and dO each); K and V row
-// fragments stay in registers, lse / delta come straight from the planes that the kernel before it wrote.
-template <typename T, int D, int QSPLIT> constexpr int dkv_tile_lds() { return 2 * QSPLIT * 2 * 32 * D * (int)sizeof(T); }
+// fragments stay in registers; lse and delta of a tile, from the planes that the kernel before it wrote, are copied along
+// with it (256 bytes each, of which the first 128 count).
+template <int D, int QSPLIT> constexpr int dkv_tile_stage() { return QSPLIT * (2 * 32 * D * 2 + 512); }
+template <int D, int QSPLIT> constexpr int dkv_tile_lds() {
+  return 2 * dkv_tile_stage<D, QSPLIT>();
+}
 template <typename T, int D, int KG, int QSPLIT>
 __device__ __forceinline__ void dkv_tile_body(const AttnBwdParams &p, int bx, int gx, int by, int gy, char *sAll) {
   using M = Mma<T>;
   using Frag = typename M::Frag;
   constexpr int BN = 32 * KG, BM = 32, NW = KG * QSPLIT, SLOTF = 32 * D;
   constexpr int TILEB = BM * D * (int)sizeof(T);          // bytes of one Q (or dO) tile
-  constexpr int STAGEB = QSPLIT * 2 * TILEB;              // per split: Q tile, dO tile
+  constexpr int STAGEB = dkv_tile_stage<D, QSPLIT>();     // per split: Q tile, dO tile; behind them, per split: lse, delta
+  static_assert(sizeof(T) == 2, "dkv_tile_stage");
   static_assert(QSPLIT * 2 == NW, "one whole tile per wavefront");
 
   const int b = seq_by_length(p.cu_k, gy, by);
@@ -228,12 +242,19 @@ __device__ __forceinline__ void dkv_tile_body(const AttnBwdParams &p, int bx, in
   const int ntq = i_begin < sq ? (sq - i_begin + BM - 1) / BM : 0;
   const int it_per_head = (ntq + QSPLIT - 1) / QSPLIT;
   const int niter = it_per_head * hper;
-  auto issue = [&](int stage, int g, int ti) {
-    const int tq = ti * QSPLIT + cp_sp;
-    if (tq < ntq)
-      copy_tile<T, D, BM>(cp_g + (int64_t)(h_first + g) * D, cp_stride, i_begin + tq * BM, sq, cp_dst + (uint32_t)(stage * STAGEB), cl, lane);
+  int gi = 0, si = 0;                                     // head and step of the next iteration to be copied
+  const float *ld_g = p.ld2 + (cp_do ? p.ld2_plane : 0) + c;
+  auto issue = [&](int slot) {
+    const int tq = si * QSPLIT + cp_sp, row0 = i_begin + tq * BM;
+    if (tq < ntq) {
+      copy_tile<T, D, BM>(cp_g + (int64_t)(h_first + gi) * D, cp_stride, row0, sq, cp_dst + (uint32_t)(slot * STAGEB), cl, lane);
+      const float *src = ld_g + ((int64_t)b * p.hq + (h_first + gi)) * p.ld2_pitch + row0;
+      asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off"
+                   : : "v"(src), "s"(lds0 + (uint32_t)(slot * STAGEB + QSPLIT * 2 * TILEB + (cp_sp * 2 + cp_do) * 256)) : "memory", "m0");
+    }
+    if (++si == it_per_head) { si = 0; ++gi; }
   };
-  if (niter > 0) issue(0, 0, 0);
+  if (niter > 0) issue(0);
 
   Frag Kf[D / 16], Vf[D / 16];
   {
@@ -256,37 +277,26 @@ __device__ __forceinline__ void dkv_tile_body(const AttnBwdParams &p, int bx, in
     }
   const RowLane rl = row_lane<D>(lane);
   const TrLane tl = tr_lane<D>(lane);
-  // lse (exp2 units) and delta of the rows 8 vb + 4 hh + e of this wavefront's query tile (no branch: past the last tile it
-  // loads the last one's)
-  floatx4 l4[4], d4[4];
-  auto load_ld = [&](int g, int ti) {
-    const int tq = ti * QSPLIT + qs < ntq ? ti * QSPLIT + qs : ntq - 1;
-    const float *src = p.ld2 + ((int64_t)b * p.hq + (h_first + g)) * p.ld2_pitch + (i_begin + tq * BM) + 4 * hh;
-#pragma unroll
-    for (int vb = 0; vb < 4; ++vb) {
-      l4[vb] = *reinterpret_cast<const floatx4 *>(src + 8 * vb);
-      d4[vb] = *reinterpret_cast<const floatx4 *>(src + p.ld2_plane + 8 * vb);
-    }
-  };
-#pragma unroll
-  for (int vb = 0; vb < 4; ++vb) {
-    l4[vb] = (floatx4)(0.f);
-    d4[vb] = (floatx4)(0.f);
-  }
-  if (niter > 0) load_ld(0, 0);
-  dma_wait_all();
-  __syncthreads();
-
-  int g = 0, ti = 0;                                // head and step of iteration it
+  loaded_here(Kf);
+  loaded_here(Vf);
+  int ti = 0;                                             // step of iteration it
 #pragma unroll 1
   for (int it = 0; it < niter; ++it) {
-    int gn = g, tn = ti + 1;                        // ... and of iteration it + 1
-    if (tn == it_per_head) { tn = 0; ++gn; }
-    const bool have_next = it + 1 < niter;
-    if (have_next) issue((it + 1) & 1, gn, tn);
+    dma_wait_all();
+    __syncthreads();                                      // this stage has landed, and everyone is done with the other one
+    if (it + 1 < niter) issue((it + 1) & 1);
     const int tq = ti * QSPLIT + qs, i0 = i_begin + tq * BM;
     if (tq < ntq && !(causal && i0 + BM - 1 < jw0)) {
       const uint32_t qt = lds0 + (uint32_t)((it & 1) * STAGEB + qs * 2 * TILEB), dt = qt + (uint32_t)TILEB;
+      // lse (exp2 units) and delta of the rows 8 vb + 4 hh + e
+      typedef __attribute__((address_space(3))) const floatx4 *lds_f4;
+      const uint32_t lt = lds0 + (uint32_t)((it & 1) * STAGEB + QSPLIT * 2 * TILEB + qs * 512 + 16 * hh);
+      floatx4 l4[4], d4[4];
+#pragma unroll
+      for (int vb = 0; vb < 4; ++vb) {
+        l4[vb] = *(lds_f4)(lt + 32 * vb);
+        d4[vb] = *(lds_f4)(lt + 256 + 32 * vb);
+      }
       floatx16 S, dP;
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
@@ -327,14 +337,9 @@ __device__ __forceinline__ void dkv_tile_body(const AttnBwdParams &p, int bx, in
           dKt[t] = M::mma(tr_frag<T, D>(qt, tl, t, s), dSb[s], dKt[t]);
         }
     }
-    if (have_next) {
-      g = gn;
-      ti = tn;
-    }
-    load_ld(g, ti);
-    dma_wait_all();
-    __syncthreads();
+    if (++ti == it_per_head) ti = 0;
   }
+  __syncthreads();
 
   // add the splits' partial sums through LDS in a fixed order, halving: (0 += 2, 1 += 3), then 0 += 1; per (split, key
   // group): dK, then dV
@@ -402,8 +407,38 @@ __device__ __forceinline__ void dkv_tile_body(const AttnBwdParams &p, int bx, in
 
 template <typename T, int D, int KG, int QSPLIT, int WPS>
 __global__ void __launch_bounds__(64 * KG * QSPLIT, WPS) attn_bwd_dkv_tile_kernel(const AttnBwdParams p) {
-  __shared__ __attribute__((aligned(1024))) char sAll[dkv_tile_lds<T, D, QSPLIT>()];
+  __shared__ __attribute__((aligned(1024))) char sAll[dkv_tile_lds<D, QSPLIT>()];
   dkv_tile_body<T, D, KG, QSPLIT>(p, blockIdx.x, gridDim.x, blockIdx.y, gridDim.y, sAll);
+}
+
+// delta, with the lse / delta planes, in front of the two passes in one launch: two lanes a row, which add in the order of the
+// dQ kernel's prologue.  (Where all of a sequence's attention is on one key, dS is the difference of two roundings: in another
+// order dQ and dK would be other noise.)
+template <typename T, int D> __global__ void __launch_bounds__(256) attn_bwd_delta_kernel(const AttnBwdParams p) {
+  const int b = blockIdx.y, q0 = p.cu_q[b] >> p.q_shift, sq = (p.cu_q[b + 1] >> p.q_shift) - q0, hh = threadIdx.x & 1;
+  const int rows = p.delta_tail ? p.max_sq : sq, padded = (sq + 31) / 32 * 32, all = rows > padded ? rows : padded;
+  for (int64_t item = (int64_t)blockIdx.x * 128 + (threadIdx.x >> 1); item < (int64_t)all * p.hq; item += (int64_t)gridDim.x * 128) {
+    const int i = (int)(item / p.hq), h = (int)(item % p.hq);
+    float s = 0.f;
+    if (i < sq) {
+      const T *dp = reinterpret_cast<const T *>(p.dout) + (int64_t)(q0 + i) * p.do_stride + (int64_t)h * D + 8 * hh;
+      const T *op = reinterpret_cast<const T *>(p.out) + (int64_t)(q0 + i) * p.o_stride + (int64_t)h * D + 8 * hh;
+      typename Mma<T>::Frag df[D / 16], of[D / 16];
+#pragma unroll
+      for (int ks = 0; ks < D / 16; ++ks) {
+        df[ks] = frag_ld<T>(dp + ks * 16);
+        of[ks] = frag_ld<T>(op + ks * 16);
+      }
+#pragma unroll
+      for (int ks = 0; ks < D / 16; ++ks)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) s += to_f(df[ks][j]) * to_f(of[ks][j]);
+    }
+    s += __shfl_xor(s, 1, 64);                   // both lanes of a row are at the same item
+    const int64_t head = (int64_t)b * p.hq + h;
+    if (hh == 0 && i < rows) p.delta[head * p.max_sq + i] = s;
+    if (i < padded) p.ld2[(hh ? p.ld2_plane : 0) + head * p.ld2_pitch + i] = hh ? s : i < sq ? p.lse[head * p.lse_pitch + i] * 1.4426950408889634f : 0.f;
+  }
 }
 
 // Both passes in one launch, behind the delta kernel: ndkv workgroups a sequence do dK/dV and, after those of all sequences,
@@ -411,7 +446,7 @@ __global__ void __launch_bounds__(64 * KG * QSPLIT, WPS) attn_bwd_dkv_tile_kerne
 template <typename T, int D, int RG, int SPLIT, int KG, int QSPLIT, int WPS>
 __global__ void __launch_bounds__(64 * RG * SPLIT, WPS) attn_bwd_both_tile_kernel(const AttnBwdParams p, int ndkv, int ndq, int batch) {
   static_assert(RG * SPLIT == KG * QSPLIT, "one workgroup shape");
-  constexpr int A = dq_tile_lds<T, D, RG, SPLIT>(), B = dkv_tile_lds<T, D, QSPLIT>();
+  constexpr int A = dq_tile_lds<D, RG, SPLIT>(), B = dkv_tile_lds<D, QSPLIT>();
   __shared__ __attribute__((aligned(1024))) char sAll[A > B ? A : B];
   const int i = blockIdx.x, j = i - ndkv * batch;
   if (j < 0) dkv_tile_body<T, D, KG, QSPLIT>(p, i % ndkv, ndkv, i / ndkv, batch, sAll);
@@ -434,6 +469,8 @@ static int launch_dkv_tile(const AttnBwdParams &p, int batch, int max_sk, hipStr
 
 template <typename T, int D, int RG, int SPLIT, int KG, int QSPLIT, int WPS>
 static int launch_both_tile(const AttnBwdParams &p, int batch, int max_sk, hipStream_t st) {
+  const int64_t items = (int64_t)p.ld2_pitch * p.hq, blocks = cdiv(items, 128) < 4096 ? cdiv(items, 128) : 4096;
+  hipLaunchKernelGGL((attn_bwd_delta_kernel<T, D>), dim3((unsigned)blocks, (unsigned)batch), dim3(256), 0, st, p);
   const int64_t ndkv = cdiv(max_sk, 32 * KG) * p.hk * p.hsplit, ndq = cdiv(p.max_sq, 32 * RG) * p.hq;
   hipLaunchKernelGGL((attn_bwd_both_tile_kernel<T, D, RG, SPLIT, KG, QSPLIT, WPS>), dim3((unsigned)((ndkv + ndq) * batch)),
                      dim3(64 * RG * SPLIT), 0, st, p, (int)ndkv, (int)ndq, batch);

@@ -11,7 +11,8 @@
 // spilled (52 bytes a lane), read back by 5 loads in the loop.
 // Measured against the register-staged kernels that these head dims ran before, forward, causal: 16 heads x 2 x 512,
 // head dim 64 15.5 -> 9.4 us; 32 query / 8 kv heads x 4096, head dim 64 192 -> 94, 96 272 -> 132, 256 910 -> 329 us; 16
-// heads x 2048, head dim 192 324 -> 56 us.
+// heads x 2048, head dim 192 324 -> 56 us.  With the wait for Q in front of the loop (loaded_here): 16 x 2 x 512 10.0 -> 8.5 us
+// with its launch, 16 x 1024 12.5 -> 11.1, head dim 192 32 -> 29.5 us.
 #include "attn_tile.h"
 
 namespace dh {
@@ -84,11 +85,11 @@ __global__ void __launch_bounds__(64 * RG * SPLIT, WPS) attn_fwd_tile_kernel(con
     if (tile < ntiles) copy_tile<T, D, RPW>(cp_g, cp_stride, tile * BN + cp_r0, sk, cp_dst + (uint32_t)((it & 1) * STAGEB), cl, lane);
   };
   if (niter > 0) issue(0);
-  dma_wait_all();
-  __syncthreads();
-
+  if constexpr (D < 256 || RG == 2) loaded_here(Qf);        // (more of them would be spilled in the 128-row form at 256)
 #pragma unroll 1
   for (int it = 0; it < niter; ++it) {
+    dma_wait_all();
+    __syncthreads();   // this stage has landed, and everyone is done with the other one
     if (it + 1 < niter) issue(it + 1);
     const int tile = it * SPLIT + sp, n0 = tile * BN;
     if (tile < ntiles && !(causal && n0 > wrow0 + 31)) {
@@ -146,9 +147,8 @@ __global__ void __launch_bounds__(64 * RG * SPLIT, WPS) attn_fwd_tile_kernel(con
         for (int t = 0; t < D / 32; ++t)
           O[t] = M::mma(tr_frag<T, D>(vt, tl, t, s), Pb[s], O[t]);
     }
-    dma_wait_all();
-    __syncthreads();   // the next stage has landed, and everyone is done with the current one
   }
+  __syncthreads();
 
   // merge the splits: slot x = (split - 1) * RG + row group holds O, the m and l planes follow the slots
   float *xo = reinterpret_cast<float *>(sAll), *xml = xo + (SPLIT - 1) * RG * SLOTF;
