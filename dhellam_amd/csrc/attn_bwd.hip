@@ -1079,10 +1079,8 @@ namespace dh {
 // Query heads of a kv head are split over workgroups (each with fp32 partial dK / dV that a second kernel adds up)
 // only as far as it takes to give every compute unit one workgroup: beyond that the partials cost more than the
 // finer grain gives (ring step, 32 q / 8 kv heads: 4 splits 669 us, 2 splits 633 us, none 609 us).
-static int pick_hsplit(int max_sk, int batch, int hq, int hk, int bn) {
+static int pick_hsplit(int64_t blocks, int hq, int hk) {
   const int ratio = hq / hk;
-  if (ratio == 1) return 1;
-  const int64_t blocks = cdiv(max_sk, bn) * hk * batch;
   int hsplit = 1;
   for (int s = 1; s <= ratio; ++s)
     if (ratio % s == 0 && blocks * s <= 256) hsplit = s;
@@ -1143,7 +1141,7 @@ static bool bwd_short(int max_sq, int max_sk, int causal, int64_t total_q, int h
 
 // Key splits of a GQA group over workgroups.  The hand-ordered causal dK/dV kernel takes two key tiles a workgroup.
 static int bwd_hsplit(int max_sk, int batch, int hq, int hk, bool paired) {
-  return pick_hsplit(paired ? (max_sk + 1) / 2 : max_sk, batch, hq, hk, DKV_ROWS);
+  return pick_hsplit(cdiv(paired ? (max_sk + 1) / 2 : max_sk, DKV_ROWS) * hk * batch, hq, hk);
 }
 
 // Whether dK/dV and dQ go into one launch of the tile kernels, behind the delta kernel (2 us).  Either pass alone leaves
@@ -1163,21 +1161,25 @@ static int bwd_hsplit(int max_sk, int batch, int hq, int hk, bool paired) {
 //   causal: 8 x 1500 62 / 84, 32 x 512 36 / 41.
 // A group split eight ways from 512 rows on (8 query / 1 kv head x 1024: 58 / 46) and rectangular calls that are not
 // causal stay with the hand-ordered kernels: callers size the workspace there to choose between their two forms of dQ.
-static bool bwd_both_pays(int batch, int max_sq, int max_sk, int64_t total_q, int64_t total_k, int hq, int hk, int d, int causal) {
-  if (max_sq <= 0 || max_sk <= 0) return false;
+// A group that is left in pieces of several heads makes dK/dV's workgroups that much longer: from 512 rows on not here.  One
+// long sequence among short ones, whole calls, hand-ordered / here with the splits of the grid laid out for the longest / with
+// those of the work: 12 query / 4 kv heads x 791 + 76 + 32 77 / 86 / 57, 4 / 2 x 2746 + 7 135 / 168 / 117.
+struct BwdBoth { bool pays; int hsplit; };      // key splits of a GQA group: by the workgroups with work
+static BwdBoth bwd_both(int batch, int max_sq, int max_sk, int64_t total_q, int64_t total_k, int hq, int hk, int d, int causal) {
+  if (max_sq <= 0 || max_sk <= 0) return {false, 1};
   auto tiles = [&](int longest, int64_t total) {
     const int64_t grid = cdiv(longest, 64) * batch, real = total / 64 + batch;
     return grid < real ? grid : real;
   };
-  const int hs = bwd_hsplit(max_sk, batch, hq, hk, false);
+  const int hs = pick_hsplit(tiles(max_sk, total_k) * hk, hq, hk);
   const int64_t a = tiles(max_sq, total_q) * hq, b = tiles(max_sk, total_k) * hk * hs;
   if (d == 128) {
-    if (!causal) return a + b <= 256 && max_sq == max_sk;
-    if (max_sq >= 512 && hs >= 8) return false;
-    return a + b <= 384 || (a + b <= 512 && max_sq >= 256 && max_sq < 1024);
+    if (max_sq >= 512 && (hs >= 8 || hs < hq / hk)) return {false, hs};
+    if (!causal) return {a + b <= 256 && max_sq == max_sk, hs};
+    return {a + b <= 384 || (a + b <= 512 && max_sq >= 256 && max_sq < 1024), hs};
   }
-  if (a + b <= (causal ? 384 : 256)) return true;
-  if (causal && max_sq >= 1024) return b <= 256;
+  if (a + b <= (causal ? 384 : 256)) return {true, hs};
+  if (causal && max_sq >= 1024) return {b <= 256, hs};
   // rounds of 256, in units of a dQ workgroup's time: one pass after the other, and both with the dK/dV workgroups first
   const double rho = 1.3 * (hq / hk / hs), apart = (double)cdiv(a, 256) + (double)cdiv(b, 256) * rho;
   const int64_t full = b / 256, more = b % 256;
@@ -1186,7 +1188,7 @@ static bool bwd_both_pays(int batch, int max_sq, int max_sk, int64_t total_q, in
     return (x > 0 ? (int64_t)x * (256 - more) : 0) + (y > 0 ? (int64_t)y * more : 0);
   };
   const double t = apart / 1.2;
-  return t >= (double)cdiv(b, 256) * rho && room(t) >= a;
+  return {t >= (double)cdiv(b, 256) * rho && room(t) >= a, hs};
 }
 
 // What one 16-bit call runs.
@@ -1195,17 +1197,19 @@ struct AttnBwdRoute {
   bool hand_dkv, hand_dq;      // head dim 128's hand-ordered kernels
   bool big_dq;       // 128-row query tiles in dQ
   bool both;         // dK/dV and dQ in one launch of the tile kernels, behind the delta kernel
+  int hsplit;        // workgroups that share a GQA group in dK/dV
 };
 static AttnBwdRoute attn_bwd_route(int batch, int max_sq, int max_sk, int64_t total_q, int64_t total_k, int hq, int hk, int d,
                                    int causal, bool room_for_ds) {
-  const bool both = bwd_both_pays(batch, max_sq, max_sk, total_q, total_k, hq, hk, d, causal);
-  const bool short_rows = d == 128 && (both || bwd_short(max_sq, max_sk, causal, total_q, hq)), big = dq_big_grid(batch, max_sq, hq, causal);
+  const BwdBoth both = bwd_both(batch, max_sq, max_sk, total_q, total_k, hq, hk, d, causal);
+  const bool short_rows = d == 128 && (both.pays || bwd_short(max_sq, max_sk, causal, total_q, hq)), big = dq_big_grid(batch, max_sq, hq, causal);
   AttnBwdRoute r;
   r.keep_ds = room_for_ds && max_sk > 0 && !short_rows;
   r.hand_dkv = d == 128 && !short_rows;
   r.hand_dq = r.hand_dkv && (!causal || !big || attn_causal_fills(max_sq, hq, batch, total_q));
   r.big_dq = r.hand_dq ? big : d <= 128 && attn_wgs(max_sq, 128, hq, batch, 0) >= 2 * 256;
-  r.both = both && !r.big_dq;
+  r.both = both.pays && !r.big_dq;
+  r.hsplit = r.both ? both.hsplit : bwd_hsplit(max_sk, batch, hq, hk, d == 128 && causal);
   return r;
 }
 
@@ -1391,7 +1395,7 @@ static int attn_bwd_entry(const void *dout, const void *q, const void *k, const 
   p.ds = route.keep_ds ? (void *)ds_ws : nullptr;
   p.ds_nqt = 2 * (int)cdiv(max_seqlen_q, 64);
   p.ds_nkb = 2 * (int)cdiv(max_seqlen_k < total_k ? max_seqlen_k : total_k, 64) + 1;
-  p.hsplit = bwd_hsplit(max_seqlen_k, batch, hq, hk, d == 128 && causal && !route.both);
+  p.hsplit = route.hsplit;
   p.dk_part = nullptr;
   p.dv_part = nullptr;
   if (p.hsplit > 1) {
