@@ -14,6 +14,8 @@
 // The product is formed as C^T (weights in the MFMA A slot) so that each lane
 // ends up with runs of 4 consecutive output columns of one row: 8-byte stores.
 // Group row ranges are read on the device from the offsets table.
+#include <cmath>
+
 #include "mma.h"
 #include <atomic>
 
@@ -578,6 +580,11 @@ __global__ void __launch_bounds__(256) gg_split_reduce_kernel(const GGParams p, 
 // 102 -> 42.  In the steady state two workgroups of a compute unit take 0.95 us per slice of two 128x128 tiles
 // (1.13 PFLOP/s, 27 bytes per cycle and compute unit out of L2); the start and end of a round of tiles cost 5 us.
 //
+// With more 128x128 tiles than that, a single stage and four workgroups a compute unit (34 KB of LDS, at most 128 registers) hide
+// loads and stores behind each other better than two of two stages: a workgroup waits for each of its slices, three others
+// work meanwhile.  Weight gradients of few rows, mostly stores: 16 experts of 72 rows, 5632 x 4096 236 -> 180 us (3.1 -> 4.1 TB/s),
+// 2816 x 4096 118 -> 96; 8 x 250 rows, 5632 x 1024 44 -> 38, 1024 rows 107 -> 95.
+//
 // LDS: a k-contiguous operand as [rows][64 k] (128-byte rows, 16-byte chunk XOR (row / 2) % 8), a k-strided one as
 // [64 k][128 columns] (256-byte rows, chunk XOR 4 (k % 4) + (k / 4) % 4), as in grouped_gemm_w8_kernel; a wavefront
 // copies 1 KB per instruction, so the XOR is applied to the global chunk that a lane fetches.  Buffer descriptors cut
@@ -595,15 +602,17 @@ __host__ __device__ __forceinline__ int gg_t_pieces(int slots, int tiles, int ns
   return pc < 2 || nsl - nsl / pc < 12 ? 1 : pc;
 }
 
-template <int FORM, int BM, int BN> struct GGT {
+template <int FORM, int BM, int BN, int ST = 0> struct GGT {
   static constexpr bool AKS = FORM == 2, BKS = FORM >= 1;
   static constexpr int NW = BN / 32;                            // wavefronts
   static constexpr int WM = BM == 32 ? 1 : 2, WN = NW / WM;     // over the tile
   static constexpr int MI = BM / (32 * WM), NI = BN / (32 * WN); // 32x32 blocks of a wavefront
-  static constexpr int NST = BN == 256 ? 3 : BM == 128 ? 2 : BM == 64 ? 3 : 4;  // stages: 144 KB; 64, 72, 80 KB
+  static constexpr int NST = ST ? ST : BN == 256 ? 3 : BM == 128 ? 2 : BM == 64 ? 3 : 4;  // stages: 144 KB; 64, 72, 80 KB
   static constexpr int ABYTES = BM * 128, STAGE = ABYTES + BN * 128;
   static constexpr int ACPW = BM / (8 * NW), BCPW = BN / (8 * NW), CPW = ACPW + BCPW;   // copies of a wavefront per slice
-  static constexpr int PER_CU = BN == 256 ? 1 : 2;              // workgroups that share a compute unit
+  static constexpr int PER_CU = ST == 1 ? 4 : BN == 256 ? 1 : 2; // workgroups that share a compute unit
+  static constexpr int EP = NI * 64 + 8, EPB = NW * 32 * MI * EP;   // row of a wavefront's block on its way to c in bytes, and all of them
+  static constexpr int LDS = NST * STAGE > EPB ? NST * STAGE : EPB;
 };
 
 struct GGUnit { int g, rb, re, tm, tn, s0, s1, piece; bool on; };   // slices s0..s1 of tile (tm, tn) of group g
@@ -651,14 +660,14 @@ __device__ __forceinline__ GGUnit gg_t_unit(const GGParams &p, int id) {
   return u;
 }
 
-template <typename T, int FORM, int BM, int BN>
-__global__ void __launch_bounds__(2 * BN, 2) grouped_gemm_t_kernel(const GGParams p) {
-  using C = GGT<FORM, BM, BN>;
+template <typename T, int FORM, int BM, int BN, int ST>
+__global__ void __launch_bounds__(2 * BN, ST == 1 ? 4 : 2) grouped_gemm_t_kernel(const GGParams p) {
+  using C = GGT<FORM, BM, BN, ST>;
   using M = Mma<T>;
   using Frag = typename M::Frag;
   constexpr bool AKS = C::AKS, BKS = C::BKS;
   constexpr int MI = C::MI, NI = C::NI;
-  __shared__ __attribute__((aligned(1024))) unsigned char smem[C::NST * C::STAGE];
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[C::LDS];
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 31, hh = lane >> 5;
@@ -781,7 +790,7 @@ __global__ void __launch_bounds__(2 * BN, 2) grouped_gemm_t_kernel(const GGParam
   int st = 0;
   auto slice = [&](auto morec, int s) {
     constexpr bool MORE = decltype(morec)::value;                 // slice s + NST - 1 exists
-    if (MORE || s + C::NST - 2 < cnt) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((C::NST - 2) * C::CPW) : "memory");
+    if (C::NST > 1 && (MORE || s + C::NST - 2 < cnt)) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(C::NST > 1 ? (C::NST - 2) * C::CPW : 0) : "memory");
     else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
     const uint32_t cur = lds0 + (uint32_t)(st * C::STAGE);
     const uint32_t free = lds0 + (uint32_t)((st == 0 ? C::NST - 1 : st - 1) * C::STAGE);   // stage of slices s - 1 and s + NST - 1
@@ -810,10 +819,21 @@ __global__ void __launch_bounds__(2 * BN, 2) grouped_gemm_t_kernel(const GGParam
     }
   };
   int s = 0;
+  if constexpr (C::NST == 1) {                                    // what is in flight is the other workgroups' business
 #pragma unroll 1
-  for (; s + C::NST - 1 < cnt; ++s) slice(std::true_type{}, s);
+    for (; s < cnt; ++s) {
+      if (s > 0) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      descriptors(u.s0 + s);
+#pragma unroll
+      for (int x = 0; x < C::CPW; ++x) copy(x, u.s0 + s, lds0);
+      slice(std::false_type{}, s);
+    }
+  } else {
 #pragma unroll 1
-  for (; s < cnt; ++s) slice(std::false_type{}, s);
+    for (; s + C::NST - 1 < cnt; ++s) slice(std::true_type{}, s);
+#pragma unroll 1
+    for (; s < cnt; ++s) slice(std::false_type{}, s);
+  }
 
   if (u.piece >= 0) {                                             // fp32 piece in accumulator layout, 1 KB per instruction
     float *dst = p.ws + (size_t)u.piece * (BM * BN) + (size_t)(w * MI * NI) * 1024 + (size_t)lane * 4;
@@ -852,8 +872,7 @@ __global__ void __launch_bounds__(2 * BN, 2) grouped_gemm_t_kernel(const GGParam
     return;
   }
   // whole row segments of the wavefront's block through its own LDS region (rows 8 bytes apart in the banks)
-  constexpr int EP = NI * 64 + 8, LPR = NI * 4;                   // region row in bytes, lanes per row of 16-byte pieces
-  static_assert(C::NW * 32 * MI * EP <= C::NST * C::STAGE, "staging fits in the stages");
+  constexpr int EP = C::EP, LPR = NI * 4;                         // region row in bytes, lanes per row of 16-byte pieces
   __syncthreads();                                                // everyone is done with the stages
   unsigned char *ep = smem + w * (32 * MI * EP);
 #pragma unroll
@@ -1045,9 +1064,9 @@ static int launch_gg_w8(GGParams p, int64_t m_extent, void *workspace, size_t wo
   return DH_OK;
 }
 
-template <typename T, int FORM, int BM, int BN>
+template <typename T, int FORM, int BM, int BN, int ST = 0>
 static int launch_gg_t(GGParams p, int64_t m_extent, void *workspace, size_t workspace_bytes, hipStream_t st) {
-  using C = GGT<FORM, BM, BN>;
+  using C = GGT<FORM, BM, BN, ST>;
   constexpr int BLOCKS = BM * BN / 1024;
   int cus = 0;
   const int rc = gg_compute_units(cus);
@@ -1076,10 +1095,17 @@ static int launch_gg_t(GGParams p, int64_t m_extent, void *workspace, size_t wor
     }
   }
   DH_CHECK(grid > 0 && grid < (1ll << 31), "grouped GEMM: too many tiles");
-  hipLaunchKernelGGL((grouped_gemm_t_kernel<T, FORM, BM, BN>), dim3((unsigned)grid), dim3(2 * BN), 0, st, p);
+  hipLaunchKernelGGL((grouped_gemm_t_kernel<T, FORM, BM, BN, ST>), dim3((unsigned)grid), dim3(2 * BN), 0, st, p);
   if (reduce > 0)
     hipLaunchKernelGGL((gg_t_reduce_kernel<T, FORM, BM, BN>), dim3((unsigned)cdiv(reduce * BLOCKS, 4)), dim3(256), 0, st, p);
   return DH_OK;
+}
+
+// Row tiles of `bm` that rows in `groups` uneven groups come to: the mean of groups of the average size and of one standard
+// deviation of a random routing above and below it.
+static double gg_tiles(int64_t rows, int groups, int bm) {
+  const double avg = (double)rows / groups, dev = groups > 1 ? std::sqrt(avg) : 0;
+  return groups * (std::ceil((avg - dev) / bm) + std::ceil(avg / bm) + std::ceil((avg + dev) / bm)) / 3;
 }
 
 template <typename T, int FORM>
@@ -1092,6 +1118,9 @@ static int dispatch_gg_t(const GGParams &p, int64_t m_extent, void *workspace, s
     return DH_OK;
   }
   if constexpr (FORM == 2) {
+    // (the one-stage form: above.  Accumulating, only products of few tiles come here)
+    if (!p.accumulate && p.groups * cdiv(p.m_dim, 128) * cdiv(p.n_dim, 128) > 512)
+      return launch_gg_t<T, FORM, 128, 128, 1>(p, m_extent, workspace, workspace_bytes, st);
     return launch_gg_t<T, FORM, 128, 128>(p, m_extent, workspace, workspace_bytes, st);
   } else {
     // Rows per tile.  Small ones where a group's rows fit one tile (weights are then read once, by more workgroups the
@@ -1113,50 +1142,57 @@ static int dispatch_gg_t(const GGParams &p, int64_t m_extent, void *workspace, s
     // 202 -> 178 us); short ones cannot hide the first loads and last stores of their single workgroup per compute unit
     // (16384 rows, n = 1408 of 1024: 60 -> 71 us)
     if (p.k_dim >= 1536) return launch_gg_t<T, FORM, 128, 256>(p, m_extent, workspace, workspace_bytes, st);
+    // more tiles than two workgroups on every compute unit take: the one-stage form, us two stages / one, 8 groups, n = 5632 of
+    // 1024: 128 rows a group (528 tiles) 36 / 31, 1024 125 / 105; 64 groups, n = 1408 of 1024: 72 rows (748) 39 / 37, 256 79 / 67; 16
+    // groups, n = 1408 of 512: 256 rows (440) 14.5 / 16.3, 384 (616) 22.4 / 19.8.  Of longer reductions 128x256 tiles run better
+    if (gg_tiles(m_extent, p.groups, 128) * (double)cdiv(p.n_dim, 128) > 512)
+      return launch_gg_t<T, FORM, 128, 128, 1>(p, m_extent, workspace, workspace_bytes, st);
     return launch_gg_t<T, FORM, 128, 128>(p, m_extent, workspace, workspace_bytes, st);
   }
 }
 
-// NT / NN: whether 256x256 tiles, one workgroup per compute unit, are the faster ones.  Both kernels run in rounds of equal
-// tiles, so the two times follow from the number of rounds (the last one of the 256x256 tiles is split along k where it is at
-// most half full) and of k slices; the constants (us) are a least-squares fit to 330 products of 1 to 64 groups, 192 to 4096 rows
-// a group, n and k from 512 to 8192, which the formulas meet to 13 and 11 %.  What is picked is 0.4 % from the better kernel on
-// average (by a count of tiles and a shortest k, as before: 1.8 %).  256x256 / smaller, us: 8 groups of 512 rows, n = 2816 of 2048
-// 50 / 63 (176 tiles); 8 x 1024, n = 5632 of 1024 96 / 113 (704 tiles), n = 3072 of 1024 73 / 62 (384: the second round half
-// empty), n = 1408 of 1024 33 / 35 (192).  Groups of fewer rows leave most of a tile empty.
+// NT / NN: whether 256x256 tiles, one workgroup per compute unit, are the faster ones.  All kernels run in rounds of equal
+// tiles, so the times follow from the number of rounds (the last one of the 256x256 tiles is split along k where it is at
+// most half full; the one-stage form's rounds run into each other) and of k slices; the constants (us) are least-squares fits
+// to 330 products of 1 to 64 groups, 192 to 4096 rows a group, n and k from 512 to 8192, which the formulas meet to 13 and 11 %.
+// Rows that are routed at random fill more tiles than groups of their average (gg_tiles).  256x256 / smaller, us: 16 groups of 128
+// rows, n = 4096 of 2816 93 / 104, of 72 rows 86 / 76, of 384 154 / 164 (groups of 360 to 410 rows: 2 tiles of 256, 3 or 4 of 128); 2 x
+// 640, n = 7168 of 4096 80 / 112, 2 x 256 52 / 44; 8 x 1024, n = 5632 of 1024 126 / 105, n = 1024 of 2816 62 / 80.
 static bool gg_w8_pays(int64_t rows, int groups, int64_t n, int64_t k) {
   const int64_t avg = rows / groups;
-  if (avg < 192) return false;
+  if (avg < 96) return false;
   const double ns = (double)cdiv(k, 64);
-  const int64_t tiles = groups * cdiv(avg, 256) * cdiv(n, 256), rem = tiles % 256;
+  const int64_t tiles = (int64_t)std::ceil(gg_tiles(rows, groups, 256)) * cdiv(n, 256), rem = tiles % 256;
   const double round = 14.3 + 1.357 * ns;
   double big = 4.6 + (double)(tiles / 256) * round;
   if (rem > 128) big += round;
   else if (rem > 0) big += 26.3 + 1.357 * (ns > 1 ? ns / (double)(256 / rem < ns ? 256 / rem : ns) : 1.0);
   double small;
   if (k >= 1536) {
-    const int64_t t = groups * cdiv(avg, 128) * cdiv(n, 256);
-    small = 2 * t <= 256 ? 15.4 + 0.932 * ns * (double)t / 256 : (double)cdiv(t, 256) * (9.4 + 0.932 * ns);
+    const int64_t t = (int64_t)std::ceil(gg_tiles(rows, groups, 128)) * cdiv(n, 256);
+    if (2 * t <= 256) small = 15.4 + 0.932 * ns * (double)t / 256;
+    else if (t < 256) small = 9.4 + 0.932 * ns * (0.25 + 0.75 * (double)t / 256);
+    else small = (double)cdiv(t, 256) * (9.4 + 0.932 * ns);
   } else {
-    const int64_t t = groups * cdiv(avg, 128) * cdiv(n, 128);
-    const double part = (double)t / 512 > 8 / ns ? (double)t / 512 : 8 / ns;
-    small = 2 * t <= 512 ? 6 + 1.205 * ns * part : (double)cdiv(t, 512) * 1.205 * ns;
+    const double t = gg_tiles(rows, groups, 128) * (double)cdiv(n, 128), part = t / 512 > 8 / ns ? t / 512 : 8 / ns;
+    small = 2 * t <= 512 ? 6 + 1.205 * ns * part : t <= 512 ? 1.205 * ns : 6 + 2.3 * ns * t / 1024;
   }
   return big < small;
 }
 
-// The same for TN, its constants from 60 products of 250 to 2048 rows a group (what is picked is 0.9 % from the better kernel on
-// average; below six slices, where uneven groups add some, 10 % is asked for); us, 256x256 / 128x128 tiles: 8 groups of 250 rows, 7168 x 4096 184 / 208, 5632 x 1024 44 / 41; of 1024 rows 443 / 575 and
-// 94 / 113, 3072 x 1024 59 / 62, of 512 rows 39 / 36.  Accumulating, which the smaller tiles do with 8-byte accesses, from two
-// thirds of a tile for every compute unit on: one group of 256 rows, 8192 x 3584 32 / 54, 1280 x 8192 15 / 24, but 8192 x 1024
-// (128 tiles) 15 / 16, of 4096 rows 84 / 74.
+// The same for TN (constants from 80 products of 16 to 2048 rows a group; below six slices, where uneven groups add some, 10 % is
+// asked for); us, 256x256 / 128x128 tiles: 16 groups of 5632 x 4096: 192 rows 275 / 289, 512 452 / 496, 1024 726 / 844; 8 groups of 5632 x
+// 1024: 256 rows 47 / 41, 1024 100 / 104.  Accumulating, which the smaller tiles do with 8-byte accesses, from two thirds of a
+// tile for every compute unit on: 16 groups of 5632 x 4096: 16 rows 267 / 569, 256 364 / 684; of 1408 x 512 (192 tiles) 11 / 20, 18 / 27; one
+// group of 16 rows, 4096 x 4096 13 / 33, of 256 rows, 1280 x 8192 15 / 24, but 8192 x 1024 (128 tiles) 15 / 16, of 4096 rows 84 / 74.
 static bool gg_w8_tn_pays(int64_t rows, int groups, int64_t m, int64_t n, int accumulate) {
   const int64_t avg = rows / groups;
-  if (avg < 192) return false;
   const double ns = (double)cdiv(avg, 64);
   const int64_t tiles = groups * cdiv(m, 256) * cdiv(n, 256), small = groups * cdiv(m, 128) * cdiv(n, 128);
   if (accumulate && tiles >= 160) return true;
-  return (double)cdiv(tiles, 256) * (8.5 + 1.38 * ns) * (avg < 384 ? 1.1 : 1.0) < 0.8 + (double)small / 512 * (3.5 + 1.11 * ns);
+  if (avg < 192) return false;
+  return (double)cdiv(tiles, 256) * (8.5 + 1.38 * ns) * (avg < 384 ? 1.1 : 1.0) <
+         (accumulate || small <= 512 ? 0.8 + (double)small / 512 * (3.5 + 1.11 * ns) : (double)small / 1024 * (6.3 + 1.85 * ns));
 }
 
 static int gg_common_checks(const void *a, const void *b, void *c, const int32_t *offs, int groups, int dtype) {

@@ -423,11 +423,12 @@ bool dgrad_grouped(int64_t t, int64_t n, int64_t k) {
 // better of its two layouts) / here, N, K at T = 200, 1000, 1904, 4096: 7168, 8192 76 / 62, 154 / 125, 244 / 197, 411 / 378;
 // 8192, 3584 40 / 32, 79 / 61, 124 / 97, 205 / 190; 32000, 2048 at 512, 1064, 4096 93 / 85, 164 / 135, 442 / 432; 1280, 8192 (160
 // tiles) 18 / 15, 40 / 30, 54 / 45, but 80 / 84: few tiles of many whole slices stay with the library, as does 8192, 1024 (128 tiles)
-// 14 / 16, 31 / 29, 44 / 44, 69 / 83.  Small weights of few rows: 3072, 1024 at 64, 256, 368 10.4 / 7.6, 10.5 / 9.4, 12.4 / 10.5, at 512
+// 14 / 16, 31 / 29, 44 / 44, 69 / 83.  Few rows, T = 16, 64, 100: 32000, 4096 126 / 96, 121 / 103, 145 / 112; 4096, 4096 18 / 13, 16 / 14,
+// 21 / 15; 1280, 8192 14 / 11, 13 / 11, 26 / 12.  Small weights of few rows: 3072, 1024 at 64, 256, 368 10.4 / 7.6, 10.5 / 9.4, 12.4 / 10.5, at 512
 // 12.2 / 12.4.
 bool wgrad_grouped(int64_t t, int64_t n, int64_t k) {
   const int64_t tiles = (n + 255) / 256 * ((k + 255) / 256);
-  if (t >= 192 && tiles >= 160) return !(tiles < 224 && t % 64 == 0 && t >= 2048) && 2 * t * std::max(n, k) < (int64_t)1 << 31;
+  if (t > 0 && tiles >= 160) return !(tiles < 224 && t % 64 == 0 && t >= 2048) && 2 * t * std::max(n, k) < (int64_t)1 << 31;
   return t > 0 && t <= 384 && n * k <= 3200000;
 }
 

@@ -566,3 +566,51 @@ def test_grouped_gemm_tn_256_tiles(dtype):
     moe.grouped_gemm_tn(a, b, offs, out=acc, accumulate=True)
     assert_close(acc, ref + base.float(), dtype, "TN accumulate")
     assert torch.equal(acc[1], base[1]), "accumulating an empty group must leave the output as it was"
+
+
+@pytest.mark.parametrize("form", ["nt", "nn", "tn"])
+@pytest.mark.parametrize("rows,n,k", [
+    ([0, 1, 63, 64, 65, 127, 128, 129, 130, 255, 257, 300] * 4, 1000, 72),      # tiles that end anywhere; a k tail
+    ([131] * 47 + [5], 1096, 200), ([140, 120] * 30, 1408, 1024),
+])
+def test_grouped_gemm_one_stage_tiles(form, rows, n, k):
+    """More 128x128 tiles than two workgroups on every compute unit take: the form with one stage.  |error| against fp64 of the
+    same bf16 inputs: one bf16 rounding of the result and fp32 sums of K products."""
+    from dhellam_amd.operators import moe
+    g = torch.Generator().manual_seed(7)
+    G, total = len(rows), sum(rows)
+    offs = torch.tensor([0] + rows).cumsum(0).to(torch.int32)
+    mk = lambda *s: torch.randn(*s, generator=g).bfloat16()
+    if form == "tn":
+        a, b = mk(total, n), mk(total, k)
+        got = moe.grouped_gemm_tn(a.cuda(), b.cuda(), offs.cuda())
+        pairs = [(a[x:y].double().t() @ b[x:y].double(), a[x:y].double().abs().t() @ b[x:y].double().abs()) for x, y in zip(offs[:-1], offs[1:])]
+        out = got.cpu().double()
+    else:
+        a, w = mk(total, k), mk(G, n, k)
+        got = (moe.grouped_gemm_nt(a.cuda(), w.cuda(), offs.cuda()) if form == "nt"
+               else moe.grouped_gemm_nn(a.cuda(), w.transpose(1, 2).contiguous().cuda(), offs.cuda())).cpu().double()
+        pairs = [(a[x:y].double() @ w[i].double().t(), a[x:y].double().abs() @ w[i].double().abs().t())
+                 for i, (x, y) in enumerate(zip(offs[:-1], offs[1:]))]
+        out = [got[x:y] for x, y in zip(offs[:-1], offs[1:])]
+    depth = max(rows) if form == "tn" else k
+    for have, (want, mass) in zip(out, pairs):
+        assert ((have - want).abs() <= want.abs() * 2.0 ** -8 + mass * depth * 2.0 ** -24 + 1e-30).all()
+
+
+@pytest.mark.parametrize("rows", [[0, 1, 63, 64, 65, 7, 16, 130], [3] * 8])
+def test_grouped_gemm_tn_accumulates_few_rows(rows):
+    """Accumulating weight gradients of few rows on the 256x256 tiles: c += a^T b with one rounding; an empty group leaves its c."""
+    from dhellam_amd.operators import moe
+    g = torch.Generator().manual_seed(8)
+    m, n = 1304, 1096
+    offs = torch.tensor([0] + rows).cumsum(0).to(torch.int32)
+    a, b, c = (torch.randn(*s, generator=g).bfloat16() for s in ((sum(rows), m), (sum(rows), n), (len(rows), m, n)))
+    got = c.cuda()
+    moe.grouped_gemm_tn(a.cuda(), b.cuda(), offs.cuda(), out=got, accumulate=True)
+    for i, (x, y) in enumerate(zip(offs[:-1], offs[1:])):
+        p, mass = a[x:y].double().t() @ b[x:y].double(), a[x:y].double().abs().t() @ b[x:y].double().abs()
+        want = c[i].double() + p
+        assert ((got[i].cpu().double() - want).abs() <= want.abs() * 2.0 ** -8 + mass * max(rows) * 2.0 ** -24 + 1e-30).all()
+        if x == y:
+            assert torch.equal(got[i].cpu(), c[i])
