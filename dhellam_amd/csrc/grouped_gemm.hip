@@ -1157,10 +1157,12 @@ static int dispatch_gg_t(const GGParams &p, int64_t m_extent, void *workspace, s
 // to 330 products of 1 to 64 groups, 192 to 4096 rows a group, n and k from 512 to 8192, which the formulas meet to 13 and 11 %.
 // Rows that are routed at random fill more tiles than groups of their average (gg_tiles).  256x256 / smaller, us: 16 groups of 128
 // rows, n = 4096 of 2816 93 / 104, of 72 rows 86 / 76, of 384 154 / 164 (groups of 360 to 410 rows: 2 tiles of 256, 3 or 4 of 128); 2 x
-// 640, n = 7168 of 4096 80 / 112, 2 x 256 52 / 44; 8 x 1024, n = 5632 of 1024 126 / 105, n = 1024 of 2816 62 / 80.
+// 640, n = 7168 of 4096 80 / 112, 2 x 256 52 / 44; 8 x 1024, n = 5632 of 1024 126 / 105, n = 1024 of 2816 62 / 80.  Many groups of few rows
+// read their weights too slowly in large tiles for the formula: 64 groups, n = 1024 of 2048: 128 rows 102 / 81, 256 167 / 112, 384 150
+// / 152, 640 181 / 243.
 static bool gg_w8_pays(int64_t rows, int groups, int64_t n, int64_t k) {
   const int64_t avg = rows / groups;
-  if (avg < 96) return false;
+  if (avg < 96 || avg < 6 * groups) return false;
   const double ns = (double)cdiv(k, 64);
   const int64_t tiles = (int64_t)std::ceil(gg_tiles(rows, groups, 256)) * cdiv(n, 256), rem = tiles % 256;
   const double round = 14.3 + 1.357 * ns;
