@@ -20,28 +20,44 @@ constexpr int MOE_MAX_E = 64;
 constexpr int MOE_MAX_K = 8;
 constexpr int SORT_ITEMS = 1024;  // assignments per block (4 rounds of 256)
 
+// Top K of E logits a token, E lanes (the next power of two) holding one each.  In every round the best of what is left: the
+// largest, of equals the lowest expert id, a NaN only where the lowest id that is left holds one (the rule of a scan that
+// starts there and moves on to what is greater).  A thread a token, scanning its row K times, was a chain of K E dependent
+// loads on a few workgroups: 3316 tokens of 64 experts, 8 of them chosen, 78 -> 10 us, 1914 of 16, 4 chosen, 11 -> 5, 8192 of 8, 2
+// chosen, 6.8 -> 4.8.
+template <int G>
 __global__ void __launch_bounds__(256)
 moe_route_kernel(const float *__restrict__ logits, int32_t *__restrict__ topk_idx, float *__restrict__ gates,
                  int64_t tokens, int E, int K) {
-  for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < tokens; t += (int64_t)gridDim.x * 256) {
-    const float *row = logits + t * E;
+  const int e = threadIdx.x % G, group = (threadIdx.x & 63) / G * G;             // expert; first lane of the token's
+  for (int64_t t0 = (int64_t)blockIdx.x * (256 / G); t0 < tokens; t0 += (int64_t)gridDim.x * (256 / G)) {
+    const int64_t t = t0 + threadIdx.x / G;
+    const float v = t < tokens && e < E ? logits[t * E + e] : 0.f;
+    const uint64_t nan = __ballot(v != v) >> group;                              // bit x: expert x of this token
     uint64_t taken = 0;
     float sel[MOE_MAX_K];
     int idx[MOE_MAX_K];
 #pragma unroll
     for (int j = 0; j < MOE_MAX_K; ++j) {
       if (j < K) {
-        int best = -1;
-        float bv = 0.f;
-        for (int e = 0; e < E; ++e) {
-          if ((taken >> e) & 1) continue;
-          const float v = row[e];
-          // strict > keeps the lowest expert id among equal values; NaN never wins
-          if (best < 0 || v > bv) {
-            best = e;
-            bv = v;
+        const int first = (int)__builtin_ctzll(~taken);
+        float bv = v;
+        int best = e;
+        if (e >= E || v != v || ((taken >> e) & 1)) {                            // no candidate: loses to all that are
+          bv = -INFINITY;
+          best = G;
+        }
+#pragma unroll
+        for (int d = G >> 1; d > 0; d >>= 1) {
+          const float ov = __shfl_xor(bv, d, 64);
+          const int oi = __shfl_xor(best, d, 64);
+          if (ov > bv || (ov == bv && oi < best)) {
+            bv = ov;
+            best = oi;
           }
         }
+        if ((nan >> first) & 1) best = first;
+        bv = __shfl(v, group + best, 64);
         taken |= (uint64_t)1 << best;
         sel[j] = bv;
         idx[j] = best;
@@ -55,12 +71,14 @@ moe_route_kernel(const float *__restrict__ logits, int32_t *__restrict__ topk_id
         ex[j] = expf(sel[j] - sel[0]);
         den += ex[j];
       }
+    if (t < tokens) {
 #pragma unroll
-    for (int j = 0; j < MOE_MAX_K; ++j)
-      if (j < K) {
-        topk_idx[t * K + j] = idx[j];
-        gates[t * K + j] = ex[j] / den;
-      }
+      for (int j = 0; j < MOE_MAX_K; ++j)
+        if (j < K && e == j) {
+          topk_idx[t * K + j] = idx[j];
+          gates[t * K + j] = ex[j] / den;
+        }
+    }
   }
 }
 
@@ -123,16 +141,22 @@ __device__ __forceinline__ void moe_rank_items(const int32_t *__restrict__ exper
                                                int64_t base, int64_t n, int E) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const uint64_t lt_mask = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+  int lg = 0;
+  while ((1 << lg) < E) ++lg;
   for (int r = 0; r < SORT_ITEMS / 256; ++r) {
     const int64_t i = base + r * 256 + threadIdx.x;
     int my = i < n ? expert_of[i] : -1;
-    if (my >= E) my = -1;  // an id outside [0, E) gets no place (its dest_row is -1)
-    int rank_in_wave = 0;
-    for (int e = 0; e < E; ++e) {
-      const uint64_t m = __ballot(my == e);
-      if (lane == 0) wcnt[w][e] = __popcll(m);
-      if (my == e) rank_in_wave = __popcll(m & lt_mask);
+    if (my >= E || my < 0) my = -1;  // an id outside [0, E) gets no place (its dest_row is -1)
+    // the lanes with the same expert: one ballot for every bit of the id
+    uint64_t same = __ballot(my >= 0);
+    for (int b = 0; b < lg; ++b) {
+      const uint64_t m = __ballot((my >> b) & 1);
+      same &= (my >> b) & 1 ? m : ~m;
     }
+    const int rank_in_wave = __popcll(same & lt_mask);
+    if (lane < E) wcnt[w][lane] = 0;
+    __builtin_amdgcn_wave_barrier();
+    if (my >= 0 && rank_in_wave == 0) wcnt[w][my] = __popcll(same);
     __syncthreads();
     if (my >= 0) {
       int pos = running[my] + rank_in_wave;
@@ -197,14 +221,20 @@ moe_sort_one_kernel(const int32_t *__restrict__ expert_of, int32_t *__restrict__
       }
     }
   };
+  // the 256 counters of an expert, by the next power of two's share of the threads, each of them reading its counters from a
+  // place of its own (the experts' counters lie on the same banks).  Together with
+  // the ballots a bit of the id (moe_rank_items; before: one an expert): 64 experts, 26528 items 36 -> 17 us, 16, 7656 13.5 -> 9.6,
+  // 8, 16384 16 -> 11.
+  int lg = 2;
+  while ((1 << lg) < E) ++lg;
+  const int parts = 256 >> lg, se = tid / parts, part = tid % parts;
   auto sums = [&](int *out) {
     __syncthreads();
-    for (int e = w; e < E; e += 4) {
-      int s = cnt[e * 256 + lane] + cnt[e * 256 + 64 + lane] + cnt[e * 256 + 128 + lane] + cnt[e * 256 + 192 + lane];
-#pragma unroll
-      for (int d = 32; d > 0; d >>= 1) s += __shfl_xor(s, d, 64);
-      if (lane == 0) out[e] = s;
-    }
+    int s = 0;
+    if (se < E)
+      for (int i = 0; i < 1 << lg; ++i) s += cnt[se * 256 + part + parts * ((i + se) & ((1 << lg) - 1))];
+    for (int d = parts >> 1; d > 0; d >>= 1) s += __shfl_xor(s, d, 64);
+    if (part == 0 && se < E) out[se] = s;
     __syncthreads();
   };
   if (blockIdx.x > 0) count(0, base);
@@ -487,10 +517,11 @@ extern "C" int dh_moe_route_topk(const float *logits, int32_t *topk_idx, float *
   DH_CHECK(k >= 1 && k <= MOE_MAX_K && k <= experts, "k=%d must be in [1, min(%d, experts)]", k, MOE_MAX_K);
   if (tokens == 0) return DH_OK;
   DH_CHECK(logits && topk_idx && gates, "null pointer");
-  int64_t blocks = cdiv(tokens, 256);
+  const int lanes = experts <= 8 ? 8 : experts <= 16 ? 16 : experts <= 32 ? 32 : 64;
+  int64_t blocks = cdiv(tokens, 256 / lanes);
   if (blocks > 4096) blocks = 4096;
-  hipLaunchKernelGGL(moe_route_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, logits, topk_idx,
-                     gates, tokens, experts, k);
+  const auto kernel = lanes == 8 ? moe_route_kernel<8> : lanes == 16 ? moe_route_kernel<16> : lanes == 32 ? moe_route_kernel<32> : moe_route_kernel<64>;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, logits, topk_idx, gates, tokens, experts, k);
   DH_LAUNCH_CHECK();
   return DH_OK;
 }

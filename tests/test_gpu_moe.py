@@ -614,3 +614,27 @@ def test_grouped_gemm_tn_accumulates_few_rows(rows):
         assert ((got[i].cpu().double() - want).abs() <= want.abs() * 2.0 ** -8 + mass * max(rows) * 2.0 ** -24 + 1e-30).all()
         if x == y:
             assert torch.equal(got[i].cpu(), c[i])
+
+
+@pytest.mark.parametrize("T,E,k", [(5, 1, 1), (33, 3, 2), (9, 8, 8), (67, 9, 3), (40, 33, 8), (31, 64, 8), (700, 5, 4)])
+def test_route_picks_as_a_scan_does(T, E, k):
+    """Ties, infinities, NaN and both zeros: every choice is that of a scan which starts at the lowest id left and moves on to
+    what is greater, so a NaN is chosen only where it is the lowest id left."""
+    from dhellam_amd.operators import moe
+    g = torch.Generator().manual_seed(E)
+    x = torch.randint(-2, 3, (T, E), generator=g).float()
+    for value, share in ((float("nan"), 0.15), (float("inf"), 0.1), (float("-inf"), 0.2), (-0.0, 0.1)):
+        x[torch.rand(T, E, generator=g) < share] = value
+    idx, gates, _ = moe.route_topk(x.cuda(), k)
+    for t in range(T):
+        row, left, sel = x[t].tolist(), list(range(E)), []
+        for _ in range(k):
+            best = left[0]
+            for e in left[1:]:
+                if row[e] > row[best]:
+                    best = e
+            sel.append(best)
+            left.remove(best)
+        assert idx[t].tolist() == sel
+        if all(abs(row[e]) < 1e30 for e in sel):
+            assert torch.allclose(gates[t].cpu(), torch.softmax(x[t][sel], 0), atol=1e-6)
