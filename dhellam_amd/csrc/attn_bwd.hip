@@ -1171,10 +1171,14 @@ static BwdBoth bwd_both(int batch, int max_sq, int max_sk, int64_t total_q, int6
     const int64_t grid = cdiv(longest, 64) * batch, real = total / 64 + batch;
     return grid < real ? grid : real;
   };
-  const int hs = pick_hsplit(tiles(max_sk, total_k) * hk, hq, hk);
+  int hs = pick_hsplit(tiles(max_sk, total_k) * hk, hq, hk);
+  // A group of few heads and rows stays whole where that is an iteration or two more for its workgroup (each of 128 query rows,
+  // 64 from head dim 128 on): the sum of the pieces is a launch of 2.5 us.  us, split / whole, causal: 4 query / 2 kv heads x 60 rows,
+  // head dim 64 12.5 / 11.2, 96 14.7 / 13.3, 128 15.2 / 14.2, 256 25.0 / 26.3; 12 / 4 x 60 13.1 / 12.6, 15.2 / 15.3, 15.8 / 16.3; 16 / 4 x 60 13.4 / 13.7.
+  if (hs == hq / hk && (hs - 1) * cdiv(max_sq, d < 128 ? 128 : 64) <= (d == 64 ? 2 : d <= 128 ? 1 : 0)) hs = 1;
   const int64_t a = tiles(max_sq, total_q) * hq, b = tiles(max_sk, total_k) * hk * hs;
   if (d == 128) {
-    if (max_sq >= 512 && (hs >= 8 || hs < hq / hk)) return {false, hs};
+    if (max_sq >= 512 && (hs >= 8 || hs < hq / hk)) return {false, hs};      // (512 rows are never left whole above)
     if (!causal) return {a + b <= 256 && max_sq == max_sk, hs};
     return {a + b <= 384 || (a + b <= 512 && max_sq >= 256 && max_sq < 1024), hs};
   }
