@@ -572,6 +572,7 @@ def test_grouped_gemm_tn_256_tiles(dtype):
 @pytest.mark.parametrize("rows,n,k", [
     ([0, 1, 63, 64, 65, 127, 128, 129, 130, 255, 257, 300] * 4, 1000, 72),      # tiles that end anywhere; a k tail
     ([131] * 47 + [5], 1096, 200), ([140, 120] * 30, 1408, 1024),
+    ([1152, 0, 1152, 1152, 1152] + [0] * 59, 1408, 1480),        # fewer tiles than the groups let one expect: k in two pieces
 ])
 def test_grouped_gemm_one_stage_tiles(form, rows, n, k):
     """More 128x128 tiles than two workgroups on every compute unit take: the form with one stage.  |error| against fp64 of the
