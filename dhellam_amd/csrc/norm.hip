@@ -371,8 +371,9 @@ norm_bwd_generic_wgrad_kernel(const T *__restrict__ dy, const T *__restrict__ x,
 // therefore does both: the rows w, w + G, ... for dx exactly as norm_bwd_kernel does (same arithmetic, same bits),
 // and the column slab [SW w, SW w + SW) over ALL rows for dgamma / dbeta, reading that slab a second time (from
 // L2 / the last-level cache: the operands were just streamed through it).  Row groups of the slab are added
-// through LDS in a fixed order.  1024 threads, one 16-byte vector of the row per thread (cols <= 1024 vectors).
-template <typename T, bool LN, bool ADD>
+// through LDS in a fixed order.  1024 threads: a row by all of them, one 16-byte vector each (513 to 1024 vectors), or narrower
+// rows side by side, one per TPR threads of VPT vectors as in norm_bwd_kernel (same sums, same bits of dx).
+template <typename T, bool LN, bool ADD, int TPR, int VPT>
 __global__ void __launch_bounds__(1024)
 norm_bwd_onepass_kernel(const T *__restrict__ dy, const T *__restrict__ x, const float *__restrict__ mu,
                         const float *__restrict__ rsigma, const T *__restrict__ gamma, const T *__restrict__ add_to_dx,
@@ -410,8 +411,82 @@ norm_bwd_onepass_kernel(const T *__restrict__ dy, const T *__restrict__ x, const
     }
   }
 
+  // ---- row phase, narrow rows: dx of rows RPB blockIdx.x + 0 .. RPB - 1, and so on by the grid ----
+  if constexpr (TPR < 1024) {
+    constexpr int RPB = BT / TPR;
+    const int lane = tid % TPR, sub = tid / TPR;
+    Vec<T> g[VPT];
+#pragma unroll
+    for (int i = 0; i < VPT; ++i)
+      if (lane + i * TPR < nvec) g[i] = ldg(gamma + (int64_t)(lane + i * TPR) * N);
+    auto row_sum = [&](float v) {            // over the threads of the row, in the order of norm_bwd_kernel
+      v = wave_sum(v);
+      if constexpr (TPR > 64) {
+        __syncthreads();
+        if ((tid & 63) == 0) red[tid >> 6] = v;
+        __syncthreads();
+        v = 0.f;
+#pragma unroll
+        for (int i = 0; i < TPR / 64; ++i) v += red[sub * (TPR / 64) + i];
+      }
+      return v;
+    };
+    for (int64_t row0 = (int64_t)blockIdx.x * RPB; row0 < rows; row0 += (int64_t)gridDim.x * RPB) {
+      const int64_t row = row0 + sub;
+      const bool active = row < rows;
+      Vec<T> xv[VPT], dv[VPT], rv[VPT];
+#pragma unroll
+      for (int i = 0; i < VPT; ++i) {
+        const int v = lane + i * TPR;
+        if (active && v < nvec) {
+          xv[i] = ldg(x + row * cols + (int64_t)v * N);
+          dv[i] = ldg(dy + row * cols + (int64_t)v * N);
+          if (ADD && VPT < 4) rv[i] = ldg(add_to_dx + row * cols + (int64_t)v * N);
+        }
+      }
+      const float rs = active ? rsigma[row] : 0.f;
+      const float mean = LN && active ? mu[row] : 0.f;
+      float s1 = 0.f, s2 = 0.f;
+#pragma unroll
+      for (int i = 0; i < VPT; ++i)
+        if (active && lane + i * TPR < nvec) {
+#pragma unroll
+          for (int j = 0; j < N; ++j) {
+            const float xh = (to_f(xv[i].v[j]) - mean) * rs;
+            const float gg = to_f(dv[i].v[j]) * (to_f(g[i].v[j]) + gamma_shift);
+            s1 += gg * xh;
+            if (LN) s2 += gg;
+          }
+        }
+      // (the values are unpacked again below: kept as floats over the sums they did not fit the 128 registers of a thread)
+#pragma unroll
+      for (int i = 0; i < VPT; ++i)
+        asm volatile("" : "+v"(reinterpret_cast<dh_u32x4 &>(xv[i])), "+v"(reinterpret_cast<dh_u32x4 &>(dv[i])), "+v"(reinterpret_cast<dh_u32x4 &>(g[i])));
+      s1 = row_sum(s1);
+      if (LN) s2 = row_sum(s2);
+      const float c1 = s1 * inv_cols, c2 = s2 * inv_cols;
+#pragma unroll
+      for (int i = 0; i < VPT; ++i) {
+        const int v = lane + i * TPR;
+        if (active && v < nvec) {
+          if (ADD && VPT == 4) rv[i] = ldg(add_to_dx + row * cols + (int64_t)v * N);
+          Vec<T> o;
+#pragma unroll
+          for (int j = 0; j < N; ++j) {
+            const float xh = (to_f(xv[i].v[j]) - mean) * rs;
+            const float gg = to_f(dv[i].v[j]) * (to_f(g[i].v[j]) + gamma_shift);
+            float f = rs * (gg - xh * c1 - c2);
+            if (ADD) f += to_f(rv[i].v[j]);
+            o.v[j] = from_f<T>(f);
+          }
+          stg(dx + row * cols + (int64_t)v * N, o);
+        }
+      }
+    }
+  }
+
   // ---- row phase: dx of rows blockIdx.x, blockIdx.x + gridDim.x, ... ----
-  {
+  if constexpr (TPR == 1024) {
     const int v = tid;
     const bool vvalid = v < nvec;
     Vec<T> g;
@@ -674,7 +749,12 @@ static int64_t bwd_blocks(int64_t rows, int64_t cols, int elt) {
 // Whether the backward runs as one launch (norm_bwd_onepass_kernel): rows of 513 .. 1024 vectors (one vector per
 // thread of a 1024-thread workgroup) and operands small enough that the second, column-wise read of dy and x is
 // served by the caches (32 MiB of dy + x; the 512 x 8192 16-bit rows of a sequence-parallel shard are 16 MiB).
+// Narrower rows, up to about as many as they have columns: the slabs are few workgroups' work (cols / 32 of them), the second
+// launch of the two 3 us.  us, two launches / one, bf16 LayerNorm (RMSNorm): 64 x 1024 7.7 / 5.7 (6.3 / 4.6), 512 x 1024 11.7 / 6.8,
+// 1024 x 1024 13.2 / 9.6 (9.7 / 8.0), 2048 x 1024 16.3 / 15.2 (12.4 / 12.7); 512 x 4096 17.3 / 8.1, 1024 x 4096 24.5 / 15.1, 2048 x 4096
+// 30.5 / 27.1 (23.7 / 23.7); 768 x 512 10.9 / 9.0 (7.8 / 7.1), 1024 x 512 11.0 / 10.7 (7.9 / 8.4).
 static bool bwd_onepass(const NormPlan &p, int64_t rows, int64_t cols, int elt) {
+  if (p.vec && p.tpr < 1024) return rows > 0 && rows <= (cols < 768 ? 768 : cols < 1280 ? cols : 1280);
   return p.vec && p.tpr == 1024 && p.vpt == 1 && rows > 0 && 2 * rows * cols * elt <= (32ll << 20);
 }
 
@@ -732,12 +812,20 @@ static int launch_bwd(const NormPlan &p, const T *dy, const T *x, const float *m
   const int64_t nb = bwd_blocks(rows, cols, sizeof(T));
   if (bwd_onepass(p, rows, cols, sizeof(T))) {
     const unsigned g = (unsigned)cdiv(cols, 32);
-    if (add)
-      hipLaunchKernelGGL((norm_bwd_onepass_kernel<T, LN, true>), dim3(g), dim3(1024), 0, st, dy, x, mu, rs, gamma, add,
-                         dx, dgamma, dbeta, rows, (int)cols, shift, accumulate);
-    else
-      hipLaunchKernelGGL((norm_bwd_onepass_kernel<T, LN, false>), dim3(g), dim3(1024), 0, st, dy, x, mu, rs, gamma, add,
-                         dx, dgamma, dbeta, rows, (int)cols, shift, accumulate);
+#define L2(TPR, VPT, ADD)                                                                                              \
+  hipLaunchKernelGGL((norm_bwd_onepass_kernel<T, LN, ADD, TPR, VPT>), dim3(g), dim3(1024), 0, st, dy, x, mu, rs, gamma, add, dx, \
+                     dgamma, dbeta, rows, (int)cols, shift, accumulate)
+#define L(TPR, VPT)                                                   \
+  do {                                                                \
+    if (add) L2(TPR, VPT, true); else L2(TPR, VPT, false);             \
+  } while (0)
+    if (p.tpr == 1024) L(1024, 1);
+    else if (p.tpr == 256) L(256, 2);
+    else if (p.vpt == 1) L(64, 1);
+    else if (p.vpt == 2) L(64, 2);
+    else L(64, 4);
+#undef L
+#undef L2
     return 0;
   }
   if (!p.vec) {

@@ -559,3 +559,13 @@ def test_reused_swiglu_gradient_buffer_drops_the_transposed_twin():
     out = torch.empty((2 * f, k), dtype=dtype, device="cuda")
     _Clib.wgrad_gemm(buf, x, out, False)
     assert_close(out, (buf.double().t() @ x.double()).cpu(), dtype, "wgrad of the rewritten buffer")
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("rows,cols", [(1, 8), (17, 520), (769, 512), (768, 264), (300, 1032), (1024, 1024), (1025, 1024), (33, 2056),
+                                       (1280, 2048), (1281, 2048), (259, 4096)])
+@pytest.mark.parametrize("ln", [False, True])
+def test_norm_backward_of_narrow_rows(dtype, rows, cols, ln):
+    """One launch and two, on both sides of the line between them: one, two and four vectors a thread, a row by 64 and by 256
+    threads, columns that end inside a slab of 32, more row groups than rows and fewer."""
+    test_norm_fwd_bwd(dtype, rows, cols, ln)
