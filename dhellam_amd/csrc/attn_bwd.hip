@@ -1159,8 +1159,8 @@ static int bwd_hsplit(int max_sk, int batch, int hq, int hk, bool paired) {
 //   one round: 16 x 300 28 / 20 causal, 26 / 20 not, 8 x 1024 51 / 35 causal, 41 / 35 not;
 //   causal, up to a round and a half: 8 x 1500 66 / 47; two: 32 x 512 44 / 40, 16 x 1024 55 / 57, 16 x 16 x 60 22.8 / 22.5; not
 //   causal: 8 x 1500 62 / 84, 32 x 512 36 / 41.
-// A group split eight ways from 512 rows on (8 query / 1 kv head x 1024: 58 / 46) and rectangular calls that are not
-// causal stay with the hand-ordered kernels: callers size the workspace there to choose between their two forms of dQ.
+// A group split eight ways from 512 rows on (8 query / 1 kv head x 1024: 58 / 46) and rectangular calls of several sequences that
+// are not causal stay with the hand-ordered kernels: callers size the workspace there to choose between their two forms of dQ.
 // A group that is left in pieces of several heads makes dK/dV's workgroups that much longer: from 512 rows on not here.  One
 // long sequence among short ones, whole calls, hand-ordered / here with the splits of the grid laid out for the longest / with
 // those of the work: 12 query / 4 kv heads x 791 + 76 + 32 77 / 86 / 57, 4 / 2 x 2746 + 7 135 / 168 / 117.
@@ -1179,7 +1179,7 @@ static BwdBoth bwd_both(int batch, int max_sq, int max_sk, int64_t total_q, int6
   const int64_t a = tiles(max_sq, total_q) * hq, b = tiles(max_sk, total_k) * hk * hs;
   if (d == 128) {
     if (max_sq >= 512 && (hs >= 8 || hs < hq / hk)) return {false, hs};      // (512 rows are never left whole above)
-    if (!causal) return {a + b <= 256 && max_sq == max_sk, hs};
+    if (!causal) return {a + b <= 256 && (max_sq == max_sk || batch == 1), hs};
     return {a + b <= 384 || (a + b <= 512 && max_sq >= 256 && max_sq < 1024), hs};
   }
   if (a + b <= (causal ? 384 : 256)) return {true, hs};
