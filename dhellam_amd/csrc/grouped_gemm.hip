@@ -38,7 +38,7 @@ struct GGParams {
   int max_rows;          // rows the stacked operands hold: group ranges read from offs are cut off there
   float *ws;             // split last round: fp32 partial tiles, one per workgroup
   int zero_tail;         // NT/NN on grouped_gemm_w8_kernel: the kernel itself zeroes the rows of c past the last group
-  int sk_grid;           // grouped_gemm_w8_kernel: > 0: a split kernel of that many workgroups follows and takes the last round of tiles if it splits it;
+  int sk_grid;           // grouped_gemm_w8_kernel: > 0: so many workgroups behind the tiles may take the last round of them in pieces;
                          // grouped_gemm_t_kernel, NT/NN: > 0: places for workgroups, over which the tiles may be split along k
   int pieces;            // grouped_gemm_t_kernel, TN: k pieces per tile
 };
@@ -452,7 +452,7 @@ __global__ void __launch_bounds__(512) grouped_gemm_w8_kernel(const GGParams p) 
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                    // the last copies (zeros) have landed before the stages are used again
     __syncthreads();
 
-    if constexpr (SK) {
+    if (SK && part != nullptr) {
       // 16 bytes per lane and instruction: piece w * 32 + block of the tile, 1 KB each
       float *dst = part + (size_t)w * 32 * 256 + (size_t)lane * 4;
 #pragma unroll
@@ -473,44 +473,46 @@ __global__ void __launch_bounds__(512) grouped_gemm_w8_kernel(const GGParams p) 
     int tm, tn;
     gg_tile_of(pid, p.tiles_m, p.tiles_n, tm, tn);
     segment(g, rb, re, tm, tn, 0, (re - rb + 63) / 64, nullptr);
-  } else if constexpr (!SK) {
+  } else {
     // The grid is sized for the host's upper bound of the tile count (it does not know how the rows split into
     // groups); the chunks of the XCDs are cut from the real count, so that every XCD gets its share of real tiles.
     int tiles_m;
     const GGGroupTable gt = gg_group_table(p, base, tiles_m);
     const int ntiles = tiles_m * p.tiles_n;
-    int kept = ntiles;
-    if (p.sk_grid > 0) {
-      // the tiles past the last full round of sk_grid tiles belong to the split kernel, if it splits them
-      const int full = ntiles / p.sk_grid, rem = ntiles - full * p.sk_grid;
-      if (gg_sk_pieces(p.sk_grid, rem, nsl) > 1) kept = full * p.sk_grid;
+    int kept = ntiles, rem = 0, pieces = 1;
+    if constexpr (SK) {
+      // The tiles (in the order of gg_tile_of) run in rounds of sk_grid = the number of compute units.  When the last round
+      // holds at most half as many tiles as there are compute units it is split along k: as many pieces per tile as fit
+      // (unit w behind the full rounds: tile w % rem, piece w / rem, so that neighbours work on neighbouring tiles), summed
+      // afterwards in k order.  288 tiles on 256 compute units then take 1 1/8 tile times instead of 2.  The pieces are the last
+      // workgroups of the same launch: they start as compute units run out of full-round tiles, not when the last of them has
+      // ended.  bf16 NT, 1280 rows x 2 groups, 7168 x 4096: 82.8 -> 78.5 us against a kernel of their own behind; 16 groups of
+      // 256 rows, 4096 x 2816: 149 -> 146; nothing to split: one launch of 5 us less.  (A resident workgroup that also looped
+      // over the full rounds was 3-6 % slower on them than one workgroup per tile.)
+      const int full = ntiles / p.sk_grid;
+      rem = ntiles - full * p.sk_grid;
+      pieces = gg_sk_pieces(p.sk_grid, rem, nsl);
+      if (pieces > 1) kept = full * p.sk_grid;
     }
-    if ((int)blockIdx.x >= kept) return;
-    const int pid = gg_xcd_chunk((int)blockIdx.x, kept);              // (the XCDs share the tiles that are computed here)
+    int pid, s0 = 0, s1 = nsl;
+    float *part = nullptr;
+    if ((int)blockIdx.x < kept) {
+      pid = gg_xcd_chunk((int)blockIdx.x, kept);                      // (the XCDs share the tiles that are computed here)
+    } else if (SK && pieces > 1 && (int)blockIdx.x - kept < p.sk_grid) {
+      const int wg = gg_xcd_chunk((int)blockIdx.x - kept, p.sk_grid);  // neighbouring tiles on one XCD (kept: whole rounds)
+      if (wg >= rem * pieces) return;
+      const int pc = wg / rem;
+      pid = kept + wg % rem;
+      s0 = pc * nsl / pieces;
+      s1 = (pc + 1) * nsl / pieces;
+      part = p.ws + (size_t)wg * (256 * 256);
+    } else {
+      return;
+    }
     int tm_all, tn, g, rb, re, tm;
     gg_tile_of(pid, tiles_m, p.tiles_n, tm_all, tn);
     gg_locate(gt, tm_all, g, rb, re, tm);
-    segment(g, rb, re, tm, tn, 0, nsl, nullptr);
-  } else {
-    // The last round of tiles, split along k.  The tiles (in the order of gg_tile_of) run in rounds of gridDim.x = the
-    // number of compute units; grouped_gemm_w8_kernel<.., false> in front of this kernel takes the full rounds, one
-    // workgroup per tile.  When the last round holds at most half as many tiles as there are workgroups, it is left to
-    // this kernel: as many k pieces per tile as fit (workgroup w: tile w % rem, piece w / rem, so that neighbours work
-    // on neighbouring tiles), summed afterwards in k order.  288 tiles on 256 compute units then take 1 1/8 tile
-    // times instead of 2.  (A resident workgroup that also looped over the full rounds was 3-6 % slower on them than
-    // one workgroup per tile.)
-    int tiles_m;
-    const GGGroupTable gt = gg_group_table(p, base, tiles_m);
-    const int tiles = tiles_m * p.tiles_n;
-    const int grid = (int)gridDim.x, full = tiles / grid, rem = tiles - full * grid;
-    const int pieces = gg_sk_pieces(grid, rem, nsl);
-    const int wg = gg_xcd_chunk((int)blockIdx.x, grid);                // neighbouring tiles on one XCD
-    if (pieces == 1 || wg >= rem * pieces) return;
-    const int ts = wg % rem, pc = wg / rem;
-    int tm_all, tn, g, rb, re, tm;
-    gg_tile_of(full * grid + ts, tiles_m, p.tiles_n, tm_all, tn);
-    gg_locate(gt, tm_all, g, rb, re, tm);
-    segment(g, rb, re, tm, tn, pc * nsl / pieces, (pc + 1) * nsl / pieces, p.ws + (size_t)wg * (256 * 256));
+    segment(g, rb, re, tm, tn, s0, s1, part);
   }
 }
 #undef GG_W8_BARRIER
@@ -1051,16 +1053,16 @@ static int launch_gg_w8(GGParams p, int64_t m_extent, void *workspace, size_t wo
     if (workspace_bytes < (size_t)grid * 256 * 256 * sizeof(float)) grid = 0;
   }
   // With a workspace the last round of tiles may be split along k (decided on the device, where the tile count is
-  // known): the first kernel then leaves that round to the split kernel.  When nothing is split the two extra
-  // launches cost a few microseconds; a split saves up to half a tile time (45 us and more).
+  // known) by up to `grid` workgroups more.  Where nothing is split the sum's launch is for nothing (5 us); a split saves up to
+  // half a tile time (45 us and more).
   p.sk_grid = grid;
-  hipLaunchKernelGGL((grouped_gemm_w8_kernel<T, BKS ? 1 : 0, false>), dim3((unsigned)(p.tiles_m * p.tiles_n)), dim3(512), 0, st, p);
-  if (grid > 0) {
-    p.ws = reinterpret_cast<float *>(workspace);
-    p.zero_tail = 0;                                    // done by the kernel above
-    hipLaunchKernelGGL((grouped_gemm_w8_kernel<T, BKS ? 1 : 0, true>), dim3((unsigned)grid), dim3(512), 0, st, p);
-    hipLaunchKernelGGL((gg_split_reduce_kernel<T>), dim3((unsigned)(16 * grid / 2)), dim3(256), 0, st, p, grid);   // at most grid / 2 tiles are split
+  if (grid == 0) {
+    hipLaunchKernelGGL((grouped_gemm_w8_kernel<T, BKS ? 1 : 0, false>), dim3((unsigned)(p.tiles_m * p.tiles_n)), dim3(512), 0, st, p);
+    return DH_OK;
   }
+  p.ws = reinterpret_cast<float *>(workspace);
+  hipLaunchKernelGGL((grouped_gemm_w8_kernel<T, BKS ? 1 : 0, true>), dim3((unsigned)(p.tiles_m * p.tiles_n + grid)), dim3(512), 0, st, p);
+  hipLaunchKernelGGL((gg_split_reduce_kernel<T>), dim3((unsigned)(16 * grid / 2)), dim3(256), 0, st, p, grid);   // at most grid / 2 tiles are split
   return DH_OK;
 }
 
