@@ -1276,8 +1276,11 @@ extern "C" int dh_grouped_gemm_tn_ws(const void *a, const void *b, void *c, cons
   p.a = a; p.b = b; p.c = c; p.offs = offs; p.groups = groups;
   p.m_dim = m; p.n_dim = n; p.lda = m; p.ldb = n; p.ldc = n;
   p.c_group_stride = m * n; p.accumulate = accumulate; p.max_rows = (int)max_rows;
-  // (the offsets of the 256x256 tiles have to fit the 32-bit buffer addressing)
-  if (gg_w8_tn_pays(max_rows, groups, m, n, accumulate) && max_rows * (m > n ? m : n) * (int64_t)dtype_size(dtype) < (1ll << 31))
+  // The offsets of the 256x256 tiles have to fit the 32-bit buffer addressing: of the operands, of the 64 rows of a slice, however
+  // few of them there are, and, accumulating, of a tile's 256 rows of c.  (Otherwise the rows asked for above keep them short.)
+  const bool fits = max_rows * (m > n ? m : n) * (int64_t)dtype_size(dtype) < (1ll << 31) &&
+                    (!accumulate || (m <= GG_MAX_LD && n <= GG_MAX_LD));
+  if (fits && gg_w8_tn_pays(max_rows, groups, m, n, accumulate))
     rc = dtype == DH_BF16 ? launch_gg_w8_tn<bf16_t>(p, (hipStream_t)stream) : launch_gg_w8_tn<f16_t>(p, (hipStream_t)stream);
   else
     rc = dtype == DH_BF16 ? dispatch_gg_t<bf16_t, 2>(p, m, workspace, workspace_bytes, (hipStream_t)stream)

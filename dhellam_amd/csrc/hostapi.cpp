@@ -417,6 +417,9 @@ bool dgrad_grouped(int64_t t, int64_t n, int64_t k) {
   return n >= 5120 && (t * k <= 2800000 || t * k >= 14000000);
 }
 
+// The row lengths (elements) that the grouped kernel's tiles address: longer ones have a kernel there for a few rows only.
+constexpr int64_t kGroupedMaxRow = (1 << 22) - 8;
+
 // Weight gradient dY [T, N]^T X [T, K]: the same question.  The library reads both operands along their strided dimension
 // here, its slowest layout (one of them materialised transposed first gains 10 % and costs most of that); the grouped kernel's
 // LDS transpose reads cost it nothing, and it adds to what is there without a read of its own.  us accumulating, library (the
@@ -428,6 +431,7 @@ bool dgrad_grouped(int64_t t, int64_t n, int64_t k) {
 // 12.2 / 12.4.
 bool wgrad_grouped(int64_t t, int64_t n, int64_t k) {
   const int64_t tiles = (n + 255) / 256 * ((k + 255) / 256);
+  if (n > kGroupedMaxRow || k > kGroupedMaxRow) return false;
   if (t > 0 && tiles >= 160) return !(tiles < 224 && t % 64 == 0 && t >= 2048) && 2 * t * std::max(n, k) < (int64_t)1 << 31;
   return t > 0 && t <= 384 && n * k <= 3200000;
 }

@@ -523,6 +523,23 @@ def test_grouped_gemm_tn_rows_longer_than_the_tiled_kernels_take(m, n, accumulat
         assert_close(c[e], ref, torch.bfloat16, f"tn, group {e}", local=False)
 
 
+@pytest.mark.parametrize("n", [4300800, (1 << 23) + 4096])
+def test_grouped_gemm_tn_adds_to_rows_past_the_32_bit_offsets(n):
+    """Accumulating few rows into a gradient of 256 rows of ``n`` values: the last rows of a tile of old values begin 2 GiB and
+    more behind its first one (at 2^23 + 4096 columns, offsets past 4 GiB)."""
+    from dhellam_amd.operators import moe
+    m, rows = 256, 16
+    offs = torch.tensor([0, rows], dtype=torch.int32, device="cuda")
+    g = torch.Generator(device="cuda").manual_seed(9)
+    a, b = ((torch.randn(rows, w, generator=g, device="cuda") * 0.5).to(torch.bfloat16) for w in (m, n))
+    old = (torch.arange(m, device="cuda") % 37 + 2).to(torch.bfloat16)
+    c = old[None, :, None].expand(1, m, n).contiguous()
+    moe.grouped_gemm_tn(a, b, offs, c, True)
+    for lo in range(0, n, 1 << 20):
+        ref = a.float().t() @ b[:, lo:lo + (1 << 20)].float() + old.float()[:, None]
+        assert_close(c[0][:, lo:lo + (1 << 20)], ref, torch.bfloat16, f"columns {lo}..", local=False)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("n,k", [(3848, 1544),      # whole rounds; the last k slice holds 8 columns
                                  (4104, 1600),      # 272 tiles: the last 16 in pieces of one and two slices
