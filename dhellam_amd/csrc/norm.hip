@@ -810,7 +810,10 @@ static int launch_bwd(const NormPlan &p, const T *dy, const T *x, const float *m
                       const T *add, T *dx, T *dgamma, T *dbeta, float *part, int64_t rows, int64_t cols,
                       float shift, int accumulate, hipStream_t st) {
   const int64_t nb = bwd_blocks(rows, cols, sizeof(T));
-  if (bwd_onepass(p, rows, cols, sizeof(T))) {
+  // dx in the place of dy or x: the one-launch kernel's column sums would read what other workgroups have overwritten; the
+  // two-launch kernel has every vector in registers before it stores there.
+  const auto overlap = [&](const T *a) { return dx < a + rows * cols && a < dx + rows * cols; };
+  if (bwd_onepass(p, rows, cols, sizeof(T)) && !overlap(dy) && !overlap(x)) {
     const unsigned g = (unsigned)cdiv(cols, 32);
 #define L2(TPR, VPT, ADD)                                                                                              \
   hipLaunchKernelGGL((norm_bwd_onepass_kernel<T, LN, ADD, TPR, VPT>), dim3(g), dim3(1024), 0, st, dy, x, mu, rs, gamma, add, dx, \
@@ -830,11 +833,11 @@ static int launch_bwd(const NormPlan &p, const T *dy, const T *x, const float *m
   }
   if (!p.vec) {
     int64_t g = rows < 4096 ? rows : 4096;
-    hipLaunchKernelGGL((norm_bwd_generic_kernel<T, LN>), dim3((unsigned)g), dim3(256), 0, st, dy, x, mu, rs, gamma,
-                       add, dx, rows, cols, shift);
-    const int64_t rpc = cdiv(rows, nb);
+    const int64_t rpc = cdiv(rows, nb);      // (first: dx may be written in the place of dy or x)
     hipLaunchKernelGGL((norm_bwd_generic_wgrad_kernel<T, LN>), dim3((unsigned)cdiv(cols, 64), (unsigned)nb),
                        dim3(256), 0, st, dy, x, mu, rs, part, rows, cols, rpc);
+    hipLaunchKernelGGL((norm_bwd_generic_kernel<T, LN>), dim3((unsigned)g), dim3(256), 0, st, dy, x, mu, rs, gamma,
+                       add, dx, rows, cols, shift);
   } else {
     const bool nt = stream_hint((add ? 4 : 3) * rows * cols * (int64_t)sizeof(T));
 #define L3(BT, TPR, VPT, NT, ADD)                                                                            \

@@ -35,7 +35,8 @@ def pylayernorm_bwd(d_ln_out, inp, mu, rsigma, ln_weight, bwd_sm_margin, zero_ce
     added to dinp inside the kernel (the residual-branch gradient the reference
     adds afterwards, dstb.py:391,401); ``dgamma_out`` / ``dbeta_out`` are
     accumulated into in place (the reference's ``main_grad.add_``, dstb.py:392-393);
-    ``dgrad_out`` is a contiguous tensor of the input's size that receives dinp instead of a new one.
+    ``dgrad_out`` is a contiguous tensor of the input's size that receives dinp instead of a new one
+    (``d_ln_out``, ``inp`` or ``add_to_dgrad`` itself, if that is not needed any more).
     """
     if dgrad_out is not None:
         _lib.mark_written(dgrad_out)

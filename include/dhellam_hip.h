@@ -69,8 +69,8 @@ int dh_add_norm_fwd(const void *x, const void *residual, void *sum_out,
 size_t dh_norm_bwd_workspace_bytes(int64_t rows, int64_t cols);
 
 /* dx = d(loss)/dx (+ add_to_dx if non-NULL: the residual-branch gradient the
- * reference adds in a separate launch, dhellam/core/dstb.py:387-405).
- * dgamma/dbeta [cols] in `dtype`; mu == NULL selects RMSNorm (dbeta may be
+ * reference adds in a separate launch, dhellam/core/dstb.py:387-405).  dx may
+ * be dy, x or add_to_dx itself.  dgamma/dbeta [cols] in `dtype`; mu == NULL selects RMSNorm (dbeta may be
  * NULL).  accumulate_wgrad != 0: dgamma/dbeta are added to instead of
  * overwritten.  workspace: workspace_bytes bytes, at least
  * dh_norm_bwd_workspace_bytes(rows, cols) or the call is refused with

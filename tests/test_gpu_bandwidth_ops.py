@@ -569,3 +569,26 @@ def test_norm_backward_of_narrow_rows(dtype, rows, cols, ln):
     """One launch and two, on both sides of the line between them: one, two and four vectors a thread, a row by 64 and by 256
     threads, columns that end inside a slab of 32, more row groups than rows and fewer."""
     test_norm_fwd_bwd(dtype, rows, cols, ln)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,cols", [(64, 512), (160, 1024), (700, 2048), (512, 4096),      # one launch where nothing overlaps
+                                       (128, 8192),                                           # ... by whole workgroups
+                                       (2000, 1024), (33, 1001)])                             # two launches; the generic kernels
+@pytest.mark.parametrize("ln", [False, True])
+def test_norm_backward_in_the_place_of_an_operand(dtype, rows, cols, ln):
+    """``dgrad_out`` that is the gradient or the input itself: dx is the same, and the weight gradients are those of the operands
+    as they were."""
+    from dhellam_amd.operators.layernorm import pylayernorm_bwd
+    x, dy, add = (randn((rows, cols), dtype, s).cuda() for s in (61, 62, 63))
+    gamma = (1 + randn((cols,), torch.float32, 64, std=0.1)).to(dtype).cuda()
+    xf = x.float()
+    mu = xf.mean(1) if ln else None
+    rs = 1 / ((xf - mu[:, None] if ln else xf).square().mean(1) + 1e-5).sqrt()
+    ref = [t for t in pylayernorm_bwd(dy, x, mu, rs, gamma, 0, False, None, add_to_dgrad=add)[:3] if t is not None]
+    for place in range(3):
+        ops = [t.clone() for t in (dy, x, add)]
+        got = pylayernorm_bwd(ops[0], ops[1], mu, rs, gamma, 0, False, None, add_to_dgrad=ops[2], dgrad_out=ops[place])[:3]
+        assert got[0].data_ptr() == ops[place].data_ptr()
+        for g, r, name in zip([t for t in got if t is not None], ref, ("dx", "dgamma", "dbeta")):
+            assert_close(g, r, dtype, f"{name}, dx in operand {place}")
