@@ -751,10 +751,20 @@ static int64_t bwd_blocks(int64_t rows, int64_t cols, int elt) {
 // served by the caches (32 MiB of dy + x; the 512 x 8192 16-bit rows of a sequence-parallel shard are 16 MiB).
 // Narrower rows, up to about as many as they have columns: the slabs are few workgroups' work (cols / 32 of them), the second
 // launch of the two 3 us.  us, two launches / one, bf16 LayerNorm (RMSNorm): 64 x 1024 7.7 / 5.7 (6.3 / 4.6), 512 x 1024 11.7 / 6.8,
-// 1024 x 1024 13.2 / 9.6 (9.7 / 8.0), 2048 x 1024 16.3 / 15.2 (12.4 / 12.7); 512 x 4096 17.3 / 8.1, 1024 x 4096 24.5 / 15.1, 2048 x 4096
-// 30.5 / 27.1 (23.7 / 23.7); 768 x 512 10.9 / 9.0 (7.8 / 7.1), 1024 x 512 11.0 / 10.7 (7.9 / 8.4).
+// 1024 x 1024 13.3 / 9.6 (9.7 / 8.0), 2048 x 1024 16.3 / 15.2 (12.4 / 12.7); 512 x 4096 17.2 / 8.0, 1024 x 4096 24.3 / 15.0, 2048 x 4096
+// 30.5 / 27.1 (23.7 / 23.7); fp32 64 x 1024 7.6 / 6.0, 1024 x 1024 13.8 / 10.5 (10.4 / 9.0), 1024 x 1536 19.8 / 17.4 (15.1 / 14.0), 1280 x
+// 2048 24.5 / 19.1.
+// Below 768 columns the line is the steps of 16 rows that a workgroup takes for dx, one behind the other, at most 768 rows:
+// two steps and three from 256 columns on in 16 bits, three and four in fp32 (a slab row is half the bytes of a thread), four
+// from 384 on.  bf16: 8 columns, 16, 64 and 768 rows 5.7 / 4.1, 6.3 / 7.9, 9.7 / 65; 64, 64 and 128 rows 6.3 / 6.2, 6.6 / 9.0; 128, 128 and 256
+// 6.6 / 6.6, 7.7 / 9.2; 256, 384 and 768 8.5 / 8.5 (6.4 / 6.3), 10.5 / 12.7; 384, 768 10.9 / 10.3 (7.8 / 8.1); 512, 768 11.0 / 9.0 (7.9 / 7.1), 1024
+// 11.0 / 10.7 (7.9 / 8.4).  fp32: 64, 64 and 128 5.5 / 4.9, 5.7 / 6.5; 256, 512 and 768 9.3 / 7.6, 9.9 / 9.6 (7.2 / 7.7); 384, 768 11.1 / 9.5.
 static bool bwd_onepass(const NormPlan &p, int64_t rows, int64_t cols, int elt) {
-  if (p.vec && p.tpr < 1024) return rows > 0 && rows <= (cols < 768 ? 768 : cols < 1280 ? cols : 1280);
+  if (p.vec && p.tpr < 1024) {
+    if (cols >= 768) return rows > 0 && rows <= (cols < 1280 ? cols : 1280);
+    const int64_t steps = cols >= 384 ? 4 : (cols >= 256 ? 3 : 2) + (elt == 4 ? 1 : 0), most = 16 * steps * cdiv(cols, 32);
+    return rows > 0 && rows <= (most < 768 ? most : 768);
+  }
   return p.vec && p.tpr == 1024 && p.vpt == 1 && rows > 0 && 2 * rows * cols * elt <= (32ll << 20);
 }
 
@@ -930,6 +940,12 @@ __global__ void __launch_bounds__(256) zero_bytes_kernel(uint8_t *p, int64_t n) 
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) p[i] = 0;
 }
 }  // namespace dh
+
+extern "C" int dh_norm_bwd_one_launch(int64_t rows, int64_t cols, int dtype) {
+  if (rows <= 0 || cols <= 0 || (dtype != DH_F32 && dtype != DH_BF16 && dtype != DH_F16)) return 0;
+  const int elt = (int)dh::dtype_size(dtype);
+  return dh::bwd_onepass(dh::norm_plan(cols, elt, true), rows, cols, elt) ? 1 : 0;
+}
 
 extern "C" int dh_norm_bwd(const void *dy, const void *x, const float *mu, const float *rsigma, const void *gamma,
                            const void *add_to_dx, void *dx, void *dgamma, void *dbeta, void *workspace,

@@ -67,6 +67,9 @@ int dh_add_norm_fwd(const void *x, const void *residual, void *sum_out,
 
 /* Bytes of fp32 scratch dh_norm_bwd needs for its dgamma/dbeta partial sums. */
 size_t dh_norm_bwd_workspace_bytes(int64_t rows, int64_t cols);
+/* Whether dh_norm_bwd takes one launch for these sizes (16-byte aligned
+ * operands, dx in a place of its own). */
+int dh_norm_bwd_one_launch(int64_t rows, int64_t cols, int dtype);
 
 /* dx = d(loss)/dx (+ add_to_dx if non-NULL: the residual-branch gradient the
  * reference adds in a separate launch, dhellam/core/dstb.py:387-405).  dx may

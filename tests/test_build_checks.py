@@ -22,3 +22,13 @@ def test_weight_gradients_of_very_long_rows_stay_with_the_library():
     assert _host.wgrad_grouped(16, edge, 256) and _host.wgrad_grouped(16, 256, edge)
     assert not _host.wgrad_grouped(16, edge + 8, 256) and not _host.wgrad_grouped(16, 256, edge + 8)
     assert not _host.wgrad_grouped(16, 5000000, 256)
+
+
+@pytest.mark.parametrize("dtype,rows,cols,one", [
+    (1, 16, 8, 1), (1, 64, 64, 1), (1, 512, 512, 1), (1, 1024, 1024, 1), (1, 1280, 4096, 1), (1, 512, 8192, 1),
+    (1, 64, 8, 0), (1, 768, 64, 0), (1, 256, 128, 0), (1, 768, 256, 0), (1, 1024, 512, 0), (1, 1025, 1024, 0), (1, 2048, 8192, 0),
+    (0, 48, 8, 1), (0, 512, 256, 1), (0, 768, 384, 1), (0, 1024, 1024, 1), (0, 1280, 2048, 1), (0, 256, 64, 0), (0, 768, 256, 0)])
+def test_norm_backward_in_one_launch_is_for_rows_that_few_workgroups_can_take(dtype, rows, cols, one):
+    """The one launch has a workgroup per 32 columns: with few columns it is the faster form for few rows only."""
+    from dhellam_amd import _lib
+    assert _lib.load().dh_norm_bwd_one_launch(rows, cols, dtype) == one

@@ -563,7 +563,7 @@ def test_reused_swiglu_gradient_buffer_drops_the_transposed_twin():
 
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("rows,cols", [(1, 8), (17, 520), (769, 512), (768, 264), (300, 1032), (1024, 1024), (1025, 1024), (33, 2056),
-                                       (1280, 2048), (1281, 2048), (259, 4096)])
+                                       (1280, 2048), (1281, 2048), (259, 4096), (32, 8), (33, 8), (432, 264), (433, 264)])
 @pytest.mark.parametrize("ln", [False, True])
 def test_norm_backward_of_narrow_rows(dtype, rows, cols, ln):
     """One launch and two, on both sides of the line between them: one, two and four vectors a thread, a row by 64 and by 256
