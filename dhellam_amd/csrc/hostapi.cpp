@@ -402,23 +402,42 @@ bool grouped_ok(const Tensor &x, at::ScalarType type) {
          x.size(1) % 8 == 0 && (uintptr_t)x.data_ptr() % 16 == 0;
 }
 
-// Data gradient grad [T, N] @ weight [N, K] as given: whether the grouped kernel with one group is the faster one.  It splits
-// long reductions of few rows over the chip and needs no whole slices; the library's kernels for this layout are at their
-// best where N is short.  us, library / here, of a sweep over N = 1000 to 32000, K = 512 to 8192, T = 64 to 4096:
-//   N that is no multiple of 64: 1000 x 1024 at T = 1904 15 / 11, 4000 x 1024 at 1000 27 / 23, 16032 x 4096 at 512 113 / 71
-//   N >= 16000: 32000 x 1024 at 200, 1000, 4096 101 / 33, 175 / 69, 323 / 215; x 4096 209 / 76, 313 / 211, 770 / 738
-//   5120 <= N < 16000, by K T: 8192 x 1024 at 64, 1000, 1904 36 / 16, 44 / 31, 58 / 43, at 3000 65 / 64; x 2048 at 1000 58 / 45,
-//     at 1904 71 / 73, at 3000 94 / 112; x 3584 at 768 84 / 57, at 1000 70 / 70; 7168 x 8192 at 200 50 / 41, at 512 64 / 68;
-//     and again where 256x256 tiles fill the chip: 7168 x 8192 at 1904, 4096 173 / 164, 346 / 330, 8192 x 3584 at 4096 184 / 180
-//   below: the library (3072 x 1024 at 1000 18 / 21, 1280 x 8192 at 1904 38 / 41)
-bool dgrad_grouped(int64_t t, int64_t n, int64_t k) {
-  if (t <= 0 || n < 1000) return false;
-  if (n % 64 != 0 || n >= 16000) return true;
-  return n >= 5120 && (t * k <= 2800000 || t * k >= 14000000);
-}
-
 // The row lengths (elements) that the grouped kernel's tiles address: longer ones have a kernel there for a few rows only.
 constexpr int64_t kGroupedMaxRow = (1 << 22) - 8;
+
+// Data gradient grad [T, N] @ weight [N, K] as given: whether the grouped kernel with one group is the faster one.  It splits
+// long reductions of few rows over the chip and needs no whole slices; the library's kernels for this layout are at their
+// best where N is short and the result small.  us, library / here, of sweeps over N = 1000 to 50304, K = 64 to 8192, T = 1 to 16384:
+//   N >= 16000: 32000 x 1024 at 8, 200, 1000, 4096, 16384 94 / 21, 101 / 33, 174 / 68, 336 / 214, 800 / 738; x 4096 at 8, 1000, 4096, 16384 122 / 50,
+//     323 / 211, 769 / 719, 3058 / 2923
+//   more than 125 rows for every column of a narrow result, store after store: 8192 x 64 at 6000, 16384 1.18 and 0.52 times as fast, x 128
+//     at 12000, 16384 1.09 and 0.60; from N = 12000 on only up to 64 columns (32000 x 64 at 16384 0.94, x 128 1.21 times)
+//   results of up to 65536 values, where there is little to split (not the narrowest, where the library is slow as well, and not
+//     those with rows of 4096 and more): 5120 x 256 at 48, 256 10.6 / 12, 10.8 / 13.9, 8192 x 1024 at 16, 48, 65 0.82, 0.84, 1.35 times; from 9000
+//     on here again (12288 x 256 at 1, 200 1.04, 1.36 times).  At exactly 64 rows the library's choice is a poor one: 8192 x 1024
+//     36 / 17, 5120 x 256 25 / 13, where 63 and 65 rows are 0.8 times as fast here
+//   5120 <= N < 16000, by K T: 8192 x 1024 at 100, 1000, 1904 1.5 times, 44 / 31, 58 / 43, at 3000 65 / 64; x 2048 at 1000 58 / 45,
+//     at 1904 71 / 73, at 3000 94 / 112; x 3584 at 768 84 / 57, at 1000 70 / 70; 7168 x 8192 at 200 50 / 41, at 512 64 / 68;
+//     and again where 256x256 tiles fill the chip: 7168 x 8192 at 1904, 4096 173 / 164, 346 / 330, 8192 x 3584 at 4096 184 / 180
+//   N that is no multiple of 64: to 1152 all (1000 x 1024 at 8, 1904, 16384 10.6 / 8.1, 15 / 11, 43 / 36); from 2900 on by the size of the
+//     result as above, up to 5900 (4008 x 256 at 128, 512, 1000 0.86, 1.41 times, 20 / 16, 6008 x 128 at 256 0.96); in between large results,
+//     and from 1440 on few rows and narrow long results (1256 x 1024 at 8, 1000, 8192 0.93, 0.87, 1.18 times; 1504 x 512 at 32, 1000,
+//     8192 1.08, 0.94, 0.79, x 128 at 512, 1000 0.97, 1.40; 2008 x 1024 at 64, 1000, 4096, 8192 1.42, 0.84, 0.83, 1.09)
+//   below: the library (3072 x 1024 at 1000 18 / 21, 1280 x 8192 at 1904 38 / 41)
+// Over the 2254 products of the sweeps 23 are more than 5 % slower here than by the library, none of them by 20 %.
+bool dgrad_grouped(int64_t t, int64_t n, int64_t k) {
+  if (t <= 0 || n < 1000 || n > kGroupedMaxRow || k > kGroupedMaxRow) return false;
+  const int64_t size = t * k;
+  const bool ragged = n % 64 != 0;
+  if (ragged && n < 1152) return true;
+  if (t > 125 * k && (n < 12000 || k <= 64)) return false;
+  if (n >= 16000) return true;
+  if (ragged && n < 2900)
+    return size > (n < 1440 ? 2000000 : 4300000) || (n >= 1440 && (t <= 56 || t == 64 || (t >= 1000 && k > 64 && k < 256)));
+  if (!ragged && n < 5120) return false;
+  if (size <= 65536 && k > 64 && k < 4096 && t != 64 && n < (ragged ? 5900 : 9000)) return false;
+  return ragged || size <= 2800000 || size >= 14000000;
+}
 
 // Weight gradient dY [T, N]^T X [T, K]: the same question.  The library reads both operands along their strided dimension
 // here, its slowest layout (one of them materialised transposed first gains 10 % and costs most of that); the grouped kernel's
@@ -1003,6 +1022,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("grouped_gemm_tn", &grouped_gemm_tn);
   m.def("wgrad", &wgrad);
   m.def("wgrad_grouped", &wgrad_grouped);
+  m.def("dgrad_grouped", &dgrad_grouped);
   m.def("embedding_fwd", &embedding_fwd);
   m.def("embedding_bwd", &embedding_bwd);
   m.def("cross_entropy_fwd", &cross_entropy_fwd);

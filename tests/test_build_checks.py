@@ -32,3 +32,17 @@ def test_norm_backward_in_one_launch_is_for_rows_that_few_workgroups_can_take(dt
     """The one launch has a workgroup per 32 columns: with few columns it is the faster form for few rows only."""
     from dhellam_amd import _lib
     assert _lib.load().dh_norm_bwd_one_launch(rows, cols, dtype) == one
+
+
+@pytest.mark.parametrize("t,n,k,grouped", [
+    # measured the faster one here, on both sides of every line
+    (1000, 32000, 1024, 1), (16384, 16032, 4096, 1), (8, 16000, 256, 1), (1000, 8192, 1024, 1), (65, 8192, 1024, 1), (64, 5120, 256, 1),
+    (200, 12288, 256, 1), (8192, 7168, 8192, 1), (8, 5120, 4096, 1), (16384, 1000, 64, 1), (8192, 1256, 1024, 1), (32, 1504, 512, 1),
+    (1000, 1504, 128, 1), (64, 2008, 1024, 1), (1000, 4008, 256, 1), (256, 6008, 128, 1), (6000, 8192, 64, 1), (12000, 8192, 128, 1),
+    # ... and by the library
+    (16384, 8192, 64, 0), (16384, 8192, 128, 0), (16384, 32000, 64, 0), (256, 5120, 256, 0), (48, 8192, 1024, 0), (63, 5120, 256, 0),
+    (1000, 1256, 1024, 0), (8, 1256, 1024, 0), (8192, 1504, 512, 0), (1000, 2008, 1024, 0), (128, 4008, 256, 0), (3000, 8192, 2048, 0),
+    (1000, 3072, 1024, 0), (1904, 1280, 8192, 0), (16, (1 << 22), 256, 0)])
+def test_data_gradients_go_where_they_were_measured_the_faster(t, n, k, grouped):
+    from dhellam_amd import _host
+    assert _host.dgrad_grouped(t, n, k) == bool(grouped)
