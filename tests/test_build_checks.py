@@ -46,3 +46,13 @@ def test_norm_backward_in_one_launch_is_for_rows_that_few_workgroups_can_take(dt
 def test_data_gradients_go_where_they_were_measured_the_faster(t, n, k, grouped):
     from dhellam_amd import _host
     assert _host.dgrad_grouped(t, n, k) == bool(grouped)
+
+
+@pytest.mark.parametrize("t,n,k,grouped", [
+    (24, 100000, 8, 1), (64, 100000, 8, 0), (200, 8, 100000, 0), (32, 32, 100000, 1), (64, 100000, 32, 0),
+    (128, 50304, 64, 1), (2000, 50304, 64, 0), (8192, 64, 65536, 0), (1000, 50304, 96, 1), (2000, 50304, 96, 0), (1000, 128, 50304, 1),
+    (2000, 128, 50304, 0), (3000, 264, 30000, 1), (4096, 30000, 264, 0), (8192, 320, 65536, 0), (2000, 192, 50304, 1), (8192, 512, 50304, 1),
+    (4096, 7168, 8192, 1), (4096, 8192, 3584, 1), (4096, 1280, 8192, 0), (1000, 1280, 8192, 1), (384, 32000, 96, 1), (385, 1280, 2048, 0)])
+def test_weight_gradients_go_where_they_were_measured_the_faster(t, n, k, grouped):
+    from dhellam_amd import _host
+    assert _host.wgrad_grouped(t, n, k) == bool(grouped)
