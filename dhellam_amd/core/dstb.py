@@ -340,7 +340,8 @@ class DCFunc:
     bda_attn = bda_mlp
 
     @staticmethod
-    def swiglu(config, data, stream):
+    def swiglu(config, data, stream, grad_type=None):
+        """``grad_type``: type of the gradient that the weight gradient behind is added to, where it is not the input's."""
         (input,) = data
         input = input.view(config.micro_batch_size, config.seq_length, -1)
         # the weight-gradient product of the row projection behind the activation takes this result transposed when
@@ -348,7 +349,8 @@ class DCFunc:
         f = input.shape[-1] // 2
         want_t = (f < config.hidden_size and config.tokens * f >= WGRAD_TRANSPOSE_MIN_ELEMS
                   and wgrad_rows_ok(config.tokens, config.hidden_size)
-                  and not _host.wgrad_grouped(config.tokens, config.hidden_size, f))
+                  and not (grad_type in (None, input.dtype)             # (the grouped kernel adds to its operands' type only)
+                           and _host.wgrad_grouped(config.tokens, config.hidden_size, f)))
         output, _ = swiglu(input, stream, False, with_transposed=want_t)
         return output
 
@@ -387,7 +389,8 @@ class DCFunc:
     gemm_wgrad_mlp_l = gemm_wgrad_attn_l
 
     @staticmethod
-    def swiglu_bwd(config, data, stream):
+    def swiglu_bwd(config, data, stream, grad_type=None):
+        """``grad_type``: as for ``swiglu``."""
         swiglu_input, grad_output = data
         swiglu_input = swiglu_input.view(-1, swiglu_input.shape[-1])
         # the weight-gradient product of the column projection wants this gradient transposed when the layer is
@@ -395,7 +398,7 @@ class DCFunc:
         rows, n2 = swiglu_input.shape
         want_t = (config.hidden_size >= WGRAD_TRANSPOSE_GRAD_MIN_K and rows * n2 >= WGRAD_TRANSPOSE_MIN_ELEMS
                   and config.hidden_size >= n2 and wgrad_rows_ok(rows, n2)      # (fewer inputs than outputs: the input is the operand transposed)
-                  and not _host.wgrad_grouped(rows, n2, config.hidden_size))
+                  and not (grad_type in (None, swiglu_input.dtype) and _host.wgrad_grouped(rows, n2, config.hidden_size)))
         dgrad, _ = swiglu_back(grad_output, swiglu_input, None, stream, profiling=False, with_transposed=want_t)
         return dgrad
 
@@ -618,8 +621,14 @@ def _h_all_gather(c):
                               bwd_strand=bool(c.name) and c.name.endswith("_bwd"))
 
 
+def _other_grad_type(c, weight_key):
+    """{"grad_type": ...} where the gradient of that weight is kept in another type than the activations."""
+    grad = getattr(c.weight.get(weight_key), "main_grad", None)
+    return {} if grad is None or grad.dtype == c.x.dtype else {"grad_type": grad.dtype}
+
+
 def _h_swiglu(c):
-    output = c.dcfunc.swiglu(c.config, (c.x,), c.stream)
+    output = c.dcfunc.swiglu(c.config, (c.x,), c.stream, **_other_grad_type(c, "linear_mlp_weight"))
     c.act["swiglu_input"] = c.x
     return output
 
@@ -666,7 +675,7 @@ def _h_placeholder(c):
 
 
 def _h_swiglu_bwd(c):
-    output = c.dcfunc.swiglu_bwd(c.config, (c.g("swiglu_input"), c.x), c.stream)
+    output = c.dcfunc.swiglu_bwd(c.config, (c.g("swiglu_input"), c.x), c.stream, **_other_grad_type(c, "column_mlp_weight"))
     c.act["swiglu_dgrad"] = output
     return output
 

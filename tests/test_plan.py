@@ -126,3 +126,25 @@ def test_cu_mask_words():
         except ValueError:
             continue
         raise AssertionError(bad)
+
+
+@pytest.mark.parametrize("main_grad,twin", [("bfloat16", False), ("float32", True), (None, False)])
+def test_swiglu_writes_its_transpose_where_the_weight_gradient_will_read_it(monkeypatch, main_grad, twin):
+    """At these sizes the grouped kernel forms the weight gradients of 16-bit weights, without a transposed operand; it does not
+    add to an fp32 ``main_grad``, whose product the library forms from the transpose that the activation left."""
+    import torch
+    cfg = dstb.LayerConfig(hidden_size=8192, num_attention_heads=64, num_query_groups=8, ffn_hidden_size=28672, seq_length=4096,
+                           tensor_model_parallel_size=8)
+    meta = lambda *shape: torch.empty(*shape, dtype=torch.bfloat16, device="meta")
+    weights = {"linear_mlp_weight": meta(8192, 3584), "column_mlp_weight": meta(7168, 8192)}
+    if main_grad:
+        for w in weights.values():
+            w.main_grad = torch.empty(w.shape, dtype=getattr(torch, main_grad), device="meta")
+    asked = []
+    monkeypatch.setattr(dstb, "swiglu", lambda y, *a, with_transposed, **k: (asked.append(with_transposed), (y, 0))[1])
+    monkeypatch.setattr(dstb, "swiglu_back", lambda g, y, *a, with_transposed, **k: (asked.append(with_transposed), (y, 0))[1])
+    act = {"swiglu_input": meta(4096, 7168)}
+    run = lambda op, x: dstb._Ctx(dstb.DCFunc, op, cfg, weights, act, x, None, None, ())
+    dstb._h_swiglu(run(12, act["swiglu_input"]))
+    dstb._h_swiglu_bwd(run(21, meta(4096, 3584)))
+    assert asked == [twin, twin]
