@@ -1164,6 +1164,12 @@ static int bwd_hsplit(int max_sk, int batch, int hq, int hk, bool paired) {
 // A group that is left in pieces of several heads makes dK/dV's workgroups that much longer: from 512 rows on not here.  One
 // long sequence among short ones, whole calls, hand-ordered / here with the splits of the grid laid out for the longest / with
 // those of the work: 12 query / 4 kv heads x 791 + 76 + 32 77 / 86 / 57, 4 / 2 x 2746 + 7 135 / 168 / 117.
+// A batch of one long sequence and many short ones has a grid for 128-row tiles, most of it empty, and the work of a few 64-row
+// ones.  Backward, hand-ordered / two launches of the tile kernels / one: 8 heads, 1000 rows and 7 x 1 62 / 63 / 46, 4 query / 2 kv heads, 2163 and 7 x
+// 2 135 / 158 / 73, 12 / 4, 386 + 382 and 14 x 1 59 / 59 / 45.  Of 99 such batches of up to 24 sequences 5 are slower in one launch (by up to
+// 7 %); of 51 larger ones 17, by up to a third (4 heads, 599 and 47 x 1 51 / 58 / 68; 4 / 2, 451 and 31 more 57 / 58 / 76): not there.  At the
+// other head dims, where the two launches are these kernels too, such batches keep the 128-row dQ tiles.
+static bool dq_tile_fills(int max_sq, int hq, int batch) { return attn_wgs(max_sq, 128, hq, batch, 0) >= 2 * 256; }
 struct BwdBoth { bool pays; int hsplit; };      // key splits of a GQA group: by the workgroups with work
 static BwdBoth bwd_both(int batch, int max_sq, int max_sk, int64_t total_q, int64_t total_k, int hq, int hk, int d, int causal) {
   if (max_sq <= 0 || max_sk <= 0) return {false, 1};
@@ -1178,6 +1184,7 @@ static BwdBoth bwd_both(int batch, int max_sq, int max_sk, int64_t total_q, int6
   if (hs == hq / hk && (hs - 1) * cdiv(max_sq, d < 128 ? 128 : 64) <= (d == 64 ? 2 : d <= 128 ? 1 : 0)) hs = 1;
   const int64_t a = tiles(max_sq, total_q) * hq, b = tiles(max_sk, total_k) * hk * hs;
   if (d == 128) {
+    if (batch > 24 && dq_tile_fills(max_sq, hq, batch)) return {false, hs};
     if (max_sq >= 512 && (hs >= 8 || hs < hq / hk)) return {false, hs};      // (512 rows are never left whole above)
     if (!causal) return {a + b <= 256 && (max_sq == max_sk || batch == 1), hs};
     return {a + b <= 384 || (a + b <= 512 && max_sq >= 256 && max_sq < 1024), hs};
@@ -1211,8 +1218,9 @@ static AttnBwdRoute attn_bwd_route(int batch, int max_sq, int max_sk, int64_t to
   r.keep_ds = room_for_ds && max_sk > 0 && !short_rows;
   r.hand_dkv = d == 128 && !short_rows;
   r.hand_dq = r.hand_dkv && (!causal || !big || attn_causal_fills(max_sq, hq, batch, total_q));
-  r.big_dq = r.hand_dq ? big : d <= 128 && attn_wgs(max_sq, 128, hq, batch, 0) >= 2 * 256;
-  r.both = both.pays && !r.big_dq;
+  const bool fills = d <= 128 && dq_tile_fills(max_sq, hq, batch);
+  r.both = both.pays && (d == 128 || !fills);
+  r.big_dq = r.hand_dq ? big : fills && !r.both;
   r.hsplit = r.both ? both.hsplit : bwd_hsplit(max_sk, batch, hq, hk, d == 128 && causal);
   return r;
 }

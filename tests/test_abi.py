@@ -76,6 +76,18 @@ def test_attention_route(batch, max_q, total_q, hq, causal, hand):
     assert lib.dh_attn_bwd_path(batch, max_q, max_q, total_q, total_q, hq, hq, 96, causal, 1 << 40) & 7 == 0
 
 
+@pytest.mark.parametrize("lens,hq,hk,one,path", [
+    ([1000] + [1] * 7, 8, 8, 1, 0), ([1500] + [20] * 15, 4, 4, 1, 0), ([386, 382] + [1] * 14, 12, 4, 1, 0),
+    ([599] + [1] * 47, 4, 4, 0, 9), ([599] + [1] * 23, 4, 4, 1, 0)])
+def test_attention_backward_of_one_long_sequence_among_many_short_ones(lens, hq, hk, one, path):
+    """The one launch, or the hand-ordered dK/dV (1; 8: with 128-row dQ tiles): not the other kernels in two launches."""
+    _ensure_lib()
+    lib = _lib.load()
+    sizes = len(lens), max(lens), max(lens), sum(lens), sum(lens), hq, hk, 128, 1
+    assert lib.dh_attn_bwd_one_launch(*sizes) == one
+    assert lib.dh_attn_bwd_path(*sizes, 1 << 40) == path
+
+
 def test_product_does_not_import_the_oracle():
     """Nothing under dhellam_amd/ may import, read or run the oracle (it is the checker)."""
     for dirpath, _, files in list(os.walk(os.path.join(ROOT, "dhellam_amd"))) + list(os.walk(os.path.join(ROOT, "dhellam"))):
