@@ -83,15 +83,8 @@ def build(verbose: bool = False, jobs: int | None = None) -> Path:
     return LIB_PATH
 
 
-def check_grouped_gemm_loops(verbose: bool = False) -> int:
-    """The chip-filling grouped GEMM kernel (``grouped_gemm_w8_kernel``) copies its operands to LDS from assembly, which
-    the compiler does not count: that no copy overtakes a fragment read and no read a copy rests on the order of reads,
-    waits, copies and barriers that the source lays down.  This check holds the generated code to it.  It compiles
-    ``grouped_gemm.hip`` to device assembly and, in the main loop of every instantiation of the kernel (the innermost
-    loop with 128 MFMAs: two k slices), cuts the code at its barriers: clusters of 16 MFMAs have to alternate with
-    clusters of none, copies may stand in the latter only, each of these has to begin by waiting for the wavefront's
-    earlier LDS reads, and where copies are published the wait for them is the one the source counts.  It also refuses
-    scratch accesses and accumulator copies inside the loop.  Returns the number of loops checked; raises on a violation."""
+def grouped_gemm_assembly() -> list:
+    """The instantiations of ``grouped_gemm_w8_kernel`` as device assembly of ``grouped_gemm.hip``, a list of lines each."""
     import re
     import tempfile
     with tempfile.TemporaryDirectory() as td:
@@ -101,65 +94,109 @@ def check_grouped_gemm_loops(verbose: bool = False) -> int:
         if res.returncode != 0:
             raise RuntimeError("hipcc -S failed for grouped_gemm.hip:\n" + res.stderr)
         lines = out.read_text().split("\n")
+    starts = [i for i, l in enumerate(lines) if re.match(r"^_ZN2dh22grouped_gemm_w8_kernel\w+:", l)]
+    if not starts:
+        raise RuntimeError("no grouped_gemm_w8_kernel instantiation found in the assembly")
+    # (a kernel may hold several s_endpgm)
+    return [lines[a:next(i for i in range(a, len(lines)) if lines[i].startswith(".Lfunc_end"))] for a in starts]
 
-    checked = 0
-    for a in [i for i, l in enumerate(lines) if re.match(r"^_ZN2dh22grouped_gemm_w8_kernel\w+:", l)]:
-        b = next(i for i in range(a, len(lines)) if lines[i].startswith(".Lfunc_end"))   # (a kernel may hold several s_endpgm)
-        fn = lines[a:b]
-        name = fn[0].split(":")[0]
-        labels = {m.group(1): i for i, l in enumerate(fn) if (m := re.match(r"^(\.LBB\d+_\d+):", l))}
-        loops = []
-        for i, l in enumerate(fn):
-            m = re.match(r"\s+s_c?branch\w* (\.LBB\d+_\d+)", l)
-            if m and m.group(1) in labels and labels[m.group(1)] < i:
-                body = [x.split(";")[0].strip() for x in fn[labels[m.group(1)] + 1:i]]
-                body = [x for x in body if x and not x.endswith(":")]
-                if sum("v_mfma" in x for x in body) == 128:
-                    loops.append(body)
-        if not loops:
-            raise RuntimeError(f"{name}: no main loop with 128 MFMAs found (the kernel's structure changed: update "
-                               "check_grouped_gemm_loops)")
-        body = min(loops, key=len)
-        for l in body:
-            if "scratch_" in l or "v_accvgpr" in l:
-                raise RuntimeError(f"{name}: '{l}' inside the main loop")
-        clusters, cluster = [], []
-        for l in body:
-            if l.startswith("s_barrier"):
-                clusters.append(cluster)
-                cluster = []
-            else:
-                cluster.append(l)
-        clusters[0] = cluster + clusters[0]                  # what follows the last barrier runs into the loop's head
-        if len(clusters) != 16:
-            raise RuntimeError(f"{name}: {len(clusters)} barriers in the main loop, expected 16")
-        copies = 0
+
+def check_grouped_gemm_loops(verbose: bool = False) -> int:
+    """The chip-filling grouped GEMM kernel (``grouped_gemm_w8_kernel``) copies its operands to LDS from assembly, which
+    the compiler does not count: that no copy overtakes a fragment read and no read a copy rests on the order of reads,
+    waits, copies and barriers that the source lays down.  This holds the generated code of every instantiation to it
+    (``check_grouped_gemm_order``).  Returns the number of instantiations checked; raises on a violation."""
+    kernels = grouped_gemm_assembly()
+    for fn in kernels:
+        body = check_grouped_gemm_order(fn)
+        if verbose:
+            print(f"checked {fn[0].split(':')[0]}: {body} lines", flush=True)
+    return len(kernels)
+
+
+def check_grouped_gemm_order(fn: list) -> int:
+    """One instantiation of ``grouped_gemm_w8_kernel`` as assembly: the copies of the first two slices, published by the
+    counted wait and a barrier before anything is read, and one more barrier for half of the wavefronts; the main loop (the
+    innermost loop with 128 MFMAs: two slices) and, behind it, the last slice of an odd number.  In the slices, cut at their
+    barriers, clusters of 16 MFMAs have to alternate with clusters of none, copies may stand in the latter only, each of these
+    has to begin by waiting for the wavefront's earlier LDS reads, and where copies are published the wait for them is the one
+    the source counts.  Behind the last slice everything has landed, past a barrier, before LDS is used again.  No scratch
+    accesses, no copies of accumulators, and no register moves among MFMAs.  Returns the lines of the loop."""
+    import re
+    name = fn[0].split(":")[0]
+    code = [l.split(";")[0].strip() for l in fn]
+    labels = {m.group(1): i for i, l in enumerate(code) if (m := re.match(r"^(\.LBB\d+_\d+):", l))}
+    mfmas = lambda part: sum("v_mfma" in x for x in part)
+    barriers = lambda part: [i for i, x in enumerate(part) if x.startswith("s_barrier")]
+    copies = lambda part: [i for i, x in enumerate(part) if x.startswith("buffer_load")]
+
+    def need(ok, what):
+        if not ok:
+            raise RuntimeError(f"{name}: {what}")
+
+    loops = []
+    for i, l in enumerate(code):
+        m = re.match(r"s_c?branch\w* (\.LBB\d+_\d+)", l)
+        if m and m.group(1) in labels and labels[m.group(1)] < i and mfmas(code[labels[m.group(1)] + 1:i]) == 128:
+            loops.append((labels[m.group(1)] + 1, i))
+    need(loops, "no main loop with 128 MFMAs found (the kernel's structure changed: update check_grouped_gemm_order)")
+    lo, hi = min(loops, key=lambda x: x[1] - x[0])
+    plain = lambda part: [x for x in part if x and not x.endswith(":")]
+    first, body, rest = plain(code[:lo]), plain(code[lo:hi]), plain(code[hi:])
+    need(mfmas(first) == 0 and mfmas(rest) == 64, f"{mfmas(first)} and {mfmas(rest)} MFMAs before and behind the main loop, expected 0 and 64")
+
+    def check_slices(clusters, where):
+        total = 0
         for n, cl in enumerate(clusters):
-            mfma = sum("v_mfma" in x for x in cl)
-            dma = [i for i, x in enumerate(cl) if x.startswith("buffer_load")]
-            if mfma != (16 if n % 2 else 0):
-                raise RuntimeError(f"{name}: cluster {n} holds {mfma} MFMAs")
-            copies += len(dma)
+            dma = copies(cl)
+            need(mfmas(cl) == (16 if n % 2 else 0), f"{where}: cluster {n} holds {mfmas(cl)} MFMAs")
+            need(not any("scratch_" in x or "v_accvgpr" in x for x in cl), f"{where}: scratch or accumulator copies in cluster {n}")
+            total += len(dma)
             if n % 2:
-                if dma:
-                    raise RuntimeError(f"{name}: a copy among the MFMAs of cluster {n}")
+                need(not dma, f"{where}: a copy among the MFMAs of cluster {n}")
+                need(not any(x.startswith("v_mov_b") for x in cl), f"{where}: a register move among the MFMAs of cluster {n}")
                 continue
             waits = [i for i, x in enumerate(cl) if x == "s_waitcnt lgkmcnt(0)"]
             reads = [i for i, x in enumerate(cl) if x.startswith("ds_read")]
-            if not waits or (reads and reads[0] < waits[0]) or (dma and dma[0] < waits[0]):
-                raise RuntimeError(f"{name}: cluster {n} does not begin with the wait for the earlier reads")
-            if any(not x.endswith("lds") for x in (cl[i] for i in dma)):
-                raise RuntimeError(f"{name}: a load to registers in cluster {n}")
-            if dma and "s_waitcnt vmcnt(8)" not in cl[dma[-1]:]:
-                raise RuntimeError(f"{name}: cluster {n} publishes copies without the counted wait")
-        if copies != 16:
-            raise RuntimeError(f"{name}: {copies} copies in the main loop, expected 16")
-        checked += 1
-        if verbose:
-            print(f"checked {name}: {len(body)} lines", flush=True)
-    if checked == 0:
-        raise RuntimeError("no grouped_gemm_w8_kernel instantiation found in the assembly")
-    return checked
+            need(waits and not (reads and reads[0] < waits[0]) and not (dma and dma[0] < waits[0]),
+                 f"{where}: cluster {n} does not begin with the wait for the earlier reads")
+            need(all(cl[i].endswith("lds") for i in dma), f"{where}: a load to registers in cluster {n}")
+            need(not dma or "s_waitcnt vmcnt(8)" in cl[dma[-1]:], f"{where}: cluster {n} publishes copies without the counted wait")
+        need(total == len(clusters), f"{where}: {total} copies, expected {len(clusters)}")
+
+    def cut(part):
+        at = [-1] + barriers(part)
+        return [part[x + 1:y] for x, y in zip(at, at[1:])], part[at[-1] + 1:]
+
+    # the first two slices
+    dma = copies(first)
+    need(len(dma) == 16 and all(first[i].endswith("lds") for i in dma), f"{len(dma)} loads before the main loop, expected 16 copies")
+    need("s_waitcnt vmcnt(0)" in first[:dma[0]], "the stores before the first copies are not waited for")
+    behind = first[dma[-1] + 1:]
+    bars = barriers(behind)
+    need(len(bars) == 2, f"{len(bars)} barriers between the first copies and the main loop, expected 2")
+    need("s_waitcnt vmcnt(8)" in behind[:bars[0]], "the first slice is published without the counted wait")
+    reads = [i for i, x in enumerate(first) if x.startswith("ds_read")]
+    need(reads and reads[0] > dma[-1] + 1 + bars[1], "a fragment is read before the first slice is published")
+    # the loop
+    clusters, head = cut(body)
+    need(len(clusters) == 16, f"{len(clusters)} barriers in the main loop, expected 16")
+    clusters[0] = head + clusters[0]                     # what follows the last barrier runs into the loop's head
+    check_slices(clusters, "main loop")
+    # the last slice of an odd number
+    at = barriers(rest)
+    need(len(at) >= 10, f"{len(at)} barriers behind the main loop, expected 10 and more")
+    clusters, _ = cut(rest[:at[7] + 1])
+    waits = [i for i, x in enumerate(clusters[0]) if x == "s_waitcnt lgkmcnt(0)"]    # (the blocks that the branches over it lead to)
+    need(waits and not any(x.startswith("ds_read") for x in clusters[0][:waits[-1]]), "last slice: a read before the wait for the earlier ones")
+    clusters[0] = clusters[0][waits[-1]:]
+    check_slices(clusters, "last slice")
+    # and what follows: the other half's barrier, the last copies, a barrier, and only then LDS again
+    behind = rest[at[7] + 1:]
+    used = next((i for i, x in enumerate(behind) if x.startswith(("ds_", "global_store", "buffer_load"))), len(behind))
+    landed = next((i for i, x in enumerate(behind) if re.match(r"s_waitcnt vmcnt\(0\)", x)), len(behind))
+    need(landed < used and any(landed < i < used for i in barriers(behind)), "LDS is used again before the last copies have landed")
+    return len(body)
 
 
 EXT_PKG = ROOT / "dhellam"

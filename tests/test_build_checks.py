@@ -4,8 +4,11 @@ import shutil
 import pytest
 
 
-@pytest.mark.skipif(shutil.which("hipcc") is None and not __import__("os").path.exists("/opt/rocm/bin/hipcc"),
-                    reason="needs hipcc")
+needs_hipcc = pytest.mark.skipif(shutil.which("hipcc") is None and not __import__("os").path.exists("/opt/rocm/bin/hipcc"),
+                                 reason="needs hipcc")
+
+
+@needs_hipcc
 def test_grouped_gemm_loads_are_left_alone_until_used():
     """The chip-filling grouped GEMM copies its operands to LDS from assembly and orders reads, waits, copies and barriers
     by hand: the compiled loop has to keep that order, without spills, in all of the ten instantiations (NT / NN with and
@@ -13,6 +16,28 @@ def test_grouped_gemm_loads_are_left_alone_until_used():
     verifies that; a violation raises."""
     from dhellam_amd.build import check_grouped_gemm_loops
     assert check_grouped_gemm_loops() == 10
+
+
+@pytest.fixture(scope="module")
+def gemm_kernels():
+    from dhellam_amd.build import grouped_gemm_assembly
+    return grouped_gemm_assembly()
+
+
+@needs_hipcc
+@pytest.mark.parametrize("where", ["before the loop", "main loop", "last slice", "behind it"])
+def test_grouped_gemm_check_covers_the_first_and_the_last_slices(gemm_kernels, where):
+    """A counted wait that is missing anywhere on the way is found: in front of the main loop, in it, in the separately compiled
+    slice of an odd number, and the last wait before LDS is used again."""
+    from dhellam_amd.build import check_grouped_gemm_order
+    for fn in gemm_kernels:
+        counted = [i for i, l in enumerate(fn) if l.strip() == "s_waitcnt vmcnt(8)"]
+        assert len(counted) == 1 + 6 + 3
+        last = next(i for i in range(counted[-1], len(fn)) if fn[i].strip().startswith("s_waitcnt vmcnt(0)"))
+        bad = list(fn)
+        bad[{"before the loop": counted[0], "main loop": counted[3], "last slice": counted[8], "behind it": last}[where]] = ""
+        with pytest.raises(RuntimeError):
+            check_grouped_gemm_order(bad)
 
 
 def test_weight_gradients_of_very_long_rows_stay_with_the_library():
