@@ -87,6 +87,7 @@ SIGNATURES = {
     "dh_grouped_gemm_nn": (_i32, [_vp] * 4 + [_i32, _i64, _i64, _i64, _i32, _vp, _sz, _vp]),
     "dh_grouped_gemm_tn": (_i32, [_vp] * 4 + [_i32, _i64, _i64, _i64, _i32, _i32, _vp]),
     "dh_grouped_gemm_tn_ws": (_i32, [_vp] * 4 + [_i32, _i64, _i64, _i64, _i32, _i32, _vp, _sz, _vp]),
+    "dh_grouped_gemm_tn_tiles": (_i32, [_i32, _i64, _i64, _i64, _i32]),
 }
 
 _lib = None

@@ -1120,7 +1120,7 @@ static int dispatch_gg_t(const GGParams &p, int64_t m_extent, void *workspace, s
     return DH_OK;
   }
   if constexpr (FORM == 2) {
-    // (the one-stage form: above.  Accumulating, only products of few tiles come here)
+    // (the one-stage form: above.  Accumulating, only products of few tiles and narrow ones come here)
     if (!p.accumulate && p.groups * cdiv(p.m_dim, 128) * cdiv(p.n_dim, 128) > 512)
       return launch_gg_t<T, FORM, 128, 128, 1>(p, m_extent, workspace, workspace_bytes, st);
     return launch_gg_t<T, FORM, 128, 128>(p, m_extent, workspace, workspace_bytes, st);
@@ -1188,15 +1188,26 @@ static bool gg_w8_pays(int64_t rows, int groups, int64_t n, int64_t k) {
 // asked for); us, 256x256 / 128x128 tiles: 16 groups of 5632 x 4096: 192 rows 275 / 289, 512 452 / 496, 1024 726 / 844; 8 groups of 5632 x
 // 1024: 256 rows 47 / 41, 1024 100 / 104.  Accumulating, which the smaller tiles do with 8-byte accesses, from two thirds of a
 // tile for every compute unit on: 16 groups of 5632 x 4096: 16 rows 267 / 569, 256 364 / 684; of 1408 x 512 (192 tiles) 11 / 20, 18 / 27; one
-// group of 16 rows, 4096 x 4096 13 / 33, of 256 rows, 1280 x 8192 15 / 24, but 8192 x 1024 (128 tiles) 15 / 16, of 4096 rows 84 / 74.
+// group of 16 rows, 4096 x 4096 13 / 33, of 256 rows, 1280 x 8192 15 / 24, but 8192 x 1024 (128 tiles) 15 / 16, of 4096 rows 84 / 74.  Not where
+// most of a tile is past the matrix: as fast as the smaller ones where a third of it is output (500 products of up to 480 columns
+// the narrow way; up to a tenth 0.58 of their speed, to 0.2 0.8, to 0.3 0.9, 0.3 to 0.4 1.0, 0.5 to 0.6 1.17, beyond 0.7 1.5).
 static bool gg_w8_tn_pays(int64_t rows, int groups, int64_t m, int64_t n, int accumulate) {
   const int64_t avg = rows / groups;
   const double ns = (double)cdiv(avg, 64);
   const int64_t tiles = groups * cdiv(m, 256) * cdiv(n, 256), small = groups * cdiv(m, 128) * cdiv(n, 128);
-  if (accumulate && tiles >= 160) return true;
+  if (accumulate && tiles >= 160 && 100 * m * n >= 35 * 65536 * (tiles / groups)) return true;
   if (avg < 192) return false;
   return (double)cdiv(tiles, 256) * (8.5 + 1.38 * ns) * (avg < 384 ? 1.1 : 1.0) <
          (accumulate || small <= 512 ? 0.8 + (double)small / 512 * (3.5 + 1.11 * ns) : (double)small / 1024 * (6.3 + 1.85 * ns));
+}
+
+// Tiles of a TN product: 256, 128 (dispatch_gg_t), or 0 (rows too long for tiles).  The offsets of the 256x256 tiles have to fit
+// the 32-bit buffer addressing: of the operands, of the 64 rows of a slice, however few of them there are, and, accumulating, of
+// a tile's 256 rows of c.  (Otherwise the rows that gg_w8_tn_pays asks for keep them short.)
+static int gg_tn_tiles(int64_t rows, int groups, int64_t m, int64_t n, int accumulate) {
+  const bool fits = rows * (m > n ? m : n) * 2 < (1ll << 31) && (!accumulate || (m <= GG_MAX_LD && n <= GG_MAX_LD));
+  if (fits && gg_w8_tn_pays(rows, groups, m, n, accumulate)) return 256;
+  return m > GG_MAX_LD || n > GG_MAX_LD ? 0 : 128;
 }
 
 static int gg_common_checks(const void *a, const void *b, void *c, const int32_t *offs, int groups, int dtype) {
@@ -1276,11 +1287,7 @@ extern "C" int dh_grouped_gemm_tn_ws(const void *a, const void *b, void *c, cons
   p.a = a; p.b = b; p.c = c; p.offs = offs; p.groups = groups;
   p.m_dim = m; p.n_dim = n; p.lda = m; p.ldb = n; p.ldc = n;
   p.c_group_stride = m * n; p.accumulate = accumulate; p.max_rows = (int)max_rows;
-  // The offsets of the 256x256 tiles have to fit the 32-bit buffer addressing: of the operands, of the 64 rows of a slice, however
-  // few of them there are, and, accumulating, of a tile's 256 rows of c.  (Otherwise the rows asked for above keep them short.)
-  const bool fits = max_rows * (m > n ? m : n) * (int64_t)dtype_size(dtype) < (1ll << 31) &&
-                    (!accumulate || (m <= GG_MAX_LD && n <= GG_MAX_LD));
-  if (fits && gg_w8_tn_pays(max_rows, groups, m, n, accumulate))
+  if (gg_tn_tiles(max_rows, groups, m, n, accumulate) == 256)
     rc = dtype == DH_BF16 ? launch_gg_w8_tn<bf16_t>(p, (hipStream_t)stream) : launch_gg_w8_tn<f16_t>(p, (hipStream_t)stream);
   else
     rc = dtype == DH_BF16 ? dispatch_gg_t<bf16_t, 2>(p, m, workspace, workspace_bytes, (hipStream_t)stream)
@@ -1288,6 +1295,10 @@ extern "C" int dh_grouped_gemm_tn_ws(const void *a, const void *b, void *c, cons
   if (rc) return rc;
   DH_LAUNCH_CHECK();
   return DH_OK;
+}
+
+extern "C" int dh_grouped_gemm_tn_tiles(int groups, int64_t max_rows, int64_t m, int64_t n, int accumulate) {
+  return groups < 1 || max_rows < 0 || m <= 0 || n <= 0 ? 0 : dh::gg_tn_tiles(max_rows, groups, m, n, accumulate);
 }
 
 extern "C" int dh_grouped_gemm_tn(const void *a, const void *b, void *c, const int32_t *offs, int groups,

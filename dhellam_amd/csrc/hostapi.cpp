@@ -448,18 +448,18 @@ bool dgrad_grouped(int64_t t, int64_t n, int64_t k) {
 // 14 / 16, 31 / 29, 44 / 44, 69 / 83.  Few rows, T = 16, 64, 100: 32000, 4096 126 / 96, 121 / 103, 145 / 112; 4096, 4096 18 / 13, 16 / 14,
 // 21 / 15; 1280, 8192 14 / 11, 13 / 11, 26 / 12.  Small weights of few rows: 3072, 1024 at 64, 256, 368 10.4 / 7.6, 10.5 / 9.4, 12.4 / 10.5, at 512
 // 12.2 / 12.4.
-// Narrow weights fill a part of their tiles only, and the rest is stored as slowly.  N, K with the share that is output, times as fast
-// here as the library, T = 24, 64, 200, 1000, 2000, 4096: 100000, 8 (0.03) 5.8, 0.69, 0.70, 0.87, 1.07, 0.83; 100000, 32 (0.12) 6.7, 0.72, 0.79,
-// 1.24, 1.30, 0.89; 50304, 64 (0.25) 1.23, 1.23, 0.90, 0.96, 0.80, 0.72; 50304, 96 (0.37) 1.54, 1.40, 1.33, 1.29, 0.99, 0.85; 128, 50304 (0.50) 1.85, 1.66, 1.54,
-// 1.24, 0.96, 0.81; 264, 30000 (0.51) 2.2, 2.0, 1.85, 1.45, 1.25, 0.86; 50304, 192 (0.75) 1.34 at 32, 1.41, 1.30, 1.36, 1.13.
+// Narrow weights fill a part of their tiles only, and the rest is computed all the same: long reductions are better off with the
+// library.  N, K with the share of the 256x256 tiles that is output, times as fast here, T = 24, 64, 200, 1000, 2000, 4096: 100000, 8
+// (0.03) 12.7, 1.48, 1.23, 1.28, 1.33, 1.01; 32, 100000 (0.12) 8.2, 0.98, 1.03, 1.64, 1.57, 1.08; 50304, 64 (0.25) 1.27, 1.25, 1.02, 1.10, 0.98, 0.84; 50304, 96
+// (0.37) 1.56, 1.39, 1.30, 1.29, 1.01, 0.86; 128, 50304 (0.50) 1.85, 1.66, 1.53, 1.23, 0.97, 0.84; 264, 30000 (0.51) 2.2, 2.0, 1.83, 1.43, 1.25, 0.85; 50304, 192
+// (0.75) 1.34 at 32, 1.41, 1.30, 1.36, 1.13.
 bool wgrad_grouped(int64_t t, int64_t n, int64_t k) {
   const int64_t tiles = (n + 255) / 256 * ((k + 255) / 256);
   if (t <= 0 || n > kGroupedMaxRow || k > kGroupedMaxRow) return false;
   if (tiles < 160) return t <= 384 && n * k <= 3200000;
   if ((tiles < 224 && t % 64 == 0 && t >= 2048) || 2 * t * std::max(n, k) >= (int64_t)1 << 31) return false;
   const double share = (double)(n * k) / (double)(tiles * 65536);
-  if (share >= 0.7) return true;
-  return t <= (share < 0.15 ? 32 : share < 0.3 ? 128 : std::min(n, k) <= 128 ? 1500 : 3500);
+  return share >= 0.7 || t <= (std::min(n, k) <= 128 ? 1500 : 3500);
 }
 
 // out [N, K] (+)= grad [T, N]^T @ data [T, K] by the grouped kernel; false, and nothing done, where it is not the faster one or does

@@ -420,6 +420,10 @@ int dh_grouped_gemm_tn_ws(const void *a, const void *b, void *c,
                           const int32_t *offs, int groups, int64_t max_rows,
                           int64_t m, int64_t n, int accumulate, int dtype,
                           void *workspace, size_t workspace_bytes, void *stream);
+/* The tiles that a TN call of these sizes runs on: 256 (256x256), 128 (128x128),
+ * 0: rows too long for tiles, or nothing to do. */
+int dh_grouped_gemm_tn_tiles(int groups, int64_t max_rows, int64_t m, int64_t n,
+                             int accumulate);
 
 /* Zeros in n device buffers (16-byte aligned, sizes multiples of 4), one launch for up to 32 of them. */
 int dh_zero_many(void *const *ptrs, const int64_t *nbytes, int n, void *stream);

@@ -74,10 +74,22 @@ def test_data_gradients_go_where_they_were_measured_the_faster(t, n, k, grouped)
 
 
 @pytest.mark.parametrize("t,n,k,grouped", [
-    (24, 100000, 8, 1), (64, 100000, 8, 0), (200, 8, 100000, 0), (32, 32, 100000, 1), (64, 100000, 32, 0),
-    (128, 50304, 64, 1), (2000, 50304, 64, 0), (8192, 64, 65536, 0), (1000, 50304, 96, 1), (2000, 50304, 96, 0), (1000, 128, 50304, 1),
+    (24, 100000, 8, 1), (1000, 8, 100000, 1), (4096, 100000, 8, 0), (32, 32, 100000, 1), (1000, 100000, 32, 1),
+    (1000, 50304, 64, 1), (2000, 50304, 64, 0), (8192, 64, 65536, 0), (1000, 50304, 96, 1), (2000, 50304, 96, 0), (1000, 128, 50304, 1),
     (2000, 128, 50304, 0), (3000, 264, 30000, 1), (4096, 30000, 264, 0), (8192, 320, 65536, 0), (2000, 192, 50304, 1), (8192, 512, 50304, 1),
     (4096, 7168, 8192, 1), (4096, 8192, 3584, 1), (4096, 1280, 8192, 0), (1000, 1280, 8192, 1), (384, 32000, 96, 1), (385, 1280, 2048, 0)])
 def test_weight_gradients_go_where_they_were_measured_the_faster(t, n, k, grouped):
     from dhellam_amd import _host
     assert _host.wgrad_grouped(t, n, k) == bool(grouped)
+
+
+@pytest.mark.parametrize("groups,rows,m,n,accumulate,tiles", [
+    (16, 256, 5632, 4096, 1, 256), (1, 16, 4096, 4096, 1, 256), (32, 64, 1304, 136, 1, 256), (8, 2048, 5632, 1024, 0, 128),
+    (8, 16384, 5632, 4096, 0, 256), (16, 1600, 5632, 4096, 0, 128), (1, 4096, 8192, 1024, 1, 128),
+    # most of a 256-wide tile past the matrix
+    (32, 64, 5552, 8, 1, 128), (64, 6400, 16, 4112, 1, 128), (16, 4465, 32, 10704, 1, 128), (64, 1446, 1056, 80, 1, 128),
+    # rows past the 32-bit offsets of a tile's old values
+    (1, 16, 256, 4300800, 1, 0), (1, 16, 4300800, 256, 1, 0), (1, 16, 256, (1 << 22) - 8, 1, 256)])
+def test_tiles_of_a_grouped_weight_gradient(groups, rows, m, n, accumulate, tiles):
+    from dhellam_amd import _lib
+    assert _lib.load().dh_grouped_gemm_tn_tiles(groups, rows, m, n, accumulate) == tiles
