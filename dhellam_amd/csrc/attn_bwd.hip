@@ -1161,6 +1161,9 @@ static int bwd_hsplit(int max_sk, int batch, int hq, int hk, bool paired) {
 //   causal: 8 x 1500 62 / 84, 32 x 512 36 / 41.
 // A group split eight ways from 512 rows on (8 query / 1 kv head x 1024: 58 / 46) and rectangular calls of several sequences that
 // are not causal stay with the hand-ordered kernels: callers size the workspace there to choose between their two forms of dQ.
+// Few query rows of many keys are not for it either: dQ is a long chain of key tiles for a few workgroups here and a product over kept dS
+// there: 8 query / 1 kv head x 27 rows x 5086 keys 60 / 122, 4 / 2 x 66 x 918 28 / 33, 1 / 1 x 363 x 1427 31 / 40, 1423 x 2767 60 / 69, but
+// 1833 x 2547 70 / 64 and 12 / 4 x 193 x 450 30 / 26.
 // A group that is left in pieces of several heads makes dK/dV's workgroups that much longer: from 512 rows on not here.  One
 // long sequence among short ones, whole calls, hand-ordered / here with the splits of the grid laid out for the longest / with
 // those of the work: 12 query / 4 kv heads x 791 + 76 + 32 77 / 86 / 57, 4 / 2 x 2746 + 7 135 / 168 / 117.
@@ -1186,7 +1189,7 @@ static BwdBoth bwd_both(int batch, int max_sq, int max_sk, int64_t total_q, int6
   if (d == 128) {
     if (batch > 24 && dq_tile_fills(max_sq, hq, batch)) return {false, hs};
     if (max_sq >= 512 && (hs >= 8 || hs < hq / hk)) return {false, hs};      // (512 rows are never left whole above)
-    if (!causal) return {a + b <= 256 && (max_sq == max_sk || batch == 1), hs};
+    if (!causal) return {a + b <= 256 && (max_sq == max_sk || (batch == 1 && (max_sk <= 600 || 2 * (int64_t)max_sk <= 3 * (int64_t)max_sq))), hs};
     return {a + b <= 384 || (a + b <= 512 && max_sq >= 256 && max_sq < 1024), hs};
   }
   if (a + b <= (causal ? 384 : 256)) return {true, hs};

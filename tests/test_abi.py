@@ -88,6 +88,13 @@ def test_attention_backward_of_one_long_sequence_among_many_short_ones(lens, hq,
     assert lib.dh_attn_bwd_path(*sizes, 1 << 40) == path
 
 
+@pytest.mark.parametrize("q,k,one", [(12, 7147, 0), (363, 1427, 0), (44, 601, 0), (44, 600, 1), (600, 900, 1), (600, 901, 0), (3000, 20, 1)])
+def test_attention_backward_of_few_rows_and_many_keys(q, k, one):
+    """At head dim 128, not causal: dQ of a few rows over many keys is not left to the few workgroups of the one launch."""
+    _ensure_lib()
+    assert _lib.load().dh_attn_bwd_one_launch(1, q, k, q, k, 1, 1, 128, 0) == one
+
+
 def test_product_does_not_import_the_oracle():
     """Nothing under dhellam_amd/ may import, read or run the oracle (it is the checker)."""
     for dirpath, _, files in list(os.walk(os.path.join(ROOT, "dhellam_amd"))) + list(os.walk(os.path.join(ROOT, "dhellam"))):

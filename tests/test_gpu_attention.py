@@ -454,6 +454,7 @@ def test_attention_chip_filling_tiles_of_other_head_dims(dtype, d, lens, hq, hk,
     (128, [1000] + [1] * 7, [1000] + [1] * 7, 8, 8, True, 1), (128, [3, 421, 5] + [2] * 13, [3, 421, 5] + [2] * 13, 8, 8, True, 1),
     (128, [599] + [1, 2] * 23, [599] + [1, 2] * 23, 4, 4, True, 0),     # ... of a grid for 128-row tiles
     (128, [224], [112], 4, 2, False, 1), (128, [97], [200], 6, 2, False, 1), (128, [300, 40], [200, 97], 4, 2, False, 0),
+    (128, [44], [1300], 4, 2, False, 0), (128, [3], [600], 6, 2, False, 1), (128, [450], [675], 1, 1, False, 1),      # many keys
     (192, [97, 2], [97, 2], 4, 2, True, 1), (192, [65], [31], 2, 2, False, 1),
     (256, [129, 60], [129, 60], 2, 1, True, 1), (256, [32], [64], 4, 4, False, 1), (64, [50, 0], [20, 70], 2, 2, False, 1),
 ])
