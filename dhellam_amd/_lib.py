@@ -74,6 +74,7 @@ SIGNATURES = {
     "dh_attn_bwd_halves": (_i32, [_vp] * 11 + [_sz] + [_vp] * 2 + [_i32] * 6 + [_i64] * 2 + [_i32] * 3 + [_i64] * 8 + [_f32, _i32, _i32, _i32, _vp]),
     "dh_attn_merge": (_i32, [_vp, _vp, _vp, _vp, _i32, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _vp]),
     "dh_moe_route_topk": (_i32, [_vp, _vp, _vp, _i64, _i32, _i32, _vp]),
+    "dh_moe_route_lanes": (_i32, [_i64, _i32, _i32]),
     "dh_moe_sort_workspace_bytes": (_sz, [_i64, _i32]),
     "dh_moe_sort": (_i32, [_vp] * 6 + [_sz, _i64, _i32, _vp]),
     "dh_moe_sort_static_max_assign": (_i64, []),

@@ -20,11 +20,63 @@ constexpr int MOE_MAX_E = 64;
 constexpr int MOE_MAX_K = 8;
 constexpr int SORT_ITEMS = 1024;  // assignments per block (4 rounds of 256)
 
-// Top K of E logits a token, E lanes (the next power of two) holding one each.  In every round the best of what is left: the
-// largest, of equals the lowest expert id, a NaN only where the lowest id that is left holds one (the rule of a scan that
-// starts there and moves on to what is greater).  A thread a token, scanning its row K times, was a chain of K E dependent
-// loads on a few workgroups: 3316 tokens of 64 experts, 8 of them chosen, 78 -> 10 us, 1914 of 16, 4 chosen, 11 -> 5, 8192 of 8, 2
-// chosen, 6.8 -> 4.8.
+// Top K of E logits a token.  In every round the best of what is left: the largest, of equals the lowest expert id, a NaN only
+// where the lowest id that is left holds one (the rule of a scan that starts there and moves on to what is greater).
+// Two forms.  A thread a token scans its row K times: a chain of K E dependent loads, with few tokens on a few workgroups.  E lanes
+// (the next power of two) a token hold one logit each and compare by exchange: short, but E times the lanes.
+// us, scan / lanes, at T tokens: 64 experts, 8 chosen 1000 85 / 7.5, 16384 78 / 26, 65536 82 / 91, 131072 237 / 180, 1 chosen 16384 10.1 / 8.2, 65536 11.6 / 23.8;
+// 24, 2 chosen 16384 7.5 / 6.0, 65536 7.7 / 17.9; 8, 2 chosen 1000 3.9 / 2.9, 32768 3.9 / 3.8, 131072 5.7 / 9.0; 2, 1 chosen 64 1.9 / 2.3, 65536 2.4 / 4.6.
+// The line follows what the two cost: 1.7 + 0.15 K E us, flat up to 65536 tokens (a workgroup a compute unit), against 2.2 + 0.25 K and
+// 0.05 + 0.036 K ns for every 16 lanes; past them scans of up to 24 logits, or of one round, stay the faster.
+static int moe_route_lanes(int64_t tokens, int E, int K) {
+  const int lanes = E <= 8 ? 8 : E <= 16 ? 16 : E <= 32 ? 32 : 64;
+  if (tokens > 80000) return E <= 24 || K == 1 ? 1 : lanes;
+  return (double)tokens * lanes * (3.0 + 2.3 * K) > (0.15 * K * E - 0.5 - 0.25 * K) * 1e6 ? 1 : lanes;
+}
+
+__global__ void __launch_bounds__(256)
+moe_route_scan_kernel(const float *__restrict__ logits, int32_t *__restrict__ topk_idx, float *__restrict__ gates,
+                      int64_t tokens, int E, int K) {
+  for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < tokens; t += (int64_t)gridDim.x * 256) {
+    const float *row = logits + t * E;
+    uint64_t taken = 0;
+    float sel[MOE_MAX_K];
+    int idx[MOE_MAX_K];
+#pragma unroll
+    for (int j = 0; j < MOE_MAX_K; ++j) {
+      if (j < K) {
+        int best = -1;
+        float bv = 0.f;
+        for (int e = 0; e < E; ++e) {
+          if ((taken >> e) & 1) continue;
+          const float v = row[e];
+          if (best < 0 || v > bv) {
+            best = e;
+            bv = v;
+          }
+        }
+        taken |= (uint64_t)1 << best;
+        sel[j] = bv;
+        idx[j] = best;
+      }
+    }
+    float den = 0.f;
+    float ex[MOE_MAX_K];
+#pragma unroll
+    for (int j = 0; j < MOE_MAX_K; ++j)
+      if (j < K) {
+        ex[j] = expf(sel[j] - sel[0]);
+        den += ex[j];
+      }
+#pragma unroll
+    for (int j = 0; j < MOE_MAX_K; ++j)
+      if (j < K) {
+        topk_idx[t * K + j] = idx[j];
+        gates[t * K + j] = ex[j] / den;
+      }
+  }
+}
+
 template <int G>
 __global__ void __launch_bounds__(256)
 moe_route_kernel(const float *__restrict__ logits, int32_t *__restrict__ topk_idx, float *__restrict__ gates,
@@ -509,6 +561,10 @@ moe_unpermute_bwd_kernel(const T *__restrict__ dout, const T *__restrict__ y, co
 
 }  // namespace dh
 
+extern "C" int dh_moe_route_lanes(int64_t tokens, int experts, int k) {
+  return tokens < 1 || experts < 1 || experts > dh::MOE_MAX_E || k < 1 || k > experts || k > dh::MOE_MAX_K ? 0 : dh::moe_route_lanes(tokens, experts, k);
+}
+
 extern "C" int dh_moe_route_topk(const float *logits, int32_t *topk_idx, float *gates, int64_t tokens, int experts,
                                  int k, void *stream) {
   using namespace dh;
@@ -517,10 +573,10 @@ extern "C" int dh_moe_route_topk(const float *logits, int32_t *topk_idx, float *
   DH_CHECK(k >= 1 && k <= MOE_MAX_K && k <= experts, "k=%d must be in [1, min(%d, experts)]", k, MOE_MAX_K);
   if (tokens == 0) return DH_OK;
   DH_CHECK(logits && topk_idx && gates, "null pointer");
-  const int lanes = experts <= 8 ? 8 : experts <= 16 ? 16 : experts <= 32 ? 32 : 64;
+  const int lanes = moe_route_lanes(tokens, experts, k);
   int64_t blocks = cdiv(tokens, 256 / lanes);
   if (blocks > 4096) blocks = 4096;
-  const auto kernel = lanes == 8 ? moe_route_kernel<8> : lanes == 16 ? moe_route_kernel<16> : lanes == 32 ? moe_route_kernel<32> : moe_route_kernel<64>;
+  const auto kernel = lanes == 1 ? moe_route_scan_kernel : lanes == 8 ? moe_route_kernel<8> : lanes == 16 ? moe_route_kernel<16> : lanes == 32 ? moe_route_kernel<32> : moe_route_kernel<64>;
   hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, logits, topk_idx, gates, tokens, experts, k);
   DH_LAUNCH_CHECK();
   return DH_OK;

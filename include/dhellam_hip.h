@@ -317,6 +317,8 @@ int dh_attn_merge(const void *const *outs, const float *const *lses,
  * the k selected logits.  experts <= 64, k <= 8. */
 int dh_moe_route_topk(const float *logits, int32_t *topk_idx, float *gates,
                       int64_t tokens, int experts, int k, void *stream);
+/* Lanes that such a call gives a token (1: a scan of its row); 0: nothing to do. */
+int dh_moe_route_lanes(int64_t tokens, int experts, int k);
 
 size_t dh_moe_sort_workspace_bytes(int64_t n_assign, int experts);
 /* Stable counting sort of the flat assignment list topk_idx [n_assign]

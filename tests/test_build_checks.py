@@ -93,3 +93,12 @@ def test_weight_gradients_go_where_they_were_measured_the_faster(t, n, k, groupe
 def test_tiles_of_a_grouped_weight_gradient(groups, rows, m, n, accumulate, tiles):
     from dhellam_amd import _lib
     assert _lib.load().dh_grouped_gemm_tn_tiles(groups, rows, m, n, accumulate) == tiles
+
+
+@pytest.mark.parametrize("tokens,experts,k,lanes", [
+    (1, 1, 1, 1), (64, 2, 2, 1), (100, 3, 3, 8), (1000, 5, 4, 8), (8192, 8, 2, 8), (65536, 8, 2, 1), (131072, 8, 8, 1), (16384, 16, 4, 16),
+    (65536, 16, 2, 1), (8192, 24, 2, 32), (65536, 24, 2, 1), (16384, 64, 8, 64), (65536, 64, 1, 1), (131072, 64, 8, 64), (262144, 48, 1, 1)])
+def test_lanes_of_the_routing(tokens, experts, k, lanes):
+    """A scan where it was measured the faster: few experts, or tokens enough to fill the chip with a thread each."""
+    from dhellam_amd import _lib
+    assert _lib.load().dh_moe_route_lanes(tokens, experts, k) == lanes

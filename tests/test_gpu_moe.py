@@ -634,7 +634,8 @@ def test_grouped_gemm_tn_accumulates_few_rows(rows, m, n):
             assert torch.equal(got[i].cpu(), c[i])
 
 
-@pytest.mark.parametrize("T,E,k", [(5, 1, 1), (33, 3, 2), (9, 8, 8), (67, 9, 3), (40, 33, 8), (31, 64, 8), (700, 5, 4)])
+@pytest.mark.parametrize("T,E,k", [(5, 1, 1), (33, 3, 2), (9, 8, 8), (67, 9, 3), (40, 33, 8), (31, 64, 8), (700, 5, 4),
+                                   (33, 8, 2), (4500, 4, 3), (3001, 24, 1), (18000, 8, 1)])      # lanes a token, and scans
 def test_route_picks_as_a_scan_does(T, E, k):
     """Ties, infinities, NaN and both zeros: every choice is that of a scan which starts at the lowest id left and moves on to
     what is greater, so a NaN is chosen only where it is the lowest id left."""
