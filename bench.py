@@ -288,7 +288,8 @@ def kernel_rooflines(cfg):
     add(f"head_block_fwd_bwd[{T}x{H} -> {Vp}]", "mfma", 6.0 * T * H * Vp, ms, "6THV flop (logits GEMM fwd, dgrad, wgrad; norm, cross entropy, loss around them)")
     parallel_state.set_tensor_model_parallel(0, 1)
     del table, dh_, em_out, hid
-    # --- the layer's twelve dense products (library kernels through dh_gemm), as the layer calls them -------
+    # --- the layer's twelve dense products, as the layer calls them -----------------------------------------
+    from dhellam_amd import _host
     from dhellam_amd._Clib import keep_transposed
     from dhellam_amd.operators.layernorm_column import dgrad_bwd, gemm_fwd, wgrad_bwd
     for name, n_out, k_in in (("qkv", cfg.qkv_per_rank, H), ("attn_out", H, hq * d), ("fc1", 2 * F, H), ("fc2", H, F)):
@@ -299,8 +300,11 @@ def kernel_rooflines(cfg):
         for what, fn in (("fwd", lambda: gemm_fwd(None, x, w, None, "TN", False, 0, True, None)),
                          ("dgrad", lambda: dgrad_bwd(None, dy, w, None, "NN", False, 0, True, None)),
                          ("wgrad", lambda: wgrad_bwd(None, dy, x, dw, True, "NT", False, 0, True, None))):
+            how = ("hipBLASLt through dh_gemm" + (", against the resident W^T" if what == "dgrad" else "") if what != "wgrad" else
+                   "the grouped kernel, operands as they are" if _host.wgrad_grouped(T, n_out, k_in) else
+                   "hipBLASLt through dh_gemm, with the transpose of one operand")
             add(f"dense_gemm[{name} {what} T={T} N={n_out} K={k_in}]", "mfma", flop, time_gpu(fn, iters=10, warmup=3),
-                "2TNK flop (hipBLASLt through dh_gemm; dgrad against the resident W^T; wgrad includes the transpose of dY where it is used)")
+                f"2TNK flop ({how})")
         del x, w, dy, dw
     return res
 

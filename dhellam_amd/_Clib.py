@@ -145,19 +145,20 @@ def transpose_2d(src: torch.Tensor, out: Optional[torch.Tensor] = None, stream=N
 
 
 # The weight-gradient product dW[N, K] = dY[T, N]^T X[T, K] reads both operands along their strided dimension, the
-# GEMM library's slowest layout here.  Most of these products are the grouped kernel's (``wgrad`` of the host path says which
-# and why); what follows is about the rest, and about fp32 ``main_grad``.  Measured at T = 4096, bf16, accumulating (us; N, K = 7168, 8192 / 8192, 3584 /
-# 1280, 8192 / 8192, 1024):   as given 464 / 233 / 105 / 85;   dY^T row-major 380 / 190 / 87 / 72;   X^T row-major
-# (the layout ``dh_gemm`` refuses, ``dh_gemm_tt``) 383 / 188 / 95 / 70;   both row-major (the forward's layout)
-# 335 / 165 / 76 / 61.  One transposed operand is worth 15-20 % whichever it is, so the SMALLER one is transposed
-# (dh_transpose_2d moves 5.5-6 TB/s: [4096, 8192] in 24 us, [4096, 3584] in 11 us, [4096, 1024] in 8 us): X when the
-# weight has fewer inputs than outputs (fc2, the attention output projection, the vocabulary projection), dY
-# otherwise (qkv, fc1 -- where the kernel that produces dY writes the transpose alongside).  Both transposed would
-# be faster still, but for that layout the library picks a kernel that splits tiles over workgroups, and its
-# accumulation into dW does not always give the same bits when another kernel shares the GPU (1 step in 40-100
-# of the double-strand schedule differed from the serial one in the last bits of one weight gradient; giving each
-# stream its own workspace does not change that), while the two schedules are required to agree bit for bit: not
-# used.
+# GEMM library's slowest layout here.  Large weights and few rows are the grouped kernel's (``wgrad_grouped`` of the host
+# path, with its sweeps), which needs no transposed operand; what follows is about the rest -- of the layer's four the qkv
+# and attention output projections at whole rows -- and about fp32 ``main_grad``, which that kernel does not add to.
+# Library, T = 4096, bf16, accumulating (us; N, K = 7168, 8192 / 8192, 3584 / 1280, 8192 / 8192, 1024):   as given 464 / 233 /
+# 105 / 85;   dY^T row-major 380 / 190 / 87 / 72;   X^T row-major (the layout ``dh_gemm`` refuses, ``dh_gemm_tt``) 383 / 188 / 95 /
+# 70;   both row-major (the forward's layout) 335 / 165 / 76 / 61;   grouped kernel 371 / 185 / 84 / 83.  One transposed
+# operand is worth 15-20 % whichever it is, so the SMALLER one is transposed (dh_transpose_2d moves 5.5-6 TB/s: [4096, 8192] in
+# 24 us, [4096, 3584] in 11 us, [4096, 1024] in 8 us): X when the weight has fewer inputs than outputs (the attention output
+# projection; with fp32 gradients fc2 and the vocabulary projection too), dY otherwise (qkv; with fp32 gradients fc1).  For fc1 and
+# fc2 SwiGLU then writes the transpose alongside.  Both transposed would be faster still, but for that layout the library
+# picks a kernel that splits tiles over workgroups, and its accumulation into dW does not always give the same bits when
+# another kernel shares the GPU (1 step in 40-100 of the double-strand schedule differed from the serial one in the last
+# bits of one weight gradient; giving each stream its own workspace does not change that), while the two schedules are
+# required to agree bit for bit: not used.
 # The library's transposed layouts need a row count of whole 64-deep slices, or enough rows for a ragged last one not to
 # matter: at T = 1000 fc1 takes 160 us as given and 165 + 8 us with dY^T, fc2 83 against 85 + 5, at T = 1024 147 / 130 + 6
 # and 75 / 69 + 5 us; at T = 2000 the two are level (262 / 242 + 11, 131 / 124 + 7).  Narrow weights gain earlier: N = 1280

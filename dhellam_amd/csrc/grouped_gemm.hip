@@ -6,9 +6,9 @@
 //   NT  c[r, n]  = sum_k a[r, k] * w[g][n, k]      forward  (both k-contiguous)
 //   NN  c[r, n]  = sum_k a[r, k] * w[g][k, n]      dgrad    (w strided in k)
 //   TN  c[g][m,n] = sum_r a[r, m] * b[r, n]        wgrad    (both strided in k = r)
-// Two kernels.  grouped_gemm_w8_kernel (products that fill the chip): 256x256 tiles, eight wavefronts in two alternating
-// groups, optionally one workgroup per compute unit that takes whole tiles in rounds and a k piece of a tile
-// of the last round.  grouped_gemm_t_kernel (everything else): smaller tiles, copied straight to LDS, split along k where
+// Two kernels.  grouped_gemm_w8_kernel (products that fill the chip): a workgroup per 256x256 tile, eight wavefronts in two
+// alternating groups; with a workspace further workgroups of the launch may take the last round of tiles in k pieces.
+// grouped_gemm_t_kernel (everything else): smaller tiles, copied straight to LDS, split along k where
 // there are few of them.  k-contiguous operands are read from LDS as 16-byte row fragments; k-strided operands stay
 // row-major in LDS and are read with transpose loads, so no operand is ever transposed in memory.
 // The product is formed as C^T (weights in the MFMA A slot) so that each lane
