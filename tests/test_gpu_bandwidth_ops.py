@@ -209,6 +209,7 @@ def test_wgrad_and_dgrad_by_the_grouped_kernel(dtype, T, N, K):
     from dhellam_amd import _host
     from dhellam_amd.operators.layernorm_column import dgrad_bwd, wgrad_bwd
     assert _host.wgrad_grouped(T, N, K) == ((T, N) != (385, 1280))
+    assert _host.dgrad_grouped(T, N, K) == (N in (10248, 1000))
     dy, x, w = (randn(s, dtype, i, std=0.5).cuda() for i, s in enumerate(((T, N), (T, K), (N, K))))
     ref = (dy.double().t() @ x.double()).cpu()
     d, _ = wgrad_bwd(None, dy, x, None, False, "NT", False, 0, True, None)
@@ -568,6 +569,10 @@ def test_reused_swiglu_gradient_buffer_drops_the_transposed_twin():
 def test_norm_backward_of_narrow_rows(dtype, rows, cols, ln):
     """One launch and two, on both sides of the line between them: one, two and four vectors a thread, a row by 64 and by 256
     threads, columns that end inside a slab of 32, more row groups than rows and fewer."""
+    from dhellam_amd import _lib
+    two = [(769, 512), (768, 264), (1025, 1024), (1281, 2048)] + ([] if dtype == torch.float32 else [(33, 8), (433, 264)])
+    code = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}[dtype]
+    assert _lib.load().dh_norm_bwd_one_launch(rows, cols, code) == ((rows, cols) not in two)
     test_norm_fwd_bwd(dtype, rows, cols, ln)
 
 

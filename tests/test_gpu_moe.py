@@ -619,8 +619,11 @@ def test_grouped_gemm_one_stage_tiles(form, rows, n, k):
 @pytest.mark.parametrize("rows,m,n", [([0, 1, 63, 64, 65, 7, 16, 130], 1304, 1096), ([3] * 8, 1304, 1096),
                                       ([0, 1, 63, 64, 65, 7, 16, 130], 24, 5128), ([3] * 8, 5128, 80)])     # narrow: 128x128 tiles
 def test_grouped_gemm_tn_accumulates_few_rows(rows, m, n):
-    """Accumulating weight gradients of few rows on the 256x256 tiles: c += a^T b with one rounding; an empty group leaves its c."""
+    """Accumulating weight gradients of few rows on the 256x256 tiles, narrow ones on the smaller: c += a^T b with one rounding; an
+    empty group leaves its c."""
+    from dhellam_amd import _lib
     from dhellam_amd.operators import moe
+    assert _lib.load().dh_grouped_gemm_tn_tiles(len(rows), sum(rows), m, n, 1) == (256 if min(m, n) > 100 else 128)
     g = torch.Generator().manual_seed(8)
     offs = torch.tensor([0] + rows).cumsum(0).to(torch.int32)
     a, b, c = (torch.randn(*s, generator=g).bfloat16() for s in ((sum(rows), m), (sum(rows), n), (len(rows), m, n)))
