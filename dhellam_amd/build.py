@@ -22,6 +22,7 @@ CSRC = PKG / "csrc"
 LIB_DIR = PKG / "lib"
 LIB_PATH = LIB_DIR / "libdhellam_hip.so"
 OBJ_DIR = ROOT / "build" / "obj"
+GEN_DIR = ROOT / "build" / "gen"          # sources that are written by programs: attn_loops.inc
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
@@ -39,11 +40,18 @@ CXXFLAGS = [
     "-Wno-unknown-pragmas",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     f"-I{ROOT / 'include'}",
+    f"-I{GEN_DIR}",
 ]
 
 
 def sources() -> list[Path]:
     return sorted(CSRC.glob("*.hip"))
+
+
+def generate_sources() -> None:
+    """Writes ``attn_loops.inc``: the main loops of the attention kernels with one wavefront on a SIMD (``csrc/attn_loops.py``)."""
+    GEN_DIR.mkdir(parents=True, exist_ok=True)
+    subprocess.run([sys.executable, str(CSRC / "attn_loops.py"), str(GEN_DIR / "attn_loops.inc")], check=True)
 
 
 def _compile(src: Path, verbose: bool) -> Path:
@@ -65,6 +73,7 @@ def build(verbose: bool = False, jobs: int | None = None) -> Path:
     """Compile every ``csrc/*.hip`` for gfx950 and link the shared library."""
     OBJ_DIR.mkdir(parents=True, exist_ok=True)
     LIB_DIR.mkdir(parents=True, exist_ok=True)
+    generate_sources()
     srcs = sources()
     if not srcs:
         raise RuntimeError(f"no HIP sources under {CSRC}")

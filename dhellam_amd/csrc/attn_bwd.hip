@@ -5,7 +5,7 @@
 //   delta   : delta_i = sum_d dO[i,d] * O[i,d]                      (streaming; for fp32 and where dS is kept: the
 //             recomputing dQ kernels form delta in their prologue and run first)
 //   dK/dV   : a workgroup owns 64 key/value rows (K, V fragments stay in
-//             registers, for head dim 128 in LDS), walks the
+//             registers, for head dim 128 K in LDS), walks the
 //             query heads of its GQA group and the query tiles that attend to
 //             it; S = Q K^T and dP = dO V^T are computed
 //             with the key index on lanes so that P and dS feed dV^T += dO^T P
@@ -33,7 +33,7 @@ struct AttnBwdParams {
   int64_t o_stride;
   const float *lse;
   float *delta;              // fp32 [batch][hq][max_sq]: rowsum(dO * O); written by the delta kernel or by the dQ kernel
-  float *ld2;                // fp32 [2][plane]: lse * log2(e), then delta, each [batch][hq][ld2_pitch]
+  float *ld2;                // fp32 [2][plane]: lse * log2(e), then -delta, each [batch][hq][ld2_pitch]
   int64_t ld2_plane;         // elements between the two planes
   int ld2_pitch;             // max_sq rounded up to 32: every 32-row query tile of a head is one aligned 128-byte run
   void *dq, *dk, *dv;
@@ -105,7 +105,7 @@ attn_delta_kernel(const T *__restrict__ dout, const T *__restrict__ out, float *
       if (ld2) {             // the copy the dK/dV kernels stream: lse in exp2 units next to delta
         const int64_t a2 = ((int64_t)b * hq + h) * ld2_pitch + i;
         ld2[a2] = lse[((int64_t)b * hq + h) * lse_pitch + i] * 1.4426950408889634f;
-        ld2[ld2_plane + a2] = s;
+        ld2[ld2_plane + a2] = -s;
       }
     }
   }
@@ -144,6 +144,12 @@ attn_bwd_gqa_sum_kernel(const float *__restrict__ dk_part, const float *__restri
 // (no staging registers, no bank conflicts), two pipeline stages held in separate LDS
 // objects, causal work made uniform by pairing tile i with tile n-1-i.
 // ---------------------------------------------------------------------------------------------
+
+}  // namespace dh
+
+#include "attn_bwd_dkv128.h"
+
+namespace dh {
 
 // dQ: 8 wavefronts = RG query row groups x SPLIT key splits (as the forward kernel); the
 // partial dQ of the splits are added through LDS in split order.  As in the forward kernel
@@ -267,7 +273,7 @@ __global__ void __launch_bounds__(512) attn_bwd_dq_d128_kernel(const AttnBwdPara
         if (row_q < p.ld2_pitch) {
           const int64_t a2 = ((int64_t)b * p.hq + h) * p.ld2_pitch + row_q;
           p.ld2[a2] = row_ok ? lse_c : 0.f;
-          p.ld2[p.ld2_plane + a2] = del_c;
+          p.ld2[p.ld2_plane + a2] = -del_c;
         }
       }
     }
@@ -692,380 +698,12 @@ static int launch_dq_d128(const AttnBwdParams &p, int batch, hipStream_t st) {
   return DH_OK;
 }
 
-// dK/dV with eight wavefronts: 2 key row groups (32 rows each) x 4 query splits, i.e. two wavefronts per
-// SIMD whose matrix and softmax phases interleave.  To fit that into 256 registers per wavefront the K / V
-// tiles of the workgroup live in LDS (read as row fragments every iteration) instead of registers, the
-// accumulators are ordinary variables, and lse / delta of a query tile come straight from memory (one
-// aligned 128-byte run per tile and plane), loaded one iteration ahead.  LDS: two stages of four Q + dO tile
-// pairs (128 KB) + the K and V tiles (32 KB).  The splits' partial dK/dV are added through LDS in a fixed
-// order.  Causal: the workgroup owns key tiles j and n-1-j, so every workgroup does the same amount of
-// work.  The main loop is one rolled body; the Q / dO tiles of the next iteration come in with assembly
-// copies (scalar bases) issued between the matrix instructions.
-template <typename T, bool STORE_DS>
-__global__ void __launch_bounds__(512) attn_bwd_dkv_d128_kernel(const AttnBwdParams p) {
-  using M = Mma<T>;
-  using Frag = typename M::Frag;
-  constexpr int D = 128, KG = 2, QSPLIT = 4, BN = 32 * KG, BM = 32;
-  constexpr int QT = BM * D;                          // elements of one Q (or dO) tile
-  constexpr int QTB = QT * (int)sizeof(T);
-  constexpr int SLOT = 2 * QT;                        // Q tile, dO tile
-  constexpr int SLOTB = SLOT * (int)sizeof(T);
-  constexpr int STAGE = QSPLIT * SLOT;
-  constexpr int STAGEB = STAGE * (int)sizeof(T);
-  constexpr int KVT = BN * D;                         // elements of the K (or V) tile
-  constexpr int KVTB = KVT * (int)sizeof(T);
-  __shared__ __attribute__((aligned(1024))) T sAll[2 * STAGE + 2 * KVT];
-
-  const int b = seq_by_length(p.cu_q, gridDim.y, blockIdx.y);
-  const int G = p.hk * p.hsplit;
-  int hg, px;
-  xcd_group_item(blockIdx.x, G, gridDim.x / G, hg, px);
-  const int hkv = hg / p.hsplit, hs = hg % p.hsplit;
-  const int q0 = p.cu_q[b] >> p.q_shift, sq = (p.cu_q[b + 1] >> p.q_shift) - q0;
-  const int k0 = p.cu_k[b] >> p.k_shift, sk = (p.cu_k[b + 1] >> p.k_shift) - k0;
-  const int nkt = (sk + BN - 1) / BN;
-  const int causal = p.causal;
-  const int q_stride = (int)p.q_stride, do_stride = (int)p.do_stride;
-  const float scale_log2 = p.scale_log2;
-  int kt[2], nk;
-  if (causal) {
-    const int pair = px;
-    if (2 * pair >= nkt) return;
-    kt[0] = pair; kt[1] = nkt - 1 - pair;             // heavy (early keys) first
-    nk = (kt[0] == kt[1]) ? 1 : 2;
-  } else {
-    if (px >= nkt) return;
-    kt[0] = px; kt[1] = 0; nk = 1;
-  }
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform: copy bookkeeping stays scalar
-  const int c = lane & 31, hh = lane >> 5;
-  const int kg = w % KG, qs = w / KG;
-  const int ratio = p.hq / p.hk;
-  const int hper = ratio / p.hsplit;
-  const int h_first = hkv * ratio + hs * hper;
-  const uint32_t lds0 = (uint32_t)(uintptr_t)sAll;
-  const uint32_t ldsKV = lds0 + 2u * STAGEB;
-
-  // ---- copies: wavefront w brings one whole tile per iteration: Q (w even) or dO (w odd) of split w / 2 ----
-  CopyLane cl0;
-  cl0.l16 = lane & 15;
-  cl0.lrow = lane >> 4;
-  const int cp_slot = w >> 1, cp_do = w & 1;
-  const int cp_stride = cp_do ? do_stride : q_stride;
-  const T *cp_gt = reinterpret_cast<const T *>(cp_do ? p.dout : p.q) + (int64_t)q0 * cp_stride;
-  const char *cp_g = reinterpret_cast<const char *>(cp_gt);
-  const int cp_dst0 = cp_slot * SLOT + cp_do * QT;    // elements inside a stage
-  const uint32_t cp_step = (uint32_t)(4 * cp_stride) * (uint32_t)sizeof(T);
-  uint32_t cp_off[4];                                 // tiles use swz(row): chunk ^= 4 * (row % 4) + (row / 4) % 4
-  {
-    const uint32_t rowb = (uint32_t)(cl0.lrow * cp_stride) * (uint32_t)sizeof(T);
-    const uint32_t chunk = (uint32_t)(cl0.l16 ^ (4 * cl0.lrow)) << 4;
-#pragma unroll
-    for (int x = 0; x < 4; ++x) cp_off[x] = rowb + (chunk ^ (uint32_t)(x << 4));
-  }
-  typedef __attribute__((address_space(3))) const Frag *lds_frag;
-  typedef short4v __attribute__((address_space(3))) *lds_tr;
-
-  for (int ki = 0; ki < nk; ++ki) {
-    const int j0 = kt[ki] * BN;
-    const int jw0 = j0 + 32 * kg;
-    const int jrow = jw0 + c;
-    // this workgroup's K and V tiles -> LDS: wavefronts 0, 1 bring the two halves of K, wavefronts 2, 3 of V
-    if (w < 4) {
-      const int half = w & 1, isv = w >> 1;
-      const T *gsrc = reinterpret_cast<const T *>(isv ? p.v : p.k) + (int64_t)k0 * (isv ? p.v_stride : p.k_stride) +
-                      (int64_t)hkv * D;
-      dma_tile32_general<T, 8>(sAll + 2 * STAGE + isv * KVT + half * 32 * D, gsrc, (int)(isv ? p.v_stride : p.k_stride), 1,
-                               j0 + 32 * half, 0, sk, cl0);
-    }
-    floatx16 dKt[D / 32], dVt[D / 32];
-#pragma unroll
-    for (int t = 0; t < D / 32; ++t)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        dKt[t][v] = 0.f;
-        dVt[t][v] = 0.f;
-      }
-    const int i_begin = causal ? (j0 / BM) * BM : 0;
-    const int ntq = i_begin < sq ? (sq - i_begin + BM - 1) / BM : 0;
-    const int it_per_head = (ntq + QSPLIT - 1) / QSPLIT;
-    const int niter = it_per_head * hper;
-
-    auto issue_general = [&](int st, int g, int ti) {
-      const int h = h_first + g;
-      const int tq = ti * QSPLIT + cp_slot;
-      if (tq < ntq)
-        dma_tile32_general<T, 8>(sAll + st + cp_dst0, cp_gt + (int64_t)h * D, cp_stride, 1, i_begin + tq * BM, 0, sq, cl0);
-    };
-    // lse (exp2 units) and delta of the rows 8*vb + 4*hh + e of this wavefront's query tile in iteration (g, ti)
-    floatx4 l4[4], d4[4];
-    auto load_ld = [&](int g, int ti) {
-      const int tq = ti * QSPLIT + qs;
-      if (tq < ntq) {
-        int lx = lane;
-        asm volatile("" : "+v"(lx));       // the address is formed here, not kept across the loop
-        const float *src = p.ld2 + ((int64_t)b * p.hq + (h_first + g)) * p.ld2_pitch + (i_begin + tq * BM) + 4 * (lx >> 5);
-#pragma unroll
-        for (int vb = 0; vb < 4; ++vb) {
-          l4[vb] = *reinterpret_cast<const floatx4 *>(src + 8 * vb);
-          d4[vb] = *reinterpret_cast<const floatx4 *>(src + p.ld2_plane + 8 * vb);
-        }
-      }
-    };
-#pragma unroll
-    for (int vb = 0; vb < 4; ++vb)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        l4[vb][e] = 0.f;
-        d4[vb][e] = 0.f;
-      }
-
-    if (niter > 0) {
-      issue_general(0, 0, 0);
-      load_ld(0, 0);
-    }
-    dma_wait_all();
-    __syncthreads();
-
-    const char *cp_src = nullptr;
-    uint32_t cp_dst = 0;
-    bool fcopy = false;
-#define DH_DKV_COPY(i)                                                                                  \
-    do {                                                                                                \
-      if (fcopy) {                                                                                      \
-        __builtin_amdgcn_sched_barrier(0);                                                              \
-        dma_block_fast(cp_src, cp_off[(i) & 3], cp_dst);                                                \
-        cp_src += cp_step;                                                                              \
-        cp_dst += 1024;                                                                                 \
-        __builtin_amdgcn_sched_barrier(0);                                                              \
-      }                                                                                                 \
-    } while (0)
-
-    int g = 0, ti = 0;                                // head and step of iteration it
-#pragma unroll 1
-    for (int it = 0; it < niter; ++it) {
-      int gn = g, tn = ti + 1;                        // ... and of iteration it + 1
-      if (tn == it_per_head) { tn = 0; ++gn; }
-      const bool have_next = it + 1 < niter;
-      const uint32_t cur = lds0 + (uint32_t)((it & 1) * STAGEB);
-      const int nxt_el = ((it + 1) & 1) * STAGE;
-      {
-        const int hn = h_first + gn;
-        const int tq = tn * QSPLIT + cp_slot;
-        const int row0 = i_begin + tq * BM;
-        const bool copy = have_next && tq < ntq;
-        fcopy = copy && row0 + BM <= sq;
-        cp_src = cp_g + ((int64_t)row0 * cp_stride + (int64_t)hn * D) * (int)sizeof(T);
-        cp_dst = lds0 + (uint32_t)((nxt_el + cp_dst0) * (int)sizeof(T));
-        if (copy && !fcopy)
-          dma_tile32_general<T, 8>(sAll + nxt_el + cp_dst0, cp_gt + (int64_t)hn * D, cp_stride, 1, row0, 0, sq, cl0);
-      }
-      const int tq = ti * QSPLIT + qs;
-      const int i0 = i_begin + tq * BM;
-      const bool act = tq < ntq && !(causal && i0 + BM - 1 < jw0);
-      if (act) {
-        // Fragment reads: lane byte offsets inside a slot; the other fragments are reached by XOR / immediate
-        // offsets.  They are recomputed from the lane id here (a dozen instructions) rather than kept in
-        // registers across the loop, which has none to spare.
-        int ln = lane;
-        asm volatile("" : "+v"(ln));
-        const int lc = ln & 31, lh = ln >> 5, r = ln & 15;
-        const uint32_t rowsw = (uint32_t)(lc * 256 + ((lh ^ swz(lc)) << 4));            // row lc, chunk lh
-        const int ta_x = 4 * (r >> 2) + lh;                 // transpose reads: swz of rows 4*lh + r/4 (+8)
-        const int t_lc = 2 * ((ln >> 4) & 1) + ((r & 3) >> 1);
-        const uint32_t t_row = (uint32_t)((4 * lh + (r >> 2)) * 256 + ((r & 3) & 1) * 8);
-        const uint32_t slot = cur + (uint32_t)(qs * SLOTB);
-        uint32_t qb = slot + rowsw, kb = ldsKV + (uint32_t)(kg * 32 * 256) + rowsw;
-        uint32_t ta = slot + t_row + (uint32_t)((t_lc ^ ta_x) << 4);
-        uint32_t tb = slot + t_row + 8 * 256 + (uint32_t)((t_lc ^ (ta_x + 2)) << 4);
-        asm volatile("" : "+v"(qb), "+v"(ta), "+v"(tb), "+v"(kb));   // derive the other addresses here
-        floatx16 S, dP;
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          S[v] = 0.f;
-          dP[v] = 0.f;
-        }
-        // S = Q K^T and dP = dO V^T with the key index on lanes; the four fragments of step ks + 1 are
-        // requested before the matrix instructions of step ks (the scheduling barriers pin that order)
-        {
-          Frag fq[2], fk[2], fo[2], fv[2];
-          fq[0] = *(lds_frag)(qb);
-          fk[0] = *(lds_frag)(kb);
-          fo[0] = *(lds_frag)(qb + QTB);
-          fv[0] = *(lds_frag)(kb + KVTB);
-#pragma unroll
-          for (int ks = 0; ks < D / 16; ++ks) {
-            const int cb = ks & 1, nb = cb ^ 1;
-            if (ks + 1 < D / 16) {
-              const uint32_t aq = qb ^ (uint32_t)((ks + 1) << 5), ak = kb ^ (uint32_t)((ks + 1) << 5);
-              fq[nb] = *(lds_frag)(aq);
-              fk[nb] = *(lds_frag)(ak);
-              fo[nb] = *(lds_frag)(aq + QTB);
-              fv[nb] = *(lds_frag)(ak + KVTB);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            S = M::mma(fq[cb], fk[cb], S);
-            dP = M::mma(fo[cb], fv[cb], dP);
-            __builtin_amdgcn_sched_barrier(0);
-            DH_DKV_COPY(ks);                          // one copy block per step: all eight are out before the softmax
-          }
-        }
-        if ((causal && i0 < jw0 + 31) || (i0 + BM > sq) || (STORE_DS && jw0 + 32 > sk)) {
-          // masked scores become -inf, i.e. P = dS = 0 (lse and delta of rows past the sequence end are zeros);
-          // keys past the end matter only when dS is kept: the dQ product would meet them
-#pragma unroll
-          for (int v = 0; v < 16; ++v) {
-            const int i = i0 + acc_row(v, hh);
-            if (i >= sq || (causal && jrow > i) || (STORE_DS && jrow >= sk)) S[v] = -INFINITY;
-          }
-        }
-        Frag Pb[2], dSb[2];
-#pragma unroll
-        for (int s = 0; s < 2; ++s) {
-          float pv[8], dsv[8];
-#pragma unroll
-          for (int u = 0; u < 2; ++u) {
-            const int vb = 2 * s + u;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const int v = 4 * vb + e;
-              const float pe = fast_exp2(S[v] * scale_log2 - l4[vb][e]);
-              pv[4 * u + e] = pe;
-              dsv[4 * u + e] = pe * (dP[v] - d4[vb][e]);
-            }
-          }
-          Pb[s] = frag_pack<T>(pv);
-          dSb[s] = frag_pack<T>(dsv);
-        }
-        if (STORE_DS) {
-          // the packed dS fragments go out as they are, 1 KB per fragment and wavefront
-          const int64_t blk = (((int64_t)b * p.hq + (h_first + g)) * p.ds_nqt + (i0 >> 5)) * p.ds_nkb + (jw0 >> 5);
-          int lx = lane;
-          asm volatile("" : "+v"(lx));
-          Frag *dst = reinterpret_cast<Frag *>(reinterpret_cast<char *>(p.ds) + blk * 2048) + lx;
-          dst[0] = dSb[0];
-          dst[64] = dSb[1];
-        }
-        if (have_next) load_ld(gn, tn);               // next tile's lse / delta, in flight across the barrier
-        // dV^T += dO^T P and dK^T += Q^T dS; the eight copy blocks of this wavefront go out in between.
-        // Step u = (s, which, t): which = 0 reads dO^T (for dV), 1 reads Q^T (for dK); the fragments of
-        // step u + 1 are requested before the matrix instruction of step u.
-        {
-          constexpr int AH = 2;                      // steps requested ahead
-          short4v x0[AH + 1], x1[AH + 1];
-          auto rd = [&](int u) {
-            const int sx = u >> 3, which = (u >> 2) & 1, t = u & 3;
-            const uint32_t a0 = (ta ^ (uint32_t)(t << 6)) + (uint32_t)(sx * 16 * 256) + (which ? 0u : (uint32_t)QTB);
-            const uint32_t a1 = (tb ^ (uint32_t)(t << 6)) + (uint32_t)(sx * 16 * 256) + (which ? 0u : (uint32_t)QTB);
-            x0[u % (AH + 1)] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr)(a0));
-            x1[u % (AH + 1)] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr)(a1));
-          };
-#pragma unroll
-          for (int u = 0; u < AH; ++u) rd(u);
-#pragma unroll
-          for (int u = 0; u < 16; ++u) {
-            const int sx = u >> 3, which = (u >> 2) & 1, t = u & 3, cb = u % (AH + 1);
-            if (u + AH < 16) rd(u + AH);
-            __builtin_amdgcn_sched_barrier(0);
-            if (which == 0) dVt[t] = M::mma(frag_join<T>(x0[cb], x1[cb]), Pb[sx], dVt[t]);
-            else dKt[t] = M::mma(frag_join<T>(x0[cb], x1[cb]), dSb[sx], dKt[t]);
-            __builtin_amdgcn_sched_barrier(0);
-          }
-        }
-      } else {
-        if (have_next) load_ld(gn, tn);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) DH_DKV_COPY(i);
-      }
-      g = gn;
-      ti = tn;
-      dma_wait_all();
-      __syncthreads();   // the next stage has landed, and everyone is done with the current one
-    }
-#undef DH_DKV_COPY
-
-    // add the splits' partial sums through LDS in a fixed order: (0 += 2, 1 += 3), then 0 += 1.
-    // Slot (split, key group) holds dK then dV, 16 KB each, in the stage area.
-    static_assert(2 * STAGE * sizeof(T) >= (size_t)2 * KG * 2 * 4096 * sizeof(float), "exchange area");
-    typedef __attribute__((address_space(3))) float *lds_f;
-#pragma unroll
-    for (int round = 0; round < 2; ++round) {
-      const int senders_from = round == 0 ? 2 : 1, senders_to = round == 0 ? 4 : 2;
-      if (qs >= senders_from && qs < senders_to) {
-        int lx = lane;
-        asm volatile("" : "+v"(lx));       // one base register + immediate offsets, computed here
-        const uint32_t xb = lds0 + (uint32_t)((((qs - senders_from) * KG + kg) * 2 * 4096 + lx) * 4);
-        lds_f dst = (lds_f)(xb);
-#pragma unroll
-        for (int t = 0; t < D / 32; ++t)
-#pragma unroll
-          for (int v = 0; v < 16; ++v) {
-            dst[(t * 16 + v) * 64] = dKt[t][v];
-            dst[4096 + (t * 16 + v) * 64] = dVt[t][v];
-          }
-      }
-      __syncthreads();
-      if (qs < senders_from) {
-        int lx = lane;
-        asm volatile("" : "+v"(lx));
-        const uint32_t xb = lds0 + (uint32_t)(((qs * KG + kg) * 2 * 4096 + lx) * 4);
-        lds_f src = (lds_f)(xb);
-#pragma unroll
-        for (int t = 0; t < D / 32; ++t)
-#pragma unroll
-          for (int v = 0; v < 16; ++v) {
-            dKt[t][v] += src[(t * 16 + v) * 64];
-            dVt[t][v] += src[4096 + (t * 16 + v) * 64];
-          }
-      }
-      __syncthreads();
-    }
-    // the store addresses are derived from the lane id here, so that nothing but the id lives through the loop
-    int ln = lane;
-    asm volatile("" : "+v"(ln));
-    if (qs == 0 && jw0 + (ln & 31) < sk) {
-      const int hh = ln >> 5, jrow = jw0 + (ln & 31);
-      if (p.hsplit == 1) {
-        T *dkp = reinterpret_cast<T *>(p.dk) + (int64_t)(k0 + jrow) * p.dk_stride + (int64_t)hkv * D;
-        T *dvp = reinterpret_cast<T *>(p.dv) + (int64_t)(k0 + jrow) * p.dv_stride + (int64_t)hkv * D;
-#pragma unroll
-        for (int t = 0; t < D / 32; ++t)
-#pragma unroll
-          for (int vb = 0; vb < 4; ++vb) {
-            struct alignas(8) { T v[4]; } a, bq;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              a.v[e] = static_cast<T>(dKt[t][4 * vb + e] * p.scale);
-              bq.v[e] = static_cast<T>(dVt[t][4 * vb + e]);
-            }
-            *reinterpret_cast<decltype(a) *>(dkp + 32 * t + 8 * vb + 4 * hh) = a;
-            *reinterpret_cast<decltype(bq) *>(dvp + 32 * t + 8 * vb + 4 * hh) = bq;
-          }
-      } else {
-        const int64_t off = (((int64_t)hs * p.total_k + (k0 + jrow)) * p.hk + hkv) * D;
-#pragma unroll
-        for (int t = 0; t < D / 32; ++t)
-#pragma unroll
-          for (int vb = 0; vb < 4; ++vb) {
-            *reinterpret_cast<float4 *>(p.dk_part + off + 32 * t + 8 * vb + 4 * hh) =
-                make_float4(dKt[t][4 * vb] * p.scale, dKt[t][4 * vb + 1] * p.scale, dKt[t][4 * vb + 2] * p.scale,
-                            dKt[t][4 * vb + 3] * p.scale);
-            *reinterpret_cast<float4 *>(p.dv_part + off + 32 * t + 8 * vb + 4 * hh) =
-                make_float4(dVt[t][4 * vb], dVt[t][4 * vb + 1], dVt[t][4 * vb + 2], dVt[t][4 * vb + 3]);
-          }
-      }
-    }
-    __syncthreads();   // the K / V tiles and the exchange area are rewritten by the next key tile
-  }
-}
-
 template <typename T>
 static int launch_dkv_d128(const AttnBwdParams &p, int batch, int max_sk, hipStream_t st) {
   const int nkt = (int)cdiv(max_sk, 64);
   dim3 grid((unsigned)((p.causal ? (nkt + 1) / 2 : nkt) * p.hk * p.hsplit), (unsigned)batch);
-  if (p.ds) hipLaunchKernelGGL((attn_bwd_dkv_d128_kernel<T, true>), grid, dim3(512), 0, st, p);
-  else hipLaunchKernelGGL((attn_bwd_dkv_d128_kernel<T, false>), grid, dim3(512), 0, st, p);
+  if (p.ds) hipLaunchKernelGGL((attn_bwd_dkv128_kernel<T, true>), grid, dim3(256), 0, st, p);
+  else hipLaunchKernelGGL((attn_bwd_dkv128_kernel<T, false>), grid, dim3(256), 0, st, p);
   return DH_OK;
 }
 
@@ -1114,6 +752,7 @@ int attn_bwd_f32(const void *dout, const void *q, const void *k, const void *v, 
                  int dq_accumulate, hipStream_t st);
 
 constexpr int DKV_ROWS = 64;  // key rows of a dK/dV workgroup
+constexpr int64_t DKV_MAX_STRIDE = 1ll << 26;   // elements: 32 rows of them are less than 4 GiB
 
 // Keeping dS for the dQ product costs 2 bytes per (head, query, key) of workspace, written once and read once.
 // It pays where the recomputing dQ kernel runs its small-grid form (fewer than 256 workgroups of 128 query rows:
@@ -1213,10 +852,11 @@ struct AttnBwdRoute {
   bool both;         // dK/dV and dQ in one launch of the tile kernels, behind the delta kernel
   int hsplit;        // workgroups that share a GQA group in dK/dV
 };
+// `wide`: token strides that the 32-bit copy offsets of the dK/dV kernel do not reach across a tile.
 static AttnBwdRoute attn_bwd_route(int batch, int max_sq, int max_sk, int64_t total_q, int64_t total_k, int hq, int hk, int d,
-                                   int causal, bool room_for_ds) {
+                                   int causal, bool room_for_ds, bool wide = false) {
   const BwdBoth both = bwd_both(batch, max_sq, max_sk, total_q, total_k, hq, hk, d, causal);
-  const bool short_rows = d == 128 && (both.pays || bwd_short(max_sq, max_sk, causal, total_q, hq)), big = dq_big_grid(batch, max_sq, hq, causal);
+  const bool short_rows = d == 128 && (both.pays || wide || bwd_short(max_sq, max_sk, causal, total_q, hq)), big = dq_big_grid(batch, max_sq, hq, causal);
   AttnBwdRoute r;
   r.keep_ds = room_for_ds && max_sk > 0 && !short_rows;
   r.hand_dkv = d == 128 && !short_rows;
@@ -1369,7 +1009,8 @@ static int attn_bwd_entry(const void *dout, const void *q, const void *k, const 
   // process-wide limit); they take the tail of the workspace
   size_t dsb = ds_bytes(batch, max_seqlen_q, total_k, hq, d, dtype, causal);
   if (dsb > 0 && base_bytes + align256(dsb) > workspace_bytes) dsb = 0;
-  const AttnBwdRoute route = attn_bwd_route(batch, max_seqlen_q, max_seqlen_k, total_q, total_k, hq, hk, d, causal, dsb > 0);
+  const AttnBwdRoute route = attn_bwd_route(batch, max_seqlen_q, max_seqlen_k, total_q, total_k, hq, hk, d, causal, dsb > 0,
+                                            q_stride > DKV_MAX_STRIDE || k_stride > DKV_MAX_STRIDE || do_stride > DKV_MAX_STRIDE);
   uint8_t *ds_ws = (uint8_t *)(((uintptr_t)workspace + 255) & ~(uintptr_t)255) + (base_bytes - 256);
   const bool delta_in_dq = dtype != DH_F32 && !route.keep_ds;
   if (max_seqlen_q > 0 && !delta_in_dq) {

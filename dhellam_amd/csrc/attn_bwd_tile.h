@@ -98,7 +98,7 @@ __device__ __forceinline__ void dq_tile_body(const AttnBwdParams &p, int bx, int
       if (row_q < p.ld2_pitch) {          // both, side by side, in whole 32-row tiles (padding rows: zeros)
         const int64_t a2 = ((int64_t)b * p.hq + h) * p.ld2_pitch + row_q;
         p.ld2[a2] = row_ok ? lse_c : 0.f;
-        p.ld2[p.ld2_plane + a2] = del_c;
+        p.ld2[p.ld2_plane + a2] = -del_c;
       }
     }
   }
@@ -324,7 +324,7 @@ __device__ __forceinline__ void dkv_tile_body(const AttnBwdParams &p, int bx, in
         for (int j = 0; j < 8; ++j) {
           const int v = 8 * s + j;
           pv[j] = fast_exp2(S[v] * scale_log2 - l4[v >> 2][v & 3]);
-          dsv[j] = pv[j] * (dP[v] - d4[v >> 2][v & 3]);
+          dsv[j] = pv[j] * (dP[v] + d4[v >> 2][v & 3]);      // (the plane holds -delta)
         }
         Pb[s] = frag_pack<T>(pv);
         dSb[s] = frag_pack<T>(dsv);
@@ -437,7 +437,7 @@ template <typename T, int D> __global__ void __launch_bounds__(256) attn_bwd_del
     s += __shfl_xor(s, 1, 64);                   // both lanes of a row are at the same item
     const int64_t head = (int64_t)b * p.hq + h;
     if (hh == 0 && i < rows) p.delta[head * p.max_sq + i] = s;
-    if (i < padded) p.ld2[(hh ? p.ld2_plane : 0) + head * p.ld2_pitch + i] = hh ? s : i < sq ? p.lse[head * p.lse_pitch + i] * 1.4426950408889634f : 0.f;
+    if (i < padded) p.ld2[(hh ? p.ld2_plane : 0) + head * p.ld2_pitch + i] = hh ? -s : i < sq ? p.lse[head * p.lse_pitch + i] * 1.4426950408889634f : 0.f;
   }
 }
 

@@ -1,0 +1,425 @@
+"""Writes the main loops of the one-wavefront-per-SIMD attention kernels as assembly (``attn_loops.inc``).
+
+The kernels around them (``attn_bwd_dkv128.h``) are HIP; only the loop is laid down instruction by instruction, because with
+one wavefront on a SIMD the order of its instructions IS the schedule: a ``16x16x32`` MFMA occupies the matrix pipe for 16 cycles,
+a wavefront issues one instruction in about 5, so two or three others fit beneath each MFMA for free and anything that stands
+in the wrong place is paid in full.  (Written as single asm statements the compiler puts an ``s_nop`` between any two of which one
+reads what the other wrote, 74 in a tile of 128 MFMAs: 10 % of the loop.)
+
+``Stream`` keeps the account that hand-written assembly gets wrong: it counts LDS reads in flight (they complete in order) and
+places the waits, and it refuses
+  * an MFMA or vector instruction that reads a register whose LDS read nothing has waited for,
+  * a vector instruction on the result of an MFMA with fewer than two MFMAs between them,
+  * an MFMA on a register that a vector instruction wrote fewer than two instructions ago,
+  * the result of a transcendental in the very next instruction,
+  * an LDS read into a register that an earlier read has not filled yet,
+  * an MFMA on a fragment that a later read has replaced.
+"""
+import re
+import sys
+
+
+def regs(text, kind="v"):
+    """The registers of one kind that an operand list names by number, as a set."""
+    out = set()
+    for lo, hi in re.findall(r"(?<![\w\]])%s\[(\d+):(\d+)\]" % kind, text):
+        out |= set(range(int(lo), int(hi) + 1))
+    out |= {int(n) for n in re.findall(r"(?<![\w\[%%])%s(\d+)\b" % kind, text)}
+    return out
+
+
+def v(n, count=1):
+    return "v%d" % n if count == 1 else "v[%d:%d]" % (n, n + count - 1)
+
+
+def s(n, count=1):
+    return "s%d" % n if count == 1 else "s[%d:%d]" % (n, n + count - 1)
+
+
+class Stream:
+    """A straight piece of code with its account of what is in flight."""
+
+    def __init__(self, dtype):
+        self.mfma_name = "v_mfma_f32_16x16x32_" + {"bf16": "bf16", "f16": "f16"}[dtype]
+        self.pack_name = "v_cvt_pk_%s_f32" % dtype
+        self.lines = []
+        self.reads = []                # LDS reads that may be in flight, oldest first: sets of registers
+        self.mfma_at, self.mfmas = {}, 0
+        self.valu_at, self.count = {}, 0
+        self.holds = {}                # what the last LDS read into a register brought
+        self.trans = set()
+
+    def put(self, text):
+        self.lines.append(text)
+        self.count += 1
+        self.trans = set()
+
+    def fresh(self, used):
+        for r in self.reads:
+            assert not (r & used), ("read in flight", used, self.lines[-3:])
+
+    # -- LDS --
+    def lds(self, text, dst, width, what=None):
+        d = set(range(dst, dst + width))
+        self.holds.update((r, what) for r in d)
+        for r in self.reads:
+            assert not (r & d), ("two reads in flight into", d)
+        self.reads.append(d)
+        self.put(text)
+
+    def wait(self, used):
+        """Waits for the reads into `used`, if they may be in flight."""
+        last = max((i for i, r in enumerate(self.reads) if r & used), default=-1)
+        if last >= 0:
+            left = len(self.reads) - 1 - last
+            self.reads = self.reads[last + 1:]
+            self.put("s_waitcnt lgkmcnt(%d)" % min(left, 15))
+
+    # -- matrix and vector --
+    def mfma(self, d, x, y, c, holds=()):
+        used = regs(x, "v") | regs(y, "v") | regs(c, "v")
+        for operand, what in holds:
+            for r in regs(operand, "v"):
+                assert self.holds.get(r) == what, ("another read came in between", r, what, self.holds.get(r))
+        self.fresh(used | regs(d, "v"))
+        for r in used:
+            assert self.count - self.valu_at.get(r, -99) >= 3, ("MFMA too soon behind", r, self.lines[-3:])
+        self.put("%s %s, %s, %s, %s" % (self.mfma_name, d, x, y, c))
+        self.mfmas += 1
+        for r in regs(d, "v"):
+            self.mfma_at[r] = self.mfmas
+
+    def valu(self, op, d, *src, trans=False):
+        used = set().union(*[regs(x, "v") for x in src])
+        self.fresh(used | regs(d, "v"))
+        assert not (self.trans & used), ("behind a transcendental", op, d, src)
+        for r in used | regs(d, "v"):
+            assert self.mfmas - self.mfma_at.get(r, -99) >= 2, ("too soon behind the MFMA of", r, self.lines[-3:])
+        self.put("%s %s" % (op, ", ".join((d,) + src)))
+        for r in regs(d, "v"):
+            self.valu_at[r] = self.count
+        self.trans = regs(d, "v") if trans else set()
+
+    def settled(self):
+        """Behind a wait that covers every MFMA."""
+        self.mfma_at = {}
+
+
+class DKV:
+    """dK/dV: the loop over a wavefront's tiles of 32 query rows, two stages unrolled.
+
+    Steps of four MFMAs (one per block of 16 keys): 0..7 S (k step, row block), 8..15 dP, 16..23 dV (d block), 24..31 dK.
+    """
+    KEEP = 100                                     # VGPRs below this are the compiler's (operands)
+    S, DP, PP, DSP, RING, L4, D4, E = 100, 132, 164, 180, 196, 228, 236, 244
+    NEG = 248
+    RSQ, RSD, RSL, QSTEP, DSTEP, QWRAP, DWRAP, LWRAP, DSC, DSS, DSTEP_DS, WRAP_DS, T, CTC = 40, 44, 48, 52, 54, 56, 58, 60, 62, 64, 66, 68, 70, 76
+    LOOK = 15                                      # MFMAs between an LDS read and its use
+    ROWB, QTB, SLOTB = 256, 8192, 16640
+
+    def __init__(self, dtype, store_ds):
+        self.store_ds = store_ds
+        self.x = Stream(dtype)
+        # K fragments of three k steps lie where dP and P's pairs come to be
+        self.fk = [[self.DP + 4 * kb for kb in range(4)], [self.DP + 16 + 4 * kb for kb in range(4)], [self.PP + 4 * kb for kb in range(4)]]
+        self.ops = self.tile_reads()
+
+    def ring(self, step):
+        return self.RING + 4 * (step % 8)
+
+    def tile_reads(self):
+        """LDS reads of a tile in order: (first MFMA that uses it, destination, width, function of the stage's offset)."""
+        ops = []
+        for step in range(32):
+            u, r = 4 * step, self.ring(step)
+            if step < 8:
+                ks, qb = step // 2, step % 2
+                if qb == 0:
+                    for kb in range(4):
+                        ops.append((u + kb, self.fk[ks % 3][kb], 4, lambda st, d, ks=ks, kb=kb: "ds_read_b128 %s, %%[rk%d] offset:%d" % (v(d, 4), ks, 16 * self.ROWB * kb)))
+                        if kb == 0:
+                            ops.append((u, r, 4, lambda st, d, ks=ks: "ds_read_b128 %s, %%[rq%d] offset:%d" % (v(d, 4), ks, st)))
+                else:
+                    ops.append((u, r, 4, lambda st, d, ks=ks: "ds_read_b128 %s, %%[rq%d] offset:%d" % (v(d, 4), ks, st + 16 * self.ROWB)))
+            elif step < 16:
+                ks, qb = (step - 8) // 2, step % 2
+                ops.append((u, r, 4, lambda st, d, ks=ks, qb=qb: "ds_read_b128 %s, %%[rq%d] offset:%d" % (v(d, 4), ks, st + self.QTB + 16 * self.ROWB * qb)))
+                if step in (8, 9):
+                    ops.append((u, self.D4 + 4 * qb, 4, lambda st, d, qb=qb: "ds_read_b128 %s, %%[ldr] offset:%d" % (v(d, 4), st + 128 + 64 * qb)))
+                    ops.append((u, self.L4 + 4 * qb, 4, lambda st, d, qb=qb: "ds_read_b128 %s, %%[ldr] offset:%d" % (v(d, 4), st + 64 * qb)))
+            else:
+                t, off = step % 8, self.QTB if step < 24 else 0
+                for h in range(2):
+                    ops.append((u, r + 2 * h, 2, lambda st, d, t=t, off=off, h=h: "ds_read_b64_tr_b16 %s, %%[ta%d] offset:%d" % (v(d, 2), t, st + off + 16 * self.ROWB * h)))
+        # the slot behind which each is issued: LOOK MFMAs ahead, one a slot (negative: during the tile before)
+        slot, out = -10 ** 9, []
+        for use, d, n, f in ops:
+            slot = max(slot + 1, use - self.LOOK)
+            assert slot < use
+            out.append((slot, use, d, n, f))
+        return out
+
+    def vector_work(self):
+        """Vector instructions behind each MFMA: {slot: [function, ..]}.
+
+        Pair j of P and of dS: rows 2 (j % 2) .. of row block (j / 2) % 2, key block j / 4."""
+        x, work = self.x, {}
+
+        def at(j):
+            kb, qb, e = j >> 2, (j >> 1) & 1, 2 * (j & 1)
+            return kb, qb, e, self.S + 4 * (4 * qb + kb) + e, self.DP + 4 * (4 * qb + kb) + e
+
+        def p_fma(j):
+            kb, qb, e, p, _ = at(j)
+            for i in range(2):
+                x.valu("v_fma_f32", v(p + i), v(p + i), "%[scale]", "-" + v(self.L4 + 4 * qb + e + i))
+
+        def p_exp(j):
+            p = at(j)[3]
+            for i in range(2):
+                x.valu("v_exp_f32", v(p + i), v(p + i), trans=True)
+
+        def p_pack(j):
+            p = at(j)[3]
+            x.valu(x.pack_name, v(self.PP + 4 * (j >> 2) + (j & 3)), v(p), v(p + 1))
+
+        def ds_mul(j):
+            _, _, _, p, d = at(j)
+            for i in range(2):
+                x.valu("v_mul_f32", v(p + i), v(p + i), v(d + i))
+
+        def ds_pack(j):
+            p = at(j)[3]
+            x.valu(x.pack_name, v(self.DSP + 4 * (j >> 2) + (j & 3)), v(p), v(p + 1))
+
+        def put(slot, f, j):
+            work.setdefault(slot, []).append(lambda: f(j))
+        # P beneath dP (MFMAs 32..63) and the first of dV, dS beneath the rest of dV
+        for j in range(16):
+            base = 33 + 29 * j // 15
+            put(base, p_fma, j)
+            put(base + 1, p_exp, j)
+            put(base + 2, p_pack, j)
+            base = 68 + 26 * j // 16
+            put(base, ds_mul, j)
+            put(base + 1, ds_pack, j)
+        return work
+
+    def advance(self):
+        """To the tile that is copied next, as pieces of scalar code: its rows (a descriptor of no bytes behind the last tile)."""
+        R = self
+        out = [["s_mov_b32 s%d, %%[ct]" % R.CTC, "s_add_u32 %[ct], %[ct], 4"]]
+        if self.store_ds:
+            out += [["s_mov_b64 %s, %s" % (s(R.DSS, 2), s(R.DSC, 2))], ["s_add_u32 %s, %s, %s" % (s(R.DSC), s(R.DSC), s(R.DSTEP_DS)), "s_addc_u32 %s, %s, %s" % (s(R.DSC + 1), s(R.DSC + 1), s(R.DSTEP_DS + 1))]]
+        for p, st in ((R.RSQ, R.QSTEP), (R.RSD, R.DSTEP)):
+            out.append(["s_add_u32 %s, %s, %s" % (s(p), s(p), s(st)), "s_addc_u32 %s, %s, %s" % (s(p + 1), s(p + 1), s(st + 1))])
+        out.append(["s_add_u32 %s, %s, 0x200" % (s(R.RSL), s(R.RSL)), "s_addc_u32 %s, %s, 0" % (s(R.RSL + 1), s(R.RSL + 1))])
+        out.append(["s_cmp_ge_i32 %[ct], %[ntq]", "s_cbranch_scc1 WRAP{0}", "BACK{0}:"])
+        t = s(R.T)
+        out.append(["s_lshl_b32 %s, %%[ct], 5" % t, "s_sub_i32 %s, %%[rows], %s" % (t, t)])
+        out.append(["s_min_i32 %s, %s, 32" % (t, t), "s_sub_i32 %s, %s, 1" % (t, t)])
+        out.append(["s_mul_i32 %s, %s, %%[qrowb]" % (s(R.RSQ + 2), t), "s_mul_i32 %s, %s, %%[drowb]" % (s(R.RSD + 2), t)])
+        out.append(["s_add_u32 %s, %s, 0x100" % (s(R.RSQ + 2), s(R.RSQ + 2)), "s_add_u32 %s, %s, 0x100" % (s(R.RSD + 2), s(R.RSD + 2))])
+        out.append(["s_cmp_gt_i32 %[rem], 1"] + ["s_cselect_b32 %s, %s, 0" % (s(r + 2), s(r + 2)) for r in (R.RSQ, R.RSD)] +
+                   ["s_cselect_b32 %s, %%[ldbytes], 0" % s(R.RSL + 2)])
+        return out
+
+    def wrap(self, i):
+        """Out of line: the copied tile is past the head's last one; the same tile of the next head."""
+        R = self
+        self.label("WRAP%d" % i)
+        pairs = [(R.RSQ, R.QWRAP), (R.RSD, R.DWRAP), (R.RSL, R.LWRAP)] + ([(R.DSC, R.WRAP_DS)] if self.store_ds else [])
+        for p, w in pairs:
+            self.x.put("s_add_u32 %s, %s, %s" % (s(p), s(p), s(w)))
+            self.x.put("s_addc_u32 %s, %s, %s" % (s(p + 1), s(p + 1), s(w + 1)))
+        self.x.put("s_sub_u32 %[ct], %[ct], %[ntq]")
+        self.x.put("s_cmp_ge_i32 %[ct], %[ntq]")
+        self.x.put("s_cbranch_scc1 %s" % self.ref("WRAP%d" % i))
+        self.x.put("s_branch %s" % self.ref("BACK%d" % i))
+
+    def ref(self, name):
+        return "L%s_%%=" % name
+
+    def label(self, name):
+        self.x.lines.append(self.ref(name) + ":")
+
+    def scalar(self, piece, i):
+        for line in piece:
+            if line == "BACK{0}:":
+                self.label("BACK%d" % i)
+            elif "WRAP{0}" in line:
+                self.x.put("s_cbranch_scc1 %s" % self.ref("WRAP%d" % i))
+            else:
+                self.x.put(line)
+
+    def mask(self, i):
+        """Out of line: scores past the diagonal (and, where dS is kept, of keys past the end) become -inf."""
+        x = self.x
+        self.label("MASK%d" % i)
+        x.put("s_nop 15")
+        x.put("s_nop 7")
+        tmp = self.E
+        x.put("v_mov_b32 %s, 0xff800000" % v(self.NEG))
+        x.put("s_lshl_b32 %s, %s, 5" % (s(self.T), s(self.CTC)))
+        x.put("v_subrev_u32 %s, %s, %%[vx]" % (v(tmp), s(self.T)))
+        for qb in range(2):
+            for kb in range(4):
+                for e in range(4):
+                    r = v(self.S + 4 * (4 * qb + kb) + e)
+                    x.put("v_cmp_lt_i32 vcc, %d, %s" % (16 * qb + e - 16 * kb, v(tmp)))
+                    x.put("s_nop 1")
+                    x.put("v_cndmask_b32 %s, %s, %s, vcc" % (r, r, v(self.NEG)))
+        if self.store_ds:
+            for kb in range(4):
+                x.put("v_cmp_le_i32 vcc, %d, %%[vy]" % (-16 * kb))
+                x.put("s_nop 1")
+                for qb in range(2):
+                    for e in range(4):
+                        r = v(self.S + 4 * (4 * qb + kb) + e)
+                        x.put("v_cndmask_b32 %s, %s, %s, vcc" % (r, r, v(self.NEG)))
+        x.put("s_branch %s" % self.ref("MASKED%d" % i))
+
+    def tile(self, stage):
+        x, st, nx = self.x, self.SLOTB * stage, self.SLOTB * (1 - stage)
+        issue = {}
+        for slot, use, d, n, f in self.ops:
+            if slot >= 0:
+                issue.setdefault(slot, []).append((f(st, d), d, n, use // 4))
+        for slot, use, d, n, f in self.ops:          # the next tile's first ones
+            if slot < 0:
+                issue.setdefault(128 + slot, []).append((f(nx, d), d, n, use // 4))
+        first_ahead = 128 + min(o[0] for o in self.ops)
+        work = self.vector_work()
+        copies = [("q", i) for i in range(8)] + [("d", i) for i in range(8)] + [("l", 0)]
+        adv = self.advance()
+        adv_at = {97 + i: p for i, p in enumerate(adv)}
+        assert 97 + len(adv) <= first_ahead + 16
+        nstores = 8 if self.store_ds else 0
+        for m in range(128):
+            step, kb = m // 4, m % 4
+            r = self.ring(step)
+            copy = copies[m // 2 + (m == 31)] if m < 32 and (m % 2 == 0 or m == 31) and m // 2 + (m == 31) < 17 else None
+            if copy:
+                c, i = copy
+                x.put("s_add_u32 m0, %%[wbase], %d" % (nx + {"q": 1024 * i, "d": self.QTB + 1024 * i, "l": 2 * self.QTB}[c]))
+            if m == first_ahead:
+                x.put("s_waitcnt vmcnt(%d)" % nstores)         # the next tile has landed
+            if m == 32:                                        # scores of the diagonal
+                x.put("s_cbranch_vccnz %s" % self.ref("MASK%d" % stage))
+                self.label("MASKED%d" % stage)
+            frag = v(r, 4)
+            if step < 8:
+                ks, qb = step // 2, step % 2
+                d, y = self.S + 4 * (4 * qb + kb), v(self.fk[ks % 3][kb], 4)
+                need = set(range(r, r + 4)) | regs(y, "v")
+                c = "0" if ks == 0 else v(d, 4)
+                out = v(d, 4)
+            elif step < 16:
+                ks, qb = (step - 8) // 2, step % 2
+                d, y = self.DP + 4 * (4 * qb + kb), "%%[V%d%d]" % (kb, ks)
+                need = set(range(r, r + 4)) | (set(range(self.D4 + 4 * qb, self.D4 + 4 * qb + 4)) if ks == 0 else set())
+                c = v(self.D4 + 4 * qb, 4) if ks == 0 else v(d, 4)
+                out = v(d, 4)
+            else:
+                t = step % 8
+                out = c = "%%[%s%d%d]" % ("dv" if step < 24 else "dk", kb, t)
+                y = v((self.PP if step < 24 else self.DSP) + 4 * kb, 4)
+                need = set(range(r, r + 4))
+            if kb == 0 and step % 2 == 0:                      # one wait for two steps where the later reads are old enough
+                later = self.ring(step + 1) if step < 31 else None
+                if later is not None:
+                    need |= set(range(later, later + 4))
+                if step < 8:
+                    need |= set(range(self.fk[(step // 2) % 3][0], self.fk[(step // 2) % 3][0] + 16))
+                if step == 8:
+                    need |= set(range(self.L4, self.L4 + 8)) | set(range(self.D4, self.D4 + 8))
+            x.wait(need)
+            x.mfma(out, frag, y, c, [(frag, step)] + ([(y, step & ~1)] if step < 8 else []) + ([(c, step)] if step in (8, 9) else []))
+            if copy:
+                c, i = copy
+                if c == "l":
+                    x.put("buffer_load_dword %%[cld], %s, 0 offen lds" % s(self.RSL, 4))
+                else:
+                    x.put("buffer_load_dwordx4 %%[c%s%d], %s, %s offen lds" % (c, i & 3, s(self.RSQ if c == "q" else self.RSD, 4), "0" if i < 4 else "%%[%s16]" % c))
+            for text, d, n, what in issue.get(m, []):
+                x.lds(text, d, n, what)
+            for f in work.get(m, []):
+                f()
+            if m == 20:                                        # whether this tile has scores to mask: vcc for the branch at 32
+                x.put("s_cmp_lt_i32 %s, %%[mct]" % s(self.CTC))
+                x.put("s_cselect_b64 vcc, -1, 0")
+                if self.store_ds:
+                    x.put("s_cmp_lg_u32 %[dsmask], 0")
+                    x.put("s_cselect_b64 vcc, -1, vcc")
+            if self.store_ds and 98 <= m < 98 + 8:
+                i = m - 98
+                kb_, qb_ = i >> 1, i & 1
+                x.put("global_store_dwordx2 %%[dso], %s, %s offset:%d" % (v(self.DSP + 4 * kb_ + 2 * qb_, 2), s(self.DSS, 2), (kb_ >> 1) * 2048 + qb_ * 1024 + (kb_ & 1) * 256))
+            if m == 96:
+                x.put("s_sub_u32 %[rem], %[rem], 1")
+            shift = 10 if self.store_ds else 0                 # behind the stores, which need the tile's own address
+            if m - shift in adv_at:
+                self.scalar(adv_at[m - shift], stage)
+
+    def text(self):
+        x, R = self.x, self
+        for dst, name in ((R.RSQ, "qp"), (R.RSD, "dp"), (R.RSL, "lp"), (R.QSTEP, "qstep"), (R.DSTEP, "dstep"), (R.QWRAP, "qwrap"),
+                          (R.DWRAP, "dwrap"), (R.LWRAP, "lwrap")) + (((R.DSC, "dsp"), (R.DSTEP_DS, "dsstep"), (R.WRAP_DS, "dswrap")) if self.store_ds else ()):
+            x.put("s_mov_b64 %s, %%[%s]" % (s(dst, 2), name))
+        for r in (R.RSQ, R.RSD, R.RSL):
+            x.put("s_mov_b32 %s, 0x20000" % s(r + 3))
+        for i in range(4):
+            x.put("v_mov_b32 %s, 0" % v(R.RING + i))
+        x.put("s_nop 3")
+        for i in range(64):                        # dV = dK = 0
+            x.put("%s %%[d%s%d%d], %s, %s, 0" % (x.mfma_name, "vk"[i // 32], i // 8 % 4, i % 8, v(R.RING, 4), v(R.RING, 4)))
+        x.put("s_waitcnt vmcnt(0)")
+        x.put("s_barrier")                         # the K tile and the first tile are there
+        x.put("s_cmp_eq_u32 %[rem], 0")
+        x.put("s_cbranch_scc1 %s" % self.ref("END"))
+        for piece in self.advance():
+            self.scalar(piece, 2)
+        for slot, use, d, n, f in self.ops:
+            if slot < 0:
+                x.lds(f(0, d), d, n, use // 4)
+        start = [set(r) for r in x.reads]
+        self.label("LOOP")
+        for stage in range(2):
+            self.tile(stage)
+            assert len(x.reads) <= len(start) and x.reads == start[-len(x.reads):], "the two ends of the loop differ"
+            x.reads = [set(r) for r in start]
+            x.put("s_cmp_eq_u32 %[rem], 0")
+            x.put("s_cbranch_scc%d %s" % ((1, self.ref("END")) if stage == 0 else (0, self.ref("LOOP"))))
+        x.put("s_branch %s" % self.ref("END"))
+        for i in range(3):
+            self.wrap(i)
+        for i in range(2):
+            self.mask(i)
+        self.label("END")
+        x.put("s_waitcnt vmcnt(0) lgkmcnt(0)")
+        x.put("s_nop 15")
+        x.put("s_nop 7")
+        return x.lines
+
+
+def define(name, lines):
+    return "#define %s \\\n" % name + " \\\n".join('  "%s\\n\\t"' % l for l in lines) + "\n"
+
+
+def clobbers(name, first_v, last_v, first_s, last_s):
+    names = ["v%d" % i for i in range(first_v, last_v + 1)] + ["s%d" % i for i in range(first_s, last_s + 1)] + ["vcc", "memory"]
+    return "#define %s %s\n" % (name, ", ".join('"%s"' % n for n in names))
+
+
+def generate():
+    out = ["// Written by attn_loops.py.\n#pragma once\n"]
+    for dtype in ("bf16", "f16"):
+        for ds in (False, True):
+            out.append(define("DH_DKV128_LOOP_%s%s" % (dtype.upper(), "_DS" if ds else ""), DKV(dtype, ds).text()))
+    out.append(clobbers("DH_DKV128_CLOBBERS", DKV.KEEP, DKV.NEG, DKV.RSQ, DKV.CTC))
+    return "".join(out)
+
+
+if __name__ == "__main__":
+    with open(sys.argv[1], "w") as f:
+        f.write(generate())

@@ -102,3 +102,34 @@ def test_lanes_of_the_routing(tokens, experts, k, lanes):
     """A scan where it was measured the faster: few experts, or tokens enough to fill the chip with a thread each."""
     from dhellam_amd import _lib
     assert _lib.load().dh_moe_route_lanes(tokens, experts, k) == lanes
+
+
+@pytest.fixture(scope="module")
+def loops():
+    import importlib.util
+    from dhellam_amd.build import CSRC
+    spec = importlib.util.spec_from_file_location("attn_loops", CSRC / "attn_loops.py")
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+    return mod
+
+
+def test_attention_loops_keep_their_own_account(loops):
+    """The attention loops are written with an account of what is in flight; every form of them passes it."""
+    assert loops.generate().count("#define DH_") >= 5
+
+
+@pytest.mark.parametrize("fault,code", [
+    ("read in flight", lambda x: (x.lds("", 100, 4), x.mfma("v[104:107]", "v[100:103]", "v[108:111]", "0"))),
+    ("two reads in flight", lambda x: (x.lds("", 100, 4), x.lds("", 102, 4))),
+    ("another read", lambda x: (x.lds("", 100, 4, 1), x.lds("", 104, 4, 2), x.wait({100, 104}), x.mfma("v[112:115]", "v[100:103]", "v[104:107]", "0", [("v[104:107]", 3)]))),
+    ("too soon behind the MFMA", lambda x: (x.mfma("v[100:103]", "v[104:107]", "v[108:111]", "0"), x.valu("v_mul_f32", "v1", "v100", "v2"))),
+    ("MFMA too soon", lambda x: (x.valu("v_mul_f32", "v100", "v1", "v2"), x.mfma("v[104:107]", "v[100:103]", "v[108:111]", "0"))),
+    ("transcendental", lambda x: (x.valu("v_exp_f32", "v100", "v1", trans=True), x.valu("v_mul_f32", "v1", "v100", "v2"))),
+])
+def test_attention_loops_refuse_what_the_hardware_would_not_wait_for(loops, fault, code):
+    with pytest.raises(AssertionError, match=fault):
+        code(loops.Stream("bf16"))
+    x = loops.Stream("bf16")              # waited for, the reads that may be in flight are the younger ones
+    x.lds("", 100, 4), x.lds("", 104, 4), x.wait({100})
+    assert x.lines[-1] == "s_waitcnt lgkmcnt(1)" and x.reads == [set(range(104, 108))]
