@@ -1,7 +1,7 @@
 // Flash-attention backward on bf16/fp16 MFMA (gfx950), deterministic (no
 // floating-point atomics).
 //
-// Three kernels:
+// Three kernels (head dim 128 has them in attn_bwd_dkv128.h and attn_bwd_dq128.h, one wavefront on a SIMD):
 //   delta   : delta_i = sum_d dO[i,d] * O[i,d]                      (streaming; for fp32 and where dS is kept: the
 //             recomputing dQ kernels form delta in their prologue and run first)
 //   dK/dV   : a workgroup owns 64 key/value rows (K, V fragments stay in
@@ -19,6 +19,7 @@
 //             dS^T feeds dQ^T += K^T dS^T.
 // Recomputing S and dP in both passes costs 7 matrix products instead of 5 but
 // needs no fp32 dQ accumulator in memory and no atomics.
+#include <algorithm>
 #include <atomic>
 
 #include "attn_route.h"
@@ -148,6 +149,7 @@ attn_bwd_gqa_sum_kernel(const float *__restrict__ dk_part, const float *__restri
 }  // namespace dh
 
 #include "attn_bwd_dkv128.h"
+#include "attn_bwd_dq128.h"
 
 namespace dh {
 
@@ -689,6 +691,14 @@ static int launch_dq2_d128(const AttnBwdParams &p, int batch, hipStream_t st) {
   return DH_OK;
 }
 
+template <typename T, int RG>
+static int launch_dq128(const AttnBwdParams &p, int batch, hipStream_t st) {
+  const int nqt = (int)cdiv(p.max_sq, 64 * RG);
+  dim3 grid((unsigned)((p.causal ? (nqt + 1) / 2 : nqt) * p.hq), (unsigned)batch);
+  hipLaunchKernelGGL((attn_bwd_dq128_kernel<T, RG>), grid, dim3(256), 0, st, p);
+  return DH_OK;
+}
+
 template <typename T, int RG, int SPLIT, int BN>
 static int launch_dq_d128(const AttnBwdParams &p, int batch, hipStream_t st) {
   constexpr int BM = 32 * RG;
@@ -752,7 +762,7 @@ int attn_bwd_f32(const void *dout, const void *q, const void *k, const void *v, 
                  int dq_accumulate, hipStream_t st);
 
 constexpr int DKV_ROWS = 64;  // key rows of a dK/dV workgroup
-constexpr int64_t DKV_MAX_STRIDE = 1ll << 26;   // elements: 32 rows of them are less than 4 GiB
+constexpr int64_t ROWS_MAX_STRIDE = 1ll << 26;   // elements: 32 rows of them are less than 4 GiB
 
 // Keeping dS for the dQ product costs 2 bytes per (head, query, key) of workspace, written once and read once.
 // It pays where the recomputing dQ kernel runs its small-grid form (fewer than 256 workgroups of 128 query rows:
@@ -844,15 +854,27 @@ static BwdBoth bwd_both(int batch, int max_sq, int max_sk, int64_t total_q, int6
   return {t >= (double)cdiv(b, 256) * rho && room(t) >= a, hs};
 }
 
+// Workgroups of recomputing dQ with work, tiles of `rows`.  The kernel with one wavefront a SIMD takes them where they come to four fifths of
+// the compute units, in tiles of 256 rows (K and V are read once for four wavefronts) or else of 128: its loop is the faster one
+// (1860 and 1915 cycles for what took 3400), but a tile's rows are loaded and stored in 24000, which the kernel of eight wavefronts
+// hides better where little follows.  Whole backward, us, eight wavefronts / 128 / 256 rows, causal unless said: 32 query / 8
+// kv heads x 4096 469 / 409 / 381, x 2048 (128 tiles of 256) 159 / 148 / 176, 8 x 1024 331 / 331 / 297, 16 x 512 243 / 255 / 229, not causal 16 heads x
+// 2048 141 / 125 / 142, 2786 + 479 (208 tiles) 277 / 240 / 220, 8 / 1 x 4096 237 / 203 / 242, 1022 to 223 (88 and 160 tiles) 80 / 87 / 93.
+static int64_t dq_wgs(int rows, int max_sq, int hq, int batch, int causal, int64_t total_q) {
+  const int64_t bound = (int64_t)batch * max_sq, q = total_q < bound ? total_q : bound;
+  return (int64_t)((double)attn_wgs(max_sq, rows, hq, batch, causal) * (double)q / (double)bound);
+}
+
 // What one 16-bit call runs.
 struct AttnBwdRoute {
   bool keep_ds;      // dK/dV keeps dS and dQ is one product over it; else dQ recomputes, first, and forms delta
   bool hand_dkv, hand_dq;      // head dim 128's hand-ordered kernels
   bool big_dq;       // 128-row query tiles in dQ
+  int dq_rows;       // ... of the hand-ordered kernels: tiles of 256 or 128 rows on one wavefront a SIMD, or 0: the one of eight wavefronts
   bool both;         // dK/dV and dQ in one launch of the tile kernels, behind the delta kernel
   int hsplit;        // workgroups that share a GQA group in dK/dV
 };
-// `wide`: token strides that the 32-bit copy offsets of the dK/dV kernel do not reach across a tile.
+// `wide`: token strides that the 32-bit copy offsets of the hand-ordered kernels do not reach across a tile.
 static AttnBwdRoute attn_bwd_route(int batch, int max_sq, int max_sk, int64_t total_q, int64_t total_k, int hq, int hk, int d,
                                    int causal, bool room_for_ds, bool wide = false) {
   const BwdBoth both = bwd_both(batch, max_sq, max_sk, total_q, total_k, hq, hk, d, causal);
@@ -864,6 +886,7 @@ static AttnBwdRoute attn_bwd_route(int batch, int max_sq, int max_sk, int64_t to
   const bool fills = d <= 128 && dq_tile_fills(max_sq, hq, batch);
   r.both = both.pays && (d == 128 || !fills);
   r.big_dq = r.hand_dq ? big : fills && !r.both;
+  r.dq_rows = !(r.hand_dq && big) ? 0 : dq_wgs(256, max_sq, hq, batch, causal, total_q) >= 208 ? 256 : dq_wgs(128, max_sq, hq, batch, causal, total_q) >= 208 ? 128 : 0;
   r.hsplit = r.both ? both.hsplit : bwd_hsplit(max_sk, batch, hq, hk, d == 128 && causal);
   return r;
 }
@@ -878,7 +901,7 @@ static int bwd_passes(const AttnBwdParams &p, const AttnBwdRoute &r, int batch, 
     else rc = launch_both_tile<T, D, 2, 2, 2, 2, 1>(p, batch, max_sk, st);
   } else if (max_sq > 0 && !r.keep_ds) {
     if constexpr (D == 128) {
-      if (r.hand_dq) rc = r.big_dq ? launch_dq_d128<T, 4, 2, 32>(p, batch, st) : launch_dq_d128<T, 2, 4, 32>(p, batch, st);
+      if (r.hand_dq) rc = r.big_dq ? (r.dq_rows == 256 ? launch_dq128<T, 4>(p, batch, st) : r.dq_rows == 128 ? launch_dq128<T, 2>(p, batch, st) : launch_dq_d128<T, 4, 2, 32>(p, batch, st)) : launch_dq_d128<T, 2, 4, 32>(p, batch, st);
       else rc = r.big_dq ? launch_dq_tile<T, D, 4, 2, 2>(p, batch, st) : launch_dq_tile<T, D, 2, 4, 2>(p, batch, st);
     } else if constexpr (D < 128) {
       rc = r.big_dq ? launch_dq_tile<T, D, 4, 2, D == 64 ? 4 : 2>(p, batch, st) : launch_dq_tile<T, D, 2, 4, 2>(p, batch, st);
@@ -1010,7 +1033,7 @@ static int attn_bwd_entry(const void *dout, const void *q, const void *k, const 
   size_t dsb = ds_bytes(batch, max_seqlen_q, total_k, hq, d, dtype, causal);
   if (dsb > 0 && base_bytes + align256(dsb) > workspace_bytes) dsb = 0;
   const AttnBwdRoute route = attn_bwd_route(batch, max_seqlen_q, max_seqlen_k, total_q, total_k, hq, hk, d, causal, dsb > 0,
-                                            q_stride > DKV_MAX_STRIDE || k_stride > DKV_MAX_STRIDE || do_stride > DKV_MAX_STRIDE);
+                                            std::max({q_stride, k_stride, v_stride, do_stride}) > ROWS_MAX_STRIDE);
   uint8_t *ds_ws = (uint8_t *)(((uintptr_t)workspace + 255) & ~(uintptr_t)255) + (base_bytes - 256);
   const bool delta_in_dq = dtype != DH_F32 && !route.keep_ds;
   if (max_seqlen_q > 0 && !delta_in_dq) {

@@ -402,6 +402,214 @@ class DKV:
         return x.lines
 
 
+class Keys:
+    """What the loops over key tiles have in common: a wavefront holds 64 query rows (four blocks of 16) and walks tiles of 32 keys of
+    its stream; the wavefronts of a stream, two or four, copy a tile together (`copies` of its 16 KB each: K or V, or half of
+    one), three tiles ahead into four stages, and meet at one barrier a tile, placed where the tile's last LDS read has been waited for.
+
+    The query index is on lanes: block (kb, qb) of S^T is key rows 16 kb + 4 g + v and query 16 qb + r of lane 16 g + r.
+    """
+    STAGES, TILEB, STAGEB = 4, 8192, 16384         # bytes of a K (or V) tile and of a stage of a stream
+    ROWB = 256
+
+    def __init__(self, dtype, copies):
+        self.x = Stream(dtype)
+        self.copies = copies
+
+    def ref(self, name):
+        return "L%s_%%=" % name
+
+    def label(self, name):
+        self.x.lines.append(self.ref(name) + ":")
+
+    # scalar registers: the descriptor of the rows that are copied next and how many are left of them; the tile's first key
+    RSC, CSTEP, CLEFT, KEY, T = 40, 44, 46, 47, 48
+
+    def enter(self):
+        x = self.x
+        for dst, name in ((self.RSC, "cp"), (self.CSTEP, "cstep")):
+            x.put("s_mov_b64 %s, %%[%s]" % (s(dst, 2), name))
+        x.put("s_mov_b32 %s, 0x20000" % s(self.RSC + 3))
+        x.put("s_mov_b32 %s, %%[left]" % s(self.CLEFT))
+        x.put("s_mov_b32 %s, %%[key]" % s(self.KEY))
+
+    def rows_left(self):
+        """Pieces of scalar code: the descriptor's length for the rows that are left."""
+        r, t = self, s(self.T)
+        return [["s_min_i32 %s, %s, %d" % (t, s(r.CLEFT), 4 * r.copies), "s_mul_i32 %s, %s, %%[crowb]" % (t, t)],
+                ["s_sub_u32 %s, %s, %%[crowb]" % (t, t), "s_add_u32 %s, %s, 0x100" % (t, t)],
+                ["s_cmp_gt_i32 %s, 0" % s(r.CLEFT), "s_cselect_b32 %s, %s, 0" % (s(r.RSC + 2), t)]]
+
+    def to_next_rows(self):
+        r = self
+        return [["s_add_u32 %s, %s, %s" % (s(r.RSC), s(r.RSC), s(r.CSTEP)), "s_addc_u32 %s, %s, %s" % (s(r.RSC + 1), s(r.RSC + 1), s(r.CSTEP + 1))],
+                ["s_sub_i32 %s, %s, %%[keystep]" % (s(r.CLEFT), s(r.CLEFT))]] + self.rows_left()
+
+    def copy(self, i, stage, before):
+        """Copy i of a tile, on both sides of an MFMA."""
+        if before:
+            self.x.put("s_add_u32 m0, %%[cdst], %d" % (stage * self.STAGEB + 1024 * i))
+        else:
+            self.x.put("buffer_load_dwordx4 %%[cl%d], %s, %s offen lds" % (i & 3, s(self.RSC, 4), "0" if i < 4 else "%[c16]"))
+
+    def loop(self, tile, first_reads):
+        """The unrolled stages of the loop between its labels; `first_reads(stage)` are those in front of the first tile."""
+        x = self.x
+        x.put("s_cmp_eq_u32 %[rem], 0")
+        x.put("s_cbranch_scc1 %s" % self.ref("END"))
+        first_reads()
+        start = [set(r) for r in x.reads]
+        self.label("LOOP")
+        for stage in range(self.STAGES):
+            tile(stage)
+            assert x.reads == start[len(start) - len(x.reads):], "the two ends of the loop differ"
+            x.reads = [set(r) for r in start]
+            x.put("s_sub_u32 %[rem], %[rem], 1")
+            x.put("s_cmp_eq_u32 %[rem], 0")
+            last = stage == self.STAGES - 1
+            x.put("s_cbranch_scc%d %s" % (0 if last else 1, self.ref("LOOP" if last else "END")))
+        x.put("s_branch %s" % self.ref("END"))
+
+    def leave(self):
+        self.label("END")
+        self.x.put("s_waitcnt vmcnt(0) lgkmcnt(0)")
+        self.x.put("s_nop 15")
+        self.x.put("s_nop 7")
+
+    def mask_lanes(self, cx, cy):
+        """cx = key - row and cy = key - keys of the tile's element (0, 0) of a lane."""
+        self.x.put("v_add_u32 %s, %s, %%[vx]" % (v(cx), s(self.KEY)))
+        self.x.put("v_add_u32 %s, %s, %%[vy]" % (v(cy), s(self.KEY)))
+
+    def mask(self, first, value, cx, cy):
+        """The values of a tile (registers from `first`, [qb][kb][v]) past the diagonal or the last key become `value`."""
+        x = self.x
+        for qb in range(4):
+            for kb in range(2):
+                for e in range(4):
+                    r = v(first + 4 * (2 * qb + kb) + e)
+                    for c, op, bound in ((cx, "lt", 16 * qb - 16 * kb - e), (cy, "le", -16 * kb - e)):
+                        x.put("v_cmp_%s_i32 vcc, %d, %s" % (op, bound, v(c)))
+                        x.put("s_nop 1")
+                        x.put("v_cndmask_b32 %s, %s, %s, vcc" % (r, r, value))
+
+
+class DQ(Keys):
+    """dQ: S^T = K Q^T, dP^T = V dO^T - delta, dQ^T += K^T dS^T; 96 MFMAs a tile, a query block after the other in each phase, so that
+    P and dS of a block are formed beneath the next blocks' MFMAs."""
+    KEEP = 72
+    S, DP, DSP, KF, VF, KT, CX, CY, ZERO = 72, 104, 136, 152, 184, 216, 248, 249, 250
+
+    def reads(self, stage):
+        """(first MFMA that uses it, MFMA behind which it is issued, destination, width, text) in the order of issue."""
+        st, nx, out = stage * self.STAGEB, (stage + 1) % self.STAGES * self.STAGEB, []
+        for i in range(8):
+            ks, kb = i // 2, i % 2
+            out.append((32 + i, 8 + 2 * i, self.VF + 4 * i, 4, "ds_read_b128 %s, %%[rk%d] offset:%d" % (v(self.VF + 4 * i, 4), ks, st + self.TILEB + 16 * self.ROWB * kb)))
+        for i in range(16):
+            t, h = i // 2, i % 2
+            d = self.KT + 4 * t + 2 * h
+            out.append((64 + t, 26 + 3 * i // 2, d, 2, "ds_read_b64_tr_b16 %s, %%[ta%d] offset:%d" % (v(d, 2), t, st + 16 * self.ROWB * h)))
+        for i in range(8):
+            out.append((96 + i, self.AT_BARRIER + 2 * i, self.KF + 4 * i, 4, self.k_read(i, nx)))
+        return out
+
+    AT_BARRIER = 74
+
+    def k_read(self, i, st):
+        return "ds_read_b128 %s, %%[rk%d] offset:%d" % (v(self.KF + 4 * i, 4), i // 2, st + 16 * self.ROWB * (i % 2))
+
+    def first_reads(self):
+        for i in range(8):
+            self.x.lds(self.k_read(i, 0), self.KF + 4 * i, 4, 96 + i)
+
+    def vector_work(self):
+        x, work = self.x, {}
+
+        def put(slot, f, *args, **kw):
+            work.setdefault(slot, []).append(lambda: f(*args, **kw))
+        for j in range(16):                        # pairs: query block j / 4, key block (j / 2) % 2, rows 2 (j % 2) ..
+            qb, kb, e = j >> 2, (j >> 1) & 1, 2 * (j & 1)
+            p, d = self.S + 4 * (2 * qb + kb) + e, self.DP + 4 * (2 * qb + kb) + e
+            at = 9 + 43 * j // 15
+            for i in range(2):
+                put(at, x.valu, "v_fma_f32", v(p + i), v(p + i), "%[scale]", "-%%[lse%d]" % qb)
+            for i in range(2):
+                put(at + 1, x.valu, "v_exp_f32", v(p + i), v(p + i), trans=True)
+            at = self.AT_MASK + 15 * j // 8
+            for i in range(2):
+                put(at, x.valu, "v_mul_f32", v(p + i), v(p + i), v(d + i))
+            put(at + 1, x.valu, x.pack_name, v(self.DSP + 4 * qb + 2 * kb + e // 2), v(p), v(p + 1))
+        return work
+
+    AT_MASK = 55
+
+    def tile(self, stage):
+        x, work, issue = self.x, self.vector_work(), {}
+        for use, at, d, n, text in self.reads(stage):
+            issue.setdefault(at, []).append((text, d, n, use))
+        next_rows = dict(zip(range(40, 56, 3), self.to_next_rows()))
+        for m in range(96):
+            phase, qb, i = m // 32, m // 8 % 4, m % 8
+            copies = (m - 1) // 3 if m % 3 == 1 and m < 3 * self.copies else None
+            if copies is not None:
+                self.copy(copies, (stage + 3) % self.STAGES, True)
+            if m == self.AT_BARRIER:
+                x.put("s_waitcnt vmcnt(%d)" % (2 * self.copies))       # the next tile has landed ..
+                x.put("s_barrier")                 # .. both its halves, and nobody reads this one any more
+            if m == self.AT_MASK:
+                x.put("s_cmp_gt_i32 %s, %%[mlim]" % s(self.KEY))
+                x.put("s_cbranch_scc1 %s" % self.ref("MASK%d" % stage))
+                self.label("MASKED%d" % stage)
+            if phase < 2:
+                ks, kb = i // 2, i % 2
+                d, frag = (self.S, self.DP)[phase] + 4 * (2 * qb + kb), (self.KF, self.VF)[phase] + 4 * i
+                args = (v(d, 4), v(frag, 4), "%%[%s%d%d]" % ("qd"[phase], qb, ks), v(d, 4) if ks else ("0", "%%[nd%d]" % qb)[phase])
+                holds = [(v(frag, 4), (96 if phase == 0 else 32) + i)]
+            else:
+                frag = self.KT + 4 * i
+                acc = "%%[o%d%d]" % (qb, i)
+                args = (acc, v(frag, 4), v(self.DSP + 4 * qb, 4), acc)
+                holds = [(v(frag, 4), 64 + i)]
+            need = set(range(frag, frag + 4))
+            if qb == 0 and i % 2 == 0:             # one wait for two fragments
+                need |= set(range(frag, frag + 8))
+            x.wait(need)
+            x.mfma(*args, holds)
+            if copies is not None:
+                self.copy(copies, 0, False)
+            for text, d, n, use in issue.get(m, []):
+                x.lds(text, d, n, use)
+            for f in work.get(m, []):
+                f()
+            for line in next_rows.get(m, []):
+                x.put(line)
+            if m == 80:
+                x.put("s_add_u32 %s, %s, %%[keystep]" % (s(self.KEY), s(self.KEY)))
+
+    def text(self):
+        x = self.x
+        self.enter()
+        for line in sum(self.rows_left(), []):
+            x.put(line)
+        x.put("v_mov_b32 %s, 0" % v(self.ZERO))
+        for i in range(4):
+            x.put("v_mov_b32 %s, 0" % v(self.KT + i))
+        x.put("s_nop 3")
+        for i in range(32):
+            x.put("%s %%[o%d%d], %s, %s, 0" % (x.mfma_name, i // 8, i % 8, v(self.KT, 4), v(self.KT, 4)))
+        x.put("s_waitcnt vmcnt(%d)" % (2 * self.copies))
+        x.put("s_barrier")
+        self.loop(self.tile, self.first_reads)
+        for stage in range(self.STAGES):
+            self.label("MASK%d" % stage)
+            self.mask_lanes(self.CX, self.CY)
+            self.mask(self.S, v(self.ZERO), self.CX, self.CY)
+            x.put("s_branch %s" % self.ref("MASKED%d" % stage))
+        self.leave()
+        return x.lines
+
+
 def define(name, lines):
     return "#define %s \\\n" % name + " \\\n".join('  "%s\\n\\t"' % l for l in lines) + "\n"
 
@@ -416,7 +624,10 @@ def generate():
     for dtype in ("bf16", "f16"):
         for ds in (False, True):
             out.append(define("DH_DKV128_LOOP_%s%s" % (dtype.upper(), "_DS" if ds else ""), DKV(dtype, ds).text()))
+        for copies in (4, 8):
+            out.append(define("DH_DQ128_LOOP_%s_%d" % (dtype.upper(), copies), DQ(dtype, copies).text()))
     out.append(clobbers("DH_DKV128_CLOBBERS", DKV.KEEP, DKV.NEG, DKV.RSQ, DKV.CTC))
+    out.append(clobbers("DH_DQ128_CLOBBERS", DQ.KEEP, DQ.ZERO, Keys.RSC, Keys.T))
     return "".join(out)
 
 
