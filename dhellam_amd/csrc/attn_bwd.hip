@@ -762,7 +762,6 @@ int attn_bwd_f32(const void *dout, const void *q, const void *k, const void *v, 
                  int dq_accumulate, hipStream_t st);
 
 constexpr int DKV_ROWS = 64;  // key rows of a dK/dV workgroup
-constexpr int64_t ROWS_MAX_STRIDE = 1ll << 26;   // elements: 32 rows of them are less than 4 GiB
 
 // Keeping dS for the dQ product costs 2 bytes per (head, query, key) of workspace, written once and read once.
 // It pays where the recomputing dQ kernel runs its small-grid form (fewer than 256 workgroups of 128 query rows:

@@ -427,20 +427,46 @@ static int launch_attn_fwd_d128(const AttnFwdParams &p, int batch, hipStream_t s
 
 }  // namespace dh
 
+#include "attn_fwd128.h"
 #include "attn_fwd_tile.h"
 
 namespace dh {
 
+template <typename T>
+static int launch_attn_fwd128(const AttnFwdParams &p, int batch, hipStream_t st) {
+  const int nqt = (int)cdiv(p.max_sq, 256);
+  dim3 grid((unsigned)((p.causal ? (nqt + 1) / 2 : nqt) * p.hq), (unsigned)batch);
+  hipLaunchKernelGGL((attn_fwd128_kernel<T>), grid, dim3(256), 0, st, p);
+  return DH_OK;
+}
+
 struct AttnFwdRoute {
   bool hand;      // head dim 128's hand-ordered kernel
   bool big;       // 128-row query tiles
+  bool rows256;   // instead of either: head dim 128 on one wavefront a SIMD, 256-row query tiles
 };
+
+// Whether the kernel with one wavefront a SIMD is the faster one at head dim 128: its loop takes 1710 cycles for what took 2900, but its
+// 256-row tiles have to fill the chip, and short rows leave much of them empty.  Sequences of one length: their workgroups take
+// 70 % of the places in their rounds of 256.  Several lengths: two rounds of real work, four fifths of one where nothing is causal
+// (no pairs of a long and a short tile that one long sequence keeps apart).  us, before / here, 32 query heads, causal unless said:
+//   4096 (256 workgroups) 199 / 144, 8 x 1024 141 / 124, 16 x 512 106 / 99, 12 heads x 8192 (192) 294 / 215, not causal 2048 (256) 84 / 66, 4096 x
+//   2048 keys 183 / 131; not full: 2048 (128) 53 / 81, 12 heads x 5000 (120) 127 / 148; short: 27 x 300 119 / 142;
+//   documents of 1 to 3324 tokens (552) 248 / 203; 3000 + 2 x 1000 (320) 154 / 159, 1694 + 925 + 949 (270) 83 / 114; not causal, 16 heads,
+//   2786 + 479 (206) 101 / 82, 8 heads, 1022 to 223 (72) 27 / 34.
+static bool fwd_rows256(int max_sq, int hq, int batch, int64_t total_q, int causal) {
+  if (max_sq < 512) return false;
+  const int64_t bound = (int64_t)batch * max_sq, rows = total_q < bound ? total_q : bound, n = attn_wgs(max_sq, 256, hq, batch, causal);
+  if (10 * rows >= 9 * bound) return 10 * n >= 7 * 256 * ((n + 255) / 256);
+  return (int64_t)((double)n * (double)rows / (double)bound) >= (causal ? 512 : 208);
+}
 static AttnFwdRoute attn_fwd_route(int max_sq, int hq, int d, int batch, int64_t total_q, int causal) {
+  const bool r256 = d == 128 && fwd_rows256(max_sq, hq, batch, total_q, causal);
   // not causal: from 96 workgroups of 64 rows on (4 heads x 4277 87 against 93 us, 4 x 6547 129 / 144, 32 x 7813 1028 / 1158;
   // at 1000 rows and below level)
   if (d == 128 && (causal ? attn_causal_fills(max_sq, hq, batch, total_q) : attn_wgs(max_sq, 64, hq, batch, 0) >= 96))
-    return {true, attn_wgs(max_sq, 128, hq, batch, causal) >= ATTN_128ROW_MIN_WG};
-  return {false, attn_wgs(max_sq, 128, hq, batch, 0) >= (d < 128 ? 2 * 256 : 256)};
+    return {true, attn_wgs(max_sq, 128, hq, batch, causal) >= ATTN_128ROW_MIN_WG, r256};
+  return {false, attn_wgs(max_sq, 128, hq, batch, 0) >= (d < 128 ? 2 * 256 : 256), r256};
 }
 
 // All other cases: 128-row query tiles when they give every compute unit its workgroups (two at 64 and 96,
@@ -462,7 +488,7 @@ int attn_fwd_f32(const void *q, const void *k, const void *v, void *out, float *
 
 extern "C" int dh_attn_fwd_path(int batch, int max_seqlen_q, int64_t total_q, int hq, int d, int causal) {
   const dh::AttnFwdRoute r = dh::attn_fwd_route(max_seqlen_q, hq, d, batch, total_q, causal);
-  return (r.hand ? 1 : 0) | (r.big ? 2 : 0);
+  return (r.hand ? 1 : 0) | (r.big ? 2 : 0) | (r.rows256 ? 4 : 0);
 }
 
 extern "C" int dh_attn_fwd_state(const void *q, const void *k, const void *v, void *out, float *lse, int64_t *rng_state,
@@ -506,7 +532,9 @@ extern "C" int dh_attn_fwd_state(const void *q, const void *k, const void *v, vo
   p.rng_state = rng_state;
   const AttnFwdRoute r = attn_fwd_route(max_seqlen_q, hq, d, batch, total_q, causal);
   int rc;
-  if (r.hand) {
+  if (r.rows256 && k_stride <= ROWS_MAX_STRIDE && v_stride <= ROWS_MAX_STRIDE) {
+    rc = dtype == DH_BF16 ? launch_attn_fwd128<bf16_t>(p, batch, st) : launch_attn_fwd128<f16_t>(p, batch, st);
+  } else if (r.hand) {
     if (dtype == DH_BF16) rc = r.big ? launch_attn_fwd_d128<bf16_t, 4, 2, 64, DH_FWD_LAG>(p, batch, st) : launch_attn_fwd_d128<bf16_t, 2, 4, 32, DH_FWD_LAG>(p, batch, st);
     else rc = r.big ? launch_attn_fwd_d128<f16_t, 4, 2, 64, DH_FWD_LAG>(p, batch, st) : launch_attn_fwd_d128<f16_t, 2, 4, 32, DH_FWD_LAG>(p, batch, st);
   } else {

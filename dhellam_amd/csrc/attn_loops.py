@@ -100,10 +100,6 @@ class Stream:
             self.valu_at[r] = self.count
         self.trans = regs(d, "v") if trans else set()
 
-    def settled(self):
-        """Behind a wait that covers every MFMA."""
-        self.mfma_at = {}
-
 
 class DKV:
     """dK/dV: the loop over a wavefront's tiles of 32 query rows, two stages unrolled.
@@ -481,10 +477,10 @@ class Keys:
         self.x.put("v_add_u32 %s, %s, %%[vx]" % (v(cx), s(self.KEY)))
         self.x.put("v_add_u32 %s, %s, %%[vy]" % (v(cy), s(self.KEY)))
 
-    def mask(self, first, value, cx, cy):
+    def mask(self, first, value, cx, cy, blocks=(0, 1, 2, 3)):
         """The values of a tile (registers from `first`, [qb][kb][v]) past the diagonal or the last key become `value`."""
         x = self.x
-        for qb in range(4):
+        for qb in blocks:
             for kb in range(2):
                 for e in range(4):
                     r = v(first + 4 * (2 * qb + kb) + e)
@@ -610,12 +606,251 @@ class DQ(Keys):
         return x.lines
 
 
+class FWD(Keys):
+    """Forward: S^T = K Q^T, P = 2^(S c - m), O^T += V^T P^T; 64 MFMAs a tile.  The query blocks go in two groups, A (0, 1) and B (2, 3), and
+    the tile in quarters of 16 MFMAs,
+        S of A | O of B, of the tile before | S of B | O of A,
+    so that the softmax of either group has two quarters of MFMAs above it before its product is due.
+
+    m is only a reference for the exponentials: it moves (``move``, out of line) when the eight values of some lane sum to more than
+    2^8, which also is how the first tile sets it.  One branch asks that of a group, some instructions behind the comparisons (the
+    branch directly behind each block's comparison cost 70 cycles apiece).  Tiles with scores to mask run a copy of the tile's code that
+    masks a group's scores in front of its softmax.  O is a[0:127] (query block, d block); at the end it goes to LDS as 64 rows of
+    fp32, 16-byte chunks XORed with the row.
+    """
+    KEEP = 48
+    S, KF, VT, P, PP, TS, MT, MX, TY, CX, CY, NEG = 48, 80, 112, 144, 160, 176, 180, 188, 189, 190, 191, 192
+    RET, OVER, BOUND = 50, 52, 54
+    AT_BARRIER = 46
+
+    def __init__(self, dtype):
+        super().__init__(dtype, 4)
+
+    def k_read(self, i, st):
+        return "ds_read_b128 %s, %%[rk%d] offset:%d" % (v(self.KF + 4 * i, 4), i // 2, st + 16 * self.ROWB * (i % 2))
+
+    def first_reads(self):
+        for i in range(8):
+            self.x.lds(self.k_read(i, 0), self.KF + 4 * i, 4, "k")
+
+    def reads(self, stage):
+        """(MFMA behind which it is issued, destination, width, text, what)."""
+        st, nx, out = stage * self.STAGEB + self.TILEB, (stage + 1) % self.STAGES * self.STAGEB, []
+        for i in range(16):
+            t, h = i // 2, i % 2
+            d = self.VT + 4 * t + 2 * h
+            out.append((31 + i, d, 2, "ds_read_b64_tr_b16 %s, %%[ta%d] offset:%d" % (v(d, 2), t, st + 16 * self.ROWB * h), "v"))
+        for i in range(8):
+            out.append((self.AT_BARRIER + 1 + 2 * i, self.KF + 4 * i, 4, self.k_read(i, nx), "k"))
+        return out
+
+    def probs(self, qb):
+        return [self.P + 8 * (qb & 1) + i for i in range(8)]
+
+    def softmax(self, qb):
+        """P of a block, packed, the sum of a lane's eight values and whether it is too large, as a list of instructions."""
+        x, p, sc, ts, out = self.x, self.probs(qb), [self.S + 8 * qb + i for i in range(8)], v(self.TS + qb), []
+        for i in range(0, 8, 2):
+            out += [lambda i=i, k=k: x.valu("v_fma_f32", v(p[i + k]), v(sc[i + k]), "%[scale]", "-%%[m%d]" % qb) for k in range(2)]
+            if i:                                  # of the two values before
+                out.append(lambda i=i: x.valu(x.pack_name, v(self.PP + 4 * qb + i // 2 - 1), v(p[i - 2]), v(p[i - 1])))
+            out += [lambda i=i, k=k: x.valu("v_exp_f32", v(p[i + k]), v(p[i + k]), trans=True) for k in range(2)]
+            if i == 2:
+                out.append(lambda: x.valu("v_add_f32", ts, v(p[0]), v(p[1])))
+            elif i:
+                out += [lambda i=i, k=k: x.valu("v_add_f32", ts, ts, v(p[i - 2 + k])) for k in range(2)]
+        out += [lambda: x.valu("v_add_f32", ts, ts, v(p[6])),
+                lambda: x.valu(x.pack_name, v(self.PP + 4 * qb + 3), v(p[6]), v(p[7])),
+                lambda: x.valu("v_add_f32", ts, ts, v(p[7])),
+                lambda: x.put("v_cmp_lt_f32 %s, %s, %s" % ("vcc" if qb & 1 else s(self.OVER, 2), s(self.BOUND), ts))]
+        return out
+
+    def check(self, group, name):
+        x = self.x
+        x.put("s_or_b64 vcc, vcc, %s" % s(self.OVER, 2))
+        x.put("s_cbranch_vccnz %s" % self.ref("GROW%d%s" % (group, name)))
+        self.label("GROWN%d%s" % (group, name))
+        self.stubs.append((group, name))
+        for qb in (2 * group, 2 * group + 1):
+            x.valu("v_add_f32", "%%[l%d]" % qb, "%%[l%d]" % qb, v(self.TS + qb))
+
+    def move(self, qb):
+        """Out of line, called: the reference moves to the largest score of the row so far; O, l and P follow."""
+        x, sc, mx, ty = self.x, [self.S + 8 * qb + i for i in range(8)], v(self.MX), v(self.TY)
+        p = [self.MT + i for i in range(8)]
+        self.label("MOVE%d" % qb)
+        x.put("s_nop 15")
+        for i in range(8):
+            x.put("v_mul_f32 %s, %%[scale], %s" % (v(p[i]), v(sc[i])))
+        x.put("v_max3_f32 %s, %s, %s, %s" % (mx, v(p[0]), v(p[1]), v(p[2])))
+        x.put("v_max3_f32 %s, %s, %s, %s" % (mx, mx, v(p[3]), v(p[4])))
+        x.put("v_max3_f32 %s, %s, %s, %s" % (mx, mx, v(p[5]), v(p[6])))
+        x.put("v_max_f32 %s, %s, %s" % (mx, mx, v(p[7])))
+        for swap in ("v_permlane32_swap_b32", "v_permlane16_swap_b32"):
+            x.put("v_mov_b32 %s, %s" % (ty, mx))
+            x.put("s_nop 1")
+            x.put("%s %s, %s" % (swap, mx, ty))
+            x.put("s_nop 1")
+            x.put("v_max_f32 %s, %s, %s" % (mx, mx, ty))
+        x.put("v_max_f32 %s, %s, %%[m%d]" % (mx, mx, qb))
+        x.put("v_sub_f32 %s, %%[m%d], %s" % (ty, qb, mx))
+        x.put("v_exp_f32 %s, %s" % (ty, ty))
+        x.put("v_mov_b32 %%[m%d], %s" % (qb, mx))
+        x.put("s_nop 0")
+        x.put("v_mul_f32 %%[l%d], %%[l%d], %s" % (qb, qb, ty))
+        for i in range(0, 32, 8):                  # eight of the block's 32 registers at a time
+            for k in range(8):
+                x.put("v_accvgpr_read_b32 %s, a%d" % (v(p[k]), 32 * qb + i + k))
+            for k in range(8):
+                x.put("v_mul_f32 %s, %s, %s" % (v(p[k]), v(p[k]), ty))
+            for k in range(8):
+                x.put("v_accvgpr_write_b32 a%d, %s" % (32 * qb + i + k, v(p[k])))
+        for i in range(8):
+            x.put("v_fma_f32 %s, %s, %%[scale], -%%[m%d]" % (v(p[i]), v(sc[i]), qb))
+        for i in range(8):
+            x.put("v_exp_f32 %s, %s" % (v(p[i]), v(p[i])))
+        x.put("s_nop 0")
+        ts = v(self.TS + qb)
+        x.put("v_add_f32 %s, %s, %s" % (ts, v(p[0]), v(p[1])))
+        for i in range(2, 8):
+            x.put("v_add_f32 %s, %s, %s" % (ts, ts, v(p[i])))
+        for i in range(4):
+            x.put("%s %s, %s, %s" % (x.pack_name, v(self.PP + 4 * qb + i), v(p[2 * i]), v(p[2 * i + 1])))
+        x.put("s_nop 7")
+        x.put("s_setpc_b64 %s" % s(self.RET, 2))
+
+    def scores_mfma(self, group, m):
+        """MFMA m of 16: S of a group, a block after the other."""
+        qb, ks, kb = 2 * group + m // 8, m % 8 // 2, m % 2
+        d, frag = self.S + 4 * (2 * qb + kb), self.KF + 4 * (m % 8)
+        need = set(range(frag, frag + 8)) if m < 8 and m % 2 == 0 else set(range(frag, frag + 4))      # one wait for two fragments
+        self.x.wait(need)
+        self.x.mfma(v(d, 4), v(frag, 4), "%%[q%d%d]" % (qb, ks), v(d, 4) if ks else "0", [(v(frag, 4), "k")])
+
+    def out_mfma(self, group, m):
+        """MFMA m of 16: O of a group."""
+        qb, t = 2 * group + m // 8, m % 8
+        frag, acc = self.VT + 4 * t, "a[%d:%d]" % (32 * (2 * group + m // 8) + 4 * (m % 8), 32 * (2 * group + m // 8) + 4 * (m % 8) + 3)
+        self.x.wait(set(range(frag, frag + 8)) if m < 8 and m % 2 == 0 else set(range(frag, frag + 4)))
+        self.x.mfma(acc, v(frag, 4), v(self.PP + 4 * qb, 4), acc)
+
+    B_HEAD = 15                                    # MFMAs of the tile beneath which B's softmax begins; the rest of it is in the next tile
+
+    def b_softmax(self, head):
+        todo = self.softmax(2) + self.softmax(3)
+        n = (len(todo) * self.B_HEAD + 13) // (self.B_HEAD + 12)
+        return todo[:n] if head else todo[n:]
+
+    def body(self, stage, masked):
+        x, issue, work = self.x, {}, {}
+        name = "%s%d" % ("M" if masked else "T", stage)
+        for at, d, n, text, what in self.reads(stage):
+            issue.setdefault(at, []).append((text, d, n, what))
+
+        def spread(todo, first, slots):
+            for i, f in enumerate(todo):
+                work.setdefault(first + slots * i // len(todo), []).append(f)
+        spread(self.b_softmax(False), 0, 12)
+        work.setdefault(14, []).append(lambda: self.check(1, name))
+        spread(self.softmax(0) + self.softmax(1), 17, 27)
+        work.setdefault(45, []).append(lambda: self.check(0, name))
+        spread(self.b_softmax(True), 49, self.B_HEAD)
+        next_rows = dict(zip(range(18, 40, 4), self.to_next_rows()))
+        for m in range(64):
+            copy = (m - 49) // 4 if m >= 49 and (m - 49) % 4 == 0 else None
+            if copy is not None:
+                self.copy(copy, (stage + 3) % self.STAGES, True)
+            if masked and m in (16, 48):
+                x.put("s_nop 15")
+                if m == 16:
+                    self.mask_lanes(self.CX, self.CY)
+                self.mask(self.S, v(self.NEG), self.CX, self.CY, (0, 1) if m == 16 else (2, 3))
+            if m == self.AT_BARRIER:
+                x.put("s_waitcnt vmcnt(%d)" % self.copies)     # the next tile has landed ..
+                x.put("s_barrier")                 # .. all of it, and everybody has what it needs of the tile before
+            (self.scores_mfma, self.out_mfma)[m // 16 % 2]((0, 1, 1, 0)[m // 16], m % 16)
+            if copy is not None:
+                self.copy(copy, 0, False)
+            for text, d, n, what in issue.get(m, []):
+                x.lds(text, d, n, what)
+            for f in work.get(m, []):
+                f()
+            for line in next_rows.get(m, []):
+                x.put(line)
+        x.put("s_add_u32 %s, %s, %%[keystep]" % (s(self.KEY), s(self.KEY)))
+
+    def tile(self, stage):
+        x = self.x
+        x.put("s_cmp_gt_i32 %s, %%[mlim]" % s(self.KEY))
+        x.put("s_cbranch_scc1 %s" % self.ref("MASKED%d" % stage))
+        self.begin = getattr(self, "begin", None) or [set(r) for r in x.reads]
+        self.body(stage, False)
+        self.label("DONE%d" % stage)
+
+    def text(self):
+        x, self.stubs = self.x, []
+        self.enter()
+        for line in sum(self.rows_left(), []):
+            x.put(line)
+        # the group B of a tile in front of the first: no scores, no values
+        x.put("v_mov_b32 %s, 0xff800000" % v(self.NEG))
+        for i in range(16):
+            x.put("v_mov_b32 %s, %s" % (v(self.S + 16 + i), v(self.NEG)))
+        for i in range(32):
+            x.put("v_mov_b32 %s, 0" % v(self.VT + i))
+        x.put("s_mov_b32 %s, 0x43800000" % s(self.BOUND))
+        x.put("s_nop 3")
+        for i in range(32):
+            x.put("%s a[%d:%d], %s, %s, 0" % (x.mfma_name, 4 * i, 4 * i + 3, v(self.VT, 4), v(self.VT, 4)))
+        for f in self.b_softmax(True):
+            f()
+            if x.trans:
+                x.put("s_nop 0")
+        x.put("s_waitcnt vmcnt(%d)" % (2 * self.copies))
+        x.put("s_barrier")
+        self.loop(self.tile, self.first_reads)
+        end = [set(r) for r in x.reads]
+        for stage in range(self.STAGES):
+            self.label("MASKED%d" % stage)
+            x.reads = [set(r) for r in self.begin]
+            self.body(stage, True)
+            assert x.reads == end[len(end) - len(x.reads):], "the masked tile ends otherwise"
+            x.put("s_branch %s" % self.ref("DONE%d" % stage))
+        self.leave()                               # the last tile's B
+        x.reads = []
+        for f in self.b_softmax(False):
+            f()
+            if x.trans:
+                x.put("s_nop 0")
+        self.check(1, "E")
+        x.put("s_nop 3")
+        for m in range(16):
+            self.out_mfma(1, m)
+        x.put("s_nop 15")
+        x.put("s_nop 7")
+        x.put("s_barrier")                         # everyone is done with the tiles
+        for qb in range(4):
+            for t in range(8):
+                x.put("ds_write_b128 %%[wo%d], a[%d:%d] offset:%d" % (t, 32 * qb + 4 * t, 32 * qb + 4 * t + 3, 8192 * qb))
+        x.put("s_waitcnt lgkmcnt(0)")
+        x.put("s_branch %s" % self.ref("OUT"))
+        for group, name in self.stubs:
+            self.label("GROW%d%s" % (group, name))
+            for qb in (2 * group, 2 * group + 1):
+                x.put("s_call_b64 %s, %s" % (s(self.RET, 2), self.ref("MOVE%d" % qb)))
+            x.put("s_branch %s" % self.ref("GROWN%d%s" % (group, name)))
+        for qb in range(4):
+            self.move(qb)
+        self.label("OUT")
+        return x.lines
+
+
 def define(name, lines):
     return "#define %s \\\n" % name + " \\\n".join('  "%s\\n\\t"' % l for l in lines) + "\n"
 
 
-def clobbers(name, first_v, last_v, first_s, last_s):
-    names = ["v%d" % i for i in range(first_v, last_v + 1)] + ["s%d" % i for i in range(first_s, last_s + 1)] + ["vcc", "memory"]
+def clobbers(name, first_v, last_v, first_s, last_s, agprs=0):
+    names = ["a%d" % i for i in range(agprs)] + ["v%d" % i for i in range(first_v, last_v + 1)] + ["s%d" % i for i in range(first_s, last_s + 1)] + ["vcc", "memory"]
     return "#define %s %s\n" % (name, ", ".join('"%s"' % n for n in names))
 
 
@@ -626,8 +861,10 @@ def generate():
             out.append(define("DH_DKV128_LOOP_%s%s" % (dtype.upper(), "_DS" if ds else ""), DKV(dtype, ds).text()))
         for copies in (4, 8):
             out.append(define("DH_DQ128_LOOP_%s_%d" % (dtype.upper(), copies), DQ(dtype, copies).text()))
+        out.append(define("DH_FWD128_LOOP_%s" % dtype.upper(), FWD(dtype).text()))
     out.append(clobbers("DH_DKV128_CLOBBERS", DKV.KEEP, DKV.NEG, DKV.RSQ, DKV.CTC))
     out.append(clobbers("DH_DQ128_CLOBBERS", DQ.KEEP, DQ.ZERO, Keys.RSC, Keys.T))
+    out.append(clobbers("DH_FWD128_CLOBBERS", FWD.KEEP, FWD.NEG, Keys.RSC, FWD.BOUND, 128))
     return "".join(out)
 
 

@@ -12,6 +12,9 @@ static inline int64_t attn_wgs(int max_sq, int rows, int hq, int batch, int caus
   return (causal ? (t + 1) / 2 : t) * hq * batch;
 }
 
+// Largest token stride (elements) of the kernels with one wavefront a SIMD: 32 rows of it are less than 4 GiB, the reach of a copy.
+constexpr int64_t ROWS_MAX_STRIDE = 1ll << 26;
+
 // fewest workgroups of 128 query rows for which the 128-row kernels are taken
 constexpr int ATTN_128ROW_MIN_WG = 256;
 

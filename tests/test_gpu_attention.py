@@ -509,3 +509,39 @@ def test_attention_delta_is_zero_past_a_sequence(d, lens, hq, hk, causal, dtype)
         assert (delta[i, :, n:] == 0).all()
         assert ((delta[i, :, :n].t() - want[at:at + n]).abs() <= bound[at:at + n]).all()
         at += n
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("lens_q,lens_k,hq,hk,causal", [
+    ([513] * 6, [513] * 6, 32, 8, True),                       # one row past two tiles, one key past 16
+    ([600] * 4, [37, 2, 640, 1], 32, 4, False),                   # fewer tiles of keys than stages
+    ([1023, 300, 1, 77, 513, 255] * 2, [64, 1, 130, 33, 31, 95] * 2, 32, 32, False),
+])
+def test_attention_on_one_wavefront_a_simd(dtype, lens_q, lens_k, hq, hk, causal):
+    """The kernels of 256-row query tiles (forward, recomputing dQ) at the edges of their tiles."""
+    from dhellam_amd import _Clib
+    assert _fwd_path(lens_q, hq, 128, causal) & 4
+    _Clib.set_attn_bwd_ds_limit(0)
+    try:
+        _run_fwd_bwd(dtype, lens_q, lens_k, hq, hk, 128, causal, oracle_dtype=torch.float32)
+    finally:
+        _Clib.set_attn_bwd_ds_limit()
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("growth", [0.0, 12.0, -12.0])
+def test_attention_forward_when_scores_grow_along_the_keys(causal, growth):
+    """Scores that rise by many binades from key tile to key tile (the reference of the exponentials has to follow in some rows and
+    not in others), that fall, and rows of nothing but equal scores."""
+    from dhellam_amd import _Clib
+    n, hq, d, dtype = 1024, 64, 128, torch.bfloat16
+    assert _fwd_path([n, n], hq, d, causal) & 4
+    q, k, v = (randn((2 * n, h, d), dtype, 60 + i) for i, h in enumerate((hq, 8, 8)))
+    ramp = torch.linspace(0, abs(growth), n).repeat(2)
+    k = ((ramp.flip(0) if growth < 0 else ramp) + 1)[:, None, None].mul(k.float()).to(dtype)
+    q[::3] = 0
+    cu, scale = _cu([n, n]), 1.0 / math.sqrt(d)
+    res = _Clib.pymha_varlen_fwd(q.cuda(), k.cuda(), v.cuda(), cu.cuda(), cu.cuda(), n, n, 0.0, scale, causal, False, 0, False)
+    oo, lo = OA.attn_fwd(q, k, v, cu, cu, scale, causal, torch.float32)
+    assert_close(res[0], oo, dtype, "out")
+    assert_close(res[5], lo, torch.float32, "lse")
