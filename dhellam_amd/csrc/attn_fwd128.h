@@ -9,10 +9,12 @@ namespace dh {
 // of a tile, three tiles ahead; loop and meeting point are attn_loops.py's.  S^T = K Q^T has the query index on lanes, so that P^T
 // is the operand of O^T += V^T P^T as it is, and the reference m of the exponentials and the sums l are one a lane and block.
 // Whether m has to move is asked of the sum of a lane's eight values, which is needed anyway, instead of their maximum: 112
-// vector instructions and four comparisons, 24 LDS reads and 4 copies for 64 MFMAs.
-// What it measured: 1710 cycles a tile, of which the matrix pipe is busy 1024: a wavefront issues an instruction in 5 cycles, and there are
-// about 290 (barrier 85, the two branches 75).  32 query / 8 kv heads, 4096 rows x 2048 keys 155 -> 120 us (1.14 PFLOP/s), causal
-// 4096 153 -> 126, seven packed sequences of 1 to 3324 tokens 212 -> 185.
+// vector instructions and four comparisons, 24 LDS reads and 4 copies for 68 MFMAs.
+// What it measured: 1740 cycles a tile, of which the matrix pipe is busy 1088: a wavefront issues an instruction in 5 cycles, and there are
+// about 290 (barrier 85, the two branches 75).  32 query / 8 kv heads, 4096 rows x 2048 keys 155 -> 127 us (1.08 PFLOP/s), causal
+// 4096 153 -> 134, seven packed sequences of 1 to 3324 tokens 212 -> 191.  Errors against 64 bits (bf16, 4096 causal | scores three
+// times as wide): out 2.080e-3 -> 2.085e-3 | 1.77e-3 -> 1.68e-3, dq 2.440e-3 -> 2.438e-3 | 5.00e-3 -> 4.81e-3, lse 5.8e-8 -> 5.5e-8.  Without the
+// sums of rounded P and with the first tile as the reference 2.12e-3 | 1.89e-3, and 5 % faster.
 // O goes through LDS (the loop writes it there) and out in whole rows.  Causal: row tiles i and n - 1 - i.
 template <typename T>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) attn_fwd128_kernel(const AttnFwdParams p) {
@@ -100,12 +102,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
     const int vx = causal ? 4 * g - r - wrow0 : -(1 << 30), vy = 4 * g - sk;      // key - row and key - keys, but for the tile's first key
     // tiles from this key on have something to mask
     const int mlim = causal && wrow0 - BN + 1 < sk - BN ? wrow0 - BN + 1 : sk - BN;
-    float m[4] = {-1e30f, -1e30f, -1e30f, -1e30f}, l[4] = {0.f, 0.f, 0.f, 0.f};
+    float m[4] = {-1e30f, -1e30f, -1e30f, -1e30f}, l[4] = {0.f, 0.f, 0.f, 0.f}, n[4];
 #define DH_ROW(x, X, qb) [x##qb##0] "a"(X[qb][0]), [x##qb##1] "a"(X[qb][1]), [x##qb##2] "a"(X[qb][2]), [x##qb##3] "a"(X[qb][3])
 #define DH_LOOP(TEXT)                                                                                                                \
   asm volatile(TEXT                                                                                                                 \
                : [m0] "+v"(m[0]), [m1] "+v"(m[1]), [m2] "+v"(m[2]), [m3] "+v"(m[3]), [l0] "+v"(l[0]), [l1] "+v"(l[1]),                \
-                 [l2] "+v"(l[2]), [l3] "+v"(l[3]), [rem] "+s"(rem)                                                                   \
+                 [l2] "+v"(l[2]), [l3] "+v"(l[3]), [n0] "=&v"(n[0]), [n1] "=&v"(n[1]), [n2] "=&v"(n[2]), [n3] "=&v"(n[3]),            \
+                 [rem] "+s"(rem)                                                                                                     \
                : DH_ROW(q, Q, 0), DH_ROW(q, Q, 1), DH_ROW(q, Q, 2), DH_ROW(q, Q, 3), [rk0] "v"(rk[0]), [rk1] "v"(rk[1]),              \
                  [rk2] "v"(rk[2]), [rk3] "v"(rk[3]), [ta0] "v"(ta[0]), [ta1] "v"(ta[1]), [ta2] "v"(ta[2]), [ta3] "v"(ta[3]),          \
                  [ta4] "v"(ta[4]), [ta5] "v"(ta[5]), [ta6] "v"(ta[6]), [ta7] "v"(ta[7]), [cl0] "v"(cl[0]), [cl1] "v"(cl[1]),          \
@@ -125,7 +128,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
       lt += __shfl_xor(lt, 32, 64);
       const int row = wrow0 + 16 * qb + r;
       if (g == 0) {
-        sInv[w][16 * qb + r] = lt > 0.f ? 1.0f / lt : 0.f;
+        sInv[w][16 * qb + r] = n[qb] > 0.f ? 1.0f / n[qb] : 0.f;
         if (row < sq) p.lse[((int64_t)b * p.hq + h) * p.max_sq + row] = lt > 0.f ? m[qb] * 0.6931471805599453f + logf(lt) : -INFINITY;
       }
     }

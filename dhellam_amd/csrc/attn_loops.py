@@ -100,6 +100,11 @@ class Stream:
             self.valu_at[r] = self.count
         self.trans = regs(d, "v") if trans else set()
 
+    def settle(self):
+        """Waits for every MFMA."""
+        self.put("s_nop 15")
+        self.mfma_at = {}
+
 
 class DKV:
     """dK/dV: the loop over a wavefront's tiles of 32 query rows, two stages unrolled.
@@ -612,19 +617,22 @@ class FWD(Keys):
         S of A | O of B, of the tile before | S of B | O of A,
     so that the softmax of either group has two quarters of MFMAs above it before its product is due.
 
-    m is only a reference for the exponentials: it moves (``move``, out of line) when the eight values of some lane sum to more than
-    2^8, which also is how the first tile sets it.  One branch asks that of a group, some instructions behind the comparisons (the
+    m is only a reference for the exponentials: the first 64 keys set it ahead of the loop, so that the largest of few scores is 1
+    exactly, and it moves (``move``, out of line) when the eight values of some lane sum to more than 2^8.  One branch asks that of a group, some instructions behind the comparisons (the
     branch directly behind each block's comparison cost 70 cycles apiece).  Tiles with scores to mask run a copy of the tile's code that
-    masks a group's scores in front of its softmax.  O is a[0:127] (query block, d block); at the end it goes to LDS as 64 rows of
+    masks a group's scores in front of its softmax.  O is divided by the sums of P as it was rounded, which one MFMA with ones a block
+    brings, in a[128:143]: where a few scores dominate a row their rounding then cancels.  O is a[0:127] (query block, d block); at the end it goes to LDS as 64 rows of
     fp32, 16-byte chunks XORed with the row.
     """
     KEEP = 48
     S, KF, VT, P, PP, TS, MT, MX, TY, CX, CY, NEG = 48, 80, 112, 144, 160, 176, 180, 188, 189, 190, 191, 192
+    ONES, SUMS = 194, 128
     RET, OVER, BOUND = 50, 52, 54
     AT_BARRIER = 46
 
     def __init__(self, dtype):
         super().__init__(dtype, 4)
+        self.ones = {"bf16": "0x3f803f80", "f16": "0x3c003c00"}[dtype]
 
     def k_read(self, i, st):
         return "ds_read_b128 %s, %%[rk%d] offset:%d" % (v(self.KF + 4 * i, 4), i // 2, st + 16 * self.ROWB * (i % 2))
@@ -686,25 +694,18 @@ class FWD(Keys):
         x.put("v_max3_f32 %s, %s, %s, %s" % (mx, mx, v(p[3]), v(p[4])))
         x.put("v_max3_f32 %s, %s, %s, %s" % (mx, mx, v(p[5]), v(p[6])))
         x.put("v_max_f32 %s, %s, %s" % (mx, mx, v(p[7])))
-        for swap in ("v_permlane32_swap_b32", "v_permlane16_swap_b32"):
-            x.put("v_mov_b32 %s, %s" % (ty, mx))
-            x.put("s_nop 1")
-            x.put("%s %s, %s" % (swap, mx, ty))
-            x.put("s_nop 1")
-            x.put("v_max_f32 %s, %s, %s" % (mx, mx, ty))
+        self.row_max(mx, ty)
         x.put("v_max_f32 %s, %s, %%[m%d]" % (mx, mx, qb))
         x.put("v_sub_f32 %s, %%[m%d], %s" % (ty, qb, mx))
         x.put("v_exp_f32 %s, %s" % (ty, ty))
         x.put("v_mov_b32 %%[m%d], %s" % (qb, mx))
         x.put("s_nop 0")
         x.put("v_mul_f32 %%[l%d], %%[l%d], %s" % (qb, qb, ty))
-        for i in range(0, 32, 8):                  # eight of the block's 32 registers at a time
-            for k in range(8):
-                x.put("v_accvgpr_read_b32 %s, a%d" % (v(p[k]), 32 * qb + i + k))
-            for k in range(8):
-                x.put("v_mul_f32 %s, %s, %s" % (v(p[k]), v(p[k]), ty))
-            for k in range(8):
-                x.put("v_accvgpr_write_b32 a%d, %s" % (32 * qb + i + k, v(p[k])))
+        acc = [32 * qb + i for i in range(32)] + [self.SUMS + 4 * qb + i for i in range(4)]
+        for i in range(0, 36, 8):                  # eight of the block's registers at a time
+            for f in ("v_accvgpr_read_b32 {p}, a{a}", "v_mul_f32 {p}, {p}, {y}", "v_accvgpr_write_b32 a{a}, {p}"):
+                for k, n in enumerate(acc[i:i + 8]):
+                    x.put(f.format(p=v(p[k]), a=n, y=ty))
         for i in range(8):
             x.put("v_fma_f32 %s, %s, %%[scale], -%%[m%d]" % (v(p[i]), v(sc[i]), qb))
         for i in range(8):
@@ -718,6 +719,46 @@ class FWD(Keys):
             x.put("%s %s, %s, %s" % (x.pack_name, v(self.PP + 4 * qb + i), v(p[2 * i]), v(p[2 * i + 1])))
         x.put("s_nop 7")
         x.put("s_setpc_b64 %s" % s(self.RET, 2))
+
+    def row_max(self, mx, ty):
+        """The largest of the four lanes 16 apart."""
+        x = self.x
+        for swap in ("v_permlane32_swap_b32", "v_permlane16_swap_b32"):
+            x.put("v_mov_b32 %s, %s" % (ty, mx))
+            x.put("s_nop 1")
+            x.put("%s %s, %s" % (swap, mx, ty))
+            x.put("s_nop 1")
+            x.put("v_max_f32 %s, %s, %s" % (mx, mx, ty))
+
+    def reference(self):
+        """m from the scores of the first two tiles (where they are masked, or there are none, it stays very low)."""
+        x = self.x
+        for st in range(2):
+            for i in range(8):
+                x.lds(self.k_read(i, st * self.STAGEB), self.KF + 4 * i, 4, "k")
+            for m in range(32):
+                self.scores_mfma(m // 16, m % 16)
+            x.settle()
+            x.put("s_cmp_gt_i32 %s, %%[mlim]" % s(self.KEY))
+            x.put("s_cbranch_scc1 %s" % self.ref("FIRST%d" % st))
+            self.label("FIRSTED%d" % st)
+            x.put("s_add_u32 %s, %s, %%[keystep]" % (s(self.KEY), s(self.KEY)))
+            for qb in range(4):
+                p, mx = self.probs(qb), v(self.TS + qb)
+                for i in range(8):
+                    x.put("v_mul_f32 %s, %%[scale], %s" % (v(p[i]), v(self.S + 8 * qb + i)))
+                rest = p if st else p[1:]
+                first = mx if st else v(p[0])
+                x.put("v_max3_f32 %s, %s, %s, %s" % (mx, first, v(rest[0]), v(rest[1])))
+                for i in range(2, len(rest) - 1, 2):
+                    x.put("v_max3_f32 %s, %s, %s, %s" % (mx, mx, v(rest[i]), v(rest[i + 1])))
+                if len(rest) % 2:
+                    x.put("v_max_f32 %s, %s, %s" % (mx, mx, v(rest[-1])))
+        for st in range(2):
+            x.put("s_sub_u32 %s, %s, %%[keystep]" % (s(self.KEY), s(self.KEY)))
+        for qb in range(4):
+            self.row_max(v(self.TS + qb), v(self.TY))
+            x.put("v_max_f32 %%[m%d], %%[m%d], %s" % (qb, qb, v(self.TS + qb)))
 
     def scores_mfma(self, group, m):
         """MFMA m of 16: S of a group, a block after the other."""
@@ -733,6 +774,9 @@ class FWD(Keys):
         frag, acc = self.VT + 4 * t, "a[%d:%d]" % (32 * (2 * group + m // 8) + 4 * (m % 8), 32 * (2 * group + m // 8) + 4 * (m % 8) + 3)
         self.x.wait(set(range(frag, frag + 8)) if m < 8 and m % 2 == 0 else set(range(frag, frag + 4)))
         self.x.mfma(acc, v(frag, 4), v(self.PP + 4 * qb, 4), acc)
+        if t == 7:
+            acc = "a[%d:%d]" % (self.SUMS + 4 * qb, self.SUMS + 4 * qb + 3)
+            self.x.mfma(acc, v(self.ONES, 4), v(self.PP + 4 * qb, 4), acc)
 
     B_HEAD = 15                                    # MFMAs of the tile beneath which B's softmax begins; the rest of it is in the next tile
 
@@ -792,22 +836,25 @@ class FWD(Keys):
         self.enter()
         for line in sum(self.rows_left(), []):
             x.put(line)
-        # the group B of a tile in front of the first: no scores, no values
         x.put("v_mov_b32 %s, 0xff800000" % v(self.NEG))
+        x.put("s_waitcnt vmcnt(%d)" % self.copies)
+        x.put("s_barrier")                         # the first two tiles are there
+        self.reference()
+        # the group B of a tile in front of the first: no scores, no values
         for i in range(16):
             x.put("v_mov_b32 %s, %s" % (v(self.S + 16 + i), v(self.NEG)))
         for i in range(32):
             x.put("v_mov_b32 %s, 0" % v(self.VT + i))
+        for i in range(4):
+            x.put("v_mov_b32 %s, %s" % (v(self.ONES + i), self.ones))
         x.put("s_mov_b32 %s, 0x43800000" % s(self.BOUND))
         x.put("s_nop 3")
-        for i in range(32):
+        for i in range(36):
             x.put("%s a[%d:%d], %s, %s, 0" % (x.mfma_name, 4 * i, 4 * i + 3, v(self.VT, 4), v(self.VT, 4)))
         for f in self.b_softmax(True):
             f()
             if x.trans:
                 x.put("s_nop 0")
-        x.put("s_waitcnt vmcnt(%d)" % (2 * self.copies))
-        x.put("s_barrier")
         self.loop(self.tile, self.first_reads)
         end = [set(r) for r in x.reads]
         for stage in range(self.STAGES):
@@ -830,10 +877,17 @@ class FWD(Keys):
         x.put("s_nop 7")
         x.put("s_barrier")                         # everyone is done with the tiles
         for qb in range(4):
+            x.put("v_accvgpr_read_b32 %%[n%d], a%d" % (qb, self.SUMS + 4 * qb))
+        for qb in range(4):
             for t in range(8):
                 x.put("ds_write_b128 %%[wo%d], a[%d:%d] offset:%d" % (t, 32 * qb + 4 * t, 32 * qb + 4 * t + 3, 8192 * qb))
         x.put("s_waitcnt lgkmcnt(0)")
         x.put("s_branch %s" % self.ref("OUT"))
+        for st in range(2):
+            self.label("FIRST%d" % st)
+            self.mask_lanes(self.CX, self.CY)
+            self.mask(self.S, v(self.NEG), self.CX, self.CY)
+            x.put("s_branch %s" % self.ref("FIRSTED%d" % st))
         for group, name in self.stubs:
             self.label("GROW%d%s" % (group, name))
             for qb in (2 * group, 2 * group + 1):
@@ -864,7 +918,7 @@ def generate():
         out.append(define("DH_FWD128_LOOP_%s" % dtype.upper(), FWD(dtype).text()))
     out.append(clobbers("DH_DKV128_CLOBBERS", DKV.KEEP, DKV.NEG, DKV.RSQ, DKV.CTC))
     out.append(clobbers("DH_DQ128_CLOBBERS", DQ.KEEP, DQ.ZERO, Keys.RSC, Keys.T))
-    out.append(clobbers("DH_FWD128_CLOBBERS", FWD.KEEP, FWD.NEG, Keys.RSC, FWD.BOUND, 128))
+    out.append(clobbers("DH_FWD128_CLOBBERS", FWD.KEEP, FWD.ONES + 3, Keys.RSC, FWD.BOUND, FWD.SUMS + 16))
     return "".join(out)
 
 
