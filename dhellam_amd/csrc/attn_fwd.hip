@@ -432,41 +432,57 @@ static int launch_attn_fwd_d128(const AttnFwdParams &p, int batch, hipStream_t s
 
 namespace dh {
 
-template <typename T>
+template <typename T, int RG>
 static int launch_attn_fwd128(const AttnFwdParams &p, int batch, hipStream_t st) {
-  const int nqt = (int)cdiv(p.max_sq, 256);
+  const int nqt = (int)cdiv(p.max_sq, 64 * RG);
   dim3 grid((unsigned)((p.causal ? (nqt + 1) / 2 : nqt) * p.hq), (unsigned)batch);
-  hipLaunchKernelGGL((attn_fwd128_kernel<T>), grid, dim3(256), 0, st, p);
+  hipLaunchKernelGGL((attn_fwd128_kernel<T, RG>), grid, dim3(256), 0, st, p);
   return DH_OK;
 }
 
 struct AttnFwdRoute {
   bool hand;      // head dim 128's hand-ordered kernel
   bool big;       // 128-row query tiles
-  bool rows256;   // instead of either: head dim 128 on one wavefront a SIMD, 256-row query tiles
+  int rows;       // instead of either, where not 0: head dim 128 on one wavefront a SIMD, query tiles of 256 or 128 rows
 };
 
-// Whether the kernel with one wavefront a SIMD is the faster one at head dim 128: its loop takes 1710 cycles for what took 2900, but its
-// 256-row tiles have to fill the chip, and short rows leave much of them empty.  Sequences of one length: their workgroups take
-// 70 % of the places in their rounds of 256.  Several lengths: two rounds of real work, four fifths of one where nothing is causal
-// (no pairs of a long and a short tile that one long sequence keeps apart).  us, before / here, 32 query heads, causal unless said:
-//   4096 (256 workgroups) 199 / 144, 8 x 1024 141 / 124, 16 x 512 106 / 99, 12 heads x 8192 (192) 294 / 215, not causal 2048 (256) 84 / 66, 4096 x
-//   2048 keys 183 / 131; not full: 2048 (128) 53 / 81, 12 heads x 5000 (120) 127 / 148; short: 27 x 300 119 / 142;
-//   documents of 1 to 3324 tokens (552) 248 / 203; 3000 + 2 x 1000 (320) 154 / 159, 1694 + 925 + 949 (270) 83 / 114; not causal, 16 heads,
-//   2786 + 479 (206) 101 / 82, 8 heads, 1022 to 223 (72) 27 / 34.
-static bool fwd_rows256(int max_sq, int hq, int batch, int64_t total_q, int causal) {
-  if (max_sq < 512) return false;
-  const int64_t bound = (int64_t)batch * max_sq, rows = total_q < bound ? total_q : bound, n = attn_wgs(max_sq, 256, hq, batch, causal);
-  if (10 * rows >= 9 * bound) return 10 * n >= 7 * 256 * ((n + 255) / 256);
-  return (int64_t)((double)n * (double)rows / (double)bound) >= (causal ? 512 : 208);
+// Query rows of a tile where the kernel with one wavefront a SIMD is the faster one at head dim 128 (else 0).  Its loop takes 1740 cycles
+// for what took 2900, but its tiles are larger, so it depends on what of the chip they leave empty: places in the last round
+// of 256 workgroups, rows past the end, an odd tile without its pair.  us, before / here, 32 query heads, causal unless said:
+//   256 rows, one length, 70 % of the places: 4096 (256 workgroups) 199 / 144, 8 x 1024 141 / 124, 16 x 512 106 / 99, 12 heads x 8192 (192) 294 /
+//     215, not causal 2048 (256) 84 / 66, 4096 x 2048 keys 183 / 131, x 64 keys 40 / 32; less: 2048 (128) 53 / 81, 12 heads x 5000 (120) 127 /
+//     148, 27 x 300 119 / 142, 128 heads x 700 (three tiles, 256) 44 / 54.
+//   256 rows, several lengths: two rounds of real work, four fifths of one where nothing is causal (no pairs of a long and a short
+//     tile that one long sequence keeps apart): documents of 1 to 3324 tokens (552) 248 / 203; 3000 + 2 x 1000 (320) 154 / 159, 1694 + 925 +
+//     949 (270) 83 / 114; not causal, 16 heads, 2786 + 479 (206) 101 / 82, 8 heads, 1022 to 223 (72) 27 / 34.
+//   128 rows (two splits of the keys) where those are too few.  Causal: long rows and full rounds, 16 heads x 4096 (256) 91 / 84, 12
+//     heads x 5000 (240) 131 / 92, 8 x 8192 157 / 138, but 32 x 2048 (256) 54 / 55, 16 x 3000 (192) 62 / 64.  Not causal: against 64-row tiles
+//     where those are more than a round, 32 x 600 (160) 28 / 20, 600 x 100 keys 18 / 14, 16 x 1100 (144) 37 / 26, but 8 x 2048 (128) 29 / 36, 512 x 8192
+//     keys (128) 98 / 111; against 128-row tiles from 1024 keys on, 16 x 2048 (256) 44 / 42, but x 512 keys 18 / 19, x 64 10 / 13; several
+//     lengths 2786 + 479 (412) 106 / 93, 8 heads, 1022 to 223 (144) 27 / 30.
+static int fwd_rows(int max_sq, int max_sk, int hq, int batch, int64_t total_q, int causal) {
+  if (max_sq < 512) return 0;
+  const int64_t bound = (int64_t)batch * max_sq, rows = total_q < bound ? total_q : bound;
+  const int64_t n = attn_wgs(max_sq, 256, hq, batch, causal), n2 = attn_wgs(max_sq, 128, hq, batch, causal);
+  auto fill = [](int64_t w) { return (double)w / (256.0 * (double)((w + 255) / 256)); };
+  if (10 * rows >= 9 * bound) {
+    const int t = (max_sq + 255) / 256;
+    const double used = (causal ? (double)t / (2 * ((t + 1) / 2)) : 1.0) * (double)max_sq / (256.0 * t);
+    if (fill(n) * used >= 0.7) return 256;
+    if (causal) return max_sq >= 2560 && max_sk >= 1024 && fill(n2) >= 0.85 ? 128 : 0;
+    return n2 > 128 && (n2 < ATTN_128ROW_MIN_WG || max_sk >= 1024) ? 128 : 0;
+  }
+  const double share = (double)rows / (double)bound;
+  if ((double)n * share >= (causal ? 512 : 208)) return 256;
+  return !causal && max_sk >= 1024 && (double)n2 * share >= 384 ? 128 : 0;
 }
-static AttnFwdRoute attn_fwd_route(int max_sq, int hq, int d, int batch, int64_t total_q, int causal) {
-  const bool r256 = d == 128 && fwd_rows256(max_sq, hq, batch, total_q, causal);
+static AttnFwdRoute attn_fwd_route(int max_sq, int max_sk, int hq, int d, int batch, int64_t total_q, int causal) {
+  const int r1 = d == 128 ? fwd_rows(max_sq, max_sk, hq, batch, total_q, causal) : 0;
   // not causal: from 96 workgroups of 64 rows on (4 heads x 4277 87 against 93 us, 4 x 6547 129 / 144, 32 x 7813 1028 / 1158;
   // at 1000 rows and below level)
   if (d == 128 && (causal ? attn_causal_fills(max_sq, hq, batch, total_q) : attn_wgs(max_sq, 64, hq, batch, 0) >= 96))
-    return {true, attn_wgs(max_sq, 128, hq, batch, causal) >= ATTN_128ROW_MIN_WG, r256};
-  return {false, attn_wgs(max_sq, 128, hq, batch, 0) >= (d < 128 ? 2 * 256 : 256), r256};
+    return {true, attn_wgs(max_sq, 128, hq, batch, causal) >= ATTN_128ROW_MIN_WG, r1};
+  return {false, attn_wgs(max_sq, 128, hq, batch, 0) >= (d < 128 ? 2 * 256 : 256), r1};
 }
 
 // All other cases: 128-row query tiles when they give every compute unit its workgroups (two at 64 and 96,
@@ -487,8 +503,8 @@ int attn_fwd_f32(const void *q, const void *k, const void *v, void *out, float *
 }  // namespace dh
 
 extern "C" int dh_attn_fwd_path(int batch, int max_seqlen_q, int64_t total_q, int hq, int d, int causal) {
-  const dh::AttnFwdRoute r = dh::attn_fwd_route(max_seqlen_q, hq, d, batch, total_q, causal);
-  return (r.hand ? 1 : 0) | (r.big ? 2 : 0) | (r.rows256 ? 4 : 0);
+  const dh::AttnFwdRoute r = dh::attn_fwd_route(max_seqlen_q, max_seqlen_q, hq, d, batch, total_q, causal);
+  return (r.hand ? 1 : 0) | (r.big ? 2 : 0) | (r.rows ? 4 : 0);
 }
 
 extern "C" int dh_attn_fwd_state(const void *q, const void *k, const void *v, void *out, float *lse, int64_t *rng_state,
@@ -530,10 +546,11 @@ extern "C" int dh_attn_fwd_state(const void *q, const void *k, const void *v, vo
   p.causal = causal;
   p.q_shift = q_shift; p.k_shift = k_shift;
   p.rng_state = rng_state;
-  const AttnFwdRoute r = attn_fwd_route(max_seqlen_q, hq, d, batch, total_q, causal);
+  const AttnFwdRoute r = attn_fwd_route(max_seqlen_q, max_seqlen_k, hq, d, batch, total_q, causal);
   int rc;
-  if (r.rows256 && k_stride <= ROWS_MAX_STRIDE && v_stride <= ROWS_MAX_STRIDE) {
-    rc = dtype == DH_BF16 ? launch_attn_fwd128<bf16_t>(p, batch, st) : launch_attn_fwd128<f16_t>(p, batch, st);
+  if (r.rows && k_stride <= ROWS_MAX_STRIDE && v_stride <= ROWS_MAX_STRIDE) {
+    if (dtype == DH_BF16) rc = r.rows == 256 ? launch_attn_fwd128<bf16_t, 4>(p, batch, st) : launch_attn_fwd128<bf16_t, 2>(p, batch, st);
+    else rc = r.rows == 256 ? launch_attn_fwd128<f16_t, 4>(p, batch, st) : launch_attn_fwd128<f16_t, 2>(p, batch, st);
   } else if (r.hand) {
     if (dtype == DH_BF16) rc = r.big ? launch_attn_fwd_d128<bf16_t, 4, 2, 64, DH_FWD_LAG>(p, batch, st) : launch_attn_fwd_d128<bf16_t, 2, 4, 32, DH_FWD_LAG>(p, batch, st);
     else rc = r.big ? launch_attn_fwd_d128<f16_t, 4, 2, 64, DH_FWD_LAG>(p, batch, st) : launch_attn_fwd_d128<f16_t, 2, 4, 32, DH_FWD_LAG>(p, batch, st);

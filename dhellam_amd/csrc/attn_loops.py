@@ -630,8 +630,8 @@ class FWD(Keys):
     RET, OVER, BOUND = 50, 52, 54
     AT_BARRIER = 46
 
-    def __init__(self, dtype):
-        super().__init__(dtype, 4)
+    def __init__(self, dtype, copies):
+        super().__init__(dtype, copies)
         self.ones = {"bf16": "0x3f803f80", "f16": "0x3c003c00"}[dtype]
 
     def k_read(self, i, st):
@@ -801,7 +801,8 @@ class FWD(Keys):
         spread(self.b_softmax(True), 49, self.B_HEAD)
         next_rows = dict(zip(range(18, 40, 4), self.to_next_rows()))
         for m in range(64):
-            copy = (m - 49) // 4 if m >= 49 and (m - 49) % 4 == 0 else None
+            gap = 16 // self.copies
+            copy = (m - 49) // gap if m >= 49 and (m - 49) % gap == 0 and (m - 49) // gap < self.copies else None
             if copy is not None:
                 self.copy(copy, (stage + 3) % self.STAGES, True)
             if masked and m in (16, 48):
@@ -915,7 +916,8 @@ def generate():
             out.append(define("DH_DKV128_LOOP_%s%s" % (dtype.upper(), "_DS" if ds else ""), DKV(dtype, ds).text()))
         for copies in (4, 8):
             out.append(define("DH_DQ128_LOOP_%s_%d" % (dtype.upper(), copies), DQ(dtype, copies).text()))
-        out.append(define("DH_FWD128_LOOP_%s" % dtype.upper(), FWD(dtype).text()))
+        for copies in (4, 8):
+            out.append(define("DH_FWD128_LOOP_%s_%d" % (dtype.upper(), copies), FWD(dtype, copies).text()))
     out.append(clobbers("DH_DKV128_CLOBBERS", DKV.KEEP, DKV.NEG, DKV.RSQ, DKV.CTC))
     out.append(clobbers("DH_DQ128_CLOBBERS", DQ.KEEP, DQ.ZERO, Keys.RSC, Keys.T))
     out.append(clobbers("DH_FWD128_CLOBBERS", FWD.KEEP, FWD.ONES + 3, Keys.RSC, FWD.BOUND, FWD.SUMS + 16))

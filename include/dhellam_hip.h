@@ -192,7 +192,8 @@ int dh_attn_fwd_state(const void *q, const void *k, const void *v, void *out,
 
 /* Which kernels a 16-bit call of these sizes runs (what the entries themselves
  * go by).  Forward: bit 0 = head dim 128's hand-ordered kernel, bit 1 = query
- * tiles of 128 rows (else 64).  Backward: bit 0 = head dim 128's hand-ordered
+ * tiles of 128 rows (else 64), bit 2 = head dim 128's kernel of one wavefront a
+ * SIMD instead of either (with at least as many keys as query rows).  Backward: bit 0 = head dim 128's hand-ordered
  * dK/dV kernel, bit 1 = dQ from kept dS, else bit 2 = the hand-ordered
  * recomputing dQ kernel and bit 3 = its query tiles have 128 rows (all
  * clear: the other kernels, which for small calls run in one launch, as

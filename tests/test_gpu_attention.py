@@ -513,12 +513,14 @@ def test_attention_delta_is_zero_past_a_sequence(d, lens, hq, hk, causal, dtype)
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("lens_q,lens_k,hq,hk,causal", [
-    ([513] * 6, [513] * 6, 32, 8, True),                       # one row past two tiles, one key past 16
-    ([600] * 4, [37, 2, 640, 1], 32, 4, False),                   # fewer tiles of keys than stages
+    ([1001] * 4, [1001] * 4, 32, 8, True),                     # rows and keys that end inside a tile
+    ([767] * 4, [37, 2, 640, 1], 32, 4, False),                   # fewer tiles of keys than stages
     ([1023, 300, 1, 77, 513, 255] * 2, [64, 1, 130, 33, 31, 95] * 2, 32, 32, False),
+    ([600], [333], 32, 8, False),                              # 128-row tiles, two splits, an odd number of key tiles
+    ([2689], [2689], 20, 4, True),
 ])
 def test_attention_on_one_wavefront_a_simd(dtype, lens_q, lens_k, hq, hk, causal):
-    """The kernels of 256-row query tiles (forward, recomputing dQ) at the edges of their tiles."""
+    """The kernels of 256- and 128-row query tiles (forward, recomputing dQ) at the edges of their tiles."""
     from dhellam_amd import _Clib
     assert _fwd_path(lens_q, hq, 128, causal) & 4
     _Clib.set_attn_bwd_ds_limit(0)
