@@ -1032,7 +1032,7 @@ static int attn_bwd_entry(const void *dout, const void *q, const void *k, const 
   size_t dsb = ds_bytes(batch, max_seqlen_q, total_k, hq, d, dtype, causal);
   if (dsb > 0 && base_bytes + align256(dsb) > workspace_bytes) dsb = 0;
   const AttnBwdRoute route = attn_bwd_route(batch, max_seqlen_q, max_seqlen_k, total_q, total_k, hq, hk, d, causal, dsb > 0,
-                                            std::max({q_stride, k_stride, v_stride, do_stride}) > ROWS_MAX_STRIDE);
+                                            std::max({q_stride, k_stride, v_stride, do_stride, o_stride}) > ROWS_MAX_STRIDE / 2);
   uint8_t *ds_ws = (uint8_t *)(((uintptr_t)workspace + 255) & ~(uintptr_t)255) + (base_bytes - 256);
   const bool delta_in_dq = dtype != DH_F32 && !route.keep_ds;
   if (max_seqlen_q > 0 && !delta_in_dq) {

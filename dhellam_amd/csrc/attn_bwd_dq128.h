@@ -16,8 +16,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
   constexpr int D = 128, BM = 64 * RG, BN = 32, SPLIT = 4 / RG, STAGES = 4;
   constexpr int COPIES = 16 / RG, CROWS = 4 * COPIES;  // 1 KB copies of a wavefront a tile, and their rows
   constexpr uint32_t ROWB = 2 * D, TILEB = BN * ROWB, STAGEB = 2 * TILEB, STREAMB = STAGES * STAGEB;
-  static_assert(SPLIT == 1 || SPLIT * STREAMB == 4 * 32768, "exchange area");
-  __shared__ __attribute__((aligned(1024))) char sAll[SPLIT * STREAMB];
+  // the tiles; behind them (and, with two splits, in the stages that are filled last) 16 KB a wavefront for its own rows
+  constexpr uint32_t OWN = 64 * ROWB, LDS = SPLIT * STREAMB + (RG == 4 ? 4 : 2) * OWN;
+  static_assert(OWN == STAGEB && (SPLIT == 1 || SPLIT * STREAMB == 4 * 32768), "own rows, exchange area");
+  __shared__ __attribute__((aligned(1024))) char sAll[LDS];
 
   const int b = __builtin_amdgcn_readfirstlane(seq_by_length(p.cu_q, gridDim.y, blockIdx.y));
   // the query heads of one kv head read the same K / V rows: keep a kv head on one XCD's L2
@@ -81,22 +83,35 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
     floatx4 nd[4];
     float lse[4], del[4];
     {
-      int4s O[4][4];
+      // rows of Q, dO and O through LDS, a KB a copy (gathered from memory, 16 rows of 64 bytes a load, the three took 18000 to 25000
+      // cycles of a tile's rows)
+      const uint32_t own = lds0 + (RG == 4 ? STREAMB + (uint32_t)w * OWN : w < 2 ? (uint32_t)w * STREAMB + 3 * STAGEB : 2 * STREAMB + (uint32_t)(w - 2) * OWN);
+      typedef __attribute__((address_space(3))) const int4s *lds_i4;
+      const int rows = sq - wrow0 < 64 ? sq - wrow0 : 64;
+      auto fetch = [&](const void *base, int64_t stride, int4s (&f)[4][4]) {
+        const uint32_t rowb = (uint32_t)stride * 2u;
+        uint32_t off[4];
+        rows_lanes(off, lane, rowb);
+        const int4s rs = rows_rsrc(reinterpret_cast<const T *>(base) + (int64_t)(q0 + wrow0) * stride + (int64_t)h * D, rows > 0 ? (uint32_t)(rows - 1) * rowb + ROWB : 0u);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) copy_1k(off[i & 3], rs, (uint32_t)(i >> 2) * 16u * rowb, own + 1024u * i);
+        dma_wait_all();
+#pragma unroll
+        for (int qb = 0; qb < 4; ++qb)
+#pragma unroll
+          for (int ks = 0; ks < 4; ++ks) f[qb][ks] = *(lds_i4)(own + (uint32_t)(qb * 4096 + r * 256) + ((uint32_t)((4 * ks + g) ^ swz16(r)) << 4));
+#pragma unroll
+        for (int qb = 0; qb < 4; ++qb) loaded_here(f[qb]);      // read, before anything else is copied there
+      };
 #pragma unroll
       for (int qb = 0; qb < 4; ++qb) {
-        const int row = wrow0 + 16 * qb + r, row_ld = row < sq ? row : sq - 1;
-        const T *op = reinterpret_cast<const T *>(p.out) + (int64_t)(q0 + row_ld) * p.o_stride + (int64_t)h * D + 8 * g;
-        const T *qp = reinterpret_cast<const T *>(p.q) + (int64_t)(q0 + row_ld) * p.q_stride + (int64_t)h * D + 8 * g;
-        const T *dp = reinterpret_cast<const T *>(p.dout) + (int64_t)(q0 + row_ld) * p.do_stride + (int64_t)h * D + 8 * g;
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-          dO[qb][ks] = *reinterpret_cast<const int4s *>(dp + 32 * ks);
-          O[qb][ks] = *reinterpret_cast<const int4s *>(op + 32 * ks);
-          Q[qb][ks] = *reinterpret_cast<const int4s *>(qp + 32 * ks);
-        }
-        lse[qb] = p.lse[((int64_t)b * p.hq + h) * p.lse_pitch + row_ld];
+        const int row = wrow0 + 16 * qb + r;
+        lse[qb] = p.lse[((int64_t)b * p.hq + h) * p.lse_pitch + (row < sq ? row : sq - 1)];
       }
-      __builtin_amdgcn_sched_barrier(0);              // all loads are out before the first of them is waited for
+      int4s O[4][4];
+      fetch(p.q, p.q_stride, Q);
+      fetch(p.dout, p.do_stride, dO);
+      fetch(p.out, p.o_stride, O);
 #pragma unroll
       for (int qb = 0; qb < 4; ++qb) {
         del[qb] = 0.f;
