@@ -617,7 +617,7 @@ class FWD(Keys):
         S of A | O of B, of the tile before | S of B | O of A,
     so that the softmax of either group has two quarters of MFMAs above it before its product is due.
 
-    m is only a reference for the exponentials: the first 64 keys set it ahead of the loop, so that the largest of few scores is 1
+    m is only a reference for the exponentials: the first 64 keys set it ahead of the loop (``reference``), so that the largest of few scores is 1
     exactly, and it moves (``move``, out of line) when the eight values of some lane sum to more than 2^8.  One branch asks that of a group, some instructions behind the comparisons (the
     branch directly behind each block's comparison cost 70 cycles apiece).  Tiles with scores to mask run a copy of the tile's code that
     masks a group's scores in front of its softmax.  O is divided by the sums of P as it was rounded, which one MFMA with ones a block
@@ -731,18 +731,28 @@ class FWD(Keys):
             x.put("v_max_f32 %s, %s, %s" % (mx, mx, ty))
 
     def reference(self):
-        """m from the scores of the first two tiles (where they are masked, or there are none, it stays very low)."""
-        x = self.x
+        """m from the scores of the first 64 keys, whichever split has them (where they are masked, or there are none, it stays very
+        low): a row's reference, by which its P is rounded, is then the same with and without splits."""
+        x, split = self.x, self.copies == 8
+        if split:
+            x.put("s_mov_b32 %s, 0" % s(self.KEY))
+            x.put("s_lshl_b32 %s, %%[key], 11" % s(self.T))      # 32 keys on is the next stream's tile
+            for ks in range(4):
+                x.put("v_subrev_u32 %s, %s, %%[rk%d]" % (v(self.VT + ks), s(self.T), ks))
         for st in range(2):
+            if split and st:
+                for ks in range(4):
+                    x.put("v_add_u32 %s, 0x%x, %s" % (v(self.VT + ks), self.STAGES * self.STAGEB, v(self.VT + ks)))
             for i in range(8):
-                x.lds(self.k_read(i, st * self.STAGEB), self.KF + 4 * i, 4, "k")
+                text = self.k_read(i, 0 if split else st * self.STAGEB)
+                x.lds(re.sub(r"%\[rk(\d)\]", lambda a: v(self.VT + int(a[1])), text) if split else text, self.KF + 4 * i, 4, "k")
             for m in range(32):
                 self.scores_mfma(m // 16, m % 16)
             x.settle()
             x.put("s_cmp_gt_i32 %s, %%[mlim]" % s(self.KEY))
             x.put("s_cbranch_scc1 %s" % self.ref("FIRST%d" % st))
             self.label("FIRSTED%d" % st)
-            x.put("s_add_u32 %s, %s, %%[keystep]" % (s(self.KEY), s(self.KEY)))
+            x.put("s_add_u32 %s, %s, 32" % (s(self.KEY), s(self.KEY)))
             for qb in range(4):
                 p, mx = self.probs(qb), v(self.TS + qb)
                 for i in range(8):
@@ -754,8 +764,7 @@ class FWD(Keys):
                     x.put("v_max3_f32 %s, %s, %s, %s" % (mx, mx, v(rest[i]), v(rest[i + 1])))
                 if len(rest) % 2:
                     x.put("v_max_f32 %s, %s, %s" % (mx, mx, v(rest[-1])))
-        for st in range(2):
-            x.put("s_sub_u32 %s, %s, %%[keystep]" % (s(self.KEY), s(self.KEY)))
+        x.put("s_mov_b32 %s, %%[key]" % s(self.KEY))
         for qb in range(4):
             self.row_max(v(self.TS + qb), v(self.TY))
             x.put("v_max_f32 %%[m%d], %%[m%d], %s" % (qb, qb, v(self.TS + qb)))
