@@ -33,6 +33,7 @@ SIGNATURES = {
     "dh_comm_proxy_stop": (_i32, [_vp, _vp]),
     "dh_comm_proxy_log": (_i32, [_vp, _i32, _i64, _vp, _vp, _vp]),
     "dh_gemm": (_i32, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _i32, _i32, _i32, _i32, _i32, _vp, _sz, _vp]),
+    "dh_gemm_f32_path": (_i32, [_i64, _i64, _i64, _i32, _i32]),
     "dh_gemm_tt": (_i32, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _i32, _i32, _i32, _vp, _sz, _vp]),
     "dh_stream_create_cu_mask": (_i32, [_vp, _i32, _vp]),
     "dh_stream_destroy": (_i32, [_vp]),

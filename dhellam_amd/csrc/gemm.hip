@@ -1,6 +1,5 @@
 // Dense GEMM entry point: the reference's cuBLASLt call (csrc/operators/gemm.cu:3-170) made with hipBLASLt.
-// Host code only: plain dense products are library work on this path; the hand-written matrix kernels of
-// this library are the attention and grouped-GEMM ones.
+// Host code only: plain dense products are library work on this path, but for the fp32 ones that gemm_f32.hip is faster at.
 //
 // Convention of the reference, kept as is: A, B and D are row-major arrays handed to a column-major
 // library, so with
@@ -17,6 +16,7 @@
 
 #include "common.h"
 #include "dhellam_hip.h"
+#include "gemm_f32.h"
 
 namespace {
 
@@ -115,6 +115,10 @@ static int gemm_entry(const void *a, const void *b, void *d, int64_t a_rows, int
   int dev = 0;
   DH_HIP(hipGetDevice(&dev));
   DH_CHECK(dev >= 0 && dev < 64, "device %d out of range", dev);
+  if (dtype == DH_F32) {
+    const dh::GemmF32 g{(const float *)b, (const float *)a, (float *)d, n, m, k, transb != 0, transa == 0, accumulate != 0};
+    if (dh::gemm_f32_pays(g)) return dh::launch_gemm_f32(g, stream);
+  }
   Plan pl;
   hipblasLtHandle_t h;
   {
@@ -146,6 +150,10 @@ extern "C" int dh_gemm(const void *a, const void *b, void *d, int64_t a_rows, in
   DH_CHECK(!(transa && transb), "TT layout not allowed");
   return gemm_entry(a, b, d, a_rows, a_cols, b_rows, b_cols, transa, transb, accumulate, dtype, out_dtype, workspace,
                     workspace_bytes, stream);
+}
+
+extern "C" int dh_gemm_f32_path(int64_t m, int64_t n, int64_t k, int transa, int transb) {
+  return dh::gemm_f32_pays(dh::GemmF32{nullptr, nullptr, nullptr, n, m, k, transb != 0, transa == 0, false});
 }
 
 // The layout dh_gemm refuses: D [n, m] = B^T @ A^T for A [m, k] and B [k, n], i.e. the weight-gradient product

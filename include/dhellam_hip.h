@@ -501,6 +501,10 @@ int dh_gemm(const void *a, const void *b, void *d, int64_t a_rows, int64_t a_col
             int transa, int transb, int accumulate, int dtype, int out_dtype, void *workspace,
             size_t workspace_bytes, void *stream);
 
+/* Whether an fp32 product D [n, m] of 16-byte aligned operands runs this library's
+ * own kernel (1) or hipBLASLt's (0); what dh_gemm itself goes by. */
+int dh_gemm_f32_path(int64_t m, int64_t n, int64_t k, int transa, int transb);
+
 /* The one layout dh_gemm refuses (as the reference does, "TT layout not allowed", csrc/operators/gemm.cu:3-170):
  * D [n, m] = B^T @ A^T for A [m, k] and B [k, n], both row-major.  It is the weight-gradient product dW = dY^T X
  * with X handed over transposed (A = X^T [K, T]) and dY [T, N] as it is: the cheaper of the two operands to

@@ -104,6 +104,17 @@ def test_lanes_of_the_routing(tokens, experts, k, lanes):
     assert _lib.load().dh_moe_route_lanes(tokens, experts, k) == lanes
 
 
+@pytest.mark.parametrize("rows,cols,k,form,own", [
+    (1024, 5632, 1024, "TN", 1), (1024, 2816, 1024, "TN", 1), (777, 2816, 1024, "TN", 0), (1024, 1536, 1024, "TN", 0), (1024, 4000, 2048, "TN", 0),
+    (1024, 16032, 1024, "TN", 0), (1024, 2816, 1000, "TN", 0), (1000, 5568, 256, "NN", 1), (1024, 2816, 1023, "NN", 0), (1024, 2818, 1024, "NN", 0),
+    (5632, 1024, 1024, "NT", 1), (5632, 1024, 1001, "NT", 1), (1024, 1024, 1024, "NT", 0), (512, 512, 64, "NT", 1), (4, 4, 1, "NT", 1),
+    (514, 512, 64, "NT", 0), (512, 514, 64, "NT", 0), (512, 512, 193, "NT", 0), (4352, 768, 227, "NT", 0), (1 << 21, 8, 64, "NT", 0)])
+def test_fp32_products_go_where_they_were_measured_the_faster(rows, cols, k, form, own):
+    """D [rows, cols]; what the copies cannot take (lengths that are no multiples of 16 bytes) is the library's."""
+    from dhellam_amd import _lib
+    assert _lib.load().dh_gemm_f32_path(cols, rows, k, form[0] == "T", form[1] == "T") == own
+
+
 @pytest.fixture(scope="module")
 def loops():
     import importlib.util

@@ -395,6 +395,39 @@ def test_dense_gemm_layouts(dtype, t, n, k):
     assert_close(y5, ref_y, dtype, "strided weight")
 
 
+@pytest.mark.parametrize("rows,cols,k,form", [
+    (600, 4484, 32, "TN"), (1001, 3004, 96, "TN"), (1024, 2816, 1024, "TN"),                # tiles that end inside rows and columns; 1, 3 and 32 slices
+    (600, 4484, 64, "NN"), (1024, 2816, 256, "NN"),
+    (4, 4, 1, "NT"), (68, 132, 33, "NT"), (512, 704, 64, "NT"), (4, 6144, 192, "NT"), (5500, 1028, 257, "NT"), (2816, 1024, 1536, "NT")])
+def test_fp32_products_of_the_own_kernel(rows, cols, k, form):
+    """Against fp64, beside garbage: nothing past the operands is read into a result, nothing past D is written.  A chain of k sums of
+    terms of one size is off by about sqrt(k) / 2 roundings of 2^-24 of the largest of them; four times that is asked."""
+    from dhellam_amd import _Clib, _lib
+    transa, transb = form[0] == "T", form[1] == "T"
+    assert _lib.load().dh_gemm_f32_path(cols, rows, k, transa, transb)
+    f32, pad = torch.float32, 64
+
+    def held(n, m, seed):
+        """[n, m] with NaNs behind it."""
+        flat = torch.full((n * m + pad,), float("nan"), device="cuda")
+        flat[:n * m] = randn((n * m,), f32, seed).cuda()
+        return flat[:n * m].view(n, m), flat
+
+    x, _ = held(*((k, rows) if transb else (rows, k)), 1)
+    y, _ = held(*((cols, k) if transa else (k, cols)), 2)
+    ref = (x.t() if transb else x).double() @ (y.t() if transa else y).double()
+    bound = 4 * 0.5 * max(k, 4) ** 0.5 * 2.0 ** -24
+    for accumulate in (False, True):
+        d, flat = held(rows, cols, 3)
+        want = ref + d.double() if accumulate else ref
+        _Clib.dense_gemm(y, x, d, transa, transb, accumulate)
+        assert ((d.double() - want).norm() / want.norm()).item() <= bound
+        assert flat[rows * cols:].isnan().all()
+        again, _ = held(rows, cols, 3)
+        _Clib.dense_gemm(y, x, again, transa, transb, accumulate)
+        assert torch.equal(d, again)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("t,n,k", [(256, 384, 512), (4096, 1280, 1024), (100, 72, 40)])
 def test_dgrad_against_resident_transpose(dtype, t, n, k):
