@@ -885,7 +885,12 @@ static AttnBwdRoute attn_bwd_route(int batch, int max_sq, int max_sk, int64_t to
   const bool fills = d <= 128 && dq_tile_fills(max_sq, hq, batch);
   r.both = both.pays && (d == 128 || !fills);
   r.big_dq = r.hand_dq ? big : fills && !r.both;
-  r.dq_rows = !(r.hand_dq && big) ? 0 : dq_wgs(256, max_sq, hq, batch, causal, total_q) >= 208 ? 256 : dq_wgs(128, max_sq, hq, batch, causal, total_q) >= 208 ? 128 : 0;
+  const bool ragged = !causal && 10 * total_q < 9 * (int64_t)batch * max_sq;
+  r.dq_rows = 0;
+  if (r.hand_dq && big && (!ragged || attn_long_rows(total_q, batch))) {
+    if (dq_wgs(256, max_sq, hq, batch, causal, total_q) >= 208 && (!ragged || attn_ragged_fills(hq, batch, total_q))) r.dq_rows = 256;
+    else if (dq_wgs(128, max_sq, hq, batch, causal, total_q) >= 208) r.dq_rows = 128;
+  }
   r.hsplit = r.both ? both.hsplit : bwd_hsplit(max_sk, batch, hq, hk, d == 128 && causal);
   return r;
 }

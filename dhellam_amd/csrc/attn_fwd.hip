@@ -472,8 +472,9 @@ static int fwd_rows(int max_sq, int max_sk, int hq, int batch, int64_t total_q, 
     if (causal) return max_sq >= 2560 && max_sk >= 1024 && fill(n2) >= 0.85 ? 128 : 0;
     return n2 > 128 && (n2 < ATTN_128ROW_MIN_WG || max_sk >= 1024) ? 128 : 0;
   }
+  if (!causal && !attn_long_rows(rows, batch)) return 0;
   const double share = (double)rows / (double)bound;
-  if ((double)n * share >= (causal ? 512 : 208)) return 256;
+  if ((double)n * share >= (causal ? 512 : 208) && (causal || attn_ragged_fills(hq, batch, rows))) return 256;
   return !causal && max_sk >= 1024 && (double)n2 * share >= 384 ? 128 : 0;
 }
 static AttnFwdRoute attn_fwd_route(int max_sq, int max_sk, int hq, int d, int batch, int64_t total_q, int causal) {

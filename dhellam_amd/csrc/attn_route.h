@@ -12,6 +12,17 @@ static inline int64_t attn_wgs(int max_sq, int rows, int hq, int batch, int caus
   return (causal ? (t + 1) / 2 : t) * hq * batch;
 }
 
+// Calls of several lengths that are not causal, where the kernels of one wavefront a SIMD pay: their tiles start and end in as many cycles as 10
+// to 14 tiles of keys take, so the sequences are 350 rows long on average, and 256-row tiles, of which half a one lies past each sequence's end,
+// fill 70 % of their rounds of 256 workgroups.  us, whole calls, eight wavefronts / here: 32 heads, 12 sequences of 54 to 782 rows (average 340)
+// 344 / 390, 16 x 10 to 448 (129) 99.5 / 104, 16 heads 778 to 2 (268 workgroups by this count, 288 in fact) 155 / 159; but 32 x 84 to
+// 624 (352) 236 / 226, 32 x 169 to 755 (446) 324 / 283, 32 / 8 x 300 to 1029 (604) 545 / 464, 16 x 84 to 2620 (1280) 863 / 775.
+static inline bool attn_long_rows(int64_t total_q, int batch) { return total_q >= 350ll * batch; }
+static inline bool attn_ragged_fills(int hq, int batch, int64_t total_q) {
+  const double wgs = ((double)total_q / 256 + 0.5 * batch) * hq;
+  return wgs >= 0.7 * 256 * (double)(((int64_t)wgs + 255) / 256);
+}
+
 // Largest token stride (elements) of the kernels with one wavefront a SIMD: 32 rows of it are less than 4 GiB, the reach of a copy.
 constexpr int64_t ROWS_MAX_STRIDE = 1ll << 26;
 
