@@ -86,22 +86,23 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
     }
     const uint32_t ldr = wbase + LD + 16 * (uint32_t)g;
 
-    // K tile: 16 rows a wavefront (zeros past the end; those columns of dK and dV are not stored, nor are V's, which repeat the last row)
+    // K and V tile: 16 rows of each a wavefront (zeros past the end; those columns of dK and dV are not stored).  V waits in the
+    // second stages for being read as fragments: gathered from memory, 16 rows of 64 bytes a load in every wavefront, it cost 1 % of a long
+    // backward and 3 % of a batch of short ones (whole calls, seven documents 710 -> 705 us, 16 heads, eight sequences of 12 to 748 rows 92 -> 90).
     {
       const int row = j0 + 16 * w, rows = sk - row < 16 ? sk - row : 16;
+      const uint32_t v_rowb = (uint32_t)p.v_stride * 2u;
       const int4s rsk = rows_rsrc(reinterpret_cast<const T *>(p.k) + (int64_t)(k0 + row) * p.k_stride + (int64_t)hkv * D,
                                   rows > 0 ? (uint32_t)(rows - 1) * k_rowb + ROWB : 0u);
+      const int4s rsv = rows_rsrc(reinterpret_cast<const T *>(p.v) + (int64_t)(k0 + row) * p.v_stride + (int64_t)hkv * D,
+                                  rows > 0 ? (uint32_t)(rows - 1) * v_rowb + ROWB : 0u);
+      uint32_t cv[4];
+      rows_lanes(cv, lane, v_rowb);
 #pragma unroll
-      for (uint32_t x = 0; x < 4; ++x) copy_1k(ck[x], rsk, 0u, lds0 + KT + (uint32_t)w * 16 * ROWB + 1024u * x);
-    }
-    int4s V[4][4];
-#pragma unroll
-    for (int kb = 0; kb < 4; ++kb) {
-      int j = j0 + 16 * kb + r;
-      j = j < sk ? j : sk - 1;
-      const T *vp = reinterpret_cast<const T *>(p.v) + (int64_t)(k0 + j) * p.v_stride + (int64_t)hkv * D + 8 * g;
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks) V[kb][ks] = *reinterpret_cast<const int4s *>(vp + 32 * ks);
+      for (uint32_t x = 0; x < 4; ++x) {
+        copy_1k(cv[x], rsv, 0u, wbase + SLOTB + 1024u * x);
+        copy_1k(ck[x], rsk, 0u, lds0 + KT + (uint32_t)w * 16 * ROWB + 1024u * x);
+      }
     }
     const int i_begin = causal ? j0 : 0;
     const int ntq = i_begin < sq ? (sq - i_begin + BM - 1) / BM : 0;
@@ -129,6 +130,16 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
         copy_1k(cd[i & 3], rsd, i < 4 ? 0u : d16, wbase + QTB + 1024u * i);
       }
       copy_256(c_ld, rows_rsrc(lp, rem > 0 ? ldbytes : 0u), wbase + LD);
+    }
+    int4s V[4][4];
+    {
+      typedef __attribute__((address_space(3))) const int4s *lds_i4;
+      asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) V[kb][ks] = *(lds_i4)(rk[ks] - KT + (uint32_t)kb * WAVEB + SLOTB);
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");      // (the loop copies to the second stages)
     }
     const int vx = causal ? r - 4 * g : -(1 << 20);   // key - row of a score, but for what the loop adds
     floatx4 dV[4][8], dK[4][8];                       // key block, d block
