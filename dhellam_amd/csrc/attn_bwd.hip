@@ -1070,7 +1070,7 @@ static int attn_bwd_entry(const void *dout, const void *q, const void *k, const 
   p.q_stride = q_stride; p.k_stride = k_stride; p.v_stride = v_stride; p.do_stride = do_stride;
   p.dq_stride = dq_stride; p.dk_stride = dk_stride; p.dv_stride = dv_stride;
   p.scale = softmax_scale;
-  p.scale_log2 = softmax_scale * 1.4426950408889634f;
+  p.scale_log2 = attn_scale_log2(softmax_scale);
   p.causal = causal;
   p.q_shift = q_shift; p.k_shift = k_shift; p.lse_pitch = lse_pitch;
   p.dq_accumulate = dq_accumulate ? 1 : 0;

@@ -543,13 +543,14 @@ extern "C" int dh_attn_fwd_state(const void *q, const void *k, const void *v, vo
   p.max_sq = max_seqlen_q; p.hq = hq; p.hk = hk;
   p.q_stride = q_stride; p.k_stride = k_stride; p.v_stride = v_stride; p.o_stride = o_stride;
   p.scale = softmax_scale;
-  p.scale_log2 = softmax_scale * 1.4426950408889634f;
+  p.scale_log2 = attn_scale_log2(softmax_scale);
   p.causal = causal;
   p.q_shift = q_shift; p.k_shift = k_shift;
   p.rng_state = rng_state;
   const AttnFwdRoute r = attn_fwd_route(max_seqlen_q, max_seqlen_k, hq, d, batch, total_q, causal);
   int rc;
-  if (r.rows && k_stride <= ROWS_MAX_STRIDE && v_stride <= ROWS_MAX_STRIDE) {
+  // (one wavefront a SIMD: every call has scores of -inf ahead of the scale, which must not turn their sign)
+  if (r.rows && p.scale_log2 > 0.f && k_stride <= ROWS_MAX_STRIDE && v_stride <= ROWS_MAX_STRIDE) {
     if (dtype == DH_BF16) rc = r.rows == 256 ? launch_attn_fwd128<bf16_t, 4>(p, batch, st) : launch_attn_fwd128<bf16_t, 2>(p, batch, st);
     else rc = r.rows == 256 ? launch_attn_fwd128<f16_t, 4>(p, batch, st) : launch_attn_fwd128<f16_t, 2>(p, batch, st);
   } else if (r.hand) {

@@ -2,9 +2,14 @@
 // workgroup of 512 threads per compute unit, causal ones all of one length) or the compiler-scheduled ones that run the
 // other head dims (smaller workgroups, shorter start and end).  Host code, shared by forward and backward.
 #pragma once
+#include <float.h>
 #include <stdint.h>
 
 namespace dh {
+
+// The scale of scores in exp2 units.  Masked scores are -inf ahead of the scale, so that 0 times them would be none: the smallest normal
+// number takes its place, which leaves finite scores where 0 puts them.
+static inline float attn_scale_log2(float scale) { return scale == 0.f ? FLT_MIN : scale * 1.4426950408889634f; }
 
 // Workgroups of a hand-ordered kernel with query tiles of `rows`: one per tile, causal ones take two.
 static inline int64_t attn_wgs(int max_sq, int rows, int hq, int batch, int causal) {

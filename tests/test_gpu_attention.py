@@ -547,3 +547,33 @@ def test_attention_forward_when_scores_grow_along_the_keys(causal, growth):
     oo, lo = OA.attn_fwd(q, k, v, cu, cu, scale, causal, torch.float32)
     assert_close(res[0], oo, dtype, "out")
     assert_close(res[5], lo, torch.float32, "lse")
+
+
+def _bwd(do, q, k, v, out, lse, cq, ck, mq, mk, scale, causal):
+    from dhellam_amd import _Clib
+    return _Clib.pymha_varlen_bwd(do, q, k, v, out, lse, cq, ck, mq, mk, 0.0, scale, causal, None, True, 0, False,
+                                  torch.cuda.current_stream().cuda_stream)[:3]
+
+
+def _draw(dtype, lens_q, lens_k, hq, hk, seed):
+    tq, tk = sum(lens_q), sum(lens_k)
+    return [randn((t, h, 128), dtype, seed + i).cuda() for i, (t, h) in enumerate(((tq, hq), (tk, hk), (tk, hk), (tq, hq)))]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n,m,hq,causal", [(2048, 256, 32, False), (1100, 352, 32, False), (512, 96, 8, False), (4096, 4096, 32, True), (2689, 2689, 40, True)])
+def test_attention_with_a_scale_of_zero(dtype, n, m, hq, causal):
+    """All scores equal: out and dV are means over the keys that a row sees, dQ and dK nothing.  (A mean of rounded values is off by
+    half a unit of the last place at most, and so is a sum of products with weights that are rounded once.)"""
+    from dhellam_amd import _Clib
+    q, k, v, do = _draw(dtype, [n], [m], hq, 8, 80)
+    cq, ck = _cu([n]).cuda(), _cu([m]).cuda()
+    res = _Clib.pymha_varlen_fwd(q, k, v, cq, ck, n, m, 0.0, 0.0, causal, False, 0, False)
+    keys = torch.arange(1, n + 1, device="cuda").double() if causal else torch.full((n,), float(m), device="cuda", dtype=torch.float64)
+    mean = (v.double().cumsum(0) if causal else v.double().sum(0, keepdim=True)) / keys[:, None, None]
+    assert_close(res[0], mean.repeat_interleave(hq // 8, 1).cpu(), dtype, "out")
+    assert_close(res[5], keys.log().expand(1, hq, -1).cpu(), torch.float32, "lse")
+    dq, dk, dv = _bwd(do, q, k, v, res[0], res[5], cq, ck, n, m, 0.0, causal)
+    assert (dq == 0).all() and (dk == 0).all()
+    part = (do.double() / keys[:, None, None]).view(n, 8, hq // 8, 128).sum(2)
+    assert_close(dv, (part.flip(0).cumsum(0).flip(0) if causal else part.sum(0).expand(m, -1, -1)).cpu(), dtype, "dv")
