@@ -108,6 +108,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
     const int vx = causal ? 4 * g - r - wrow0 : -(1 << 30), vy = 4 * g - sk;      // key - row and key - keys, but for the tile's first key
     // tiles from this key on have something to mask
     const int mlim = causal && wrow0 - BN + 1 < sk - BN ? wrow0 - BN + 1 : sk - BN;
+    const int alim = causal ? wrow0 + 31 : 1 << 30;   // ... and past this key lie behind the first 32 rows
     float m[4] = {-1e30f, -1e30f, -1e30f, -1e30f}, l[4] = {0.f, 0.f, 0.f, 0.f}, n[4];
 #define DH_ROW(x, X, qb) [x##qb##0] "a"(X[qb][0]), [x##qb##1] "a"(X[qb][1]), [x##qb##2] "a"(X[qb][2]), [x##qb##3] "a"(X[qb][3])
 #define DH_LOOP(TEXT)                                                                                                                \
@@ -121,7 +122,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
                  [cl2] "v"(cl[2]), [cl3] "v"(cl[3]), [wo0] "v"(wo[0]), [wo1] "v"(wo[1]), [wo2] "v"(wo[2]), [wo3] "v"(wo[3]),          \
                  [wo4] "v"(wo[4]), [wo5] "v"(wo[5]), [wo6] "v"(wo[6]), [wo7] "v"(wo[7]), [vx] "v"(vx), [vy] "v"(vy),                  \
                  [scale] "s"(p.scale_log2), [cp] "s"(cp), [cstep] "s"(cstep), [left] "s"(left), [key] "s"(sp * BN),                   \
-                 [keystep] "s"(SPLIT * BN), [crowb] "s"(c_rowb), [c16] "s"(c16), [cdst] "s"(cdst), [mlim] "s"(mlim)                   \
+                 [keystep] "s"(SPLIT * BN), [crowb] "s"(c_rowb), [c16] "s"(c16), [cdst] "s"(cdst), [mlim] "s"(mlim), [alim] "s"(alim)                  \
                : DH_FWD128_CLOBBERS)
     if constexpr (__is_same(T, bf16_t)) {
       if constexpr (COPIES == 4) DH_LOOP(DH_FWD128_LOOP_BF16_4);

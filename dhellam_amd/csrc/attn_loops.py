@@ -48,6 +48,15 @@ class Stream:
         self.valu_at, self.count = {}, 0
         self.holds = {}                # what the last LDS read into a register brought
         self.trans = set()
+        self.pad = False               # out of line: waits where it would refuse (MFMAs are left out there)
+
+    def state(self):
+        """The account at this point, for a piece of code that is entered from here (``resume``)."""
+        return [set(r) for r in self.reads], dict(self.mfma_at), self.mfmas, dict(self.valu_at), self.count, dict(self.holds)
+
+    def resume(self, state):
+        reads, mfma_at, self.mfmas, valu_at, self.count, holds = state
+        self.reads, self.mfma_at, self.valu_at, self.holds, self.trans = [set(r) for r in reads], dict(mfma_at), dict(valu_at), dict(holds), set()
 
     def put(self, text):
         self.lines.append(text)
@@ -82,6 +91,8 @@ class Stream:
             for r in regs(operand, "v"):
                 assert self.holds.get(r) == what, ("another read came in between", r, what, self.holds.get(r))
         self.fresh(used | regs(d, "v"))
+        while self.pad and any(self.count - self.valu_at.get(r, -99) < 3 for r in used):
+            self.put("s_nop 0")
         for r in used:
             assert self.count - self.valu_at.get(r, -99) >= 3, ("MFMA too soon behind", r, self.lines[-3:])
         self.put("%s %s, %s, %s, %s" % (self.mfma_name, d, x, y, c))
@@ -92,7 +103,11 @@ class Stream:
     def valu(self, op, d, *src, trans=False):
         used = set().union(*[regs(x, "v") for x in src])
         self.fresh(used | regs(d, "v"))
+        if self.pad and self.trans & used:
+            self.put("s_nop 0")
         assert not (self.trans & used), ("behind a transcendental", op, d, src)
+        if self.pad and any(self.mfmas - self.mfma_at.get(r, -99) < 2 for r in used | regs(d, "v")):
+            self.settle()
         for r in used | regs(d, "v"):
             assert self.mfmas - self.mfma_at.get(r, -99) >= 2, ("too soon behind the MFMA of", r, self.lines[-3:])
         self.put("%s %s" % (op, ", ".join((d,) + src)))
@@ -627,7 +642,7 @@ class FWD(Keys):
     KEEP = 48
     S, KF, VT, P, PP, TS, MT, MX, TY, CX, CY, NEG = 48, 80, 112, 144, 160, 176, 180, 188, 189, 190, 191, 192
     ONES, SUMS = 194, 128
-    RET, OVER, BOUND = 50, 52, 54
+    RET, OVER, BOUND, BACK = 50, 52, 54, 56
     AT_BARRIER = 46
 
     def __init__(self, dtype, copies):
@@ -794,9 +809,10 @@ class FWD(Keys):
         n = (len(todo) * self.B_HEAD + 13) // (self.B_HEAD + 12)
         return todo[:n] if head else todo[n:]
 
-    def body(self, stage, masked):
+    def body(self, stage, masked, without_a=False):
+        """The code of a tile; where it lies behind the rows of group A their product is left out."""
         x, issue, work = self.x, {}, {}
-        name = "%s%d" % ("M" if masked else "T", stage)
+        name = "%s%d" % ("L" if without_a else "M" if masked else "T", stage)
         for at, d, n, text, what in self.reads(stage):
             issue.setdefault(at, []).append((text, d, n, what))
 
@@ -815,14 +831,17 @@ class FWD(Keys):
             if copy is not None:
                 self.copy(copy, (stage + 3) % self.STAGES, True)
             if masked and m in (16, 48):
-                x.put("s_nop 15")
+                x.settle()
                 if m == 16:
                     self.mask_lanes(self.CX, self.CY)
                 self.mask(self.S, v(self.NEG), self.CX, self.CY, (0, 1) if m == 16 else (2, 3))
             if m == self.AT_BARRIER:
                 x.put("s_waitcnt vmcnt(%d)" % self.copies)     # the next tile has landed ..
                 x.put("s_barrier")                 # .. all of it, and everybody has what it needs of the tile before
-            (self.scores_mfma, self.out_mfma)[m // 16 % 2]((0, 1, 1, 0)[m // 16], m % 16)
+            if m == 48 and without_a:
+                x.wait(set(range(self.VT, self.VT + 32)))
+            if m < 48 or not without_a:
+                (self.scores_mfma, self.out_mfma)[m // 16 % 2]((0, 1, 1, 0)[m // 16], m % 16)
             if copy is not None:
                 self.copy(copy, 0, False)
             for text, d, n, what in issue.get(m, []):
@@ -833,16 +852,42 @@ class FWD(Keys):
                 x.put(line)
         x.put("s_add_u32 %s, %s, %%[keystep]" % (s(self.KEY), s(self.KEY)))
 
+    def last_b(self, name):
+        """The product of the last tile's group B."""
+        x = self.x
+        x.resume(self.begin[0])
+        x.reads = []
+        for f in self.b_softmax(False):
+            f()
+            if x.trans:
+                x.put("s_nop 0")
+        self.check(1, name)
+        x.put("s_nop 3")
+        for m in range(16):
+            self.out_mfma(1, m)
+
+    def idle(self, stage):
+        """A tile behind all rows of the wavefront: its share of the copies, and the others' meeting point."""
+        x = self.x
+        for line in sum(self.to_next_rows(), []):
+            x.put(line)
+        x.put("s_waitcnt vmcnt(%d)" % self.copies)
+        x.put("s_barrier")
+        for i in range(self.copies):
+            self.copy(i, (stage + 3) % self.STAGES, True)
+            x.put("s_nop 0")
+            self.copy(i, 0, False)
+
     def tile(self, stage):
         x = self.x
         x.put("s_cmp_gt_i32 %s, %%[mlim]" % s(self.KEY))
         x.put("s_cbranch_scc1 %s" % self.ref("MASKED%d" % stage))
-        self.begin = getattr(self, "begin", None) or [set(r) for r in x.reads]
+        self.begin[stage] = x.state()
         self.body(stage, False)
         self.label("DONE%d" % stage)
 
     def text(self):
-        x, self.stubs = self.x, []
+        x, self.stubs, self.begin = self.x, [], {}
         self.enter()
         for line in sum(self.rows_left(), []):
             x.put(line)
@@ -869,20 +914,41 @@ class FWD(Keys):
         end = [set(r) for r in x.reads]
         for stage in range(self.STAGES):
             self.label("MASKED%d" % stage)
-            x.reads = [set(r) for r in self.begin]
-            self.body(stage, True)
-            assert x.reads == end[len(end) - len(x.reads):], "the masked tile ends otherwise"
-            x.put("s_branch %s" % self.ref("DONE%d" % stage))
-        self.leave()                               # the last tile's B
-        x.reads = []
-        for f in self.b_softmax(False):
-            f()
-            if x.trans:
-                x.put("s_nop 0")
-        self.check(1, "E")
-        x.put("s_nop 3")
-        for m in range(16):
-            self.out_mfma(1, m)
+            x.put("s_cmp_gt_i32 %s, %%[alim]" % s(self.KEY))
+            x.put("s_cbranch_scc1 %s" % self.ref("LATE%d" % stage))
+            for without_a in (False, True):
+                if without_a:
+                    self.label("LATE%d" % stage)
+                    x.put("s_add_u32 %s, %%[alim], 32" % s(self.T))
+                    x.put("s_cmp_gt_i32 %s, %s" % (s(self.KEY), s(self.T)))
+                    x.put("s_cbranch_scc1 %s" % self.ref("IDLE%d" % stage))
+                x.resume(self.begin[stage])
+                x.pad = without_a
+                self.body(stage, True, without_a)
+                x.pad = False
+                assert x.reads == end[len(end) - len(x.reads):], "the masked tile ends otherwise"
+                x.put("s_branch %s" % self.ref("DONE%d" % stage))
+        for stage in range(self.STAGES):
+            self.label("IDLE%d" % stage)
+            x.put("s_waitcnt lgkmcnt(0)")
+            x.put("s_nop 15")
+            x.put("s_call_b64 %s, %s" % (s(self.BACK, 2), self.ref("LASTB")))
+            x.put("s_branch %s" % self.ref("REST%d" % stage))
+        for stage in range(self.STAGES):
+            self.label("REST%d" % stage)
+            self.idle(stage)
+            x.put("s_sub_u32 %[rem], %[rem], 1")
+            x.put("s_cmp_lg_u32 %[rem], 0")
+            x.put("s_cbranch_scc%d %s" % ((1, self.ref("REST0")) if stage == self.STAGES - 1 else (0, self.ref("RESTED"))))
+        self.label("RESTED")
+        x.put("s_waitcnt vmcnt(0)")
+        x.put("s_branch %s" % self.ref("WRITE"))
+        self.label("LASTB")
+        self.last_b("R")
+        x.put("s_setpc_b64 %s" % s(self.BACK, 2))
+        self.leave()
+        self.last_b("E")
+        self.label("WRITE")
         x.put("s_nop 15")
         x.put("s_nop 7")
         x.put("s_barrier")                         # everyone is done with the tiles
@@ -929,7 +995,7 @@ def generate():
             out.append(define("DH_FWD128_LOOP_%s_%d" % (dtype.upper(), copies), FWD(dtype, copies).text()))
     out.append(clobbers("DH_DKV128_CLOBBERS", DKV.KEEP, DKV.NEG, DKV.RSQ, DKV.CTC))
     out.append(clobbers("DH_DQ128_CLOBBERS", DQ.KEEP, DQ.ZERO, Keys.RSC, Keys.T))
-    out.append(clobbers("DH_FWD128_CLOBBERS", FWD.KEEP, FWD.ONES + 3, Keys.RSC, FWD.BOUND, FWD.SUMS + 16))
+    out.append(clobbers("DH_FWD128_CLOBBERS", FWD.KEEP, FWD.ONES + 3, Keys.RSC, FWD.BACK + 1, FWD.SUMS + 16))
     return "".join(out)
 
 

@@ -577,3 +577,30 @@ def test_attention_with_a_scale_of_zero(dtype, n, m, hq, causal):
     assert (dq == 0).all() and (dk == 0).all()
     part = (do.double() / keys[:, None, None]).view(n, 8, hq // 8, 128).sum(2)
     assert_close(dv, (part.flip(0).cumsum(0).flip(0) if causal else part.sum(0).expand(m, -1, -1)).cpu(), dtype, "dv")
+
+
+# causal calls on each of the kernels with one wavefront a SIMD: 256-row tiles, 128-row tiles (two splits of the keys)
+_CAUSAL_TILES = [([1024, 1001], 64, 8), ([2689], 20, 4), ([512, 491], 64, 64)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("lens,hq,hk", _CAUSAL_TILES[:2])
+@pytest.mark.parametrize("key", [70, 335, 999])
+def test_attention_forward_of_a_value_that_is_not_finite(dtype, lens, hq, hk, key):
+    """A later key's V reaches no causal row outside its own block of 32: those rows stay what they are, bit for bit."""
+    from dhellam_amd import _Clib
+    assert _fwd_path(lens, hq, 128, True) & 4
+    q, k, v, _ = _draw(dtype, lens, lens, hq, hk, 84)
+    cu, n, scale = _cu(lens).cuda(), max(lens), 1.0 / math.sqrt(128)
+
+    def run(v):
+        r = _Clib.pymha_varlen_fwd(q, k, v, cu, cu, n, n, 0.0, scale, True, False, 0, False)
+        return r[0], r[5]
+    out, lse = run(v)
+    first = key // 32 * 32
+    for bad in (float("nan"), float("inf")):
+        w = v.clone()
+        w[key] = bad
+        o2, l2 = run(w)
+        assert torch.equal(o2[:first], out[:first]) and all(torch.equal(l2[i, :, :m], lse[i, :, :m]) for i, m in enumerate(lens))
+        assert torch.equal(o2[lens[0]:], out[lens[0]:]) and not o2[key].isfinite().any()
