@@ -155,6 +155,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
     const int vx = causal ? 4 * g - r - wrow0 : -(1 << 30), vy = 4 * g - sk;      // key - row and key - keys, but for the tile's first key
     // tiles from this key on have something to mask
     const int mlim = causal && wrow0 - BN + 1 < sk - BN ? wrow0 - BN + 1 : sk - BN;
+    const int alim = causal ? wrow0 + 31 : 1 << 30;   // ... and past this key lie behind the first 32 rows
     floatx4 o[4][8];                                  // query block, d block
 #define DH_ACC4(qb, t) [o##qb##t] "=&a"(o[qb][t])
 #define DH_ACC(qb) \
@@ -170,7 +171,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
                  [lse0] "v"(lse[0]), [lse1] "v"(lse[1]), [lse2] "v"(lse[2]), [lse3] "v"(lse[3]), [nd0] "v"(nd[0]), [nd1] "v"(nd[1]),  \
                  [nd2] "v"(nd[2]), [nd3] "v"(nd[3]), [vx] "v"(vx), [vy] "v"(vy), [scale] "s"(p.scale_log2), [cp] "s"(cp),             \
                  [cstep] "s"(cstep), [left] "s"(left), [key] "s"(key), [keystep] "s"(SPLIT * BN), [crowb] "s"(c_rowb), [c16] "s"(c16), \
-                 [cdst] "s"(cdst), [mlim] "s"(mlim)                                                                                  \
+                 [cdst] "s"(cdst), [mlim] "s"(mlim), [alim] "s"(alim)                                                                                 \
                : DH_DQ128_CLOBBERS)
     if constexpr (__is_same(T, bf16_t)) {
       if constexpr (COPIES == 4) DH_LOOP(DH_DQ128_LOOP_BF16_4);

@@ -561,22 +561,32 @@ class DQ(Keys):
     AT_MASK = 55
 
     def tile(self, stage):
+        x = self.x
+        self.piece(stage, 0, self.AT_MASK)
+        x.put("s_cmp_gt_i32 %s, %%[mlim]" % s(self.KEY))
+        x.put("s_cbranch_scc1 %s" % self.ref("MASK%d" % stage))
+        self.label("MASKED%d" % stage)
+        self.masked_from[stage] = x.state()
+        self.piece(stage, self.AT_MASK, 96)
+        self.label("DONE%d" % stage)
+
+    def piece(self, stage, first, end, without=()):
+        """MFMAs `first` to `end` of a tile and what goes with them; the products of the query blocks `without` are left out."""
         x, work, issue = self.x, self.vector_work(), {}
         for use, at, d, n, text in self.reads(stage):
             issue.setdefault(at, []).append((text, d, n, use))
         next_rows = dict(zip(range(40, 56, 3), self.to_next_rows()))
-        for m in range(96):
+        for m in range(first, end):
             phase, qb, i = m // 32, m // 8 % 4, m % 8
             copies = (m - 1) // 3 if m % 3 == 1 and m < 3 * self.copies else None
             if copies is not None:
                 self.copy(copies, (stage + 3) % self.STAGES, True)
+            if m == 64 and without:
+                x.settle()
+                x.wait(set(range(self.KT, self.KT + 32)))
             if m == self.AT_BARRIER:
                 x.put("s_waitcnt vmcnt(%d)" % (2 * self.copies))       # the next tile has landed ..
                 x.put("s_barrier")                 # .. both its halves, and nobody reads this one any more
-            if m == self.AT_MASK:
-                x.put("s_cmp_gt_i32 %s, %%[mlim]" % s(self.KEY))
-                x.put("s_cbranch_scc1 %s" % self.ref("MASK%d" % stage))
-                self.label("MASKED%d" % stage)
             if phase < 2:
                 ks, kb = i // 2, i % 2
                 d, frag = (self.S, self.DP)[phase] + 4 * (2 * qb + kb), (self.KF, self.VF)[phase] + 4 * i
@@ -587,11 +597,12 @@ class DQ(Keys):
                 acc = "%%[o%d%d]" % (qb, i)
                 args = (acc, v(frag, 4), v(self.DSP + 4 * qb, 4), acc)
                 holds = [(v(frag, 4), 64 + i)]
-            need = set(range(frag, frag + 4))
-            if qb == 0 and i % 2 == 0:             # one wait for two fragments
-                need |= set(range(frag, frag + 8))
-            x.wait(need)
-            x.mfma(*args, holds)
+            if phase < 2 or qb not in without:
+                need = set(range(frag, frag + 4))
+                if qb == 0 and i % 2 == 0:         # one wait for two fragments
+                    need |= set(range(frag, frag + 8))
+                x.wait(need)
+                x.mfma(*args, holds)
             if copies is not None:
                 self.copy(copies, 0, False)
             for text, d, n, use in issue.get(m, []):
@@ -616,12 +627,28 @@ class DQ(Keys):
             x.put("%s %%[o%d%d], %s, %s, 0" % (x.mfma_name, i // 8, i % 8, v(self.KT, 4), v(self.KT, 4)))
         x.put("s_waitcnt vmcnt(%d)" % (2 * self.copies))
         x.put("s_barrier")
+        self.masked_from = {}
         self.loop(self.tile, self.first_reads)
+        end = [set(r) for r in x.reads]
         for stage in range(self.STAGES):
             self.label("MASK%d" % stage)
             self.mask_lanes(self.CX, self.CY)
             self.mask(self.S, v(self.ZERO), self.CX, self.CY)
-            x.put("s_branch %s" % self.ref("MASKED%d" % stage))
+            x.put("s_cmp_gt_i32 %s, %%[alim]" % s(self.KEY))
+            x.put("s_cbranch_scc0 %s" % self.ref("MASKED%d" % stage))
+            # keys behind the first 32 rows, or behind all 64: their blocks get no product
+            x.put("s_add_u32 %s, %%[alim], 32" % s(self.T))
+            x.put("s_cmp_gt_i32 %s, %s" % (s(self.KEY), s(self.T)))
+            x.put("s_cbranch_scc1 %s" % self.ref("IDLE%d" % stage))
+            x.pad = True
+            for without in ((0, 1), (0, 1, 2, 3)):
+                if len(without) == 4:
+                    self.label("IDLE%d" % stage)
+                x.resume(self.masked_from[stage])
+                self.piece(stage, self.AT_MASK, 96, without)
+                assert x.reads == end[len(end) - len(x.reads):], "the tile ends otherwise"
+                x.put("s_branch %s" % self.ref("DONE%d" % stage))
+            x.pad = False
         self.leave()
         return x.lines
 

@@ -604,3 +604,27 @@ def test_attention_forward_of_a_value_that_is_not_finite(dtype, lens, hq, hk, ke
         o2, l2 = run(w)
         assert torch.equal(o2[:first], out[:first]) and all(torch.equal(l2[i, :, :m], lse[i, :, :m]) for i, m in enumerate(lens))
         assert torch.equal(o2[lens[0]:], out[lens[0]:]) and not o2[key].isfinite().any()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("lens,hq,hk", _CAUSAL_TILES)
+@pytest.mark.parametrize("key", [70, 335, 480])
+def test_attention_backward_of_keys_that_are_not_finite(dtype, lens, hq, hk, key):
+    """A later key's K or V reaches no row of dQ outside its own block of 32."""
+    from dhellam_amd import _Clib
+    q, k, v, do = _draw(dtype, lens, lens, hq, hk, 88)
+    cu, n, scale = _cu(lens).cuda(), max(lens), 1.0 / math.sqrt(128)
+    r = _Clib.pymha_varlen_fwd(q, k, v, cu, cu, n, n, 0.0, scale, True, False, 0, False)
+    first = key // 32 * 32
+    _Clib.set_attn_bwd_ds_limit(0)
+    try:
+        dq = _bwd(do, q, k, v, r[0], r[5], cu, cu, n, n, scale, True)[0]
+        for bad in (float("nan"), float("inf")):
+            for which in range(2):
+                kv = [k.clone(), v.clone()]
+                kv[which][key] = bad
+                dq2 = _bwd(do, q, *kv, r[0], r[5], cu, cu, n, n, scale, True)[0]
+                assert torch.equal(dq2[:first], dq[:first]) and torch.equal(dq2[lens[0]:], dq[lens[0]:])
+                assert dq2[key].isnan().any()
+    finally:
+        _Clib.set_attn_bwd_ds_limit()
