@@ -22,6 +22,8 @@ namespace dh {
 // dK/dV of 32 query / 8 kv heads, 4096 rows x 2048 keys 300 -> 211 us (1.30 PFLOP/s at 1.5 GHz), causal 4096 304 -> 213, 8 / 1 heads x
 // 4096 keeping dS 95 -> 77, seven packed sequences of 1 to 3324 tokens 444 -> 300.
 // Rows past the sequence are zeros in LDS (buffer descriptors) and in the lse / delta planes: P = 1 there meets dO = 0, and dS = 0.
+// Key blocks that no row of a tile sees get no
+// products: a row's dO that is not finite reaches dV and dK of the keys in its block of 32 and before, no further.
 // The wavefronts' partial sums go through LDS and are added in the order of the wavefronts.
 template <typename T, bool STORE_DS>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) attn_bwd_dkv128_kernel(const AttnBwdParams p) {
@@ -156,7 +158,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
                  [rk0] "v"(rk[0]), [rk1] "v"(rk[1]), [rk2] "v"(rk[2]), [rk3] "v"(rk[3]), [ta0] "v"(ta[0]), [ta1] "v"(ta[1]),          \
                  [ta2] "v"(ta[2]), [ta3] "v"(ta[3]), [ta4] "v"(ta[4]), [ta5] "v"(ta[5]), [ta6] "v"(ta[6]), [ta7] "v"(ta[7]),          \
                  [cq0] "v"(cq[0]), [cq1] "v"(cq[1]), [cq2] "v"(cq[2]), [cq3] "v"(cq[3]), [cd0] "v"(cd[0]), [cd1] "v"(cd[1]),          \
-                 [cd2] "v"(cd[2]), [cd3] "v"(cd[3]), [cld] "v"(c_ld), [ldr] "v"(ldr), [vx] "v"(vx), [scale] "s"(p.scale_log2),        \
+                 [cd2] "v"(cd[2]), [cd3] "v"(cd[3]), [cld] "v"(c_ld), [ldr] "v"(ldr), [vx] "v"(vx), [scale] "s"(p.scale_log2), \
                  [wbase] "s"(wbase), [ntq] "s"(ntq), [rows] "s"(rows), [mct] "s"(mct), [qrowb] "s"(q_rowb), [drowb] "s"(do_rowb),     \
                  [q16] "s"(q16), [d16] "s"(d16), [ldbytes] "s"(ldbytes), [qp] "s"(qp), [dp] "s"(dp), [lp] "s"(lp),                    \
                  [qstep] "s"(qstep), [dstep] "s"(dstep), [qwrap] "s"(qwrap), [dwrap] "s"(dwrap), [lwrap] "s"(lwrap) __VA_ARGS__       \

@@ -269,23 +269,17 @@ class DKV:
                 self.x.put(line)
 
     def mask(self, i):
-        """Out of line: scores past the diagonal (and, where dS is kept, of keys past the end) become -inf."""
+        """Out of line: scores past the diagonal and, where dS is kept, of keys past the end become -inf.  The first tile of a causal one has 32 keys that no row of it sees: no products of theirs."""
         x = self.x
         self.label("MASK%d" % i)
         x.put("s_nop 15")
         x.put("s_nop 7")
-        tmp = self.E
+        diag = v(self.E)
         x.put("v_mov_b32 %s, 0xff800000" % v(self.NEG))
         x.put("s_lshl_b32 %s, %s, 5" % (s(self.T), s(self.CTC)))
-        x.put("v_subrev_u32 %s, %s, %%[vx]" % (v(tmp), s(self.T)))
-        for qb in range(2):
-            for kb in range(4):
-                for e in range(4):
-                    r = v(self.S + 4 * (4 * qb + kb) + e)
-                    x.put("v_cmp_lt_i32 vcc, %d, %s" % (16 * qb + e - 16 * kb, v(tmp)))
-                    x.put("s_nop 1")
-                    x.put("v_cndmask_b32 %s, %s, %s, vcc" % (r, r, v(self.NEG)))
         if self.store_ds:
+            x.put("s_cmp_eq_u32 %[dsmask], 0")
+            x.put("s_cbranch_scc1 %s" % self.ref("KEYS%d" % i))
             for kb in range(4):
                 x.put("v_cmp_le_i32 vcc, %d, %%[vy]" % (-16 * kb))
                 x.put("s_nop 1")
@@ -293,9 +287,36 @@ class DKV:
                     for e in range(4):
                         r = v(self.S + 4 * (4 * qb + kb) + e)
                         x.put("v_cndmask_b32 %s, %s, %s, vcc" % (r, r, v(self.NEG)))
-        x.put("s_branch %s" % self.ref("MASKED%d" % i))
+            self.label("KEYS%d" % i)
+        x.put("s_cmp_ge_i32 %s, %%[mct]" % s(self.CTC))
+        x.put("s_cbranch_scc1 %s" % self.ref("MASKED%d" % i))
+        x.put("v_subrev_u32 %s, %s, %%[vx]" % (diag, s(self.T)))
+        for qb in range(2):
+            for kb in range(4):
+                for e in range(4):
+                    r = v(self.S + 4 * (4 * qb + kb) + e)
+                    x.put("v_cmp_lt_i32 vcc, %d, %s" % (16 * qb + e - 16 * kb, diag))
+                    x.put("s_nop 1")
+                    x.put("v_cndmask_b32 %s, %s, %s, vcc" % (r, r, v(self.NEG)))
+        x.put("s_cmp_lg_u32 %s, 0" % s(self.CTC))
+        x.put("s_cbranch_scc1 %s" % self.ref("MASKED%d" % i))
+        x.pad = True
+        x.resume(self.masked_from[i])
+        self.piece(i, 32, 128, (2, 3))
+        x.pad = False
+        x.put("s_branch %s" % self.ref("DONE%d" % i))
 
     def tile(self, stage):
+        x = self.x
+        self.piece(stage, 0, 32)
+        x.put("s_cbranch_vccnz %s" % self.ref("MASK%d" % stage))      # scores to mask
+        self.label("MASKED%d" % stage)
+        self.masked_from[stage] = x.state()
+        self.piece(stage, 32, 128)
+        self.label("DONE%d" % stage)
+
+    def piece(self, stage, first, end, without=()):
+        """MFMAs `first` to `end` of a tile and what goes with them; dV and dK of the key blocks `without` get nothing."""
         x, st, nx = self.x, self.SLOTB * stage, self.SLOTB * (1 - stage)
         issue = {}
         for slot, use, d, n, f in self.ops:
@@ -311,7 +332,7 @@ class DKV:
         adv_at = {97 + i: p for i, p in enumerate(adv)}
         assert 97 + len(adv) <= first_ahead + 16
         nstores = 8 if self.store_ds else 0
-        for m in range(128):
+        for m in range(first, end):
             step, kb = m // 4, m % 4
             r = self.ring(step)
             copy = copies[m // 2 + (m == 31)] if m < 32 and (m % 2 == 0 or m == 31) and m // 2 + (m == 31) < 17 else None
@@ -320,9 +341,6 @@ class DKV:
                 x.put("s_add_u32 m0, %%[wbase], %d" % (nx + {"q": 1024 * i, "d": self.QTB + 1024 * i, "l": 2 * self.QTB}[c]))
             if m == first_ahead:
                 x.put("s_waitcnt vmcnt(%d)" % nstores)         # the next tile has landed
-            if m == 32:                                        # scores of the diagonal
-                x.put("s_cbranch_vccnz %s" % self.ref("MASK%d" % stage))
-                self.label("MASKED%d" % stage)
             frag = v(r, 4)
             if step < 8:
                 ks, qb = step // 2, step % 2
@@ -350,7 +368,8 @@ class DKV:
                 if step == 8:
                     need |= set(range(self.L4, self.L4 + 8)) | set(range(self.D4, self.D4 + 8))
             x.wait(need)
-            x.mfma(out, frag, y, c, [(frag, step)] + ([(y, step & ~1)] if step < 8 else []) + ([(c, step)] if step in (8, 9) else []))
+            if step < 16 or kb not in without:
+                x.mfma(out, frag, y, c, [(frag, step)] + ([(y, step & ~1)] if step < 8 else []) + ([(c, step)] if step in (8, 9) else []))
             if copy:
                 c, i = copy
                 if c == "l":
@@ -375,7 +394,7 @@ class DKV:
                 x.put("s_sub_u32 %[rem], %[rem], 1")
             shift = 10 if self.store_ds else 0                 # behind the stores, which need the tile's own address
             if m - shift in adv_at:
-                self.scalar(adv_at[m - shift], stage)
+                self.scalar(adv_at[m - shift], stage + (3 if without else 0))
 
     def text(self):
         x, R = self.x, self
@@ -399,6 +418,7 @@ class DKV:
             if slot < 0:
                 x.lds(f(0, d), d, n, use // 4)
         start = [set(r) for r in x.reads]
+        self.masked_from = {}
         self.label("LOOP")
         for stage in range(2):
             self.tile(stage)
@@ -407,10 +427,12 @@ class DKV:
             x.put("s_cmp_eq_u32 %[rem], 0")
             x.put("s_cbranch_scc%d %s" % ((1, self.ref("END")) if stage == 0 else (0, self.ref("LOOP"))))
         x.put("s_branch %s" % self.ref("END"))
-        for i in range(3):
-            self.wrap(i)
+        end = [set(r) for r in x.reads]
         for i in range(2):
             self.mask(i)
+            assert x.reads == end, "the tile ends otherwise"
+        for i in range(5):
+            self.wrap(i)
         self.label("END")
         x.put("s_waitcnt vmcnt(0) lgkmcnt(0)")
         x.put("s_nop 15")

@@ -628,3 +628,23 @@ def test_attention_backward_of_keys_that_are_not_finite(dtype, lens, hq, hk, key
                 assert dq2[key].isnan().any()
     finally:
         _Clib.set_attn_bwd_ds_limit()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("lens,hq,hk", [([1024, 1001], 64, 8), ([1537], 19, 19)])
+@pytest.mark.parametrize("row", [5, 70, 671])
+def test_attention_backward_of_rows_that_are_not_finite(dtype, lens, hq, hk, row, ds_path):
+    """An earlier row's dO reaches no key of dK or dV outside its own block of 32."""
+    from dhellam_amd import _Clib
+    assert _bwd_path(lens, lens, hq, hk, 128, True) & 1
+    q, k, v, do = _draw(dtype, lens, lens, hq, hk, 92)
+    cu, n, scale = _cu(lens).cuda(), max(lens), 1.0 / math.sqrt(128)
+    r = _Clib.pymha_varlen_fwd(q, k, v, cu, cu, n, n, 0.0, scale, True, False, 0, False)
+    _, dk, dv = _bwd(do, q, k, v, r[0], r[5], cu, cu, n, n, scale, True)
+    behind = row // 32 * 32 + 32
+    for bad in (float("nan"), float("inf")):
+        d2 = do.clone()
+        d2[row] = bad
+        _, dk2, dv2 = _bwd(d2, q, k, v, r[0], r[5], cu, cu, n, n, scale, True)
+        assert torch.equal(dk2[behind:], dk[behind:]) and torch.equal(dv2[behind:], dv[behind:])
+        assert not dv2[0].isfinite().all()
