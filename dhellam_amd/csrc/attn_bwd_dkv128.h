@@ -21,8 +21,8 @@ namespace dh {
 // left to the compiler the loop took 3020 cycles with 32x32x16 and 3300 with 16x16x32, but 245 us (1.63 GHz) and 228 (1.9 GHz).
 // dK/dV of 32 query / 8 kv heads, 4096 rows x 2048 keys 300 -> 211 us (1.30 PFLOP/s at 1.5 GHz), causal 4096 304 -> 213, 8 / 1 heads x
 // 4096 keeping dS 95 -> 77, seven packed sequences of 1 to 3324 tokens 444 -> 300.
-// Rows past the sequence are zeros in LDS (buffer descriptors) and in the lse / delta planes: P = 1 there meets dO = 0, and dS = 0.
-// Key blocks that no row of a tile sees get no
+// Rows past the sequence are zeros in LDS (buffer descriptors) and in the lse / delta planes, and their scores are masked: P = 1 would meet
+// dO = 0 as well, but the score of such a row and a key that holds an infinity is none.  Key blocks that no row of a tile sees get no
 // products: a row's dO that is not finite reaches dV and dK of the keys in its block of 32 and before, no further.
 // The wavefronts' partial sums go through LDS and are added in the order of the wavefronts.
 template <typename T, bool STORE_DS>
@@ -121,7 +121,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
     const int64_t qwrap = (int64_t)ROWB - (int64_t)ntq * BM * q_rowb, dwrap = (int64_t)ROWB - (int64_t)ntq * BM * do_rowb;
     const int64_t lwrap = ((int64_t)p.ld2_pitch - (int64_t)ntq * BM) * 4;
     const uint32_t ldbytes = (uint32_t)(p.ld2_plane * 4) + 128u, q16 = 16u * q_rowb, d16 = 16u * do_rowb;
-    const int rows = sq - i_begin, mct = causal ? 2 : 0;
+    // tiles with scores to mask: the first two of a causal one, and the one that the rows end in
+    const int rows = sq - i_begin, mct = causal ? 2 : 0, pct = (rows & (BM - 1)) != 0 && p.scale_log2 > 0.f ? ntq - 1 : -1;
     {
       const int left = rows - ct * BM < BM ? rows - ct * BM : BM;
       const int4s rsq = rows_rsrc(qp, rem > 0 ? (uint32_t)(left - 1) * q_rowb + ROWB : 0u);
@@ -144,6 +145,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");      // (the loop copies to the second stages)
     }
     const int vx = causal ? r - 4 * g : -(1 << 20);   // key - row of a score, but for what the loop adds
+    const int vz = 4 * g - rows;                      // row - rows
     floatx4 dV[4][8], dK[4][8];                       // key block, d block
 #define DH_ACC4(x, X, kb, t) [x##kb##t] "=a"(X[kb][t])
 #define DH_ACC(x, X, kb)                                                                                                             \
@@ -158,8 +160,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
                  [rk0] "v"(rk[0]), [rk1] "v"(rk[1]), [rk2] "v"(rk[2]), [rk3] "v"(rk[3]), [ta0] "v"(ta[0]), [ta1] "v"(ta[1]),          \
                  [ta2] "v"(ta[2]), [ta3] "v"(ta[3]), [ta4] "v"(ta[4]), [ta5] "v"(ta[5]), [ta6] "v"(ta[6]), [ta7] "v"(ta[7]),          \
                  [cq0] "v"(cq[0]), [cq1] "v"(cq[1]), [cq2] "v"(cq[2]), [cq3] "v"(cq[3]), [cd0] "v"(cd[0]), [cd1] "v"(cd[1]),          \
-                 [cd2] "v"(cd[2]), [cd3] "v"(cd[3]), [cld] "v"(c_ld), [ldr] "v"(ldr), [vx] "v"(vx), [scale] "s"(p.scale_log2), \
-                 [wbase] "s"(wbase), [ntq] "s"(ntq), [rows] "s"(rows), [mct] "s"(mct), [qrowb] "s"(q_rowb), [drowb] "s"(do_rowb),     \
+                 [cd2] "v"(cd[2]), [cd3] "v"(cd[3]), [cld] "v"(c_ld), [ldr] "v"(ldr), [vx] "v"(vx), [vz] "v"(vz), [scale] "s"(p.scale_log2), \
+                 [wbase] "s"(wbase), [ntq] "s"(ntq), [rows] "s"(rows), [mct] "s"(mct), [pct] "s"(pct), [qrowb] "s"(q_rowb), [drowb] "s"(do_rowb),     \
                  [q16] "s"(q16), [d16] "s"(d16), [ldbytes] "s"(ldbytes), [qp] "s"(qp), [dp] "s"(dp), [lp] "s"(lp),                    \
                  [qstep] "s"(qstep), [dstep] "s"(dstep), [qwrap] "s"(qwrap), [dwrap] "s"(dwrap), [lwrap] "s"(lwrap) __VA_ARGS__       \
                : DH_DKV128_CLOBBERS)

@@ -129,7 +129,7 @@ class DKV:
     KEEP = 100                                     # VGPRs below this are the compiler's (operands)
     S, DP, PP, DSP, RING, L4, D4, E = 100, 132, 164, 180, 196, 228, 236, 244
     NEG = 248
-    RSQ, RSD, RSL, QSTEP, DSTEP, QWRAP, DWRAP, LWRAP, DSC, DSS, DSTEP_DS, WRAP_DS, T, CTC = 40, 44, 48, 52, 54, 56, 58, 60, 62, 64, 66, 68, 70, 76
+    RSQ, RSD, RSL, QSTEP, DSTEP, QWRAP, DWRAP, LWRAP, DSC, DSS, DSTEP_DS, WRAP_DS, T, CTC, PADS = 40, 44, 48, 52, 54, 56, 58, 60, 62, 64, 66, 68, 70, 76, 78
     LOOK = 15                                      # MFMAs between an LDS read and its use
     ROWB, QTB, SLOTB = 256, 8192, 16640
 
@@ -269,14 +269,29 @@ class DKV:
                 self.x.put(line)
 
     def mask(self, i):
-        """Out of line: scores past the diagonal and, where dS is kept, of keys past the end become -inf.  The first tile of a causal one has 32 keys that no row of it sees: no products of theirs."""
+        """Out of line: scores past the diagonal, of rows past the end (their Q is 0, but 0 times an infinity is none) and, where dS is
+        kept, of keys past the end become -inf.  The first tile of a causal one has 32 keys that no row of it sees: no products of theirs."""
         x = self.x
         self.label("MASK%d" % i)
         x.put("s_nop 15")
         x.put("s_nop 7")
-        diag = v(self.E)
+        diag, rows = v(self.E), v(self.E + 1)
         x.put("v_mov_b32 %s, 0xff800000" % v(self.NEG))
         x.put("s_lshl_b32 %s, %s, 5" % (s(self.T), s(self.CTC)))
+        x.put("s_cmp_lg_u32 %s, %%[pct]" % s(self.CTC))
+        x.put("s_cbranch_scc1 %s" % self.ref("WHOLE%d" % i))
+        x.put("v_add_u32 %s, %s, %%[vz]" % (rows, s(self.T)))
+        for qb in range(2):
+            if qb:
+                x.put("v_add_u32 %s, 16, %s" % (rows, rows))
+            for e in range(4):
+                x.put("v_cmp_le_i32 %s, %d, %s" % (s(self.PADS + 2 * e, 2), -e, rows))
+            x.put("s_nop 1")
+            for kb in range(4):
+                for e in range(4):
+                    r = v(self.S + 4 * (4 * qb + kb) + e)
+                    x.put("v_cndmask_b32 %s, %s, %s, %s" % (r, r, v(self.NEG), s(self.PADS + 2 * e, 2)))
+        self.label("WHOLE%d" % i)
         if self.store_ds:
             x.put("s_cmp_eq_u32 %[dsmask], 0")
             x.put("s_cbranch_scc1 %s" % self.ref("KEYS%d" % i))
@@ -383,6 +398,8 @@ class DKV:
             if m == 20:                                        # whether this tile has scores to mask: vcc for the branch at 32
                 x.put("s_cmp_lt_i32 %s, %%[mct]" % s(self.CTC))
                 x.put("s_cselect_b64 vcc, -1, 0")
+                x.put("s_cmp_eq_u32 %s, %%[pct]" % s(self.CTC))
+                x.put("s_cselect_b64 vcc, -1, vcc")
                 if self.store_ds:
                     x.put("s_cmp_lg_u32 %[dsmask], 0")
                     x.put("s_cselect_b64 vcc, -1, vcc")
@@ -1042,7 +1059,7 @@ def generate():
             out.append(define("DH_DQ128_LOOP_%s_%d" % (dtype.upper(), copies), DQ(dtype, copies).text()))
         for copies in (4, 8):
             out.append(define("DH_FWD128_LOOP_%s_%d" % (dtype.upper(), copies), FWD(dtype, copies).text()))
-    out.append(clobbers("DH_DKV128_CLOBBERS", DKV.KEEP, DKV.NEG, DKV.RSQ, DKV.CTC))
+    out.append(clobbers("DH_DKV128_CLOBBERS", DKV.KEEP, DKV.NEG, DKV.RSQ, DKV.PADS + 7))
     out.append(clobbers("DH_DQ128_CLOBBERS", DQ.KEEP, DQ.ZERO, Keys.RSC, Keys.T))
     out.append(clobbers("DH_FWD128_CLOBBERS", FWD.KEEP, FWD.ONES + 3, Keys.RSC, FWD.BACK + 1, FWD.SUMS + 16))
     return "".join(out)

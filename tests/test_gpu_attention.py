@@ -648,3 +648,23 @@ def test_attention_backward_of_rows_that_are_not_finite(dtype, lens, hq, hk, row
         _, dk2, dv2 = _bwd(d2, q, k, v, r[0], r[5], cu, cu, n, n, scale, True)
         assert torch.equal(dk2[behind:], dk[behind:]) and torch.equal(dv2[behind:], dv[behind:])
         assert not dv2[0].isfinite().all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,keys,hq,hk", [([800, 515], [960, 640], 48, 8), ([1537], [1600], 19, 19)])
+def test_attention_backward_of_keys_that_no_row_sees(dtype, rows, keys, hq, hk, ds_path):
+    """Causal, more keys than rows: what K holds behind the last row is met by nothing, also by the zeros that fill up the last tile
+    of rows."""
+    from dhellam_amd import _Clib
+    assert _bwd_path(rows, keys, hq, hk, 128, True) & 1
+    q, k, v, do = _draw(dtype, rows, keys, hq, hk, 96)
+    cq, ck, mq, mk, scale = _cu(rows).cuda(), _cu(keys).cuda(), max(rows), max(keys), 1.0 / math.sqrt(128)
+    r = _Clib.pymha_varlen_fwd(q, k, v, cq, ck, mq, mk, 0.0, scale, True, False, 0, False)
+    clean = _bwd(do, q, k, v, r[0], r[5], cq, ck, mq, mk, scale, True)
+    for bad in (float("nan"), float("-inf")):
+        k2, at = k.clone(), 0
+        for i, j in zip(rows, keys):
+            k2[at + i:at + j] = bad
+            at += j
+        _, dk, dv = _bwd(do, q, k2, v, r[0], r[5], cq, ck, mq, mk, scale, True)
+        assert torch.equal(dk, clean[1]) and torch.equal(dv, clean[2])
