@@ -24,6 +24,9 @@ template <int D> struct AttnTile {
   }
 };
 
+// Largest token stride (elements of 16 bits) whose offsets across 15 rows fit the 32 bits of a lane's offset.
+constexpr int64_t TILE_MAX_STRIDE = 1ll << 27;
+
 // A wavefront's lane offsets for the copies of 16 rows.
 template <int D> struct TileCopy { uint32_t off[AttnTile<D>::PAT]; };
 template <int D> __device__ __forceinline__ void tile_copy_lane(int i, int lane, int &row, int &chunk) {
@@ -43,11 +46,11 @@ template <int D> __device__ __forceinline__ TileCopy<D> tile_copy(int lane, uint
   return c;
 }
 // Rows row0 .. row0 + ROWS - 1 of `g` (ROWS and the tile row at `dst` multiples of 16) to LDS byte address `dst`; `rows`:
-// rows of the sequence, later ones repeat the last.  The copies are not counted by the compiler (dma_wait_all).
+// rows of the sequence, later ones repeat the last.  Rows past the reach of the lane offsets are addressed one by one.  The copies are not counted by the compiler (dma_wait_all).
 template <typename T, int D, int ROWS>
 __device__ __forceinline__ void copy_tile(const T *g, int64_t stride, int row0, int rows, uint32_t dst, const TileCopy<D> &c, int lane) {
   constexpr int PAT = AttnTile<D>::PAT;
-  if (row0 + ROWS <= rows) {
+  if (row0 + ROWS <= rows && stride <= TILE_MAX_STRIDE) {
     const char *src = reinterpret_cast<const char *>(g + (int64_t)row0 * stride);
 #pragma unroll
     for (int q = 0; q < ROWS / 16; ++q) {

@@ -216,3 +216,25 @@ def test_attention_past_2_31_elements():
         for name, big, one in (("out", out[sl], o1), ("lse", lse[bi], l1[0]), ("dq", dq[sl], dq1), ("dk", dk[sl], dk1),
                                ("dv", dv[sl], dv1)):
             assert_close(big, one.cpu(), BF, f"{name}[{bi}]", scale=0.1)
+
+
+@pytest.mark.parametrize("causal,hq,hk", [(False, 136, 136), (True, 8, 2)])
+def test_attention_of_rows_too_far_apart_for_a_lane_offset(causal, hq, hk):
+    """Token strides of 3 * 2^26 elements: 16 rows lie further apart than 4 GiB.  Same results as from dense copies, on whichever kernels
+    either call runs (the first backward ran hand-ordered ones before their copies took 16 rows at a time)."""
+    from dhellam_amd import _Clib
+    _need(26)
+    n, d, stride = 50, 128, 3 << 26
+    held = torch.empty(n * stride, dtype=BF, device="cuda")
+    q, k, v = (held.as_strided((n, h, d), (stride, d, 1), at * d) for h, at in ((hq, 0), (hk, hq), (hk, hq + hk)))
+    dense = [_randn(t.shape, 30 + i) for i, t in enumerate((q, k, v))]
+    for t, x in zip((q, k, v), dense):
+        t.copy_(x)
+    do, cu, scale = _randn((n, hq, d), 33), torch.tensor([0, n], dtype=torch.int32, device="cuda"), d ** -0.5
+    got = []
+    for a in ((q, k, v), dense):
+        r = _Clib.pymha_varlen_fwd(*a, cu, cu, n, n, 0.0, scale, causal, False, 0, False)
+        got.append([r[0]] + _Clib.pymha_varlen_bwd(do, *a, r[0], r[5], cu, cu, n, n, 0.0, scale, causal, None, True, 0, False,
+                                                   torch.cuda.current_stream().cuda_stream)[:3])
+    for far, near, what in zip(*got, ("out", "dq", "dk", "dv")):
+        assert_close(far, near.cpu(), BF, what)
