@@ -63,7 +63,9 @@ SIGNATURES = {
     "dh_attn_fwd_total": (_i32, [_vp] * 7 + [_i32] * 5 + [_i64] + [_i32] * 3 + [_i64] * 4 + [_f32, _i32, _i32, _vp]),
     "dh_attn_fwd_state": (_i32, [_vp] * 8 + [_i32] * 5 + [_i64] + [_i32] * 3 + [_i64] * 4 + [_f32, _i32, _i32, _vp]),
     "dh_attn_fwd_path": (_i32, [_i32, _i32, _i64, _i32, _i32, _i32]),
+    "dh_attn_fwd_rows": (_i32, [_i32] * 3 + [_i64] + [_i32] * 3),
     "dh_attn_bwd_path": (_i32, [_i32] * 3 + [_i64] * 2 + [_i32] * 4 + [_sz]),
+    "dh_attn_bwd_dq_rows": (_i32, [_i32] * 3 + [_i64] * 2 + [_i32] * 4 + [_sz]),
     "dh_attn_bwd_one_launch": (_i32, [_i32] * 3 + [_i64] * 2 + [_i32] * 4),
     "dh_attn_bwd_workspace_bytes": (_sz, [_i64, _i64, _i32, _i32, _i32, _i32, _i32, _i32]),
     "dh_attn_bwd_min_workspace_bytes": (_sz, [_i64, _i64, _i32, _i32, _i32, _i32, _i32, _i32]),

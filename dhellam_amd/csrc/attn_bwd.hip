@@ -983,14 +983,25 @@ extern "C" int dh_attn_bwd_one_launch(int batch, int max_seqlen_q, int max_seqle
   return dh::attn_bwd_route(batch, max_seqlen_q, max_seqlen_k, total_q, total_k, hq, hk, d, causal, false).both ? 1 : 0;
 }
 
-extern "C" int dh_attn_bwd_path(int batch, int max_seqlen_q, int max_seqlen_k, int64_t total_q, int64_t total_k, int hq, int hk, int d,
-                                int causal, size_t workspace_bytes) {
+// The route of a 16-bit call with a workspace of so many bytes.
+static dh::AttnBwdRoute bwd_route_in(int batch, int max_seqlen_q, int max_seqlen_k, int64_t total_q, int64_t total_k, int hq, int hk, int d,
+                                     int causal, size_t workspace_bytes) {
   using namespace dh;
   const size_t base = bwd_base_bytes(total_k, batch, max_seqlen_q, hq, hk, d, DH_BF16);
   const size_t dsb = ds_bytes(batch, max_seqlen_q, total_k, hq, d, DH_BF16, causal);
-  const AttnBwdRoute r = attn_bwd_route(batch, max_seqlen_q, max_seqlen_k, total_q, total_k, hq, hk, d, causal,
-                                        dsb > 0 && base + align256(dsb) <= workspace_bytes);
+  return attn_bwd_route(batch, max_seqlen_q, max_seqlen_k, total_q, total_k, hq, hk, d, causal, dsb > 0 && base + align256(dsb) <= workspace_bytes);
+}
+
+extern "C" int dh_attn_bwd_path(int batch, int max_seqlen_q, int max_seqlen_k, int64_t total_q, int64_t total_k, int hq, int hk, int d,
+                                int causal, size_t workspace_bytes) {
+  const dh::AttnBwdRoute r = bwd_route_in(batch, max_seqlen_q, max_seqlen_k, total_q, total_k, hq, hk, d, causal, workspace_bytes);
   return (r.hand_dkv ? 1 : 0) | (r.keep_ds ? 2 : (r.hand_dq ? 4 : 0) | (r.big_dq ? 8 : 0));
+}
+
+extern "C" int dh_attn_bwd_dq_rows(int batch, int max_seqlen_q, int max_seqlen_k, int64_t total_q, int64_t total_k, int hq, int hk, int d,
+                                   int causal, size_t workspace_bytes) {
+  const dh::AttnBwdRoute r = bwd_route_in(batch, max_seqlen_q, max_seqlen_k, total_q, total_k, hq, hk, d, causal, workspace_bytes);
+  return r.keep_ds ? 0 : r.dq_rows;
 }
 
 static int attn_bwd_entry(const void *dout, const void *q, const void *k, const void *v, const void *out,

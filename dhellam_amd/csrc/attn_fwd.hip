@@ -508,6 +508,10 @@ extern "C" int dh_attn_fwd_path(int batch, int max_seqlen_q, int64_t total_q, in
   return (r.hand ? 1 : 0) | (r.big ? 2 : 0) | (r.rows ? 4 : 0);
 }
 
+extern "C" int dh_attn_fwd_rows(int batch, int max_seqlen_q, int max_seqlen_k, int64_t total_q, int hq, int d, int causal) {
+  return dh::attn_fwd_route(max_seqlen_q, max_seqlen_k, hq, d, batch, total_q, causal).rows;
+}
+
 extern "C" int dh_attn_fwd_state(const void *q, const void *k, const void *v, void *out, float *lse, int64_t *rng_state,
                                  const int32_t *cu_seqlens_q, const int32_t *cu_seqlens_k, int q_shift, int k_shift,
                                  int batch, int max_seqlen_q, int max_seqlen_k, int64_t total_q, int hq, int hk, int d,

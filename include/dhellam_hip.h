@@ -192,17 +192,27 @@ int dh_attn_fwd_state(const void *q, const void *k, const void *v, void *out,
 
 /* Which kernels a 16-bit call of these sizes runs (what the entries themselves
  * go by).  Forward: bit 0 = head dim 128's hand-ordered kernel, bit 1 = query
- * tiles of 128 rows (else 64), bit 2 = head dim 128's kernel of one wavefront a
- * SIMD instead of either (with at least as many keys as query rows).  Backward: bit 0 = head dim 128's hand-ordered
- * dK/dV kernel, bit 1 = dQ from kept dS, else bit 2 = the hand-ordered
- * recomputing dQ kernel and bit 3 = its query tiles have 128 rows (all
- * clear: the other kernels, which for small calls run in one launch, as
- * dh_attn_bwd_one_launch tells). */
+ * tiles of 128 rows (else 64), bit 2 = for as many keys as query rows, head dim
+ * 128's kernel of one wavefront a SIMD instead of either.  Backward: bit 0 = head
+ * dim 128's hand-ordered dK/dV kernel, bit 1 = dQ from kept dS, else bit 2 = a
+ * hand-ordered recomputing dQ kernel and bit 3 = its query tiles have 128 rows
+ * or more (all clear: the other kernels, which for small calls run in one
+ * launch, as dh_attn_bwd_one_launch tells).
+ * dh_attn_fwd_rows, dh_attn_bwd_dq_rows: the query rows of a tile, 256 or 128,
+ * where the forward / the recomputing dQ run on one wavefront a SIMD, else 0.
+ * The entries keep to other kernels where a softmax scale is negative (forward)
+ * or a token stride exceeds 2^26 elements (forward, K and V; backward 2^25, any
+ * input). */
 int dh_attn_fwd_path(int batch, int max_seqlen_q, int64_t total_q, int hq,
                      int d, int causal);
+int dh_attn_fwd_rows(int batch, int max_seqlen_q, int max_seqlen_k,
+                     int64_t total_q, int hq, int d, int causal);
 int dh_attn_bwd_path(int batch, int max_seqlen_q, int max_seqlen_k,
                      int64_t total_q, int64_t total_k, int hq, int hk, int d,
                      int causal, size_t workspace_bytes);
+int dh_attn_bwd_dq_rows(int batch, int max_seqlen_q, int max_seqlen_k,
+                        int64_t total_q, int64_t total_k, int hq, int hk, int d,
+                        int causal, size_t workspace_bytes);
 int dh_attn_bwd_one_launch(int batch, int max_seqlen_q, int max_seqlen_k,
                            int64_t total_q, int64_t total_k, int hq, int hk,
                            int d, int causal);

@@ -76,6 +76,21 @@ def test_attention_route(batch, max_q, total_q, hq, causal, hand):
     assert lib.dh_attn_bwd_path(batch, max_q, max_q, total_q, total_q, hq, hq, 96, causal, 1 << 40) & 7 == 0
 
 
+@pytest.mark.parametrize("batch,max_q,max_k,total_q,hq,causal,fwd,dq", [
+    (1, 4096, 4096, 4096, 32, 1, 256, 256), (1, 2048, 2048, 2048, 32, 1, 0, 128), (1, 2689, 2689, 2689, 20, 1, 128, 0),
+    (1, 700, 2000, 700, 44, 0, 128, 128), (1, 700, 700, 700, 44, 0, 0, 128),                 # the forward by the number of keys
+    (1, 600, 333, 600, 32, 0, 128, 0), (1, 511, 2000, 511, 64, 0, 0, 128), (0, 0, 0, 0, 8, 1, 0, 0), (1, 4096, 0, 4096, 32, 0, 256, 256)])
+def test_attention_tiles_on_one_wavefront_a_simd(batch, max_q, max_k, total_q, hq, causal, fwd, dq):
+    """Head dim 128 without room for dS: query rows of a tile, forward and dQ, on both sides of the lines."""
+    _ensure_lib()
+    lib = _lib.load()
+    assert lib.dh_attn_fwd_rows(batch, max_q, max_k, total_q, hq, 128, causal) == fwd
+    assert lib.dh_attn_bwd_dq_rows(batch, max_q, max_k, total_q, total_q, hq, hq, 128, causal, 0) == dq
+    assert lib.dh_attn_fwd_rows(batch, max_q, max_k, total_q, hq, 96, causal) == 0
+    if max_q == max_k:
+        assert bool(lib.dh_attn_fwd_path(batch, max_q, total_q, hq, 128, causal) & 4) == (fwd > 0)
+
+
 @pytest.mark.parametrize("lens,hq,hk,one,path", [
     ([1000] + [1] * 7, 8, 8, 1, 0), ([1500] + [20] * 15, 4, 4, 1, 0), ([386, 382] + [1] * 14, 12, 4, 1, 0),
     ([599] + [1] * 47, 4, 4, 0, 9), ([599] + [1] * 23, 4, 4, 1, 0)])

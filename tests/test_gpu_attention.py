@@ -668,3 +668,67 @@ def test_attention_backward_of_keys_that_no_row_sees(dtype, rows, keys, hq, hk, 
             at += j
         _, dk, dv = _bwd(do, q, k2, v, r[0], r[5], cq, ck, mq, mk, scale, True)
         assert torch.equal(dk, clean[1]) and torch.equal(dv, clean[2])
+
+
+def _tiles(lens_q, lens_k, hq, hk, causal):
+    """Query rows of a tile on one wavefront a SIMD (0: other kernels), forward and recomputing dQ."""
+    from dhellam_amd import _lib
+    lib, n, mq, mk, tq, tk = _lib.load(), len(lens_q), max(lens_q), max(lens_k), sum(lens_q), sum(lens_k)
+    return (lib.dh_attn_fwd_rows(n, mq, mk, tq, hq, 128, causal),
+            lib.dh_attn_bwd_dq_rows(n, mq, mk, tq, tk, hq, hk, 128, causal, 0))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("lens_q,lens_k,hq,hk,causal,fwd,dq", [
+    ([1100], [333], 32, 8, False, 0, 128),                     # two splits of an odd number of key tiles
+    ([1100], [20], 32, 8, False, 0, 128),                      # a second split without a key
+    ([1100, 1090], [40, 31], 16, 8, False, 0, 128),
+    ([1100], [1100], 32, 32, False, 128, 128),
+    ([700], [2000], 44, 44, False, 128, 128),                  # by the number of keys
+    ([512, 491], [512, 491], 64, 64, True, 0, 128),
+    ([961], [961], 64, 8, True, 0, 128),                       # odd numbers of tiles behind the diagonal
+    ([600], [20], 32, 8, False, 128, 0),
+    ([2689], [2689], 40, 8, True, 256, 256),
+    ([767] * 4, [37, 2, 640, 1], 32, 4, False, 256, 256),
+])
+def test_attention_query_tiles_on_one_wavefront_a_simd(dtype, lens_q, lens_k, hq, hk, causal, fwd, dq):
+    """Each form of the forward and of the recomputing dQ, at the ends of its tiles and splits."""
+    from dhellam_amd import _Clib
+    assert _tiles(lens_q, lens_k, hq, hk, causal) == (fwd, dq)
+    _Clib.set_attn_bwd_ds_limit(0)
+    try:
+        _run_fwd_bwd(dtype, lens_q, lens_k, hq, hk, 128, causal, oracle_dtype=torch.float32)
+    finally:
+        _Clib.set_attn_bwd_ds_limit()
+
+
+@pytest.mark.parametrize("lens_q,lens_k,hq,hk,tiles", [
+    ([600, 600], [0, 333], 16, 4, (128, 0)), ([1100, 1090], [40, 0], 32, 8, (0, 256)), ([1100, 1090], [40, 0], 16, 8, (0, 128)),
+    ([767] * 4, [37, 0, 640, 33], 32, 4, (256, 256)),
+])
+def test_attention_of_sequences_without_keys(lens_q, lens_k, hq, hk, tiles):
+    """Rows that see nothing: out, dQ and delta are 0 and lse is -inf; the other sequences' results are those of a call without them."""
+    from dhellam_amd import _Clib
+    assert _tiles(lens_q, lens_k, hq, hk, False) == tiles
+    q, k, v, do = _draw(torch.bfloat16, lens_q, lens_k, hq, hk, 100)
+    cq, ck, mq, mk, scale = _cu(lens_q).cuda(), _cu(lens_k).cuda(), max(lens_q), max(lens_k), 1.0 / math.sqrt(128)
+    _Clib.set_attn_bwd_ds_limit(0)
+    try:
+        r = _Clib.pymha_varlen_fwd(q, k, v, cq, ck, mq, mk, 0.0, scale, False, False, 0, False)
+        dq, dk, dv = _bwd(do, q, k, v, r[0], r[5], cq, ck, mq, mk, scale, False)
+    finally:
+        _Clib.set_attn_bwd_ds_limit()
+    aq = ak = 0
+    for i, (n, m) in enumerate(zip(lens_q, lens_k)):
+        sq, sk = slice(aq, aq + n), slice(ak, ak + m)
+        if m == 0:
+            assert (r[0][sq] == 0).all() and (dq[sq] == 0).all() and (r[5][i, :, :n] == float("-inf")).all()
+        else:
+            cpu = [t.cpu() for t in (do[sq], q[sq], k[sk], v[sk])]
+            one = _cu([n]), _cu([m]), scale, False, torch.float32
+            oo, lo = OA.attn_fwd(*cpu[1:], *one)
+            want = OA.attn_bwd(*cpu, r[0][sq].cpu(), r[5][i:i + 1, :, :n].cpu().double(), *one)
+            for got, ref, what in ((r[0][sq], oo, "out"), (dq[sq], want[0], "dq"), (dk[sk], want[1], "dk"), (dv[sk], want[2], "dv")):
+                assert_close(got, ref, torch.bfloat16, what)
+            assert_close(r[5][i, :, :n], lo[0], torch.float32, "lse")
+        aq, ak = aq + n, ak + m

@@ -238,3 +238,28 @@ def test_attention_of_rows_too_far_apart_for_a_lane_offset(causal, hq, hk):
                                                    torch.cuda.current_stream().cuda_stream)[:3])
     for far, near, what in zip(*got, ("out", "dq", "dk", "dv")):
         assert_close(far, near.cpu(), BF, what)
+
+
+@pytest.mark.parametrize("stride", [(1 << 25) + 64, (1 << 26) + 64])
+def test_attention_of_keys_too_far_apart_for_one_wavefront_a_simd(stride):
+    """Token strides of K and V just past what the copies of those kernels reach, backward and forward: other kernels, same results."""
+    from dhellam_amd import _Clib, _lib
+    _need(14)
+    n, m, hq, hk, d = 1100, 45, 32, 8, 128
+    lib = _lib.load()
+    assert lib.dh_attn_fwd_rows(1, 600, m, 600, hq, d, 0) == 128 and lib.dh_attn_bwd_dq_rows(1, n, m, n, m, hq, hk, d, 0, 0) == 128
+    held = torch.empty(m * stride, dtype=BF, device="cuda")
+    far = [held.as_strided((m, hk, d), (stride, d, 1), at * d) for at in (0, hk)]
+    near = [_randn((m, hk, d), 40 + i) for i in range(2)]
+    for t, x in zip(far, near):
+        t.copy_(x)
+    for rows in (600, n):
+        q, do = _randn((rows, hq, d), 42), _randn((rows, hq, d), 43)
+        cq, ck = (torch.tensor([0, t], dtype=torch.int32, device="cuda") for t in (rows, m))
+        got = []
+        for k, v in (far, near):
+            r = _Clib.pymha_varlen_fwd(q, k, v, cq, ck, rows, m, 0.0, d ** -0.5, False, False, 0, False)
+            got.append([r[0]] + _Clib.pymha_varlen_bwd(do, q, k, v, r[0], r[5], cq, ck, rows, m, 0.0, d ** -0.5, False, None, True, 0,
+                                                       False, torch.cuda.current_stream().cuda_stream)[:3])
+        for a, b, what in zip(*got, ("out", "dq", "dk", "dv")):
+            assert_close(a, b.cpu(), BF, what)
