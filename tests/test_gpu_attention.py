@@ -732,3 +732,22 @@ def test_attention_of_sequences_without_keys(lens_q, lens_k, hq, hk, tiles):
                 assert_close(got, ref, torch.bfloat16, what)
             assert_close(r[5][i, :, :n], lo[0], torch.float32, "lse")
         aq, ak = aq + n, ak + m
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("lens,hq,causal,rows", [([1100], 32, False, 128), ([2689], 20, True, 128), ([1024, 1001], 64, True, 256)])
+@pytest.mark.parametrize("growth", [12.0, -12.0])
+def test_attention_forward_when_scores_grow_in_every_form(dtype, lens, hq, causal, rows, growth):
+    """The reference of the exponentials moves in both types, and in two splits of the keys each by itself."""
+    from dhellam_amd import _Clib
+    assert _tiles(lens, lens, hq, 4, causal)[0] == rows
+    q, k, v, _ = (t.cpu() for t in _draw(dtype, lens, lens, hq, 4, 104))
+    ramp = torch.cat([torch.linspace(0, abs(growth), n) for n in lens])
+    k = ((ramp.flip(0) if growth < 0 else ramp) + 1)[:, None, None].mul(k.float()).to(dtype)
+    q[::3] = 0
+    cu, n, scale = _cu(lens), max(lens), 1.0 / math.sqrt(128)
+    res = _Clib.pymha_varlen_fwd(q.cuda(), k.cuda(), v.cuda(), cu.cuda(), cu.cuda(), n, n, 0.0, scale, causal, False, 0, False)
+    oo, lo = OA.attn_fwd(q, k, v, cu, cu, scale, causal, torch.float32)
+    assert_close(res[0], oo, dtype, "out")
+    for i, m in enumerate(lens):
+        assert_close(res[5][i, :, :m], lo[i, :, :m], torch.float32, "lse")
