@@ -53,6 +53,7 @@ __device__ __forceinline__ void dq_tile_body(const AttnBwdParams &p, int bx, int
   const int64_t cp_stride = cp_v ? p.v_stride : p.k_stride;
   const T *cp_g = reinterpret_cast<const T *>(cp_v ? p.v : p.k) + (int64_t)k0 * cp_stride + (int64_t)hkv * D;
   const TileCopy<D> cl = tile_copy<D>(lane, (uint32_t)(cp_stride * (int64_t)sizeof(T)));
+  const int cp_whole = tile_whole_rows(sk, cp_stride);
   const uint32_t cp_dst = lds0 + (uint32_t)(cp_v * SPLIT * TILEB + cp_sp * TILEB + cp_r0 * D * (int)sizeof(T));
 
   int nk_end = sk;
@@ -61,7 +62,7 @@ __device__ __forceinline__ void dq_tile_body(const AttnBwdParams &p, int bx, int
   const int niter = (ntiles + SPLIT - 1) / SPLIT;
   auto issue = [&](int it) {
     const int tile = it * SPLIT + cp_sp;
-    if (tile < ntiles) copy_tile<T, D, RPW>(cp_g, cp_stride, tile * BN + cp_r0, sk, cp_dst + (uint32_t)((it & 1) * STAGEB), cl, lane);
+    if (tile < ntiles) copy_tile<T, D, RPW>(cp_g, cp_stride, tile * BN + cp_r0, sk, cp_whole, cp_dst + (uint32_t)((it & 1) * STAGEB), cl, lane);
   };
   if (niter > 0) issue(0);
 
@@ -236,6 +237,7 @@ __device__ __forceinline__ void dkv_tile_body(const AttnBwdParams &p, int bx, in
   const int64_t cp_stride = cp_do ? p.do_stride : p.q_stride;
   const T *cp_g = reinterpret_cast<const T *>(cp_do ? p.dout : p.q) + (int64_t)q0 * cp_stride;
   const TileCopy<D> cl = tile_copy<D>(lane, (uint32_t)(cp_stride * (int64_t)sizeof(T)));
+  const int cp_whole = tile_whole_rows(sq, cp_stride);
   const uint32_t cp_dst = lds0 + (uint32_t)((cp_sp * 2 + cp_do) * TILEB);
 
   const int i_begin = causal ? j0 : 0;
@@ -247,7 +249,7 @@ __device__ __forceinline__ void dkv_tile_body(const AttnBwdParams &p, int bx, in
   auto issue = [&](int slot) {
     const int tq = si * QSPLIT + cp_sp, row0 = i_begin + tq * BM;
     if (tq < ntq) {
-      copy_tile<T, D, BM>(cp_g + (int64_t)(h_first + gi) * D, cp_stride, row0, sq, cp_dst + (uint32_t)(slot * STAGEB), cl, lane);
+      copy_tile<T, D, BM>(cp_g + (int64_t)(h_first + gi) * D, cp_stride, row0, sq, cp_whole, cp_dst + (uint32_t)(slot * STAGEB), cl, lane);
       const float *src = ld_g + ((int64_t)b * p.hq + (h_first + gi)) * p.ld2_pitch + row0;
       asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off"
                    : : "v"(src), "s"(lds0 + (uint32_t)(slot * STAGEB + QSPLIT * 2 * TILEB + (cp_sp * 2 + cp_do) * 256)) : "memory", "m0");

@@ -57,6 +57,7 @@ __global__ void __launch_bounds__(64 * RG * SPLIT, WPS) attn_fwd_tile_kernel(con
   const int64_t cp_stride = cp_v ? p.v_stride : p.k_stride;
   const T *cp_g = reinterpret_cast<const T *>(cp_v ? p.v : p.k) + (int64_t)k0 * cp_stride + (int64_t)hkv * D;
   const TileCopy<D> cl = tile_copy<D>(lane, (uint32_t)(cp_stride * (int64_t)sizeof(T)));
+  const int cp_whole = tile_whole_rows(sk, cp_stride);
   const uint32_t cp_dst = lds0 + (uint32_t)(cp_v * SPLIT * TILEB + cp_sp * TILEB + cp_r0 * D * (int)sizeof(T));
 
   const int wrow0 = m0 + rg * 32, row_q = wrow0 + c;
@@ -82,7 +83,7 @@ __global__ void __launch_bounds__(64 * RG * SPLIT, WPS) attn_fwd_tile_kernel(con
 
   auto issue = [&](int it) {
     const int tile = it * SPLIT + cp_sp;
-    if (tile < ntiles) copy_tile<T, D, RPW>(cp_g, cp_stride, tile * BN + cp_r0, sk, cp_dst + (uint32_t)((it & 1) * STAGEB), cl, lane);
+    if (tile < ntiles) copy_tile<T, D, RPW>(cp_g, cp_stride, tile * BN + cp_r0, sk, cp_whole, cp_dst + (uint32_t)((it & 1) * STAGEB), cl, lane);
   };
   if (niter > 0) issue(0);
   if constexpr (D < 256 || RG == 2) loaded_here(Qf);        // (more of them would be spilled in the 128-row form at 256)

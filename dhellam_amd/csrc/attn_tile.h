@@ -46,11 +46,13 @@ template <int D> __device__ __forceinline__ TileCopy<D> tile_copy(int lane, uint
   return c;
 }
 // Rows row0 .. row0 + ROWS - 1 of `g` (ROWS and the tile row at `dst` multiples of 16) to LDS byte address `dst`; `rows`:
-// rows of the sequence, later ones repeat the last.  Rows past the reach of the lane offsets are addressed one by one.  The copies are not counted by the compiler (dma_wait_all).
+// rows of the sequence, later ones repeat the last; `whole`: the rows that the lane offsets reach (tile_whole_rows), others
+// are addressed one by one.  The copies are not counted by the compiler (dma_wait_all).
+__device__ __forceinline__ int tile_whole_rows(int rows, int64_t stride) { return stride <= TILE_MAX_STRIDE ? rows : 0; }
 template <typename T, int D, int ROWS>
-__device__ __forceinline__ void copy_tile(const T *g, int64_t stride, int row0, int rows, uint32_t dst, const TileCopy<D> &c, int lane) {
+__device__ __forceinline__ void copy_tile(const T *g, int64_t stride, int row0, int rows, int whole, uint32_t dst, const TileCopy<D> &c, int lane) {
   constexpr int PAT = AttnTile<D>::PAT;
-  if (row0 + ROWS <= rows && stride <= TILE_MAX_STRIDE) {
+  if (row0 + ROWS <= whole) {
     const char *src = reinterpret_cast<const char *>(g + (int64_t)row0 * stride);
 #pragma unroll
     for (int q = 0; q < ROWS / 16; ++q) {
