@@ -21,9 +21,10 @@ namespace dh {
 // left to the compiler the loop took 3020 cycles with 32x32x16 and 3300 with 16x16x32, but 245 us (1.63 GHz) and 228 (1.9 GHz).
 // dK/dV of 32 query / 8 kv heads, 4096 rows x 2048 keys 300 -> 211 us (1.30 PFLOP/s at 1.5 GHz), causal 4096 304 -> 213, 8 / 1 heads x
 // 4096 keeping dS 95 -> 77, seven packed sequences of 1 to 3324 tokens 444 -> 300.
-// Rows past the sequence are zeros in LDS (buffer descriptors) and in the lse / delta planes, and their scores are masked: P = 1 would meet
-// dO = 0 as well, but the score of such a row and a key that holds an infinity is none.  Key blocks that no row of a tile sees get no
-// products: a row's dO that is not finite reaches dV and dK of the keys in its block of 32 and before, no further.
+// Rows past the sequence are zeros in LDS (buffer descriptors) and in the lse / delta planes: P = 1 there meets dO = 0, and dS = 0.
+// Where a key may have no other row (the diagonal's tiles) they are masked: the score of a row of zeros and a key that holds an
+// infinity is none.  Key blocks that no row of a tile sees get no products: a row's dO that is not finite reaches dV and dK of the
+// keys in its block of 32 and before, no further.
 // The wavefronts' partial sums go through LDS and are added in the order of the wavefronts.
 template <typename T, bool STORE_DS>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) attn_bwd_dkv128_kernel(const AttnBwdParams p) {
@@ -121,8 +122,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
     const int64_t qwrap = (int64_t)ROWB - (int64_t)ntq * BM * q_rowb, dwrap = (int64_t)ROWB - (int64_t)ntq * BM * do_rowb;
     const int64_t lwrap = ((int64_t)p.ld2_pitch - (int64_t)ntq * BM) * 4;
     const uint32_t ldbytes = (uint32_t)(p.ld2_plane * 4) + 128u, q16 = 16u * q_rowb, d16 = 16u * do_rowb;
-    // tiles with scores to mask: the first two of a causal one, and the one that the rows end in
-    const int rows = sq - i_begin, mct = causal ? 2 : 0, pct = (rows & (BM - 1)) != 0 && p.scale_log2 > 0.f ? ntq - 1 : -1;
+    // tiles with scores to mask: the first two of a causal one; and which of them the rows end in
+    const int rows = sq - i_begin, mct = causal ? 2 : 0, pct = (rows & (BM - 1)) != 0 ? ntq - 1 : -1;
     {
       const int left = rows - ct * BM < BM ? rows - ct * BM : BM;
       const int4s rsq = rows_rsrc(qp, rem > 0 ? (uint32_t)(left - 1) * q_rowb + ROWB : 0u);

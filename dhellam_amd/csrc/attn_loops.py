@@ -269,15 +269,37 @@ class DKV:
                 self.x.put(line)
 
     def mask(self, i):
-        """Out of line: scores past the diagonal, of rows past the end (their Q is 0, but 0 times an infinity is none) and, where dS is
-        kept, of keys past the end become -inf.  The first tile of a causal one has 32 keys that no row of it sees: no products of theirs."""
+        """Out of line: scores past the diagonal and, where dS is kept, of keys past the end become -inf.  So do those of rows past the
+        end: their Q is 0, but a key that no row sees may hold what 0 times it is none (keys that some row sees lie in other tiles too, and
+        made dQ of that row none there).  The first tile of a causal one has 32 keys that no row of it sees: no products of theirs."""
         x = self.x
         self.label("MASK%d" % i)
         x.put("s_nop 15")
         x.put("s_nop 7")
         diag, rows = v(self.E), v(self.E + 1)
         x.put("v_mov_b32 %s, 0xff800000" % v(self.NEG))
+        if self.store_ds:
+            x.put("s_cmp_eq_u32 %[dsmask], 0")
+            x.put("s_cbranch_scc1 %s" % self.ref("KEYS%d" % i))
+            for kb in range(4):
+                x.put("v_cmp_le_i32 vcc, %d, %%[vy]" % (-16 * kb))
+                x.put("s_nop 1")
+                for qb in range(2):
+                    for e in range(4):
+                        r = v(self.S + 4 * (4 * qb + kb) + e)
+                        x.put("v_cndmask_b32 %s, %s, %s, vcc" % (r, r, v(self.NEG)))
+            self.label("KEYS%d" % i)
+            x.put("s_cmp_ge_i32 %s, %%[mct]" % s(self.CTC))
+            x.put("s_cbranch_scc1 %s" % self.ref("MASKED%d" % i))
         x.put("s_lshl_b32 %s, %s, 5" % (s(self.T), s(self.CTC)))
+        x.put("v_subrev_u32 %s, %s, %%[vx]" % (diag, s(self.T)))
+        for qb in range(2):
+            for kb in range(4):
+                for e in range(4):
+                    r = v(self.S + 4 * (4 * qb + kb) + e)
+                    x.put("v_cmp_lt_i32 vcc, %d, %s" % (16 * qb + e - 16 * kb, diag))
+                    x.put("s_nop 1")
+                    x.put("v_cndmask_b32 %s, %s, %s, vcc" % (r, r, v(self.NEG)))
         x.put("s_cmp_lg_u32 %s, %%[pct]" % s(self.CTC))
         x.put("s_cbranch_scc1 %s" % self.ref("WHOLE%d" % i))
         x.put("v_add_u32 %s, %s, %%[vz]" % (rows, s(self.T)))
@@ -292,27 +314,6 @@ class DKV:
                     r = v(self.S + 4 * (4 * qb + kb) + e)
                     x.put("v_cndmask_b32 %s, %s, %s, %s" % (r, r, v(self.NEG), s(self.PADS + 2 * e, 2)))
         self.label("WHOLE%d" % i)
-        if self.store_ds:
-            x.put("s_cmp_eq_u32 %[dsmask], 0")
-            x.put("s_cbranch_scc1 %s" % self.ref("KEYS%d" % i))
-            for kb in range(4):
-                x.put("v_cmp_le_i32 vcc, %d, %%[vy]" % (-16 * kb))
-                x.put("s_nop 1")
-                for qb in range(2):
-                    for e in range(4):
-                        r = v(self.S + 4 * (4 * qb + kb) + e)
-                        x.put("v_cndmask_b32 %s, %s, %s, vcc" % (r, r, v(self.NEG)))
-            self.label("KEYS%d" % i)
-        x.put("s_cmp_ge_i32 %s, %%[mct]" % s(self.CTC))
-        x.put("s_cbranch_scc1 %s" % self.ref("MASKED%d" % i))
-        x.put("v_subrev_u32 %s, %s, %%[vx]" % (diag, s(self.T)))
-        for qb in range(2):
-            for kb in range(4):
-                for e in range(4):
-                    r = v(self.S + 4 * (4 * qb + kb) + e)
-                    x.put("v_cmp_lt_i32 vcc, %d, %s" % (16 * qb + e - 16 * kb, diag))
-                    x.put("s_nop 1")
-                    x.put("v_cndmask_b32 %s, %s, %s, vcc" % (r, r, v(self.NEG)))
         x.put("s_cmp_lg_u32 %s, 0" % s(self.CTC))
         x.put("s_cbranch_scc1 %s" % self.ref("MASKED%d" % i))
         x.pad = True
@@ -398,8 +399,6 @@ class DKV:
             if m == 20:                                        # whether this tile has scores to mask: vcc for the branch at 32
                 x.put("s_cmp_lt_i32 %s, %%[mct]" % s(self.CTC))
                 x.put("s_cselect_b64 vcc, -1, 0")
-                x.put("s_cmp_eq_u32 %s, %%[pct]" % s(self.CTC))
-                x.put("s_cselect_b64 vcc, -1, vcc")
                 if self.store_ds:
                     x.put("s_cmp_lg_u32 %[dsmask], 0")
                     x.put("s_cselect_b64 vcc, -1, vcc")
