@@ -3,6 +3,8 @@
 #include "attn_loops.inc"
 #include "attn_rows.h"
 
+#include <type_traits>
+
 namespace dh {
 
 // A workgroup of four wavefronts owns 64 key rows; each wavefront holds all of them (dK and dV: 256 accumulator registers, V: 64
@@ -186,21 +188,31 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
 #undef DH_ACC4
     __syncthreads();                                  // everyone is done with the tiles
 
-    // add the wavefronts' partial sums in their order: wavefront w ends up with key block w
+    // add the wavefronts' partial sums in their order: wavefront w ends up with key block w.  (Those without a tile have none: 1 MB less
+    // through LDS where sequences are a tile or two long.)
+    const int nact = total < NW ? (total > 1 ? total : 1) : NW;
     typedef __attribute__((address_space(3))) floatx4 *lds_f4;
     auto sum_up = [&](const floatx4 (&acc)[4][8], floatx4 (&sum)[8]) {
       const lds_f4 dst = (lds_f4)(lds0 + (uint32_t)w * 32768u) + lane;
+      if (w < nact) {
 #pragma unroll
-      for (int kb = 0; kb < 4; ++kb)
+        for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
-        for (int t = 0; t < 8; ++t) dst[64 * (8 * kb + t)] = acc[kb][t];
-      __syncthreads();
-#pragma unroll
-      for (int x = 0; x < NW; ++x) {
-        const lds_f4 src = (lds_f4)(lds0 + (uint32_t)x * 32768u + (uint32_t)w * 8192u) + lane;
-#pragma unroll
-        for (int t = 0; t < 8; ++t) sum[t] = x == 0 ? src[64 * t] : sum[t] + src[64 * t];
+          for (int t = 0; t < 8; ++t) dst[64 * (8 * kb + t)] = acc[kb][t];
       }
+      __syncthreads();
+      auto add = [&](auto parts) {
+#pragma unroll
+        for (int x = 0; x < decltype(parts)::value; ++x) {
+          const lds_f4 src = (lds_f4)(lds0 + (uint32_t)x * 32768u + (uint32_t)w * 8192u) + lane;
+#pragma unroll
+          for (int t = 0; t < 8; ++t) sum[t] = x == 0 ? src[64 * t] : sum[t] + src[64 * t];
+        }
+      };
+      if (nact == NW) add(std::integral_constant<int, NW>());
+      else if (nact == 3) add(std::integral_constant<int, 3>());
+      else if (nact == 2) add(std::integral_constant<int, 2>());
+      else add(std::integral_constant<int, 1>());
       __syncthreads();
     };
     floatx4 sK[8], sV[8];
