@@ -28,23 +28,18 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
   __shared__ float sM[4][64], sN[4][64], sL[4][64];    // of each row: reference, sum of P as rounded and sum of P
   rng_state_zero(p);
 
-  const int b = __builtin_amdgcn_readfirstlane(seq_by_length(p.cu_q, gridDim.y, blockIdx.y));
-  // the query heads of one kv head read the same K / V rows: keep a kv head on one XCD's L2
-  const int ratio = p.hq / p.hk, P = gridDim.x / p.hq;
-  int hkv, item;
-  xcd_group_item(blockIdx.x, p.hk, ratio * P, hkv, item);
-  const int h = hkv * ratio + item / P, px = item % P;
+  const RowWork work = row_work<BM>(p.cu_q, p.q_shift, p.max_sq, p.hq, p.hk, p.causal);
+  if (work.b < 0) return;
+  const int b = __builtin_amdgcn_readfirstlane(work.b), h = __builtin_amdgcn_readfirstlane(work.h), px = __builtin_amdgcn_readfirstlane(work.px);
+  const int hkv = __builtin_amdgcn_readfirstlane(work.hkv);
   const int q0 = p.cu_q[b] >> p.q_shift, sq = (p.cu_q[b + 1] >> p.q_shift) - q0;
   const int k0 = p.cu_k[b] >> p.k_shift, sk = (p.cu_k[b + 1] >> p.k_shift) - k0;
   const int nqt = (sq + BM - 1) / BM;
   const int causal = p.causal;
   int qt0 = px, qt1 = 0, nq = 1;
   if (causal) {
-    if (2 * px >= nqt) return;
     qt0 = nqt - 1 - px; qt1 = px;
     nq = qt0 == qt1 ? 1 : 2;
-  } else if (px >= nqt) {
-    return;
   }
   const int tid = threadIdx.x;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
