@@ -21,6 +21,7 @@
 // needs no fp32 dQ accumulator in memory and no atomics.
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 
 #include "attn_route.h"
 #include "mma.h"
@@ -853,15 +854,34 @@ static BwdBoth bwd_both(int batch, int max_sq, int max_sk, int64_t total_q, int6
   return {t >= (double)cdiv(b, 256) * rho && room(t) >= a, hs};
 }
 
-// Workgroups of recomputing dQ with work, tiles of `rows`.  The kernel with one wavefront a SIMD takes them where they come to four fifths of
-// the compute units, in tiles of 256 rows (K and V are read once for four wavefronts) or else of 128: its loop is the faster one
-// (1860 and 1915 cycles for what took 3400), but a tile's rows are loaded and stored in 24000, which the kernel of eight wavefronts
-// hides better where little follows.  Whole backward, us, eight wavefronts / 128 / 256 rows, causal unless said: 32 query / 8
-// kv heads x 4096 469 / 409 / 381, x 2048 (128 tiles of 256) 159 / 148 / 176, 8 x 1024 331 / 331 / 297, 16 x 512 243 / 255 / 229, not causal 16 heads x
-// 2048 141 / 125 / 142, 2786 + 479 (208 tiles) 277 / 240 / 220, 8 / 1 x 4096 237 / 203 / 242, 1022 to 223 (88 and 160 tiles) 80 / 87 / 93.
-static int64_t dq_wgs(int rows, int max_sq, int hq, int batch, int causal, int64_t total_q) {
-  const int64_t bound = (int64_t)batch * max_sq, q = total_q < bound ? total_q : bound;
-  return (int64_t)((double)attn_wgs(max_sq, rows, hq, batch, causal) * (double)q / (double)bound);
+// Query rows of a tile of recomputing dQ where 128-row tiles fill the chip: 256 or 128 on one wavefront a SIMD, or 0: 128 on eight wavefronts.
+// What ends first by this count, in thousands of cycles: a tile's rows are loaded and stored in 15 and 16.5 where the eight wavefronts take
+// 9, a tile of 32 keys takes 1.9 for 256 rows or, in two splits, 0.96 for 128 (eight wavefronts 1.8); workgroups run in rounds of 256, a
+// last one that is not full ends sooner, and those of several lengths fill each other's (not causal: 6 % better on one wavefront than the count
+// says).  Fitted to 504 whole backward calls of random sizes that the forms tell apart: 1.0 % slower than the best of the three, none slower
+// than on eight wavefronts throughout; a line at 208 workgroups of either tile was 4.3 % and 27.  us, eight wavefronts / 128 / 256 rows, not
+// causal: 16 query / 4 kv heads x 12 x 140 46 / 47 / 36, 64 / 8 x 32 of up to 183 271 / 247 / 212, 32 / 8 x 5 x 908 273 / 261 / 250, 64 / 8 x 24 x 56
+// 71 / 89 / 92, 32 / 32 x 16 x 56 39 / 47 / 49; causal: 32 / 32 x 12 of up to 1591 851 / 819 / 781, 64 / 8 x 8 x 631 350 / 365 / 363, 24 / 8 x 24 x 765 513 / 526 / 539.
+static int dq_rows(int max_sq, int max_sk, int64_t total_q, int64_t total_k, int hq, int batch, int causal) {
+  const double bound = (double)batch * max_sq, q = (double)total_q < bound ? (double)total_q : bound;
+  const bool ragged = 10 * q < 9 * bound;
+  auto cycles = [&](int rows, double ends, double tile) {
+    const int64_t t = cdiv(max_sq, rows);
+    double wgs = (double)attn_wgs(max_sq, rows, hq, batch, causal), keys = (double)max_sk / 32;
+    if (ragged) wgs = std::min(wgs, (causal ? (q / rows + batch) / 2 : q / rows + 0.5 * batch) * hq);
+    if (causal) {                                     // of two tiles i and n - 1 - i, or of the only one
+      keys = (double)((t > 1 ? t + 1 : 1) * rows / 32 - (t * rows - max_sq) / 32);
+      if (ragged) keys = std::min(keys, (1.5 * q / batch + rows) / 32);
+      if (t > 1) ends *= 2;
+    } else if (ragged) {
+      keys = (double)total_k / batch / 32;
+    }
+    const double x = wgs / 256;
+    return (x <= 1 ? 1 : ragged ? x + 0.05 : 0.5 * std::ceil(x) + 0.5 * x) * (ends + keys * tile);
+  };
+  const double one = ragged && !causal ? 0.94 : 1;
+  const double w8 = cycles(128, 9.0, 1.8), w4 = one * cycles(256, 15.0, 1.86), w2 = one * cycles(128, 16.5, 0.96);
+  return w8 <= w4 && w8 <= w2 ? 0 : w4 <= w2 ? 256 : 128;
 }
 
 // What one 16-bit call runs.
@@ -885,12 +905,7 @@ static AttnBwdRoute attn_bwd_route(int batch, int max_sq, int max_sk, int64_t to
   const bool fills = d <= 128 && dq_tile_fills(max_sq, hq, batch);
   r.both = both.pays && (d == 128 || !fills);
   r.big_dq = r.hand_dq ? big : fills && !r.both;
-  const bool ragged = !causal && 10 * total_q < 9 * (int64_t)batch * max_sq;
-  r.dq_rows = 0;
-  if (r.hand_dq && big && (!ragged || attn_long_rows(total_q, batch))) {
-    if (dq_wgs(256, max_sq, hq, batch, causal, total_q) >= 208 && (!ragged || attn_ragged_fills(hq, batch, total_q))) r.dq_rows = 256;
-    else if (dq_wgs(128, max_sq, hq, batch, causal, total_q) >= 208) r.dq_rows = 128;
-  }
+  r.dq_rows = r.hand_dq && big ? dq_rows(max_sq, max_sk, total_q, total_k, hq, batch, causal) : 0;
   r.hsplit = r.both ? both.hsplit : bwd_hsplit(max_sk, batch, hq, hk, d == 128 && causal);
   return r;
 }

@@ -680,11 +680,11 @@ def _tiles(lens_q, lens_k, hq, hk, causal):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("lens_q,lens_k,hq,hk,causal,fwd,dq", [
-    ([1100], [333], 32, 8, False, 0, 128),                     # two splits of an odd number of key tiles
-    ([1100], [20], 32, 8, False, 0, 128),                      # a second split without a key
-    ([1100, 1090], [40, 31], 16, 8, False, 0, 128),
-    ([1100], [1100], 32, 32, False, 128, 128),
+    ([2048], [333], 16, 8, False, 0, 128),                     # two splits of an odd number of key tiles
+    ([1024, 1019], [333, 20], 16, 8, False, 0, 128),           # a second split without a key
+    ([2000], [2000], 16, 16, False, 128, 128),
     ([700], [2000], 44, 44, False, 128, 128),                  # by the number of keys
+    ([1100], [45], 32, 8, False, 0, 256),
     ([512, 491], [512, 491], 64, 64, True, 0, 128),
     ([961], [961], 64, 8, True, 0, 128),                       # odd numbers of tiles behind the diagonal
     ([600], [20], 32, 8, False, 128, 0),
@@ -703,7 +703,7 @@ def test_attention_query_tiles_on_one_wavefront_a_simd(dtype, lens_q, lens_k, hq
 
 
 @pytest.mark.parametrize("lens_q,lens_k,hq,hk,tiles", [
-    ([600, 600], [0, 333], 16, 4, (128, 0)), ([1100, 1090], [40, 0], 32, 8, (0, 256)), ([1100, 1090], [40, 0], 16, 8, (0, 128)),
+    ([600, 600], [0, 333], 16, 4, (128, 0)), ([1024, 1019], [333, 0], 16, 8, (0, 128)),
     ([767] * 4, [37, 0, 640, 33], 32, 4, (256, 256)),
 ])
 def test_attention_of_sequences_without_keys(lens_q, lens_k, hq, hk, tiles):

@@ -247,7 +247,7 @@ def test_attention_of_keys_too_far_apart_for_one_wavefront_a_simd(stride):
     _need(14)
     n, m, hq, hk, d = 1100, 45, 32, 8, 128
     lib = _lib.load()
-    assert lib.dh_attn_fwd_rows(1, 600, m, 600, hq, d, 0) == 128 and lib.dh_attn_bwd_dq_rows(1, n, m, n, m, hq, hk, d, 0, 0) == 128
+    assert lib.dh_attn_fwd_rows(1, 600, m, 600, hq, d, 0) == 128 and lib.dh_attn_bwd_dq_rows(1, n, m, n, m, hq, hk, d, 0, 0) == 256
     held = torch.empty(m * stride, dtype=BF, device="cuda")
     far = [held.as_strided((m, hk, d), (stride, d, 1), at * d) for at in (0, hk)]
     near = [_randn((m, hk, d), 40 + i) for i in range(2)]
