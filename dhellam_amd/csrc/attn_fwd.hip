@@ -448,18 +448,19 @@ struct AttnFwdRoute {
 
 // Query rows of a tile where the kernel with one wavefront a SIMD is the faster one at head dim 128 (else 0).  Its loop takes 1740 cycles
 // for what took 2900, but its tiles are larger, so it depends on what of the chip they leave empty: places in the last round
-// of 256 workgroups, rows past the end, an odd tile without its pair.  us, before / here, 32 query heads, causal unless said:
-//   256 rows, one length, 70 % of the places: 4096 (256 workgroups) 199 / 144, 8 x 1024 141 / 124, 16 x 512 106 / 99, 12 heads x 8192 (192) 294 /
-//     215, not causal 2048 (256) 84 / 66, 4096 x 2048 keys 183 / 131, x 64 keys 40 / 32; less: 2048 (128) 53 / 81, 12 heads x 5000 (120) 127 /
-//     148, 27 x 300 119 / 142, 128 heads x 700 (three tiles, 256) 44 / 54.
-//   256 rows, several lengths: two rounds of real work, four fifths of one where nothing is causal (no pairs of a long and a short
-//     tile that one long sequence keeps apart): documents of 1 to 3324 tokens (552) 248 / 203; 3000 + 2 x 1000 (320) 154 / 159, 1694 + 925 +
-//     949 (270) 83 / 114; not causal, 16 heads, 2786 + 479 (206) 101 / 82, 8 heads, 1022 to 223 (72) 27 / 34.
-//   128 rows (two splits of the keys) where those are too few.  Causal: long rows and full rounds, 16 heads x 4096 (256) 91 / 84, 12
-//     heads x 5000 (240) 131 / 92, 8 x 8192 157 / 138, but 32 x 2048 (256) 54 / 55, 16 x 3000 (192) 62 / 64.  Not causal: against 64-row tiles
-//     where those are more than a round, 32 x 600 (160) 28 / 20, 600 x 100 keys 18 / 14, 16 x 1100 (144) 37 / 26, but 8 x 2048 (128) 29 / 36, 512 x 8192
-//     keys (128) 98 / 111; against 128-row tiles from 1024 keys on, 16 x 2048 (256) 44 / 42, but x 512 keys 18 / 19, x 64 10 / 13; several
-//     lengths 2786 + 479 (412) 106 / 93, 8 heads, 1022 to 223 (144) 27 / 30.
+// of 256 workgroups, rows past the end, an odd tile without its pair.  us, other kernels / here (128-row tiles where three are given), causal
+// unless said:
+//   256 rows, one length, 70 % of the places: 32 heads x 3377 (224 workgroups) 128 / 112, 4 x 3 x 8185 (192) 282 / 207, 64 x 2 x 1851 (512) 172 / 160, 32 x 24
+//     x 835 386 / 343, not causal 24 x 24 x 658 270 / 206, 8 x 6805 (216) 210 / 167; less: 32 x 2641 (192, 86 % of them used) 85 / 92, 8 x 32 x 627 (512, 61 %) 82 / 98.
+//     Where a second round is half empty 128-row tiles fill theirs better, or nothing does: 64 x 3003 (384) 182 / 201 / 178, 12 x 4 x 3823 215 / 236 / 203, not
+//     causal 4 x 5 x 4799 (380) 246 / 250 / 220, 24 x 5 x 1511 (360) 116 / 132 / 120.  Within the rule and slower: 40 x 6 x 1633 254 / 277, 40 x 8 x 998 157 / 167.
+//   256 rows, several lengths: two rounds of real work, four fifths of one where nothing is causal; causal rows of 430 on average:
+//     64 heads, 8 of 558 193 / 129, 32 x 16 of 720 235 / 184, 16 x 24 of 593 151 / 136, but 16 x 32 of 395 103 / 119, 16 x 32 of 420 108 / 119.
+//   128 rows (two splits of the keys) where those are too few.  Causal: long rows and full rounds, 32 x 2 x 2702 (704) 170 / 168, 12 x 4 x 3602 206 / 197. Not
+//     causal: against 64-row tiles where those are more than a round, 32 x 602 (160) 26 / 19, 600 x 100 keys 18 / 14, 12 x 1363 (132 of 128 rows, 264 of
+//     64) 39 / 27, but 12 x 1284 (132, 252) 21 / 27, 8 x 2048 (128) 29 / 36, and of 31 random ones 16 x 2 x 534 rows x 2730 keys 39 / 43; against 128-row tiles from 1024 keys on,
+//     64 x 1520 97 / 90, but 16 x 2048 x 512 keys 18 / 19; several lengths 2786 + 479 (412) 106 / 93, 8 heads, 1022 to 223 (144) 27 / 30.
+// Of 600 random calls 7 are slower here than on the other kernels: five causal ones with an odd number of tiles by 7 to 11 %, 8 x 2 of up to 1261 rows 24 / 29.
 static int fwd_rows(int max_sq, int max_sk, int hq, int batch, int64_t total_q, int causal) {
   if (max_sq < 512) return 0;
   const int64_t bound = (int64_t)batch * max_sq, rows = total_q < bound ? total_q : bound;
@@ -468,11 +469,12 @@ static int fwd_rows(int max_sq, int max_sk, int hq, int batch, int64_t total_q, 
   if (10 * rows >= 9 * bound) {
     const int t = (max_sq + 255) / 256;
     const double used = (causal ? (double)t / (2 * ((t + 1) / 2)) : 1.0) * (double)max_sq / (256.0 * t);
-    if (fill(n) * used >= 0.7) return 256;
+    if (fill(n) * used >= 0.7 && (n <= 256 || fill(n) >= 0.76 || (!causal && max_sk < 1024))) return 256;
     if (causal) return max_sq >= 2560 && max_sk >= 1024 && fill(n2) >= 0.85 ? 128 : 0;
-    return n2 > 128 && (n2 < ATTN_128ROW_MIN_WG || max_sk >= 1024) ? 128 : 0;
+    if (n2 >= ATTN_128ROW_MIN_WG) return max_sk >= 1024 ? 128 : 0;
+    return n2 > 128 && attn_wgs(max_sq, 64, hq, batch, 0) > 256 ? 128 : 0;
   }
-  if (!causal && !attn_long_rows(rows, batch)) return 0;
+  if (causal ? rows < 430ll * batch : !attn_long_rows(rows, batch)) return 0;
   const double share = (double)rows / (double)bound;
   if ((double)n * share >= (causal ? 512 : 208) && (causal || attn_ragged_fills(hq, batch, rows))) return 256;
   return !causal && max_sk >= 1024 && (double)n2 * share >= 384 ? 128 : 0;

@@ -79,6 +79,9 @@ def test_attention_route(batch, max_q, total_q, hq, causal, hand):
 @pytest.mark.parametrize("batch,max_q,max_k,total_q,hq,causal,fwd,dq", [
     (1, 4096, 4096, 4096, 32, 1, 256, 256), (1, 2048, 2048, 2048, 32, 1, 0, 128), (1, 2689, 2689, 2689, 20, 1, 128, 0),
     (1, 700, 2000, 700, 44, 0, 128, 128), (1, 700, 700, 700, 44, 0, 0, 256),                 # the forward by the number of keys
+    (1, 1284, 1284, 1284, 12, 0, 0, 0), (1, 1363, 1363, 1363, 12, 0, 128, 0), (6, 512, 512, 3072, 64, 1, 0, 256),          # the forward's rounds
+    (1, 3003, 3003, 3003, 64, 1, 128, 128), (5, 4799, 4799, 23995, 4, 0, 128, 128), (32, 605, 605, 12640, 16, 1, 0, 256),
+    (8, 812, 812, 4464, 64, 1, 256, 256),
     (1, 600, 333, 600, 32, 0, 128, 0), (0, 0, 0, 0, 8, 1, 0, 0), (1, 4096, 0, 4096, 32, 0, 256, 256),
     (5, 628, 628, 3140, 32, 1, 0, 128), (16, 512, 512, 8192, 16, 1, 256, 256), (8, 1024, 1024, 8192, 32, 1, 256, 256),     # dQ: rounds of work
     (8, 96, 96, 768, 32, 0, 0, 0), (12, 140, 140, 1680, 16, 0, 0, 256), (1, 2048, 333, 2048, 16, 0, 0, 128), (1, 2048, 20, 2048, 16, 0, 0, 0)])
