@@ -189,8 +189,9 @@ static bool gemm_f32_takes(const GemmF32 &g) {
 // 1024 rows, 5632 of 1024 (1408 tiles) 110 / 100, 2816 of 1024 (704) 69 / 53, 3072 (768) 55 / 54, data gradients [1024, 1024] x [1024,
 // 2816] 70 / 53, [1000, 256] x [256, 5568] (1392) 81 / 31, weight gradients 5632 x 1024 of 1024 rows 117 / 104, 1024 x 2816 70 / 54; but fewer
 // tiles, 1024 rows 1536 of 1024 (384) 32 / 37, 777 rows 2816 (572, 0.74 of the places) 45 / 54, a longer reduction 1024 rows, 4000 of
-// 2048 (1008, 0.66) 123 / 170, more tiles 1024 rows, 16032 of 1024 (4016) 262 / 300.  Random calls within the rule, library / here: 44 of three
-// forms 1.02 to 2.6, but two forwards 0.90 and 0.95.
+// 2048 (1008, 0.66) 123 / 170, more tiles 1024 rows, 16032 of 1024 (4016) 262 / 300, weight gradients of two rounds from 1281 rows on 3520 x
+// 1684 of 1504 rows 137 / 148.  350 random calls within the rule but for these, library / here on average: forwards 1.17, data gradients 1.16, weight gradients
+// 1.29; 9 of them below 0.97, the worst 0.90.
 // Weight gradients of few rows are launches more than products: up to 192 rows 1.5 times (80 calls, one 0.96), 64 rows 512 x 512 11 / 5; at 227
 // rows 4352 x 768 21 / 24.
 // The sums run along k in one chain, as the library's do in these ranges: errors against 64 bits are the same (5.7e-7 at k = 1024).
@@ -199,7 +200,7 @@ bool gemm_f32_pays(const GemmF32 &g) {
   const int64_t tiles = cdiv(g.rows, 64) * cdiv(g.cols, 64);
   if (tiles > 1536) return false;
   if (g.x_strided && g.k <= 192) return true;
-  return g.k <= (g.x_strided ? 1536 : 1024) && tiles >= 640 && 6 * tiles >= 5 * 768 * cdiv(tiles, 768);
+  return g.k <= (!g.x_strided ? 1024 : tiles > 768 ? 1280 : 1536) && tiles >= 640 && 6 * tiles >= 5 * 768 * cdiv(tiles, 768);
 }
 
 int launch_gemm_f32(const GemmF32 &g, void *stream) {

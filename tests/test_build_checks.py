@@ -115,6 +115,13 @@ def test_fp32_products_go_where_they_were_measured_the_faster(rows, cols, k, for
     assert _lib.load().dh_gemm_f32_path(cols, rows, k, form[0] == "T", form[1] == "T") == own
 
 
+@pytest.mark.parametrize("rows,k,own", [(5632, 1280, 1), (5632, 1281, 0), (2816, 1536, 1), (2816, 1537, 0)])
+def test_fp32_weight_gradients_of_two_rounds_end_sooner(rows, k, own):
+    """[rows, 1024] of k rows: 1408 and 704 tiles of 64 x 64."""
+    from dhellam_amd import _lib
+    assert _lib.load().dh_gemm_f32_path(1024, rows, k, 0, 1) == own
+
+
 @pytest.fixture(scope="module")
 def loops():
     import importlib.util
