@@ -751,3 +751,42 @@ def test_attention_forward_when_scores_grow_in_every_form(dtype, lens, hq, causa
     assert_close(res[0], oo, dtype, "out")
     for i, m in enumerate(lens):
         assert_close(res[5][i, :, :m], lo[i, :, :m], torch.float32, "lse")
+
+
+@pytest.mark.parametrize("lens,hq,hk,causal,bound,tiles", [
+    ([500 + i % 40 for i in range(65)], 8, 1, True, 540, (0, 256)),             # more sequences than are sorted
+    ([800 + i % 5 for i in range(65)], 8, 2, False, 804, (256, 256)),
+    ([100 + 7 * i for i in range(64)], 8, 8, True, 541, (0, 256)),              # as many as are
+    ([300, 0, 513, 769, 64, 1, 700, 257], 40, 40, True, 769, (0, 256)),         # one head a kv head, an empty sequence
+    ([785 - i for i in range(20)], 24, 8, True, 785, (256, 256)),               # odd numbers of tiles
+    ([785 - i for i in range(20)], 20, 20, True, 785, (0, 256)),                # kv heads that go round the XCDs
+    ([769 + i for i in range(12)], 40, 40, True, 780, (256, 256)),
+    ([600 + i % 9 for i in range(24)], 24, 8, True, 608, (0, 128)),
+    ([700, 300, 513, 1000, 640], 24, 8, False, 2048, (128, 256)),               # a bound that no sequence reaches
+    ([257, 1100, 1, 300, 700, 700], 48, 16, False, 1100, (256, 256)),
+])
+def test_attention_workgroups_of_several_lengths(lens, hq, hk, causal, bound, tiles):
+    """Every tile of every sequence and head is somebody's: kernels of one wavefront a SIMD count the workgroups that sequences have."""
+    from dhellam_amd import _Clib, _lib
+    lib, dtype, scale = _lib.load(), torch.bfloat16, 1.0 / math.sqrt(128)
+    sizes = len(lens), bound, bound, sum(lens)
+    assert (lib.dh_attn_fwd_rows(*sizes, hq, 128, causal), lib.dh_attn_bwd_dq_rows(*sizes, sum(lens), hq, hk, 128, causal, 0)) == tiles
+    q, k, v, do = _draw(dtype, lens, lens, hq, hk, 108)
+    cu = _cu(lens).cuda()
+    _Clib.set_attn_bwd_ds_limit(0)
+    try:
+        r = _Clib.pymha_varlen_fwd(q, k, v, cu, cu, bound, bound, 0.0, scale, causal, False, 0, False)
+        got = _Clib.pymha_varlen_bwd(do, q, k, v, r[0], r[5], cu, cu, bound, bound, 0.0, scale, causal, None, True, 0, False,
+                                     torch.cuda.current_stream().cuda_stream)
+    finally:
+        _Clib.set_attn_bwd_ds_limit()
+    cpu = [t.cpu() for t in (do, q, k, v)]
+    oo, lo = OA.attn_fwd(*cpu[1:], cu.cpu(), cu.cpu(), scale, causal, torch.float32)
+    lse = torch.full((len(lens), hq, max(lens)), float("-inf"), dtype=torch.float64)
+    for i, n in enumerate(lens):
+        lse[i, :, :n] = r[5][i, :, :n].cpu().double()
+        assert_close(r[5][i, :, :n], lo[i, :, :n], torch.float32, "lse")
+        assert (got[3][i, :, n:] == 0).all()
+    want = OA.attn_bwd(*cpu, r[0].cpu(), lse, cu.cpu(), cu.cpu(), scale, causal, torch.float32)
+    for a, b, what in zip([r[0], *got[:3]], [oo, *want[:3]], ("out", "dq", "dk", "dv")):
+        assert_close(a, b, dtype, what)
