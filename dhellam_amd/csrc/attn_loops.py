@@ -6,14 +6,17 @@ a wavefront issues one instruction in about 5, so two or three others fit beneat
 in the wrong place is paid in full.  (Written as single asm statements the compiler puts an ``s_nop`` between any two of which one
 reads what the other wrote, 74 in a tile of 128 MFMAs: 10 % of the loop.)
 
-``Stream`` keeps the account that hand-written assembly gets wrong: it counts LDS reads in flight (they complete in order) and
-places the waits, and it refuses
+``Stream`` keeps the account of the loops' LDS reads, MFMAs and vector instructions (``lds``, ``mfma``, ``valu``): it counts reads in
+flight (they complete in order) and places the waits, and it refuses
   * an MFMA or vector instruction that reads a register whose LDS read nothing has waited for,
   * a vector instruction on the result of an MFMA with fewer than two MFMAs between them,
   * an MFMA on a register that a vector instruction wrote fewer than two instructions ago,
   * the result of a transcendental in the very next instruction,
   * an LDS read into a register that an earlier read has not filled yet,
   * an MFMA on a fragment that a later read has replaced.
+What goes out through ``put`` (masks, the moving reference, the code in front of and behind the loops) is not looked at and waits by
+``s_nop``.  Which stage of LDS a copy may fill is no matter of registers: ``tests/test_build_checks.py`` runs the finished text and
+checks that no copy goes to a stage that is still read, and no read to one that has not landed.
 """
 import re
 import sys
@@ -1045,7 +1048,7 @@ def define(name, lines):
 
 
 def clobbers(name, first_v, last_v, first_s, last_s, agprs=0):
-    names = ["a%d" % i for i in range(agprs)] + ["v%d" % i for i in range(first_v, last_v + 1)] + ["s%d" % i for i in range(first_s, last_s + 1)] + ["vcc", "memory"]
+    names = ["a%d" % i for i in range(agprs)] + ["v%d" % i for i in range(first_v, last_v + 1)] + ["s%d" % i for i in range(first_s, last_s + 1)] + ["vcc", "scc", "m0", "memory"]
     return "#define %s %s\n" % (name, ", ".join('"%s"' % n for n in names))
 
 

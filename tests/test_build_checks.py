@@ -1,4 +1,5 @@
 """Build-time checks that need no GPU."""
+import re
 import shutil
 
 import pytest
@@ -151,3 +152,102 @@ def test_attention_loops_refuse_what_the_hardware_would_not_wait_for(loops, faul
     x = loops.Stream("bf16")              # waited for, the reads that may be in flight are the younger ones
     x.lds("", 100, 4), x.lds("", 104, 4), x.wait({100})
     assert x.lines[-1] == "s_waitcnt lgkmcnt(1)" and x.reads == [set(range(104, 108))]
+
+
+def run_stages(lines, stage_bytes, shared, took, rounds=3):
+    """Runs a loop's text, following the branches whose label `took` names, and checks the stages of LDS: a copy goes to a stage whose reads have
+    all been waited for, and, where wavefronts share a stage, only past a barrier behind that; a read goes to a stage whose copies
+    have been waited for, and past a barrier behind that.  The first round only fills the books.  Returns the copies seen."""
+    at = {l[:-1]: i for i, l in enumerate(lines) if l.endswith(":")}
+    pc, back, seen, copies = at["LLOOP_%="], [], -1, 0
+    reads, copying = [], []                       # in flight, oldest first: stages (stores as None)
+    unread, landed, ready = set(), set(), set()   # read and not yet known to everyone; landed; landed and known to everyone
+    m0 = None
+    while True:
+        l = lines[pc]
+        pc += 1
+        if l == "LLOOP_%=:":
+            seen += 1
+            if seen == rounds:
+                return copies
+        if l.endswith(":"):
+            continue
+        op, _, rest = l.partition(" ")
+        label = rest.split()[-1] if rest else ""
+        if op == "s_branch" or (op.startswith("s_cbranch") and (label in ("LLOOP_%=", "LREST0_%=") or took(label, op))):
+            pc = at[label]
+            if label == "LREST0_%=":              # the rounds of a wavefront past its rows
+                seen += 1
+                if seen == rounds:
+                    return copies
+        elif op == "s_call_b64":
+            back.append(pc)
+            pc = at[label]
+        elif op == "s_setpc_b64":
+            pc = back.pop()
+        elif op == "s_waitcnt":
+            for kind, n in re.findall(r"(vmcnt|lgkmcnt)\((\d+)\)", rest):
+                queue = copying if kind == "vmcnt" else reads
+                done, queue[:] = queue[:max(0, len(queue) - int(n))], queue[max(0, len(queue) - int(n)):]
+                if kind == "vmcnt":
+                    landed |= {s for s in done if s is not None and s not in queue}
+                if not shared:
+                    ready = set(landed)
+        elif op == "s_barrier":
+            ready, unread = set(landed), set(reads)
+        elif op == "s_add_u32" and rest.startswith("m0, "):
+            m0 = int(rest.split(", ")[2]) // stage_bytes
+        elif op.startswith("buffer_load"):
+            if seen > 0:
+                assert m0 not in reads and (not shared or m0 not in unread), ("copied over while it is read", m0, lines[pc - 4:pc])
+                copies += 1
+            copying.append(m0)
+            landed.discard(m0), ready.discard(m0)
+        elif op.startswith("global_store"):
+            copying.append(None)
+        elif op.startswith("ds_read") and "%[rk" in rest and not shared:
+            reads.append(None)                    # the K tile, which stays
+        elif op.startswith("ds_read"):
+            stage = int((re.findall(r"offset:(\d+)", rest) or ["0"])[0]) // stage_bytes
+            if seen > 0:
+                assert stage in ready, ("read before it has landed", stage, lines[pc - 4:pc])
+            reads.append(stage)
+            if shared:
+                unread.add(stage)
+
+
+def _loop(loops, kind, form):
+    x = {"fwd": loops.FWD, "dq": loops.DQ, "dkv": loops.DKV}[kind]("bf16", form)
+    return x.text(), x.SLOTB if kind == "dkv" else x.STAGEB
+
+
+PATHS = {
+    "plain": lambda label, op: False,
+    "masked": lambda label, op: re.match(r"LMASK", label) is not None,
+    "late": lambda label, op: re.match(r"L(MASK|LATE)", label) is not None and op != "s_cbranch_scc0",
+    "idle": lambda label, op: re.match(r"L(MASK|LATE|IDLE)", label) is not None and op != "s_cbranch_scc0",
+}
+
+
+@pytest.mark.parametrize("kind,form", [("fwd", 4), ("fwd", 8), ("dq", 4), ("dq", 8), ("dkv", False), ("dkv", True)])
+@pytest.mark.parametrize("path", PATHS)
+def test_attention_loops_copy_to_stages_that_nobody_reads(loops, kind, form, path):
+    text, stage = _loop(loops, kind, form)
+    assert run_stages(text, stage, kind != "dkv", PATHS[path]) >= 16
+
+
+@pytest.mark.parametrize("kind,form,was,becomes,what", [
+    ("fwd", 4, "s_waitcnt vmcnt(4)", "s_waitcnt vmcnt(8)", "landed"), ("dq", 8, "s_waitcnt vmcnt(16)", "s_waitcnt vmcnt(24)", "landed"),
+    ("dkv", True, "s_waitcnt vmcnt(8)", "s_waitcnt vmcnt(12)", "landed"), ("fwd", 4, "s_barrier", "s_nop 0", "read"),
+    ("dq", 4, "s_barrier", "s_nop 0", "read")])
+def test_attention_loops_with_a_wait_less_are_found(loops, kind, form, was, becomes, what):
+    text, stage = _loop(loops, kind, form)
+    assert was in text
+    with pytest.raises(AssertionError, match=what):
+        run_stages([becomes if l == was else l for l in text], stage, kind != "dkv", PATHS["plain"])
+
+
+def test_attention_loops_name_what_they_change(loops):
+    """Scalar condition and m0 as well: a value of the compiler's must not live across a loop in them."""
+    names = [l for l in loops.generate().split("\n") if "_CLOBBERS" in l]
+    assert len(names) == 3 and all(all('"%s"' % r in l for r in ("vcc", "scc", "m0", "memory")) for l in names)
