@@ -97,9 +97,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
     {
       const int row = j0 + 16 * w, rows = sk - row < 16 ? sk - row : 16;
       const uint32_t v_rowb = (uint32_t)p.v_stride * 2u;
-      const int4s rsk = rows_rsrc(reinterpret_cast<const T *>(p.k) + (int64_t)(k0 + row) * p.k_stride + (int64_t)hkv * D,
+      const int4v rsk = rows_rsrc(reinterpret_cast<const T *>(p.k) + (int64_t)(k0 + row) * p.k_stride + (int64_t)hkv * D,
                                   rows > 0 ? (uint32_t)(rows - 1) * k_rowb + ROWB : 0u);
-      const int4s rsv = rows_rsrc(reinterpret_cast<const T *>(p.v) + (int64_t)(k0 + row) * p.v_stride + (int64_t)hkv * D,
+      const int4v rsv = rows_rsrc(reinterpret_cast<const T *>(p.v) + (int64_t)(k0 + row) * p.v_stride + (int64_t)hkv * D,
                                   rows > 0 ? (uint32_t)(rows - 1) * v_rowb + ROWB : 0u);
       uint32_t cv[4];
       rows_lanes(cv, lane, v_rowb);
@@ -128,8 +128,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
     const int rows = sq - i_begin, mct = causal ? 2 : 0, pct = (rows & (BM - 1)) != 0 ? ntq - 1 : -1;
     {
       const int left = rows - ct * BM < BM ? rows - ct * BM : BM;
-      const int4s rsq = rows_rsrc(qp, rem > 0 ? (uint32_t)(left - 1) * q_rowb + ROWB : 0u);
-      const int4s rsd = rows_rsrc(dp, rem > 0 ? (uint32_t)(left - 1) * do_rowb + ROWB : 0u);
+      const int4v rsq = rows_rsrc(qp, rem > 0 ? (uint32_t)(left - 1) * q_rowb + ROWB : 0u);
+      const int4v rsd = rows_rsrc(dp, rem > 0 ? (uint32_t)(left - 1) * do_rowb + ROWB : 0u);
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         copy_1k(cq[i & 3], rsq, i < 4 ? 0u : q16, wbase + 1024u * i);
@@ -137,9 +137,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
       }
       copy_256(c_ld, rows_rsrc(lp, rem > 0 ? ldbytes : 0u), wbase + LD);
     }
-    int4s V[4][4];
+    int4v V[4][4];
     {
-      typedef __attribute__((address_space(3))) const int4s *lds_i4;
+      typedef __attribute__((address_space(3))) const int4v *lds_i4;
       asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
       for (int kb = 0; kb < 4; ++kb)

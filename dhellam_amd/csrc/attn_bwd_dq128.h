@@ -71,7 +71,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
 #pragma unroll
     for (int st = 0; st < STAGES - 1; ++st) {
       const int row = (sp + SPLIT * st) * BN, rows = sk - crow - row < CROWS ? sk - crow - row : CROWS;
-      const int4s rs = rows_rsrc(c_base + (int64_t)row * c_rowb, rows > 0 ? (uint32_t)(rows - 1) * c_rowb + ROWB : 0u);
+      const int4v rs = rows_rsrc(c_base + (int64_t)row * c_rowb, rows > 0 ? (uint32_t)(rows - 1) * c_rowb + ROWB : 0u);
 #pragma unroll
       for (int i = 0; i < COPIES; ++i) copy_1k(cl[i & 3], rs, i < 4 ? 0u : c16, cdst + st * STAGEB + 1024u * i);
     }
@@ -79,20 +79,20 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
     const char *cp = c_base + (int64_t)next * c_rowb;
     const int64_t cstep = (int64_t)SPLIT * BN * c_rowb;
 
-    int4s Q[4][4], dO[4][4];                          // query block, k step
+    int4v Q[4][4], dO[4][4];                          // query block, k step
     floatx4 nd[4];
     float lse[4], del[4];
     {
       // rows of Q, dO and O through LDS, a KB a copy (gathered from memory, 16 rows of 64 bytes a load, the three took 18000 to 25000
       // cycles of a tile's rows)
       const uint32_t own = lds0 + (RG == 4 ? STREAMB + (uint32_t)w * OWN : w < 2 ? (uint32_t)w * STREAMB + 3 * STAGEB : 2 * STREAMB + (uint32_t)(w - 2) * OWN);
-      typedef __attribute__((address_space(3))) const int4s *lds_i4;
+      typedef __attribute__((address_space(3))) const int4v *lds_i4;
       const int rows = sq - wrow0 < 64 ? sq - wrow0 : 64;
-      auto fetch = [&](const void *base, int64_t stride, int4s (&f)[4][4]) {
+      auto fetch = [&](const void *base, int64_t stride, int4v (&f)[4][4]) {
         const uint32_t rowb = (uint32_t)stride * 2u;
         uint32_t off[4];
         rows_lanes(off, lane, rowb);
-        const int4s rs = rows_rsrc(reinterpret_cast<const T *>(base) + (int64_t)(q0 + wrow0) * stride + (int64_t)h * D, rows > 0 ? (uint32_t)(rows - 1) * rowb + ROWB : 0u);
+        const int4v rs = rows_rsrc(reinterpret_cast<const T *>(base) + (int64_t)(q0 + wrow0) * stride + (int64_t)h * D, rows > 0 ? (uint32_t)(rows - 1) * rowb + ROWB : 0u);
 #pragma unroll
         for (int i = 0; i < 16; ++i) copy_1k(off[i & 3], rs, (uint32_t)(i >> 2) * 16u * rowb, own + 1024u * i);
         dma_wait_all();
@@ -108,7 +108,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
         const int row = wrow0 + 16 * qb + r;
         lse[qb] = p.lse[((int64_t)b * p.hq + h) * p.lse_pitch + (row < sq ? row : sq - 1)];
       }
-      int4s O[4][4];
+      int4v O[4][4];
       fetch(p.q, p.q_stride, Q);
       fetch(p.dout, p.do_stride, dO);
       fetch(p.out, p.o_stride, O);

@@ -68,7 +68,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
 #pragma unroll
     for (int st = 0; st < STAGES - 1; ++st) {
       const int row = (sp + SPLIT * st) * BN, rows = sk - crow - row < CROWS ? sk - crow - row : CROWS;
-      const int4s rs = rows_rsrc(c_base + (int64_t)row * c_rowb, rows > 0 ? (uint32_t)(rows - 1) * c_rowb + ROWB : 0u);
+      const int4v rs = rows_rsrc(c_base + (int64_t)row * c_rowb, rows > 0 ? (uint32_t)(rows - 1) * c_rowb + ROWB : 0u);
 #pragma unroll
       for (int i = 0; i < COPIES; ++i) copy_1k(cl[i & 3], rs, i < 4 ? 0u : c16, cdst + st * STAGEB + 1024u * i);
     }
@@ -77,13 +77,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
     const char *cp = c_base + (int64_t)next * c_rowb;
     const int64_t cstep = (int64_t)SPLIT * BN * c_rowb;
 
-    int4s Q[4][4];                                    // query block, k step
+    int4v Q[4][4];                                    // query block, k step
 #pragma unroll
     for (int qb = 0; qb < 4; ++qb) {
       const int row = wrow0 + 16 * qb + r, row_ld = row < sq ? row : sq - 1;
       const T *qp = reinterpret_cast<const T *>(p.q) + (int64_t)(q0 + row_ld) * p.q_stride + (int64_t)h * D + 8 * g;
 #pragma unroll
-      for (int ks = 0; ks < 4; ++ks) Q[qb][ks] = *reinterpret_cast<const int4s *>(qp + 32 * ks);
+      for (int ks = 0; ks < 4; ++ks) Q[qb][ks] = *reinterpret_cast<const int4v *>(qp + 32 * ks);
     }
     // fragment reads: row r, chunk 4 ks + g; transposed: rows 4 g + r / 4 (and 16 further), chunk 2 t + (r % 4) / 2; O: row r, 16-byte
     // chunk 4 t + g of 32

@@ -5,23 +5,6 @@
 
 namespace dh {
 
-typedef int f32_rsrc __attribute__((ext_vector_type(4)));
-
-// Raw buffer descriptor: lanes of a copy that lie at or past `bytes` bring zeros.
-__device__ __forceinline__ f32_rsrc f32_desc(const char *base, int64_t bytes) {
-  const uint64_t a = (uint64_t)(uintptr_t)base;
-  const uint32_t n = bytes <= 0 ? 0u : bytes > 0x7fffffffll ? 0x7fffffffu : (uint32_t)bytes;
-  return f32_rsrc{__builtin_amdgcn_readfirstlane((int)(uint32_t)a), __builtin_amdgcn_readfirstlane((int)((uint32_t)(a >> 32) & 0xffffu)),
-                  __builtin_amdgcn_readfirstlane((int)n), 0x00020000};
-}
-// 64 lanes x 16 bytes to LDS byte address `dst`; the compiler does not count it among what is in flight.
-__device__ __forceinline__ void f32_copy(uint32_t lane_off, const f32_rsrc &rsrc, uint32_t off, uint32_t dst) {
-  asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
-               :
-               : "v"(lane_off), "s"(rsrc), "s"(off), "s"(dst)
-               : "memory", "m0");
-}
-
 // One operand of a tile: 64 rows of X (or columns of Y) by slices of 32 along k, 8 KB each in LDS.
 //   k contiguous: [64][32], 16-byte chunk XOR (row / 2) % 8: 16 rows' reads of one chunk hit 16 different chunks of 256 bytes; a lane
 //     reads four consecutive k of its row at once.
@@ -49,7 +32,7 @@ template <bool STRIDED> struct F32Side {
     off[0] = (uint32_t)wq * CROWS * ldb;
     off[1] = (uint32_t)(wq + 4) * CROWS * ldb;
   }
-  __device__ __forceinline__ f32_rsrc slice(int s, int nsl) const { return f32_desc(base + s * step, s >= nsl ? 0 : STRIDED ? len - s * step : len); }
+  __device__ __forceinline__ int4v slice(int s, int nsl) const { return raw_rsrc(base + s * step, s >= nsl ? 0 : STRIDED ? len - s * step : len); }
 };
 
 template <bool STRIDED> struct F32Reads {
@@ -108,11 +91,11 @@ __global__ void __launch_bounds__(256, 3) gemm_f32_kernel(const GemmF32 g, int t
   for (int q = 0; q < 4; ++q) acc[q >> 1][q & 1] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int s = 0; s < (int)STAGES; ++s) {
-    const f32_rsrc rx = X.slice(s, nsl), ry = Y.slice(s, nsl);
+    const int4v rx = X.slice(s, nsl), ry = Y.slice(s, nsl);
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
-      f32_copy(X.lane_off, rx, X.off[q], dst + s * STAGE + 4096u * q);
-      f32_copy(Y.lane_off, ry, Y.off[q], dst + s * STAGE + SIDE + 4096u * q);
+      copy_1k(X.lane_off, rx, X.off[q], dst + s * STAGE + 4096u * q);
+      copy_1k(Y.lane_off, ry, Y.off[q], dst + s * STAGE + SIDE + 4096u * q);
     }
   }
   asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"(2 * CPW) : "memory");
@@ -127,7 +110,7 @@ __global__ void __launch_bounds__(256, 3) gemm_f32_kernel(const GemmF32 g, int t
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       floatx4 y1[2], x1[2];
-      f32_rsrc rx, ry;
+      int4v rx, ry;
       if (j == 1) {
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(CPW) : "memory");
         rx = X.slice(it + 3, nsl);       // (past the end: zeros that nobody uses)
@@ -144,8 +127,8 @@ __global__ void __launch_bounds__(256, 3) gemm_f32_kernel(const GemmF32 g, int t
           y1[i] = RY.get(from + SIDE, i, 1 - j);
           x1[i] = RX.get(from, i, 1 - j);
         } else if (j == 1) {
-          f32_copy(X.lane_off, rx, X.off[i - 2], dst + now + 4096u * (i - 2));
-          f32_copy(Y.lane_off, ry, Y.off[i - 2], dst + now + SIDE + 4096u * (i - 2));
+          copy_1k(X.lane_off, rx, X.off[i - 2], dst + now + 4096u * (i - 2));
+          copy_1k(Y.lane_off, ry, Y.off[i - 2], dst + now + SIDE + 4096u * (i - 2));
         }
         __builtin_amdgcn_sched_barrier(0);
       }

@@ -111,28 +111,6 @@ __device__ __forceinline__ void gg_locate(const GGGroupTable &gt, int tm_all, in
 // accumulating 1091 -> 806 and 531 -> 413.  One group of 8192 x 8192 x 8192: NT 802 -> 721 (1.52 PFLOP/s; the library 709), TN
 // 849 -> 783 (1.40; the library 928).  What bounds it: power (matrix pipes 82 % busy at 1.76 GHz, TN 71 % at 1.92), and per tile
 // about 8 us of first copies and last stores.
-typedef int gg_i32x4 __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ gg_i32x4 gg_rsrc(const void *ptr, int64_t bytes) {
-  const uint64_t a = (uint64_t)(uintptr_t)ptr;
-  const uint32_t nb = bytes <= 0 ? 0u : (bytes > 0x7fffffffll ? 0x7fffffffu : (uint32_t)bytes);
-  gg_i32x4 r;
-  r[0] = __builtin_amdgcn_readfirstlane((int)(uint32_t)a);
-  r[1] = __builtin_amdgcn_readfirstlane((int)((uint32_t)(a >> 32) & 0xffffu));   // stride 0: raw buffer
-  r[2] = __builtin_amdgcn_readfirstlane((int)nb);
-  r[3] = 0x00020000;
-  return r;
-}
-
-// One 1 KB copy global -> LDS: lane offset + scalar offset from the descriptor's base, wave-uniform LDS byte address.
-template <typename T>
-__device__ __forceinline__ void gg_copy_lds(uint32_t lane_off, const gg_i32x4 &rsrc, uint32_t off, uint32_t lds_dst) {
-  asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
-               :
-               : "v"(lane_off), "s"(rsrc), "s"(off), "s"(lds_dst)
-               : "memory", "m0");
-}
-
 // The outputs of a wavefront (wm = w / 4, wn = w % 4): quarter (qm, qn) holds rows 128 qm + 64 wm + 16 mi + .. and columns
 // 128 qn + 32 wn + 16 nj + .. of the tile; its 16x16 blocks lie transposed in the accumulators (lane % 16: output row, four
 // consecutive columns 4 (lane / 16) + .. a lane).
@@ -279,24 +257,24 @@ __global__ void __launch_bounds__(512) grouped_gemm_w8_kernel(const GGParams p) 
     // the scalar offset with the length, so a row past the end reads as zero whichever block it is in.
     // (k-strided operands: cut at the last k row, i.e. the group's last row for TN; in the other direction a tile that
     // reaches past n or m reads what follows in the operand, into outputs that are not stored)
-    const gg_i32x4 rsa_ = AKS ? gg_rsrc(ag, (int64_t)(row_end - row_begin) * lda_b - (int64_t)m0 * (int)sizeof(T))
-                             : gg_rsrc(ag, (int64_t)(a_rext < 256 ? a_rext : 256) * lda_b);
-    const gg_i32x4 rsb_ = AKS ? gg_rsrc(bg, (int64_t)(row_end - row_begin) * ldb_b - (int64_t)n0 * (int)sizeof(T))
-                       : BKS ? gg_rsrc(bg, (int64_t)p.k_dim * ldb_b - (int64_t)n0 * (int)sizeof(T))
-                             : gg_rsrc(bg, (int64_t)(b_rext < 256 ? b_rext : 256) * ldb_b);
+    const int4v rsa_ = AKS ? raw_rsrc(ag, (int64_t)(row_end - row_begin) * lda_b - (int64_t)m0 * (int)sizeof(T))
+                             : raw_rsrc(ag, (int64_t)(a_rext < 256 ? a_rext : 256) * lda_b);
+    const int4v rsb_ = AKS ? raw_rsrc(bg, (int64_t)(row_end - row_begin) * ldb_b - (int64_t)n0 * (int)sizeof(T))
+                       : BKS ? raw_rsrc(bg, (int64_t)p.k_dim * ldb_b - (int64_t)n0 * (int)sizeof(T))
+                             : raw_rsrc(bg, (int64_t)(b_rext < 256 ? b_rext : 256) * ldb_b);
     // The descriptors come out of v_readfirstlane, and a memory instruction may read such a scalar register five wait
     // states later at the earliest.  The compiler keeps that distance for its own instructions, not for the copies issued
     // from assembly: without this the first of them went out with the previous contents of the length, now and then
     // (a group of fewer than 64 rows then took rows of its neighbour into its weight gradient).
-    gg_i32x4 rsa = rsa_, rsb = rsb_;
+    int4v rsa = rsa_, rsb = rsb_;
     asm volatile("s_nop 4" : "+s"(rsa), "+s"(rsb));
     const int cnt = s1 - s0;                                             // slices of this segment
     // TN: what is added to (nothing to read if nothing is)
     const uint32_t ldc_b = (uint32_t)p.ldc * (uint32_t)sizeof(T);
     T *const cbase = reinterpret_cast<T *>(p.c) + (AKS ? (int64_t)g * p.c_group_stride : 0);
-    gg_i32x4 rsc = AKS ? gg_rsrc(cbase + (int64_t)m0 * p.ldc + n0,
+    int4v rsc = AKS ? raw_rsrc(cbase + (int64_t)m0 * p.ldc + n0,
                                  p.accumulate ? (int64_t)(a_rext < 256 ? a_rext : 256) * ldc_b - (int64_t)n0 * (int)sizeof(T) : 0)
-                       : gg_i32x4{0, 0, 0, 0};
+                       : int4v{0, 0, 0, 0};
     if constexpr (AKS) asm volatile("s_nop 4" : "+s"(rsc));
     // What the copies of a slice read.  For the slices past the last one it is switched to nothing, or, for TN, to the old tile: rows
     // of 512 bytes one behind the other over both stages, which are full of it when the last MFMAs end (a read of its own
@@ -335,13 +313,13 @@ __global__ void __launch_bounds__(512) grouped_gemm_w8_kernel(const GGParams p) 
       const uint32_t at = stage + (uint32_t)h * REG;
       const uint32_t off = AKS && past ? at / 512 * ldc_b : (uint32_t)(s0 + s) * kstep_a + (uint32_t)h * half_a;
 #pragma unroll
-      for (int x = 0; x < 2; ++x) gg_copy_lds<T>(ca[x], rsa, off, cp_lds + at + (uint32_t)(x * 1024));
+      for (int x = 0; x < 2; ++x) copy_1k(ca[x], rsa, off, cp_lds + at + (uint32_t)(x * 1024));
     };
     auto copy_b = [&](int h, int s, uint32_t stage) {
       const uint32_t at = stage + OFF_B + (uint32_t)h * REG;
       const uint32_t off = AKS && past ? at / 512 * ldc_b : (uint32_t)(s0 + s) * kstep_b + (uint32_t)h * half_b;
 #pragma unroll
-      for (int x = 0; x < 2; ++x) gg_copy_lds<T>(cb[x], rsb, off, cp_lds + at + (uint32_t)(x * 1024));
+      for (int x = 0; x < 2; ++x) copy_1k(cb[x], rsb, off, cp_lds + at + (uint32_t)(x * 1024));
     };
     GGAcc8 acc;
 #pragma unroll
@@ -703,10 +681,10 @@ __global__ void __launch_bounds__(2 * BN, ST == 1 ? 4 : 2) grouped_gemm_t_kernel
   }
   const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
   const int kc_tail = (int)(k_total % 64);                        // k-contiguous operands: chunks past it read as zero
-  gg_i32x4 ra, rb;
+  int4v ra, rb;
   auto descriptors = [&](int s) {
-    ra = gg_rsrc(ag + s * kstep_a, a_len - s * kstep_a);
-    rb = gg_rsrc(bg + s * kstep_b, b_len - s * kstep_b);
+    ra = raw_rsrc(ag + s * kstep_a, a_len - s * kstep_a);
+    rb = raw_rsrc(bg + s * kstep_b, b_len - s * kstep_b);
     asm volatile("s_nop 4" : "+s"(ra), "+s"(rb));                 // readfirstlane -> memory instruction
   };
   // copy x (of C::CPW) of slice s into stage st
@@ -719,7 +697,7 @@ __global__ void __launch_bounds__(2 * BN, ST == 1 ? 4 : 2) grouped_gemm_t_kernel
         const int ch = ((lane & 7) ^ (lane >> 4)) ^ (4 * (b & 1));
         if (ch * 8 >= kc_tail) v = OUT;
       }
-      gg_copy_lds<T>(v, ra, (uint32_t)((AKS ? 4 : 8) * b) * lda_b, stage + (uint32_t)(b * 1024));
+      copy_1k(v, ra, (uint32_t)((AKS ? 4 : 8) * b) * lda_b, stage + (uint32_t)(b * 1024));
     } else {
       const int y = x - C::ACPW, b = w * C::BCPW + y;             // (a k-strided B tile of 256 columns is two of 128)
       uint32_t v = vb[y];
@@ -728,7 +706,7 @@ __global__ void __launch_bounds__(2 * BN, ST == 1 ? 4 : 2) grouped_gemm_t_kernel
         if (ch * 8 >= kc_tail) v = OUT;
       }
       const uint32_t off = BKS ? (uint32_t)(4 * (b & 15)) * ldb_b + (uint32_t)((b >> 4) * 256) : (uint32_t)(8 * b) * ldb_b;
-      gg_copy_lds<T>(v, rb, off, stage + (uint32_t)(C::ABYTES + b * 1024));
+      copy_1k(v, rb, off, stage + (uint32_t)(C::ABYTES + b * 1024));
     }
   };
 

@@ -142,6 +142,21 @@ __device__ __forceinline__ void dma_block_fast(const char *base, uint32_t lane_o
                : "memory", "m0");
 }
 
+// Raw buffer descriptor of `bytes` bytes, at most 2 GiB: the lanes of a copy that lie at or past them bring zeros.
+__device__ __forceinline__ int4v raw_rsrc(const void *base, int64_t bytes) {
+  const uint64_t a = (uint64_t)(uintptr_t)base;
+  const uint32_t n = bytes <= 0 ? 0u : bytes > 0x7fffffffll ? 0x7fffffffu : (uint32_t)bytes;
+  return int4v{__builtin_amdgcn_readfirstlane((int)(uint32_t)a), __builtin_amdgcn_readfirstlane((int)((uint32_t)(a >> 32) & 0xffffu)),   // stride 0
+               __builtin_amdgcn_readfirstlane((int)n), 0x00020000};
+}
+// 64 lanes x 16 bytes from descriptor base + lane offset + `off` to LDS byte address `dst`, not counted by the compiler either.
+__device__ __forceinline__ void copy_1k(uint32_t lane_off, const int4v &rsrc, uint32_t off, uint32_t dst) {
+  asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
+               :
+               : "v"(lane_off), "s"(rsrc), "s"(off), "s"(dst)
+               : "memory", "m0");
+}
+
 // NBLK copy blocks (4 rows each, consecutive rows of one tile) of a wavefront in general form: rows past the last key
 // are clamped per lane (they are masked in the scores, and their V rows meet zero probabilities).  Kept
 // as a rolled loop: it runs once per query tile and for tiles that reach past the keys.
