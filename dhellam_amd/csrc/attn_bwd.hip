@@ -765,10 +765,10 @@ int attn_bwd_f32(const void *dout, const void *q, const void *k, const void *v, 
 constexpr int DKV_ROWS = 64;  // key rows of a dK/dV workgroup
 
 // Keeping dS for the dQ product costs 2 bytes per (head, query, key) of workspace, written once and read once.
-// It pays where the recomputing dQ kernel runs its small-grid form (fewer than 256 workgroups of 128 query rows:
-// the 8-head shard at 4096 tokens 181 -> 155 us, at 2048 tokens 95 -> 80 us); with the chip full the recomputing
-// kernel is the faster one (32 heads x 4096: 610 against 669 us; 16 heads: 321 against 329), as the extra
-// memory traffic then costs more than the two products saved.  Above the byte limit dS is never kept.
+// It pays where the recomputing dQ kernel runs its small-grid form (fewer than 256 workgroups of 128 query rows: whole backward, us,
+// recomputing / keeping: the 8-head shard at 4096 tokens 149 / 122, at 2048 tokens 86 / 71); with the chip full the recomputing
+// kernel is the faster one (32 heads x 4096 386 / 479; 16 heads 217 / 275), as the extra memory traffic then costs more
+// than the two products saved.  Above the byte limit dS is never kept.
 static std::atomic<size_t> g_ds_limit{(size_t)1280 << 20};
 static std::atomic<int> g_ds_when_full{0};   // 1: keep dS also where the recomputing dQ kernel would fill the chip
 
@@ -778,11 +778,10 @@ static bool dq_big_grid(int batch, int max_sq, int hq, int causal) {
 }
 
 // Head dim 128 with short sequences and little to do altogether: the kernels of the other head dims start and end sooner
-// than the hand-ordered ones, and dS is not kept.  Backward, us, hand-ordered / other: causal, query rows times heads up to
-// 16384: 32 heads x 100 36 / 27, 8 x 300 41 / 34, 32 x 500 52 / 47, 8 x 8 x 256 47 / 41; above: 64 heads x 300 50 / 57, 16 x 4 x
-// 300 43 / 51, 32 x 32 x 300 329 / 381, 20 to 470 tokens x 32 heads 72 / 83.  Not causal only the shortest: 12 heads x 19
-// 20.6 / 19.1, 4 x 34 20.9 / 20.1, but 8 x 169 + 18 27 / 30, 16 x 22 to 326 44 / 56.  (512 rows and more: within 5 % at few heads,
-// 60 / 81 at 32 x 2 x 512.)
+// than the hand-ordered ones, and dS is not kept.  Backward, us, hand-ordered / other (two launches): causal, query rows times heads up to
+// 16384: 32 heads x 100 32 / 22, 8 x 300 36 / 28, 32 x 500 44 / 37, 8 x 8 x 256 40 / 29; above: 64 heads x 300 41 / 47, 16 x 4 x
+// 300 42 / 48, 32 x 32 x 300 456 / 491, 20 to 470 tokens x 32 heads 81 / 86.  Not causal only the shortest: 12 heads x 19
+// 18.5 / 16.2, 4 x 34 19.1 / 17.2, but 8 x 169 + 18 23 / 25, 16 x 22 to 326 30 / 32.  (512 rows and more: 56 / 76 at 32 x 2 x 512.)
 static bool bwd_short(int max_sq, int max_sk, int causal, int64_t total_q, int hq) {
   if (max_sq >= 512 || max_sk >= 512) return false;
   return causal ? total_q * hq <= 16384 : max_sq <= 48 && max_sk <= 48;
@@ -805,21 +804,22 @@ static int bwd_hsplit(int max_sk, int batch, int hq, int hk, bool paired) {
 //   otherwise by the model: 16 x 1500 not causal (1.28 predicted) 71 / 58 | 234 / 183, 32 / 8 x 600 + 300 (1.38) 49 / 37 | 152 / 100, 32
 //     x 300 (1.15, not taken) 18.8 / 18.5 | 42 / 42, 16 x 1024 (1.0) 29.3 / 30.9 | 89 / 93.
 // Head dim 128 has the hand-ordered kernels to compare with, whose workgroups start and end later but run 1.5 times as fast:
-//   one round: 16 x 300 28 / 20 causal, 26 / 20 not, 8 x 1024 51 / 35 causal, 41 / 35 not;
-//   causal, up to a round and a half: 8 x 1500 66 / 47; two: 32 x 512 44 / 40, 16 x 1024 55 / 57, 16 x 16 x 60 22.8 / 22.5; not
-//   causal: 8 x 1500 62 / 84, 32 x 512 36 / 41.
-// A group split eight ways from 512 rows on (8 query / 1 kv head x 1024: 58 / 46) and rectangular calls of several sequences that
+//   one round: 16 x 300 36 / 20 causal, 26 / 20 not, 8 x 1024 48 / 36 causal, 38 / 36 not;
+//   causal, up to a round and a half: 8 x 1500 58 / 48; two: 32 x 512 44 / 41, 16 x 1024 52 / 57, 16 x 16 x 60 22.9 / 22.6; not
+//   causal: 8 x 1500 50 / 86, 32 x 512 35 / 42.
+// A group split eight ways from 512 rows on (8 query / 1 kv head x 1024: 55 / 43) and rectangular calls of several sequences that
 // are not causal stay with the hand-ordered kernels: callers size the workspace there to choose between their two forms of dQ.
 // Few query rows of many keys are not for it either: dQ is a long chain of key tiles for a few workgroups here and a product over kept dS
-// there: 8 query / 1 kv head x 27 rows x 5086 keys 60 / 122, 4 / 2 x 66 x 918 28 / 33, 1 / 1 x 363 x 1427 31 / 40, 1423 x 2767 60 / 69, but
-// 1833 x 2547 70 / 64 and 12 / 4 x 193 x 450 30 / 26.
+// there: 8 query / 1 kv head x 27 rows x 5086 keys 55 / 124, 4 / 2 x 66 x 918 29 / 34, 1 / 1 x 363 x 1427 31 / 42, 1423 x 2767 50 / 71, but
+// 12 / 4 x 193 x 450 32 / 27.  (The line was drawn against a dK/dV of eight wavefronts.  With the present one long rows of few heads that are not
+// causal are slower here: 1 / 1 x 1500 x 2000 46 / 55, 1833 x 2547 53 / 66, 3000 x 20 50 / 77, 2 / 2 x 4000 86 / 105, but 4 / 4 x 1500 47 / 48.)
 // A group that is left in pieces of several heads makes dK/dV's workgroups that much longer: from 512 rows on not here.  One
-// long sequence among short ones, whole calls, hand-ordered / here with the splits of the grid laid out for the longest / with
-// those of the work: 12 query / 4 kv heads x 791 + 76 + 32 77 / 86 / 57, 4 / 2 x 2746 + 7 135 / 168 / 117.
+// long sequence among short ones, hand-ordered / here: 12 query / 4 kv heads x 791 + 76 + 32 54 / 41, 4 / 2 x 2746 + 7 81 / 80 (with the
+// splits of the grid laid out for the longest instead of those of the work, whole calls, 57 -> 86 and 117 -> 168).
 // A batch of one long sequence and many short ones has a grid for 128-row tiles, most of it empty, and the work of a few 64-row
-// ones.  Backward, hand-ordered / two launches of the tile kernels / one: 8 heads, 1000 rows and 7 x 1 62 / 63 / 46, 4 query / 2 kv heads, 2163 and 7 x
-// 2 135 / 158 / 73, 12 / 4, 386 + 382 and 14 x 1 59 / 59 / 45.  Of 99 such batches of up to 24 sequences 5 are slower in one launch (by up to
-// 7 %); of 51 larger ones 17, by up to a third (4 heads, 599 and 47 x 1 51 / 58 / 68; 4 / 2, 451 and 31 more 57 / 58 / 76): not there.  At the
+// ones.  Backward, hand-ordered / two launches of the tile kernels / one: 8 heads, 1000 rows and 7 x 1 58 / 62 / 47, 4 query / 2 kv heads, 2163 and 7 x
+// 2 109 / 157 / 73, 12 / 4, 386 + 382 and 14 x 1 50 / 59 / 45.  Of 99 such batches of up to 24 sequences 5 were slower in one launch (by up to
+// 7 %); of 51 larger ones 17, by up to a third (4 heads, 599 and 47 x 1 49 / 58 / 68; 4 / 2, 451 and 31 x 3 52 / 56 / 67): not there.  At the
 // other head dims, where the two launches are these kernels too, such batches keep the 128-row dQ tiles.
 static bool dq_tile_fills(int max_sq, int hq, int batch) { return attn_wgs(max_sq, 128, hq, batch, 0) >= 2 * 256; }
 struct BwdBoth { bool pays; int hsplit; };      // key splits of a GQA group: by the workgroups with work

@@ -1,6 +1,7 @@
-// Which of the two families of 16-bit attention kernels a call at head dim 128 takes: the hand-ordered ones (one
-// workgroup of 512 threads per compute unit, causal ones all of one length) or the compiler-scheduled ones that run the
-// other head dims (smaller workgroups, shorter start and end).  Host code, shared by forward and backward.
+// Which of the families of 16-bit attention kernels a call at head dim 128 takes: the hand-ordered ones, one workgroup a compute unit and
+// causal ones all of one length (dK/dV always, the forward and the recomputing dQ where tiles of 256 or 128 rows pay, on one wavefront a SIMD: fwd_rows
+// and dq_rows; else on two, 512 threads), or the compiler-scheduled ones that run the other head dims (smaller workgroups, shorter start and
+// end).  Host code, shared by forward and backward.
 #pragma once
 #include <float.h>
 #include <stdint.h>
@@ -36,18 +37,17 @@ constexpr int ATTN_128ROW_MIN_WG = 256;
 
 // Causal calls: whether the hand-ordered forward / recomputing dQ kernel is the faster one.  Its workgroups run in rounds
 // of 256 (compute units), so what counts is how full the last round is; sequences shorter than the longest have fewer of
-// them (`total_q` rows altogether: the share of the longest sequence's grid that has work).  us, hand-ordered / other,
-// forward unless said:
+// them (`total_q` rows altogether: the share of the longest sequence's grid that has work).  Forward, us, eight wavefronts / other:
 //   one length, full rounds (85 % of the places): 8 heads x 2 x 2048 34 / 39, 8 x 4 x 2048 50 / 71, 32 x 4 x 4096 624 / 706,
-//     16 x 16 x 700 85 / 96; not full: 8 heads x 4 x 3000 111 / 102, 12 x 11264 536 / 444, 32 x 4352 232 / 193 (dQ pass
-//     and dK/dV 906 / 859);
+//     16 x 16 x 700 85 / 96; not full: 8 heads x 4 x 3000 111 / 102, 12 x 11264 536 / 444, 32 x 4352 232 / 193;
 //   several lengths (the longest first, so that rounds overlap): from two rounds of real work on it does not matter how
-//     they come out: 1 to 3324 tokens x 32 heads (4 rounds) 215 / 225, backward 677 / 704; 3000 + 2 x 1000 x 32 (2.5)
-//     129 / 138, backward 392 / 411; with one round only where the longest is long: 4096 + 2000 +
-//     300 x 16 (1.6) 120 / 129, but 4 to 1423 x 32 (1.1) 54 / 48, 1575 + 302 x 32 (1.0) 54 / 43;
+//     they come out: 1 to 3324 tokens x 32 heads (4 rounds) 215 / 225; 3000 + 2 x 1000 x 32 (2.5) 129 / 138; with one round only where the
+//     longest is long: 4096 + 2000 + 300 x 16 (1.6) 120 / 129, but 4 to 1423 x 32 (1.1) 54 / 48, 1575 + 302 x 32 (1.0) 54 / 43;
 //   64-row tiles need long rows as well: 8 heads x 4096 52 / 69, 16 x 2048 35 / 38, but 32 x 1024 26 / 25, 8 x 8 x 512 22 / 18;
 //   128-row ones from 512 on: 32 x 4 x 512 28 / 30, but 16 x 32 x 300 86 / 71.
-// The dQ pass follows the forward: what it gains or loses lies between 1 and 20 % on the same side.
+// The dQ pass follows the forward: with eight wavefronts it gained or lost between 1 and 20 % on the same side.  On one wavefront a SIMD it would be the
+// faster one beyond the line too (whole backward, other dQ / hand-ordered: 32 x 4352 646 / 640, 12 x 11264 1283 / 1261, 8 x 4 x 3000 305 / 277, 32 x 1575 +
+// 302 137 / 121; but 16 x 4096 + 2000 + 300, on this side, 326 / 323).
 static inline bool attn_causal_fills(int max_sq, int hq, int batch, int64_t total_q) {
   if (max_sq <= 0 || batch <= 0) return false;
   const bool big = attn_wgs(max_sq, 128, hq, batch, 1) >= ATTN_128ROW_MIN_WG;
