@@ -188,8 +188,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
 #undef DH_ACC4
     __syncthreads();                                  // everyone is done with the tiles
 
-    // add the wavefronts' partial sums in their order: wavefront w ends up with key block w.  (Those without a tile have none: 1 MB less
-    // through LDS where sequences are a tile or two long.)
+    // add the wavefronts' partial sums in their order: wavefront w ends up with key block w.  (Those without a tile have none: of
+    // 512 KB through LDS a key tile, 128 are left where sequences are one tile long.)
     const int nact = total < NW ? (total > 1 ? total : 1) : NW;
     typedef __attribute__((address_space(3))) floatx4 *lds_f4;
     auto sum_up = [&](const floatx4 (&acc)[4][8], floatx4 (&sum)[8]) {

@@ -11,6 +11,10 @@ namespace dh {
 // one lse and one delta a lane and dS^T is the operand of dQ^T += K^T dS^T as it is: 112 vector instructions, 32 LDS reads and 8 copies
 // for 96 MFMAs.  The prologue forms delta = rowsum(dO O), writes it and the planes that dK/dV reads: this kernel runs before it.
 // Two splits' partial sums go through LDS; each adds up and stores half of the rows.  Causal: row tiles i and n - 1 - i.
+// What it measured: 1860 cycles a tile (two splits 1915 for two), of which the matrix pipe is busy 1536, and 15000 and 16500 cycles to load and
+// store a tile's rows; the eight wavefronts 3400 and 9000.  32 query / 8 kv heads, causal 4096 210 -> 166 us, 4096 rows x 2048 keys 213 -> 166, seven
+// packed sequences of 1 to 3324 tokens 283 -> 234.  Key blocks that no row of a block of 32 sees get no products: a key that is not finite reaches
+// dQ of the rows in its block and behind, no further.
 template <typename T, int RG>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) attn_bwd_dq128_kernel(const AttnBwdParams p) {
   constexpr int D = 128, BM = 64 * RG, BN = 32, SPLIT = 4 / RG, STAGES = 4;

@@ -12,10 +12,11 @@ namespace dh {
 // Whether m has to move is asked of the sum of a lane's eight values, which is needed anyway, instead of their maximum: 112
 // vector instructions and four comparisons, 24 LDS reads and 4 copies for 68 MFMAs.
 // What it measured: 1740 cycles a tile, of which the matrix pipe is busy 1088: a wavefront issues an instruction in 5 cycles, and there are
-// about 290 (barrier 85, the two branches 75).  32 query / 8 kv heads, 4096 rows x 2048 keys 155 -> 127 us (1.08 PFLOP/s), causal
-// 4096 153 -> 134, seven packed sequences of 1 to 3324 tokens 212 -> 191.  Errors against 64 bits (bf16, 4096 causal | scores three
-// times as wide): out 2.080e-3 -> 2.085e-3 | 1.77e-3 -> 1.68e-3, dq 2.440e-3 -> 2.438e-3 | 5.00e-3 -> 4.81e-3, lse 5.8e-8 -> 5.5e-8.  Without the
-// sums of rounded P and with the first tile as the reference 2.12e-3 | 1.89e-3, and 5 % faster.
+// about 290 (barrier 85, the two branches 75).  32 query / 8 kv heads, 4096 rows x 2048 keys 157 -> 129 us (1.07 PFLOP/s), causal
+// 4096 156 -> 133, seven packed sequences of 1 to 3324 tokens 215 -> 184.  Errors of out against 64 bits, the eight wavefronts / here: narrow scores
+// (queries and keys of variance 1) a little larger, since fewer rows have their largest P at exactly 1 (bf16 causal 4096 2.087e-3 / 2.096e-3, fp16
+// 2.606e-4 / 2.617e-4, 32 heads x 600 in 128-row tiles 2.282e-3 / 2.311e-3), scores three and eight times as wide smaller (2.103e-3 / 1.940e-3,
+// 1.809e-3 / 1.703e-3).  Without the sums of rounded P and with the first tile as the reference 2.12e-3 where it is 2.09e-3, and 5 % faster.
 // O goes through LDS (the loop writes it there) and out in whole rows.  (Q through LDS as well, into the half that the tiles leave free, brought
 // nothing: packed sequences 1.256 times the eight wavefronts against 1.255 to 1.268.)  Causal: row tiles i and n - 1 - i.
 template <typename T, int RG>
